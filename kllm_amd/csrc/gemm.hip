@@ -14,6 +14,7 @@
 // A split product writes `nsplit` partial results [nsplit][n][m] in float32;
 // the consumer adds them.
 #include "common.hpp"
+#include "gemm_ring.hpp"
 #include "kllm_kernels.h"
 
 namespace kllm {
@@ -169,28 +170,25 @@ __device__ __forceinline__ floatx16 mfma_tile_step(floatx4 a, floatx4 b, floatx1
 // different slots, so that the 16-byte reads of 16 lanes spread over all 64 banks.
 __device__ __forceinline__ int mfma_swz(int row) { return (row >> 1) & 7; }
 
-// WR x WC waves, each with WTM x 2 MFMA tiles of 32 x 32: a workgroup's tile is 32 WTM WR rows
-// of X by 64 WC rows of W (128 x 128 with four waves, 256 x 128 and 256 x 256 with eight; for
-// decode batches 64 x 128 and 64 x 64 with two).
+// WR x WC waves, each with 2 x 2 MFMA tiles of 32 x 32: a workgroup's tile is 64 WR rows of X by
+// 64 WC rows of W (128 x 128 with four waves, 256 x 128 with eight; for decode batches 64 x 128
+// and 64 x 64 with two).
 // MODE 0: one product; 1 (DUAL): gate and up products with the gate in the epilogue; 2: one product
 // with an activation without a gate in the epilogue.
-template <typename T, typename TOUT, int MODE, int WR, int MSTAGES, int WC = 2, int WTM = 2, int WTN = 2>
+template <typename T, typename TOUT, int MODE, int WR, int MSTAGES, int WC = 2, int WTM = 2>
 __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2))) void gemm_mfma_kernel(const T* __restrict__ X,
                                                              const T* __restrict__ W,
                                                              TOUT* __restrict__ Y, int n, int m,
                                                              int k, int tiles_x, int tiles_y, int kslice, int act,
                                                              const float* __restrict__ act_params, int xcds) {
   constexpr bool DUAL = MODE == 1;
+  constexpr int WTN = 2;
   typedef typename MfmaOperand<T>::type op_t;   // 16 bytes of a row
   constexpr int EPC = 16 / sizeof(T);           // elements of a 16-byte chunk
   constexpr int MBK = MROW / sizeof(T);         // elements of K per stage
   constexpr int BM = 32 * WTM * WR;             // rows of X per workgroup
   constexpr int BN = 32 * WTN * WC;             // rows of W per workgroup
   constexpr int NW = WR * WC;                   // waves
-  // DUAL with an odd number of column tiles a wave: gate and up rows share every tile of 32
-  // columns, 16 each (see the epilogue); with an even number they have tiles of their own.
-  constexpr bool PAIRED = DUAL && WTN % 2 == 1;
-  static_assert(!DUAL || PAIRED || WTN == 2, "DUAL: two column tiles a wave (gate, up) or an odd number of shared ones");
   constexpr int XI = BM / 8 / NW;               // load instructions of X per wave and stage (8 rows each)
   constexpr int WI = BN / 8 / NW;
   constexpr int XBYTES = BM * MROW, WBYTES = BN * MROW;
@@ -223,14 +221,8 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2)
   for (int i = 0; i < WI; ++i) {
     const int r = 8 * (WI * wave + i) + lane / 8;             // DUAL: the first half of the rows gate, the second up
     wchunk[i] = ((lane % 8) ^ mfma_swz(r)) * EPC;
-    long col, up;
-    if (PAIRED) {                                              // ... or 16 gate rows and their 16 up rows in turn
-      col = col0 + 16 * (r / 32) + r % 16;
-      up = r % 32 >= 16;
-    } else {
-      col = DUAL ? col0 + r % (BN / 2) : col0 + r;
-      up = DUAL && r >= BN / 2;
-    }
+    const long col = DUAL ? col0 + r % (BN / 2) : col0 + r;
+    const bool up = DUAL && r >= BN / 2;
     const long wrow = min(col, (long)m - 1) + (up ? m : 0);
     wsrc[i] = W + wrow * k + wchunk[i];
   }
@@ -292,7 +284,7 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2)
       }
 #pragma unroll
       for (int j = 0; j < WTN; ++j) {
-        const int r = (DUAL && !PAIRED ? j * (BN / 2) + wc * 32 : wc * 32 * WTN + j * 32) + lane % 32;
+        const int r = (DUAL ? j * (BN / 2) + wc * 32 : wc * 32 * WTN + j * 32) + lane % 32;
         br[j] = *reinterpret_cast<const op_t*>(ws + r * MROW + (chunk ^ mfma_swz(r)) * 16);
       }
     };
@@ -308,30 +300,6 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2)
     }
   }
 
-  if (PAIRED) {
-    // Lanes c and c + 16 of a tile of 32 columns hold the gate and the up sum of one output
-    // column, for 16 rows each.  They share the rows out: the lane with the gates takes the
-    // first eight and is sent their up sums, the lane with the up sums the other eight and is
-    // sent their gates; every lane then has eight outputs to gate and to store.
-    const int cl = lane % 32;
-    const bool has_gate = cl < 16;
-#pragma unroll
-    for (int j = 0; j < WTN; ++j) {
-      const long c = col0 + 16 * (wc * WTN + j) + cl % 16;
-#pragma unroll
-      for (int i = 0; i < WTM; ++i)
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-          const float lo = acc[i][j][t], hi = acc[i][j][8 + t];
-          const float got = __shfl_xor(has_gate ? hi : lo, 16, kWave);
-          const float gate = has_gate ? lo : got, up = has_gate ? got : hi;
-          const int e = has_gate ? t : 8 + t;
-          const long r = row0 + wr * 32 * WTM + i * 32 + 8 * (e / 4) + 4 * (lane / 32) + e % 4;
-          if (c < m && r < n) Y[r * m + c] = from_f32<TOUT>(gate_act(gate, act) * up);
-        }
-    }
-    return;
-  }
   if (DUAL) {
     const long c = col0 + wc * 32 + lane % 32;
     if (c >= m) return;
@@ -369,12 +337,12 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2)
     }
 }
 
-template <typename T, typename TOUT, int MODE, int WR, int MSTAGES, int WC = 2, int WTM = 2, int WTN = 2>
+template <typename T, typename TOUT, int MODE, int WR, int MSTAGES, int WC = 2, int WTM = 2>
 static int launch_mfma_tile(const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int act,
                             hipStream_t stream, const float* act_params = nullptr) {
   constexpr bool DUAL = MODE == 1;
   constexpr int MBK = MROW / sizeof(T);
-  constexpr int BM = 32 * WTM * WR, BN = 32 * WTN * WC;
+  constexpr int BM = 32 * WTM * WR, BN = 64 * WC;
   const int tx = ceil_div(m, DUAL ? BN / 2 : BN), ty = ceil_div(n, BM);
   const int kslice = ceil_div(ceil_div(k, nsplit), MBK) * MBK;
   const int xcds = device_xcds();
@@ -382,18 +350,20 @@ static int launch_mfma_tile(const void* x, const void* w, void* y, int n, int m,
   const size_t lds = (size_t)MSTAGES * (BM + BN) * MROW;
   static int raised = 0;
   if (lds > 64 * 1024 && !raised) {
-    hipError_t e = hipFuncSetAttribute((const void*)gemm_mfma_kernel<T, TOUT, MODE, WR, MSTAGES, WC, WTM, WTN>,
+    hipError_t e = hipFuncSetAttribute((const void*)gemm_mfma_kernel<T, TOUT, MODE, WR, MSTAGES, WC, WTM>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) KLLM_FAIL((int)e, "gemm mfma: cannot raise the LDS limit: %s", hipGetErrorString(e));
     raised = 1;
   }
-  hipLaunchKernelGGL((gemm_mfma_kernel<T, TOUT, MODE, WR, MSTAGES, WC, WTM, WTN>), grid, dim3(64 * WR * WC), lds, stream,
+  hipLaunchKernelGGL((gemm_mfma_kernel<T, TOUT, MODE, WR, MSTAGES, WC, WTM>), grid, dim3(64 * WR * WC), lds, stream,
                      (const T*)x, (const T*)w, (TOUT*)y, n, m, k, tx, ty, kslice, act, act_params, xcds);
   return 0;
 }
 
 constexpr long kNarrowBelow = 40000000;   // weights (elements) below which a decode batch gets tiles of 64 columns
 
+// bfloat16 products of more than 64 rows run on gemm_ring.hip's tiles; here are decode batches of
+// both types and float32 prompts.
 // Tiles of 256 rows of X (eight waves) fetch a quarter less per flop than two tiles of 128;
 // they are taken when they still give every CU two rounds of work and the last round is not
 // mostly idle (8,192 x 2,560 x 2,048, two and a half rounds: 113 us against 101 us with 128 rows).  The thresholds follow
@@ -424,44 +394,19 @@ static int launch_mfma(const void* x, const void* w, void* y, int n, int m, int 
       return launch_mfma_tile<T, TOUT, MODE, 1, 3>(x, w, y, n, m, k, nsplit, act, stream, act_params);
     return launch_mfma_tile<T, TOUT, MODE, 1, 2>(x, w, y, n, m, k, nsplit, act, stream, act_params);
   }
-  // 256 x 256 tiles (eight waves of 128 x 64, one workgroup a CU) fetch a third less again and
-  // are 10-27 % faster (2,048 x 28,672 x 4,096: 499 us against 561 us) where their rounds fill
-  // the chip: three quarters of the CUs busy on average, counting the last round.  With 80, 128,
-  // 320 or 352 such tiles on 256 CUs they lose by as much.  bfloat16 only: float32 is bound by
-  // its products, not its loads.  Tiles of 256 rows are for more than 128 rows: below, half of
-  // every tile's products would be of rows that are not there (a decode step of 72 tokens at
-  // 1.1B sizes: 2.60 -> 2.54 ms, of 128 at Llama-3-8B sizes: 11.98 -> 11.84 ms).
-  if (sizeof(T) == 2 && n > 128) {
-    const long big = (long)ceil_div(n, 256) * ceil_div(m, DUAL ? 128 : 256) * nsplit;
-    const long rounds = ceil_div(big, (long)cus);
-    const bool big_fits = 4 * big >= 3 * rounds * cus;
-    // 256 x 192 tiles (eight waves of 64 x 96; with the gate, 96 output columns whose gate and
-    // up rows share the column tiles): the fastest tile here where its rounds fill the chip
-    // (2,048 x 11,264 x 2,048: 103 us against 123 us with 256 x 128; 2,048 x 12,288 x 4,096: 195
-    // against 227 us with 128 x 128 and 241 us with 256 x 256; 512 x 22,016 x 4,096: 93 against
-    // 113 us with 256 x 256), taken when its last round is at least 85 % full and it does not
-    // need more time than 256 x 256 by their tiles' sizes and rounds.
-    const long mid = (long)ceil_div(n, 256) * ceil_div(m, DUAL ? 96 : 192) * nsplit;
-    const long mid_rounds = ceil_div(mid, (long)cus);
-    // (a single round of them from three fifths of the CUs on: 768 x 11,264 x 2,048 on 177 tiles 50 us
-    // against 63 us, 1,536 x 6,144 x 4,096 on 192 tiles 92 against 115; on 118 tiles, 512 rows,
-    // 50 against 39)
-    // for a product that is not cut along K, counting only the rows that are there (640 rows
-    // in three tiles of 256: slower, 3.34 -> 3.63 ms for the whole step at 1.1B sizes)
-    const bool one_round = mid_rounds == 1 && nsplit == 1 &&
-                           5L * mid * n >= 3L * cus * 256 * ceil_div(n, 256);
-    const bool mid_fits = 100 * mid >= 85 * mid_rounds * cus || one_round;
-    if (mid_fits && (!big_fits || 3 * mid_rounds <= 4 * rounds))
-      return launch_mfma_tile<T, TOUT, MODE, 4, 2, 2, 2, 3>(x, w, y, n, m, k, nsplit, act, stream, act_params);
-    if (big_fits)
-      return launch_mfma_tile<T, TOUT, MODE, 2, 2, 4, 4>(x, w, y, n, m, k, nsplit, act, stream, act_params);
+  if constexpr (sizeof(T) == 2) {
+    if (k < kRingMaxK)
+      return gemm_ring(x, w, y, n, m, k, nsplit, MODE == 1 ? RING_GATE : MODE == 2 ? RING_UNARY : RING_SUMS, sizeof(TOUT) == 4,
+                       act, act_params, stream);
+    return launch_mfma_tile<T, TOUT, MODE, 1, 2>(x, w, y, n, m, k, nsplit, act, stream, act_params);
+  } else {
+    const long tall = (long)ceil_div(n, 256) * tx * nsplit;
+    if (tall >= 2L * cus && 10 * tall >= 9L * ceil_div(tall, (long)cus) * cus)   // two rounds at least, nine tenths full
+      return launch_mfma_tile<T, TOUT, MODE, 4, 2>(x, w, y, n, m, k, nsplit, act, stream, act_params);
+    const long tiles = (long)ceil_div(n, 128) * tx * nsplit;
+    if (tiles <= cus) return launch_mfma_tile<T, TOUT, MODE, 2, 3>(x, w, y, n, m, k, nsplit, act, stream, act_params);   // one per CU at most
+    return launch_mfma_tile<T, TOUT, MODE, 2, 2>(x, w, y, n, m, k, nsplit, act, stream, act_params);
   }
-  const long tall = (long)ceil_div(n, 256) * tx * nsplit;
-  if (tall >= 2L * cus && 10 * tall >= 9L * ceil_div(tall, (long)cus) * cus)   // two rounds at least, nine tenths full
-    return launch_mfma_tile<T, TOUT, MODE, 4, 2>(x, w, y, n, m, k, nsplit, act, stream, act_params);
-  const long tiles = (long)ceil_div(n, 128) * tx * nsplit;
-  if (tiles <= cus) return launch_mfma_tile<T, TOUT, MODE, 2, 3>(x, w, y, n, m, k, nsplit, act, stream, act_params);   // one per CU at most
-  return launch_mfma_tile<T, TOUT, MODE, 2, 2>(x, w, y, n, m, k, nsplit, act, stream, act_params);
 }
 
 // ------------------------------------------------------------------ bf16 MFMA skinny

@@ -1,0 +1,398 @@
+// Matrix products of prompt size, bfloat16: Y[n, m] = X[n, k] . W[m, k]^T for more than 64 rows of X.
+//
+// One workgroup of eight waves a CU and output tile (256 x 256, 256 x 192 or 128 x 256; two
+// workgroups a CU for 128 x 128).  A tile's rows of X and of W come in two halves each; a stage is 64
+// of K (whole cache lines of 128 bytes), so a stage is four sub-tiles, X0 X1 W0 W1, and LDS holds
+// two stages of them: a ring of eight buffers.
+//
+// What bounds a kernel of this kind is the way from memory into LDS: with two whole stages that are
+// filled, waited for and read one after the other, a CU has one stage in flight for one stage's
+// time and waits for the rest (2,048 x 28,672 x 4,096: 499 us, matrix units busy 36 %).  Here a
+// wave multiplies one quarter of its output at a time, a phase: (X0 W0) (X0 W1) (X1 W1) (X1 W0),
+// the next stage in the mirrored order (X0 W1) (X0 W0) (X1 W0) (X1 W1).  Every phase then reads
+// exactly one new sub-tile from LDS (the other operand is in registers already), which frees
+// its buffer at once, and in the next phase two loads a wave ask for the sub-tile two stages
+// on that goes there.  A load has six to seven phases of eight to land; the wait is for a count
+// (twelve younger loads a wave stay in flight, about 96 KB a CU), never for everything.
+//
+// A phase is two intervals between barriers: reading (LDS -> registers, the next loads) and
+// multiplying.  The waves 4-7 run one interval behind the waves 0-3, and wave i and wave i + 4 share a
+// SIMD: while one multiplies, the other reads, without either wave's code having to interleave the two.
+//
+// Measured with the chip's counters: 2,271 cycles a stage of 256 x 256 where the matrix instructions
+// alone take 2,048 (90 %), whatever the caches hold.  With random operands on all CUs the chip then
+// lowers its clock (2.4 -> 1.7 GHz): power bounds the large products now, not operands.
+// Against the two-stage tiles before, in us: 2,048 x 28,672 x 4,096 (gate) 498 -> 369; 2,048 x 11,264 x
+// 2,048 (gate) 104 -> 79; 2,048 x 6,144 x 4,096 99 -> 78; 2,048 x 4,096 x 14,336 212 -> 167; 500 x
+// 22,016 x 4,096 (gate) 101 -> 79; 500 x 4,096 x 11,008 52 (8 slices) -> 43 (4); 1,500 x 5,632 x 2,048
+// 49 -> 39; 72 x 2,048 x 2,048 11.2 -> 8.4.  Matrix instructions of 32 x 32 in place of 16 x 16 take 2,630
+// cycles a stage (two chains of accumulators a phase do not cover their latency) at the same clock.
+//
+// The operands' roles are exchanged (A = W, B = X): a lane's four accumulators are four neighbouring
+// columns of one row of Y, stored in one instruction.
+#include "gemm_ring.hpp"
+
+#include <math.h>
+
+#include "common.hpp"
+#include "kllm_kernels.h"
+
+namespace kllm {
+
+__device__ __attribute__((aligned(16))) unsigned char g_ring_zeros[16];   // zero-initialised
+
+// Neither the compiler's scheduler nor its memory operations cross this.
+__device__ __forceinline__ void ring_fence() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// This wave's LDS reads are done and at most VM of its loads are in flight.
+template <int VM>
+__device__ __forceinline__ void ring_wait() {
+  static_assert(VM < 64, "vmcnt has six bits");
+  __builtin_amdgcn_s_waitcnt((VM & 0xF) | ((VM >> 4) << 14) | 0x0070);
+}
+
+__device__ __forceinline__ void ring_barrier() {
+  ring_fence();
+  __builtin_amdgcn_s_barrier();
+  ring_fence();
+}
+
+// WR x WC = 8 waves; a wave's part of a sub-tile of X is TM tiles of 16 rows, of W TN.  TAIL: some slice
+// is no multiple of 128, what lies behind its end is read as zeros.
+template <typename TOUT, int MODE, int WR, int WC, int TM, int TN, bool TAIL>
+__global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
+                                                           TOUT* __restrict__ Y, int n, int m, int k, int tiles_x,
+                                                           int tiles_y, int kslice, int act,
+                                                           const float* __restrict__ act_params, int xcds) {
+  constexpr bool GATE = MODE == RING_GATE;
+  constexpr int XR = WR * TM * 16, WS = WC * TN * 16;      // rows of a sub-tile of X, of W
+  constexpr int BM = 2 * XR, BN = GATE ? WS : 2 * WS;      // rows and columns of the output tile
+  constexpr int XB = XR * 128, WB = WS * 128;              // bytes of a sub-tile
+  static_assert(WR * WC == 8 && XR % 64 == 0 && WS % 32 == 0, "eight waves; whole or half load instructions");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];   // X [stage 2][half 2], then W likewise
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int wr = wave / WC, wc = wave % WC, behind = wave / 4;
+
+  // Workgroups are numbered so that the XCDs (which take them round-robin, each with an L2 of its own)
+  // get contiguous runs of tiles, in bands of eight row tiles: a run covers about as many rows as columns.
+  const int total = tiles_x * tiles_y;
+  const int per_xcd = (total + xcds - 1) / xcds;
+  const int id = ((int)blockIdx.x % xcds) * per_xcd + (int)blockIdx.x / xcds;
+  if (id >= total) return;
+  const int band = id / (8 * tiles_x), in_band = id - band * 8 * tiles_x;
+  const int band_rows = min(8, tiles_y - band * 8);
+  const int tcol = in_band / band_rows;
+  const int row0 = (band * 8 + in_band - tcol * band_rows) * BM, col0 = tcol * BN;
+
+  // blockIdx.y: a slice of K (a multiple of 128); its sums go to Y[blockIdx.y]
+  const int kbeg = blockIdx.y * kslice, klen = min(k, kbeg + kslice) - kbeg;    // (TAIL: may be empty, its sums are zeros)
+  const int stages = TAIL ? max(2, (klen + 127) / 128 * 2) : klen / 64;
+  Y += (long)blockIdx.y * n * m;
+
+  // Loads: a wave takes XR / 8 rows of a sub-tile, eight rows an instruction (the second of a W
+  // sub-tile of 96 rows four, with half its lanes).  Lane l serves row l / 8 and, since such a load puts
+  // its 16 bytes at LDS base + 16 l, slot l % 8 of that row.  Row r keeps chunk c (8 elements) in slot
+  // c ^ (r / 2 % 8), so that the 16-byte reads of 16 rows' chunk c meet all banks.  Rows that do not
+  // exist are clamped to the last (their results are never stored).
+  constexpr int XPW = XR / 8, WPW = WS / 8;                // rows per wave
+  constexpr int XL = (XPW + 7) / 8, WL = (WPW + 7) / 8;    // load instructions per wave
+  unsigned xoff[2][XL], woff[2][WL];                        // bytes from the tile's first row, at K = kbeg
+  int xchunk[XL], wchunk[WL];
+#pragma unroll
+  for (int i = 0; i < XL; ++i) {
+    const int r = XPW * wave + 8 * i + lane / 8;
+    xchunk[i] = (lane % 8) ^ ((r >> 1) & 7);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      xoff[h][i] = (unsigned)(min(row0 + h * XR + r, n - 1) - row0) * (unsigned)k * 2u + xchunk[i] * 16u;
+  }
+#pragma unroll
+  for (int i = 0; i < WL; ++i) {
+    const int r = WPW * wave + 8 * i + lane / 8;
+    wchunk[i] = (lane % 8) ^ ((r >> 1) & 7);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)       // GATE: the first half of a tile's rows of W are gates, the second their up rows
+      woff[h][i] = (unsigned)(min(col0 + (GATE ? 0 : h * WS) + r, m - 1) - col0) * (unsigned)k * 2u + wchunk[i] * 16u;
+  }
+  const bf16_t* const xbase = X + (long)row0 * k + kbeg;
+  const bf16_t* const wbase[2] = {W + (long)col0 * k + kbeg, W + ((long)col0 + (GATE ? m : 0)) * k + kbeg};
+
+  auto load = [&](const char* src, unsigned off, int chunk, int left, unsigned char* dst) {
+    const char* at = src + off;
+    if (TAIL) at = chunk * 8 < left ? at : reinterpret_cast<const char*>(g_ring_zeros);
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)at,
+                                     (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+  };
+  auto load_x = [&](int t, int h) {
+    unsigned char* dst = lds + ((t & 1) * 2 + h) * XB + XPW * wave * 128;
+    const char* src = reinterpret_cast<const char*>(xbase) + (long)t * 128;
+#pragma unroll
+    for (int i = 0; i < XL; ++i)
+      if (XPW - 8 * i >= 8 || lane < 8 * (XPW - 8 * i)) load(src, xoff[h][i], xchunk[i], klen - 64 * t, dst + 1024 * i);
+  };
+  auto load_w = [&](int t, int h) {
+    unsigned char* dst = lds + 4 * XB + ((t & 1) * 2 + h) * WB + WPW * wave * 128;
+    const char* src = reinterpret_cast<const char*>(wbase[h]) + (long)t * 128;
+#pragma unroll
+    for (int i = 0; i < WL; ++i)
+      if (WPW - 8 * i >= 8 || lane < 8 * (WPW - 8 * i)) load(src, woff[h][i], wchunk[i], klen - 64 * t, dst + 1024 * i);
+  };
+
+  // MFMA 16x16x32: lane l holds A[l % 16][8 (l / 16) ..], B likewise, D[4 (l / 16) + i][l % 16].
+  const int lrow = lane % 16, lch = lane / 16;
+  const int at = lrow * 128 + (lch ^ ((lrow >> 1) & 7)) * 16;       // (rows 16 apart share their permutation)
+  const unsigned char* const xrd[2] = {lds + wr * TM * 2048 + at, lds + wr * TM * 2048 + (at ^ 64)};
+  const unsigned char* const wrd[2] = {lds + 4 * XB + wc * TN * 2048 + at, lds + 4 * XB + wc * TN * 2048 + (at ^ 64)};
+  bf16x8 xf[TM][2], wf[2][TN][2];                           // [tile][half of the stage's K]
+  auto read_x = [&](int parity, int h) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) xf[i][s] = *reinterpret_cast<const bf16x8*>(xrd[s] + (parity * 2 + h) * XB + i * 2048);
+  };
+  auto read_w = [&](int parity, int h) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) wf[h][j][s] = *reinterpret_cast<const bf16x8*>(wrd[s] + (parity * 2 + h) * WB + j * 2048);
+  };
+  floatx4 acc[2][2][TM][TN];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[a][b][i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](int hx, int hw) {
+    __builtin_amdgcn_s_setprio(1);                          // before the SIMD's other wave, which reads
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          acc[hx][hw][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[hw][j][s], xf[i][s], acc[hx][hw][i][j], 0, 0, 0);
+    __builtin_amdgcn_s_setprio(0);
+  };
+
+  // The order in which phases read the sub-tiles, one each: W0 | X0 W1 X1 W1' X0' W0' X1' W0'' | X0'' ...
+  // (a dash: the next stage), and the loads are asked for in the same order.  A sub-tile is waited for in
+  // the phase before the one that reads it, by every wave in front of that phase's first barrier: the
+  // waves that run an interval behind have then waited before the others read.  Its buffer's last
+  // readers have waited for their reads in front of that barrier too, a whole interval before the loads
+  // that overwrite it are asked for.
+  load_w(0, 0);
+  load_x(0, 0);
+  load_w(0, 1);
+  load_x(0, 1);
+  load_w(1, 1);
+  load_x(1, 0);
+  load_w(1, 0);
+  load_x(1, 1);
+  ring_fence();
+  constexpr int KEEP = 3 * (XL + WL);                       // loads behind the sub-tile that the next phase reads
+  ring_wait<KEEP>();
+  ring_barrier();
+  read_w(0, 0);
+  ring_wait<KEEP>();
+  ring_barrier();
+  if (behind) ring_barrier();
+#define KLLM_RING_PHASE(READ, LOAD, VM, HX, HW) \
+  do {                                          \
+    READ;                                       \
+    LOAD;                                       \
+    ring_fence();                               \
+    ring_wait<(VM)>();                          \
+    ring_barrier();                             \
+    multiply(HX, HW);                           \
+    ring_barrier();                             \
+  } while (0)
+  for (int t = 0; t + 2 < stages; t += 2) {
+    KLLM_RING_PHASE(read_x(0, 0), load_w(t + 2, 0), KEEP, 0, 0);
+    KLLM_RING_PHASE(read_w(0, 1), load_x(t + 2, 0), KEEP, 0, 1);
+    KLLM_RING_PHASE(read_x(0, 1), load_w(t + 2, 1), KEEP, 1, 1);
+    KLLM_RING_PHASE(read_w(1, 1), load_x(t + 2, 1), KEEP, 1, 0);
+    KLLM_RING_PHASE(read_x(1, 0), load_w(t + 3, 1), KEEP, 0, 1);
+    KLLM_RING_PHASE(read_w(1, 0), load_x(t + 3, 0), KEEP, 0, 0);
+    KLLM_RING_PHASE(read_x(1, 1), load_w(t + 3, 0), KEEP, 1, 0);
+    KLLM_RING_PHASE(read_w(0, 0), load_x(t + 3, 1), KEEP, 1, 1);
+  }
+  // the last two stages: nothing more is asked for, the waits count down what is still on its way
+  KLLM_RING_PHASE(read_x(0, 0), , 3 * XL + 2 * WL, 0, 0);
+  KLLM_RING_PHASE(read_w(0, 1), , 2 * XL + 2 * WL, 0, 1);
+  KLLM_RING_PHASE(read_x(0, 1), , 2 * XL + WL, 1, 1);
+  KLLM_RING_PHASE(read_w(1, 1), , XL + WL, 1, 0);
+  KLLM_RING_PHASE(read_x(1, 0), , XL, 0, 1);
+  KLLM_RING_PHASE(read_w(1, 0), , 0, 0, 0);
+  KLLM_RING_PHASE(read_x(1, 1), , 0, 1, 0);
+  multiply(1, 1);
+  if (!behind) ring_barrier();
+#undef KLLM_RING_PHASE
+
+  float a_pos = 0.f, a_neg = 0.f;
+  if (MODE == RING_UNARY && act == ACT_XIELU) {
+    a_pos = softplus_f32(act_params[0]);
+    a_neg = softplus_f32(act_params[1]);
+  }
+  const bool vec = m % 4 == 0 && (reinterpret_cast<uintptr_t>(Y) & (4 * sizeof(TOUT) - 1)) == 0;
+#pragma unroll
+  for (int hx = 0; hx < 2; ++hx)
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int r = row0 + hx * XR + (wr * TM + i) * 16 + lrow;
+      if (r >= n) continue;
+#pragma unroll
+      for (int hw = 0; hw < (GATE ? 1 : 2); ++hw)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const int c = col0 + hw * WS + (wc * TN + j) * 16 + 4 * lch;
+          typedef TOUT vec_t __attribute__((ext_vector_type(4)));
+          vec_t v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            float s = acc[hx][hw][i][j][e];
+            if (GATE) s = gate_act(s, act) * acc[hx][1][i][j][e];
+            if (MODE == RING_UNARY) s = unary_act(s, act, a_pos, a_neg);
+            v[e] = from_f32<TOUT>(s);
+          }
+          TOUT* dst = Y + (long)r * m + c;
+          if (vec && c + 3 < m) {
+            *reinterpret_cast<vec_t*>(dst) = v;
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (c + e < m) dst[e] = v[e];
+          }
+        }
+    }
+}
+
+// ------------------------------------------------------------------ which tile, how many slices of K
+//
+// A product's time in us is put together from what a tile costs a CU: rounds of the chip times (stages
+// x a stage's time + what a tile costs beside its stages), against the time its weights need from
+// memory, plus its output and a launch.  The constants are fitted to a sweep of 13 numbers of rows from
+// 72 to 2,048 and 12 sizes of W from 2,048 x 2,048 to 28,672 x 4,096, with every tile and 1 to 8
+// slices (2,700 products on the full chip, at the clock it holds there): 10 % spread around the
+// fit; the tile and slices that it chooses take 0.9 % longer than the fastest of the
+// sweep on the mean, 12 % at worst.  A 256 x 128 and a 128 x 192 tile were in the sweep too and won nothing
+// that these four do not come within a per cent of.
+struct RingTile {
+  int rows, cols;          // of a product without a gate (with one: half as many columns)
+  int per_cu;              // workgroups a CU holds
+  float stage, tile;       // us a stage of 64 of K (per_cu of them side by side), and beside the stages
+  float stage_alone;       // ... with one workgroup on the CU
+};
+static const RingTile kRingTiles[] = {
+    {256, 256, 1, 1.04f, 3.0f, 1.04f}, {256, 192, 1, 0.835f, 2.6f, 0.835f}, {128, 256, 1, 0.68f, 1.4f, 0.68f},
+    {128, 128, 2, 0.88f, 0.0f, 0.60f}};
+constexpr int kRingTileCount = 4;
+
+static int ring_kslice(int k, int nsplit) { return ceil_div(ceil_div(k, nsplit), 128) * 128; }
+
+static float ring_time(const RingTile& t, int n, int m, int k, int nsplit, bool gate, bool f32_out) {
+  const long cus = device_cus();
+  const long tiles = (long)ceil_div(n, t.rows) * ceil_div(m, gate ? t.cols / 2 : t.cols) * nsplit;
+  const int stages = ring_kslice(k, nsplit) / 64;
+  const long full = tiles / (t.per_cu * cus), rest = tiles % (t.per_cu * cus);
+  float busy = (float)full * (stages * t.stage + t.tile);
+  if (rest) busy += stages * (rest > cus ? t.stage : t.stage_alone) + t.tile;
+  const float weights = 0.2e-6f * 2.f * (gate ? 2.f : 1.f) * m * (float)k;      // 5 TB/s
+  const float out = 0.2e-6f * (f32_out ? 4.f : 2.f) * nsplit * n * (float)m;
+  const float b2 = busy * busy, w2 = weights * weights;
+  return 3.3f + sqrtf(sqrtf(b2 * b2 + w2 * w2)) + out;
+}
+
+static int ring_tile(int n, int m, int k, int nsplit, bool gate, bool f32_out, float* us = nullptr) {
+  int best = 0;
+  float least = 0.f;
+  for (int i = 0; i < kRingTileCount; ++i) {
+    const float t = ring_time(kRingTiles[i], n, m, k, nsplit, gate, f32_out);
+    if (i == 0 || t < least) least = t, best = i;
+  }
+  if (us) *us = least;
+  return best;
+}
+
+template <typename TOUT, int MODE, int WR, int WC, int TM, int TN, bool TAIL>
+static int ring_launch(const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int act,
+                       const float* act_params, hipStream_t stream) {
+  constexpr int XR = WR * TM * 16, WS = WC * TN * 16, BM = 2 * XR, BN = MODE == RING_GATE ? WS : 2 * WS;
+  const int tx = ceil_div(m, BN), ty = ceil_div(n, BM), xcds = device_xcds();
+  const dim3 grid(ceil_div((long)tx * ty, xcds) * xcds, nsplit);   // padded so that every XCD gets as many
+  const size_t lds = (size_t)4 * (XR + WS) * 128;
+  static int raised = 0;
+  if (lds > 64 * 1024 && !raised) {
+    hipError_t e = hipFuncSetAttribute((const void*)gemm_ring_kernel<TOUT, MODE, WR, WC, TM, TN, TAIL>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) KLLM_FAIL((int)e, "gemm ring: cannot raise the LDS limit: %s", hipGetErrorString(e));
+    raised = 1;
+  }
+  hipLaunchKernelGGL((gemm_ring_kernel<TOUT, MODE, WR, WC, TM, TN, TAIL>), grid, dim3(512), lds, stream, (const bf16_t*)x,
+                     (const bf16_t*)w, (TOUT*)y, n, m, k, tx, ty, ring_kslice(k, nsplit), act, act_params, xcds);
+  return 0;
+}
+
+template <typename TOUT, int MODE, bool TAIL>
+static int ring_shape(int tile, const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int act,
+                      const float* ap, hipStream_t st) {
+  switch (tile) {
+    case 0: return ring_launch<TOUT, MODE, 2, 4, 4, 2, TAIL>(x, w, y, n, m, k, nsplit, act, ap, st);
+    case 1: return ring_launch<TOUT, MODE, 4, 2, 2, 3, TAIL>(x, w, y, n, m, k, nsplit, act, ap, st);
+    case 2: return ring_launch<TOUT, MODE, 2, 4, 2, 2, TAIL>(x, w, y, n, m, k, nsplit, act, ap, st);
+    default: return ring_launch<TOUT, MODE, 2, 4, 2, 1, TAIL>(x, w, y, n, m, k, nsplit, act, ap, st);
+  }
+}
+
+template <typename TOUT, int MODE>
+static int ring_tail(int tile, const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int act,
+                     const float* ap, hipStream_t st) {
+  const bool whole = k % 128 == 0 && (long)ring_kslice(k, nsplit) * (nsplit - 1) < k;
+  return !whole ? ring_shape<TOUT, MODE, true>(tile, x, w, y, n, m, k, nsplit, act, ap, st)
+                : ring_shape<TOUT, MODE, false>(tile, x, w, y, n, m, k, nsplit, act, ap, st);
+}
+
+int gemm_ring(const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int mode, bool f32_out, int act,
+              const float* act_params, hipStream_t stream) {
+  KLLM_REQUIRE(k < kRingMaxK, "gemm ring: K=%d", k);
+  const int tile = ring_tile(n, m, k, nsplit, mode == RING_GATE, f32_out);
+  if (mode == RING_GATE) return ring_tail<bf16_t, RING_GATE>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
+  if (mode == RING_UNARY) return ring_tail<bf16_t, RING_UNARY>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
+  if (f32_out) return ring_tail<float, RING_SUMS>(tile, x, w, y, n, m, k, nsplit, act, act_params, stream);
+  return ring_tail<bf16_t, RING_SUMS>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
+}
+
+}  // namespace kllm
+
+using namespace kllm;
+
+// The slices that take the least time together with the kernel that adds them: its reads beyond the
+// 4.5 us that a launch takes whatever it holds (22 MB at 5 TB/s).  Slices of unequal length keep CUs
+// waiting: cuts that leave more than a tenth of K unused are out.
+extern "C" int kllm_gemm_prompt_slices(int n, int m, int k) {
+  if (n <= 0 || m <= 0 || k <= 0) return 1;
+  int best = 1;
+  float least = 0.f;
+  for (int ns : {1, 2, 3, 4, 6, 8}) {
+    const long slice = ring_kslice(k, ns);
+    if (ns > 1 && (slice * (ns - 1) >= k || 10 * slice * ns > 11L * k)) continue;
+    float us;
+    ring_tile(n, m, k, ns, false, true, &us);
+    us += fmaxf(4.5f, 0.2e-6f * 4.f * ns * n * (float)m);
+    if (ns == 1 || us < least) least = us, best = ns;
+  }
+  return best;
+}
+
+// Rows and columns of the tile that a product gets, as rows * 1000 + columns (of W's rows, gates included).
+extern "C" int kllm_gemm_prompt_tile(int n, int m, int k, int nsplit, int gate, int f32_out) {
+  if (n <= 0 || m <= 0 || k <= 0 || nsplit <= 0) return -1;
+  const RingTile& t = kRingTiles[ring_tile(n, m, k, nsplit, gate != 0, f32_out != 0)];
+  return t.rows * 1000 + t.cols;
+}

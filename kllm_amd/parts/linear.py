@@ -15,7 +15,8 @@ rotary + append, SiLU gate); with the compute dtype as result it returns
   bfloat16  n <= 64: MFMA skinny (n <= 16 and one float32 result wanted: the
             decode-batch kernel with all of K in a workgroup; from 17 rows on: MFMA
             tiles of 64 rows)
-            else: MFMA tiles (K in slices where the tiles alone do not fill the chip),
+            else: MFMA tiles (K in slices where the library's estimate of the product and of
+            the kernel that adds the slices is the least with them),
             or the vendor library (torch.matmul) when the engine option
             ``gemm`` is "library" -- the reference uses its vendor library for
             every product (backend/model.cu:494-503)
@@ -56,32 +57,16 @@ def _skinny_split(n, m, k):
     return int(nsplit)
 
 
-def _mfma_split(n, m, k):
-    """Slices of K for the tiled MFMA kernel.  A product with fewer 128 x 128
-    tiles than the chip has room for workgroups (a portion of a prompt, a
-    projection to a narrow output) is bound by how many workgroups stream the
-    weights: up to 8 slices of at least 512 of K bring it to about 512
-    workgroups (measured, 72 rows: 2048 -> 2560 in 9 us instead of 26 us,
-    5632 -> 2048 in 13 us instead of 62 us; 2048 rows, 5632 -> 2048: 57 us
-    instead of 68 us with two slices, the second sum's traffic included)."""
-    tiles = -(-n // 128) * -(-m // 128)
+def _mfma_split(m, k):
+    """Slices of K for the MFMA kernel's tiles of 64 rows and 128 columns (decode batches against
+    the largest weights).  With fewer tiles than the chip has room for workgroups the product is
+    bound by how many of them stream the weights: up to 8 slices of at least 512 of K bring it to
+    about 512 workgroups, 1,024 where K is deep and the tiles alone leave CUs idle."""
+    tiles = -(-m // 128)
     nsplit = 1
-    # slices of at least 512 of K (512 rows, 2,048 -> 2,048 with the norm behind it: 22.1 us in
-    # 4 slices, 23.5 in 8); a deep K bears twice the workgroups if the tiles alone leave CUs idle (1,024 rows, 14,336 -> 4,096:
-    # 136 us in 4 slices, 160 in 2; 512 rows: 83 us in 8, 94 in 4)
     reach = (4 if k >= 8192 and tiles <= K.device_cus() else 2) * K.device_cus()
     while nsplit * 2 <= min(8, reach // tiles, k // 512):
         nsplit *= 2
-    if nsplit == 1 and n > 64:
-        # More 128 x 128 tiles than workgroups fit, but few 256 x 256 ones: slices of at least
-        # 2,048 of K that make those one full round of the chip (2,048 rows, 4,096 wide, with the
-        # norm behind: K = 4,096 114 us in 2 slices against 126 us; 11,008: 208 against 246;
-        # 14,336: 263 against 305)
-        big, cus = -(-n // 256) * -(-m // 256), K.device_cus()
-        for slices in (2, 3, 4):
-            if k // slices >= 2048 and 4 * slices * big >= 3 * cus and slices * big <= cus:
-                nsplit = slices
-                break
     while nsplit > 1 and (-(-(-(-k // nsplit)) // 64) * 64) * (nsplit - 1) >= k:   # no empty slice
         nsplit -= 1
     return nsplit
@@ -118,14 +103,14 @@ def _tiles_beat_skinny(n, m, k):
 
 
 def _decode_tile_split(n, m, k):
-    """Slices of K for a decode batch on the tiled kernel.  Against the largest weights: as
-    for prompts.  Below (tiles of 64 columns): slices of at least 256 of K until every CU
+    """Slices of K for a decode batch on the tiled kernel.  Against the largest weights: see
+    ``_mfma_split``.  Below (tiles of 64 columns): slices of at least 256 of K until every CU
     has a workgroup, then further ones of at least 512, up to 16 (measured at 64 rows, in us
     by slices: 2,048 x 5,632: 14.9 with 4, 9.8 with 8; 11,264 x 2,048: 17.3 with 2, 14.3 with 4,
     17.7 with 8; 4,096 x 4,096: 12.2 with 4, 10.3 with 8, 11.2 with 16)."""
     cols = K.gemm_decode_tile_cols(n, m, k)     # the library's choice: 64 below 40 M weights
     if cols != 64:
-        return _mfma_split(n, m, k)
+        return _mfma_split(m, k)
     tiles, cus = -(-m // cols), K.device_cus()
     nsplit = 1
     while nsplit < 16 and ((tiles * nsplit < cus and k // (2 * nsplit) >= 256) or k // (2 * nsplit) >= 512):
@@ -157,7 +142,7 @@ def choose(dtype, n, m, k, options=None):
         return K.GEMM_SKINNY_BF16, _skinny_split(n, m, k)
     if options.get("gemm") == "library":
         return "library", 1
-    return K.GEMM_MFMA_BF16, _mfma_split(n, m, k)
+    return K.GEMM_MFMA_BF16, K.gemm_prompt_slices(n, m, k)
 
 
 @functools.lru_cache(maxsize=4096)

@@ -417,6 +417,41 @@ def test_gemm_swiglu_at_prompt_sizes(n, f, k, dtype):
                                               else 1e-5 * want.abs().max() + 1e-5)
 
 
+@pytest.mark.parametrize("n,m,k,nsplit,gate,tile", [
+    (65, 515, 8, 1, False, (128, 128)), (65, 130, 64, 1, True, (128, 128)),         # less than a stage, one stage
+    (127, 257, 72, 1, False, (128, 128)), (129, 64, 128, 1, True, (128, 128)),      # an odd number of stages; one pair
+    (193, 131, 192, 3, False, (128, 128)), (100, 96, 640, 4, False, (128, 128)),    # slices of K that hold nothing
+    (257, 515, 1032, 3, False, (128, 128)),
+    (513, 7001, 520, 1, False, (128, 256)), (257, 5602, 520, 1, True, (128, 256)),  # ragged in rows, columns and K
+    (2047, 4099, 520, 1, False, (256, 192)), (700, 5602, 520, 1, True, (256, 192)),
+    (2047, 7001, 520, 1, False, (256, 256)), (1500, 4099, 520, 1, True, (256, 256)),
+    (2047, 7004, 768, 1, False, (256, 256)),                                         # whole stages, whole stores
+])
+def test_prompt_products_on_every_tile(n, m, k, nsplit, gate, tile):
+    """bfloat16 products of more than 64 rows against a product in double, at the edges of tiles,
+    stages and slices, and nothing written beside the output.  A sum of k products of unit normals in
+    32 bits is off by less than k^1/2 2^-24 times a few; the bound leaves a factor of eight."""
+    k_ = K()
+    assert k_.gemm_prompt_tile(n, m, k, nsplit, gate, not gate) == tile
+    rows = 2 * m if gate else m
+    x = rnd(n, k, seed=1, dtype=torch.bfloat16)
+    w = rnd(rows, k, seed=2, dtype=torch.bfloat16, scale=k ** -0.5 if gate else 1.0)
+    want = _gpu_reference(x, w)
+    guard = torch.full((n * m * nsplit + 64,), 7.0, device=DEV, dtype=torch.bfloat16 if gate else torch.float32)
+    if gate:
+        h = guard[:n * m].view(n, m)
+        h.fill_(float("nan"))
+        k_.gemm_swiglu(x, w, h)
+        want = P.silu(want[:, :m]) * want[:, m:]
+        assert (h.double() - want).abs().max() < 0.005 * want.abs().max()
+    else:
+        y = guard[:n * m * nsplit].view(nsplit, n, m)
+        y.fill_(float("nan"))
+        k_.gemm(x, w, y, k_.GEMM_MFMA_BF16, nsplit)
+        assert (y.double().sum(0) - want).abs().max() < 1e-5 * max(k, 64) ** 0.5 * 8
+    assert bool((guard[n * m * nsplit:] == 7.0).all())
+
+
 @pytest.mark.parametrize("n", [5, 8, 16, 33, 64])
 @pytest.mark.parametrize("m,k", [(2048, 2048), (2048, 5632), (4096, 14336), (2560, 2048)])
 def test_split_product_into_its_consumers(n, m, k):
