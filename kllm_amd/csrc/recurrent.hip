@@ -144,23 +144,29 @@ constexpr int kDeltaParts = 16;                              // lanes that share
 constexpr int kDeltaCols = kRecThreads / kDeltaParts;        // columns of a workgroup
 constexpr int kDeltaBlock = 16;                              // tokens staged at a time
 
-// Thread (j, p): column j of the workgroup's block of value channels, rows p, p + 16, ... of it.
-// A block of tokens' vectors goes through LDS: k and q [TB][dk] each, v [TB][16 columns], g and
-// beta [TB]; the sums over a column's rows are lane exchanges within its sixteen lanes.
+// Thread (j, p): column j of the workgroup's block of value channels, and of the state's rows the
+// runs of four that begin at 4 p, 64 + 4 p, ...: NB runs.  A block of tokens' vectors goes through
+// LDS, rows padded with zeros to 64 NB: k and q, v [16 columns], and {g, beta, k . q} per token; the
+// sums over a column's rows are lane exchanges within its sixteen lanes.
+// What bounds it is the chain from token to token on one wave a SIMD.  With D S the decayed state,
+//   u = beta (v - (D S)^T k),   S' = D S + k u^T,   o = S'^T q = (D S)^T q + (k . q) u,
+// so that both sums over the rows are made of the same numbers, run side by side and neither waits
+// for u; k . q comes from the staging.  Rows lie so that a lane reads four with one 16-byte LDS read
+// (sixteen reads of 4 bytes a token before), the next token's while this one is computed.
+// 1,500 tokens, 16 heads of 128 x 128: 635 -> 263 us.
 // VEC: the decay has one number per head and key channel (`dec` [n][H*dk], staged like the keys)
 // instead of one per head.
-template <int NR, bool VEC>
+template <int NB, bool VEC>
 __global__ __launch_bounds__(kRecThreads) void gated_delta_scan_kernel(
     const float* __restrict__ qn, const float* __restrict__ kn, const float* __restrict__ vv,
     const float* __restrict__ gb, float* __restrict__ o_out, float* __restrict__ state, long slot_stride,
     const int* __restrict__ slots, const int* __restrict__ span_start, const int* __restrict__ span_pos, int H, int G,
     int dk, int dv, const float* __restrict__ dec) {
-  extern __shared__ float lds[];
-  float* ks = lds;                                   // [TB][dk]
-  float* qs = ks + kDeltaBlock * dk;                 // [TB][dk]
-  float* vs = qs + kDeltaBlock * dk;                 // [TB][kDeltaCols]
-  float* gs = vs + kDeltaBlock * kDeltaCols;         // [TB][2]
-  float* ds = gs + 2 * kDeltaBlock;                  // [TB][dk] (VEC)
+  constexpr int ROW = 64 * NB;                       // a token's row in LDS
+  constexpr int NV = VEC ? 3 : 2;                    // vectors of a token: k, q and the decays
+  __shared__ __attribute__((aligned(16))) float rows[NV][kDeltaBlock][ROW];
+  __shared__ float vs[kDeltaBlock][kDeltaCols], os[kDeltaBlock][kDeltaCols];
+  __shared__ __attribute__((aligned(16))) float gs[kDeltaBlock][4];      // g, beta, k . q
   const int span = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
   const int g = h / (H / G);
   const int jl = tid / kDeltaParts, p = tid % kDeltaParts;
@@ -169,40 +175,39 @@ __global__ __launch_bounds__(kRecThreads) void gated_delta_scan_kernel(
   const long t0 = span_start[span], t1 = span_start[span + 1];
   const bool fresh = span_pos[span] == 0;
   float* S = state + (long)slots[span] * slot_stride + (long)h * dk * dv;
-  float s[NR];
+  floatx4 s[NB];
 #pragma unroll
-  for (int i = 0; i < NR; ++i) {
-    const int r = p + kDeltaParts * i;
-    s[i] = (col && r < dk && !fresh) ? S[(long)r * dv + j] : 0.f;
-  }
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int r = 64 * b + 4 * p + e;
+      s[b][e] = (col && r < dk && !fresh) ? S[(long)r * dv + j] : 0.f;
+    }
   const int QK = G * dk, HV = H * dv;
-  // A thread's pieces of a block of tokens: NR elements of k and of q (element i = tid + 256 j of
-  // [TB][dk]), one of v, one of g and beta.  They are asked for one block ahead and wait in
-  // registers while the block before them is multiplied.
-  int tt_of[NR], e_of[NR];
-#pragma unroll
-  for (int i = 0; i < NR; ++i) {
-    const int idx = tid + kRecThreads * i;
-    tt_of[i] = idx < kDeltaBlock * dk ? idx / dk : kDeltaBlock;      // kDeltaBlock: no such element
-    e_of[i] = idx - tt_of[i] * dk;
-  }
+  // A thread's pieces of a block of tokens: of each vector the elements tid % 64 + 64 i of tokens
+  // tid / 64 + 4 q, one of v, one of g and beta.  They are asked for one block ahead and wait in
+  // registers while the block before them is multiplied.  A token that is not there decays nothing
+  // and writes nothing: k = q = 0, g = 1, beta = 0.
+  const int e0 = tid % 64, r0 = tid / 64;
   const int v_tt = tid / kDeltaCols, v_c = blockIdx.z * kDeltaCols + tid % kDeltaCols;
   struct Pieces {
-    float k[NR], q[NR], d[VEC ? NR : 1], v, g;
+    float x[NV][4][NB], v, g;
   };
   auto fetch = [&](long tb, int nt) -> Pieces {
     Pieces P;
 #pragma unroll
-    for (int i = 0; i < NR; ++i) {
-      const bool ok = tt_of[i] < nt;
-      const long at = (tb + (ok ? tt_of[i] : 0)) * QK + (long)g * dk + (ok ? e_of[i] : 0);
-      P.k[i] = ok ? kn[at] : 0.f;
-      P.q[i] = ok ? qn[at] : 0.f;
-      if constexpr (VEC)
-        P.d[i] = ok ? dec[(tb + tt_of[i]) * (long)H * dk + (long)h * dk + e_of[i]] : 0.f;
-    }
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        const int tt = r0 + 4 * q, e = e0 + 64 * i;
+        const bool ok = tt < nt && e < dk;
+        const long at = (tb + (ok ? tt : 0)) * QK + (long)g * dk + (ok ? e : 0);
+        P.x[0][q][i] = ok ? kn[at] : 0.f;
+        P.x[1][q][i] = ok ? qn[at] : 0.f;
+        if constexpr (VEC) P.x[2][q][i] = ok ? dec[(tb + tt) * (long)H * dk + (long)h * dk + e] : 1.f;
+      }
     P.v = (v_tt < nt && v_c < dv) ? vv[(tb + v_tt) * HV + (long)h * dv + v_c] : 0.f;
-    P.g = tid < 2 * nt ? gb[(tb + tid / 2) * 2 * H + (tid % 2) * H + h] : 0.f;
+    P.g = tid < 2 * nt ? gb[(tb + tid / 2) * 2 * H + (tid % 2) * H + h] : tid % 2 ? 0.f : 1.f;
     return P;
   };
   long tb = t0;
@@ -211,52 +216,87 @@ __global__ __launch_bounds__(kRecThreads) void gated_delta_scan_kernel(
   while (tb < t1) {
     __syncthreads();                                 // the block before this one has been read
 #pragma unroll
-    for (int i = 0; i < NR; ++i) {
-      const int idx = tid + kRecThreads * i;
-      if (idx < kDeltaBlock * dk) {
-        ks[idx] = pre.k[i];
-        qs[idx] = pre.q[i];
-        if constexpr (VEC) ds[idx] = pre.d[i];
-      }
-    }
-    vs[tid] = pre.v;                                 // [TB][kDeltaCols]: kRecThreads elements
-    if (tid < 2 * kDeltaBlock) gs[tid] = pre.g;
+    for (int x = 0; x < NV; ++x)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int i = 0; i < NB; ++i) rows[x][r0 + 4 * q][e0 + 64 * i] = pre.x[x][q][i];
+    vs[v_tt][tid % kDeltaCols] = pre.v;
+    if (tid < 2 * kDeltaBlock) gs[tid / 2][tid % 2] = pre.g;
     __syncthreads();
     const long tb_next = tb + kDeltaBlock;
     const int nt_next = (int)max(0L, min((long)kDeltaBlock, t1 - tb_next));
     if (nt_next > 0) pre = fetch(tb_next, nt_next);
-    for (int tt = 0; tt < nt; ++tt) {
-      const float decay = gs[2 * tt], beta = gs[2 * tt + 1];
-      const float* kt = ks + tt * dk;
-      const float* qt = qs + tt * dk;
-      float kr[NR], dot = 0.f;
+    {   // k . q: sixteen lanes a token
+      float kq = 0.f;
 #pragma unroll
-      for (int i = 0; i < NR; ++i) {
-        const int r = p + kDeltaParts * i;
-        kr[i] = r < dk ? kt[r] : 0.f;
-        if constexpr (VEC) s[i] *= r < dk ? ds[tt * dk + r] : 0.f; else s[i] *= decay;
-        dot = fmaf(s[i], kr[i], dot);
-      }
-      dot = parts_sum<kDeltaParts>(dot);
-      const float u = beta * (vs[tt * kDeltaCols + jl] - dot);
-      float o = 0.f;
+      for (int b = 0; b < NB; ++b) {
+        const floatx4 kv = *reinterpret_cast<const floatx4*>(&rows[0][jl][64 * b + 4 * p]);
+        const floatx4 qv = *reinterpret_cast<const floatx4*>(&rows[1][jl][64 * b + 4 * p]);
 #pragma unroll
-      for (int i = 0; i < NR; ++i) {
-        const int r = p + kDeltaParts * i;
-        s[i] = fmaf(kr[i], u, s[i]);
-        o = fmaf(s[i], r < dk ? qt[r] : 0.f, o);
+        for (int e = 0; e < 4; ++e) kq = fmaf(kv[e], qv[e], kq);
       }
-      o = parts_sum<kDeltaParts>(o);
-      if (col && p == 0) o_out[(tb + tt) * HV + (long)h * dv + j] = o;
+      kq = parts_sum<kDeltaParts>(kq);
+      if (p == 0) gs[jl][2] = kq;
     }
+    __syncthreads();
+    struct Token {
+      floatx4 k[NB], q[NB], d[VEC ? NB : 1], g;
+      float v;
+    };
+    auto read = [&](int tt, Token& T) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        T.k[b] = *reinterpret_cast<const floatx4*>(&rows[0][tt][64 * b + 4 * p]);
+        T.q[b] = *reinterpret_cast<const floatx4*>(&rows[1][tt][64 * b + 4 * p]);
+        if constexpr (VEC) T.d[b] = *reinterpret_cast<const floatx4*>(&rows[NV - 1][tt][64 * b + 4 * p]);
+      }
+      T.g = *reinterpret_cast<const floatx4*>(&gs[tt][0]);
+      T.v = vs[tt][jl];
+    };
+    float kept = 0.f;                                // token p's output of this column
+    Token T[2];
+    read(0, T[0]);
+    for (int t4 = 0; t4 < nt; t4 += 4) {             // (tokens behind the last change nothing)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int tt = t4 + i;
+        read(min(tt + 1, kDeltaBlock - 1), T[(i + 1) & 1]);
+        const Token& C = T[i & 1];
+        float dk0 = 0.f, dk1 = 0.f, dq0 = 0.f, dq1 = 0.f;
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if constexpr (VEC) s[b][e] *= C.d[b][e]; else s[b][e] *= C.g[0];
+            float& a = e & 1 ? dk1 : dk0;
+            float& c = e & 1 ? dq1 : dq0;
+            a = fmaf(s[b][e], C.k[b][e], a);
+            c = fmaf(s[b][e], C.q[b][e], c);
+          }
+        const float dot = parts_sum<kDeltaParts>(dk0 + dk1), dq = parts_sum<kDeltaParts>(dq0 + dq1);
+        const float u = tt < nt ? C.g[1] * (C.v - dot) : 0.f;      // (0 also where the state is not finite)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s[b][e] = fmaf(C.k[b][e], u, s[b][e]);
+        const float o = fmaf(C.g[2], u, dq);
+        kept = p == tt ? o : kept;
+      }
+    }
+    os[p][jl] = kept;
+    __syncthreads();
+    if (v_tt < nt && v_c < dv) o_out[(tb + v_tt) * HV + (long)h * dv + v_c] = os[v_tt][tid % kDeltaCols];
     tb = tb_next;
     nt = nt_next;
   }
 #pragma unroll
-  for (int i = 0; i < NR; ++i) {
-    const int r = p + kDeltaParts * i;
-    if (col && r < dk) S[(long)r * dv + j] = s[i];
-  }
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int r = 64 * b + 4 * p + e;
+      if (col && r < dk) S[(long)r * dv + j] = s[b][e];
+    }
 }
 
 // ---------------------------------------------------------------------------- gated linear recurrence
@@ -542,22 +582,20 @@ extern "C" int kllm_gated_delta_scan(const float* qn, const float* kn, const flo
                16 * kDeltaParts);
   const dim3 grid(n_spans, H, ceil_div(dv, kDeltaCols));
   KLLM_REQUIRE(grid.z <= 65535, "gated_delta_scan: values too wide for the grid");
-  const size_t lds = ((size_t)kDeltaBlock * ((dec ? 3 : 2) * dk + kDeltaCols + 2)) * sizeof(float);
-  const int nr = ceil_div(dk, kDeltaParts);
-#define KLLM_GDS(NR)                                                                                                   \
+  const int nb = ceil_div(dk, 64);
+#define KLLM_GDS(NB)                                                                                                   \
   do {                                                                                                                 \
     if (dec)                                                                                                           \
-      hipLaunchKernelGGL((gated_delta_scan_kernel<NR, true>), grid, dim3(kRecThreads), lds, stream, qn, kn, vv, gb,    \
+      hipLaunchKernelGGL((gated_delta_scan_kernel<NB, true>), grid, dim3(kRecThreads), 0, stream, qn, kn, vv, gb,      \
                          o_out, state, slot_stride, slots, span_start, span_pos, H, G, dk, dv, dec);                   \
     else                                                                                                               \
-      hipLaunchKernelGGL((gated_delta_scan_kernel<NR, false>), grid, dim3(kRecThreads), lds, stream, qn, kn, vv, gb,   \
+      hipLaunchKernelGGL((gated_delta_scan_kernel<NB, false>), grid, dim3(kRecThreads), 0, stream, qn, kn, vv, gb,     \
                          o_out, state, slot_stride, slots, span_start, span_pos, H, G, dk, dv, dec);                   \
   } while (0)
-  if (nr <= 1) KLLM_GDS(1);
-  else if (nr <= 2) KLLM_GDS(2);
-  else if (nr <= 4) KLLM_GDS(4);
-  else if (nr <= 8) KLLM_GDS(8);
-  else KLLM_GDS(16);
+  if (nb <= 1) KLLM_GDS(1);
+  else if (nb <= 2) KLLM_GDS(2);
+  else if (nb <= 3) KLLM_GDS(3);
+  else KLLM_GDS(4);
 #undef KLLM_GDS
   KLLM_CHECK_LAUNCH("gated_delta_scan");
   return 0;
