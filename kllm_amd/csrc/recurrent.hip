@@ -301,89 +301,193 @@ __global__ __launch_bounds__(kRecThreads) void gated_delta_scan_kernel(
 
 // ---------------------------------------------------------------------------- gated linear recurrence
 
-constexpr int kGateTokens = 8;       // tokens of a tile of the gates' products
-constexpr int kGateOuts = kRecThreads / 4;   // output channels of a workgroup
+constexpr int kGateTile = 16;                 // tokens, and output channels, of a matrix instruction
+constexpr int kGateChunk = 1024;              // inputs of a block that LDS holds at a time
 
-// proj: [nsplit][n][2 W], columns y | x.  Workgroup (tile of tokens, block b of the gates, 64 of
-// its output channels): the convolved inputs of the block's channels for the tile's tokens go
-// into LDS [TT][bs]; the gates' matrices are read [block][in][out] so that neighbouring threads
-// read neighbouring weights.
-__global__ __launch_bounds__(kRecThreads) void linear_recurrence_prep_kernel(
+// proj: [nsplit][n][2 W], columns y | x.  Workgroup (NT tiles of 16 tokens, block b of the gates, OW times
+// 16 of its output channels): the convolved inputs of the block's channels for its tokens go into LDS
+// [tokens][inputs + 4], 1,024 inputs at a time; the gates' products run on the 32-bit matrix instruction 16x16x4 (an
+// FMA chain, as before).  The gates' matrices are read [block][in][out]: a lane's output channel is its
+// lane % 16, so that a load reads 64 bytes of each of four rows.  A = inputs: lane l holds token l % 16,
+// inputs 16 s + 4 (l / 16) + e of step s, e the instruction; which input a product covers is free as
+// long as both operands agree, so a lane reads four with one 16-byte LDS read.
+// KS waves share an output's inputs and meet in LDS: where there is one tile of tokens (a decode batch)
+// the matrices' way from memory bounds the time, and it needs workgroups (16 channels each) and short
+// chains; a prompt has tiles enough and is bound by its products.
+// 1,500 tokens x 2,048 channels in blocks of 256: 144 -> 63 us (FMA on eight tokens at a time, 790 MB of matrices
+// through L2); 8 tokens: 28.8 -> 17.6 us (32 workgroups then, 128 now).
+// TAPS: the convolution's, or 0 (any number).
+template <int NT, int KS, int OW, int TAPS>
+__global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel(
     const float* __restrict__ proj, int nsplit, long split_stride, const float* __restrict__ x_bias,
     const float* __restrict__ conv_w, const float* __restrict__ conv_b, int taps, const float* __restrict__ state,
     long slot_stride, const float* __restrict__ wr_t, const float* __restrict__ wi_t, const float* __restrict__ br,
     const float* __restrict__ bi, const float* __restrict__ rate, const int* __restrict__ span_of_token,
     const int* __restrict__ slots, const int* __restrict__ span_start, const int* __restrict__ span_pos,
     float* __restrict__ a_out, float* __restrict__ b_out, int n, int W, int bs) {
-  extern __shared__ float us[];                      // [TT][bs]
-  const int tile = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
-  const long tfirst = (long)tile * kGateTokens;
-  const int nt = (int)min((long)kGateTokens, n - tfirst);
+  constexpr int TT = NT * kGateTile, THREADS = kWave * KS * OW;
+  extern __shared__ __attribute__((aligned(16))) float us[];
+  const int b = blockIdx.y, tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+  const int chunk = min((bs + 15) / 16 * 16, kGateChunk), ld = chunk + 4;      // inputs in LDS at a time
+  const long tfirst = (long)blockIdx.x * TT;
+  const int nt = (int)min((long)TT, n - tfirst);
   const long cols = 2L * W;
-  for (int i = tid; i < nt * bs; i += kRecThreads) {
-    const int tt = i / bs, c = b * bs + i % bs;
-    const long t = tfirst + tt;
-    const int span = span_of_token[t];
-    // (the convolution's input carries the projection's bias; before position 0 it is zero)
-    us[i] = conv_at(proj, nsplit, split_stride, cols, W + c, x_bias - W, conv_w + (long)c * taps, taps,
-                    state + (long)slots[span] * slot_stride + (long)c * (taps - 1), span_pos[span] == 0, t,
-                    span_start[span]) + conv_b[c];
+  const int ks = wave % KS, ow = wave / KS;
+  const int col = lane % 16, quad = lane / 16;
+  const int o = (blockIdx.z * OW + ow) * kGateTile + col;
+  const int oc = min(o, bs - 1);
+  const float* wr = wr_t + (long)b * bs * bs + oc;
+  const float* wi = wi_t + (long)b * bs * bs + oc;
+  struct Pair { float r[4], i[4]; };
+  auto fetch = [&](int first) -> Pair {       // (inputs that do not exist: zeros, whatever the last row holds)
+    Pair P;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int in = first + 4 * quad + e;
+      const long at = (long)min(in, bs - 1) * bs;
+      const float r = wr[at], g = wi[at];
+      P.r[e] = in < bs ? r : 0.f;
+      P.i[e] = in < bs ? g : 0.f;
+    }
+    return P;
+  };
+  floatx4 ar[NT], ai[NT], own[NT];            // own: the outputs' own inputs
+#pragma unroll
+  for (int t = 0; t < NT; ++t) ar[t] = ai[t] = own[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  __shared__ int4 spans[TT];                  // the tokens' spans
+  if (tid < nt) {
+    const int span = span_of_token[tfirst + tid];
+    spans[tid] = int4{span_start[span], slots[span], span_pos[span] == 0, 0};
   }
-  for (int i = nt * bs + tid; i < kGateTokens * bs; i += kRecThreads) us[i] = 0.f;
-  __syncthreads();
-  const float* wr = wr_t + (long)b * bs * bs;
-  const float* wi = wi_t + (long)b * bs * bs;
-  // A workgroup takes kGateOuts output channels (blockIdx.z); four threads share an output, a
-  // quarter of the inputs each, and meet in LDS: a chain of bs / 4 multiply-adds, and four times
-  // the workgroups, where a decode step has one tile of tokens.
-  __shared__ float red[3][kGateOuts][2 * kGateTokens];
-  const int ol = tid % kGateOuts, part = tid / kGateOuts;
-  const int o = blockIdx.z * kGateOuts + ol;
-  const bool o_ok = o < bs;
-  const int per = (bs + 3) / 4, i0 = part * per, i1 = min(bs, i0 + per);
-  float ar[kGateTokens], ai[kGateTokens];
+  for (int k0 = 0; k0 < bs; k0 += chunk) {
+    __syncthreads();
+    if (TAPS > 0 && nt > 1) {
+      // A thread takes a channel for a run of RUN tokens and asks for the run's inputs at once, each
+      // for all the taps it meets, instead of for every tap of every token on its own.
+      constexpr int K = TAPS > 0 ? TAPS - 1 : 0, RUN = 8;
+      for (int i = tid; i < TT / RUN * chunk; i += THREADS) {
+        const int r = i / chunk, e = k0 + i - r * chunk, c = b * bs + e, tt0 = r * RUN;
+        const bool there = e < bs && tt0 < nt;
+        float x[RUN + K], wt[TAPS > 0 ? TAPS : 1];
+        if (there) {
 #pragma unroll
-  for (int tt = 0; tt < kGateTokens; ++tt) ar[tt] = ai[tt] = 0.f;
-  if (o_ok) {
-#pragma unroll 4
-    for (int i = i0; i < i1; ++i) {
-      const float r = wr[(long)i * bs + o], g = wi[(long)i * bs + o];
+          for (int q = 0; q < RUN + K; ++q) {        // (rows that are not there: some row that is, not used)
+            const long row = min(max(tfirst + tt0 - K + q, 0L), (long)n - 1);
+            x[q] = conv_input(proj, nsplit, split_stride, cols, W + c, x_bias - W, row);
+          }
 #pragma unroll
-      for (int tt = 0; tt < kGateTokens; ++tt) {
-        const float u = us[tt * bs + i];
-        ar[tt] = fmaf(r, u, ar[tt]);
-        ai[tt] = fmaf(g, u, ai[tt]);
+          for (int j = 0; j < TAPS; ++j) wt[j] = conv_w[(long)c * taps + j];
+        }
+        const float cb = there ? conv_b[c] : 0.f;
+#pragma unroll
+        for (int q = 0; q < RUN; ++q) {
+          float v = 0.f;
+          if (there && tt0 + q < nt) {
+            const long t = tfirst + tt0 + q;
+            const int4 sp = spans[tt0 + q];           // first row, slot, whether the span starts at position 0
+#pragma unroll
+            for (int j = 0; j < TAPS; ++j) {
+              const int back = (int)(t - K + j) - sp.x;      // rows behind the span's first
+              float in = x[q + j];
+              if (back < 0) in = sp.z ? 0.f : state[(long)sp.y * slot_stride + (long)c * K + K + back];
+              v = fmaf(wt[j], in, v);
+            }
+            v += cb;
+          }
+          us[(tt0 + q) * ld + e - k0] = v;
+        }
+      }
+    } else {
+      for (int i = tid; i < TT * chunk; i += THREADS) {
+        const int tt = i / chunk, e = k0 + i - tt * chunk, c = b * bs + e;
+        float v = 0.f;
+        if (tt < nt && e < bs) {
+          const int4 sp = spans[tt];
+          // (the convolution's input carries the projection's bias; before position 0 it is zero)
+          v = conv_at(proj, nsplit, split_stride, cols, W + c, x_bias - W, conv_w + (long)c * taps, taps,
+                      state + (long)sp.y * slot_stride + (long)c * (taps - 1), sp.z != 0, tfirst + tt, sp.x) + conv_b[c];
+        }
+        us[tt * ld + e - k0] = v;
       }
     }
-  }
-  if (part > 0) {
+    const int steps = (min(chunk, bs - k0) + 15) / 16;
+    const int per = (steps + KS - 1) / KS, s0 = ks * per, s1 = min(steps, s0 + per);
+    Pair w = fetch(k0 + 16 * min(s0, steps - 1));
+    __syncthreads();
+    if (o >= k0 && o < k0 + chunk)
 #pragma unroll
-    for (int tt = 0; tt < kGateTokens; ++tt) {
-      red[part - 1][ol][2 * tt] = ar[tt];
-      red[part - 1][ol][2 * tt + 1] = ai[tt];
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) own[t][i] = us[(t * kGateTile + 4 * quad + i) * ld + o - k0];
+    for (int s = s0; s < s1; ++s) {
+      const Pair next = fetch(k0 + 16 * min(s + 1, steps - 1));
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const floatx4 u = *reinterpret_cast<const floatx4*>(&us[(t * kGateTile + col) * ld + 16 * s + 4 * quad]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          ar[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(u[e], w.r[e], ar[t], 0, 0, 0);
+          ai[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(u[e], w.i[e], ai[t], 0, 0, 0);
+        }
+      }
+      w = next;
     }
   }
-  __syncthreads();
-  if (part > 0 || !o_ok) return;
-#pragma unroll
-  for (int q = 0; q < 3; ++q)          // in a fixed order
-#pragma unroll
-    for (int tt = 0; tt < kGateTokens; ++tt) {
-      ar[tt] += red[q][ol][2 * tt];
-      ai[tt] += red[q][ol][2 * tt + 1];
+  if constexpr (KS > 1) {                     // the waves' shares, in a fixed order
+    static_assert(OW == 1 && NT == 1, "one tile a workgroup");
+    __shared__ floatx4 red[KS - 1][2][kWave];
+    if (ks > 0) {
+      red[ks - 1][0][lane] = ar[0];
+      red[ks - 1][1][lane] = ai[0];
     }
+    __syncthreads();
+    if (ks > 0) return;
+#pragma unroll
+    for (int q = 0; q < KS - 1; ++q) {
+      ar[0] += red[q][0][lane];
+      ai[0] += red[q][1][lane];
+    }
+  }
+  if (o >= bs) return;
   const int c = b * bs + o;
   const float rb = br[c], ib = bi[c], rt = rate[c];
 #pragma unroll
-  for (int tt = 0; tt < kGateTokens; ++tt) {
-    if (tt >= nt) break;
-    const float r = sigmoid_f32(ar[tt] + rb), ig = sigmoid_f32(ai[tt] + ib);
-    const float log_a = -rt * r;
-    const float a = expf(log_a);
-    const float mult = sqrtf(fmaxf(-expm1f(2.f * log_a), 0.f));      // sqrt(1 - a^2)
-    a_out[(tfirst + tt) * W + c] = a;
-    b_out[(tfirst + tt) * W + c] = mult * ig * us[tt * bs + o];
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {             // D[token 4 quad + i][output lane % 16]
+      const int tt = t * kGateTile + 4 * quad + i;
+      if (tt >= nt) continue;
+      const float r = sigmoid_f32(ar[t][i] + rb), ig = sigmoid_f32(ai[t][i] + ib);
+      const float log_a = -rt * r;
+      const float a = expf(log_a);
+      const float mult = sqrtf(fmaxf(-expm1f(2.f * log_a), 0.f));      // sqrt(1 - a^2)
+      a_out[(tfirst + tt) * W + c] = a;
+      b_out[(tfirst + tt) * W + c] = mult * ig * own[t][i];
+    }
+}
+
+template <int NT, int KS, int OW, int TAPS>
+static int recurrence_prep_launch(const float* proj, int nsplit, long split_stride, const float* x_bias,
+                                  const float* conv_w, const float* conv_b, int taps, const float* state,
+                                  long slot_stride, const float* wr_t, const float* wi_t, const float* br,
+                                  const float* bi, const float* rate, const int* span_of_token, const int* slots,
+                                  const int* span_start, const int* span_pos, float* a_out, float* b_out, int n, int W,
+                                  int blocks, hipStream_t stream) {
+  const int bs = W / blocks;
+  const int chunk = ceil_div(bs, 16) * 16 < kGateChunk ? ceil_div(bs, 16) * 16 : kGateChunk;
+  const size_t lds = (size_t)NT * kGateTile * (chunk + 4) * sizeof(float);
+  static size_t raised_to = 48 * 1024;      // beside the kernel's own LDS
+  if (lds > raised_to) {
+    (void)hipFuncSetAttribute((const void*)linear_recurrence_prep_kernel<NT, KS, OW, TAPS>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    raised_to = lds;
   }
+  hipLaunchKernelGGL((linear_recurrence_prep_kernel<NT, KS, OW, TAPS>),
+                     dim3(ceil_div(n, NT * kGateTile), blocks, ceil_div(bs, OW * kGateTile)), dim3(kWave * KS * OW), lds,
+                     stream, proj, nsplit, split_stride, x_bias, conv_w, conv_b, taps, state, slot_stride, wr_t, wi_t, br,
+                     bi, rate, span_of_token, slots, span_start, span_pos, a_out, b_out, n, W, bs);
+  KLLM_CHECK_LAUNCH("linear_recurrence_prep");
+  return 0;
 }
 
 // S <- a S + b along a span; out = S * gelu_tanh(y + y_bias).  Eight tokens' numbers are asked
@@ -613,18 +717,17 @@ extern "C" int kllm_linear_recurrence_prep(const float* proj, int nsplit, long s
                "linear_recurrence_prep: bad sizes n=%d W=%d blocks=%d", n, W, blocks);
   KLLM_REQUIRE(taps >= 1 && taps <= kMaxTaps, "linear_recurrence_prep: %d taps (1 to %d)", taps, kMaxTaps);
   const int bs = W / blocks;
-  const size_t lds = (size_t)kGateTokens * bs * sizeof(float);
-  KLLM_REQUIRE(lds <= 128 * 1024, "linear_recurrence_prep: blocks of %d channels do not fit into LDS", bs);
-  static size_t raised_to = 48 * 1024;      // beside the kernel's own 12 KB
-  if (lds > raised_to) {
-    (void)hipFuncSetAttribute((const void*)linear_recurrence_prep_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    raised_to = lds;
-  }
-  hipLaunchKernelGGL(linear_recurrence_prep_kernel, dim3(ceil_div(n, kGateTokens), blocks, ceil_div(bs, kGateOuts)), dim3(kRecThreads), lds,
-                     stream, proj, nsplit, split_stride, x_bias, conv_w, conv_b, taps, state, slot_stride, wr_t, wi_t,
-                     br, bi, rate, span_of_token, slots, span_start, span_pos, a_out, b_out, n, W, bs);
-  KLLM_CHECK_LAUNCH("linear_recurrence_prep");
-  return 0;
+  KLLM_REQUIRE(bs <= 4096, "linear_recurrence_prep: blocks of %d channels (up to 4,096)", bs);
+  // Two tiles of tokens a workgroup and eight waves of 16 channels where the tokens give the chip
+  // workgroups enough; one tile, one group of 16 channels and the inputs shared out over four waves below.
+  const bool prompt = n > 64;
+#define KLLM_LRP(NT, KS, OW, TAPS)                                                                                        \
+  recurrence_prep_launch<NT, KS, OW, TAPS>(proj, nsplit, split_stride, x_bias, conv_w, conv_b, taps, state, slot_stride, wr_t, \
+                                     wi_t, br, bi, rate, span_of_token, slots, span_start, span_pos, a_out, b_out, n, W,  \
+                                     blocks, stream)
+  if (taps == 4) return prompt ? KLLM_LRP(2, 1, 8, 4) : KLLM_LRP(1, 4, 1, 4);
+  return prompt ? KLLM_LRP(2, 1, 8, 0) : KLLM_LRP(1, 4, 1, 0);
+#undef KLLM_LRP
 }
 
 extern "C" int kllm_linear_recurrence_scan(const float* a_in, const float* b_in, const float* proj, int nsplit,

@@ -69,3 +69,36 @@ def test_delta_scan(dk, dv, lens, fresh, per_channel):
         state[slot, 5:] = S.reshape(-1)
     close(out.view(n, H, dv), want)
     close(dev_state, state)
+
+
+@pytest.mark.parametrize("blocks,bs", [(3, 8), (2, 40), (1, 130), (2, 256), (1, 1040)])
+@pytest.mark.parametrize("lens", [[1], [1, 1, 1, 1, 1], [9, 1, 7], [40, 24], [64, 1], [3, 120, 2]])
+@pytest.mark.parametrize("taps", [1, 2, 4, 5])
+def test_recurrence_gates(blocks, bs, lens, taps):
+    """Convolution, gates' products and decays: one tile of tokens and several, requests that meet
+    within a tile and within a thread's run of tokens, blocks of odd sizes and of more inputs than LDS takes."""
+    g = torch.Generator().manual_seed(bs + taps)
+    n, W, fresh = sum(lens), blocks * bs, [i % 2 for i in range(len(lens))]
+    r = lambda *s: torch.randn(*s, generator=g)
+    proj, x_bias, conv_w, conv_b = r(2, n, 2 * W), r(W), r(W, taps) * 0.5, r(W) * 0.3
+    wr, wi, br, bi = r(blocks, bs, bs) / bs ** 0.5, r(blocks, bs, bs) / bs ** 0.5, r(W) * 0.3, r(W) * 0.3
+    rate = torch.rand(W, generator=g)
+    state = r(len(lens) + 1, 3 + W * (taps - 1))
+    start, token, span_start, span_pos, slots = spans_of(lens, fresh)
+    d = lambda t: t.to(DEV).contiguous()
+    a, b = (torch.full((n, W), float("nan"), device=DEV) for _ in range(2))
+    K().linear_recurrence_prep(d(proj), d(x_bias), d(conv_w), d(conv_b), taps, d(state), 3, d(wr), d(wi), d(br), d(bi),
+                               d(rate), token, slots, span_start, span_pos, a, b, blocks)
+    x = proj.double().sum(0)[:, W:] + x_bias.double()
+    u = torch.zeros(n, W, dtype=F64)
+    for s in range(len(lens)):
+        before = state[int(slots[s]), 3:].view(W, taps - 1).double().t() * (0.0 if fresh[s] else 1.0)
+        rows = torch.cat([before, x[start[s]:start[s + 1]]])
+        for j in range(taps):
+            u[start[s]:start[s + 1]] += rows[j:j + lens[s]] * conv_w[:, j].double()
+    u = u + conv_b.double()
+    ub = u.view(n, blocks, bs)
+    gate = lambda w, bias: torch.sigmoid(torch.einsum("nbi,bio->nbo", ub, w.double()).reshape(n, W) + bias.double())
+    log_a = -rate.double() * gate(wr, br)
+    close(a, torch.exp(log_a))
+    close(b, torch.sqrt(-torch.expm1(2 * log_a)) * gate(wi, bi) * u, rel=1e-4)   # (the root of a small difference)
