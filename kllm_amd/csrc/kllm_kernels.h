@@ -493,8 +493,8 @@ int kllm_linear_recurrence_prep(const float* proj, int nsplit, long split_stride
 /* S <- a S + b per span and channel (state [W] per slot); out [n][W] = S * gelu_tanh(y + y_bias). */
 int kllm_linear_recurrence_scan(const float* a_in, const float* b_in, const float* proj, int nsplit,
                                 long split_stride, const float* y_bias, float* state, long slot_stride,
-                                const int* slots, const int* span_start, const int* span_pos, void* out, int n_spans,
-                                int W, int dtype, hipStream_t stream);
+                                const int* slots, const int* span_start, const int* span_pos, void* out, int n,
+                                int n_spans, int W, int dtype, hipStream_t stream);
 
 /* out[i] = sa * sum over a's slices + sb * sum over b's slices (float32, `count` elements a slice). */
 int kllm_scaled_sum(float* out, const float* a, int na, long stride_a, float sa, const float* b, int nb,

@@ -102,3 +102,28 @@ def test_recurrence_gates(blocks, bs, lens, taps):
     log_a = -rate.double() * gate(wr, br)
     close(a, torch.exp(log_a))
     close(b, torch.sqrt(-torch.expm1(2 * log_a)) * gate(wi, bi) * u, rel=1e-4)   # (the root of a small difference)
+
+
+@pytest.mark.parametrize("W", [8, 72, 200])
+@pytest.mark.parametrize("lens", [[1, 1, 1], [2], [63, 64, 65], [700, 1]])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_recurrence_chain(W, lens, dtype):
+    """Spans shorter than the segments are many, as long, and much longer; a state that is read and left."""
+    g = torch.Generator().manual_seed(W)
+    n, fresh = sum(lens), [i % 2 for i in range(len(lens))]
+    a, b = torch.rand(n, W, generator=g) ** 0.1, torch.randn(n, W, generator=g)
+    proj, y_bias, state = torch.randn(3, n, 2 * W, generator=g), torch.randn(W, generator=g), torch.randn(len(lens) + 1, 2 + W, generator=g)
+    start, _, span_start, span_pos, slots = spans_of(lens, fresh)
+    dev_state, out = state.to(DEV), torch.full((n, W), float("nan"), device=DEV, dtype=dtype)
+    K().linear_recurrence_scan(a.to(DEV), b.to(DEV), proj.to(DEV), y_bias.to(DEV), dev_state, 2, slots, span_start,
+                               span_pos, len(lens), out)
+    y = torch.nn.functional.gelu(proj.double().sum(0)[:, :W] + y_bias.double(), approximate="tanh")
+    want, state = torch.zeros(n, W, dtype=F64), state.double()
+    for s in range(len(lens)):
+        S = state[int(slots[s]), 2:] * (0.0 if fresh[s] else 1.0)
+        for t in range(start[s], start[s + 1]):
+            S = a[t].double() * S + b[t].double()
+            want[t] = S * y[t]
+        state[int(slots[s]), 2:] = S
+    close(out, want, rel=4e-5 if dtype == torch.float32 else 5e-3)
+    close(dev_state, state)
