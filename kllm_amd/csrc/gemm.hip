@@ -5,8 +5,9 @@
 //   plain   one thread per output; any size; the yardstick the others are
 //           tested against
 //   tiled   true 32-bit FMA tiles through LDS, for the float32 engine
-//   mfma    MFMA tiles through LDS, for prompts: bfloat16 on 32x32x16, float32 on
-//           32x32x2 (32-bit operands, products and sums: no reduced precision)
+//   mfma    MFMA tiles through LDS: up to 64 rows of X here (decode batches; bfloat16 on 32x32x16,
+//           float32 on 32x32x2: 32-bit operands, products and sums, no reduced precision), more rows
+//           in gemm_ring.hip
 //   skinny  bfloat16 MFMA 16x16x32, weights streamed straight from memory,
 //           for up to 64 rows of X (decode batches); K may be split
 //   gemv    one wave per weight row, up to 8 rows of X; K may be split
@@ -111,9 +112,9 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const float* __rest
 }
 
 // ------------------------------------------------------------------ MFMA tiles
-// Workgroup tile 128 (rows of X) x 128 (rows of W), 128 bytes of K per stage
-// (64 bfloat16 or 32 float32), two or three LDS stages.  Four waves in 2 x 2,
-// each 2 x 2 MFMA tiles of 32 x 32.
+// Workgroup tile 64 (rows of X) x 64 or 128 (rows of W), 128 bytes of K per stage
+// (64 bfloat16 or 32 float32), two or three LDS stages.  Two waves, each one or
+// two by two MFMA tiles of 32 x 32.
 // MFMA 32x32x16 (bfloat16): lane l holds A[l%32][8*(l/32)..+7], B[l%32][...]
 // likewise, and D[8*(i/4) + 4*(l/32) + i%4][l%32] in accumulator register i.
 // MFMA 32x32x2 (float32): lane l holds A[l%32][l/32] and B[l%32][l/32], D as
@@ -135,9 +136,8 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const float* __rest
 // matrices are clamped to the last row (their results are never stored) and
 // chunks beyond K come from a page of zeros.
 //
-// Stages: two (64 KB of LDS, two workgroups per CU) when the product has more
-// tiles than CUs; three (one workgroup per CU, a deeper queue of loads) when
-// every CU gets at most one tile.
+// Stages: two when the product has more tiles than CUs; three (a deeper queue of
+// loads) when every CU gets at most one tile.
 //
 // DUAL: W is [gate rows; up rows] = [2m, k]; a workgroup takes 64 gate rows and
 // the 64 up rows that belong to them, and writes act(gate) * up for m columns
@@ -170,9 +170,8 @@ __device__ __forceinline__ floatx16 mfma_tile_step(floatx4 a, floatx4 b, floatx1
 // different slots, so that the 16-byte reads of 16 lanes spread over all 64 banks.
 __device__ __forceinline__ int mfma_swz(int row) { return (row >> 1) & 7; }
 
-// WR x WC waves, each with 2 x 2 MFMA tiles of 32 x 32: a workgroup's tile is 64 WR rows of X by
-// 64 WC rows of W (128 x 128 with four waves, 256 x 128 with eight; for decode batches 64 x 128
-// and 64 x 64 with two).
+// WR x WC waves, each with WTM x 2 MFMA tiles of 32 x 32: a workgroup's tile is 32 WTM WR rows of X by
+// 64 WC rows of W (64 x 128 and 64 x 64 with two waves).
 // MODE 0: one product; 1 (DUAL): gate and up products with the gate in the epilogue; 2: one product
 // with an activation without a gate in the epilogue.
 template <typename T, typename TOUT, int MODE, int WR, int MSTAGES, int WC = 2, int WTM = 2>
@@ -362,12 +361,7 @@ static int launch_mfma_tile(const void* x, const void* w, void* y, int n, int m,
 
 constexpr long kNarrowBelow = 40000000;   // weights (elements) below which a decode batch gets tiles of 64 columns
 
-// bfloat16 products of more than 64 rows run on gemm_ring.hip's tiles; here are decode batches of
-// both types and float32 prompts.
-// Tiles of 256 rows of X (eight waves) fetch a quarter less per flop than two tiles of 128;
-// they are taken when they still give every CU two rounds of work and the last round is not
-// mostly idle (8,192 x 2,560 x 2,048, two and a half rounds: 113 us against 101 us with 128 rows).  The thresholds follow
-// the chip's number of CUs.
+// Products of more than 64 rows run on gemm_ring.hip's tiles; here are decode batches.
 template <typename T, typename TOUT, int MODE>
 static int launch_mfma(const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int act,
                        hipStream_t stream, const float* act_params = nullptr) {
@@ -394,19 +388,10 @@ static int launch_mfma(const void* x, const void* w, void* y, int n, int m, int 
       return launch_mfma_tile<T, TOUT, MODE, 1, 3>(x, w, y, n, m, k, nsplit, act, stream, act_params);
     return launch_mfma_tile<T, TOUT, MODE, 1, 2>(x, w, y, n, m, k, nsplit, act, stream, act_params);
   }
-  if constexpr (sizeof(T) == 2) {
-    if (k < kRingMaxK)
-      return gemm_ring(x, w, y, n, m, k, nsplit, MODE == 1 ? RING_GATE : MODE == 2 ? RING_UNARY : RING_SUMS, sizeof(TOUT) == 4,
-                       act, act_params, stream);
-    return launch_mfma_tile<T, TOUT, MODE, 1, 2>(x, w, y, n, m, k, nsplit, act, stream, act_params);
-  } else {
-    const long tall = (long)ceil_div(n, 256) * tx * nsplit;
-    if (tall >= 2L * cus && 10 * tall >= 9L * ceil_div(tall, (long)cus) * cus)   // two rounds at least, nine tenths full
-      return launch_mfma_tile<T, TOUT, MODE, 4, 2>(x, w, y, n, m, k, nsplit, act, stream, act_params);
-    const long tiles = (long)ceil_div(n, 128) * tx * nsplit;
-    if (tiles <= cus) return launch_mfma_tile<T, TOUT, MODE, 2, 3>(x, w, y, n, m, k, nsplit, act, stream, act_params);   // one per CU at most
-    return launch_mfma_tile<T, TOUT, MODE, 2, 2>(x, w, y, n, m, k, nsplit, act, stream, act_params);
-  }
+  if (k < kRingMaxK)
+    return gemm_ring(x, w, y, n, m, k, nsplit, DUAL ? RING_GATE : MODE == 2 ? RING_UNARY : RING_SUMS, sizeof(T) == 4,
+                     sizeof(TOUT) == 4, act, act_params, stream);
+  return launch_mfma_tile<T, TOUT, MODE, 1, 2>(x, w, y, n, m, k, nsplit, act, stream, act_params);
 }
 
 // ------------------------------------------------------------------ bf16 MFMA skinny

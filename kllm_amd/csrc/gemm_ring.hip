@@ -1,8 +1,9 @@
-// Matrix products of prompt size, bfloat16: Y[n, m] = X[n, k] . W[m, k]^T for more than 64 rows of X.
+// Matrix products of prompt size: Y[n, m] = X[n, k] . W[m, k]^T for more than 64 rows of X, bfloat16, or
+// float32 in true 32-bit.
 //
 // One workgroup of eight waves a CU and output tile (256 x 256, 256 x 192 or 128 x 256; two
-// workgroups a CU for 128 x 128).  A tile's rows of X and of W come in two halves each; a stage is 64
-// of K (whole cache lines of 128 bytes), so a stage is four sub-tiles, X0 X1 W0 W1, and LDS holds
+// workgroups a CU for 128 x 128 and smaller).  A tile's rows of X and of W come in two halves each; a stage
+// is whole cache lines of K (128 bytes: 64 bfloat16 or 32 float32), so a stage is four sub-tiles, X0 X1 W0 W1, and LDS holds
 // two stages of them: a ring of eight buffers.
 //
 // What bounds a kernel of this kind is the way from memory into LDS: with two whole stages that are
@@ -27,6 +28,15 @@
 // 22,016 x 4,096 (gate) 101 -> 79; 500 x 4,096 x 11,008 52 (8 slices) -> 43 (4); 1,500 x 5,632 x 2,048
 // 49 -> 39; 72 x 2,048 x 2,048 11.2 -> 8.4.  Matrix instructions of 32 x 32 in place of 16 x 16 take 2,630
 // cycles a stage (two chains of accumulators a phase do not cover their latency) at the same clock.
+//
+// float32 runs the same code on 16x16x4 instructions, four for the 16 bytes that a lane reads of either
+// operand (which element of K a lane's operand stands for is free as long as A and B agree).  There
+// the matrix unit's rate bounds everything, and what counts is that the CUs get equal numbers of tiles, three of
+// 64 x 128 a CU at a time.  In us against the four-wave tiles of 128 x 128 before (and K in up to 16 slices for
+// few rows): 700 x 11,264 x 2,048 with the gate 389 -> 274 (528 tiles of 128 x 128 on 256 CUs: three on some),
+// 700 x 2,048 x 5,632 238 -> 141, 72 x 11,264 x 2,048 150 -> 87, 2,048 x 11,264 x 2,048 777 -> 707.  Tiles of
+// 128 x 128 in this kernel: 900 x 11,264 x 2,048 510 (two a CU: what is left for the last round goes to
+// CUs in pairs) against 384.
 //
 // The operands' roles are exchanged (A = W, B = X): a lane's four accumulators are four neighbouring
 // columns of one row of Y, stored in one instruction.
@@ -60,18 +70,33 @@ __device__ __forceinline__ void ring_barrier() {
   ring_fence();
 }
 
+template <typename T> struct RingOperand;                // 16 bytes of a row
+template <> struct RingOperand<bf16_t> { typedef bf16x8 type; };
+template <> struct RingOperand<float> { typedef floatx4 type; };
+
+__device__ __forceinline__ floatx4 ring_mma(bf16x8 a, bf16x8 b, floatx4 acc) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
+}
+__device__ __forceinline__ floatx4 ring_mma(floatx4 a, floatx4 b, floatx4 acc) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], acc, 0, 0, 0);
+  return acc;
+}
+
 // WR x WC = 8 waves; a wave's part of a sub-tile of X is TM tiles of 16 rows, of W TN.  TAIL: some slice
 // is no multiple of 128, what lies behind its end is read as zeros.
-template <typename TOUT, int MODE, int WR, int WC, int TM, int TN, bool TAIL>
-__global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
+template <typename T, typename TOUT, int MODE, int WR, int WC, int TM, int TN, bool TAIL>
+__global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const T* __restrict__ X, const T* __restrict__ W,
                                                            TOUT* __restrict__ Y, int n, int m, int k, int tiles_x,
                                                            int tiles_y, int kslice, int act,
                                                            const float* __restrict__ act_params, int xcds) {
   constexpr bool GATE = MODE == RING_GATE;
+  typedef typename RingOperand<T>::type op_t;
+  constexpr int EPC = 16 / sizeof(T), STAGE = 8 * EPC;     // elements of a chunk of 16 bytes, of a stage
   constexpr int XR = WR * TM * 16, WS = WC * TN * 16;      // rows of a sub-tile of X, of W
   constexpr int BM = 2 * XR, BN = GATE ? WS : 2 * WS;      // rows and columns of the output tile
   constexpr int XB = XR * 128, WB = WS * 128;              // bytes of a sub-tile
-  static_assert(WR * WC == 8 && XR % 64 == 0 && WS % 32 == 0, "eight waves; whole or half load instructions");
+  static_assert(WR * WC == 8 && XR % 32 == 0 && WS % 32 == 0, "eight waves; whole or half load instructions");
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];   // X [stage 2][half 2], then W likewise
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -88,14 +113,14 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const bf16_t* __restr
   const int tcol = in_band / band_rows;
   const int row0 = (band * 8 + in_band - tcol * band_rows) * BM, col0 = tcol * BN;
 
-  // blockIdx.y: a slice of K (a multiple of 128); its sums go to Y[blockIdx.y]
+  // blockIdx.y: a slice of K (a multiple of two stages); its sums go to Y[blockIdx.y]
   const int kbeg = blockIdx.y * kslice, klen = min(k, kbeg + kslice) - kbeg;    // (TAIL: may be empty, its sums are zeros)
-  const int stages = TAIL ? max(2, (klen + 127) / 128 * 2) : klen / 64;
+  const int stages = TAIL ? max(2, (klen + 2 * STAGE - 1) / (2 * STAGE) * 2) : klen / STAGE;
   Y += (long)blockIdx.y * n * m;
 
-  // Loads: a wave takes XR / 8 rows of a sub-tile, eight rows an instruction (the second of a W
-  // sub-tile of 96 rows four, with half its lanes).  Lane l serves row l / 8 and, since such a load puts
-  // its 16 bytes at LDS base + 16 l, slot l % 8 of that row.  Row r keeps chunk c (8 elements) in slot
+  // Loads: a wave takes an eighth of a sub-tile's rows, eight rows an instruction (four, with half its
+  // lanes, where it has only those left).  Lane l serves row l / 8 and, since such a load puts
+  // its 16 bytes at LDS base + 16 l, slot l % 8 of that row.  Row r keeps chunk c (16 bytes) in slot
   // c ^ (r / 2 % 8), so that the 16-byte reads of 16 rows' chunk c meet all banks.  Rows that do not
   // exist are clamped to the last (their results are never stored).
   constexpr int XPW = XR / 8, WPW = WS / 8;                // rows per wave
@@ -108,7 +133,7 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const bf16_t* __restr
     xchunk[i] = (lane % 8) ^ ((r >> 1) & 7);
 #pragma unroll
     for (int h = 0; h < 2; ++h)
-      xoff[h][i] = (unsigned)(min(row0 + h * XR + r, n - 1) - row0) * (unsigned)k * 2u + xchunk[i] * 16u;
+      xoff[h][i] = (unsigned)(min(row0 + h * XR + r, n - 1) - row0) * (unsigned)k * (unsigned)sizeof(T) + xchunk[i] * 16u;
   }
 #pragma unroll
   for (int i = 0; i < WL; ++i) {
@@ -116,14 +141,14 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const bf16_t* __restr
     wchunk[i] = (lane % 8) ^ ((r >> 1) & 7);
 #pragma unroll
     for (int h = 0; h < 2; ++h)       // GATE: the first half of a tile's rows of W are gates, the second their up rows
-      woff[h][i] = (unsigned)(min(col0 + (GATE ? 0 : h * WS) + r, m - 1) - col0) * (unsigned)k * 2u + wchunk[i] * 16u;
+      woff[h][i] = (unsigned)(min(col0 + (GATE ? 0 : h * WS) + r, m - 1) - col0) * (unsigned)k * (unsigned)sizeof(T) + wchunk[i] * 16u;
   }
-  const bf16_t* const xbase = X + (long)row0 * k + kbeg;
-  const bf16_t* const wbase[2] = {W + (long)col0 * k + kbeg, W + ((long)col0 + (GATE ? m : 0)) * k + kbeg};
+  const T* const xbase = X + (long)row0 * k + kbeg;
+  const T* const wbase[2] = {W + (long)col0 * k + kbeg, W + ((long)col0 + (GATE ? m : 0)) * k + kbeg};
 
   auto load = [&](const char* src, unsigned off, int chunk, int left, unsigned char* dst) {
     const char* at = src + off;
-    if (TAIL) at = chunk * 8 < left ? at : reinterpret_cast<const char*>(g_ring_zeros);
+    if (TAIL) at = chunk * EPC < left ? at : reinterpret_cast<const char*>(g_ring_zeros);
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)at,
                                      (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
   };
@@ -132,33 +157,33 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const bf16_t* __restr
     const char* src = reinterpret_cast<const char*>(xbase) + (long)t * 128;
 #pragma unroll
     for (int i = 0; i < XL; ++i)
-      if (XPW - 8 * i >= 8 || lane < 8 * (XPW - 8 * i)) load(src, xoff[h][i], xchunk[i], klen - 64 * t, dst + 1024 * i);
+      if (XPW - 8 * i >= 8 || lane < 8 * (XPW - 8 * i)) load(src, xoff[h][i], xchunk[i], klen - STAGE * t, dst + 1024 * i);
   };
   auto load_w = [&](int t, int h) {
     unsigned char* dst = lds + 4 * XB + ((t & 1) * 2 + h) * WB + WPW * wave * 128;
     const char* src = reinterpret_cast<const char*>(wbase[h]) + (long)t * 128;
 #pragma unroll
     for (int i = 0; i < WL; ++i)
-      if (WPW - 8 * i >= 8 || lane < 8 * (WPW - 8 * i)) load(src, woff[h][i], wchunk[i], klen - 64 * t, dst + 1024 * i);
+      if (WPW - 8 * i >= 8 || lane < 8 * (WPW - 8 * i)) load(src, woff[h][i], wchunk[i], klen - STAGE * t, dst + 1024 * i);
   };
 
-  // MFMA 16x16x32: lane l holds A[l % 16][8 (l / 16) ..], B likewise, D[4 (l / 16) + i][l % 16].
+  // MFMA 16x16: lane l holds 16 bytes of row l % 16 of A from chunk l / 16 on, B likewise, D[4 (l / 16) + i][l % 16].
   const int lrow = lane % 16, lch = lane / 16;
   const int at = lrow * 128 + (lch ^ ((lrow >> 1) & 7)) * 16;       // (rows 16 apart share their permutation)
   const unsigned char* const xrd[2] = {lds + wr * TM * 2048 + at, lds + wr * TM * 2048 + (at ^ 64)};
   const unsigned char* const wrd[2] = {lds + 4 * XB + wc * TN * 2048 + at, lds + 4 * XB + wc * TN * 2048 + (at ^ 64)};
-  bf16x8 xf[TM][2], wf[2][TN][2];                           // [tile][half of the stage's K]
+  op_t xf[TM][2], wf[2][TN][2];                           // [tile][half of the stage's K]
   auto read_x = [&](int parity, int h) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int s = 0; s < 2; ++s) xf[i][s] = *reinterpret_cast<const bf16x8*>(xrd[s] + (parity * 2 + h) * XB + i * 2048);
+      for (int s = 0; s < 2; ++s) xf[i][s] = *reinterpret_cast<const op_t*>(xrd[s] + (parity * 2 + h) * XB + i * 2048);
   };
   auto read_w = [&](int parity, int h) {
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int s = 0; s < 2; ++s) wf[h][j][s] = *reinterpret_cast<const bf16x8*>(wrd[s] + (parity * 2 + h) * WB + j * 2048);
+      for (int s = 0; s < 2; ++s) wf[h][j][s] = *reinterpret_cast<const op_t*>(wrd[s] + (parity * 2 + h) * WB + j * 2048);
   };
   floatx4 acc[2][2][TM][TN];
 #pragma unroll
@@ -177,7 +202,7 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const bf16_t* __restr
       for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
-          acc[hx][hw][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[hw][j][s], xf[i][s], acc[hx][hw][i][j], 0, 0, 0);
+          acc[hx][hw][i][j] = ring_mma(wf[hw][j][s], xf[i][s], acc[hx][hw][i][j]);
     __builtin_amdgcn_s_setprio(0);
   };
 
@@ -277,50 +302,64 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const bf16_t* __restr
 //
 // A product's time in us is put together from what a tile costs a CU: rounds of the chip times (stages
 // x a stage's time + what a tile costs beside its stages), against the time its weights need from
-// memory, plus its output and a launch.  The constants are fitted to a sweep of 13 numbers of rows from
-// 72 to 2,048 and 12 sizes of W from 2,048 x 2,048 to 28,672 x 4,096, with every tile and 1 to 8
+// memory, plus its output and a launch.  The constants for bfloat16 are fitted to a sweep of 13 numbers of rows
+// from 72 to 2,048 and 12 sizes of W from 2,048 x 2,048 to 28,672 x 4,096, with every tile and 1 to 8
 // slices (2,700 products on the full chip, at the clock it holds there): 10 % spread around the
 // fit; the tile and slices that it chooses take 0.9 % longer than the fastest of the
 // sweep on the mean, 12 % at worst.  A 256 x 128 and a 128 x 192 tile were in the sweep too and won nothing
-// that these four do not come within a per cent of.
+// that these four do not come within a per cent of.  float32: a stage's products at the rate that the
+// matrix unit reaches (138 TFLOP/s on the chip); one workgroup alone on its CU, a single chain of
+// products a wave, takes a third longer.
 struct RingTile {
   int rows, cols;          // of a product without a gate (with one: half as many columns)
   int per_cu;              // workgroups a CU holds
-  float stage, tile;       // us a stage of 64 of K (per_cu of them side by side), and beside the stages
+  float stage, tile;       // us a stage of 128 bytes of K (per_cu of them side by side), and beside the stages
   float stage_alone;       // ... with one workgroup on the CU
 };
-static const RingTile kRingTiles[] = {
+static const RingTile kRingTilesBf16[] = {
     {256, 256, 1, 1.04f, 3.0f, 1.04f}, {256, 192, 1, 0.835f, 2.6f, 0.835f}, {128, 256, 1, 0.68f, 1.4f, 0.68f},
     {128, 128, 2, 0.88f, 0.0f, 0.60f}};
-constexpr int kRingTileCount = 4;
+static const RingTile kRingTilesF32[] = {{64, 128, 3, 2.94f, 1.0f, 1.30f}};
+struct RingTiles {
+  const RingTile* tile;
+  int count, pair;         // elements of K in two stages
+};
+static RingTiles ring_tiles(bool f32) {
+  if (f32) return {kRingTilesF32, 1, 64};
+  return {kRingTilesBf16, 4, 128};
+}
 
-static int ring_kslice(int k, int nsplit) { return ceil_div(ceil_div(k, nsplit), 128) * 128; }
+static int ring_kslice(int k, int nsplit, int pair) { return ceil_div(ceil_div(k, nsplit), pair) * pair; }
 
-static float ring_time(const RingTile& t, int n, int m, int k, int nsplit, bool gate, bool f32_out) {
+static float ring_time(const RingTile& t, int pair, int n, int m, int k, int nsplit, bool gate, int in_bytes, int out_bytes) {
   const long cus = device_cus();
   const long tiles = (long)ceil_div(n, t.rows) * ceil_div(m, gate ? t.cols / 2 : t.cols) * nsplit;
-  const int stages = ring_kslice(k, nsplit) / 64;
+  const int stages = ring_kslice(k, nsplit, pair) / (pair / 2);
   const long full = tiles / (t.per_cu * cus), rest = tiles % (t.per_cu * cus);
   float busy = (float)full * (stages * t.stage + t.tile);
-  if (rest) busy += stages * (rest > cus ? t.stage : t.stage_alone) + t.tile;
-  const float weights = 0.2e-6f * 2.f * (gate ? 2.f : 1.f) * m * (float)k;      // 5 TB/s
-  const float out = 0.2e-6f * (f32_out ? 4.f : 2.f) * nsplit * n * (float)m;
+  if (rest) {
+    const int side = ceil_div(rest, cus);       // of them side by side on a CU
+    busy += stages * (side == 1 ? t.stage_alone : t.stage * side / t.per_cu) + t.tile;
+  }
+  const float weights = 0.2e-6f * in_bytes * (gate ? 2.f : 1.f) * m * (float)k;      // 5 TB/s
+  const float out = 0.2e-6f * out_bytes * nsplit * n * (float)m;
   const float b2 = busy * busy, w2 = weights * weights;
   return 3.3f + sqrtf(sqrtf(b2 * b2 + w2 * w2)) + out;
 }
 
-static int ring_tile(int n, int m, int k, int nsplit, bool gate, bool f32_out, float* us = nullptr) {
+static int ring_tile(bool f32, int n, int m, int k, int nsplit, bool gate, bool f32_out, float* us = nullptr) {
+  const RingTiles all = ring_tiles(f32);
   int best = 0;
   float least = 0.f;
-  for (int i = 0; i < kRingTileCount; ++i) {
-    const float t = ring_time(kRingTiles[i], n, m, k, nsplit, gate, f32_out);
+  for (int i = 0; i < all.count; ++i) {
+    const float t = ring_time(all.tile[i], all.pair, n, m, k, nsplit, gate, f32 ? 4 : 2, f32_out ? 4 : 2);
     if (i == 0 || t < least) least = t, best = i;
   }
   if (us) *us = least;
   return best;
 }
 
-template <typename TOUT, int MODE, int WR, int WC, int TM, int TN, bool TAIL>
+template <typename T, typename TOUT, int MODE, int WR, int WC, int TM, int TN, bool TAIL>
 static int ring_launch(const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int act,
                        const float* act_params, hipStream_t stream) {
   constexpr int XR = WR * TM * 16, WS = WC * TN * 16, BM = 2 * XR, BN = MODE == RING_GATE ? WS : 2 * WS;
@@ -329,43 +368,54 @@ static int ring_launch(const void* x, const void* w, void* y, int n, int m, int 
   const size_t lds = (size_t)4 * (XR + WS) * 128;
   static int raised = 0;
   if (lds > 64 * 1024 && !raised) {
-    hipError_t e = hipFuncSetAttribute((const void*)gemm_ring_kernel<TOUT, MODE, WR, WC, TM, TN, TAIL>,
+    hipError_t e = hipFuncSetAttribute((const void*)gemm_ring_kernel<T, TOUT, MODE, WR, WC, TM, TN, TAIL>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) KLLM_FAIL((int)e, "gemm ring: cannot raise the LDS limit: %s", hipGetErrorString(e));
     raised = 1;
   }
-  hipLaunchKernelGGL((gemm_ring_kernel<TOUT, MODE, WR, WC, TM, TN, TAIL>), grid, dim3(512), lds, stream, (const bf16_t*)x,
-                     (const bf16_t*)w, (TOUT*)y, n, m, k, tx, ty, ring_kslice(k, nsplit), act, act_params, xcds);
+  hipLaunchKernelGGL((gemm_ring_kernel<T, TOUT, MODE, WR, WC, TM, TN, TAIL>), grid, dim3(512), lds, stream, (const T*)x,
+                     (const T*)w, (TOUT*)y, n, m, k, tx, ty, ring_kslice(k, nsplit, 256 / (int)sizeof(T)), act,
+                     act_params, xcds);
   return 0;
 }
 
-template <typename TOUT, int MODE, bool TAIL>
+template <typename T, typename TOUT, int MODE, bool TAIL>
 static int ring_shape(int tile, const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int act,
                       const float* ap, hipStream_t st) {
-  switch (tile) {
-    case 0: return ring_launch<TOUT, MODE, 2, 4, 4, 2, TAIL>(x, w, y, n, m, k, nsplit, act, ap, st);
-    case 1: return ring_launch<TOUT, MODE, 4, 2, 2, 3, TAIL>(x, w, y, n, m, k, nsplit, act, ap, st);
-    case 2: return ring_launch<TOUT, MODE, 2, 4, 2, 2, TAIL>(x, w, y, n, m, k, nsplit, act, ap, st);
-    default: return ring_launch<TOUT, MODE, 2, 4, 2, 1, TAIL>(x, w, y, n, m, k, nsplit, act, ap, st);
+  if constexpr (sizeof(T) == 4) {
+    return ring_launch<T, TOUT, MODE, 2, 4, 1, 1, TAIL>(x, w, y, n, m, k, nsplit, act, ap, st);
+  } else {
+    switch (tile) {
+      case 0: return ring_launch<T, TOUT, MODE, 2, 4, 4, 2, TAIL>(x, w, y, n, m, k, nsplit, act, ap, st);
+      case 1: return ring_launch<T, TOUT, MODE, 4, 2, 2, 3, TAIL>(x, w, y, n, m, k, nsplit, act, ap, st);
+      case 2: return ring_launch<T, TOUT, MODE, 2, 4, 2, 2, TAIL>(x, w, y, n, m, k, nsplit, act, ap, st);
+      default: return ring_launch<T, TOUT, MODE, 2, 4, 2, 1, TAIL>(x, w, y, n, m, k, nsplit, act, ap, st);
+    }
   }
 }
 
-template <typename TOUT, int MODE>
+template <typename T, typename TOUT, int MODE>
 static int ring_tail(int tile, const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int act,
                      const float* ap, hipStream_t st) {
-  const bool whole = k % 128 == 0 && (long)ring_kslice(k, nsplit) * (nsplit - 1) < k;
-  return !whole ? ring_shape<TOUT, MODE, true>(tile, x, w, y, n, m, k, nsplit, act, ap, st)
-                : ring_shape<TOUT, MODE, false>(tile, x, w, y, n, m, k, nsplit, act, ap, st);
+  constexpr int PAIR = 256 / sizeof(T);
+  const bool whole = k % PAIR == 0 && (long)ring_kslice(k, nsplit, PAIR) * (nsplit - 1) < k;
+  return whole ? ring_shape<T, TOUT, MODE, false>(tile, x, w, y, n, m, k, nsplit, act, ap, st)
+               : ring_shape<T, TOUT, MODE, true>(tile, x, w, y, n, m, k, nsplit, act, ap, st);
 }
 
-int gemm_ring(const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int mode, bool f32_out, int act,
-              const float* act_params, hipStream_t stream) {
+int gemm_ring(const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int mode, bool f32, bool f32_out,
+              int act, const float* act_params, hipStream_t stream) {
   KLLM_REQUIRE(k < kRingMaxK, "gemm ring: K=%d", k);
-  const int tile = ring_tile(n, m, k, nsplit, mode == RING_GATE, f32_out);
-  if (mode == RING_GATE) return ring_tail<bf16_t, RING_GATE>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
-  if (mode == RING_UNARY) return ring_tail<bf16_t, RING_UNARY>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
-  if (f32_out) return ring_tail<float, RING_SUMS>(tile, x, w, y, n, m, k, nsplit, act, act_params, stream);
-  return ring_tail<bf16_t, RING_SUMS>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
+  const int tile = ring_tile(f32, n, m, k, nsplit, mode == RING_GATE, f32_out);
+  if (f32) {
+    if (mode == RING_GATE) return ring_tail<float, float, RING_GATE>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
+    if (mode == RING_UNARY) return ring_tail<float, float, RING_UNARY>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
+    return ring_tail<float, float, RING_SUMS>(tile, x, w, y, n, m, k, nsplit, act, act_params, stream);
+  }
+  if (mode == RING_GATE) return ring_tail<bf16_t, bf16_t, RING_GATE>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
+  if (mode == RING_UNARY) return ring_tail<bf16_t, bf16_t, RING_UNARY>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
+  if (f32_out) return ring_tail<bf16_t, float, RING_SUMS>(tile, x, w, y, n, m, k, nsplit, act, act_params, stream);
+  return ring_tail<bf16_t, bf16_t, RING_SUMS>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
 }
 
 }  // namespace kllm
@@ -375,15 +425,16 @@ using namespace kllm;
 // The slices that take the least time together with the kernel that adds them: its reads beyond the
 // 4.5 us that a launch takes whatever it holds (22 MB at 5 TB/s).  Slices of unequal length keep CUs
 // waiting: cuts that leave more than a tenth of K unused are out.
-extern "C" int kllm_gemm_prompt_slices(int n, int m, int k) {
+extern "C" int kllm_gemm_prompt_slices(int n, int m, int k, int dtype) {
   if (n <= 0 || m <= 0 || k <= 0) return 1;
+  const bool f32 = dtype == DT_F32;
   int best = 1;
   float least = 0.f;
   for (int ns : {1, 2, 3, 4, 6, 8}) {
-    const long slice = ring_kslice(k, ns);
+    const long slice = ring_kslice(k, ns, ring_tiles(f32).pair);
     if (ns > 1 && (slice * (ns - 1) >= k || 10 * slice * ns > 11L * k)) continue;
     float us;
-    ring_tile(n, m, k, ns, false, true, &us);
+    ring_tile(f32, n, m, k, ns, false, true, &us);
     us += fmaxf(4.5f, 0.2e-6f * 4.f * ns * n * (float)m);
     if (ns == 1 || us < least) least = us, best = ns;
   }
@@ -391,8 +442,9 @@ extern "C" int kllm_gemm_prompt_slices(int n, int m, int k) {
 }
 
 // Rows and columns of the tile that a product gets, as rows * 1000 + columns (of W's rows, gates included).
-extern "C" int kllm_gemm_prompt_tile(int n, int m, int k, int nsplit, int gate, int f32_out) {
+extern "C" int kllm_gemm_prompt_tile(int n, int m, int k, int nsplit, int gate, int dtype, int out_dtype) {
   if (n <= 0 || m <= 0 || k <= 0 || nsplit <= 0) return -1;
-  const RingTile& t = kRingTiles[ring_tile(n, m, k, nsplit, gate != 0, f32_out != 0)];
+  const bool f32 = dtype == DT_F32;
+  const RingTile& t = ring_tiles(f32).tile[ring_tile(f32, n, m, k, nsplit, gate != 0, out_dtype == DT_F32)];
   return t.rows * 1000 + t.cols;
 }

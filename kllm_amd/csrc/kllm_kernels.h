@@ -94,11 +94,11 @@ int kllm_sum_splits(const float* in, int nsplit, long count, void* out, int out_
 /* Columns of the tiles that a decode batch of n rows (at most 64) gets against w[m][k] on the
  * MFMA kernel: a caller that cuts K into slices counts its workgroups with it. */
 int kllm_gemm_decode_tile_cols(int n, int m, int k);
-/* For products of more than 64 rows in bfloat16: the slices of K that the product and the kernel that adds
+/* For products of more than 64 rows on the MFMA tiles: the slices of K that the product and the kernel that adds
  * them take the least time with, and the tile that a product of given slices gets, as
  * rows * 1000 + columns. */
-int kllm_gemm_prompt_slices(int n, int m, int k);
-int kllm_gemm_prompt_tile(int n, int m, int k, int nsplit, int gate, int f32_out);
+int kllm_gemm_prompt_slices(int n, int m, int k, int dtype);
+int kllm_gemm_prompt_tile(int n, int m, int k, int nsplit, int gate, int dtype, int out_dtype);
 /* y[nsplit][n][m] = x[n][k] . w[m][k]^T, 32-bit accumulation. */
 int kllm_gemm(const void* x, const void* w, void* y, int n, int m, int k, int dtype, int out_dtype,
               int algo, int nsplit, hipStream_t stream);

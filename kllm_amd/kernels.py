@@ -128,8 +128,8 @@ def _declare(lib):
         "kllm_device_cus": [],
         "kllm_device_xcds": [],
         "kllm_gemm_decode_tile_cols": [I, I, I],
-        "kllm_gemm_prompt_slices": [I, I, I],
-        "kllm_gemm_prompt_tile": [I, I, I, I, I, I],
+        "kllm_gemm_prompt_slices": [I, I, I, I],
+        "kllm_gemm_prompt_tile": [I, I, I, I, I, I, I],
         "kllm_gemv_max_rows": [],
         "kllm_gemv_normed_max_rows": [],
         "kllm_gemv_normed_max_parts": [],
@@ -1164,14 +1164,15 @@ def gemm_decode_tile_cols(n, m, k) -> int:
 
 
 @functools.lru_cache(maxsize=4096)
-def gemm_prompt_slices(n, m, k) -> int:
-    """Slices of K for a bfloat16 product of more than 64 rows whose sums another kernel adds."""
-    return int(library().kllm_gemm_prompt_slices(int(n), int(m), int(k)))
+def gemm_prompt_slices(n, m, k, dtype=torch.bfloat16) -> int:
+    """Slices of K for a product of more than 64 rows on the MFMA tiles whose sums another kernel adds."""
+    return int(library().kllm_gemm_prompt_slices(int(n), int(m), int(k), dtype_code(dtype)))
 
 
-def gemm_prompt_tile(n, m, k, nsplit=1, gate=False, f32_out=True):
-    """(rows, columns) of the tile that a bfloat16 product of more than 64 rows gets."""
-    code = int(library().kllm_gemm_prompt_tile(int(n), int(m), int(k), int(nsplit), int(gate), int(f32_out)))
+def gemm_prompt_tile(n, m, k, nsplit=1, gate=False, dtype=torch.bfloat16, out_dtype=torch.float32):
+    """(rows, columns) of the tile that a product of more than 64 rows gets."""
+    code = int(library().kllm_gemm_prompt_tile(int(n), int(m), int(k), int(nsplit), int(gate), dtype_code(dtype),
+                                               dtype_code(out_dtype)))
     return code // 1000, code % 1000
 
 

@@ -73,14 +73,12 @@ def _mfma_split(m, k):
 
 
 def _mfma_f32_split(n, m, k):
-    """Slices of K for the float32 MFMA kernel.  With 32-bit operands a wave's
-    own chain of products bounds the time (64 cycles for 32 x 32 x 2), not the
-    loads, so a product should give every SIMD a wave or two: up to 16 slices
-    of at least 128 of K."""
-    if n <= 64:
-        waves = -(-m // 128) * 2                      # tiles of 64 rows, two waves
-    else:
-        waves = -(-n // 128) * -(-m // 128) * 4
+    """Slices of K for the float32 MFMA kernel.  Up to 64 rows (tiles of 64 rows, two waves) a wave's
+    own chain of products bounds the time (64 cycles for 32 x 32 x 2), not the loads, so a product
+    should give every SIMD a wave or two: up to 16 slices of at least 128 of K."""
+    if n > 64:
+        return K.gemm_prompt_slices(n, m, k, torch.float32)
+    waves = -(-m // 128) * 2
     nsplit = max(1, min(16, k // 128, -(-4 * K.device_cus() // waves)))
     while nsplit > 1 and (-(-(-(-k // nsplit)) // 32) * 32) * (nsplit - 1) >= k:   # no empty slice
         nsplit -= 1

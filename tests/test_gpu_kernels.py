@@ -432,7 +432,7 @@ def test_prompt_products_on_every_tile(n, m, k, nsplit, gate, tile):
     stages and slices, and nothing written beside the output.  A sum of k products of unit normals in
     32 bits is off by less than k^1/2 2^-24 times a few; the bound leaves a factor of eight."""
     k_ = K()
-    assert k_.gemm_prompt_tile(n, m, k, nsplit, gate, not gate) == tile
+    assert k_.gemm_prompt_tile(n, m, k, nsplit, gate, torch.bfloat16, torch.bfloat16 if gate else torch.float32) == tile
     rows = 2 * m if gate else m
     x = rnd(n, k, seed=1, dtype=torch.bfloat16)
     w = rnd(rows, k, seed=2, dtype=torch.bfloat16, scale=k ** -0.5 if gate else 1.0)
@@ -448,6 +448,30 @@ def test_prompt_products_on_every_tile(n, m, k, nsplit, gate, tile):
         y = guard[:n * m * nsplit].view(nsplit, n, m)
         y.fill_(float("nan"))
         k_.gemm(x, w, y, k_.GEMM_MFMA_BF16, nsplit)
+        assert (y.double().sum(0) - want).abs().max() < 1e-5 * max(k, 64) ** 0.5 * 8
+    assert bool((guard[n * m * nsplit:] == 7.0).all())
+
+
+@pytest.mark.parametrize("n,m,k,nsplit,gate,tile", [
+    (65, 515, 4, 1, False, (64, 128)), (65, 130, 32, 1, True, (64, 128)), (127, 257, 36, 1, False, (64, 128)),
+    (129, 64, 64, 1, True, (64, 128)), (193, 131, 96, 3, False, (64, 128)), (100, 96, 320, 4, False, (64, 128)),
+    (257, 515, 1028, 3, False, (64, 128)), (511, 4099, 260, 1, False, (64, 128)),
+])
+def test_float32_prompt_products_on_every_tile(n, m, k, nsplit, gate, tile):
+    """The same tiles with 32-bit operands; the bound as above, for the gate in 32 bits too."""
+    k_, f32 = K(), torch.float32
+    assert k_.gemm_prompt_tile(n, m, k, nsplit, gate, f32, f32) == tile
+    x, w = rnd(n, k, seed=1), rnd(2 * m if gate else m, k, seed=2, scale=k ** -0.5 if gate else 1.0)
+    want = _gpu_reference(x, w)
+    guard = torch.full((n * m * nsplit + 64,), 7.0, device=DEV)
+    y = guard[:n * m * nsplit].view(nsplit, n, m)
+    y.fill_(float("nan"))
+    if gate:
+        k_.gemm_swiglu(x, w, y[0])
+        want = P.silu(want[:, :m]) * want[:, m:]
+        assert (y[0].double() - want).abs().max() < 1e-5 * want.abs().max()
+    else:
+        k_.gemm(x, w, y, k_.GEMM_MFMA_F32, nsplit)
         assert (y.double().sum(0) - want).abs().max() < 1e-5 * max(k, 64) ** 0.5 * 8
     assert bool((guard[n * m * nsplit:] == 7.0).all())
 
