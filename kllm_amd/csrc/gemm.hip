@@ -5,9 +5,8 @@
 //   plain   one thread per output; any size; the yardstick the others are
 //           tested against
 //   tiled   true 32-bit FMA tiles through LDS, for the float32 engine
-//   mfma    MFMA tiles through LDS: up to 64 rows of X here (decode batches; bfloat16 on 32x32x16,
-//           float32 on 32x32x2: 32-bit operands, products and sums, no reduced precision), more rows
-//           in gemm_ring.hip
+//   mfma    MFMA tiles through LDS (gemm_ring.hip), both types; float32 with 32-bit operands, products
+//           and sums: no reduced precision
 //   skinny  bfloat16 MFMA 16x16x32, weights streamed straight from memory,
 //           for up to 64 rows of X (decode batches); K may be split
 //   gemv    one wave per weight row, up to 8 rows of X; K may be split
@@ -109,289 +108,6 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const float* __rest
       if (c < m) Y[r * m + c] = from_f32<TOUT>(acc[i][j]);
     }
   }
-}
-
-// ------------------------------------------------------------------ MFMA tiles
-// Workgroup tile 64 (rows of X) x 64 or 128 (rows of W), 128 bytes of K per stage
-// (64 bfloat16 or 32 float32), two or three LDS stages.  Two waves, each one or
-// two by two MFMA tiles of 32 x 32.
-// MFMA 32x32x16 (bfloat16): lane l holds A[l%32][8*(l/32)..+7], B[l%32][...]
-// likewise, and D[8*(i/4) + 4*(l/32) + i%4][l%32] in accumulator register i.
-// MFMA 32x32x2 (float32): lane l holds A[l%32][l/32] and B[l%32][l/32], D as
-// above.  Which element of K a lane's operand stands for is free as long as A
-// and B agree, so a lane reads the same 16 bytes as in bfloat16 -- four
-// consecutive floats, lanes 0..31 the first four of eight and lanes 32..63 the
-// second four -- and issues four MFMAs, one per float: the tile loads, the LDS
-// layout and the reads are the same code for both types.
-//
-// Operands go from memory to LDS directly (global_load_lds, 16 bytes per
-// lane), one or two stages ahead of the MFMAs, without passing through
-// registers: nothing waits on a register stage and no ds_write is issued.
-// Such a load puts lane l's 16 bytes at LDS base + 16 l, so a wave's
-// instruction fills 8 rows x 128 bytes of an unpadded tile -- whole cache
-// lines of both operands, which measured a third faster than 64-byte rows.
-// Bank conflicts of the 16-byte reads are avoided by a swizzle instead of
-// padding: row r keeps its chunk c (8 elements) in slot c ^ swz(r), which the
-// loading lane arranges by choosing which chunk it fetches.  Rows beyond the
-// matrices are clamped to the last row (their results are never stored) and
-// chunks beyond K come from a page of zeros.
-//
-// Stages: two when the product has more tiles than CUs; three (a deeper queue of
-// loads) when every CU gets at most one tile.
-//
-// DUAL: W is [gate rows; up rows] = [2m, k]; a workgroup takes 64 gate rows and
-// the 64 up rows that belong to them, and writes act(gate) * up for m columns
-// (reference: backend/model.cu:477-483, :1112-1114) -- the gated activation
-// never exists in 32-bit in memory.
-//
-// Workgroups are numbered so that the XCDs (which take workgroups round-robin,
-// each with an L2 of its own; their number is asked of the runtime) each get a
-// contiguous run of tiles that share rows of X.
-constexpr int MBN = 128;
-constexpr int MROW = 128;                     // bytes of a tile row in LDS: one stage of K
-
-__device__ __attribute__((aligned(16))) unsigned char g_zero_chunk[16];   // zero-initialised
-
-template <typename T> struct MfmaOperand;
-template <> struct MfmaOperand<bf16_t> { typedef bf16x8 type; };
-template <> struct MfmaOperand<float> { typedef floatx4 type; };
-
-// One step of 32 bytes of K per row: acc += A . B^T for a 32 x 32 tile.
-__device__ __forceinline__ floatx16 mfma_tile_step(bf16x8 a, bf16x8 b, floatx16 acc) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-}
-__device__ __forceinline__ floatx16 mfma_tile_step(floatx4 a, floatx4 b, floatx16 acc) {
-#pragma unroll
-  for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], b[e], acc, 0, 0, 0);
-  return acc;
-}
-
-// Slot permutation of a row's eight chunks: rows of equal parity among 16 neighbours get
-// different slots, so that the 16-byte reads of 16 lanes spread over all 64 banks.
-__device__ __forceinline__ int mfma_swz(int row) { return (row >> 1) & 7; }
-
-// WR x WC waves, each with WTM x 2 MFMA tiles of 32 x 32: a workgroup's tile is 32 WTM WR rows of X by
-// 64 WC rows of W (64 x 128 and 64 x 64 with two waves).
-// MODE 0: one product; 1 (DUAL): gate and up products with the gate in the epilogue; 2: one product
-// with an activation without a gate in the epilogue.
-template <typename T, typename TOUT, int MODE, int WR, int MSTAGES, int WC = 2, int WTM = 2>
-__global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2))) void gemm_mfma_kernel(const T* __restrict__ X,
-                                                             const T* __restrict__ W,
-                                                             TOUT* __restrict__ Y, int n, int m,
-                                                             int k, int tiles_x, int tiles_y, int kslice, int act,
-                                                             const float* __restrict__ act_params, int xcds) {
-  constexpr bool DUAL = MODE == 1;
-  constexpr int WTN = 2;
-  typedef typename MfmaOperand<T>::type op_t;   // 16 bytes of a row
-  constexpr int EPC = 16 / sizeof(T);           // elements of a 16-byte chunk
-  constexpr int MBK = MROW / sizeof(T);         // elements of K per stage
-  constexpr int BM = 32 * WTM * WR;             // rows of X per workgroup
-  constexpr int BN = 32 * WTN * WC;             // rows of W per workgroup
-  constexpr int NW = WR * WC;                   // waves
-  constexpr int XI = BM / 8 / NW;               // load instructions of X per wave and stage (8 rows each)
-  constexpr int WI = BN / 8 / NW;
-  constexpr int XBYTES = BM * MROW, WBYTES = BN * MROW;
-  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];   // [MSTAGES][X tile | W tile]
-  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-  const int wr = wave / WC, wc = wave % WC;
-  const long total = (long)tiles_x * tiles_y;
-  const long per_xcd = (total + xcds - 1) / xcds;
-  const long id = (long)(blockIdx.x % xcds) * per_xcd + blockIdx.x / xcds;
-  if (id >= total) return;
-  // An XCD's run of tiles walks the shorter side fastest: it then reads only its share
-  // of the larger operand and shares the smaller one.
-  const bool x_major = tiles_x >= tiles_y;
-  const long trow = x_major ? id % tiles_y : id / tiles_x;
-  const long tcol = x_major ? id / tiles_y : id % tiles_x;
-  const long row0 = trow * BM, col0 = tcol * (DUAL ? BN / 2 : BN);
-
-  // Wave w loads rows [8 XI w, 8 XI (w+1)) of the X tile and [8 WI w, 8 WI (w+1)) of the W
-  // tile.  In one instruction lane l serves row l / 8 (of 8), slot l % 8.
-  const T* xsrc[XI];
-  const T* wsrc[WI];
-  int xchunk[XI], wchunk[WI];
-#pragma unroll
-  for (int i = 0; i < XI; ++i) {
-    const int r = 8 * (XI * wave + i) + lane / 8;
-    xchunk[i] = ((lane % 8) ^ mfma_swz(r)) * EPC;
-    xsrc[i] = X + min(row0 + r, (long)n - 1) * k + xchunk[i];
-  }
-#pragma unroll
-  for (int i = 0; i < WI; ++i) {
-    const int r = 8 * (WI * wave + i) + lane / 8;             // DUAL: the first half of the rows gate, the second up
-    wchunk[i] = ((lane % 8) ^ mfma_swz(r)) * EPC;
-    const long col = DUAL ? col0 + r % (BN / 2) : col0 + r;
-    const bool up = DUAL && r >= BN / 2;
-    const long wrow = min(col, (long)m - 1) + (up ? m : 0);
-    wsrc[i] = W + wrow * k + wchunk[i];
-  }
-  // blockIdx.y: a slice of K (kslice a multiple of a stage); its sums go to Y[blockIdx.y]
-  const int kbeg = blockIdx.y * kslice, kend = min(k, kbeg + kslice);
-  Y += (long)blockIdx.y * n * m;
-  auto issue = [&](int kt) {
-    unsigned char* base = lds + (kt % MSTAGES) * (XBYTES + WBYTES);
-    const int kk = kbeg + kt * MBK;
-#pragma unroll
-    for (int i = 0; i < XI; ++i) {
-      const T* src = kk + xchunk[i] < kend ? xsrc[i] + kk : reinterpret_cast<const T*>(g_zero_chunk);
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                       (__attribute__((address_space(3))) void*)(base + 8 * (XI * wave + i) * MROW),
-                                       16, 0, 0);
-    }
-#pragma unroll
-    for (int i = 0; i < WI; ++i) {
-      const T* src = kk + wchunk[i] < kend ? wsrc[i] + kk : reinterpret_cast<const T*>(g_zero_chunk);
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                       (__attribute__((address_space(3))) void*)(base + XBYTES + 8 * (WI * wave + i) * MROW),
-                                       16, 0, 0);
-    }
-  };
-
-  floatx16 acc[WTM][WTN];
-#pragma unroll
-  for (int i = 0; i < WTM; ++i)
-#pragma unroll
-    for (int j = 0; j < WTN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
-  const int ktiles = (kend - kbeg + MBK - 1) / MBK;
-  issue(0);
-  if (MSTAGES > 2 && ktiles > 1) issue(1);
-  for (int kt = 0; kt < ktiles; ++kt) {
-    // This wave's loads of stage kt have landed when at most the newer stage's (XI + WI
-    // instructions, with three stages) are still in flight; after the barrier so have every
-    // wave's, and every wave is done reading the stage that the next loads overwrite.  The
-    // barrier is a bare s_barrier: a fence here would also wait for the newest loads.
-    if (MSTAGES > 2 && kt + 1 < ktiles) __builtin_amdgcn_s_waitcnt(0x0F70 | (XI + WI));   // vmcnt(XI + WI)
-    else __builtin_amdgcn_s_waitcnt(0x0F70);                                             // vmcnt(0)
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (kt + MSTAGES - 1 < ktiles) issue(kt + MSTAGES - 1);
-    const unsigned char* xs = lds + (kt % MSTAGES) * (XBYTES + WBYTES);
-    const unsigned char* ws = xs + XBYTES;
-    // The operands of step ks + 1 are asked for before the MFMAs of step ks are issued, so
-    // that LDS answers while the matrix unit works.
-    op_t a[2][WTM], b[2][WTN];
-    auto read_step = [&](int ks, op_t (&ar)[WTM], op_t (&br)[WTN]) {
-      const int chunk = ks * 2 + lane / 32;
-#pragma unroll
-      for (int i = 0; i < WTM; ++i) {
-        const int r = wr * 32 * WTM + i * 32 + lane % 32;
-        ar[i] = *reinterpret_cast<const op_t*>(xs + r * MROW + (chunk ^ mfma_swz(r)) * 16);
-      }
-#pragma unroll
-      for (int j = 0; j < WTN; ++j) {
-        const int r = (DUAL ? j * (BN / 2) + wc * 32 : wc * 32 * WTN + j * 32) + lane % 32;
-        br[j] = *reinterpret_cast<const op_t*>(ws + r * MROW + (chunk ^ mfma_swz(r)) * 16);
-      }
-    };
-    read_step(0, a[0], b[0]);
-#pragma unroll
-    for (int ks = 0; ks < MROW / 32; ++ks) {
-      if (ks + 1 < MROW / 32) read_step(ks + 1, a[(ks + 1) & 1], b[(ks + 1) & 1]);
-#pragma unroll
-      for (int i = 0; i < WTM; ++i)
-#pragma unroll
-        for (int j = 0; j < WTN; ++j)
-          acc[i][j] = mfma_tile_step(a[ks & 1][i], b[ks & 1][j], acc[i][j]);
-    }
-  }
-
-  if (DUAL) {
-    const long c = col0 + wc * 32 + lane % 32;
-    if (c >= m) return;
-#pragma unroll
-    for (int i = 0; i < WTM; ++i)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const long r = row0 + wr * 32 * WTM + i * 32 + 8 * (e / 4) + 4 * (lane / 32) + e % 4;
-        const float gate = acc[i][0][e], up = acc[i][1][e];
-        if (r < n) Y[r * m + c] = from_f32<TOUT>(gate_act(gate, act) * up);
-      }
-    return;
-  }
-  // One product: the sums as they are, or (MODE 2) through an activation without a gate.
-  float a_pos = 0.f, a_neg = 0.f;
-  if constexpr (MODE == 2) {
-    if (act == ACT_XIELU) {
-      a_pos = softplus_f32(act_params[0]);
-      a_neg = softplus_f32(act_params[1]);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < WTM; ++i)
-#pragma unroll
-    for (int j = 0; j < WTN; ++j) {
-      const long c = col0 + wc * 32 * WTN + j * 32 + lane % 32;
-      if (c >= m) continue;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const long r = row0 + wr * 32 * WTM + i * 32 + 8 * (e / 4) + 4 * (lane / 32) + e % 4;
-        float v = acc[i][j][e];
-        if constexpr (MODE == 2) v = unary_act(v, act, a_pos, a_neg);
-        if (r < n) Y[r * m + c] = from_f32<TOUT>(v);
-      }
-    }
-}
-
-template <typename T, typename TOUT, int MODE, int WR, int MSTAGES, int WC = 2, int WTM = 2>
-static int launch_mfma_tile(const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int act,
-                            hipStream_t stream, const float* act_params = nullptr) {
-  constexpr bool DUAL = MODE == 1;
-  constexpr int MBK = MROW / sizeof(T);
-  constexpr int BM = 32 * WTM * WR, BN = 64 * WC;
-  const int tx = ceil_div(m, DUAL ? BN / 2 : BN), ty = ceil_div(n, BM);
-  const int kslice = ceil_div(ceil_div(k, nsplit), MBK) * MBK;
-  const int xcds = device_xcds();
-  const dim3 grid(ceil_div((long)tx * ty, xcds) * xcds, nsplit);   // padded so that every XCD gets as many
-  const size_t lds = (size_t)MSTAGES * (BM + BN) * MROW;
-  static int raised = 0;
-  if (lds > 64 * 1024 && !raised) {
-    hipError_t e = hipFuncSetAttribute((const void*)gemm_mfma_kernel<T, TOUT, MODE, WR, MSTAGES, WC, WTM>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) KLLM_FAIL((int)e, "gemm mfma: cannot raise the LDS limit: %s", hipGetErrorString(e));
-    raised = 1;
-  }
-  hipLaunchKernelGGL((gemm_mfma_kernel<T, TOUT, MODE, WR, MSTAGES, WC, WTM>), grid, dim3(64 * WR * WC), lds, stream,
-                     (const T*)x, (const T*)w, (TOUT*)y, n, m, k, tx, ty, kslice, act, act_params, xcds);
-  return 0;
-}
-
-constexpr long kNarrowBelow = 40000000;   // weights (elements) below which a decode batch gets tiles of 64 columns
-
-// Products of more than 64 rows run on gemm_ring.hip's tiles; here are decode batches.
-template <typename T, typename TOUT, int MODE>
-static int launch_mfma(const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int act,
-                       hipStream_t stream, const float* act_params = nullptr) {
-  constexpr bool DUAL = MODE == 1;
-  const int cus = device_cus();
-  const int tx = ceil_div(m, DUAL ? MBN / 2 : MBN);
-  // A decode batch: tiles of 64 rows, half the products and half the loads of X of 128.  In
-  // bfloat16 a product of few tiles keeps three stages of loads in flight (one workgroup a CU).
-  if (n <= 64) {
-    // ... and against weights below 40 M elements tiles of 64 columns (two waves of 32 x 64):
-    // twice the workgroups, which is what a product of few column tiles lacks (64 rows, 2,048
-    // x 5,632 in 8 slices: 9.8 us against 13.2 us; 11,264 x 2,048 in 4: 14.3 against 16.2; 4,096
-    // x 14,336 in 8: 32.9 against 28.7).  In float32, where a wave's chain of products bounds
-    // the time, the same halves the chain (a decode step of 64 tokens at 1.1B sizes: 4.75 ->
-    // 4.30 ms).
-    if constexpr (!DUAL) {
-      if ((long)m * k < kNarrowBelow) {
-        if ((long)ceil_div(m, 64) * nsplit <= cus)
-          return launch_mfma_tile<T, TOUT, MODE, 2, 3, 1, 1>(x, w, y, n, m, k, nsplit, act, stream, act_params);
-        return launch_mfma_tile<T, TOUT, MODE, 2, 2, 1, 1>(x, w, y, n, m, k, nsplit, act, stream, act_params);
-      }
-    }
-    if (sizeof(T) == 2 && (long)tx * nsplit <= cus)
-      return launch_mfma_tile<T, TOUT, MODE, 1, 3>(x, w, y, n, m, k, nsplit, act, stream, act_params);
-    return launch_mfma_tile<T, TOUT, MODE, 1, 2>(x, w, y, n, m, k, nsplit, act, stream, act_params);
-  }
-  if (k < kRingMaxK)
-    return gemm_ring(x, w, y, n, m, k, nsplit, DUAL ? RING_GATE : MODE == 2 ? RING_UNARY : RING_SUMS, sizeof(T) == 4,
-                     sizeof(TOUT) == 4, act, act_params, stream);
-  return launch_mfma_tile<T, TOUT, MODE, 1, 2>(x, w, y, n, m, k, nsplit, act, stream, act_params);
 }
 
 // ------------------------------------------------------------------ bf16 MFMA skinny
@@ -648,10 +364,6 @@ static int launch_skinny(const bf16_t* x, const bf16_t* w, float* y, int n, int 
   return 0;
 }
 
-extern "C" int kllm_gemm_decode_tile_cols(int n, int m, int k) {
-  return n <= 64 && (long)m * k < kNarrowBelow ? 64 : MBN;
-}
-
 extern "C" int kllm_gemm(const void* x, const void* w, void* y, int n, int m, int k, int dtype,
                          int out_dtype, int algo, int nsplit, hipStream_t stream) {
   KLLM_REQUIRE(x && w && y, "gemm: null pointer");
@@ -692,16 +404,14 @@ extern "C" int kllm_gemm(const void* x, const void* w, void* y, int n, int m, in
 
   if (algo == KLLM_GEMM_MFMA_BF16 || algo == KLLM_GEMM_MFMA_F32) {
     const bool f32 = algo == KLLM_GEMM_MFMA_F32;
-    const int stage = f32 ? MROW / 4 : MROW / 2, chunk = f32 ? 4 : 8;   // elements of K per stage, per 16 bytes
+    const int stage = f32 ? 32 : 64, chunk = f32 ? 4 : 8;   // elements of K per stage, per 16 bytes
     KLLM_REQUIRE(dtype == (f32 ? DT_F32 : DT_BF16), "gemm mfma: algorithm %d does not take dtype %d", algo, dtype);
     KLLM_REQUIRE(nsplit == 1 || out_dtype == DT_F32, "gemm mfma: K is split only for float32 partial sums");
     KLLM_REQUIRE(nsplit <= 16 && (long)(ceil_div(ceil_div(k, nsplit), stage) * stage) * (nsplit - 1) < k,
                  "gemm mfma: nsplit %d leaves an empty slice of K=%d", nsplit, k);
     KLLM_REQUIRE(k % chunk == 0 && aligned16(x) && aligned16(w),
                  "gemm mfma: K=%d must be a multiple of %d and the operands 16-byte aligned", k, chunk);
-    int rc = f32 ? launch_mfma<float, float, false>(x, w, y, n, m, k, nsplit, -1, stream)
-             : out_dtype == DT_F32 ? launch_mfma<bf16_t, float, false>(x, w, y, n, m, k, nsplit, -1, stream)
-                                   : launch_mfma<bf16_t, bf16_t, false>(x, w, y, n, m, k, 1, -1, stream);
+    int rc = gemm_ring(x, w, y, n, m, k, out_dtype == DT_F32 ? nsplit : 1, RING_SUMS, f32, out_dtype == DT_F32, -1, nullptr, stream);
     if (rc) return rc;
     KLLM_CHECK_LAUNCH("gemm mfma");
     return 0;
@@ -798,9 +508,7 @@ extern "C" int kllm_gemm_swiglu(const void* x, const void* w_gate_up, void* h, i
   KLLM_REQUIRE(k % chunk == 0 && aligned16(x) && aligned16(w_gate_up),
                "gemm_swiglu: K=%d must be a multiple of %d and the operands 16-byte aligned", k, chunk);
   KLLM_REQUIRE((long)n * f < (1L << 31), "gemm_swiglu: sizes overflow");
-  if (int rc = dtype == DT_F32 ? launch_mfma<float, float, true>(x, w_gate_up, h, n, f, k, 1, act, stream)
-                               : launch_mfma<bf16_t, bf16_t, true>(x, w_gate_up, h, n, f, k, 1, act, stream))
-    return rc;
+  if (int rc = gemm_ring(x, w_gate_up, h, n, f, k, 1, RING_GATE, dtype == DT_F32, dtype == DT_F32, act, nullptr, stream)) return rc;
   KLLM_CHECK_LAUNCH("gemm_swiglu");
   return 0;
 }
@@ -817,9 +525,7 @@ extern "C" int kllm_gemm_act(const void* x, const void* w, void* h, int n, int m
   KLLM_REQUIRE(k % chunk == 0 && aligned16(x) && aligned16(w),
                "gemm_act: K=%d must be a multiple of %d and the operands 16-byte aligned", k, chunk);
   KLLM_REQUIRE((long)n * m < (1L << 31), "gemm_act: sizes overflow");
-  if (int rc = dtype == DT_F32 ? launch_mfma<float, float, 2>(x, w, h, n, m, k, 1, act, stream, act_params)
-                               : launch_mfma<bf16_t, bf16_t, 2>(x, w, h, n, m, k, 1, act, stream, act_params))
-    return rc;
+  if (int rc = gemm_ring(x, w, h, n, m, k, 1, RING_UNARY, dtype == DT_F32, dtype == DT_F32, act, act_params, stream)) return rc;
   KLLM_CHECK_LAUNCH("gemm_act");
   return 0;
 }

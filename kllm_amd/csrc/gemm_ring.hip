@@ -1,8 +1,8 @@
-// Matrix products of prompt size: Y[n, m] = X[n, k] . W[m, k]^T for more than 64 rows of X, bfloat16, or
-// float32 in true 32-bit.
+// Matrix products on MFMA tiles: Y[n, m] = X[n, k] . W[m, k]^T, bfloat16, or float32 in true 32-bit; prompts,
+// and decode batches of more than 16 rows.
 //
-// One workgroup of eight waves a CU and output tile (256 x 256, 256 x 192 or 128 x 256; two
-// workgroups a CU for 128 x 128 and smaller).  A tile's rows of X and of W come in two halves each; a stage
+// One workgroup of eight waves a CU and output tile (256 x 256, 256 x 192 or 128 x 256; two or three
+// workgroups a CU for smaller ones).  A tile's rows of X and of W come in two halves each; a stage
 // is whole cache lines of K (128 bytes: 64 bfloat16 or 32 float32), so a stage is four sub-tiles, X0 X1 W0 W1, and LDS holds
 // two stages of them: a ring of eight buffers.
 //
@@ -74,6 +74,9 @@ template <typename T> struct RingOperand;                // 16 bytes of a row
 template <> struct RingOperand<bf16_t> { typedef bf16x8 type; };
 template <> struct RingOperand<float> { typedef floatx4 type; };
 
+template <bool WIDE> struct RingOffset { typedef unsigned type; };
+template <> struct RingOffset<true> { typedef unsigned long type; };
+
 __device__ __forceinline__ floatx4 ring_mma(bf16x8 a, bf16x8 b, floatx4 acc) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
 }
@@ -83,15 +86,20 @@ __device__ __forceinline__ floatx4 ring_mma(floatx4 a, floatx4 b, floatx4 acc) {
   return acc;
 }
 
-// WR x WC = 8 waves; a wave's part of a sub-tile of X is TM tiles of 16 rows, of W TN.  TAIL: some slice
-// is no multiple of 128, what lies behind its end is read as zeros.
-template <typename T, typename TOUT, int MODE, int WR, int WC, int TM, int TN, bool TAIL>
+// WR x WC = 8 waves; a wave's part of a sub-tile of X is TM tiles of 16 rows, of W TN.  KIND of K: RING_WHOLE;
+// RING_TAIL: some slice is no multiple of two stages, what lies behind its end is read as zeros; RING_LONG: also
+// so long that a lane's offset from its tile's first row takes 64 bits.
+enum : int { RING_WHOLE = 0, RING_TAIL = 1, RING_LONG = 2 };
+constexpr int kRingLongK = 1 << 23;        // 255 rows of bfloat16, 127 of float32: below 2^32 bytes
+
+template <typename T, typename TOUT, int MODE, int WR, int WC, int TM, int TN, int KIND>
 __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const T* __restrict__ X, const T* __restrict__ W,
                                                            TOUT* __restrict__ Y, int n, int m, int k, int tiles_x,
                                                            int tiles_y, int kslice, int act,
                                                            const float* __restrict__ act_params, int xcds) {
-  constexpr bool GATE = MODE == RING_GATE;
+  constexpr bool GATE = MODE == RING_GATE, TAIL = KIND != RING_WHOLE;
   typedef typename RingOperand<T>::type op_t;
+  typedef typename RingOffset<KIND == RING_LONG>::type off_t;
   constexpr int EPC = 16 / sizeof(T), STAGE = 8 * EPC;     // elements of a chunk of 16 bytes, of a stage
   constexpr int XR = WR * TM * 16, WS = WC * TN * 16;      // rows of a sub-tile of X, of W
   constexpr int BM = 2 * XR, BN = GATE ? WS : 2 * WS;      // rows and columns of the output tile
@@ -125,7 +133,7 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const T* __restrict__
   // exist are clamped to the last (their results are never stored).
   constexpr int XPW = XR / 8, WPW = WS / 8;                // rows per wave
   constexpr int XL = (XPW + 7) / 8, WL = (WPW + 7) / 8;    // load instructions per wave
-  unsigned xoff[2][XL], woff[2][WL];                        // bytes from the tile's first row, at K = kbeg
+  off_t xoff[2][XL], woff[2][WL];                        // bytes from the tile's first row, at K = kbeg
   int xchunk[XL], wchunk[WL];
 #pragma unroll
   for (int i = 0; i < XL; ++i) {
@@ -133,7 +141,7 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const T* __restrict__
     xchunk[i] = (lane % 8) ^ ((r >> 1) & 7);
 #pragma unroll
     for (int h = 0; h < 2; ++h)
-      xoff[h][i] = (unsigned)(min(row0 + h * XR + r, n - 1) - row0) * (unsigned)k * (unsigned)sizeof(T) + xchunk[i] * 16u;
+      xoff[h][i] = (off_t)(min(row0 + h * XR + r, n - 1) - row0) * (off_t)k * (off_t)sizeof(T) + xchunk[i] * 16u;
   }
 #pragma unroll
   for (int i = 0; i < WL; ++i) {
@@ -141,12 +149,12 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const T* __restrict__
     wchunk[i] = (lane % 8) ^ ((r >> 1) & 7);
 #pragma unroll
     for (int h = 0; h < 2; ++h)       // GATE: the first half of a tile's rows of W are gates, the second their up rows
-      woff[h][i] = (unsigned)(min(col0 + (GATE ? 0 : h * WS) + r, m - 1) - col0) * (unsigned)k * (unsigned)sizeof(T) + wchunk[i] * 16u;
+      woff[h][i] = (off_t)(min(col0 + (GATE ? 0 : h * WS) + r, m - 1) - col0) * (off_t)k * (off_t)sizeof(T) + wchunk[i] * 16u;
   }
   const T* const xbase = X + (long)row0 * k + kbeg;
   const T* const wbase[2] = {W + (long)col0 * k + kbeg, W + ((long)col0 + (GATE ? m : 0)) * k + kbeg};
 
-  auto load = [&](const char* src, unsigned off, int chunk, int left, unsigned char* dst) {
+  auto load = [&](const char* src, off_t off, int chunk, int left, unsigned char* dst) {
     const char* at = src + off;
     if (TAIL) at = chunk * EPC < left ? at : reinterpret_cast<const char*>(g_ring_zeros);
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)at,
@@ -300,6 +308,15 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const T* __restrict__
 
 // ------------------------------------------------------------------ which tile, how many slices of K
 //
+// Up to 64 rows of X (decode batches), where the weights' way from memory bounds the time, tiles of 64 rows:
+// 64 x 128, three workgroups a CU, or in bfloat16 64 x 256, two a CU, where those are at most one a CU and
+// the narrow ones more, with a slice of 512 of K at least (64 rows, in us, narrow / wide: 11,264 x 2,048 in 4
+// slices 15.2 / 14.1; 12,288 x 4,096 in 4 24.5 / 22.3; in 8 24.6 / 27.8; 4,096 x 14,336 in 8 23.9 / 31.3;
+// 2,560 x 2,048 in 16 8.1 / 9.3).  The two- and three-stage tiles of 64 x 64 and 64 x 128 before, at 64 rows: 11,264
+// x 2,048 15.1, with the gate 30.3 (now 19.6); 12,288 x 4,096 28.4; 4,096 x 14,336 in 8 29.3; 28,672 x 4,096
+// with the gate 61.2 (52.5); 2,048 x 2,048 in 8 6.4 (6.2); float32: 2,048 x 5,632 in 16 29.2 (24.6 in 11).
+//
+// More rows:
 // A product's time in us is put together from what a tile costs a CU: rounds of the chip times (stages
 // x a stage's time + what a tile costs beside its stages), against the time its weights need from
 // memory, plus its output and a launch.  The constants for bfloat16 are fitted to a sweep of 13 numbers of rows
@@ -319,6 +336,7 @@ struct RingTile {
 static const RingTile kRingTilesBf16[] = {
     {256, 256, 1, 1.04f, 3.0f, 1.04f}, {256, 192, 1, 0.835f, 2.6f, 0.835f}, {128, 256, 1, 0.68f, 1.4f, 0.68f},
     {128, 128, 2, 0.88f, 0.0f, 0.60f}};
+constexpr int kRingNarrow = 4, kRingWide = 5;      // of up to 64 rows: 64 x 128, 64 x 256
 static const RingTile kRingTilesF32[] = {{64, 128, 3, 2.94f, 1.0f, 1.30f}};
 struct RingTiles {
   const RingTile* tile;
@@ -349,6 +367,11 @@ static float ring_time(const RingTile& t, int pair, int n, int m, int k, int nsp
 
 static int ring_tile(bool f32, int n, int m, int k, int nsplit, bool gate, bool f32_out, float* us = nullptr) {
   const RingTiles all = ring_tiles(f32);
+  if (k >= kRingLongK) return f32 ? 0 : kRingNarrow;
+  if (!f32 && n <= 64) {
+    const long cus = device_cus(), narrow = (long)ceil_div(m, gate ? 64 : 128) * nsplit, wide = (long)ceil_div(m, gate ? 128 : 256) * nsplit;
+    return narrow > cus && wide <= cus && ring_kslice(k, nsplit, all.pair) >= 512 ? kRingWide : kRingNarrow;
+  }
   int best = 0;
   float least = 0.f;
   for (int i = 0; i < all.count; ++i) {
@@ -359,7 +382,7 @@ static int ring_tile(bool f32, int n, int m, int k, int nsplit, bool gate, bool 
   return best;
 }
 
-template <typename T, typename TOUT, int MODE, int WR, int WC, int TM, int TN, bool TAIL>
+template <typename T, typename TOUT, int MODE, int WR, int WC, int TM, int TN, int KIND>
 static int ring_launch(const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int act,
                        const float* act_params, hipStream_t stream) {
   constexpr int XR = WR * TM * 16, WS = WC * TN * 16, BM = 2 * XR, BN = MODE == RING_GATE ? WS : 2 * WS;
@@ -368,54 +391,54 @@ static int ring_launch(const void* x, const void* w, void* y, int n, int m, int 
   const size_t lds = (size_t)4 * (XR + WS) * 128;
   static int raised = 0;
   if (lds > 64 * 1024 && !raised) {
-    hipError_t e = hipFuncSetAttribute((const void*)gemm_ring_kernel<T, TOUT, MODE, WR, WC, TM, TN, TAIL>,
+    hipError_t e = hipFuncSetAttribute((const void*)gemm_ring_kernel<T, TOUT, MODE, WR, WC, TM, TN, KIND>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) KLLM_FAIL((int)e, "gemm ring: cannot raise the LDS limit: %s", hipGetErrorString(e));
     raised = 1;
   }
-  hipLaunchKernelGGL((gemm_ring_kernel<T, TOUT, MODE, WR, WC, TM, TN, TAIL>), grid, dim3(512), lds, stream, (const T*)x,
+  hipLaunchKernelGGL((gemm_ring_kernel<T, TOUT, MODE, WR, WC, TM, TN, KIND>), grid, dim3(512), lds, stream, (const T*)x,
                      (const T*)w, (TOUT*)y, n, m, k, tx, ty, ring_kslice(k, nsplit, 256 / (int)sizeof(T)), act,
                      act_params, xcds);
   return 0;
 }
 
-template <typename T, typename TOUT, int MODE, bool TAIL>
+template <typename T, typename TOUT, int MODE, int KIND>
 static int ring_shape(int tile, const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int act,
                       const float* ap, hipStream_t st) {
-  if constexpr (sizeof(T) == 4) {
-    return ring_launch<T, TOUT, MODE, 2, 4, 1, 1, TAIL>(x, w, y, n, m, k, nsplit, act, ap, st);
-  } else {
+  if constexpr (sizeof(T) == 2 && KIND != RING_LONG) {
     switch (tile) {
-      case 0: return ring_launch<T, TOUT, MODE, 2, 4, 4, 2, TAIL>(x, w, y, n, m, k, nsplit, act, ap, st);
-      case 1: return ring_launch<T, TOUT, MODE, 4, 2, 2, 3, TAIL>(x, w, y, n, m, k, nsplit, act, ap, st);
-      case 2: return ring_launch<T, TOUT, MODE, 2, 4, 2, 2, TAIL>(x, w, y, n, m, k, nsplit, act, ap, st);
-      default: return ring_launch<T, TOUT, MODE, 2, 4, 2, 1, TAIL>(x, w, y, n, m, k, nsplit, act, ap, st);
+      case 0: return ring_launch<T, TOUT, MODE, 2, 4, 4, 2, KIND>(x, w, y, n, m, k, nsplit, act, ap, st);
+      case 1: return ring_launch<T, TOUT, MODE, 4, 2, 2, 3, KIND>(x, w, y, n, m, k, nsplit, act, ap, st);
+      case 2: return ring_launch<T, TOUT, MODE, 2, 4, 2, 2, KIND>(x, w, y, n, m, k, nsplit, act, ap, st);
+      case 3: return ring_launch<T, TOUT, MODE, 2, 4, 2, 1, KIND>(x, w, y, n, m, k, nsplit, act, ap, st);
+      case kRingWide: return ring_launch<T, TOUT, MODE, 2, 4, 1, 2, KIND>(x, w, y, n, m, k, nsplit, act, ap, st);
     }
   }
+  return ring_launch<T, TOUT, MODE, 2, 4, 1, 1, KIND>(x, w, y, n, m, k, nsplit, act, ap, st);
 }
 
 template <typename T, typename TOUT, int MODE>
-static int ring_tail(int tile, const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int act,
+static int ring_kind(int tile, const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int act,
                      const float* ap, hipStream_t st) {
   constexpr int PAIR = 256 / sizeof(T);
+  if (k >= kRingLongK) return ring_shape<T, TOUT, MODE, RING_LONG>(tile, x, w, y, n, m, k, nsplit, act, ap, st);
   const bool whole = k % PAIR == 0 && (long)ring_kslice(k, nsplit, PAIR) * (nsplit - 1) < k;
-  return whole ? ring_shape<T, TOUT, MODE, false>(tile, x, w, y, n, m, k, nsplit, act, ap, st)
-               : ring_shape<T, TOUT, MODE, true>(tile, x, w, y, n, m, k, nsplit, act, ap, st);
+  return whole ? ring_shape<T, TOUT, MODE, RING_WHOLE>(tile, x, w, y, n, m, k, nsplit, act, ap, st)
+               : ring_shape<T, TOUT, MODE, RING_TAIL>(tile, x, w, y, n, m, k, nsplit, act, ap, st);
 }
 
 int gemm_ring(const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int mode, bool f32, bool f32_out,
               int act, const float* act_params, hipStream_t stream) {
-  KLLM_REQUIRE(k < kRingMaxK, "gemm ring: K=%d", k);
   const int tile = ring_tile(f32, n, m, k, nsplit, mode == RING_GATE, f32_out);
   if (f32) {
-    if (mode == RING_GATE) return ring_tail<float, float, RING_GATE>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
-    if (mode == RING_UNARY) return ring_tail<float, float, RING_UNARY>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
-    return ring_tail<float, float, RING_SUMS>(tile, x, w, y, n, m, k, nsplit, act, act_params, stream);
+    if (mode == RING_GATE) return ring_kind<float, float, RING_GATE>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
+    if (mode == RING_UNARY) return ring_kind<float, float, RING_UNARY>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
+    return ring_kind<float, float, RING_SUMS>(tile, x, w, y, n, m, k, nsplit, act, act_params, stream);
   }
-  if (mode == RING_GATE) return ring_tail<bf16_t, bf16_t, RING_GATE>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
-  if (mode == RING_UNARY) return ring_tail<bf16_t, bf16_t, RING_UNARY>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
-  if (f32_out) return ring_tail<bf16_t, float, RING_SUMS>(tile, x, w, y, n, m, k, nsplit, act, act_params, stream);
-  return ring_tail<bf16_t, bf16_t, RING_SUMS>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
+  if (mode == RING_GATE) return ring_kind<bf16_t, bf16_t, RING_GATE>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
+  if (mode == RING_UNARY) return ring_kind<bf16_t, bf16_t, RING_UNARY>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
+  if (f32_out) return ring_kind<bf16_t, float, RING_SUMS>(tile, x, w, y, n, m, k, nsplit, act, act_params, stream);
+  return ring_kind<bf16_t, bf16_t, RING_SUMS>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
 }
 
 }  // namespace kllm
@@ -445,6 +468,8 @@ extern "C" int kllm_gemm_prompt_slices(int n, int m, int k, int dtype) {
 extern "C" int kllm_gemm_prompt_tile(int n, int m, int k, int nsplit, int gate, int dtype, int out_dtype) {
   if (n <= 0 || m <= 0 || k <= 0 || nsplit <= 0) return -1;
   const bool f32 = dtype == DT_F32;
-  const RingTile& t = ring_tiles(f32).tile[ring_tile(f32, n, m, k, nsplit, gate != 0, out_dtype == DT_F32)];
+  const int tile = ring_tile(f32, n, m, k, nsplit, gate != 0, out_dtype == DT_F32);
+  if (!f32 && tile >= kRingNarrow) return 64000 + (tile == kRingWide ? 256 : 128);
+  const RingTile& t = ring_tiles(f32).tile[tile];
   return t.rows * 1000 + t.cols;
 }

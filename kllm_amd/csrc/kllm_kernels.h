@@ -91,12 +91,8 @@ int kllm_silu_mul(const void* gu, int in_dtype, int nsplit, long split_stride, v
 int kllm_sum_splits(const float* in, int nsplit, long count, void* out, int out_dtype,
                     hipStream_t stream);
 
-/* Columns of the tiles that a decode batch of n rows (at most 64) gets against w[m][k] on the
- * MFMA kernel: a caller that cuts K into slices counts its workgroups with it. */
-int kllm_gemm_decode_tile_cols(int n, int m, int k);
-/* For products of more than 64 rows on the MFMA tiles: the slices of K that the product and the kernel that adds
- * them take the least time with, and the tile that a product of given slices gets, as
- * rows * 1000 + columns. */
+/* Products on the MFMA tiles: for more than 64 rows the slices of K that the product and the kernel that adds
+ * them take the least time with; the tile that a product of given slices gets, as rows * 1000 + columns. */
 int kllm_gemm_prompt_slices(int n, int m, int k, int dtype);
 int kllm_gemm_prompt_tile(int n, int m, int k, int nsplit, int gate, int dtype, int out_dtype);
 /* y[nsplit][n][m] = x[n][k] . w[m][k]^T, 32-bit accumulation. */

@@ -127,7 +127,6 @@ def _declare(lib):
         "kllm_attn_decode_slices": [I, I, I, I, I, I],
         "kllm_device_cus": [],
         "kllm_device_xcds": [],
-        "kllm_gemm_decode_tile_cols": [I, I, I],
         "kllm_gemm_prompt_slices": [I, I, I, I],
         "kllm_gemm_prompt_tile": [I, I, I, I, I, I, I],
         "kllm_gemv_max_rows": [],
@@ -1158,19 +1157,13 @@ def attn_f32_fits(head_dim, page_size) -> bool:
 
 
 @functools.lru_cache(maxsize=4096)
-def gemm_decode_tile_cols(n, m, k) -> int:
-    """Columns of the tiles that the MFMA kernel gives a decode batch of these sizes."""
-    return int(library().kllm_gemm_decode_tile_cols(int(n), int(m), int(k)))
-
-
-@functools.lru_cache(maxsize=4096)
 def gemm_prompt_slices(n, m, k, dtype=torch.bfloat16) -> int:
     """Slices of K for a product of more than 64 rows on the MFMA tiles whose sums another kernel adds."""
     return int(library().kllm_gemm_prompt_slices(int(n), int(m), int(k), dtype_code(dtype)))
 
 
 def gemm_prompt_tile(n, m, k, nsplit=1, gate=False, dtype=torch.bfloat16, out_dtype=torch.float32):
-    """(rows, columns) of the tile that a product of more than 64 rows gets."""
+    """(rows, columns) of the tile that a product on the MFMA tiles gets."""
     code = int(library().kllm_gemm_prompt_tile(int(n), int(m), int(k), int(nsplit), int(gate), dtype_code(dtype),
                                                dtype_code(out_dtype)))
     return code // 1000, code % 1000

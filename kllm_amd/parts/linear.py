@@ -57,25 +57,10 @@ def _skinny_split(n, m, k):
     return int(nsplit)
 
 
-def _mfma_split(m, k):
-    """Slices of K for the MFMA kernel's tiles of 64 rows and 128 columns (decode batches against
-    the largest weights).  With fewer tiles than the chip has room for workgroups the product is
-    bound by how many of them stream the weights: up to 8 slices of at least 512 of K bring it to
-    about 512 workgroups, 1,024 where K is deep and the tiles alone leave CUs idle."""
-    tiles = -(-m // 128)
-    nsplit = 1
-    reach = (4 if k >= 8192 and tiles <= K.device_cus() else 2) * K.device_cus()
-    while nsplit * 2 <= min(8, reach // tiles, k // 512):
-        nsplit *= 2
-    while nsplit > 1 and (-(-(-(-k // nsplit)) // 64) * 64) * (nsplit - 1) >= k:   # no empty slice
-        nsplit -= 1
-    return nsplit
-
-
 def _mfma_f32_split(n, m, k):
-    """Slices of K for the float32 MFMA kernel.  Up to 64 rows (tiles of 64 rows, two waves) a wave's
-    own chain of products bounds the time (64 cycles for 32 x 32 x 2), not the loads, so a product
-    should give every SIMD a wave or two: up to 16 slices of at least 128 of K."""
+    """Slices of K for the float32 MFMA kernel.  Up to 64 rows (one row of tiles of 64 x 128) a wave's
+    own chain of products bounds the time, so a product should give every SIMD several waves:
+    up to 16 slices of at least 128 of K."""
     if n > 64:
         return K.gemm_prompt_slices(n, m, k, torch.float32)
     waves = -(-m // 128) * 2
@@ -88,31 +73,33 @@ def _mfma_f32_split(n, m, k):
 def _tiles_beat_skinny(n, m, k):
     """Decode batches of more than 16 rows (two or more of the skinny kernel's 16-row
     tiles): the tiled kernel (tiles of 64 rows, both operands through LDS in whole cache lines) takes nearly
-    the same time from 24 to 64 rows, the time of its weights; the skinny one, whose
+    the same time from 20 to 64 rows, the time of its weights; the skinny one, whose
     workgroups each stage all rows of X for 512 of K and leave up to 28 partial sums, grows
-    with the rows.  Measured, tiled against skinny in us (tiles of 64 columns below 40 M
-    weights, of 128 above), at 64 rows: 2,048 x 5,632: 9.8 / 13.5; 2,560 x 2,048: 7.0 / 8.6;
-    2,048 x 2,048: 6.1 / 6.9; 11,264 x 2,048: 14.3 / 19.7; 4,096 x 4,096: 10.3 / 15.1; 4,096 x
-    14,336: 28.7 / 41.1; 28,672 x 4,096: 58.0 / 72.7.  At 24 rows: 8.6 / 9.5; 6.4 / 6.4; 5.6 /
-    5.4; 12.3 / 13.5; 9.3 / 10.8; 27.8 / 30.5.  At 16 rows the largest gain 4,096 x 14,336: 26.9
-    / 28.2, but none in a whole step (8B sizes: 2,745 against 2,731 tok/s).  At 20 rows:
-    8.6 / 9.4; 6.2 / 6.4; 5.6 / 5.4; 12.3 / 13.4; 9.4 / 10.6; 26.1 / 30.0."""
+    with the rows.  Measured, tiled against skinny in us, at 64 rows: 2,048 x 5,632: 10.7 / 13.5;
+    2,560 x 2,048: 6.8 / 8.6; 2,048 x 2,048: 6.2 / 6.9; 11,264 x 2,048: 14.1 / 19.7; 4,096 x 4,096:
+    10.4 / 15.1; 4,096 x 14,336: 23.9 / 41.1; 28,672 x 4,096: 52.5 with the gate / 72.7.  At 20 rows:
+    9.5 / 9.4; 5.6 / 6.4; 5.2 / 5.4; 11.2 / 13.4; 8.8 / 10.6; 22.2 / 30.0."""
     return n > 16
 
 
 def _decode_tile_split(n, m, k):
-    """Slices of K for a decode batch on the tiled kernel.  Against the largest weights: see
-    ``_mfma_split``.  Below (tiles of 64 columns): slices of at least 256 of K until every CU
-    has a workgroup, then further ones of at least 512, up to 16 (measured at 64 rows, in us
-    by slices: 2,048 x 5,632: 14.9 with 4, 9.8 with 8; 11,264 x 2,048: 17.3 with 2, 14.3 with 4,
-    17.7 with 8; 4,096 x 4,096: 12.2 with 4, 10.3 with 8, 11.2 with 16)."""
-    cols = K.gemm_decode_tile_cols(n, m, k)     # the library's choice: 64 below 40 M weights
-    if cols != 64:
-        return _mfma_split(m, k)
-    tiles, cus = -(-m // cols), K.device_cus()
-    nsplit = 1
-    while nsplit < 16 and ((tiles * nsplit < cus and k // (2 * nsplit) >= 256) or k // (2 * nsplit) >= 512):
-        nsplit *= 2
+    """Slices of K for a decode batch on the tiled kernel (one row of tiles of 64).  Below 40 M weights,
+    counted in tiles of 64 columns: slices of at least 256 of K until every CU has a workgroup, then
+    further ones of at least 512, up to 16 (measured at 64 rows, in us by slices: 2,048 x 5,632:
+    14.9 with 4, 10.7 with 8; 11,264 x 2,048: 13.2 with 2, 14.1 with 4, 16.5 with 8; 4,096 x 4,096:
+    12.2 with 4, 10.4 with 8, 11.8 with 16).  Larger weights, in tiles of 128 columns: up to 8 slices
+    of at least 512 of K towards two workgroups a CU, four where K is deep (12,288 x 4,096: 26.2
+    with 2, 22.3 with 4, 24.6 with 8; 4,096 x 14,336: 34.4 with 4, 23.9 with 8)."""
+    cus, nsplit = K.device_cus(), 1
+    if m * k < 40_000_000:
+        tiles = -(-m // 64)
+        while nsplit < 16 and ((tiles * nsplit < cus and k // (2 * nsplit) >= 256) or k // (2 * nsplit) >= 512):
+            nsplit *= 2
+    else:
+        tiles = -(-m // 128)
+        reach = (4 if k >= 8192 and tiles <= cus else 2) * cus
+        while nsplit * 2 <= min(8, reach // tiles, k // 512):
+            nsplit *= 2
     while nsplit > 1 and (-(-(-(-k // nsplit)) // 64) * 64) * (nsplit - 1) >= k:   # no empty slice
         nsplit -= 1
     return nsplit

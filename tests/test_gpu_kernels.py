@@ -426,9 +426,11 @@ def test_gemm_swiglu_at_prompt_sizes(n, f, k, dtype):
     (2047, 4099, 520, 1, False, (256, 192)), (700, 5602, 520, 1, True, (256, 192)),
     (2047, 7001, 520, 1, False, (256, 256)), (1500, 4099, 520, 1, True, (256, 256)),
     (2047, 7004, 768, 1, False, (256, 256)),                                         # whole stages, whole stores
+    (17, 130, 72, 1, False, (64, 128)), (1, 257, 136, 1, True, (64, 128)), (64, 2048, 640, 5, False, (64, 128)),
+    (33, 9001, 2056, 4, False, (64, 256)), (64, 16500, 520, 1, True, (64, 256)),     # decode batches
 ])
 def test_prompt_products_on_every_tile(n, m, k, nsplit, gate, tile):
-    """bfloat16 products of more than 64 rows against a product in double, at the edges of tiles,
+    """bfloat16 products on the tiles against a product in double, at the edges of tiles,
     stages and slices, and nothing written beside the output.  A sum of k products of unit normals in
     32 bits is off by less than k^1/2 2^-24 times a few; the bound leaves a factor of eight."""
     k_ = K()
