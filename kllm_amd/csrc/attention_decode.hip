@@ -409,6 +409,11 @@ extern "C" int kllm_attn_decode_slices(int n, int KV, int H, int hd, int dtype, 
   // (measured at 2,048 keys, one workgroup against the rule below: 192 groups 23.4 against
   // 28.7 us, 128 groups 22.6 against 20.0 us)
   const int heads = H / KV < 16 ? H / KV : 16;
+  // Up to 256 keys (a tile of 32 a wave) the second kernel costs more than the keys: one workgroup of
+  // eight waves writes the output, in us against slices and their merge, in a replayed graph: 8 tokens x
+  // 4 KV heads of 64 at 128 keys 5.8 / 7.2, at 256 6.7 / 7.2, at 512 8.6 / 7.4; 16 tokens x 8 KV heads of
+  // 128 7.0 / 9.9, 8.9 / 10.9, 13.6 / 13.5.
+  if (decode_waves_whole(hdt) > kDecodeWavesShared && max_keys > 0 && max_keys <= 256) return 1;
   if (decode_waves_whole(hdt) > kDecodeWavesShared && 4 * groups >= 3L * device_cus()) {
     // ... unless the groups are a few more than the chip holds of such workgroups at a time:
     // the CUs that get a second one take twice as long as the others, and four workgroups
