@@ -13,7 +13,8 @@
 //   decode   one token, one KV head and up to 32 query heads of its group:
 //            column c is head c, all with the token's bound; the token's keys
 //            are cut into slices, a wave takes one and leaves a partial result
-//            (maximum, sum, unnormalised output) that a second kernel merges
+//            (maximum, sum, unnormalised output) that a second kernel merges (the
+//            workgroup itself where its four waves hold all slices)
 // A key tile is then read once for all 32 columns.
 //
 // MFMA 32x32x2 (lane l, g = l/32, c = l%32): A[c][g], B[g][c], D[8(i/4) + 4g +
@@ -303,7 +304,8 @@ __global__ __launch_bounds__(64 * kF32Waves) void attn_f32_mfma_kernel(const Att
   if (DECODE && a.wg_merge) {
     // The four waves of a workgroup hold four neighbouring slices of the same token and heads
     // (the number of slices is a multiple of four): they meet in LDS, each in the place of its
-    // queries, and leave one partial result, so that the second kernel reads a quarter.
+    // queries, and leave one partial result, so that the second kernel reads a quarter; four slices
+    // in all are the result.
     if (col_ok) {
 #pragma unroll
       for (int r = 0; r < HDT; ++r)
@@ -336,6 +338,10 @@ __global__ __launch_bounds__(64 * kF32Waves) void attn_f32_mfma_kernel(const Att
         const float wt = mw[w] == -INFINITY ? 0.f : expf(mw[w] - M);
         o += wt * q_lds[(w * 32 + col) * QLD + d];
         L += wt * q_lds[(w * 32 + col) * QLD + hd + 1];
+      }
+      if (nout == 1) {                                       // all of the token's keys: nothing is left to merge
+        a.out[((long)t_base * H + h_base + col) * hd + d] = o / L * out_gate(a.gate, t_base, h_base + col, d);
+        continue;
       }
       float* prow = a.part + (((long)t_base * H + h_base + col) * nout + sout) * (hd + 2);
       prow[d] = o;
@@ -429,6 +435,12 @@ int attn_f32_slices(int n, int KV, int H, int max_keys) {
   long want = (groups >= cus ? 8L : 4L) * cus / (groups > 0 ? groups : 1);
   long most = max_keys > 0 ? max_keys / 32 : 64;
   if (most > kAttnF32MaxSlices) most = kAttnF32MaxSlices;
+  // Up to 128 keys (a tile of 32 a wave) the second kernel costs more than the keys: one workgroup's four
+  // slices, which write the output (8 tokens x 4 KV heads of 64, in us, in a replayed graph: 64 keys 9.5, with two
+  // slices and the merge 11.1; 128 keys 9.9 against 12.0; 8 KV heads of 128: 13.7 against 16.6, 15.5 against
+  // 18.0).  Beyond it the matrix products of a second tile on the same SIMDs cost what the merge does (256 keys: 13.4
+  // with four slices, 13.1 with eight waves to a workgroup, 12.2 with eight slices and the merge).
+  if (max_keys > 0 && max_keys <= 32 * kF32Waves && want >= kF32Waves) return kF32Waves;
   if (want > most) want = most;
   if (want < 1) want = 1;
   return (int)want;
@@ -453,7 +465,7 @@ int attn_f32_decode(const float* q, float* out, float* part, const float* cache,
   const long items = (long)count * KV * a.col_blocks * nslices;
   if (int rc = dispatch_f32<true>(a, items, stream)) return rc;
   KLLM_CHECK_LAUNCH("attn_decode float32");
-  if (nslices > 1) {
+  if (nslices > 1 && nslices != kF32Waves) {
     launch_attn_merge<float>(out, part, count, H, hd, a.wg_merge ? nslices / kF32Waves : nslices, token_list, gate, stream);
     KLLM_CHECK_LAUNCH("attn_merge float32");
   }

@@ -1315,6 +1315,21 @@ def test_attention_window_edge(window, dtype):
         assert torch.equal(out2, out), kernel
 
 
+@pytest.mark.parametrize("H,KV,hd,ps", [(4, 2, 16, 16), (32, 4, 64, 16), (40, 1, 32, 16), (6, 3, 80, 32), (2, 1, 128, 16), (2, 2, 256, 16)])
+@pytest.mark.parametrize("window", [0, 24])
+def test_float32_decode_of_short_contexts_writes_the_output_itself(H, KV, hd, ps, window):
+    """Up to 128 keys the proposal is four slices, the waves of one workgroup, which divides by the sum
+    itself (slices without keys among them; more than 32 heads to a group: two workgroups); nothing
+    goes through the room for partial results."""
+    assert K().attn_decode_slices(7, KV, H, hd, torch.float32, 128) == 4
+    c = attention_case(H, KV, hd, ps, torch.float32, window, [(a, 1) for a in (0, 1, 30, 31, 32, 97, 127)], seed=7)
+    out = torch.full_like(c["q"], float("nan"))
+    part = torch.full((7 * H * 4 * (hd + 2),), float("nan"), device=DEV)
+    K().attn_decode(c["q"], out, part, c["cache"], c["pos"], c["sot"], c["bt"], ps, H, KV, hd, window, c["scale"], 4)
+    assert (out.cpu().double() - c["want"]).abs().max() < attn_tol(torch.float32)
+    assert torch.isnan(part).all()
+
+
 def test_attention_refuses_sizes_it_does_not_take():
     k_ = K()
     q = torch.zeros(1, 2 * 272, device=DEV)
