@@ -1,20 +1,20 @@
-// Matrix products of a decode batch (up to 32 rows of X, bfloat16) on MFMA, with
+// Matrix products of a decode batch (up to 32 rows of X in bfloat16, 16 in float32) on MFMA, with
 // the step after the product done in the same launch.  Y = X . W^T, then
 //
 //   PARTS    float32 sums [nsplit, n, m] (only this one may split K);
 //   RESID    the sums are added to the float32 residual stream in place; the
 //            new rows times the weight of the RMS norm behind the addition go
-//            out in bfloat16, and each workgroup leaves the sums of squares of
+//            out in the storage type, and each workgroup leaves the sums of squares of
 //            its columns of the new rows (reference: the fused add + norm,
 //            backend/model.cu:144-165, here without a launch of its own);
-//   SWIGLU   silu(gate) * up in bfloat16 (reference backend/model.cu:477-483);
+//   SWIGLU   silu(gate) * up in the storage type (reference backend/model.cu:477-483);
 //   ROPE     rotated queries and keys, and values, written to q_out and to
 //            the tokens' pages (reference backend/model.cu:170-201).
 //
 // The consumer of a RESID product (SWIGLU or ROPE, `SCALED`) reads those
-// bfloat16 rows x * w as its X and multiplies its float32 sums by the row's
+// rows x * w as its X and multiplies its float32 sums by the row's
 // rsqrt(sum of squares / K + eps): the RMS norm without a kernel of its own
-// and with 16-bit staging.  Against the norm kernel the rounding to bfloat16
+// and with 16-bit staging in bfloat16.  Against the norm kernel the rounding to bfloat16
 // happens before the row scale instead of after it; both round every element
 // of the normalised row once.
 //
@@ -51,15 +51,41 @@ namespace kllm {
 // workgroup or more of X in registers measured slower for the same reason).
 constexpr int FL_AHEAD = 4;
 // LDS row padding (elements): zeros behind K as far as the waves' slices reach beyond it
-// (less than 32 per wave), 8 to shift banks
-constexpr int fl_pad(int nw) { return 32 * nw + 8; }
+// (less than a step per wave), 16 bytes to shift banks
+template <typename T> struct FlType;        // 16 bytes of a row; elements of it, and of a step (64 bytes) of K
+template <> struct FlType<bf16_t> { typedef bf16x8 op_t; static constexpr int E = 8, STEP = 32, CHAINS = 1; };
+template <> struct FlType<float> { typedef floatx4 op_t; static constexpr int E = 4, STEP = 16, CHAINS = 16; };
+template <typename T> constexpr int fl_pad(int nw) { return FlType<T>::STEP * nw + FlType<T>::E; }
+
+// One step of K of a tile: bfloat16 one instruction of 32, float32 four of 4 (true 32-bit; which element of K
+// a lane's operand stands for is free as long as both operands agree).  A sum that one accumulator
+// carries through all of a wave's K would be rounded more often than the gemv's, whose 64 lanes each add
+// a 64th of it: float32 sums go in 16 chains a wave, 64 or 128 a workgroup, added in pairs at the end (error against
+// 64 bits, relative to the sums: K of 2,048 2.1e-7 with 4 chains, 1.23e-7 with 16, the gemv 1.23e-7; 5,632
+// 3.4e-7, 1.83e-7 and 1.81e-7).  The time is that of the weights and of staging the rows: 8 tokens at 1.1B sizes
+// 2.14 ms a step with the gemv, 1.70 with this, 16 tokens 3.06 and 1.83.
+__device__ __forceinline__ void fl_mma(bf16x8 a, bf16x8 b, floatx4 (&acc)[1], int) {
+  acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[0], 0, 0, 0);
+}
+__device__ __forceinline__ void fl_mma(floatx4 a, floatx4 b, floatx4 (&acc)[16], int i) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) acc[4 * i + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], acc[4 * i + e], 0, 0, 0);
+}
+__device__ __forceinline__ floatx4 fl_sum(const floatx4 (&acc)[1]) { return acc[0]; }
+__device__ __forceinline__ floatx4 fl_sum(floatx4 (&acc)[16]) {
+#pragma unroll
+  for (int d = 8; d > 0; d >>= 1)
+#pragma unroll
+    for (int e = 0; e < d; ++e) acc[e] += acc[e + d];
+  return acc[0];
+}
 constexpr int FL_SS_LOADS = 4;     // 16-byte loads per lane of a row's partial sums of squares: 16 lanes a row
 constexpr int FL_SS_MAX = 16 * 4 * FL_SS_LOADS;   // partial sums of squares per row at most
 constexpr int FL_LDS_MAX = 160 * 1024;
 constexpr int FL_TILE = 16 * 17;    // floats of one wave's partial tile in LDS: [x row][w row], padded
 
 enum : int { FL_PARTS = 0, FL_RESID = 1, FL_SWIGLU = 2, FL_ROPE = 3 };
-// FL_PARTS with act >= FL_UNARY: y is bfloat16 [n][m] = unary_act(sums, act - FL_UNARY), the
+// FL_PARTS with act >= FL_UNARY: y is [n][m] in the storage type = unary_act(sums, act - FL_UNARY), the
 // activation's learned constants (if it has any) behind norm_w.
 constexpr int FL_UNARY = 16;
 
@@ -73,7 +99,7 @@ struct FlOut {
   const int* block_table;
   int max_pages, page_size, H, KV, hd;
   int act;                      // the gate's activation (FL_SWIGLU)
-  float* resid;                 // FL_RESID: the residual stream [n][m]; y receives bfloat16 resid * norm_w
+  float* resid;                 // FL_RESID: the residual stream [n][m]; y receives resid * norm_w in the storage type
   const float* norm_w;          // FL_RESID: weight [m] of the norm behind the addition
   float* ss_out;                // FL_RESID: [n][workgroups rounded up to 4] sums of squares of the new rows
   const float* ss_in;           // SCALED: [n][ss_parts rounded up to 4], what a FL_RESID product left
@@ -116,32 +142,34 @@ __device__ __forceinline__ void fl_lds_barrier() {
 // NW waves share a tile's K; SCALED: the sums are multiplied by a row scale made from out.ss_in;
 // PASSES: the rows of X do not fit into LDS at once and go in passes of kpass of K (a kernel of
 // its own, so that the one for rows that fit carries none of it).
-template <int NT, int EP, int NW, bool SCALED, bool PASSES>
-__global__ __launch_bounds__(64 * NW) void fused_linear_kernel(const bf16_t* __restrict__ X, FlOut out,
-                                                           const bf16_t* __restrict__ W, int n, int m,
+template <typename T, int NT, int EP, int NW, bool SCALED, bool PASSES>
+__global__ __launch_bounds__(64 * NW) void fused_linear_kernel(const T* __restrict__ X, FlOut out,
+                                                           const T* __restrict__ W, int n, int m,
                                                            int k, int kslice, int tiles, int tiles_per_wg,
                                                            int x_stride, int kpass) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-  const int ld = kpass + fl_pad(NW);
-  bf16_t* xs = reinterpret_cast<bf16_t*>(lds_raw);                            // [n][ld]
-  float* part = reinterpret_cast<float*>(lds_raw + (size_t)n * ld * sizeof(bf16_t));   // [2][NW][NT][x row 16][17]
+  typedef typename FlType<T>::op_t op_t;
+  constexpr int E = FlType<T>::E, STEP = FlType<T>::STEP;
+  const int ld = kpass + fl_pad<T>(NW);
+  T* xs = reinterpret_cast<T*>(lds_raw);                                      // [n][ld]
+  float* part = reinterpret_cast<float*>(lds_raw + (size_t)n * ld * sizeof(T));   // [2][NW][NT][x row 16][17]
   float* row_scale = part + 2 * NW * NT * FL_TILE;                            // [32]
 
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
   const int g = lane / 16, c = lane % 16;
   const int kbeg = blockIdx.y * kslice;
-  const int klen = min(k, kbeg + kslice) - kbeg;            // a multiple of 8
+  const int klen = min(k, kbeg + kslice) - kbeg;            // a multiple of E
   // The slice is staged and multiplied in passes of kpass of K (one pass where all rows of the slice
   // fit into LDS; several only with one tile to a workgroup, whose sums then stay in registers).
   const int npass = PASSES ? (klen + kpass - 1) / kpass : 1;
   auto pass_len = [&](int pass) { return PASSES ? min(klen - pass * kpass, kpass) : klen; };
-  const int kw = ((pass_len(0) + NW - 1) / NW + 31) / 32 * 32;     // K of one wave in a pass
+  const int kw = ((pass_len(0) + NW - 1) / NW + STEP - 1) / STEP * STEP;     // K of one wave in a pass
   const int wk0 = wave * kw;                                // this wave's offset in the pass
-  const int steps = kw / 32;
+  const int steps = kw / STEP;
   const int tile0 = blockIdx.x * tiles_per_wg;
   const int my_tiles = min(tiles_per_wg, tiles - tile0);
   const int rsteps = (steps + 2 * FL_AHEAD - 1) / (2 * FL_AHEAD) * (2 * FL_AHEAD);   // whole turns of both buffers
-  const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  const op_t zero = op_t{};
 
   // ---- rotate-and-append epilogue: thread (pair tid % 8, token tid / 8) needs the token's
   // page and slot, and cos and sin of its pair.  Loads return in order, so the position and
@@ -159,18 +187,19 @@ __global__ __launch_bounds__(64 * NW) void fused_linear_kernel(const bf16_t* __r
   }
 
   // ---- X: wave w stages rows w, w + NW, ... of the slice straight into LDS, a kilobyte (512 of
-  // K) per instruction, without passing registers: all of them are in flight at once however
+  // K, 256 in 32 bits) per instruction, without passing registers: all of them are in flight at once however
   // many rows there are, before the weights are asked for (loads return in order).
   auto stage = [&](int pass) {
     const int plen = pass_len(pass);
-    const int kchunks = (plen + 511) / 512;
+    constexpr int CHUNK = kWave * E;
+    const int kchunks = (plen + CHUNK - 1) / CHUNK;
     for (int r = wave; r < n; r += NW) {
-      const bf16_t* src = X + (long)r * x_stride + kbeg + pass * kpass + lane * 8;
-      bf16_t* dst = xs + r * ld;
+      const T* src = X + (long)r * x_stride + kbeg + pass * kpass + lane * E;
+      T* dst = xs + r * ld;
       for (int ch = 0; ch < kchunks; ++ch)
-        if (ch * 512 + lane * 8 < plen)
-          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + ch * 512),
-                                           (__attribute__((address_space(3))) void*)(dst + ch * 512), 16, 0, 0);
+        if (ch * CHUNK + lane * E < plen)
+          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + ch * CHUNK),
+                                           (__attribute__((address_space(3))) void*)(dst + ch * CHUNK), 16, 0, 0);
     }
   };
   stage(0);
@@ -227,9 +256,9 @@ __global__ __launch_bounds__(64 * NW) void fused_linear_kernel(const bf16_t* __r
   // With a tiled copy of W (out.tiled) a tile's step is 1 KB in the order the lanes want it:
   // a load instruction reads one contiguous kilobyte instead of 64 bytes of each of 16 rows
   // (streamed alone, 2,048 x 5,632 weights: 8.5 -> 6.7 us; 11,264 x 2,048: 12.0 -> 9.9).
-  const bf16_t* far_row;                                    // first K of this lane's row of W
+  const T* far_row;                                         // first K of this lane's row of W
   int far_lane_off;                                         // this lane's offset in it, or -1: no such row
-  const int far_stride = out.tiled ? 512 : 32;              // elements from a step to the next
+  const int far_stride = out.tiled ? kWave * E : STEP;              // elements from a step to the next
   int far_tile = 0, far_s0 = 0;                             // the steps that are loaded next; a tile's passes count as tiles
   int far_wlen = 0;                                         // this wave's K in that pass
   auto tile_ptr = [&](int u) {
@@ -238,20 +267,20 @@ __global__ __launch_bounds__(64 * NW) void fused_linear_kernel(const bf16_t* __r
     far_wlen = max(0, min(pass_len(pass), wk0 + kw) - wk0);
     if (out.tiled) {     // rows that do not exist hold zeros there; a tile that does not exist reads the first
       const long tl = t < my_tiles ? tile0 + t : tile0;
-      far_row = W + ((tl * ((k + 31) / 32) + pbeg / 32) * kWave + lane) * 8;
-      far_lane_off = (wk0 / 32) * 512;
+      far_row = W + ((tl * ((k + STEP - 1) / STEP) + pbeg / STEP) * kWave + lane) * E;
+      far_lane_off = (wk0 / STEP) * (kWave * E);
       return;
     }
     const long r = t < my_tiles ? fl_row<EP>((int)tile0 + t, c, m, out) : -1;
     far_row = W + (r >= 0 ? r : 0) * k + pbeg;
-    far_lane_off = r >= 0 ? wk0 + 8 * g : -1;
+    far_lane_off = r >= 0 ? wk0 + E * g : -1;
   };
-  auto fill = [&](bf16x8 (&buf)[FL_AHEAD]) {
+  auto fill = [&](op_t (&buf)[FL_AHEAD]) {
 #pragma unroll
     for (int i = 0; i < FL_AHEAD; ++i) {
       const int s = far_s0 + i;
-      const bool valid = far_lane_off >= 0 && s < steps && 32 * s + 8 * g < far_wlen;
-      buf[i] = *reinterpret_cast<const bf16x8*>(far_row + (valid ? far_lane_off + far_stride * s : 0));
+      const bool valid = far_lane_off >= 0 && s < steps && STEP * s + E * g < far_wlen;
+      buf[i] = *reinterpret_cast<const op_t*>(far_row + (valid ? far_lane_off + far_stride * s : 0));
     }
     far_s0 += FL_AHEAD;
     if (far_s0 == rsteps) {
@@ -259,23 +288,23 @@ __global__ __launch_bounds__(64 * NW) void fused_linear_kernel(const bf16_t* __r
       tile_ptr(++far_tile);
     }
   };
-  bf16x8 bufa[FL_AHEAD], bufb[FL_AHEAD];
+  op_t bufa[FL_AHEAD], bufb[FL_AHEAD];
   tile_ptr(0);
   fill(bufa);
   fill(bufb);
 
   auto zero_behind = [&](int pass) {   // zeros in X's columns from the K of the pass to where the waves' slices reach
-    constexpr int per_row = 4 * NW;                         // threads to 32 * NW zeros of a row: 16 rows at a time
+    constexpr int per_row = 4 * NW;                         // threads to STEP * NW zeros of a row: 16 rows at a time
     const int plen = pass_len(pass);                        // (a last pass may be shorter than the others)
     const int r = tid / per_row;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
       if (t * 16 + r < n) {
-        if (!PASSES) {   // all passes alike: the slices reach less than 32 NW beyond
-          *reinterpret_cast<bf16x8*>(&xs[(t * 16 + r) * ld + plen + 8 * (tid % per_row)]) = zero;
+        if (!PASSES) {   // all passes alike: the slices reach less than STEP NW beyond
+          *reinterpret_cast<op_t*>(&xs[(t * 16 + r) * ld + plen + E * (tid % per_row)]) = zero;
         } else {
-          for (int at = plen + 8 * (tid % per_row); at < NW * kw; at += 8 * per_row)
-            *reinterpret_cast<bf16x8*>(&xs[(t * 16 + r) * ld + at]) = zero;
+          for (int at = plen + E * (tid % per_row); at < NW * kw; at += E * per_row)
+            *reinterpret_cast<op_t*>(&xs[(t * 16 + r) * ld + at]) = zero;
         }
       }
   };
@@ -331,29 +360,31 @@ __global__ __launch_bounds__(64 * NW) void fused_linear_kernel(const bf16_t* __r
   }
   fl_lds_barrier();
 
-  floatx4 acc[NT];
-  const bf16_t* xrow[NT];                                   // rows beyond n are ignored: they read row n - 1
+  constexpr int CHAINS = FlType<T>::CHAINS;
+  floatx4 acc[NT][CHAINS];
+  const T* xrow[NT];                                        // rows beyond n are ignored: they read row n - 1
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-    xrow[t] = xs + min(t * 16 + c, n - 1) * ld + wk0 + 8 * g;
+#pragma unroll
+    for (int e = 0; e < CHAINS; ++e) acc[t][e] = floatx4{0.f, 0.f, 0.f, 0.f};
+    xrow[t] = xs + min(t * 16 + c, n - 1) * ld + wk0 + E * g;
   }
   // A buffer's steps: all their rows of X are asked of LDS first, without a branch between them, so
   // that LDS answers while the wave still waits for the weights; a step beyond the wave's last
   // multiplies with zeros (its weights are whatever the first K of the row holds).
-  auto multiply = [&](const bf16x8 (&buf)[FL_AHEAD], int s0) {
-    bf16x8 b[FL_AHEAD][NT];
+  auto multiply = [&](const op_t (&buf)[FL_AHEAD], int s0) {
+    op_t b[FL_AHEAD][NT];
 #pragma unroll
     for (int i = 0; i < FL_AHEAD; ++i)
 #pragma unroll
       for (int t = 0; t < NT; ++t)
-        b[i][t] = *reinterpret_cast<const bf16x8*>(xrow[t] + 32 * min(s0 + i, steps - 1));
+        b[i][t] = *reinterpret_cast<const op_t*>(xrow[t] + STEP * min(s0 + i, steps - 1));
 #pragma unroll
     for (int i = 0; i < FL_AHEAD; ++i) {
       const bool live = s0 + i < steps;
 #pragma unroll
       for (int t = 0; t < NT; ++t)
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(buf[i], live ? b[i][t] : zero, acc[t], 0, 0, 0);
+        fl_mma(buf[i], live ? b[i][t] : zero, acc[t], i);
     }
   };
 
@@ -380,9 +411,11 @@ __global__ __launch_bounds__(64 * NW) void fused_linear_kernel(const bf16_t* __r
     float* pb = part + (tile & 1) * NW * NT * FL_TILE;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
+      const floatx4 sum = fl_sum(acc[t]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) pb[(wave * NT + t) * FL_TILE + c * 17 + 4 * g + i] = acc[t][i];
-      acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < 4; ++i) pb[(wave * NT + t) * FL_TILE + c * 17 + 4 * g + i] = sum[i];
+#pragma unroll
+      for (int e = 0; e < CHAINS; ++e) acc[t][e] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
     fl_lds_barrier();
     const int tl = tile0 + tile;
@@ -397,13 +430,13 @@ __global__ __launch_bounds__(64 * NW) void fused_linear_kernel(const bf16_t* __r
 #pragma unroll
         for (int w = 0; w < NW; ++w) v += pb[(w * NT + t) * FL_TILE + xc * 17 + r16];
         if (row < m && xr < n) {
-          if (out.act >= FL_UNARY) {       // an activation without a gate on the sums, stored in bfloat16
+          if (out.act >= FL_UNARY) {       // an activation without a gate on the sums, in the storage type
             float a_pos = 0.f, a_neg = 0.f;
             if (out.act - FL_UNARY == ACT_XIELU) {
               a_pos = softplus_f32(out.norm_w[0]);
               a_neg = softplus_f32(out.norm_w[1]);
             }
-            reinterpret_cast<bf16_t*>(out.y)[(long)xr * m + row] = (bf16_t)unary_act(v, out.act - FL_UNARY, a_pos, a_neg);
+            reinterpret_cast<T*>(out.y)[(long)xr * m + row] = from_f32<T>(unary_act(v, out.act - FL_UNARY, a_pos, a_neg));
           } else {
             reinterpret_cast<float*>(out.y)[((long)blockIdx.y * n + xr) * m + row] = v;
           }
@@ -422,7 +455,7 @@ __global__ __launch_bounds__(64 * NW) void fused_linear_kernel(const bf16_t* __r
           if (row < m && xr < n) {
             const float x = res_old[t] + v;
             out.resid[(long)xr * m + row] = x;
-            reinterpret_cast<bf16_t*>(out.y)[(long)xr * m + row] = from_f32<bf16_t>(x * res_w);
+            reinterpret_cast<T*>(out.y)[(long)xr * m + row] = from_f32<T>(x * res_w);
             ss_acc[t] += x * x;
           }
         }
@@ -447,8 +480,8 @@ __global__ __launch_bounds__(64 * NW) void fused_linear_kernel(const bf16_t* __r
           b *= rs;
         }
         if (EP == FL_SWIGLU) {
-          bf16_t* h = reinterpret_cast<bf16_t*>(out.y);
-          h[(long)xr * pairs + pair] = from_f32<bf16_t>(gate_act(a, out.act) * b);
+          T* h = reinterpret_cast<T*>(out.y);
+          h[(long)xr * pairs + pair] = from_f32<T>(gate_act(a, out.act) * b);
         } else {
           const int half = out.hd / 2;
           const int q_pairs = out.H * half, k_pairs = out.cache ? out.KV * half : 0;
@@ -460,18 +493,18 @@ __global__ __launch_bounds__(64 * NW) void fused_linear_kernel(const bf16_t* __r
             const int head = p / half, j = p % half;
             const float cc = ep_cos[t], sn = ep_sin[t];
             const float ra = a * cc - b * sn, rb = b * cc + a * sn;
-            bf16_t* o = region == 0
-                            ? reinterpret_cast<bf16_t*>(out.y) + ((long)xr * out.H + head) * out.hd
-                            : reinterpret_cast<bf16_t*>(out.cache) +
+            T* o = region == 0
+                            ? reinterpret_cast<T*>(out.y) + ((long)xr * out.H + head) * out.hd
+                            : reinterpret_cast<T*>(out.cache) +
                                   (((long)page * 2 + 0) * out.KV + head) * block + (long)slot * out.hd;
-            o[j] = from_f32<bf16_t>(ra);
-            o[j + half] = from_f32<bf16_t>(rb);
+            o[j] = from_f32<T>(ra);
+            o[j + half] = from_f32<T>(rb);
           } else {
             const int e = 2 * (pair - q_pairs - k_pairs);
             const int head = e / out.hd, j = e % out.hd;
-            bf16_t* v = reinterpret_cast<bf16_t*>(out.cache) + (((long)page * 2 + 1) * out.KV + head) * block;
-            v[(long)j * out.page_size + slot] = from_f32<bf16_t>(a);
-            v[(long)(j + 1) * out.page_size + slot] = from_f32<bf16_t>(b);
+            T* v = reinterpret_cast<T*>(out.cache) + (((long)page * 2 + 1) * out.KV + head) * block;
+            v[(long)j * out.page_size + slot] = from_f32<T>(a);
+            v[(long)(j + 1) * out.page_size + slot] = from_f32<T>(b);
           }
         }
       }
@@ -491,73 +524,75 @@ __global__ __launch_bounds__(64 * NW) void fused_linear_kernel(const bf16_t* __r
   }
 }
 
-// The tiled copy of W for an epilogue: [tile][step of 32 of K][lane][8 elements], lane (g, c)
-// holding W[row of MFMA row c][32 step + 8 g ...], zeros where the row or the K is not there.
+// The tiled copy of W for an epilogue: [tile][step of 64 bytes of K][lane][16 bytes], lane (g, c)
+// holding W[row of MFMA row c][STEP step + E g ...], zeros where the row or the K is not there.
 // One workgroup of 64 lanes per (tile, step).
-template <int EP>
-__global__ __launch_bounds__(64) void fl_tile_kernel(const bf16_t* __restrict__ W, bf16_t* __restrict__ Wt, FlOut out,
+template <typename T, int EP>
+__global__ __launch_bounds__(64) void fl_tile_kernel(const T* __restrict__ W, T* __restrict__ Wt, FlOut out,
                                                      int m, int k) {
+  typedef typename FlType<T>::op_t op_t;
+  constexpr int E = FlType<T>::E, STEP = FlType<T>::STEP;
   const int lane = threadIdx.x, g = lane / 16, c = lane % 16;
   const int step = blockIdx.y, ksteps = gridDim.y;
   const long tile = blockIdx.x;
   const long r = fl_row<EP>((int)tile, c, m, out);
-  const int kk = 32 * step + 8 * g;
-  bf16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-  if (r >= 0 && kk < k) v = *reinterpret_cast<const bf16x8*>(W + r * k + kk);      // k is a multiple of 8
-  *reinterpret_cast<bf16x8*>(Wt + ((tile * ksteps + step) * kWave + lane) * 8) = v;
+  const int kk = STEP * step + E * g;
+  op_t v = op_t{};
+  if (r >= 0 && kk < k) v = *reinterpret_cast<const op_t*>(W + r * k + kk);      // k is a multiple of E
+  *reinterpret_cast<op_t*>(Wt + ((tile * ksteps + step) * kWave + lane) * E) = v;
 }
 
-static size_t fl_lds_bytes(int n, int nt, int kslice, int nw = 4) {
-  return (size_t)n * (kslice + fl_pad(nw)) * sizeof(bf16_t) + (size_t)(2 * nw * nt * FL_TILE + 32) * sizeof(float);
+static size_t fl_lds_bytes(bool f32, int n, int nt, int kslice, int nw = 4) {
+  return (size_t)n * (kslice + (f32 ? fl_pad<float>(nw) : fl_pad<bf16_t>(nw))) * (f32 ? 4 : 2) + (size_t)(2 * nw * nt * FL_TILE + 32) * sizeof(float);
 }
 
-template <int NT, int EP, int NW, bool SCALED, bool PASSES>
+template <typename T, int NT, int EP, int NW, bool SCALED, bool PASSES>
 static int fl_launch_passes(const void* x, const FlOut& out, const void* w, int n, int m, int k, int kslice, int kpass,
                      int nsplit, int tiles, int tiles_per_wg, int x_stride, hipStream_t stream) {
-  size_t lds = fl_lds_bytes(n, NT, kpass, NW);
+  size_t lds = fl_lds_bytes(sizeof(T) == 4, n, NT, kpass, NW);
   static size_t allowed = 64 * 1024;          // one per instantiation
   if (lds > allowed) {
-    hipError_t e = hipFuncSetAttribute((const void*)fused_linear_kernel<NT, EP, NW, SCALED, PASSES>,
+    hipError_t e = hipFuncSetAttribute((const void*)fused_linear_kernel<T, NT, EP, NW, SCALED, PASSES>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, FL_LDS_MAX);
     if (e != hipSuccess) KLLM_FAIL((int)e, "fused_linear: cannot raise the LDS limit: %s", hipGetErrorString(e));
     allowed = FL_LDS_MAX;
   }
   const dim3 grid(ceil_div(tiles, tiles_per_wg), nsplit);
-  hipLaunchKernelGGL((fused_linear_kernel<NT, EP, NW, SCALED, PASSES>), grid, dim3(64 * NW), lds, stream, (const bf16_t*)x,
-                     out, (const bf16_t*)w, n, m, k, kslice, tiles, tiles_per_wg, x_stride, kpass);
+  hipLaunchKernelGGL((fused_linear_kernel<T, NT, EP, NW, SCALED, PASSES>), grid, dim3(64 * NW), lds, stream, (const T*)x,
+                     out, (const T*)w, n, m, k, kslice, tiles, tiles_per_wg, x_stride, kpass);
   return 0;
 }
 
-template <int NT, int EP, int NW, bool SCALED>
+template <typename T, int NT, int EP, int NW, bool SCALED>
 static int fl_launch(const void* x, const FlOut& out, const void* w, int n, int m, int k, int kslice, int kpass,
                      int nsplit, int tiles, int tiles_per_wg, int x_stride, hipStream_t stream) {
   if (kpass < kslice)
-    return fl_launch_passes<NT, EP, NW, SCALED, true>(x, out, w, n, m, k, kslice, kpass, nsplit, tiles, tiles_per_wg,
+    return fl_launch_passes<T, NT, EP, NW, SCALED, true>(x, out, w, n, m, k, kslice, kpass, nsplit, tiles, tiles_per_wg,
                                                       x_stride, stream);
-  return fl_launch_passes<NT, EP, NW, SCALED, false>(x, out, w, n, m, k, kslice, kslice, nsplit, tiles, tiles_per_wg,
+  return fl_launch_passes<T, NT, EP, NW, SCALED, false>(x, out, w, n, m, k, kslice, kslice, nsplit, tiles, tiles_per_wg,
                                                      x_stride, stream);
 }
 
-template <int NT, int NW>
+template <typename T, int NT, int NW>
 static int fl_launch_nw(int ep, bool scaled, const void* x, const FlOut& out, const void* w, int n, int m, int k,
                         int kslice, int kpass, int nsplit, int tiles, int tpw, int xs, hipStream_t st) {
   switch (ep) {
-    case FL_PARTS: return fl_launch<NT, FL_PARTS, NW, false>(x, out, w, n, m, k, kslice, kpass, nsplit, tiles, tpw, xs, st);
-    case FL_RESID: return fl_launch<NT, FL_RESID, NW, false>(x, out, w, n, m, k, kslice, kpass, nsplit, tiles, tpw, xs, st);
+    case FL_PARTS: return fl_launch<T, NT, FL_PARTS, NW, false>(x, out, w, n, m, k, kslice, kpass, nsplit, tiles, tpw, xs, st);
+    case FL_RESID: return fl_launch<T, NT, FL_RESID, NW, false>(x, out, w, n, m, k, kslice, kpass, nsplit, tiles, tpw, xs, st);
     case FL_SWIGLU:
-      return scaled ? fl_launch<NT, FL_SWIGLU, NW, true>(x, out, w, n, m, k, kslice, kpass, nsplit, tiles, tpw, xs, st)
-                    : fl_launch<NT, FL_SWIGLU, NW, false>(x, out, w, n, m, k, kslice, kpass, nsplit, tiles, tpw, xs, st);
+      return scaled ? fl_launch<T, NT, FL_SWIGLU, NW, true>(x, out, w, n, m, k, kslice, kpass, nsplit, tiles, tpw, xs, st)
+                    : fl_launch<T, NT, FL_SWIGLU, NW, false>(x, out, w, n, m, k, kslice, kpass, nsplit, tiles, tpw, xs, st);
     default:
-      return scaled ? fl_launch<NT, FL_ROPE, NW, true>(x, out, w, n, m, k, kslice, kpass, nsplit, tiles, tpw, xs, st)
-                    : fl_launch<NT, FL_ROPE, NW, false>(x, out, w, n, m, k, kslice, kpass, nsplit, tiles, tpw, xs, st);
+      return scaled ? fl_launch<T, NT, FL_ROPE, NW, true>(x, out, w, n, m, k, kslice, kpass, nsplit, tiles, tpw, xs, st)
+                    : fl_launch<T, NT, FL_ROPE, NW, false>(x, out, w, n, m, k, kslice, kpass, nsplit, tiles, tpw, xs, st);
   }
 }
 
-template <int NT>
+template <typename T, int NT>
 static int fl_launch_ep(int ep, bool scaled, int nw, const void* x, const FlOut& out, const void* w, int n, int m, int k,
                         int kslice, int kpass, int nsplit, int tiles, int tpw, int xs, hipStream_t st) {
-  if (nw == 8) return fl_launch_nw<NT, 8>(ep, scaled, x, out, w, n, m, k, kslice, kpass, nsplit, tiles, tpw, xs, st);
-  return fl_launch_nw<NT, 4>(ep, scaled, x, out, w, n, m, k, kslice, kpass, nsplit, tiles, tpw, xs, st);
+  if (nw == 8) return fl_launch_nw<T, NT, 8>(ep, scaled, x, out, w, n, m, k, kslice, kpass, nsplit, tiles, tpw, xs, st);
+  return fl_launch_nw<T, NT, 4>(ep, scaled, x, out, w, n, m, k, kslice, kpass, nsplit, tiles, tpw, xs, st);
 }
 
 }  // namespace kllm
@@ -566,20 +601,20 @@ using namespace kllm;
 
 static bool fl_aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
-extern "C" long kllm_fused_linear_lds_bytes(int n, int k, int nsplit) {
+extern "C" long kllm_fused_linear_lds_bytes(int n, int k, int nsplit, int dtype) {
   if (n <= 0 || k <= 0 || nsplit <= 0) return -1;
   const int kslice = ceil_div(ceil_div(k, nsplit), 32) * 32;
-  return (long)fl_lds_bytes(n, ceil_div(n, 16), kslice);
+  return (long)fl_lds_bytes(dtype == DT_F32, n, ceil_div(n, 16), kslice);
 }
 
 // K of a pass for n rows of a slice of kslice: the slice itself where its rows fit into LDS, else
 // the least number of equal passes (up to FL_MAX_PASSES) whose rows do; 0 if none does.
 constexpr int FL_MAX_PASSES = 8;
-static int fl_pass_k(int n, int kslice, int nw = 4) {
+static int fl_pass_k(bool f32, int n, int kslice, int nw = 4) {
   const int nt = ceil_div(n, 16);
   for (int passes = 1; passes <= FL_MAX_PASSES; ++passes) {
     const int kpass = ceil_div(ceil_div(kslice, passes), 32) * 32;
-    if (fl_lds_bytes(n, nt, kpass, nw) <= (size_t)FL_LDS_MAX) return kpass;
+    if (fl_lds_bytes(f32, n, nt, kpass, nw) <= (size_t)FL_LDS_MAX) return kpass;
   }
   return 0;
 }
@@ -591,22 +626,26 @@ static int fl_pass_k(int n, int kslice, int nw = 4) {
 // workgroups already share their CUs (eight: 1.042 -> 1.078 ms), for the logits (no difference),
 // and wherever eight waves' partial tiles and padding leave no room for the rows of X; sixteen
 // are slower than eight everywhere.
-static int fl_waves(int ep, int n, int kslice, int kpass4, int workgroups, int tiles_per_wg) {
+static int fl_waves(bool f32, int ep, int n, int kslice, int kpass4, int workgroups, int tiles_per_wg) {
   if (ep != FL_RESID && ep != FL_ROPE) return 4;
   if (8 * workgroups > 5 * device_cus()) return 4;   // (4,096 x 4,096 on 256 workgroups: a step of 8 tokens at 8B sizes 4.09 -> 4.12 ms with eight)
   // Eight waves' partial tiles and padding take room from the rows of X: they may need a pass
   // more than four waves would, and still win (13 tokens at 1.1B sizes: 1.172 -> 1.16 ms; 16
   // tokens, two passes either way: 1.207 -> 1.176), but passes want one tile to a workgroup.
   // From 17 rows on a pass more loses (28 tokens: 1.59 against 1.55 ms).
-  const int kpass8 = fl_pass_k(n, kslice, 8);
+  const int kpass8 = fl_pass_k(f32, n, kslice, 8);
   if (!kpass8 || (kpass8 < kslice && (tiles_per_wg > 1 || (n > 16 && kpass4 >= kslice)))) return 4;
   return 8;
 }
 
-extern "C" int kllm_fused_linear_passes(int n, int k, int nsplit) {
-  if (n <= 0 || n > KLLM_FUSED_LINEAR_MAX_ROWS || k <= 0 || nsplit <= 0) return 0;
+// Rows of X that the kernel takes: two tiles of 16 in bfloat16, one in float32 (whose rows are twice as long).
+static int fl_max_rows(bool f32) { return f32 ? 16 : KLLM_FUSED_LINEAR_MAX_ROWS; }
+
+extern "C" int kllm_fused_linear_passes(int n, int k, int nsplit, int dtype) {
+  const bool f32 = dtype == DT_F32;
+  if (n <= 0 || n > fl_max_rows(f32) || k <= 0 || nsplit <= 0) return 0;
   const int kslice = ceil_div(ceil_div(k, nsplit), 32) * 32;
-  const int kpass = fl_pass_k(n, kslice);
+  const int kpass = fl_pass_k(f32, n, kslice);
   return kpass ? ceil_div(kslice < k ? kslice : k, kpass) : 0;
 }
 
@@ -619,15 +658,19 @@ extern "C" int kllm_fused_linear_max_parts(void) { return FL_SS_MAX; }
 
 static int fl_tiles(int kind, int m) { return kind == FL_SWIGLU || kind == FL_ROPE ? ceil_div(m / 2, 8) : ceil_div(m, 16); }
 
-extern "C" long kllm_fused_linear_tiled_elements(int kind, int m, int k) {
-  if (m <= 0 || k <= 0 || k % 8) return -1;
-  return (long)fl_tiles(kind, m) * ceil_div(k, 32) * 512;
+extern "C" long kllm_fused_linear_tiled_elements(int kind, int m, int k, int dtype) {
+  const int e = dtype == DT_F32 ? 4 : 8;
+  if (m <= 0 || k <= 0 || k % e) return -1;
+  return (long)fl_tiles(kind, m) * ceil_div(k, 4 * e) * kWave * e;
 }
 
-extern "C" int kllm_fused_linear_tile(const void* w, void* wt, int kind, int m, int k, int H, int KV, int hd,
+extern "C" int kllm_fused_linear_tile(const void* w, void* wt, int kind, int m, int k, int dtype, int H, int KV, int hd,
                                       int with_kv, hipStream_t stream) {
+  KLLM_REQUIRE(dtype == DT_F32 || dtype == DT_BF16, "fused_linear_tile: unknown dtype %d", dtype);
+  const bool f32 = dtype == DT_F32;
+  const int e = f32 ? 4 : 8;
   KLLM_REQUIRE(w && wt && fl_aligned16(w) && fl_aligned16(wt), "fused_linear_tile: null or unaligned pointer");
-  KLLM_REQUIRE(m > 0 && k > 0 && k % 8 == 0 && m < (1 << 30), "fused_linear_tile: bad sizes m=%d k=%d", m, k);
+  KLLM_REQUIRE(m > 0 && k > 0 && k % e == 0 && m < (1 << 30), "fused_linear_tile: bad sizes m=%d k=%d", m, k);
   KLLM_REQUIRE(kind == FL_PARTS || kind == FL_RESID || kind == FL_SWIGLU || kind == FL_ROPE,
                "fused_linear_tile: unknown output kind %d", kind);
   FlOut out = {};
@@ -640,13 +683,18 @@ extern "C" int kllm_fused_linear_tile(const void* w, void* wt, int kind, int m, 
     out.hd = hd;
     out.cache = with_kv ? const_cast<void*>(w) : nullptr;     // only "is there a cache" is read
   }
-  const dim3 grid(fl_tiles(kind, m), ceil_div(k, 32));
+  const dim3 grid(fl_tiles(kind, m), ceil_div(k, 4 * e));
   KLLM_REQUIRE(grid.y <= 65535u, "fused_linear_tile: K=%d is too long", k);
-  const bf16_t* wp = (const bf16_t*)w;
-  bf16_t* tp = (bf16_t*)wt;
-  if (kind == FL_SWIGLU) hipLaunchKernelGGL(fl_tile_kernel<FL_SWIGLU>, grid, dim3(64), 0, stream, wp, tp, out, m, k);
-  else if (kind == FL_ROPE) hipLaunchKernelGGL(fl_tile_kernel<FL_ROPE>, grid, dim3(64), 0, stream, wp, tp, out, m, k);
-  else hipLaunchKernelGGL(fl_tile_kernel<FL_PARTS>, grid, dim3(64), 0, stream, wp, tp, out, m, k);
+#define KLLM_FLT(T)                                                                                                         \
+  do {                                                                                                                     \
+    const T* wp = (const T*)w;                                                                                             \
+    T* tp = (T*)wt;                                                                                                        \
+    if (kind == FL_SWIGLU) hipLaunchKernelGGL((fl_tile_kernel<T, FL_SWIGLU>), grid, dim3(64), 0, stream, wp, tp, out, m, k); \
+    else if (kind == FL_ROPE) hipLaunchKernelGGL((fl_tile_kernel<T, FL_ROPE>), grid, dim3(64), 0, stream, wp, tp, out, m, k); \
+    else hipLaunchKernelGGL((fl_tile_kernel<T, FL_PARTS>), grid, dim3(64), 0, stream, wp, tp, out, m, k);                    \
+  } while (0)
+  if (f32) KLLM_FLT(float); else KLLM_FLT(bf16_t);
+#undef KLLM_FLT
   KLLM_CHECK_LAUNCH("fused_linear_tile");
   return 0;
 }
@@ -654,9 +702,10 @@ extern "C" int kllm_fused_linear_tile(const void* w, void* wt, int kind, int m, 
 extern "C" int kllm_fused_linear(const void* x, int x_stride, const KllmLinearOut* yout, const void* w,
                                  int n, int m, int k, int tiles_per_wg, hipStream_t stream) {
   KLLM_REQUIRE(x && yout && w && yout->y, "fused_linear: null pointer");
-  KLLM_REQUIRE(n > 0 && n <= KLLM_FUSED_LINEAR_MAX_ROWS, "fused_linear: n=%d is outside [1, %d]", n,
-               KLLM_FUSED_LINEAR_MAX_ROWS);
-  KLLM_REQUIRE(m > 0 && k > 0 && k % 8 == 0, "fused_linear: bad sizes m=%d k=%d (K must be a multiple of 8)", m, k);
+  const bool f32 = yout->f32 != 0;
+  const int e = f32 ? 4 : 8;
+  KLLM_REQUIRE(n > 0 && n <= fl_max_rows(f32), "fused_linear: n=%d is outside [1, %d]", n, fl_max_rows(f32));
+  KLLM_REQUIRE(m > 0 && k > 0 && k % e == 0, "fused_linear: bad sizes m=%d k=%d (K must be a multiple of %d)", m, k, e);
   KLLM_REQUIRE((long)m * k < (1L << 40) && m < (1 << 30), "fused_linear: sizes overflow");
   KLLM_REQUIRE(fl_aligned16(w) && fl_aligned16(x), "fused_linear: operands must be 16-byte aligned");
   KLLM_REQUIRE(tiles_per_wg >= 1 && tiles_per_wg <= 64, "fused_linear: %d tiles per workgroup", tiles_per_wg);
@@ -669,14 +718,14 @@ extern "C" int kllm_fused_linear(const void* x, int x_stride, const KllmLinearOu
   const int kslice = ceil_div(ceil_div(k, nsplit), 32) * 32;
   KLLM_REQUIRE((long)kslice * (nsplit - 1) < k, "fused_linear: nsplit %d leaves an empty slice of K=%d", nsplit, k);
   const int nt = ceil_div(n, 16);
-  const int kpass = fl_pass_k(n, kslice);
+  const int kpass = fl_pass_k(f32, n, kslice);
   KLLM_REQUIRE(kpass > 0, "fused_linear: %d rows of K=%d need %zu bytes of LDS, more than %d even in %d passes", n,
-               kslice, fl_lds_bytes(n, nt, kslice), FL_LDS_MAX, FL_MAX_PASSES);
+               kslice, fl_lds_bytes(f32, n, nt, kslice), FL_LDS_MAX, FL_MAX_PASSES);
   KLLM_REQUIRE(kpass >= kslice || tiles_per_wg == 1,
                "fused_linear: %d rows of K=%d do not fit into LDS at once; in passes a workgroup takes one tile, not %d",
                n, kslice, tiles_per_wg);
   if (x_stride <= 0) x_stride = k;
-  KLLM_REQUIRE(x_stride >= k && x_stride % 8 == 0, "fused_linear: row stride %d of x does not fit K=%d", x_stride, k);
+  KLLM_REQUIRE(x_stride >= k && x_stride % e == 0, "fused_linear: row stride %d of x does not fit K=%d", x_stride, k);
 
   FlOut out = {};
   out.y = yout->y;
@@ -736,10 +785,11 @@ extern "C" int kllm_fused_linear(const void* x, int x_stride, const KllmLinearOu
     out.KV = KV;
     out.hd = hd;
   }
-  const int nw = fl_waves(ep, n, kslice, kpass, ceil_div(tiles, tiles_per_wg) * nsplit, tiles_per_wg);
-  const int kpass_run = nw == 4 ? kpass : fl_pass_k(n, kslice, nw);    // eight waves' partial tiles take room from the rows
-  const int rc = nt == 1 ? fl_launch_ep<1>(ep, scaled, nw, x, out, w, n, m, k, kslice, kpass_run, nsplit, tiles, tiles_per_wg, x_stride, stream)
-                         : fl_launch_ep<2>(ep, scaled, nw, x, out, w, n, m, k, kslice, kpass_run, nsplit, tiles, tiles_per_wg, x_stride, stream);
+  const int nw = fl_waves(f32, ep, n, kslice, kpass, ceil_div(tiles, tiles_per_wg) * nsplit, tiles_per_wg);
+  const int kpass_run = nw == 4 ? kpass : fl_pass_k(f32, n, kslice, nw);    // eight waves' partial tiles take room from the rows
+  const int rc = f32 ? fl_launch_ep<float, 1>(ep, scaled, nw, x, out, w, n, m, k, kslice, kpass_run, nsplit, tiles, tiles_per_wg, x_stride, stream)
+                 : nt == 1 ? fl_launch_ep<bf16_t, 1>(ep, scaled, nw, x, out, w, n, m, k, kslice, kpass_run, nsplit, tiles, tiles_per_wg, x_stride, stream)
+                         : fl_launch_ep<bf16_t, 2>(ep, scaled, nw, x, out, w, n, m, k, kslice, kpass_run, nsplit, tiles, tiles_per_wg, x_stride, stream);
   if (rc) return rc;
   KLLM_CHECK_LAUNCH("fused_linear");
   return 0;

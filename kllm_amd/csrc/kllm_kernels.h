@@ -146,7 +146,7 @@ int kllm_gemv_rope_append(const void* x, const void* w_qkv, void* q_out, const f
                           int page_size, int n, int H, int KV, int hd, int k, int dtype,
                           const KllmNormedInput* normed, hipStream_t stream);
 
-/* Products of a decode batch (bfloat16, up to KLLM_FUSED_LINEAR_MAX_ROWS rows)
+/* Products of a decode batch (bfloat16, up to KLLM_FUSED_LINEAR_MAX_ROWS rows; float32, up to 16)
  * on the matrix cores, fused with the step after them.  x is [n][k] with a row
  * stride of x_stride elements (0 = k), w is [m][k].  Output:
  *   PARTS   y float32 [nsplit][n][m]; only this one may split K
@@ -189,20 +189,21 @@ typedef struct {
   int ss_parts;
   float eps;
   int tiled;            /* w is the copy that kllm_fused_linear_tile made of the weights for this kind */
+  int f32;              /* x, w, y (but PARTS) and the cache are float32, not bfloat16; up to 16 rows */
 } KllmLinearOut;
-long kllm_fused_linear_lds_bytes(int n, int k, int nsplit);
+long kllm_fused_linear_lds_bytes(int n, int k, int nsplit, int dtype);
 /* Where that is more than LDS holds, the rows are staged and multiplied in passes over K, with
  * one tile to a workgroup (tiles_per_wg = 1): how many passes a call needs (1: all at once; 0:
  * the kernel does not take the sizes). */
-int kllm_fused_linear_passes(int n, int k, int nsplit);
+int kllm_fused_linear_passes(int n, int k, int nsplit, int dtype);
 /* A copy of w[m][k] in the order the kernel's lanes read it (a load instruction then reads one
  * contiguous kilobyte instead of 64 bytes of each of 16 rows: weights stream 20-30 % faster),
  * for one output kind (PARTS and RESID share theirs; ROPE with the heads it will be called
  * with, with_kv: whether k and v rows follow q's): wt holds
- * kllm_fused_linear_tiled_elements(kind, m, k) elements.  Pass it as w with out->tiled = 1. */
-long kllm_fused_linear_tiled_elements(int kind, int m, int k);
-int kllm_fused_linear_tile(const void* w, void* wt, int kind, int m, int k, int H, int KV, int hd, int with_kv,
-                           hipStream_t stream);
+ * kllm_fused_linear_tiled_elements(kind, m, k, dtype) elements.  Pass it as w with out->tiled = 1. */
+long kllm_fused_linear_tiled_elements(int kind, int m, int k, int dtype);
+int kllm_fused_linear_tile(const void* w, void* wt, int kind, int m, int k, int dtype, int H, int KV, int hd,
+                           int with_kv, hipStream_t stream);
 int kllm_fused_linear_resid_parts(int m, int tiles_per_wg);
 int kllm_fused_linear_max_parts(void);
 int kllm_fused_linear(const void* x, int x_stride, const KllmLinearOut* out, const void* w, int n, int m,

@@ -21,7 +21,7 @@ import torch
 DT_F32, DT_BF16 = 0, 1
 GEMM_PLAIN, GEMM_TILED_F32, GEMM_MFMA_BF16, GEMM_SKINNY_BF16, GEMM_GEMV, GEMM_GEMV_LDS, GEMM_MFMA_F32 = 0, 1, 2, 3, 4, 5, 6
 GEMV_BEST_ROWS = 0         # rows up to which they beat the MFMA kernels in bfloat16: none (a step at 1.1B sizes, one token: 1.036 against 0.963 ms)
-ABI_VERSION = 16
+ABI_VERSION = 17
 
 
 class KernelError(RuntimeError):
@@ -106,8 +106,8 @@ def _declare(lib):
         "kllm_gemv_resid_parts": [I],
         "kllm_fused_linear": [P, I, P, P, I, I, I, I, P],
         "kllm_fused_linear_resid_parts": [I, I],
-        "kllm_fused_linear_passes": [I, I, I],
-        "kllm_fused_linear_tile": [P, P, I, I, I, I, I, I, I, P],
+        "kllm_fused_linear_passes": [I, I, I, I],
+        "kllm_fused_linear_tile": [P, P, I, I, I, I, I, I, I, I, P],
         "kllm_command_op": [c_char_p],
         "kllm_command_nargs": [I],
         "kllm_run_commands": [P, L, P, P],
@@ -184,9 +184,9 @@ def _declare(lib):
         fn.restype = c_int
     lib.kllm_decayed_segment_floats.argtypes = [I, I, I, I, I]
     lib.kllm_decayed_segment_floats.restype = L
-    lib.kllm_fused_linear_lds_bytes.argtypes = [I, I, I]
+    lib.kllm_fused_linear_lds_bytes.argtypes = [I, I, I, I]
     lib.kllm_fused_linear_lds_bytes.restype = L
-    lib.kllm_fused_linear_tiled_elements.argtypes = [I, I, I]
+    lib.kllm_fused_linear_tiled_elements.argtypes = [I, I, I, I]
     lib.kllm_fused_linear_tiled_elements.restype = L
 
 
@@ -829,7 +829,7 @@ class _LinearOut(ctypes.Structure):
                 ("kind", c_int), ("nsplit", c_int), ("max_pages", c_int), ("page_size", c_int),
                 ("H", c_int), ("KV", c_int), ("hd", c_int), ("act", c_int),
                 ("resid", c_void_p), ("norm_w", c_void_p), ("ss_out", c_void_p), ("ss_in", c_void_p),
-                ("ss_parts", c_int), ("eps", c_float), ("tiled", c_int)]
+                ("ss_parts", c_int), ("eps", c_float), ("tiled", c_int), ("f32", c_int)]
 
 
 FUSED_LINEAR_MAX_ROWS = 32
@@ -861,12 +861,11 @@ def fused_tiles_per_wg(n, m, k) -> int:
 
 
 @functools.lru_cache(maxsize=4096)
-def fused_linear_fits(n, k, nsplit=1) -> bool:
-    """Whether the decode-batch products take n rows of K: bfloat16 only, K a
-    multiple of 8, and all rows of a workgroup's slice of K in LDS."""
-    if n < 1 or n > FUSED_LINEAR_MAX_ROWS or k % 8:
-        return False
-    return 0 < library().kllm_fused_linear_lds_bytes(int(n), int(k), int(nsplit)) <= FUSED_LINEAR_LDS
+def fused_linear_fits(n, k, nsplit=1, dtype=torch.bfloat16) -> bool:
+    """Whether the decode-batch products take n rows of K: K a multiple of 8 (float32: 4), and all
+    rows of a workgroup's slice of K in LDS."""
+    return fused_linear_passes(n, k, nsplit, dtype) > 0 and \
+        0 < library().kllm_fused_linear_lds_bytes(int(n), int(k), int(nsplit), dtype_code(dtype)) <= FUSED_LINEAR_LDS
 
 
 # Passes over K up to which the decode-batch kernel is taken where the rows do not fit into LDS at
@@ -879,20 +878,20 @@ FUSED_LINEAR_PASSES_BEST_ROWS = 16
 
 
 @functools.lru_cache(maxsize=4096)
-def fused_linear_passes(n, k, nsplit=1) -> int:
+def fused_linear_passes(n, k, nsplit=1, dtype=torch.bfloat16) -> int:
     """Passes over K in which the decode-batch products take n rows: 1 where all rows of a
     workgroup's slice of K fit into LDS (``fused_linear_fits``); more, with one tile to a
     workgroup, where they do not; 0 if the kernel does not take the sizes."""
-    if n < 1 or n > FUSED_LINEAR_MAX_ROWS or k % 8:
+    if n < 1 or n > FUSED_LINEAR_MAX_ROWS or k % (4 if dtype == torch.float32 else 8):
         return 0
-    return int(library().kllm_fused_linear_passes(int(n), int(k), int(nsplit)))
+    return int(library().kllm_fused_linear_passes(int(n), int(k), int(nsplit), dtype_code(dtype)))
 
 
-def fused_linear_tiles(n, m, k) -> int:
+def fused_linear_tiles(n, m, k, dtype=torch.bfloat16) -> int:
     """Tiles per workgroup with which the decode-batch kernel is taken for n rows against
     w [m, k] (``fused_tiles_per_wg`` where the rows fit into LDS at once, one where they go in
     a few passes over K), or 0 where it is not taken."""
-    passes = fused_linear_passes(n, k)
+    passes = fused_linear_passes(n, k, 1, dtype)
     if passes == 0 or (passes > 1 and (passes > FUSED_LINEAR_BEST_PASSES or n > FUSED_LINEAR_PASSES_BEST_ROWS)):
         return 0
     return fused_tiles_per_wg(n, m, k) if passes == 1 else 1
@@ -909,29 +908,30 @@ class TiledWeights:
 
 
 def fused_linear_tile(w, kind, rope=None):
-    """The tiled copy of ``w`` [m, k] (bfloat16, k a multiple of 8) for ``kind``; ``rope`` as
+    """The tiled copy of ``w`` [m, k] (k a multiple of 8, float32: of 4) for ``kind``; ``rope`` as
     for ``fused_linear`` (its heads and whether a cache is written decide the rows' order)."""
     m, k = w.shape
-    if w.dtype != torch.bfloat16 or k % 8:
-        raise KernelError("fused_linear_tile: bfloat16 weights with K a multiple of 8 only")
+    code = dtype_code(w.dtype)
+    if k % (4 if w.dtype == torch.float32 else 8):
+        raise KernelError("fused_linear_tile: K a multiple of 8 (float32: 4) only")
     base = LINEAR_PARTS if kind == LINEAR_RESID else kind
-    count = library().kllm_fused_linear_tiled_elements(base, m, k)
+    count = library().kllm_fused_linear_tiled_elements(base, m, k, code)
     if count <= 0:
         raise KernelError(f"fused_linear_tile: sizes {m} x {k} are not taken")
-    out = torch.empty(count, dtype=torch.bfloat16, device=w.device)
+    out = torch.empty(count, dtype=w.dtype, device=w.device)
     heads = (0, 0, 0, 0)
     if base == LINEAR_ROPE:
         if rope is None:
             raise KernelError("fused_linear_tile: the rope kind needs its heads")
         heads = (rope.heads, rope.kv_heads, rope.head_dim, int(rope.cache is not None))
-    _check(library().kllm_fused_linear_tile(_ptr(w, "tile w"), _ptr(out, "tile out"), base, m, k, *heads, _stream()),
+    _check(library().kllm_fused_linear_tile(_ptr(w, "tile w"), _ptr(out, "tile out"), base, m, k, code, *heads, _stream()),
            "fused_linear_tile")
     return TiledWeights(out, base, m, k, heads)
 
 
 class ScaledRows:
     """The input of a decode batch's product as a residual product (LINEAR_RESID) left it:
-    ``xw`` [n, k] bfloat16, the residual stream's rows times the norm's weight, and ``ss``
+    ``xw`` [n, k] in the compute dtype, the residual stream's rows times the norm's weight, and ``ss``
     [n, parts rounded up to 4] float32, partial sums of squares of the stream's rows.  The
     consuming product multiplies its sums by rsqrt(sum of a row's ss / k + eps)."""
 
@@ -944,10 +944,10 @@ class ScaledRows:
 
 
 @functools.lru_cache(maxsize=4096)
-def fused_resid_parts(n, m, k, tiles_per_wg=1) -> int:
+def fused_resid_parts(n, m, k, tiles_per_wg=1, dtype=torch.bfloat16) -> int:
     """Partial sums of squares per row that a LINEAR_RESID product of these sizes leaves, or 0
     if the decode-batch kernel does not take them."""
-    passes = fused_linear_passes(n, k)
+    passes = fused_linear_passes(n, k, 1, dtype)
     if passes == 0 or (passes > 1 and tiles_per_wg != 1):
         return 0
     parts = library().kllm_fused_linear_resid_parts(int(m), int(tiles_per_wg))
@@ -969,9 +969,9 @@ FUSED_LINEAR_UNARY = 16    # LINEAR_PARTS with act = this + an activation withou
 
 def fused_linear(w, y, kind, x, nsplit=1, tiles_per_wg=1, rope=None, act=ACT_SILU, resid=None, norm_weight=None,
                  ss_out=None, unary=None):
-    """One launch for a decode batch's product of x [n, k] (bfloat16; a view
+    """One launch for a decode batch's product of x [n, k] (bfloat16, or float32 up to 16 rows; a view
     with a row stride is taken) with w [m, k], and the step after it, by
-    ``kind``: LINEAR_PARTS y float32 [nsplit, n, m]; LINEAR_SWIGLU y bfloat16
+    ``kind`` (bfloat16 below is the operands' type): LINEAR_PARTS y float32 [nsplit, n, m]; LINEAR_SWIGLU y bfloat16
     [n, m/2]; LINEAR_ROPE y = q_out with ``rope`` describing rotation and
     cache; LINEAR_RESID adds the product to ``resid`` [n, m] float32 in place, writes
     y bfloat16 [n, m] = the new rows times ``norm_weight`` [m] and leaves partial sums of
@@ -981,8 +981,8 @@ def fused_linear(w, y, kind, x, nsplit=1, tiles_per_wg=1, rope=None, act=ACT_SIL
     y bfloat16 [n, m] = activation(sums), one slice."""
     m, k = w.shape
     lo = _LinearOut()
-    if w.dtype != torch.bfloat16:
-        raise KernelError("fused_linear: bfloat16 weights only")
+    typ = w.dtype
+    lo.f32 = int(dtype_code(typ) == DT_F32)
     if isinstance(w, TiledWeights):
         if w.kind != (LINEAR_PARTS if kind == LINEAR_RESID else kind):
             raise KernelError(f"fused_linear: the tiled weights were made for output kind {w.kind}, not {kind}")
@@ -999,20 +999,20 @@ def fused_linear(w, y, kind, x, nsplit=1, tiles_per_wg=1, rope=None, act=ACT_SIL
         lo.ss_in, lo.ss_parts, lo.eps = _ptr(sr.ss, "fused_linear ss", torch.float32), sr.parts, sr.eps
     n = x.shape[0]
     lo.kind, lo.nsplit, lo.act = kind, nsplit, int(act)
-    if x.dim() != 2 or x.shape[1] != k or x.dtype != torch.bfloat16 or x.stride(1) != 1 or not x.is_cuda:
+    if x.dim() != 2 or x.shape[1] != k or x.dtype != typ or x.stride(1) != 1 or not x.is_cuda:
         raise KernelError(f"fused_linear: x {tuple(x.shape)} {x.dtype} does not fit w {tuple(w.shape)}")
     x_ptr, x_stride = x.data_ptr(), (x.stride(0) if n > 1 else k)
     if kind == LINEAR_PARTS and unary is not None:
         code, params = unary
         if nsplit != 1 or (code == ACT_XIELU and (params is None or params.numel() != 2)):
             raise KernelError("fused_linear: an activation on the sums takes one slice, and xielu its two constants")
-        want, dt = (n, m), torch.bfloat16
+        want, dt = (n, m), typ
         lo.act = FUSED_LINEAR_UNARY + int(code)
         lo.norm_w = _ptr(params, "fused_linear activation constants", torch.float32, True)
     elif kind == LINEAR_PARTS:
         want, dt = (nsplit, n, m), torch.float32
     elif kind == LINEAR_RESID:
-        want, dt = (n, m), torch.bfloat16
+        want, dt = (n, m), typ
         parts = library().kllm_fused_linear_resid_parts(int(m), int(tiles_per_wg))
         if (resid is None or norm_weight is None or ss_out is None or tuple(resid.shape) != (n, m)
                 or norm_weight.numel() != m or tuple(ss_out.shape) != (n, -(-parts // 4) * 4)):
@@ -1022,11 +1022,11 @@ def fused_linear(w, y, kind, x, nsplit=1, tiles_per_wg=1, rope=None, act=ACT_SIL
         lo.norm_w = _ptr(norm_weight, "fused_linear norm weight", torch.float32)
         lo.ss_out = _ptr(ss_out, "fused_linear ss_out", torch.float32)
     elif kind == LINEAR_SWIGLU:
-        want, dt = (n, m // 2), torch.bfloat16
+        want, dt = (n, m // 2), typ
     elif kind == LINEAR_ROPE:
         if rope is None:
             raise KernelError("fused_linear: the rope epilogue needs its description")
-        want, dt = (n, rope.heads * rope.head_dim), torch.bfloat16
+        want, dt = (n, rope.heads * rope.head_dim), typ
         half = rope.head_dim // 2
         if rope.cos is not None and (tuple(rope.cos.shape) != (n, half) or tuple(rope.sin.shape) != (n, half)):
             raise KernelError("fused_linear: cos/sin shapes do not fit")
@@ -1034,7 +1034,7 @@ def fused_linear(w, y, kind, x, nsplit=1, tiles_per_wg=1, rope=None, act=ACT_SIL
         lo.sin_t = _ptr(rope.sin, "fused_linear sin", torch.float32, True)
         if rope.cache is not None:
             if (tuple(rope.cache.shape[1:]) != (2, rope.kv_heads, rope.page_size * rope.head_dim)
-                    or rope.cache.dtype != torch.bfloat16):
+                    or rope.cache.dtype != typ):
                 raise KernelError(f"fused_linear: cache {tuple(rope.cache.shape)} {rope.cache.dtype} does not fit")
             if rope.positions.numel() < n or rope.span_of_token.numel() < n:
                 raise KernelError("fused_linear: index arrays are too short")

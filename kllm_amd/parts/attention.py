@@ -30,7 +30,7 @@ import torch
 
 from .. import kernels as K
 from .base import Normed, Part, register_part
-from .linear import decode_linear, linear, linear_into, tiled_copy
+from .linear import decode_linear, fused_f32, linear, linear_into, tiled_copy
 from .spec import CacheNeed, WeightSpec
 
 
@@ -193,10 +193,11 @@ class CausalSelfAttention(Part):
     def _fused_tiles(self, n):
         """Tiles per workgroup of the decode-batch kernel for the input projections of n
         tokens, or 0 where it is not taken."""
-        if (self.runtime.dtype != torch.bfloat16 or n > K.FUSED_ROPE_BEST_ROWS or not self.plain_rotation
-                or self.runtime.options.get("no_fused_linear")):
+        rt = self.runtime
+        best = fused_f32(rt, n) if rt.dtype == torch.float32 else n <= K.FUSED_ROPE_BEST_ROWS
+        if not best or not self.plain_rotation or rt.options.get("no_fused_linear"):
             return 0
-        return K.fused_linear_tiles(n, self.w_in.shape[0], self.hidden)
+        return K.fused_linear_tiles(n, self.w_in.shape[0], self.hidden, rt.dtype)
 
     def forward(self, ctx, xn, cache, sink=None):
         dtype = self.runtime.dtype

@@ -13,7 +13,7 @@ import torch
 
 from .. import kernels as K
 from .base import Normed, Part, register_part
-from .linear import decode_batch_fits, decode_linear, linear, linear_into, tiled_copy
+from .linear import decode_batch_fits, decode_linear, fused_f32, linear, linear_into, tiled_copy
 from .spec import WeightSpec
 
 
@@ -64,10 +64,10 @@ class GatedFeedForward(Part):
         dtype, opts = self.runtime.dtype, self.runtime.options
         n = xn.rows if isinstance(xn, Normed) else xn.shape[0]
         gemv = K.gemv_fits(n, 2 * self.intermediate, self.hidden, dtype) and not opts.get("no_fused_gemv")
-        if gemv and isinstance(xn, Normed) and xn.xw is not None:
+        best = fused_f32(self.runtime, n) if dtype == torch.float32 else n <= K.FUSED_SWIGLU_BEST_ROWS
+        tiles = K.fused_linear_tiles(n, 2 * self.intermediate, self.hidden, dtype) if best else 0
+        if gemv and (isinstance(xn, Normed) and xn.xw is not None or dtype == torch.float32 and tiles > 0):
             gemv = False       # the producer was the decode-batch kernel: its consumer is, too
-        tiles = (K.fused_linear_tiles(n, 2 * self.intermediate, self.hidden)
-                 if dtype == torch.bfloat16 and n <= K.FUSED_SWIGLU_BEST_ROWS else 0)
         fused = not gemv and tiles > 0 and not opts.get("no_fused_linear")
         if isinstance(xn, Normed):     # the small-batch kernel below normalises while it stages its input,
             # the decode-batch kernel scales its sums by the row
@@ -148,7 +148,7 @@ def dense_hidden(ctx, xn, w_up, tag, tiled, act, params=None):
     if (n > 128 and opts.get("gemm") != "library" and opts.get("gemm_algo") is None
             and xn.shape[1] % (8 if xn.dtype == torch.bfloat16 else 4) == 0):
         K.gemm_act(xn, w_up, h, act, params)      # prompts
-    elif decode_batch_fits(xn) and not opts.get("no_fused_linear") and opts.get("gemm_algo") is None:
+    elif decode_batch_fits(ctx.runtime, xn) and not opts.get("no_fused_linear") and opts.get("gemm_algo") is None:
         h = decode_linear(ctx, xn, w_up, tag + ".h", tiled, unary=(act, params))      # decode batches
     else:
         K.unary_act(decode_linear(ctx, xn, w_up, tag + ".up", tiled), h, act, params)

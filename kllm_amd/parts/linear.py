@@ -6,7 +6,8 @@ rotary + append, SiLU gate); with the compute dtype as result it returns
 [n, m].  Which kernel runs depends only on the dtype and on n:
 
   n <= 8    float32: gemv with X in LDS and the whole of K in one wave (no
-            partial sums), if the sizes fit; bfloat16 up to 4 rows: the streaming
+            partial sums), if the sizes fit, and from five rows on the decode-batch kernel
+            (``fused_f32``) where its epilogue or one whole result is wanted; bfloat16 up to 4 rows: the streaming
             gemv, K cut into slices for long rows (measured faster than the
             former for a plain product; the fused epilogues are another matter)
   float32   else: MFMA tiles with 32-bit operands (true 32-bit; K in slices for
@@ -131,18 +132,18 @@ def choose(dtype, n, m, k, options=None):
 
 
 @functools.lru_cache(maxsize=4096)
-def _resid_tiles(n, m, k):
+def _resid_tiles(n, m, k, dtype=torch.bfloat16):
     """(tiles per workgroup, partial sums of squares per row) of a decode batch's residual
     product: as few tiles to a workgroup as keep the sums of squares within what the
     consumer reads (one tile where the rows go through LDS in passes over K); (1, 0) if the
     kernel does not take the sizes."""
-    passes = K.fused_linear_passes(n, k)
+    passes = K.fused_linear_passes(n, k, 1, dtype)
     if passes == 0 or (passes > 1 and (passes > K.FUSED_LINEAR_BEST_PASSES or n > K.FUSED_LINEAR_PASSES_BEST_ROWS)):
         return 1, 0
     tpw = 1
-    while K.fused_resid_parts(n, m, k, tpw) == 0 and tpw < 64 and passes == 1:
+    while K.fused_resid_parts(n, m, k, tpw, dtype) == 0 and tpw < 64 and passes == 1:
         tpw *= 2
-    return tpw, K.fused_resid_parts(n, m, k, tpw)
+    return tpw, K.fused_resid_parts(n, m, k, tpw, dtype)
 
 
 def tiled_copy(runtime, w, kind, rope=None):
@@ -150,25 +151,43 @@ def tiled_copy(runtime, w, kind, rope=None):
     (``K.fused_linear_tile``), or None where that kernel does not run: other dtypes, sizes it
     does not take, or ``EngineOptions.extra["no_tiled_weights"]`` (the copies double the
     memory of the weights they are made of; decode batches of 2 to 16 tokens stream them 20 to
-    30 % faster than the row-major matrix)."""
-    if (w is None or w.dtype != torch.bfloat16 or not w.is_cuda or w.shape[1] % 8
+    30 % faster than the row-major matrix).  float32: ``_room_for_copy``."""
+    if (w is None or not w.is_cuda or w.shape[1] % (4 if w.dtype == torch.float32 else 8)
             or runtime.options.get("no_tiled_weights") or runtime.options.get("no_fused_linear")):
+        return None
+    if w.dtype == torch.float32 and (runtime.options.get("no_mfma_f32") or not _room_for_copy(w)):
         return None
     return K.fused_linear_tile(w, kind, rope)
 
 
+def _room_for_copy(w):
+    """Whether half of the card's memory stays free behind a copy of w: a float32 model that fills
+    more of it runs from the row-major matrices alone (5 to 16 tokens at 1.1B sizes: 1.76 to 1.97 ms a step
+    without the copies, 1.66 to 1.83 with them; the sums are the same)."""
+    free, total = torch.cuda.mem_get_info(w.device)
+    return free - w.numel() * w.element_size() >= total // 2
+
+
+def fused_f32(rt, n):
+    """Whether a float32 decode batch of n tokens runs on the decode-batch kernel: up to four rows the
+    gemv with the same epilogues has the rows in registers and is the faster one (a step in ms, gemv
+    against this kernel, of 3 / 4 tokens at 1.1B sizes: 1.69 against 1.68, 1.70 against 1.64; of 4 at 8B sizes:
+    6.70 against 6.97); from five on its work per weight grows with the rows and the matrix cores' does not
+    (5 / 8 tokens at 1.1B sizes: 2.07 against 1.73, 2.14 against 1.70; 8 at 8B sizes: 8.41 against 7.82), and
+    from nine on K went in slices whose sums other kernels added (10 / 16 tokens: 2.93 against 1.66, 3.06
+    against 1.83; 16 at 8B sizes: 14.6 against 9.7)."""
+    opts = rt.options
+    return (5 <= n <= 16 and not opts.get("no_fused_linear") and not opts.get("no_mfma_f32")
+            and opts.get("gemm_algo") is None)
+
+
 def linear_into(ctx, x, w, sink, tag, w_tiled=None):
     """x . w^T added to the residual stream of ``sink`` in the product's own
-    epilogue, for up to four tokens: returns the ``Normed`` that stands for the
-    norm behind the addition, or None if the kernel with that epilogue does
-    not take these sizes (the caller then returns the product and the norm
-    adds it).  Measured at width 2048: 4 % of a decode step at one token; for
-    decode batches on the matrix cores the same was built and lost 4 % at
-    eight tokens (every workgroup of the consuming product then stages 72 KB
-    of float32 rows where it staged 32 KB of bfloat16), so it stops at four; in
-    float32, where rows are staged in 32 bits either way, the kernels for eight
-    rows with these epilogues are the slower ones (2.53 against 2.27 ms a step
-    at five to eight tokens)."""
+    epilogue: returns the ``Normed`` that stands for the norm behind the addition, or None
+    if no kernel with that epilogue takes these sizes (the caller then returns the product
+    and the norm adds it).  Up to four tokens on the gemv, whose consumer normalises the
+    float32 rows as it stages them (4 % of a step of one token at width 2048); decode batches on
+    the matrix cores, whose consumer scales its sums by the row instead."""
     from .base import Normed
     n, k = x.shape
     m = w.shape[0]
@@ -180,20 +199,21 @@ def linear_into(ctx, x, w, sink, tag, w_tiled=None):
     norm = sink.norm
     if tuple(sink.x.shape) != (n, m) or norm.weight is None or norm.weight.numel() != m:
         return None
-    parts = K.resid_parts(n, m, k, x.dtype)
+    f32 = x.dtype == torch.float32
+    parts = 0 if f32 and fused_f32(rt, n) else K.resid_parts(n, m, k, x.dtype)
     if parts:
         ss = ctx.buf(tag + ".ss", (n, -(-parts // 4) * 4), torch.float32)
         K.linear_resid(x, w, sink.x, ss)
         return Normed(sink.x, ss, parts, norm)
-    if x.dtype != torch.bfloat16 or n > K.FUSED_NORM_BEST_ROWS or rt.options.get("no_fused_linear"):
+    if not (fused_f32(rt, n) if f32 else n <= K.FUSED_NORM_BEST_ROWS) or rt.options.get("no_fused_linear"):
         return None
     # a decode batch on the matrix cores: all of K in a workgroup, the addition in the epilogue, and
-    # beside the stream its rows times the norm's weight in 16 bits for a consumer that scales its sums
-    tpw, parts = _resid_tiles(n, m, k)
+    # beside the stream its rows times the norm's weight in the compute dtype for a consumer that scales its sums
+    tpw, parts = _resid_tiles(n, m, k, x.dtype)
     if parts == 0:
         return None
     ss = ctx.buf(tag + ".ss", (n, -(-parts // 4) * 4), torch.float32)
-    xw = ctx.buf(tag + ".xw", (n, m), torch.bfloat16)
+    xw = ctx.buf(tag + ".xw", (n, m), x.dtype)
     K.fused_linear(w_tiled if w_tiled is not None else w, xw, K.LINEAR_RESID, x=x, tiles_per_wg=tpw, resid=sink.x,
                    norm_weight=norm.weight, ss_out=ss)
     return Normed(sink.x, ss, parts, norm, xw=xw)
@@ -209,8 +229,9 @@ def linear(ctx, x, w, tag, out_dtype=torch.float32, split=True, w_tiled=None):
     rt = ctx.runtime
     algo, nsplit = choose(x.dtype, n, m, k, rt.options)
     whole = not split or out_dtype != torch.float32
-    if (algo == K.GEMM_SKINNY_BF16 and whole and out_dtype == torch.float32 and n <= 16
-            and K.fused_linear_fits(n, k) and not rt.options.get("no_fused_linear")):
+    if ((algo == K.GEMM_SKINNY_BF16 or (algo == K.GEMM_MFMA_F32 and fused_f32(rt, n))) and whole
+            and out_dtype == torch.float32 and n <= 16 and K.fused_linear_fits(n, k, 1, x.dtype)
+            and not rt.options.get("no_fused_linear")):
         # one float32 result from a decode batch (the logits): all of K in one workgroup, so
         # that no partial sums have to be added afterwards
         y = ctx.buf(tag, (1, n, m), torch.float32)
@@ -247,11 +268,13 @@ def linear(ctx, x, w, tag, out_dtype=torch.float32, split=True, w_tiled=None):
     return y
 
 
-def decode_batch_fits(x):
-    """Whether a product of these rows runs on the decode-batch kernel (bfloat16, up to 16 rows,
-    all of K in a workgroup)."""
+def decode_batch_fits(rt, x):
+    """Whether a product of these rows runs on the decode-batch kernel (up to 16 rows, all of K
+    in a workgroup; float32 see ``fused_f32``)."""
     n, k = x.shape
-    return x.dtype == torch.bfloat16 and n <= 16 and k % 8 == 0 and K.fused_linear_fits(n, k)
+    if x.dtype == torch.float32 and not fused_f32(rt, n):
+        return False
+    return n <= 16 and K.fused_linear_fits(n, k, 1, x.dtype)
 
 
 def decode_linear(ctx, x, w, tag, w_tiled=None, unary=None):
@@ -259,13 +282,13 @@ def decode_linear(ctx, x, w, tag, w_tiled=None, unary=None):
     batches of up to 16 rows run on the decode-batch kernel with all of K in a workgroup (one
     result, from the tiled copy of w where there is one); everything else as ``linear`` cuts it.
     ``unary`` = (activation without a gate, its constants): only where ``decode_batch_fits``;
-    the result is then the activation of the sums in bfloat16."""
+    the result is then the activation of the sums in the compute dtype."""
     n, m = x.shape[0], w.shape[0]
     rt = ctx.runtime
-    if decode_batch_fits(x) and not rt.options.get("no_fused_linear") and rt.options.get("gemm_algo") is None:
+    if decode_batch_fits(rt, x) and not rt.options.get("no_fused_linear") and rt.options.get("gemm_algo") is None:
         tiles = 4 if m >= 16384 else 1
         if unary is not None:
-            y = ctx.buf(tag, (n, m), torch.bfloat16)
+            y = ctx.buf(tag, (n, m), x.dtype)
             K.fused_linear(w_tiled if w_tiled is not None else w, y, K.LINEAR_PARTS, x=x, tiles_per_wg=tiles, unary=unary)
             return y
         y = ctx.buf(tag, (1, n, m), torch.float32)

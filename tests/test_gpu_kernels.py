@@ -789,6 +789,81 @@ def test_fused_linear_rope_append_with_tiled_weights(H, KV, hd, ps, d):
                         rope=k_.Rope(cos, sin, got[0][1], pos, sot, bt, ps, H, KV, hd))
 
 
+@pytest.mark.parametrize("n,m,k,tpw", [(1, 48, 64, 1), (3, 72, 84, 1), (5, 100, 260, 3), (8, 2048, 5632, 1), (9, 2048, 2048, 2),
+                                       (13, 36, 3076, 1), (16, 520, 1000, 4), (16, 256, 11008, 1)])
+def test_fused_linear_float32(n, m, k, tpw):
+    """The decode-batch kernel on 32-bit operands (K no multiple of a step of 16, rows of W no multiple of 16,
+    several tiles to a workgroup, rows in one pass over K and in several), every output kind, from the matrix and
+    from its tiled copy, against float64.  A sum of K products in at least 64 chains whose results are added in
+    pairs is off by at most K / 64 + 16 roundings of the sum of the products' sizes (8 more for the steps that
+    K is padded to); the epilogues start from what the kernel itself left."""
+    k_ = K()
+    f32, u = torch.float32, 2.0 ** -24
+    x, w = rnd(n, k, seed=1), rnd(m, k, seed=2, scale=0.1)
+
+    def off(a, b, kk):
+        return (kk / 64 + 24) * u * P.linear(a.cpu().double().abs(), b.cpu().double().abs())
+    passes = k_.fused_linear_passes(n, k, 1, f32)
+    assert passes >= 1 and (tpw == 1 or passes == 1)
+    parts, eps = k_.fused_resid_parts(n, m, k, tpw, f32), 1e-5
+    nw, got = 1 + 0.2 * rnd(m, seed=4), []
+    for wt in (w, k_.fused_linear_tile(w, k_.LINEAR_PARTS)):
+        y = torch.full((1, n, m), float("nan"), device=DEV)
+        k_.fused_linear(wt, y, k_.LINEAR_PARTS, x, tiles_per_wg=tpw)
+        stream, xw = rnd(n, m, seed=3, scale=2.0), torch.full((n, m), float("nan"), device=DEV)
+        ss = torch.full((n, -(-parts // 4) * 4), float("nan"), device=DEV)
+        k_.fused_linear(wt, xw, k_.LINEAR_RESID, x, tiles_per_wg=tpw, resid=stream, norm_weight=nw, ss_out=ss)
+        got.append((y, stream, xw, ss[:, :parts].clone()))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+    want, bound = P.linear(x.cpu().double(), w.cpu().double()), off(x, w, k)
+    assert ((y[0].cpu().double() - want).abs() <= bound).all()
+    want = rnd(n, m, seed=3, scale=2.0).cpu().double() + want
+    assert ((stream.cpu().double() - want).abs() <= bound + u * want.abs()).all()
+    assert torch.equal(xw, stream * nw)
+    sq = stream.cpu().double().pow(2).sum(1)
+    assert ((got[0][3].cpu().double().sum(1) - sq).abs() <= (16 * tpw + 8) * u * sq).all()
+    # the consumers: rows times the norm's weight in, the row scale on the sums
+    sr, rows = k_.ScaledRows(xw, ss, parts, eps), xw.cpu().double()
+    scale = (sq / m + eps).rsqrt()[:, None]
+    f = 40
+    wg = rnd(2 * f, m, seed=5, scale=0.1)
+    sums, e = scale * P.linear(rows, wg.cpu().double()), scale * off(xw, wg, m)
+    e = e + 64 * u * sums.abs()
+    g, up = sums[:, :f], sums[:, f:]
+    for wt in (wg, k_.fused_linear_tile(wg, k_.LINEAR_SWIGLU)):
+        h = torch.full((n, f), float("nan"), device=DEV)
+        k_.fused_linear(wt, h, k_.LINEAR_SWIGLU, sr)
+        err = (h.cpu().double() - P.silu(g) * up).abs()
+        assert (err <= 1.2 * (up.abs() * e[:, :f] + P.silu(g).abs() * e[:, f:]) + 64 * u * (P.silu(g) * up).abs() + 1e-12).all()
+    # rotation and append: two query heads and one of keys and values, a token to a page
+    H, KV, hd, ps = 2, 1, 16, 16
+    wq = rnd((H + 2 * KV) * hd, m, seed=6, scale=0.1)
+    pos = torch.arange(5, 5 + n, dtype=torch.int32, device=DEV)
+    sot = torch.arange(n, dtype=torch.int32, device=DEV)
+    bt = (2 * n - torch.arange(2 * n, dtype=torch.int32, device=DEV)).reshape(n, 2)
+    cos, sin = rnd(n, hd // 2, seed=7), rnd(n, hd // 2, seed=8)
+    sums, e = scale * P.linear(rows, wq.cpu().double()), scale * off(xw, wq, m)
+    e = (e + 64 * u * sums.abs()).reshape(n, -1, 2, hd // 2)
+    halves = sums.reshape(n, -1, 2, hd // 2)
+    c, s = cos.cpu().double()[:, None], sin.cpu().double()[:, None]
+    a, b = halves[:, :, 0], halves[:, :, 1]
+    turned = torch.stack([a * c - b * s, b * c + a * s], 2)
+    t_off = torch.stack([e[:, :, 0] * c.abs() + e[:, :, 1] * s.abs(), e[:, :, 1] * c.abs() + e[:, :, 0] * s.abs()], 2)
+    t_off = t_off + 4 * u * torch.stack([a.abs() * c.abs() + b.abs() * s.abs(), b.abs() * c.abs() + a.abs() * s.abs()], 2)
+    for tiled in (False, True):
+        cache, q = torch.zeros((2 * n + 1, 2, KV, ps * hd), device=DEV), torch.full((n, H * hd), float("nan"), device=DEV)
+        rope = k_.Rope(cos, sin, cache, pos, sot, bt, ps, H, KV, hd)
+        k_.fused_linear(k_.fused_linear_tile(wq, k_.LINEAR_ROPE, rope) if tiled else wq, q, k_.LINEAR_ROPE, sr, rope=rope)
+        assert ((q.cpu().double().reshape(n, H, 2, -1) - turned[:, :H]).abs() <= t_off[:, :H]).all()
+        at = torch.arange(n, device=DEV)
+        page, slot = bt[at, (pos // ps).long()].long(), (pos % ps).long()
+        key = cache[page, 0].reshape(n, KV, ps, hd)[at, :, slot].cpu().double().reshape(n, KV, 2, -1)
+        val = cache[page, 1].reshape(n, KV, hd, ps)[at, :, :, slot].cpu().double().reshape(n, KV, 2, -1)
+        assert ((key - turned[:, H:H + KV]).abs() <= t_off[:, H:H + KV]).all()
+        assert ((val - halves[:, H + KV:]).abs() <= e[:, H + KV:]).all()
+        assert int((cache != 0).sum()) == 2 * n * KV * hd
+
+
 def test_fused_linear_resid_refusals():
     k_ = K()
     n, m, k = 4, 64, 64
