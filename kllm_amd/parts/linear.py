@@ -88,7 +88,10 @@ def _decode_tile_split(n, m, k):
     counted in tiles of 64 columns: slices of at least 256 of K until every CU has a workgroup, then
     further ones of at least 512, up to 16 (measured at 64 rows, in us by slices: 2,048 x 5,632:
     14.9 with 4, 10.7 with 8; 11,264 x 2,048: 13.2 with 2, 14.1 with 4, 16.5 with 8; 4,096 x 4,096:
-    12.2 with 4, 10.4 with 8, 11.8 with 16).  Larger weights, in tiles of 128 columns: up to 8 slices
+    12.2 with 4, 10.4 with 8, 11.8 with 16).  Where that stops between two powers and the tiles of 128
+    columns leave CUs idle: as many slices of 512 as there are (2,048 x 5,632 with the norm that adds
+    the slices, 8 / 11 / 15: 17 rows 14.3 / 13.5 / 13.3, 32 rows 14.7 / 14.1 / 14.3, 48 rows 15.5 / 15.0 /
+    15.1; the sums of more slices cost more with every row).  Larger weights, in tiles of 128 columns: up to 8 slices
     of at least 512 of K towards two workgroups a CU, four where K is deep (12,288 x 4,096: 26.2
     with 2, 22.3 with 4, 24.6 with 8; 4,096 x 14,336: 34.4 with 4, 23.9 with 8)."""
     cus, nsplit = K.device_cus(), 1
@@ -96,6 +99,8 @@ def _decode_tile_split(n, m, k):
         tiles = -(-m // 64)
         while nsplit < 16 and ((tiles * nsplit < cus and k // (2 * nsplit) >= 256) or k // (2 * nsplit) >= 512):
             nsplit *= 2
+        if n <= 48 and nsplit < k // 512 <= 16 and -(-m // 128) * (k // 512) <= cus:
+            nsplit = k // 512
     else:
         tiles = -(-m // 128)
         reach = (4 if k >= 8192 and tiles <= cus else 2) * cus

@@ -507,6 +507,21 @@ def test_split_product_into_its_consumers(n, m, k):
     assert (y.cpu().double() - want).abs().max() < 1e-5 * k ** 0.5 * 8
 
 
+@pytest.mark.parametrize("n", [17, 48, 49])
+@pytest.mark.parametrize("m,k,slices", [(2048, 5632, 11), (2048, 5640, 10), (2040, 7176, 13), (4096, 5632, 8)])
+def test_decode_tiles_take_whole_slices_of_512_up_to_48_rows(n, m, k, slices):
+    """Up to 48 rows and while tiles of 128 columns leave CUs idle (not at 4,096 columns): one slice for
+    every whole 512 of K, fewer where rounding a slice up to a stage would leave the last one empty."""
+    from kllm_amd.parts.linear import choose
+    k_ = K()
+    algo, nsplit = choose(torch.bfloat16, n, m, k)
+    assert algo == k_.GEMM_MFMA_BF16 and nsplit == (slices if n <= 48 else 8)
+    x, w = rnd(n, k, seed=1, dtype=torch.bfloat16, scale=0.5), rnd(m, k, seed=2, dtype=torch.bfloat16, scale=0.05)
+    parts = torch.full((nsplit, n, m), float("nan"), device=DEV)
+    k_.gemm(x, w, parts, algo, nsplit)
+    assert (parts.cpu().double().sum(0) - _gpu_reference(x, w).cpu()).abs().max() < 1e-5 * k ** 0.5 * 8
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n,f,k", [(1, 176, 64), (3, 120, 88), (8, 5632, 2048), (5, 33, 4104)])
 def test_gemv_swiglu(dtype, n, f, k):
