@@ -365,6 +365,7 @@ static float ring_time(const RingTile& t, int pair, int n, int m, int k, int nsp
   return 3.3f + sqrtf(sqrtf(b2 * b2 + w2 * w2)) + out;
 }
 
+// (`us`: the estimate, written where there is one: not for k >= kRingLongK, nor for up to 64 rows of bfloat16.)
 static int ring_tile(bool f32, int n, int m, int k, int nsplit, bool gate, bool f32_out, float* us = nullptr) {
   const RingTiles all = ring_tiles(f32);
   if (k >= kRingLongK) return f32 ? 0 : kRingNarrow;
@@ -448,15 +449,20 @@ using namespace kllm;
 // The slices that take the least time together with the kernel that adds them: its reads beyond the
 // 4.5 us that a launch takes whatever it holds (22 MB at 5 TB/s).  Slices of unequal length keep CUs
 // waiting: cuts that leave more than a tenth of K unused are out.
+// Where ring_tile does not estimate: one slice up to 64 rows of bfloat16 (decode batches, which their
+// caller cuts by a rule of its own); eight, the most here, for a K so long that a lane's offset takes 64 bits:
+// beside millions of products to a sum the slices' sums cost nothing.
 extern "C" int kllm_gemm_prompt_slices(int n, int m, int k, int dtype) {
   if (n <= 0 || m <= 0 || k <= 0) return 1;
   const bool f32 = dtype == DT_F32;
+  if (!f32 && n <= 64) return 1;
+  if (k >= kRingLongK) return 8;
   int best = 1;
   float least = 0.f;
   for (int ns : {1, 2, 3, 4, 6, 8}) {
     const long slice = ring_kslice(k, ns, ring_tiles(f32).pair);
     if (ns > 1 && (slice * (ns - 1) >= k || 10 * slice * ns > 11L * k)) continue;
-    float us;
+    float us = 0.f;
     ring_tile(f32, n, m, k, ns, false, true, &us);
     us += fmaxf(4.5f, 0.2e-6f * 4.f * ns * n * (float)m);
     if (ns == 1 || us < least) least = us, best = ns;
