@@ -314,7 +314,8 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const T* __restrict__
 // slices 15.2 / 14.1; 12,288 x 4,096 in 4 24.5 / 22.3; in 8 24.6 / 27.8; 4,096 x 14,336 in 8 23.9 / 31.3;
 // 2,560 x 2,048 in 16 8.1 / 9.3).  The two- and three-stage tiles of 64 x 64 and 64 x 128 before, at 64 rows: 11,264
 // x 2,048 15.1, with the gate 30.3 (now 19.6); 12,288 x 4,096 28.4; 4,096 x 14,336 in 8 29.3; 28,672 x 4,096
-// with the gate 61.2 (52.5); 2,048 x 2,048 in 8 6.4 (6.2); float32: 2,048 x 5,632 in 16 29.2 (24.6 in 11).
+// with the gate 61.2 (52.5); 2,048 x 2,048 in 8 6.4 (6.2); float32: 2,048 x 5,632 in 16 29.2 (in 15 slices of 384
+// 20.2; in 11 24.3, in 8 30.4).
 //
 // More rows:
 // A product's time in us is put together from what a tile costs a CU: rounds of the chip times (stages

@@ -53,9 +53,20 @@ def _skinny_split(n, m, k):
     wgs = -(-m // 64)
     while wgs * nsplit < K.device_cus() and k // (nsplit * 2) >= 128:
         nsplit *= 2
-    while (-(-(-(-k // nsplit)) // 32) * 32) * (nsplit - 1) >= k:   # no empty slice
+    return _no_empty_slice(nsplit, k, 32)
+
+
+# K of two stages of the MFMA tiles, 256 bytes: what their slices are rounded up to
+_PAIR_BF16, _PAIR_F32 = 128, 64
+
+
+def _no_empty_slice(nsplit, k, unit):
+    """The most slices up to ``nsplit`` of which none is empty, where a kernel rounds a slice of K up
+    to ``unit``."""
+    nsplit = int(nsplit)
+    while nsplit > 1 and (-(-(-(-k // nsplit)) // unit) * unit) * (nsplit - 1) >= k:
         nsplit -= 1
-    return int(nsplit)
+    return nsplit
 
 
 def _mfma_f32_split(n, m, k):
@@ -66,9 +77,7 @@ def _mfma_f32_split(n, m, k):
         return K.gemm_prompt_slices(n, m, k, torch.float32)
     waves = -(-m // 128) * 2
     nsplit = max(1, min(16, k // 128, -(-4 * K.device_cus() // waves)))
-    while nsplit > 1 and (-(-(-(-k // nsplit)) // 32) * 32) * (nsplit - 1) >= k:   # no empty slice
-        nsplit -= 1
-    return int(nsplit)
+    return _no_empty_slice(nsplit, k, _PAIR_F32)
 
 
 def _tiles_beat_skinny(n, m, k):
@@ -106,9 +115,7 @@ def _decode_tile_split(n, m, k):
         reach = (4 if k >= 8192 and tiles <= cus else 2) * cus
         while nsplit * 2 <= min(8, reach // tiles, k // 512):
             nsplit *= 2
-    while nsplit > 1 and (-(-(-(-k // nsplit)) // 64) * 64) * (nsplit - 1) >= k:   # no empty slice
-        nsplit -= 1
-    return nsplit
+    return _no_empty_slice(nsplit, k, _PAIR_BF16)
 
 
 def choose(dtype, n, m, k, options=None):

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from kllm_amd import kernels as K
+from kllm_amd.parts.linear import choose
 
 BF16, F32 = torch.bfloat16, torch.float32
 LONG = 1 << 23          # from this K on a lane's offset takes 64 bits
@@ -21,3 +22,35 @@ def test_slices_where_the_times_are_not_estimated(n, m, k, dtype, slices):
         K.gemm_prompt_slices(*other, dtype)
         K.gemm_prompt_slices.cache_clear()
         assert K.gemm_prompt_slices(n, m, k, dtype) == slices
+
+
+@pytest.mark.parametrize("n", [9, 17, 33, 48, 49, 64, 65, 128, 700, 2048])
+@pytest.mark.parametrize("dtype", [BF16, F32])
+def test_no_slice_of_k_is_empty(n, dtype):
+    """The MFMA tiles round a slice up to two stages (256 bytes of K); the skinny kernel up to 32: with the
+    kernel's own rounding the last slice must hold something, for the widths of the models here and
+    for K around every multiple of those."""
+    each = 8 if dtype == BF16 else 4
+    ks = {k + d * each for k in (64, 512, 1024, 2048, 4096, 5632, 7168, 11008, 14336) for d in (-9, -1, 0, 1, 5)}
+    cut = 0
+    for m in (256, 1000, 2048, 2560, 4096, 11264, 28672):
+        for k in sorted(ks):
+            if k <= 0:
+                continue
+            algo, nsplit = choose(dtype, n, m, k)
+            if algo not in (K.GEMM_MFMA_BF16, K.GEMM_MFMA_F32, K.GEMM_SKINNY_BF16):
+                continue
+            unit = 32 if algo == K.GEMM_SKINNY_BF16 else 256 // (16 // each)
+            kslice = -(-(-(-k // nsplit)) // unit) * unit
+            assert (nsplit - 1) * kslice < k, (m, k, nsplit, kslice)
+            cut += nsplit > 1
+    assert cut
+
+
+@pytest.mark.parametrize("n,m,k,dtype,slices", [
+    (17, 2048, 5632, F32, 15), (64, 2048, 5632, F32, 15),            # (of 384; sixteen would leave the last one empty)
+    (17, 2048, 5640, BF16, 9), (48, 2040, 7176, BF16, 12),           # (of 640)
+    (17, 2048, 5632, BF16, 11), (49, 2048, 5632, BF16, 8), (17, 4096, 5632, BF16, 8),
+])
+def test_slices_of_a_decode_batch(n, m, k, dtype, slices):
+    assert choose(dtype, n, m, k)[1] == slices
