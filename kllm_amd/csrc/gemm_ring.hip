@@ -33,10 +33,18 @@
 // operand (which element of K a lane's operand stands for is free as long as A and B agree).  There
 // the matrix unit's rate bounds everything, and what counts is that the CUs get equal numbers of tiles, three of
 // 64 x 128 a CU at a time.  In us against the four-wave tiles of 128 x 128 before (and K in up to 16 slices for
-// few rows): 700 x 11,264 x 2,048 with the gate 389 -> 274 (528 tiles of 128 x 128 on 256 CUs: three on some),
+// few rows): 700 x 11,264 x 2,048 with the gate 389 -> 264 (528 tiles of 128 x 128 on 256 CUs: three on some),
 // 700 x 2,048 x 5,632 238 -> 141, 72 x 11,264 x 2,048 150 -> 87, 2,048 x 11,264 x 2,048 777 -> 707.  Tiles of
 // 128 x 128 in this kernel: 900 x 11,264 x 2,048 510 (two a CU: what is left for the last round goes to
 // CUs in pairs) against 384.
+// A float32 sum's products go in two chains of accumulators, the halves of every phase's K, added at the
+// end: a single one's rounding grows with the slice, and the slices are fewer than those of the tiles before (error
+// against 64 bits, relative, with the four-wave tiles / one chain here / two: 65 x 2,048 x 5,632, in 16 / 8 / 8 slices, 3.4e-7 / 4.8e-7 /
+// 3.4e-7; 1,500 x 2,560 x 2,048 5.7e-7 / 8.1e-7 / 5.7e-7; 700 x 5,632 x 2,048 with the gate 1.24e-6 / 1.24e-6 / 0.85e-6).
+// It also leaves no product waiting for the one before it: 65 x 11,264 x 2,048 with the gate 80.2 -> 75.4 us, 700 rows
+// 268 -> 264, 65 x 2,048 x 5,632 with the sum of its slices 33.3 -> 31.8, 1,500 x 4,096 x 4,096 386 -> 381.  Chains of 32 of
+// K whose results are added in the loop leave less (1.8e-7 for 1,500 x 2,560 x 2,048) but cost 2 to 8 % more time.
+// Three workgroups a CU leave 80 registers a wave, which the two chains just fit.
 //
 // The operands' roles are exchanged (A = W, B = X): a lane's four accumulators are four neighbouring
 // columns of one row of Y, stored in one instruction.
@@ -93,7 +101,7 @@ enum : int { RING_WHOLE = 0, RING_TAIL = 1, RING_LONG = 2 };
 constexpr int kRingLongK = 1 << 23;        // 255 rows of bfloat16, 127 of float32: below 2^32 bytes
 
 template <typename T, typename TOUT, int MODE, int WR, int WC, int TM, int TN, int KIND>
-__global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const T* __restrict__ X, const T* __restrict__ W,
+__global__ __launch_bounds__(512, sizeof(T) == 4 ? 6 : 2) void gemm_ring_kernel(const T* __restrict__ X, const T* __restrict__ W,
                                                            TOUT* __restrict__ Y, int n, int m, int k, int tiles_x,
                                                            int tiles_y, int kslice, int act,
                                                            const float* __restrict__ act_params, int xcds) {
@@ -101,6 +109,7 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const T* __restrict__
   typedef typename RingOperand<T>::type op_t;
   typedef typename RingOffset<KIND == RING_LONG>::type off_t;
   constexpr int EPC = 16 / sizeof(T), STAGE = 8 * EPC;     // elements of a chunk of 16 bytes, of a stage
+  constexpr int CHAINS = sizeof(T) == 4 ? 2 : 1;           // of products to a sum (see above)
   constexpr int XR = WR * TM * 16, WS = WC * TN * 16;      // rows of a sub-tile of X, of W
   constexpr int BM = 2 * XR, BN = GATE ? WS : 2 * WS;      // rows and columns of the output tile
   constexpr int XB = XR * 128, WB = WS * 128;              // bytes of a sub-tile
@@ -154,7 +163,8 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const T* __restrict__
   const T* const xbase = X + (long)row0 * k + kbeg;
   const T* const wbase[2] = {W + (long)col0 * k + kbeg, W + ((long)col0 + (GATE ? m : 0)) * k + kbeg};
 
-  auto load = [&](const char* src, off_t off, int chunk, int left, unsigned char* dst) {
+  auto load = [&](const char* src, off_t& off, int chunk, int left, unsigned char* dst) {
+    if (CHAINS > 1) asm volatile("" : "+v"(off));        // (or the loop keeps 64-bit addresses instead: eight registers, spills)
     const char* at = src + off;
     if (TAIL) at = chunk * EPC < left ? at : reinterpret_cast<const char*>(g_ring_zeros);
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)at,
@@ -193,15 +203,17 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const T* __restrict__
 #pragma unroll
       for (int s = 0; s < 2; ++s) wf[h][j][s] = *reinterpret_cast<const op_t*>(wrd[s] + (parity * 2 + h) * WB + j * 2048);
   };
-  floatx4 acc[2][2][TM][TN];
+  floatx4 acc[CHAINS][2][2][TM][TN];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int s = 0; s < CHAINS; ++s)
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int a = 0; a < 2; ++a)
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+      for (int b = 0; b < 2; ++b)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[a][b][i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[s][a][b][i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
   auto multiply = [&](int hx, int hw) {
     __builtin_amdgcn_s_setprio(1);                          // before the SIMD's other wave, which reads
 #pragma unroll
@@ -210,7 +222,7 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const T* __restrict__
       for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
-          acc[hx][hw][i][j] = ring_mma(wf[hw][j][s], xf[i][s], acc[hx][hw][i][j]);
+          acc[s % CHAINS][hx][hw][i][j] = ring_mma(wf[hw][j][s], xf[i][s], acc[s % CHAINS][hx][hw][i][j]);
     __builtin_amdgcn_s_setprio(0);
   };
 
@@ -273,6 +285,9 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const T* __restrict__
     a_pos = softplus_f32(act_params[0]);
     a_neg = softplus_f32(act_params[1]);
   }
+  auto sum = [&](int hx, int hw, int i, int j, int e) {
+    return CHAINS == 1 ? acc[0][hx][hw][i][j][e] : acc[0][hx][hw][i][j][e] + acc[CHAINS - 1][hx][hw][i][j][e];
+  };
   const bool vec = m % 4 == 0 && (reinterpret_cast<uintptr_t>(Y) & (4 * sizeof(TOUT) - 1)) == 0;
 #pragma unroll
   for (int hx = 0; hx < 2; ++hx)
@@ -289,8 +304,8 @@ __global__ __launch_bounds__(512, 2) void gemm_ring_kernel(const T* __restrict__
           vec_t v;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            float s = acc[hx][hw][i][j][e];
-            if (GATE) s = gate_act(s, act) * acc[hx][1][i][j][e];
+            float s = sum(hx, hw, i, j, e);
+            if (GATE) s = gate_act(s, act) * sum(hx, 1, i, j, e);
             if (MODE == RING_UNARY) s = unary_act(s, act, a_pos, a_neg);
             v[e] = from_f32<TOUT>(s);
           }

@@ -478,6 +478,31 @@ def test_float32_prompt_products_on_every_tile(n, m, k, nsplit, gate, tile):
     assert bool((guard[n * m * nsplit:] == 7.0).all())
 
 
+@pytest.mark.parametrize("n,m,k", [(9, 1000, 1004), (17, 2048, 14336), (33, 2048, 64), (65, 2048, 2048), (65, 2560, 2048),
+                                   (100, 2048, 5632), (300, 2560, 2048), (700, 2560, 2048), (1500, 2560, 2048), (1500, 512, 4096)])
+def test_float32_products_add_in_two_chains(n, m, k):
+    """float32 products at the cut that the dispatch makes, against float64.  Half of a slice's products go to either
+    of two chains, which are added at the end, and the slices' sums one after the other.  An addition rounds by u =
+    2^-24 of a power of two at most: evenly within it, and with mantissas spread as their logarithm a mean square
+    of 0.54 u^2 / 3 of the sum; partial sums of unit normals grow as a random walk, so that a chain of c products leaves half
+    of c times that, relative to the products'.  The error in the 2-norm is u (0.09 (kslice / 2 + 1 + slices))^1/2 of the
+    result, and the bound 15 % more (one chain a slice leaves up to 41 % more)."""
+    from kllm_amd.parts.linear import choose
+    k_ = K()
+    x, w = rnd(n, k, seed=1), rnd(m, k, seed=2, scale=0.02)
+    algo, nsplit = choose(torch.float32, n, m, k)
+    assert algo == k_.GEMM_MFMA_F32
+    kslice = -(-(-(-k // nsplit)) // 64) * 64
+    parts = torch.empty(nsplit, n, m, device=DEV)
+    k_.gemm(x, w, parts, algo, nsplit)
+    total = parts[0].clone()
+    for part in parts[1:]:
+        total += part
+    want = _gpu_reference(x, w)
+    err = float((total.double() - want).norm() / want.norm())
+    assert err < 1.15 * 2.0 ** -24 * (0.09 * (kslice / 2 + 1 + nsplit)) ** 0.5, err
+
+
 @pytest.mark.parametrize("n", [5, 8, 16, 33, 64])
 @pytest.mark.parametrize("m,k", [(2048, 2048), (2048, 5632), (4096, 14336), (2560, 2048)])
 def test_split_product_into_its_consumers(n, m, k):
