@@ -737,18 +737,18 @@ extern "C" int kllm_linear_recurrence_scan(const float* a_in, const float* b_in,
                                            int n, int n_spans, int W, int dtype, hipStream_t stream) {
   KLLM_REQUIRE(a_in && b_in && proj && y_bias && state && slots && span_start && span_pos && out,
                "linear_recurrence_scan: null pointer");
-  KLLM_REQUIRE(n >= n_spans && n_spans > 0 && n_spans <= 65535 && W > 0 && nsplit >= 1,
+  KLLM_REQUIRE(n > 0 && n_spans > 0 && n_spans <= 65535 && W > 0 && nsplit >= 1,
                "linear_recurrence_scan: bad sizes n=%d spans=%d W=%d", n, n_spans, W);
   KLLM_REQUIRE(dtype == DT_F32 || dtype == DT_BF16, "linear_recurrence_scan: unknown dtype %d", dtype);
 #define KLLM_LRS(T, CH, SEGS)                                                                                         \
   hipLaunchKernelGGL((linear_recurrence_scan_kernel<T, CH, SEGS>), dim3(ceil_div(W, CH), n_spans), dim3(CH * SEGS), 0, \
                      stream, a_in, b_in, proj, nsplit, split_stride, y_bias, state, slot_stride, slots, span_start,    \
                      span_pos, (T*)out, W)
-  // (spans of single tokens have nothing to cut)
+  // (spans of single tokens have nothing to cut; there may be empty ones among the spans)
   if (dtype == DT_F32) {
-    if (n == n_spans) KLLM_LRS(float, 64, 1); else KLLM_LRS(float, 16, 64);
+    if (n <= n_spans) KLLM_LRS(float, 64, 1); else KLLM_LRS(float, 16, 64);
   } else {
-    if (n == n_spans) KLLM_LRS(bf16_t, 64, 1); else KLLM_LRS(bf16_t, 16, 64);
+    if (n <= n_spans) KLLM_LRS(bf16_t, 64, 1); else KLLM_LRS(bf16_t, 16, 64);
   }
 #undef KLLM_LRS
   KLLM_CHECK_LAUNCH("linear_recurrence_scan");

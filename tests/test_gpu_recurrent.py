@@ -127,3 +127,27 @@ def test_recurrence_chain(W, lens, dtype):
         state[int(slots[s]), 2:] = S
     close(out, want, rel=4e-5 if dtype == torch.float32 else 5e-3)
     close(dev_state, state)
+
+
+@pytest.mark.parametrize("lens", [[0, 1, 0], [0, 0, 2, 0], [3, 0], [0, 70, 0, 1], [1, 0, 40, 0, 0, 3]])
+def test_recurrence_chain_with_empty_spans(lens):
+    """Spans without tokens, also more spans than tokens: their states stay (or, where the span starts at
+    position 0, become zero), the others' outputs and states are as without them."""
+    g = torch.Generator().manual_seed(len(lens))
+    n, W, fresh = sum(lens), 72, [i % 2 for i in range(len(lens))]
+    a, b = torch.rand(n, W, generator=g) ** 0.1, torch.randn(n, W, generator=g)
+    proj, y_bias, state = torch.randn(1, n, 2 * W, generator=g), torch.randn(W, generator=g), torch.randn(len(lens) + 1, W, generator=g)
+    start, _, span_start, span_pos, slots = spans_of(lens, fresh)
+    dev_state, out = state.to(DEV), torch.full((n, W), float("nan"), device=DEV)
+    K().linear_recurrence_scan(a.to(DEV), b.to(DEV), proj.to(DEV), y_bias.to(DEV), dev_state, 0, slots, span_start,
+                               span_pos, len(lens), out)
+    y = torch.nn.functional.gelu(proj[0].double()[:, :W] + y_bias.double(), approximate="tanh")
+    want, state = torch.zeros(n, W, dtype=F64), state.double()
+    for s in range(len(lens)):
+        S = state[int(slots[s])] * (0.0 if fresh[s] else 1.0)
+        for t in range(start[s], start[s + 1]):
+            S = a[t].double() * S + b[t].double()
+            want[t] = S * y[t]
+        state[int(slots[s])] = S
+    close(out, want)
+    close(dev_state, state)
