@@ -487,11 +487,12 @@ int kllm_linear_recurrence_prep(const float* proj, int nsplit, long split_stride
                                 const float* bi, const float* rate, const int* span_of_token, const int* slots,
                                 const int* span_start, const int* span_pos, float* a_out, float* b_out, int n, int W,
                                 int blocks, hipStream_t stream);
-/* S <- a S + b per span and channel (state [W] per slot); out [n][W] = S * gelu_tanh(y + y_bias). */
+/* S <- a S + b per span and channel (state [W] per slot); out [n][W] = S * gelu_tanh(y + y_bias).
+ * longest: tokens of the longest span, or 0 if the caller does not know; only the split of the work goes by it. */
 int kllm_linear_recurrence_scan(const float* a_in, const float* b_in, const float* proj, int nsplit,
                                 long split_stride, const float* y_bias, float* state, long slot_stride,
                                 const int* slots, const int* span_start, const int* span_pos, void* out, int n,
-                                int n_spans, int W, int dtype, hipStream_t stream);
+                                int n_spans, int longest, int W, int dtype, hipStream_t stream);
 
 /* out[i] = sa * sum over a's slices + sb * sum over b's slices (float32, `count` elements a slice). */
 int kllm_scaled_sum(float* out, const float* a, int na, long stride_a, float sa, const float* b, int nb,

@@ -497,9 +497,8 @@ static int recurrence_prep_launch(const float* proj, int nsplit, long split_stri
 // from zero).  Every segment's threads first run its chain from zero, the segments' (A, B) meet in LDS,
 // those before a segment are folded into its starting state and it runs once more, now writing.  A
 // chain of n steps becomes two of n / SEGS.
-// CH channels and SEGS segments a workgroup: a prompt's chain takes many segments, and narrow groups of
-// channels so that the chip has workgroups enough (64 bytes of a row still lie side by side); single tokens
-// need neither.  1,500 tokens x 2,048 channels: 108 -> 33 us (64 channels in 16 segments: 32 workgroups).
+// CH channels and SEGS segments a workgroup (see kllm_linear_recurrence_scan); a span of up to LEAST tokens is one
+// segment, and the others' threads leave at once.
 template <typename T, int CH, int SEGS>
 __global__ __launch_bounds__(CH * SEGS) void linear_recurrence_scan_kernel(
     const float* __restrict__ a_in, const float* __restrict__ b_in, const float* __restrict__ proj, int nsplit,
@@ -512,12 +511,15 @@ __global__ __launch_bounds__(CH * SEGS) void linear_recurrence_scan_kernel(
   const bool ok = blockIdx.x * CH + lane < W;
   const int span = blockIdx.y;
   const long t0 = span_start[span], t1 = span_start[span + 1];
-  const long per = (t1 - t0 + SEGS - 1) / SEGS;
+  const long len = t1 - t0;
+  constexpr int U = 8, LEAST = 4;                         // tokens asked for at a time, of a segment at least
+  const long per = SEGS > 1 ? max((long)LEAST, (len + SEGS - 1) / SEGS) : len;
+  const bool cut = SEGS > 1 && len > LEAST;
   const long a0 = min(t1, t0 + seg * per), a1 = min(t1, a0 + per);
-  constexpr int U = 8;
   float* st = state + (long)slots[span] * slot_stride + c;
+  if (!cut && seg > 0) return;                            // (nobody meets)
   float S = span_pos[span] == 0 ? 0.f : *st;
-  if constexpr (SEGS > 1) {
+  if (cut) {
     float A = 1.f, B = 0.f;
     for (long tb = a0; tb < a1; tb += U) {
       float a[U], b[U];
@@ -561,7 +563,7 @@ __global__ __launch_bounds__(CH * SEGS) void linear_recurrence_scan_kernel(
   }
   // the last segment ends at the span's last token (an empty one has folded all); every segment has
   // read the state by then: they met behind it
-  if (ok && seg == SEGS - 1) *st = S;
+  if (ok && seg == (cut ? SEGS - 1 : 0)) *st = S;
 }
 
 // out = sa * (sum of a's slices) + sb * (sum of b's slices), element by element.
@@ -734,22 +736,36 @@ extern "C" int kllm_linear_recurrence_prep(const float* proj, int nsplit, long s
 extern "C" int kllm_linear_recurrence_scan(const float* a_in, const float* b_in, const float* proj, int nsplit,
                                            long split_stride, const float* y_bias, float* state, long slot_stride,
                                            const int* slots, const int* span_start, const int* span_pos, void* out,
-                                           int n, int n_spans, int W, int dtype, hipStream_t stream) {
+                                           int n, int n_spans, int longest, int W, int dtype, hipStream_t stream) {
   KLLM_REQUIRE(a_in && b_in && proj && y_bias && state && slots && span_start && span_pos && out,
                "linear_recurrence_scan: null pointer");
   KLLM_REQUIRE(n > 0 && n_spans > 0 && n_spans <= 65535 && W > 0 && nsplit >= 1,
                "linear_recurrence_scan: bad sizes n=%d spans=%d W=%d", n, n_spans, W);
   KLLM_REQUIRE(dtype == DT_F32 || dtype == DT_BF16, "linear_recurrence_scan: unknown dtype %d", dtype);
-#define KLLM_LRS(T, CH, SEGS)                                                                                         \
-  hipLaunchKernelGGL((linear_recurrence_scan_kernel<T, CH, SEGS>), dim3(ceil_div(W, CH), n_spans), dim3(CH * SEGS), 0, \
-                     stream, a_in, b_in, proj, nsplit, split_stride, y_bias, state, slot_stride, slots, span_start,    \
-                     span_pos, (T*)out, W)
-  // (spans of single tokens have nothing to cut; there may be empty ones among the spans)
-  if (dtype == DT_F32) {
-    if (n <= n_spans) KLLM_LRS(float, 64, 1); else KLLM_LRS(float, 16, 64);
-  } else {
-    if (n <= n_spans) KLLM_LRS(bf16_t, 64, 1); else KLLM_LRS(bf16_t, 16, 64);
-  }
+#define KLLM_LRS(CH, SEGS)                                                                                               \
+  do {                                                                                                                  \
+    const dim3 grid(ceil_div(W, CH), n_spans), wg(CH * SEGS);                                                           \
+    if (dtype == DT_F32)                                                                                                \
+      hipLaunchKernelGGL((linear_recurrence_scan_kernel<float, CH, SEGS>), grid, wg, 0, stream, a_in, b_in, proj,       \
+                         nsplit, split_stride, y_bias, state, slot_stride, slots, span_start, span_pos, (float*)out, W); \
+    else                                                                                                                \
+      hipLaunchKernelGGL((linear_recurrence_scan_kernel<bf16_t, CH, SEGS>), grid, wg, 0, stream, a_in, b_in, proj,      \
+                         nsplit, split_stride, y_bias, state, slot_stride, slots, span_start, span_pos, (bf16_t*)out, W); \
+  } while (0)
+  // The longest span's chain bounds the time, and every span, however short, takes workgroups.  Up to 16 tokens there
+  // is nothing to cut.  A long chain takes 64 segments of 16 channels where the tokens are those of few
+  // long spans (their workgroups of 1,024 threads, one a CU, run at once), else 32 of 32, and below 128 tokens 16 of 32.
+  // In us at 2,048 channels, 64 segments of 16 / 32 of 32 / 16 of 32 / 16 of 64 channels:
+  //   1,500 tokens 32 / 49 / 85 / 97; 3 x 500 27 / 20 / 32 / 35; 480 beside 4 single tokens 11 / 15 / 19 / 24;
+  //   512 beside 60 33 / 23 / 25 / 33; 8 x 250 35 / 23 / 22 / 22; 100 6.2 / 7.0 / 6.6 / 7.6; 40 beside 3 6.1 / 5.7 / 5.7 / 6.4;
+  //   16 x 64 28 / 19 / 14 / 15; 8 x 64 13 / 10 / 7.3 / 7.7; 60 x 16 59 / 33 / 22 / 36, uncut 11; 60 x 3 24 / 13 / 9.3 / 15, uncut 4.9.
+  // (64 segments of 16 for every step that is not all single tokens, without leaving early: 512 beside 60 66, 60 x 3 56.)
+  if (longest <= 0) longest = n > n_spans ? n - n_spans + 1 : 1;      // not said: the most if no span is empty
+  const long together = (long)n * ceil_div(W, 16);
+  if (longest <= 16) KLLM_LRS(64, 1);
+  else if (longest < 128) KLLM_LRS(32, 16);
+  else if (together <= (long)device_cus() * longest) KLLM_LRS(16, 64);
+  else KLLM_LRS(32, 32);
 #undef KLLM_LRS
   KLLM_CHECK_LAUNCH("linear_recurrence_scan");
   return 0;

@@ -21,7 +21,7 @@ import torch
 DT_F32, DT_BF16 = 0, 1
 GEMM_PLAIN, GEMM_TILED_F32, GEMM_MFMA_BF16, GEMM_SKINNY_BF16, GEMM_GEMV, GEMM_GEMV_LDS, GEMM_MFMA_F32 = 0, 1, 2, 3, 4, 5, 6
 GEMV_BEST_ROWS = 0         # rows up to which they beat the MFMA kernels in bfloat16: none (a step at 1.1B sizes, one token: 1.036 against 0.963 ms)
-ABI_VERSION = 17
+ABI_VERSION = 18
 
 
 class KernelError(RuntimeError):
@@ -156,7 +156,7 @@ def _declare(lib):
         "kllm_gated_delta_max_dim": [],
         "kllm_gated_delta_scan": [P, P, P, P, P, P, L, P, P, P, I, I, I, I, I, P, P],
         "kllm_linear_recurrence_prep": [P, I, L, P, P, P, I, P, L, P, P, P, P, P, P, P, P, P, P, P, I, I, I, P],
-        "kllm_linear_recurrence_scan": [P, P, P, I, L, P, P, L, P, P, P, P, I, I, I, I, P],
+        "kllm_linear_recurrence_scan": [P, P, P, I, L, P, P, L, P, P, P, P, I, I, I, I, I, P],
         "kllm_scaled_sum": [P, P, I, L, F, P, I, L, F, L, P],
         "kllm_normed_sum": [P, P, I, L, F, P, P, I, L, F, P, I, I, F, P],
         "kllm_qkv_conv_append": [P, I, L, I, I, P, I, P, L, I, P, P, I, I, F, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, I, P, P],
@@ -1812,9 +1812,10 @@ def linear_recurrence_prep(proj, x_bias, conv_w, conv_b, taps, state, conv_offse
             _ptr(a_out, "recurrence a", F32), _ptr(b_out, "recurrence b", F32), n, W, int(blocks), _stream())
 
 
-def linear_recurrence_scan(a_in, b_in, proj, y_bias, state, offset, slots, span_start, span_pos, n_spans, out):
+def linear_recurrence_scan(a_in, b_in, proj, y_bias, state, offset, slots, span_start, span_pos, n_spans, out, longest=0):
     """S <- a S + b along every span (state [W] float32 at ``offset`` floats into the slot); out
-    [n, W] = S * gelu_tanh(y + y_bias), y the first W columns of the sums ``proj`` [nsplit, n, 2 W]."""
+    [n, W] = S * gelu_tanh(y + y_bias), y the first W columns of the sums ``proj`` [nsplit, n, 2 W].
+    ``longest``: tokens of the longest span, if the caller knows it; the split of the work goes by it."""
     n, W = a_in.shape
     nsplit, stride = _splits(proj, n, 2 * W, "linear_recurrence_scan")
     addr, per_slot = _field(state, offset, "linear_recurrence_scan")
@@ -1826,7 +1827,7 @@ def linear_recurrence_scan(a_in, b_in, proj, y_bias, state, offset, slots, span_
             _ptr(b_in, "recurrence b", F32), _ptr(proj, "recurrence proj", F32), nsplit, stride,
             _ptr(y_bias, "recurrence y bias", F32), addr, per_slot, _ptr(slots, "recurrence slots", I32),
             _ptr(span_start, "recurrence span_start", I32), _ptr(span_pos, "recurrence span_pos", I32),
-            _ptr(out, "recurrence out"), n, int(n_spans), W, dtype_code(out.dtype), _stream())
+            _ptr(out, "recurrence out"), n, int(n_spans), int(longest), W, dtype_code(out.dtype), _stream())
 
 
 def scaled_sum(out, a, scale_a, b, scale_b):

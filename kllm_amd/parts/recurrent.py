@@ -254,7 +254,7 @@ class LinearRecurrenceMixer(Part):
                             ctx.n_spans, in_bias=self.x_bias)
         out = ctx.buf("rec.out", (n, W), self.runtime.dtype)
         K.linear_recurrence_scan(a, b, proj, self.y_bias, cache.state, 0, cache.slots, ctx.span_start, ctx.span_pos,
-                                 ctx.n_spans, out)
+                                 ctx.n_spans, out, longest=ctx.max_span_len)
         return decode_linear(ctx, out, self.w_o, "rec.o_proj", self._tiled.get("o"))
 
 

@@ -105,10 +105,14 @@ def test_recurrence_gates(blocks, bs, lens, taps):
 
 
 @pytest.mark.parametrize("W", [8, 72, 200])
-@pytest.mark.parametrize("lens", [[1, 1, 1], [2], [63, 64, 65], [700, 1]])
+@pytest.mark.parametrize("lens", [[1, 1, 1], [2], [63, 64, 65], [700, 1], [4, 5, 16, 1], [17, 1, 60, 1], [127, 3], [128, 1, 4, 5],
+                                  [130] * 21])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-def test_recurrence_chain(W, lens, dtype):
-    """Spans shorter than the segments are many, as long, and much longer; a state that is read and left."""
+@pytest.mark.parametrize("said", [False, True])
+def test_recurrence_chain(W, lens, dtype, said):
+    """Spans shorter than the segments are many, as long, and much longer; a state that is read and left.  Every
+    split of the work: spans uncut (up to 16 tokens), 16 segments (below 128), 64, and 32 where the
+    long spans are many (21 of 130 tokens at 200 channels); with and without the longest span's length."""
     g = torch.Generator().manual_seed(W)
     n, fresh = sum(lens), [i % 2 for i in range(len(lens))]
     a, b = torch.rand(n, W, generator=g) ** 0.1, torch.randn(n, W, generator=g)
@@ -116,7 +120,7 @@ def test_recurrence_chain(W, lens, dtype):
     start, _, span_start, span_pos, slots = spans_of(lens, fresh)
     dev_state, out = state.to(DEV), torch.full((n, W), float("nan"), device=DEV, dtype=dtype)
     K().linear_recurrence_scan(a.to(DEV), b.to(DEV), proj.to(DEV), y_bias.to(DEV), dev_state, 2, slots, span_start,
-                               span_pos, len(lens), out)
+                               span_pos, len(lens), out, longest=max(lens) if said else 0)
     y = torch.nn.functional.gelu(proj.double().sum(0)[:, :W] + y_bias.double(), approximate="tanh")
     want, state = torch.zeros(n, W, dtype=F64), state.double()
     for s in range(len(lens)):
