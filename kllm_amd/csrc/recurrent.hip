@@ -307,17 +307,20 @@ constexpr int kGateChunk = 1024;              // inputs of a block that LDS hold
 // proj: [nsplit][n][2 W], columns y | x.  Workgroup (NT tiles of 16 tokens, block b of the gates, OW times
 // 16 of its output channels): the convolved inputs of the block's channels for its tokens go into LDS
 // [tokens][inputs + 4], 1,024 inputs at a time; the gates' products run on the 32-bit matrix instruction 16x16x4 (an
-// FMA chain, as before).  The gates' matrices are read [block][in][out]: a lane's output channel is its
+// FMA chain).  The gates' matrices are read [block][in][out]: a lane's output channel is its
 // lane % 16, so that a load reads 64 bytes of each of four rows.  A = inputs: lane l holds token l % 16,
 // inputs 16 s + 4 (l / 16) + e of step s, e the instruction; which input a product covers is free as
-// long as both operands agree, so a lane reads four with one 16-byte LDS read.
+// long as both operands agree, so a lane reads four with one 16-byte LDS read.  A sum's products go in chains of 64
+// inputs that are added one after the other, as with the four threads to an output before: one chain of a block's 256
+// left 1.3 times their error against 64 bits in the added terms (1.54e-7 against 1.18e-7 relative).
 // KS waves share an output's inputs and meet in LDS: where there is one tile of tokens (a decode batch)
 // the matrices' way from memory bounds the time, and it needs workgroups (16 channels each) and short
 // chains; a prompt has tiles enough and is bound by its products.
 // 1,500 tokens x 2,048 channels in blocks of 256: 144 -> 63 us (FMA on eight tokens at a time, 790 MB of matrices
 // through L2); 8 tokens: 28.8 -> 17.6 us (32 workgroups then, 128 now).
-// TAPS: the convolution's, or 0 (any number).
-template <int NT, int KS, int OW, int TAPS>
+// TAPS: the convolution's, or 0 (any number).  ONE: a block's inputs fit into LDS at
+// once; the sums then begin behind the convolution and take no registers in it (72 instead of 89, three workgroups a CU).
+template <int NT, int KS, int OW, int TAPS, bool ONE>
 __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel(
     const float* __restrict__ proj, int nsplit, long split_stride, const float* __restrict__ x_bias,
     const float* __restrict__ conv_w, const float* __restrict__ conv_b, int taps, const float* __restrict__ state,
@@ -336,15 +339,15 @@ __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel
   const int col = lane % 16, quad = lane / 16;
   const int o = (blockIdx.z * OW + ow) * kGateTile + col;
   const int oc = min(o, bs - 1);
-  const float* wr = wr_t + (long)b * bs * bs + oc;
-  const float* wi = wi_t + (long)b * bs * bs + oc;
+  const float* wr = wr_t + (long)b * bs * bs;
+  const float* wi = wi_t + (long)b * bs * bs;
   struct Pair { float r[4], i[4]; };
   auto fetch = [&](int first) -> Pair {       // (inputs that do not exist: zeros, whatever the last row holds)
     Pair P;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int in = first + 4 * quad + e;
-      const long at = (long)min(in, bs - 1) * bs;
+      const unsigned at = (unsigned)min(in, bs - 1) * bs + oc;      // (blocks of up to 4,096 channels)
       const float r = wr[at], g = wi[at];
       P.r[e] = in < bs ? r : 0.f;
       P.i[e] = in < bs ? g : 0.f;
@@ -354,12 +357,14 @@ __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel
   floatx4 ar[NT], ai[NT], own[NT];            // own: the outputs' own inputs
 #pragma unroll
   for (int t = 0; t < NT; ++t) ar[t] = ai[t] = own[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  constexpr int CHAIN = 4;                    // steps of a chain
   __shared__ int4 spans[TT];                  // the tokens' spans
   if (tid < nt) {
     const int span = span_of_token[tfirst + tid];
     spans[tid] = int4{span_start[span], slots[span], span_pos[span] == 0, 0};
   }
-  for (int k0 = 0; k0 < bs; k0 += chunk) {
+  int k0 = 0;
+  do {
     __syncthreads();
     if (TAPS > 0 && nt > 1) {
       // A thread takes a channel for a run of RUN tokens and asks for the run's inputs at once, each
@@ -419,20 +424,32 @@ __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) own[t][i] = us[(t * kGateTile + 4 * quad + i) * ld + o - k0];
-    for (int s = s0; s < s1; ++s) {
-      const Pair next = fetch(k0 + 16 * min(s + 1, steps - 1));
+    for (int c0 = s0; c0 < s1; c0 += CHAIN) {
+      floatx4 cr[NT], ci[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) cr[t] = ci[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+      for (int s = c0; s < min(s1, c0 + CHAIN); ++s) {
+        const Pair next = fetch(k0 + 16 * min(s + 1, steps - 1));
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          const floatx4 u = *reinterpret_cast<const floatx4*>(&us[(t * kGateTile + col) * ld + 16 * s + 4 * quad]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            cr[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(u[e], w.r[e], cr[t], 0, 0, 0);
+            ci[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(u[e], w.i[e], ci[t], 0, 0, 0);
+          }
+        }
+        w = next;
+      }
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        const floatx4 u = *reinterpret_cast<const floatx4*>(&us[(t * kGateTile + col) * ld + 16 * s + 4 * quad]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          ar[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(u[e], w.r[e], ar[t], 0, 0, 0);
-          ai[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(u[e], w.i[e], ai[t], 0, 0, 0);
-        }
+        ar[t] += cr[t];
+        ai[t] += ci[t];
       }
-      w = next;
     }
-  }
+    k0 += chunk;
+  } while (!ONE && k0 < bs);
   if constexpr (KS > 1) {                     // the waves' shares, in a fixed order
     static_assert(OW == 1 && NT == 1, "one tile a workgroup");
     __shared__ floatx4 red[KS - 1][2][kWave];
@@ -466,8 +483,8 @@ __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel
     }
 }
 
-template <int NT, int KS, int OW, int TAPS>
-static int recurrence_prep_launch(const float* proj, int nsplit, long split_stride, const float* x_bias,
+template <int NT, int KS, int OW, int TAPS, bool ONE>
+static int recurrence_prep_launch_chunks(const float* proj, int nsplit, long split_stride, const float* x_bias,
                                   const float* conv_w, const float* conv_b, int taps, const float* state,
                                   long slot_stride, const float* wr_t, const float* wi_t, const float* br,
                                   const float* bi, const float* rate, const int* span_of_token, const int* slots,
@@ -478,16 +495,22 @@ static int recurrence_prep_launch(const float* proj, int nsplit, long split_stri
   const size_t lds = (size_t)NT * kGateTile * (chunk + 4) * sizeof(float);
   static size_t raised_to = 48 * 1024;      // beside the kernel's own LDS
   if (lds > raised_to) {
-    (void)hipFuncSetAttribute((const void*)linear_recurrence_prep_kernel<NT, KS, OW, TAPS>,
+    (void)hipFuncSetAttribute((const void*)linear_recurrence_prep_kernel<NT, KS, OW, TAPS, ONE>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     raised_to = lds;
   }
-  hipLaunchKernelGGL((linear_recurrence_prep_kernel<NT, KS, OW, TAPS>),
+  hipLaunchKernelGGL((linear_recurrence_prep_kernel<NT, KS, OW, TAPS, ONE>),
                      dim3(ceil_div(n, NT * kGateTile), blocks, ceil_div(bs, OW * kGateTile)), dim3(kWave * KS * OW), lds,
                      stream, proj, nsplit, split_stride, x_bias, conv_w, conv_b, taps, state, slot_stride, wr_t, wi_t, br,
                      bi, rate, span_of_token, slots, span_start, span_pos, a_out, b_out, n, W, bs);
   KLLM_CHECK_LAUNCH("linear_recurrence_prep");
   return 0;
+}
+
+template <int NT, int KS, int OW, int TAPS, typename... A>
+static int recurrence_prep_launch(int bs, A... args) {
+  return bs <= kGateChunk ? recurrence_prep_launch_chunks<NT, KS, OW, TAPS, true>(args...)
+                          : recurrence_prep_launch_chunks<NT, KS, OW, TAPS, false>(args...);
 }
 
 // S <- a S + b along a span; out = S * gelu_tanh(y + y_bias).  Eight tokens' numbers are asked
@@ -725,7 +748,7 @@ extern "C" int kllm_linear_recurrence_prep(const float* proj, int nsplit, long s
   // workgroups enough; one tile, one group of 16 channels and the inputs shared out over four waves below.
   const bool prompt = n > 64;
 #define KLLM_LRP(NT, KS, OW, TAPS)                                                                                        \
-  recurrence_prep_launch<NT, KS, OW, TAPS>(proj, nsplit, split_stride, x_bias, conv_w, conv_b, taps, state, slot_stride, wr_t, \
+  recurrence_prep_launch<NT, KS, OW, TAPS>(bs, proj, nsplit, split_stride, x_bias, conv_w, conv_b, taps, state, slot_stride, wr_t, \
                                      wi_t, br, bi, rate, span_of_token, slots, span_start, span_pos, a_out, b_out, n, W,  \
                                      blocks, stream)
   if (taps == 4) return prompt ? KLLM_LRP(2, 1, 8, 4) : KLLM_LRP(1, 4, 1, 4);

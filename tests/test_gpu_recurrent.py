@@ -104,6 +104,31 @@ def test_recurrence_gates(blocks, bs, lens, taps):
     close(b, torch.sqrt(-torch.expm1(2 * log_a)) * gate(wi, bi) * u, rel=1e-4)   # (the root of a small difference)
 
 
+@pytest.mark.parametrize("n", [8, 100, 400, 1200])
+@pytest.mark.parametrize("blocks,bs", [(4, 256), (1, 1040)])
+def test_recurrence_gates_add_in_short_chains(n, blocks, bs):
+    """How far a gate's sums are from 64 bits, read off the added term: with an input gate far below zero, sigmoid(z) =
+    exp(z), the term's relative error is z's own.  z = sum - 40, sums of spread 10: chains of 64 products, whose
+    results are added, err by 10 u (0.09 (64 + bs / 64))^1/2 in the root mean square (u = 2^-24: an addition's rounding, of mean
+    square 0.54 u^2 / 3 of a partial sum, over half the chain's length), and adding the bias by its last place's
+    2^-18 / 12^1/2; the bound is a tenth more.  (One chain of 256: 1.7 times that.)"""
+    g = torch.Generator().manual_seed(n + bs)
+    W, u = blocks * bs, 2.0 ** -24
+    r = lambda *s: torch.randn(*s, generator=g)
+    proj, wi = r(1, n, 2 * W), r(blocks, bs, bs) * 10 / bs ** 0.5
+    zeros, ones = torch.zeros(W), torch.ones(W, 1)
+    span_start, i32 = torch.tensor([0, n], dtype=torch.int32, device=DEV), torch.zeros(n, dtype=torch.int32, device=DEV)
+    d = lambda t: t.to(DEV).contiguous()
+    a, b = (torch.full((n, W), float("nan"), device=DEV) for _ in range(2))
+    K().linear_recurrence_prep(d(proj), d(zeros), d(ones), d(zeros), 1, d(r(1, 8)), 8, d(torch.zeros(blocks, bs, bs)), d(wi), d(zeros),
+                               d(zeros - 40), d(zeros + 0.5), i32, i32[:1], span_start, i32[:1], a, b, blocks)
+    x = proj[0, :, W:].double()
+    z = (x.view(n, blocks, 1, bs) @ wi.double()).reshape(n, W) - 40
+    want = (1 - torch.exp(torch.tensor(-0.5, dtype=F64))).sqrt() * torch.sigmoid(z) * x
+    err = (b.double().cpu() / want - 1)[(z > -64) & (z < -16) & (x != 0)]
+    assert float(err.pow(2).mean().sqrt()) < 1.1 * ((10 * u) ** 2 * 0.09 * (64 + bs / 64) + 2.0 ** -36 / 12) ** 0.5
+
+
 @pytest.mark.parametrize("W", [8, 72, 200])
 @pytest.mark.parametrize("lens", [[1, 1, 1], [2], [63, 64, 65], [700, 1], [4, 5, 16, 1], [17, 1, 60, 1], [127, 3], [128, 1, 4, 5],
                                   [130] * 21])
