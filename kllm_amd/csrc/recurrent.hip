@@ -316,9 +316,9 @@ constexpr int kGateChunk = 1024;              // inputs of a block that LDS hold
 // KS waves share an output's inputs and meet in LDS: where there is one tile of tokens (a decode batch)
 // the matrices' way from memory bounds the time, and it needs workgroups (16 channels each) and short
 // chains; a prompt has tiles enough and is bound by its products.
-// 1,500 tokens x 2,048 channels in blocks of 256: 144 -> 63 us (FMA on eight tokens at a time, 790 MB of matrices
-// through L2); 8 tokens: 28.8 -> 17.6 us (32 workgroups then, 128 now).
-// TAPS: the convolution's, or 0 (any number).  ONE: a block's inputs fit into LDS at
+// 1,500 tokens x 2,048 channels in blocks of 256: 140 -> 63 us (FMA on eight tokens at a time, 790 MB of matrices
+// through L2); 8 tokens: 18 -> 11 us (32 workgroups then, 128 now).
+// TAPS: the convolution's where it is 4, 8 for any number up to 8, 0 for more.  ONE: a block's inputs fit into LDS at
 // once; the sums then begin behind the convolution and take no registers in it (72 instead of 89, three workgroups a CU).
 template <int NT, int KS, int OW, int TAPS, bool ONE>
 __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel(
@@ -369,19 +369,21 @@ __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel
     if (TAPS > 0 && nt > 1) {
       // A thread takes a channel for a run of RUN tokens and asks for the run's inputs at once, each
       // for all the taps it meets, instead of for every tap of every token on its own.
-      constexpr int K = TAPS > 0 ? TAPS - 1 : 0, RUN = 8;
+      constexpr int MOST = TAPS > 0 ? TAPS : 1, RUN = 8;
+      const int K = TAPS == 4 ? 3 : taps - 1;
       for (int i = tid; i < TT / RUN * chunk; i += THREADS) {
         const int r = i / chunk, e = k0 + i - r * chunk, c = b * bs + e, tt0 = r * RUN;
         const bool there = e < bs && tt0 < nt;
-        float x[RUN + K], wt[TAPS > 0 ? TAPS : 1];
+        float x[RUN + MOST - 1], wt[MOST];
         if (there) {
 #pragma unroll
-          for (int q = 0; q < RUN + K; ++q) {        // (rows that are not there: some row that is, not used)
+          for (int q = 0; q < RUN + MOST - 1; ++q) {        // (rows that are not there: some row that is, not used)
+            if (q >= RUN + K) break;
             const long row = min(max(tfirst + tt0 - K + q, 0L), (long)n - 1);
             x[q] = conv_input(proj, nsplit, split_stride, cols, W + c, x_bias - W, row);
           }
 #pragma unroll
-          for (int j = 0; j < TAPS; ++j) wt[j] = conv_w[(long)c * taps + j];
+          for (int j = 0; j < MOST; ++j) wt[j] = conv_w[(long)c * taps + min(j, K)];
         }
         const float cb = there ? conv_b[c] : 0.f;
 #pragma unroll
@@ -391,7 +393,8 @@ __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel
             const long t = tfirst + tt0 + q;
             const int4 sp = spans[tt0 + q];           // first row, slot, whether the span starts at position 0
 #pragma unroll
-            for (int j = 0; j < TAPS; ++j) {
+            for (int j = 0; j < MOST; ++j) {
+              if (j > K) break;
               const int back = (int)(t - K + j) - sp.x;      // rows behind the span's first
               float in = x[q + j];
               if (back < 0) in = sp.z ? 0.f : state[(long)sp.y * slot_stride + (long)c * K + K + back];
@@ -744,15 +747,26 @@ extern "C" int kllm_linear_recurrence_prep(const float* proj, int nsplit, long s
   KLLM_REQUIRE(taps >= 1 && taps <= kMaxTaps, "linear_recurrence_prep: %d taps (1 to %d)", taps, kMaxTaps);
   const int bs = W / blocks;
   KLLM_REQUIRE(bs <= 4096, "linear_recurrence_prep: blocks of %d channels (up to 4,096)", bs);
-  // Two tiles of tokens a workgroup and eight waves of 16 channels where the tokens give the chip
-  // workgroups enough; one tile, one group of 16 channels and the inputs shared out over four waves below.
-  const bool prompt = n > 64;
+  // A decode batch shares a sum's inputs out over four waves and takes 16 channels a workgroup: short chains, and
+  // workgroups enough.  The workgroups of a block repeat its convolution and each tile of tokens reads the matrices
+  // again, so that from three workgroups a CU on (or what LDS lets run side by side) eight waves take 16 channels each, and two tiles of
+  // tokens at a time once those give every CU two workgroups.  In us, the three forms and, last, eight tokens at a
+  // time with FMA, 2,048 channels in blocks of 256: 64 tokens 16 / 17 / 28 / 26; 100 single tokens 26 / 25 / 37 / 26;
+  // 200 29 / 25 / 34 / 33; 500 57 / 29 / 35 / 52; 800 77 / 44 / 48 / 82; 1,500 141 / 67 / 61 / 140; 512 channels in blocks of 128: 100 9.5 /
+  // 13 / 17 / 13; 640 14 / 13 / 17 / 17; one block of 1,024: 100 58 / 75 / 110 / 89; 200 108 / 75 / 114 / 94; 1,500 673 / 155 / 220 / 405.
+  const int tiles = ceil_div(n, kGateTile), cus = device_cus();
+  const long lds = (long)kGateTile * ((ceil_div(bs, 16) * 16 < kGateChunk ? ceil_div(bs, 16) * 16 : kGateChunk) + 4) * 4;
+  const int side = 160 * 1024 / lds < 3 ? (int)(160 * 1024 / lds) : 3;
+  const bool few = (long)tiles * blocks * ceil_div(bs, kGateTile) <= (long)side * cus;
+  const bool many = (long)ceil_div(tiles, 2) * blocks * ceil_div(bs, 8 * kGateTile) >= 2L * cus;
 #define KLLM_LRP(NT, KS, OW, TAPS)                                                                                        \
   recurrence_prep_launch<NT, KS, OW, TAPS>(bs, proj, nsplit, split_stride, x_bias, conv_w, conv_b, taps, state, slot_stride, wr_t, \
                                      wi_t, br, bi, rate, span_of_token, slots, span_start, span_pos, a_out, b_out, n, W,  \
                                      blocks, stream)
-  if (taps == 4) return prompt ? KLLM_LRP(2, 1, 8, 4) : KLLM_LRP(1, 4, 1, 4);
-  return prompt ? KLLM_LRP(2, 1, 8, 0) : KLLM_LRP(1, 4, 1, 0);
+#define KLLM_LRP_TAPS(TAPS) (few ? KLLM_LRP(1, 4, 1, TAPS) : many ? KLLM_LRP(2, 1, 8, TAPS) : KLLM_LRP(1, 1, 8, TAPS))
+  if (taps == 4) return KLLM_LRP_TAPS(4);
+  return taps <= 8 ? KLLM_LRP_TAPS(8) : KLLM_LRP_TAPS(0);
+#undef KLLM_LRP_TAPS
 #undef KLLM_LRP
 }
 

@@ -77,6 +77,18 @@ def test_delta_scan(dk, dv, lens, fresh, per_channel):
 def test_recurrence_gates(blocks, bs, lens, taps):
     """Convolution, gates' products and decays: one tile of tokens and several, requests that meet
     within a tile and within a thread's run of tokens, blocks of odd sizes and of more inputs than LDS takes."""
+    check_recurrence_gates(blocks, bs, lens, taps)
+
+
+@pytest.mark.parametrize("blocks,bs,lens", [(2, 256, [300, 1, 99]), (2, 136, [33] * 30), (1, 1040, [1, 200, 100]),      # one tile of tokens, eight waves
+                                            (8, 136, [1000, 1, 1, 45]), (33, 8, [500, 1, 13])])                  # two tiles
+@pytest.mark.parametrize("taps", [1, 4, 8, 9])
+def test_recurrence_gates_of_prompts(blocks, bs, lens, taps):
+    """The same where the tokens and blocks give the chip workgroups enough for the wider forms."""
+    check_recurrence_gates(blocks, bs, lens, taps)
+
+
+def check_recurrence_gates(blocks, bs, lens, taps):
     g = torch.Generator().manual_seed(bs + taps)
     n, W, fresh = sum(lens), blocks * bs, [i % 2 for i in range(len(lens))]
     r = lambda *s: torch.randn(*s, generator=g)
