@@ -46,6 +46,36 @@ def _numel(shape) -> int:
     return n
 
 
+def room_for_copies(weights: int, cache: int, free: int, total: int) -> bool:
+    """Whether a float32 engine keeps second copies of its matrices in the order that the decode-batch
+    kernel reads them (``parts.linear.tiled_copy``; at most as many bytes as the ``weights``, which are loaded): half of the card
+    must stay for what the program allocates besides weights, copies and ``cache``, and what is
+    ``free`` now must hold the copies and the cache.  All matrices get one or none does, so that the speed of an engine does
+    not hang on the order in which they are bound."""
+    return 2 * weights + cache <= total // 2 and weights + cache <= free
+
+
+def _cache_dtype(need, default) -> torch.dtype:
+    if need.dtype is None:
+        return default
+    dt = getattr(torch, str(need.dtype), None)
+    if not isinstance(dt, torch.dtype):
+        raise ValueError(f"cache dtype {need.dtype!r} is no torch dtype")
+    return dt
+
+
+@dataclass
+class _CacheSizes:
+    """What a cache is to hold: pages asked for; pages of each paged group, and bytes of one; bytes of all state slots."""
+    asked: int
+    pages: Dict[int, int]
+    page_bytes: Dict[int, int]
+    state_bytes: int
+
+    def total(self) -> int:
+        return self.state_bytes + sum(n * self.page_bytes[g] for g, n in self.pages.items())
+
+
 class StepError(ValueError):
     """A step that cannot be run as asked (bad token id, unknown request...)."""
 
@@ -121,10 +151,15 @@ class Engine:
         self.vocab_size = self.spec.vocab_size
         specs = self.model.weight_specs()
         weights = weights_from(specs, self.spec)
+        self.max_model_len = options.max_model_len or self.spec.max_positions
+        sizes = self._size_cache()
+        if self.dtype == torch.float32:
+            numels = {s.name: _numel(s.shape) for s in specs}
+            self.runtime.second_copies = room_for_copies(4 * sum(numels.values()), sizes.total(),
+                                                         *torch.cuda.mem_get_info(self.device))
         self.model.bind(weights)
         del weights
-        self.max_model_len = options.max_model_len or self.spec.max_positions
-        self._alloc_cache()
+        self._alloc_cache(sizes)
         self._pinned: List[torch.Tensor] = []
         self._pinned_events: List[Optional[torch.cuda.Event]] = []
         self._pinned_next = 0
@@ -180,8 +215,8 @@ class Engine:
         return cls(typed, raw, weights_from, options)
 
     # ------------------------------------------------------------------ cache
-    def _alloc_cache(self):
-        """Pools and device tensors of every cache group.
+    def _size_cache(self) -> _CacheSizes:
+        """What the cache is to hold.
 
         Capacity rule: the pool holds ``num_pages`` pages (or ``max_tokens``
         tokens; by default four longest requests, engine/engine.go:30-32), but
@@ -195,8 +230,6 @@ class Engine:
         plan = self.model.cache_plan
         if o.page_size <= 0:
             raise ValueError(f"page_size {o.page_size} must be positive")
-        for part in self.model.all_parts():
-            part.check_cache(o.page_size)
         if o.num_pages is not None:
             asked = int(o.num_pages)
         else:
@@ -208,21 +241,11 @@ class Engine:
         for g, gp in enumerate(plan.groups):
             if gp.need.kind not in ("paged", "state"):
                 raise ValueError(f"unknown cache kind {gp.need.kind!r}")
-        def dtype_of(need, default):
-            if need.dtype is None:
-                return default
-            dt = getattr(torch, str(need.dtype), None)
-            if not isinstance(dt, torch.dtype):
-                raise ValueError(f"cache dtype {need.dtype!r} is no torch dtype")
-            return dt
-
-        def size_of(dt):
-            return torch.empty((), dtype=dt).element_size()
         state_bytes = sum(gp.entries * o.max_requests * _numel(gp.need.state_shape)
-                          * size_of(dtype_of(gp.need, torch.float32))
+                          * _cache_dtype(gp.need, torch.float32).itemsize
                           for gp in plan.groups if gp.need.kind == "state")
         page_bytes = {g: gp.entries * gp.need.kv_heads * o.page_size * (gp.need.head_dim + gp.need.value_width)
-                      * size_of(dtype_of(gp.need, self.dtype)) for g, gp in paged}
+                      * _cache_dtype(gp.need, self.dtype).itemsize for g, gp in paged}
         step = o.max_step_tokens or self.max_model_len or 0
         want = {}
         for g, gp in paged:
@@ -242,6 +265,14 @@ class Engine:
                     f"memory_bytes={o.memory_bytes} leaves no room for a cache page in every group "
                     f"(a page of each group takes {sum(page_bytes.values())} bytes, state slots "
                     f"{state_bytes})")
+        return _CacheSizes(asked, want, page_bytes, state_bytes)
+
+    def _alloc_cache(self, sizes: _CacheSizes):
+        """Pools and device tensors of every cache group."""
+        o, plan = self.options, self.model.cache_plan
+        asked, want, page_bytes = sizes.asked, sizes.pages, sizes.page_bytes
+        for part in self.model.all_parts():
+            part.check_cache(o.page_size)
         self.num_pages = max(want.values()) if want else 0
         groups, self._paged_group_of, self.kv, self.state = [], {}, {}, {}
         self._capacity = []
@@ -254,7 +285,7 @@ class Engine:
                     shape = (2, need.kv_heads, o.page_size * need.head_dim)
                 else:       # keys and values of different widths (or no values): the mixer lays a page out
                     shape = (need.kv_heads * o.page_size * (need.head_dim + need.value_width),)
-                self.kv[g] = torch.zeros(gp.entries, want[g], *shape, dtype=dtype_of(need, self.dtype),
+                self.kv[g] = torch.zeros(gp.entries, want[g], *shape, dtype=_cache_dtype(need, self.dtype),
                                          device=self.device)
                 self._capacity.append(
                     f"group{g}: {gp.entries} layers, {need.kv_heads} KV heads of {need.head_dim}"
@@ -266,7 +297,7 @@ class Engine:
                     + (f" (asked for {asked} pages)" if want[g] != asked else ""))
             else:
                 self.state[g] = torch.zeros(gp.entries, o.max_requests, *need.state_shape,
-                                            dtype=dtype_of(need, torch.float32), device=self.device)
+                                            dtype=_cache_dtype(need, torch.float32), device=self.device)
                 self._capacity.append(
                     f"group{g}: {gp.entries} layers with state {tuple(need.state_shape)} in {o.max_requests} slots, "
                     f"{self.state[g].numel() * self.state[g].element_size() / 2**20:.1f} MiB")

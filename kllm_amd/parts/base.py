@@ -132,6 +132,7 @@ class Runtime:
     options: Dict[str, Any] = field(default_factory=dict)
     shared: Dict[int, Any] = field(default_factory=dict)   # parts used by several layers
     tensor_epoch: int = 0                   # grows when parts may hold other tensors than before
+    second_copies: bool = True              # whether a float32 model has room for second copies of its matrices
 
     def __post_init__(self):
         if self.workspace is None:

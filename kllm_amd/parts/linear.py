@@ -163,21 +163,15 @@ def tiled_copy(runtime, w, kind, rope=None):
     (``K.fused_linear_tile``), or None where that kernel does not run: other dtypes, sizes it
     does not take, or ``EngineOptions.extra["no_tiled_weights"]`` (the copies double the
     memory of the weights they are made of; decode batches of 2 to 16 tokens stream them 20 to
-    30 % faster than the row-major matrix).  float32: ``_room_for_copy``."""
+    30 % faster than the row-major matrix).  float32: only where the engine found room for all of them behind
+    its cache (``Runtime.second_copies``); without them 5 to 16 tokens at 1.1B sizes take 1.76 to 1.97 ms a step, with
+    them 1.66 to 1.83, and the sums are the same."""
     if (w is None or not w.is_cuda or w.shape[1] % (4 if w.dtype == torch.float32 else 8)
             or runtime.options.get("no_tiled_weights") or runtime.options.get("no_fused_linear")):
         return None
-    if w.dtype == torch.float32 and (runtime.options.get("no_mfma_f32") or not _room_for_copy(w)):
+    if w.dtype == torch.float32 and (runtime.options.get("no_mfma_f32") or not runtime.second_copies):
         return None
     return K.fused_linear_tile(w, kind, rope)
-
-
-def _room_for_copy(w):
-    """Whether half of the card's memory stays free behind a copy of w: a float32 model that fills
-    more of it runs from the row-major matrices alone (5 to 16 tokens at 1.1B sizes: 1.76 to 1.97 ms a step
-    without the copies, 1.66 to 1.83 with them; the sums are the same)."""
-    free, total = torch.cuda.mem_get_info(w.device)
-    return free - w.numel() * w.element_size() >= total // 2
 
 
 def fused_f32(rt, n):

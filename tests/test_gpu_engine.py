@@ -703,6 +703,36 @@ def test_command_line_generate(model_dirs):
     assert lines[1] == "generated: [" + " ".join(map(str, want)) + "]"
 
 
+def test_second_copies_of_float32_matrices_leave_room_for_the_cache(model_dirs, monkeypatch):
+    """The copies are made of all matrices or of none: where half of the card stays beside weights, copies and the cache
+    that was asked for.  A card that the engine fills without them, one byte too small to hold them too, gets none; the
+    logits are the same bits either way."""
+    from kllm_amd.engine import Engine, EngineOptions, StepEntry
+    cfg, d = tiny.CONFIGS["A"], model_dirs("A")
+    options = dict(dtype="float32", max_tokens=4096, max_model_len=256)
+
+    def copies(engine):
+        made = [c for part in engine.model.all_parts() for c in getattr(part, "_tiled", {}).values()]
+        assert made and (all(c is None for c in made) or all(c is not None for c in made))
+        return made[0] is not None
+
+    def logits(engine):
+        engine.step([StepEntry(i, tiny.tokens(cfg, 20 + i, i), []) for i in range(8)])
+        return engine.step([StepEntry(i, tiny.tokens(cfg, 1, 50 + i), [0]) for i in range(8)]).clone()
+    first = Engine.from_dir(d, EngineOptions(**options))
+    assert copies(first)
+    weights = 4 * sum({s.name: s.shape.numel() if hasattr(s.shape, "numel") else int(np.prod(s.shape))
+                       for s in first.model.weight_specs()}.values())
+    room = 2 * (2 * weights + first.cache_bytes())
+    for free, total, want in ((room - weights, room, True), (room - 2 - weights, room - 2, False),
+                              (weights + first.cache_bytes() - 1, 4 * room, False)):
+        monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device=None: (free, total))
+        engine = Engine.from_dir(d, EngineOptions(**options))
+        monkeypatch.undo()
+        assert copies(engine) is want, (free, total)
+    assert torch.equal(logits(first), logits(engine))
+
+
 def test_command_line_options_of_the_engine_sizes(model_dirs):
     """--page-size, --num-pages, --max-step-tokens, --max-new-tokens and --sample-seed: a
     prompt longer than the step's budget is cut into portions, the tokens stay the same,

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from kllm_amd import kernels as K
+from kllm_amd.engine.engine import room_for_copies
 from kllm_amd.parts.linear import choose
 
 BF16, F32 = torch.bfloat16, torch.float32
@@ -54,3 +55,12 @@ def test_no_slice_of_k_is_empty(n, dtype):
 ])
 def test_slices_of_a_decode_batch(n, m, k, dtype, slices):
     assert choose(dtype, n, m, k)[1] == slices
+
+
+@pytest.mark.parametrize("weights,cache,free,total,room", [
+    (4, 1, 280, 288, True), (32, 80, 250, 288, True), (32, 81, 250, 288, False),    # half of the card stays
+    (32, 230, 250, 288, False), (100, 0, 180, 288, False),
+    (32, 80, 112, 288, True), (32, 80, 111, 288, False),                            # copies and cache fit into what is free
+])
+def test_room_for_second_copies_counts_the_cache(weights, cache, free, total, room):
+    assert room_for_copies(weights, cache, free, total) is room
