@@ -423,7 +423,7 @@ bool attn_f32_fits(int hd, int page_size) {
 
 extern "C" int kllm_attn_f32_fits(int hd, int page_size) { return attn_f32_fits(hd, page_size) ? 1 : 0; }
 
-int attn_f32_slices(int n, int KV, int H, int max_keys) {
+int attn_f32_slices(int n, int KV, int H, int hd, int max_keys) {
   // About four waves per CU across the chip (eight from one group per CU on, where partial
   // results cost little beside the keys), shared out over tokens x KV heads x blocks of 32
   // heads; a slice is one wave and should have 32 keys at least (measured: 64 tokens at 2,048
@@ -436,11 +436,16 @@ int attn_f32_slices(int n, int KV, int H, int max_keys) {
   long most = max_keys > 0 ? max_keys / 32 : 64;
   if (most > kAttnF32MaxSlices) most = kAttnF32MaxSlices;
   // Up to 128 keys (a tile of 32 a wave) the second kernel costs more than the keys: one workgroup's four
-  // slices, which write the output (8 tokens x 4 KV heads of 64, in us, in a replayed graph: 64 keys 9.5, with two
-  // slices and the merge 11.1; 128 keys 9.9 against 12.0; 8 KV heads of 128: 13.7 against 16.6, 15.5 against
-  // 18.0).  Beyond it the matrix products of a second tile on the same SIMDs cost what the merge does (256 keys: 13.4
-  // with four slices, 13.1 with eight waves to a workgroup, 12.2 with eight slices and the merge).
-  if (max_keys > 0 && max_keys <= 32 * kF32Waves && want >= kF32Waves) return kF32Waves;
+  // slices, which write the output (8 tokens x 4 KV heads of 64, in us, in a replayed graph: 64 keys 10.0, with two
+  // slices and the merge 11.5; 128 keys 10.4 against 12.5; 8 KV heads of 128: 14.4 against 17.0, 16.1 against
+  // 18.5).  Beyond it the matrix products of a second tile on the same SIMDs cost what the merge does (256 keys: 13.4
+  // with four slices, 13.1 with eight waves to a workgroup, 12.2 with eight slices and the merge).  Up to 64 keys, where two of
+  // the four waves have no tile, only while the workgroup's own merge is short (16 heads of 128 to a KV head, one token: 16.6
+  // against 15.2; 32 of 64: 12.7 against 11.5; 4 of 128: 14.2 against 17.0) and the groups are no more than CUs (512: 27.3
+  // against 18.6).  One tile of keys: one wave writes the output (8 tokens, 32 heads of 64 to a KV head: 9.9, in four slices 12.7).
+  const int heads = H / KV < 32 ? H / KV : 32;
+  const bool whole = max_keys > 64 ? max_keys <= 32 * kF32Waves : max_keys > 32 && heads * hd < 2048 && groups <= cus;
+  if (whole && want >= kF32Waves) return kF32Waves;
   if (want > most) want = most;
   if (want < 1) want = 1;
   return (int)want;

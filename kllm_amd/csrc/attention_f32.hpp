@@ -32,6 +32,6 @@ int attn_f32_prefill(const float* q, float* out, const float* cache, const int* 
 
 // Slices proposed for a decode batch of n tokens whose longest request has at most max_keys
 // keys (0: unknown).
-int attn_f32_slices(int n, int KV, int H, int max_keys);
+int attn_f32_slices(int n, int KV, int H, int hd, int max_keys);
 
 }  // namespace kllm

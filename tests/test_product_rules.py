@@ -64,3 +64,14 @@ def test_slices_of_a_decode_batch(n, m, k, dtype, slices):
 ])
 def test_room_for_second_copies_counts_the_cache(weights, cache, free, total, room):
     assert room_for_copies(weights, cache, free, total) is room
+
+
+@pytest.mark.parametrize("n,KV,H,hd,keys,slices", [
+    (8, 4, 32, 64, 128, 4), (8, 4, 32, 64, 64, 4), (8, 4, 32, 64, 32, 1), (8, 4, 32, 64, 16, 1), (16, 1, 40, 32, 64, 4),
+    (1, 1, 16, 128, 64, 2), (8, 1, 64, 64, 64, 2), (1, 1, 16, 128, 128, 4),      # long merges
+    (8, 32, 32, 128, 64, 4), (9, 32, 32, 128, 64, 2),                             # more groups than CUs
+])
+def test_slices_of_short_contexts_in_float32(n, KV, H, hd, keys, slices):
+    """One workgroup's four slices where they are the faster: not for a single tile of keys, nor for two where
+    its merge is long or the groups are many."""
+    assert K.attn_decode_slices(n, KV, H, hd, F32, keys) == slices
