@@ -431,26 +431,26 @@ def test_gemm_swiglu_at_prompt_sizes(n, f, k, dtype):
 ])
 def test_prompt_products_on_every_tile(n, m, k, nsplit, gate, tile):
     """bfloat16 products on the tiles against a product in double, at the edges of tiles,
-    stages and slices, and nothing written beside the output.  A sum of k products of unit normals in
-    32 bits is off by less than k^1/2 2^-24 times a few; the bound leaves a factor of eight."""
+    stages and slices, and nothing written beside the output (``sum_bound``; the gate's result is rounded to
+    bfloat16 besides)."""
     k_ = K()
     assert k_.gemm_prompt_tile(n, m, k, nsplit, gate, torch.bfloat16, torch.bfloat16 if gate else torch.float32) == tile
     rows = 2 * m if gate else m
     x = rnd(n, k, seed=1, dtype=torch.bfloat16)
     w = rnd(rows, k, seed=2, dtype=torch.bfloat16, scale=k ** -0.5 if gate else 1.0)
-    want = _gpu_reference(x, w)
+    want, off = _gpu_reference(x, w), sum_bound(x, w)
     guard = torch.full((n * m * nsplit + 64,), 7.0, device=DEV, dtype=torch.bfloat16 if gate else torch.float32)
     if gate:
         h = guard[:n * m].view(n, m)
         h.fill_(float("nan"))
         k_.gemm_swiglu(x, w, h)
-        want = P.silu(want[:, :m]) * want[:, m:]
-        assert (h.double() - want).abs().max() < 0.005 * want.abs().max()
+        want, off = gate_bound(want, off, 2.0 ** -8)
+        assert ((h.double() - want).abs() <= off).all()
     else:
         y = guard[:n * m * nsplit].view(nsplit, n, m)
         y.fill_(float("nan"))
         k_.gemm(x, w, y, k_.GEMM_MFMA_BF16, nsplit)
-        assert (y.double().sum(0) - want).abs().max() < 1e-5 * max(k, 64) ** 0.5 * 8
+        assert ((y.double().sum(0) - want).abs() <= off).all()
     assert bool((guard[n * m * nsplit:] == 7.0).all())
 
 
@@ -460,22 +460,74 @@ def test_prompt_products_on_every_tile(n, m, k, nsplit, gate, tile):
     (257, 515, 1028, 3, False, (64, 128)), (511, 4099, 260, 1, False, (64, 128)),
 ])
 def test_float32_prompt_products_on_every_tile(n, m, k, nsplit, gate, tile):
-    """The same tiles with 32-bit operands; the bound as above, for the gate in 32 bits too."""
+    """The same tiles with 32-bit operands; the bounds as above, for the gate in 32 bits too."""
     k_, f32 = K(), torch.float32
     assert k_.gemm_prompt_tile(n, m, k, nsplit, gate, f32, f32) == tile
     x, w = rnd(n, k, seed=1), rnd(2 * m if gate else m, k, seed=2, scale=k ** -0.5 if gate else 1.0)
-    want = _gpu_reference(x, w)
+    want, off = _gpu_reference(x, w), sum_bound(x, w)
     guard = torch.full((n * m * nsplit + 64,), 7.0, device=DEV)
     y = guard[:n * m * nsplit].view(nsplit, n, m)
     y.fill_(float("nan"))
     if gate:
         k_.gemm_swiglu(x, w, y[0])
-        want = P.silu(want[:, :m]) * want[:, m:]
-        assert (y[0].double() - want).abs().max() < 1e-5 * want.abs().max()
+        want, off = gate_bound(want, off, 16 * 2.0 ** -24)
+        assert ((y[0].double() - want).abs() <= off).all()
     else:
         k_.gemm(x, w, y, k_.GEMM_MFMA_F32, nsplit)
-        assert (y.double().sum(0) - want).abs().max() < 1e-5 * max(k, 64) ** 0.5 * 8
+        assert ((y.double().sum(0) - want).abs() <= off).all()
     assert bool((guard[n * m * nsplit:] == 7.0).all())
+
+
+def sum_bound(x, w):
+    """How far sums of 32-bit products may be from x . w^T.  Each of k additions rounds by at most u = 2^-24 of a partial
+    sum, evenly within it, and partial sums of independent terms grow as a random walk towards |x| |w|: the
+    error's standard deviation is below u |x| |w| / 6^1/2 whatever the order and the number of slices, and 4 u |x| |w| is
+    beyond nine of them.  (Operands cut to 16 bits of mantissa leave a deviation of 100 / k^1/2 u |x| |w|.)"""
+    return 4 * 2.0 ** -24 * x.double().norm(dim=1)[:, None] * w.double().norm(dim=1)[None, :]
+
+
+def gate_bound(sums, off, rounding):
+    """silu(gate) * up of sums that are off by ``off`` (silu's slope is below 1.1), the result rounded."""
+    m = sums.shape[1] // 2
+    g, up, eg, eu = sums[:, :m], sums[:, m:], off[:, :m], off[:, m:]
+    want = P.silu(g) * up
+    return want, 1.1 * eg * up.abs() + eu * P.silu(g).abs() + 1.1 * eg * eu + rounding * want.abs()
+
+
+@pytest.mark.parametrize("n,m,k,dtype", [
+    (2, 3, (1 << 23) + 8, torch.bfloat16), (65, 3, (1 << 23) + 8, torch.bfloat16), (2, 130, (1 << 24) + (1 << 18) + 8, torch.bfloat16),
+    (2, 3, (1 << 23) + 4, torch.float32), (65, 3, (1 << 23) + 4, torch.float32), (2, 130, (1 << 23) + (1 << 17) + 4, torch.float32),
+])
+def test_products_of_a_k_beyond_32_bit_offsets(n, m, k, dtype):
+    """K from 2^23 on takes kernels with 64-bit offsets within a tile (the last of 128 rows of W begins 4.3 GB behind the
+    first).  Operands of -1, 0 and 1: every partial sum is a whole number below 2^24, so the results are exact."""
+    k_ = K()
+    g = torch.Generator(device=DEV).manual_seed(k)
+
+    def ints(rows):
+        out = torch.empty(rows, k, device=DEV, dtype=dtype)
+        for r in range(rows):
+            out[r] = torch.randint(-1, 2, (k,), generator=g, device=DEV, dtype=torch.int8)
+        return out
+    x, w = ints(n), ints(m)
+    want = torch.zeros(n, m, device=DEV, dtype=torch.float64)
+    for a in range(0, k, 1 << 20):
+        want += _gpu_reference(x[:, a:a + (1 << 20)], w[:, a:a + (1 << 20)])
+    assert k_.gemm_prompt_tile(n, m, k, 1, False, dtype, torch.float32) == (64, 128)
+    algo = k_.GEMM_MFMA_BF16 if dtype == torch.bfloat16 else k_.GEMM_MFMA_F32
+    for nsplit in {1, 3, k_.gemm_prompt_slices(n, m, k, dtype)}:
+        y = torch.full((nsplit, n, m), float("nan"), device=DEV)
+        k_.gemm(x, w, y, algo, nsplit)
+        assert torch.equal(y.double().sum(0), want), nsplit
+    h = torch.full((n, m), float("nan"), device=DEV, dtype=dtype)
+    k_.gemm_act(x, w, h, k_.ACT_RELU_SQ)
+    square = want.clamp_min(0).pow(2)
+    assert ((h.double() - square).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -23) * square).all()
+    if m % 2 == 0:
+        h = torch.full((n, m // 2), float("nan"), device=DEV, dtype=dtype)
+        k_.gemm_swiglu(x, w, h)
+        gated = P.silu(want[:, :m // 2]) * want[:, m // 2:]
+        assert ((h.double() - gated).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -20) * gated.abs() + 1e-30).all()
 
 
 @pytest.mark.parametrize("n,m,k", [(9, 1000, 1004), (17, 2048, 14336), (33, 2048, 64), (65, 2048, 2048), (65, 2560, 2048),
@@ -544,7 +596,7 @@ def test_decode_tiles_take_whole_slices_of_512_up_to_48_rows(n, m, k, slices):
     x, w = rnd(n, k, seed=1, dtype=torch.bfloat16, scale=0.5), rnd(m, k, seed=2, dtype=torch.bfloat16, scale=0.05)
     parts = torch.full((nsplit, n, m), float("nan"), device=DEV)
     k_.gemm(x, w, parts, algo, nsplit)
-    assert (parts.cpu().double().sum(0) - _gpu_reference(x, w).cpu()).abs().max() < 1e-5 * k ** 0.5 * 8
+    assert ((parts.double().sum(0) - _gpu_reference(x, w)).abs() <= sum_bound(x, w)).all()
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
@@ -1442,6 +1494,23 @@ def test_float32_decode_of_short_contexts_writes_the_output_itself(H, KV, hd, ps
     part = torch.full((7 * H * 4 * (hd + 2),), float("nan"), device=DEV)
     K().attn_decode(c["q"], out, part, c["cache"], c["pos"], c["sot"], c["bt"], ps, H, KV, hd, window, c["scale"], 4)
     assert (out.cpu().double() - c["want"]).abs().max() < attn_tol(torch.float32)
+    assert torch.isnan(part).all()
+
+
+@pytest.mark.parametrize("H,KV,hd,ps", [(4, 2, 16, 16), (32, 4, 64, 16), (40, 1, 32, 16), (6, 3, 80, 32), (2, 1, 128, 16), (128, 1, 64, 16)])
+@pytest.mark.parametrize("window", [0, 24])
+def test_decode_of_up_to_256_keys_is_one_workgroup_a_group(H, KV, hd, ps, window):
+    """bfloat16, up to 256 keys: one slice, whose eight waves write the output (fewer keys than waves take, whole tiles and one
+    more or less, more heads than a workgroup's sixteen); nothing goes through the room for partial results.  Beyond
+    256 keys, and for heads beyond 128, there are slices again."""
+    bf16 = torch.bfloat16
+    assert all(K().attn_decode_slices(n, KV, H, hd, bf16, keys) == 1 for n in (1, 9) for keys in (16, 128, 256))
+    assert K().attn_decode_slices(1, KV, H, hd, bf16, 257) > 1 and K().attn_decode_slices(1, 2, 4, 256, bf16, 256) > 1
+    c = attention_case(H, KV, hd, ps, bf16, window, [(a, 1) for a in (0, 1, 15, 16, 31, 32, 33, 127, 128, 254, 255)], seed=7)
+    out = torch.full_like(c["q"], float("nan"))
+    part = torch.full((11 * H * (hd + 2),), float("nan"), device=DEV)
+    K().attn_decode(c["q"], out, part, c["cache"], c["pos"], c["sot"], c["bt"], ps, H, KV, hd, window, c["scale"], 1)
+    assert (out.cpu().double() - c["want"]).abs().max() < attn_tol(bf16)
     assert torch.isnan(part).all()
 
 
