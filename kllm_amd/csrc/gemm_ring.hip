@@ -34,7 +34,7 @@
 // the matrix unit's rate bounds everything, and what counts is that the CUs get equal numbers of tiles, three of
 // 64 x 128 a CU at a time.  In us against the four-wave tiles of 128 x 128 before (and K in up to 16 slices for
 // few rows): 700 x 11,264 x 2,048 with the gate 389 -> 264 (528 tiles of 128 x 128 on 256 CUs: three on some),
-// 700 x 2,048 x 5,632 238 -> 141, 72 x 11,264 x 2,048 150 -> 87, 2,048 x 11,264 x 2,048 777 -> 707.  Tiles of
+// 700 x 2,048 x 5,632 238 -> 141, 72 x 11,264 x 2,048 150 -> 76, 2,048 x 11,264 x 2,048 777 -> 697.  Tiles of
 // 128 x 128 in this kernel: 900 x 11,264 x 2,048 510 (two a CU: what is left for the last round goes to
 // CUs in pairs) against 384.
 // A float32 sum's products go in two chains of accumulators, the halves of every phase's K, added at the
@@ -330,19 +330,22 @@ __global__ __launch_bounds__(512, sizeof(T) == 4 ? 6 : 2) void gemm_ring_kernel(
 // 2,560 x 2,048 in 16 8.1 / 9.3).  The two- and three-stage tiles of 64 x 64 and 64 x 128 before, at 64 rows: 11,264
 // x 2,048 15.1, with the gate 30.3 (now 19.6); 12,288 x 4,096 28.4; 4,096 x 14,336 in 8 29.3; 28,672 x 4,096
 // with the gate 61.2 (52.5); 2,048 x 2,048 in 8 6.4 (6.2); float32: 2,048 x 5,632 in 16 29.2 (in 15 slices of 384
-// 20.2; in 11 24.3, in 8 30.4).
+// 19.4; in 11 23.1, in 8 28.8).
 //
 // More rows:
 // A product's time in us is put together from what a tile costs a CU: rounds of the chip times (stages
 // x a stage's time + what a tile costs beside its stages), against the time its weights need from
 // memory, plus its output and a launch.  The constants for bfloat16 are fitted to a sweep of 13 numbers of rows
 // from 72 to 2,048 and 12 sizes of W from 2,048 x 2,048 to 28,672 x 4,096, with every tile and 1 to 8
-// slices (2,700 products on the full chip, at the clock it holds there): 10 % spread around the
-// fit; the tile and slices that it chooses take 0.9 % longer than the fastest of the
-// sweep on the mean, 12 % at worst.  A 256 x 128 and a 128 x 192 tile were in the sweep too and won nothing
+// slices (2,700 products on the full chip): the tile and slices that it chooses take 0.9 % longer than the fastest of
+// the sweep on the mean, 12 % at worst.  It compares tiles, and is no forecast: single products of the sweep are 10 % around it
+// (estimated / measured alone in us: 72 x 2,048 x 2,048 6.8 / 7.0; 1,500 x 2,048 x 5,632 40 / 41; 1,024 x 4,096 x 4,096 33 / 36), and
+// where products run long enough for power to lower the clock every tile takes longer by about as much (2,048 x
+// 28,672 x 4,096 with the gate 293 / 358 to 391 from run to run; 2,048 x 11,264 x 2,048 67 / 80 to 88; 500 x 22,016 x 4,096
+// 64 / 72 to 79; 2,048 x 4,096 x 14,336 in two slices 136 / 163 to 175).  A 256 x 128 and a 128 x 192 tile were in the sweep too and won nothing
 // that these four do not come within a per cent of.  float32: a stage's products at the rate that the
-// matrix unit reaches (138 TFLOP/s on the chip); one workgroup alone on its CU, a single chain of
-// products a wave, takes a third longer.
+// matrix unit reaches (138 TFLOP/s on the chip); one workgroup alone on its CU took a third longer when the
+// constants were made (a single chain of products a wave; two since).
 struct RingTile {
   int rows, cols;          // of a product without a gate (with one: half as many columns)
   int per_cu;              // workgroups a CU holds

@@ -27,7 +27,7 @@ extern "C" {
 #define KLLM_GEMM_SKINNY_BF16 3
 #define KLLM_GEMM_GEMV 4
 #define KLLM_GEMM_GEMV_LDS 5 /* kllm_gemv_plain, reached through the Python wrapper */
-#define KLLM_GEMM_MFMA_F32 6 /* MFMA 32x32x2 with 32-bit operands: no reduced precision */
+#define KLLM_GEMM_MFMA_F32 6 /* MFMA 16x16x4 with 32-bit operands: no reduced precision */
 
 /* Copies the calling thread's last error text; returns its length. */
 int kllm_last_error(char* buf, int len);
@@ -232,8 +232,8 @@ int kllm_attn_generic(const void* q, void* out, const void* cache, const int* po
  * or 8 waves to a slice; head sizes 16..128 in steps of 16, 192,
  * 256, pages a multiple of 16; float32: one wave to a slice, 32-bit MFMA, head
  * sizes in steps of 8, pages a multiple of 4); `part` is float32 scratch of
- * n*H*nslices*(hd+2) elements (bfloat16 with one slice writes the output at once
- * and leaves it untouched).  kllm_attn_decode_slices proposes nslices for a batch
+ * n*H*nslices*(hd+2) elements (one slice, and in float32 four, write the output at once
+ * and leave it untouched).  kllm_attn_decode_slices proposes nslices for a batch
  * whose longest request has at most max_keys keys (0: unknown, as for contexts
  * of 2,048).  With token_list only the n_listed tokens it names are computed (q,
  * out and part stay indexed by token row). */

@@ -71,12 +71,13 @@ def _no_empty_slice(nsplit, k, unit):
 
 def _mfma_f32_split(n, m, k):
     """Slices of K for the float32 MFMA kernel.  Up to 64 rows (one row of tiles of 64 x 128) a wave's
-    own chain of products bounds the time, so a product should give every SIMD several waves:
-    up to 16 slices of at least 128 of K."""
+    own chain of products bounds the time, so a CU should have two tiles side by side: up to 16 slices of
+    at least 128 of K (2,048 x 5,632 at 64 rows, in us with the sum of the slices: 33 with 8, 27 with 11, 23 with 15; 4,096 x
+    14,336 75 with 8, 70 with 16)."""
     if n > 64:
         return K.gemm_prompt_slices(n, m, k, torch.float32)
-    waves = -(-m // 128) * 2
-    nsplit = max(1, min(16, k // 128, -(-4 * K.device_cus() // waves)))
+    tiles = -(-m // 128)
+    nsplit = max(1, min(16, k // 128, -(-2 * K.device_cus() // tiles)))
     return _no_empty_slice(nsplit, k, _PAIR_F32)
 
 
@@ -93,14 +94,16 @@ def _tiles_beat_skinny(n, m, k):
 
 
 def _decode_tile_split(n, m, k):
-    """Slices of K for a decode batch on the tiled kernel (one row of tiles of 64).  Below 40 M weights,
-    counted in tiles of 64 columns: slices of at least 256 of K until every CU has a workgroup, then
-    further ones of at least 512, up to 16 (measured at 64 rows, in us by slices: 2,048 x 5,632:
-    14.9 with 4, 10.7 with 8; 11,264 x 2,048: 13.2 with 2, 14.1 with 4, 16.5 with 8; 4,096 x 4,096:
-    12.2 with 4, 10.4 with 8, 11.8 with 16).  Where that stops between two powers and the tiles of 128
+    """Slices of K for a decode batch on the tiled kernel (one row of tiles of 64).  Below 40 M weights: slices of
+    at least 256 of K until every second CU has a tile of 128 columns, then
+    further ones of at least 512, up to 16 (at 64 rows, in us by slices, alone in a graph / with the sums added: 2,048 x 5,632:
+    13.0 / 14.9 with 4, 9.4 / 11.5 with 8; 2,048 x 2,048: 7.1 / 8.9 with 4, 5.8 / 7.6 with 8; 4,096 x 4,096: 11.3 / 13.8 with 4, 10.1 /
+    13.2 with 8, 11.4 / 15.5 with 16; 11,264 x 2,048, which gets four: 12.0 / 15.7 with 2, 13.2 / 17.3 with 4, 14.0 / 19.2 with 8;
+    at 17 rows 11.1 / 13.2, 10.6 / 13.0 and 10.8 / 13.5).  Where that stops between two powers and the tiles of 128
     columns leave CUs idle: as many slices of 512 as there are (2,048 x 5,632 with the norm that adds
     the slices, 8 / 11 / 15: 17 rows 14.3 / 13.5 / 13.3, 32 rows 14.7 / 14.1 / 14.3, 48 rows 15.5 / 15.0 /
-    15.1; the sums of more slices cost more with every row).  Larger weights, in tiles of 128 columns: up to 8 slices
+    15.1; the sums of more slices cost more with every row: 8 / 11 with the sums added, 48 rows 10.8 / 9.8, 56 11.1 / 10.5, 64
+    11.5 / 11.0).  Larger weights: up to 8 slices
     of at least 512 of K towards two workgroups a CU, four where K is deep (12,288 x 4,096: 26.2
     with 2, 22.3 with 4, 24.6 with 8; 4,096 x 14,336: 34.4 with 4, 23.9 with 8)."""
     cus, nsplit = K.device_cus(), 1
