@@ -407,7 +407,6 @@ extern "C" int kllm_gemm(const void* x, const void* w, void* y, int n, int m, in
     const int stage = f32 ? 32 : 64, chunk = f32 ? 4 : 8;   // elements of K per stage, per 16 bytes
     KLLM_REQUIRE(dtype == (f32 ? DT_F32 : DT_BF16), "gemm mfma: algorithm %d does not take dtype %d", algo, dtype);
     KLLM_REQUIRE(nsplit == 1 || out_dtype == DT_F32, "gemm mfma: K is split only for float32 partial sums");
-    // (a slice is rounded up to two stages: a cut whose last slices that empties is taken, their sums are zeros)
     KLLM_REQUIRE(nsplit <= 16 && (long)(ceil_div(ceil_div(k, nsplit), stage) * stage) * (nsplit - 1) < k,
                  "gemm mfma: nsplit %d leaves an empty slice of K=%d", nsplit, k);
     KLLM_REQUIRE(k % chunk == 0 && aligned16(x) && aligned16(w),

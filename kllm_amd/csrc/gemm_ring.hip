@@ -130,7 +130,7 @@ __global__ __launch_bounds__(512, sizeof(T) == 4 ? 6 : 2) void gemm_ring_kernel(
   const int tcol = in_band / band_rows;
   const int row0 = (band * 8 + in_band - tcol * band_rows) * BM, col0 = tcol * BN;
 
-  // blockIdx.y: a slice of K (a multiple of two stages); its sums go to Y[blockIdx.y]
+  // blockIdx.y: a slice of K (a multiple of two stages, TAIL: of one); its sums go to Y[blockIdx.y]
   const int kbeg = blockIdx.y * kslice, klen = min(k, kbeg + kslice) - kbeg;    // (TAIL: may be empty, its sums are zeros)
   const int stages = TAIL ? max(2, (klen + 2 * STAGE - 1) / (2 * STAGE) * 2) : klen / STAGE;
   Y += (long)blockIdx.y * n * m;
@@ -329,8 +329,8 @@ __global__ __launch_bounds__(512, sizeof(T) == 4 ? 6 : 2) void gemm_ring_kernel(
 // slices 15.2 / 14.1; 12,288 x 4,096 in 4 24.5 / 22.3; in 8 24.6 / 27.8; 4,096 x 14,336 in 8 23.9 / 31.3;
 // 2,560 x 2,048 in 16 8.1 / 9.3).  The two- and three-stage tiles of 64 x 64 and 64 x 128 before, at 64 rows: 11,264
 // x 2,048 15.1, with the gate 30.3 (now 19.6); 12,288 x 4,096 28.4; 4,096 x 14,336 in 8 29.3; 28,672 x 4,096
-// with the gate 61.2 (52.5); 2,048 x 2,048 in 8 6.4 (6.2); float32: 2,048 x 5,632 in 16 29.2 (in 15 slices of 384
-// 19.4; in 11 23.1, in 8 28.8).
+// with the gate 61.2 (52.5); 2,048 x 2,048 in 8 6.4 (6.2); float32: 2,048 x 5,632 in 16 29.2 (in 16 slices of 352
+// 20.8; in 15 of 384 19.2, in 11 22.9, in 8 28.9).
 //
 // More rows:
 // A product's time in us is put together from what a tile costs a CU: rounds of the chip times (stages
@@ -366,12 +366,17 @@ static RingTiles ring_tiles(bool f32) {
   return {kRingTilesBf16, 4, 128};
 }
 
-static int ring_kslice(int k, int nsplit, int pair) { return ceil_div(ceil_div(k, nsplit), pair) * pair; }
+// K of a slice: whole pairs of stages; where that would leave the last slice empty, whole stages (the odd one's
+// partner is read as zeros: as many stages as with pairs, but every workgroup has products).
+static int ring_kslice(int k, int nsplit, int pair) {
+  const int slice = ceil_div(ceil_div(k, nsplit), pair) * pair;
+  return (long)slice * (nsplit - 1) < k ? slice : ceil_div(ceil_div(k, nsplit), pair / 2) * (pair / 2);
+}
 
 static float ring_time(const RingTile& t, int pair, int n, int m, int k, int nsplit, bool gate, int in_bytes, int out_bytes) {
   const long cus = device_cus();
   const long tiles = (long)ceil_div(n, t.rows) * ceil_div(m, gate ? t.cols / 2 : t.cols) * nsplit;
-  const int stages = ring_kslice(k, nsplit, pair) / (pair / 2);
+  const int stages = 2 * ceil_div(ring_kslice(k, nsplit, pair), pair);
   const long full = tiles / (t.per_cu * cus), rest = tiles % (t.per_cu * cus);
   float busy = (float)full * (stages * t.stage + t.tile);
   if (rest) {
@@ -442,7 +447,8 @@ static int ring_kind(int tile, const void* x, const void* w, void* y, int n, int
                      const float* ap, hipStream_t st) {
   constexpr int PAIR = 256 / sizeof(T);
   if (k >= kRingLongK) return ring_shape<T, TOUT, MODE, RING_LONG>(tile, x, w, y, n, m, k, nsplit, act, ap, st);
-  const bool whole = k % PAIR == 0 && (long)ring_kslice(k, nsplit, PAIR) * (nsplit - 1) < k;
+  const int slice = ring_kslice(k, nsplit, PAIR);
+  const bool whole = k % PAIR == 0 && slice % PAIR == 0 && (long)slice * (nsplit - 1) < k;
   return whole ? ring_shape<T, TOUT, MODE, RING_WHOLE>(tile, x, w, y, n, m, k, nsplit, act, ap, st)
                : ring_shape<T, TOUT, MODE, RING_TAIL>(tile, x, w, y, n, m, k, nsplit, act, ap, st);
 }
@@ -479,7 +485,7 @@ extern "C" int kllm_gemm_prompt_slices(int n, int m, int k, int dtype) {
   int best = 1;
   float least = 0.f;
   for (int ns : {1, 2, 3, 4, 6, 8}) {
-    const long slice = ring_kslice(k, ns, ring_tiles(f32).pair);
+    const long pair = ring_tiles(f32).pair, slice = ceil_div(ceil_div(k, ns), (int)pair) * pair;
     if (ns > 1 && (slice * (ns - 1) >= k || 10 * slice * ns > 11L * k)) continue;
     float us = 0.f;
     ring_tile(f32, n, m, k, ns, false, true, &us);

@@ -56,8 +56,9 @@ def _skinny_split(n, m, k):
     return _no_empty_slice(nsplit, k, 32)
 
 
-# K of two stages of the MFMA tiles, 256 bytes: what their slices are rounded up to
-_PAIR_BF16, _PAIR_F32 = 128, 64
+# K of a stage of the MFMA tiles, 128 bytes.  Their slices are rounded up to two stages, or to one where two
+# would leave the last slice empty.
+_STAGE_BF16, _STAGE_F32 = 64, 32
 
 
 def _no_empty_slice(nsplit, k, unit):
@@ -72,13 +73,13 @@ def _no_empty_slice(nsplit, k, unit):
 def _mfma_f32_split(n, m, k):
     """Slices of K for the float32 MFMA kernel.  Up to 64 rows (one row of tiles of 64 x 128) a wave's
     own chain of products bounds the time, so a CU should have two tiles side by side: up to 16 slices of
-    at least 128 of K (2,048 x 5,632 at 64 rows, in us with the sum of the slices: 33 with 8, 27 with 11, 23 with 15; 4,096 x
+    at least 128 of K (2,048 x 5,632 at 64 rows, in us with the sum of the slices: 32 with 8, 26 with 11, 24 with 16; 4,096 x
     14,336 75 with 8, 70 with 16)."""
     if n > 64:
         return K.gemm_prompt_slices(n, m, k, torch.float32)
     tiles = -(-m // 128)
     nsplit = max(1, min(16, k // 128, -(-2 * K.device_cus() // tiles)))
-    return _no_empty_slice(nsplit, k, _PAIR_F32)
+    return _no_empty_slice(nsplit, k, _STAGE_F32)
 
 
 def _tiles_beat_skinny(n, m, k):
@@ -118,7 +119,7 @@ def _decode_tile_split(n, m, k):
         reach = (4 if k >= 8192 and tiles <= cus else 2) * cus
         while nsplit * 2 <= min(8, reach // tiles, k // 512):
             nsplit *= 2
-    return _no_empty_slice(nsplit, k, _PAIR_BF16)
+    return _no_empty_slice(nsplit, k, _STAGE_BF16)
 
 
 def choose(dtype, n, m, k, options=None):

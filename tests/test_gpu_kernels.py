@@ -478,6 +478,23 @@ def test_float32_prompt_products_on_every_tile(n, m, k, nsplit, gate, tile):
     assert bool((guard[n * m * nsplit:] == 7.0).all())
 
 
+@pytest.mark.parametrize("n,m,k,nsplit,dtype", [
+    (17, 300, 1400, 8, torch.bfloat16), (64, 513, 7176, 13, torch.bfloat16), (130, 300, 4104, 10, torch.bfloat16),      # odd stages, a rest
+    (9, 300, 5632, 16, torch.float32), (65, 131, 700, 8, torch.float32)])
+def test_slices_of_an_odd_number_of_stages(n, m, k, nsplit, dtype):
+    """Cuts whose last slice is empty when a slice is rounded up to two stages (128 of K in bfloat16, 64 in float32) and
+    is not when rounded up to one: every slice's sums are those of its own K, so that none is empty."""
+    k_, stage = K(), 64 if dtype == torch.bfloat16 else 32
+    pairs, kslice = (-(-(-(-k // nsplit)) // u) * u for u in (2 * stage, stage))
+    assert pairs * (nsplit - 1) >= k > kslice * (nsplit - 1)
+    x, w = rnd(n, k, seed=1, dtype=dtype), rnd(m, k, seed=2, dtype=dtype)
+    y = torch.full((nsplit, n, m), float("nan"), device=DEV)
+    k_.gemm(x, w, y, k_.GEMM_MFMA_BF16 if dtype == torch.bfloat16 else k_.GEMM_MFMA_F32, nsplit)
+    for s in range(nsplit):
+        a, b = x[:, s * kslice:(s + 1) * kslice], w[:, s * kslice:(s + 1) * kslice]
+        assert ((y[s].double() - _gpu_reference(a, b)).abs() <= sum_bound(a, b)).all(), s
+
+
 def sum_bound(x, w):
     """How far sums of 32-bit products may be from x . w^T.  Each of k additions rounds by at most u = 2^-24 of a partial
     sum, evenly within it, and partial sums of independent terms grow as a random walk towards |x| |w|: the
@@ -544,7 +561,9 @@ def test_float32_products_add_in_two_chains(n, m, k):
     x, w = rnd(n, k, seed=1), rnd(m, k, seed=2, scale=0.02)
     algo, nsplit = choose(torch.float32, n, m, k)
     assert algo == k_.GEMM_MFMA_F32
-    kslice = -(-(-(-k // nsplit)) // 64) * 64
+    kslice = -(-(-(-k // nsplit)) // 64) * 64           # (two stages, or one where that leaves the last slice empty)
+    if kslice * (nsplit - 1) >= k:
+        kslice = -(-(-(-k // nsplit)) // 32) * 32
     parts = torch.empty(nsplit, n, m, device=DEV)
     k_.gemm(x, w, parts, algo, nsplit)
     total = parts[0].clone()
@@ -585,10 +604,10 @@ def test_split_product_into_its_consumers(n, m, k):
 
 
 @pytest.mark.parametrize("n", [17, 48, 49])
-@pytest.mark.parametrize("m,k,slices", [(2048, 5632, 11), (2048, 5640, 9), (2040, 7176, 12), (4096, 5632, 8)])
+@pytest.mark.parametrize("m,k,slices", [(2048, 5632, 11), (2048, 5640, 10), (2040, 7176, 13), (4096, 5632, 8)])
 def test_decode_tiles_take_whole_slices_of_512_up_to_48_rows(n, m, k, slices):
     """Up to 48 rows and while tiles of 128 columns leave CUs idle (not at 4,096 columns): one slice for
-    every whole 512 of K, fewer where rounding a slice up to two stages would leave the last one empty."""
+    every whole 512 of K, fewer where rounding a slice up to a stage would leave the last one empty."""
     from kllm_amd.parts.linear import choose
     k_ = K()
     algo, nsplit = choose(torch.bfloat16, n, m, k)

@@ -28,9 +28,9 @@ def test_slices_where_the_times_are_not_estimated(n, m, k, dtype, slices):
 @pytest.mark.parametrize("n", [9, 17, 33, 48, 49, 64, 65, 128, 700, 2048])
 @pytest.mark.parametrize("dtype", [BF16, F32])
 def test_no_slice_of_k_is_empty(n, dtype):
-    """The MFMA tiles round a slice up to two stages (256 bytes of K); the skinny kernel up to 32: with the
-    kernel's own rounding the last slice must hold something, for the widths of the models here and
-    for K around every multiple of those."""
+    """The MFMA tiles round a slice up to two stages (256 bytes of K), or to one where that leaves the last slice
+    empty; the skinny kernel up to 32: with the kernel's own rounding the last slice must hold something, for the
+    widths of the models here and for K around every multiple of those."""
     each = 8 if dtype == BF16 else 4
     ks = {k + d * each for k in (64, 512, 1024, 2048, 4096, 5632, 7168, 11008, 14336) for d in (-9, -1, 0, 1, 5)}
     cut = 0
@@ -43,14 +43,16 @@ def test_no_slice_of_k_is_empty(n, dtype):
                 continue
             unit = 32 if algo == K.GEMM_SKINNY_BF16 else 256 // (16 // each)
             kslice = -(-(-(-k // nsplit)) // unit) * unit
+            if algo != K.GEMM_SKINNY_BF16 and (nsplit - 1) * kslice >= k:
+                kslice = -(-(-(-k // nsplit)) // (unit // 2)) * (unit // 2)
             assert (nsplit - 1) * kslice < k, (m, k, nsplit, kslice)
             cut += nsplit > 1
     assert cut
 
 
 @pytest.mark.parametrize("n,m,k,dtype,slices", [
-    (17, 2048, 5632, F32, 15), (64, 2048, 5632, F32, 15),            # (of 384; sixteen would leave the last one empty)
-    (17, 2048, 5640, BF16, 9), (48, 2040, 7176, BF16, 12),           # (of 640)
+    (17, 2048, 5632, F32, 16), (64, 2048, 5632, F32, 16),            # (of 352; of 384 the last one would be empty)
+    (17, 2048, 5640, BF16, 10), (48, 2040, 7176, BF16, 13),          # (of 576, not 640)
     (17, 2048, 5632, BF16, 11), (49, 2048, 5632, BF16, 8), (17, 4096, 5632, BF16, 8),
 ])
 def test_slices_of_a_decode_batch(n, m, k, dtype, slices):
