@@ -131,8 +131,8 @@ __global__ __launch_bounds__(512, sizeof(T) == 4 ? 6 : 2) void gemm_ring_kernel(
   const int row0 = (band * 8 + in_band - tcol * band_rows) * BM, col0 = tcol * BN;
 
   // blockIdx.y: a slice of K (a multiple of two stages, TAIL: of one); its sums go to Y[blockIdx.y]
-  const int kbeg = blockIdx.y * kslice, klen = min(k, kbeg + kslice) - kbeg;    // (TAIL: may be empty, its sums are zeros)
-  const int stages = TAIL ? max(2, (klen + 2 * STAGE - 1) / (2 * STAGE) * 2) : klen / STAGE;
+  const int kbeg = blockIdx.y * kslice, klen = min(k, kbeg + kslice) - kbeg;    // (never empty)
+  const int stages = TAIL ? (klen + 2 * STAGE - 1) / (2 * STAGE) * 2 : klen / STAGE;
   Y += (long)blockIdx.y * n * m;
 
   // Loads: a wave takes an eighth of a sub-tile's rows, eight rows an instruction (four, with half its
@@ -301,14 +301,29 @@ __global__ __launch_bounds__(512, sizeof(T) == 4 ? 6 : 2) void gemm_ring_kernel(
         for (int j = 0; j < TN; ++j) {
           const int c = col0 + hw * WS + (wc * TN + j) * 16 + 4 * lch;
           typedef TOUT vec_t __attribute__((ext_vector_type(4)));
-          vec_t v;
+          floatx4 q;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            float s = sum(hx, hw, i, j, e);
-            if (GATE) s = gate_act(s, act) * sum(hx, 1, i, j, e);
-            if (MODE == RING_UNARY) s = unary_act(s, act, a_pos, a_neg);
-            v[e] = from_f32<TOUT>(s);
+            q[e] = sum(hx, hw, i, j, e);
+            if (GATE) q[e] = gate_act(q[e], act) * sum(hx, 1, i, j, e);
           }
+          if constexpr (MODE == RING_UNARY) {
+            // Larger tiles have one copy of the activations to four sums: with four the kernel's end alone is longer than the
+            // instruction cache, and at 256 x 256 its loops are no longer unrolled, so that the accumulators go through
+            // scratch memory (squared ReLU / tanh in us: 1,500 x 32,000 x 1,024 254 / 267 -> 130 / 162; 1,500 x 5,632 x 2,048 60 /
+            // 68 -> 46 / 55; 700 x 5,632 x 2,048 43 / 49 -> 35 / 40).  Tiles of 128 x 128 are faster with four (300 x 2,048
+            // x 2,048 24.2 / 28.5, with one 25.5 / 29.0).
+            if constexpr (TM * TN >= 4) {
+#pragma unroll 1
+              for (int e = 0; e < 4; ++e) q = floatx4{q[1], q[2], q[3], unary_act(q[0], act, a_pos, a_neg)};
+            } else {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) q[e] = unary_act(q[e], act, a_pos, a_neg);
+            }
+          }
+          vec_t v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = from_f32<TOUT>(q[e]);
           TOUT* dst = Y + (long)r * m + c;
           if (vec && c + 3 < m) {
             *reinterpret_cast<vec_t*>(dst) = v;
@@ -448,7 +463,7 @@ static int ring_kind(int tile, const void* x, const void* w, void* y, int n, int
   constexpr int PAIR = 256 / sizeof(T);
   if (k >= kRingLongK) return ring_shape<T, TOUT, MODE, RING_LONG>(tile, x, w, y, n, m, k, nsplit, act, ap, st);
   const int slice = ring_kslice(k, nsplit, PAIR);
-  const bool whole = k % PAIR == 0 && slice % PAIR == 0 && (long)slice * (nsplit - 1) < k;
+  const bool whole = k % PAIR == 0 && slice % PAIR == 0;
   return whole ? ring_shape<T, TOUT, MODE, RING_WHOLE>(tile, x, w, y, n, m, k, nsplit, act, ap, st)
                : ring_shape<T, TOUT, MODE, RING_TAIL>(tile, x, w, y, n, m, k, nsplit, act, ap, st);
 }

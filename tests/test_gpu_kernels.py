@@ -420,7 +420,7 @@ def test_gemm_swiglu_at_prompt_sizes(n, f, k, dtype):
 @pytest.mark.parametrize("n,m,k,nsplit,gate,tile", [
     (65, 515, 8, 1, False, (128, 128)), (65, 130, 64, 1, True, (128, 128)),         # less than a stage, one stage
     (127, 257, 72, 1, False, (128, 128)), (129, 64, 128, 1, True, (128, 128)),      # an odd number of stages; one pair
-    (193, 131, 192, 3, False, (128, 128)), (100, 96, 640, 4, False, (128, 128)),    # slices of K that hold nothing
+    (193, 131, 192, 3, False, (128, 128)), (100, 96, 640, 4, False, (128, 128)),    # slices of an odd number of stages
     (257, 515, 1032, 3, False, (128, 128)),
     (513, 7001, 520, 1, False, (128, 256)), (257, 5602, 520, 1, True, (128, 256)),  # ragged in rows, columns and K
     (2047, 4099, 520, 1, False, (256, 192)), (700, 5602, 520, 1, True, (256, 192)),
@@ -493,6 +493,24 @@ def test_slices_of_an_odd_number_of_stages(n, m, k, nsplit, dtype):
     for s in range(nsplit):
         a, b = x[:, s * kslice:(s + 1) * kslice], w[:, s * kslice:(s + 1) * kslice]
         assert ((y[s].double() - _gpu_reference(a, b)).abs() <= sum_bound(a, b)).all(), s
+
+
+@pytest.mark.parametrize("n,m,k,dtype,tile", [
+    (2049, 5635, 2056, torch.bfloat16, (256, 256)), (1500, 5631, 2056, torch.bfloat16, (256, 192)), (700, 5631, 520, torch.bfloat16, (128, 256)),
+    (257, 2050, 136, torch.bfloat16, (128, 128)), (60, 300, 136, torch.bfloat16, (64, 128)), (40, 40000, 520, torch.bfloat16, (64, 256)),
+    (130, 515, 260, torch.float32, (64, 128))])
+def test_an_activation_behind_a_product_on_every_tile(n, m, k, dtype, tile):
+    """The activations of sums, four at a time: the slopes of tanh and of the logistic function are 1 at most, so the
+    results are off by no more than the sums are and by their own rounding."""
+    k_ = K()
+    assert k_.gemm_prompt_tile(n, m, k, 1, False, dtype, dtype) == tile
+    x, w = rnd(n, k, seed=1, dtype=dtype), rnd(m, k, seed=2, dtype=dtype, scale=k ** -0.5)
+    sums, off = _gpu_reference(x, w), sum_bound(x, w)
+    for act, f in ((k_.ACT_TANH, torch.tanh), (k_.ACT_SIGMOID, torch.sigmoid)):
+        h = torch.full((n, m), float("nan"), device=DEV, dtype=dtype)
+        k_.gemm_act(x, w, h, act)
+        want = f(sums)
+        assert ((h.double() - want).abs() <= off + (2.0 ** -8 if dtype == torch.bfloat16 else 16 * 2.0 ** -24) * want.abs()).all()
 
 
 def sum_bound(x, w):
