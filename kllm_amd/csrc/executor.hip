@@ -51,6 +51,7 @@ static const Op kOps[] = {
     KLLM_CMD_OP(kllm_moe_combine),
     KLLM_CMD_OP(kllm_conv_state_update),
     KLLM_CMD_OP(kllm_gated_delta_prep),
+    KLLM_CMD_OP(kllm_gated_delta_factors),
     KLLM_CMD_OP(kllm_gated_delta_scan),
     KLLM_CMD_OP(kllm_linear_recurrence_prep),
     KLLM_CMD_OP(kllm_linear_recurrence_scan),

@@ -473,12 +473,19 @@ int kllm_gated_delta_prep(const float* proj, int nsplit, long split_stride, cons
                           const float* gate_sums, int g_ns, long g_stride, int g_row, int gate_sigmoid, float* dec,
                           hipStream_t stream);
 int kllm_gated_delta_max_dim(void);
+/* What the recurrence with one decay a head needs of every sixteen tokens of a span besides the state and the values.
+ * `factors`: kllm_gated_delta_factor_floats(H, G, dk) floats (-1: sizes that are not built) for each of the step's sixteens,
+ * of which there may be ceil(n / 16) + spans; aligned to 16 bytes. */
+int kllm_gated_delta_factor_floats(int H, int G, int dk);
+int kllm_gated_delta_factors(const float* qn, const float* kn, const float* gb, const int* span_start, float* factors,
+                             int n, int n_spans, int H, int G, int dk, hipStream_t stream);
 /* The recurrence: state [H][dk][dv] per slot, o_out [n][H dv].  `dec` (or null): decays per head and
- * key channel [n][H dk], which then take the place of gb's decay. */
+ * key channel [n][H dk], which then take the place of gb's decay.  `factors` (or null, and always
+ * null with `dec`): what kllm_gated_delta_factors made of the same tokens; sixteen tokens are then taken at a time. */
 int kllm_gated_delta_scan(const float* qn, const float* kn, const float* vv, const float* gb, float* o_out,
                           float* state, long slot_stride, const int* slots, const int* span_start,
-                          const int* span_pos, int n_spans, int H, int G, int dk, int dv, const float* dec,
-                          hipStream_t stream);
+                          const int* span_pos, int n, int n_spans, int H, int G, int dk, int dv, const float* dec,
+                          const float* factors, hipStream_t stream);
 /* Gated linear recurrence.  proj columns: y (W) | x (W).  wr_t, wi_t: the gates' block-diagonal matrices
  * [blocks][in][out]; rate [W] = 8 softplus(lambda).  Writes a and the added term, [n][W] each. */
 int kllm_linear_recurrence_prep(const float* proj, int nsplit, long split_stride, const float* x_bias,

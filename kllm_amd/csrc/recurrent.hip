@@ -299,6 +299,410 @@ __global__ __launch_bounds__(kRecThreads) void gated_delta_scan_kernel(
     }
 }
 
+// The same recurrence with one decay a head, sixteen tokens of a span at a time.  From the state S in front of them,
+// with G_i the product of the decays up to token i and G_ij that of those behind token j up to i,
+//   x_i = v_i - G_i (S^T k_i)          u_i = beta_i (x_i - sum_(j<i) G_ij (k_j . k_i) u_j)
+//   o_i = G_i (S^T q_i) + sum_(j<=i) G_ij (k_j . q_i) u_j          S' = G_15 S + sum_i G_15,i k_i u_i^T
+// u = M x with M = (1 + L)^-1 diag(beta), L_ij = beta_i G_ij (k_j . k_i) below the diagonal: what does not hang on the state
+// is made for all sixteens at once (`gated_delta_factors`), and the chain of a sixteen is matrix products.
+// Token by token each wave reads every token's key and query out of LDS and waits for two sums over its lanes; here
+// a sixteen takes 2,070 cycles, of which 928 are matrix instructions.  In us, token by token and both kernels here (the
+// factors' share), 16 heads of 128 x 128: 1,500 tokens 269 / 98 (12), 8 x 256 109 / 65 (14), 480 beside 8 single tokens 118 / 61 (9),
+// 64 16.6 / 13.3 (6).  Relative errors of the outputs against 64 bits, weak to strong decays: 1.9e-7 / 1.3e-7, 9.6e-8 / 8.6e-8,
+// 8.8e-8 / 7.1e-8.  Measured and not taken: four tokens at a time by 4 x 4 matrix instructions (236), sums of the waves'
+// shares in an order of each wave's own, the update's products before the outputs' (104).
+constexpr int kSixteen = 16;
+// The factors of a sixteen, in the order that the scan's lanes read them (tokens that are not there: zeros, decays of one).
+// Per head of keys: keys [channel / 4][token][4], queries likewise, keys [token / 4][channel][4]; channels in multiples of 64.
+// Per head: M [token j / 4][token i][4], G_ij (k_j . q_i) [j % 4][j / 4][i], (G_i, G_15,i) [i].
+// The sixteens of span s begin at number t0 / 16 + s of all (each span has one more than its sixteenth of the tokens at most).
+constexpr int kHeadFactors = 2 * kSixteen * kSixteen + 2 * kSixteen;
+
+__host__ __device__ inline long sixteen_floats(int H, int G, int rows) {
+  return (long)G * 3 * kSixteen * rows + (long)H * kHeadFactors;
+}
+
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_moved(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+
+// Four lanes' four numbers: lane l's number e becomes lane e's number l.
+__device__ __forceinline__ void transpose_four(floatx4& x, int lane) {
+  const bool odd = lane & 1, high = lane & 2;
+#pragma unroll
+  for (int e = 0; e < 4; e += 2) {
+    const float got = dpp_moved<0xB1>(odd ? x[e] : x[e + 1]);
+    x[e] = odd ? got : x[e];
+    x[e + 1] = odd ? x[e + 1] : got;
+  }
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const float got = dpp_moved<0x4E>(high ? x[e] : x[e + 2]);
+    x[e] = high ? got : x[e];
+    x[e + 2] = high ? x[e + 2] : got;
+  }
+}
+
+// Workgroup (sixteen, head of keys).  The sums go by the 64-bit matrix instruction (wave w takes the channels 16 w + 64 i),
+// then a wave makes a head's factors.  L to the power of 16 is zero, so that (1 + L)^-1 = (1 + L^8) (1 + L^4) (1 + L^2) (1 - L); an operand on the left is read from its transpose in the
+// layout of a result, so every power is made with its transpose.  Everything is 64-bit until it is written.
+template <int NB, bool V4>
+__global__ __launch_bounds__(kRecThreads, NB <= 2 && V4 ? 4 : 2) void gated_delta_factors_kernel(
+    const float* __restrict__ qn, const float* __restrict__ kn, const float* __restrict__ gb,
+    const int* __restrict__ span_start, float* __restrict__ factors, int n_spans, int H, int G, int dk) {
+  constexpr int T = kSixteen, WAVES = kRecThreads / kWave, ROWS = 64 * NB;
+  __shared__ doublex4 part[2][WAVES][kWave];
+  __shared__ double runs[WAVES][4][T];               // runs[w][p][l]: the decays of the 2^p tokens up to l
+  const int g = blockIdx.y, per = H / G, lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), low = lane % 16, high = lane / 16;
+  const int QK = G * dk;
+  auto mul = [](const doublex4& left_t, const doublex4& right, doublex4 c) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f64_16x16x4f64(left_t[e], right[e], c, 0, 0, 0);
+    return c;
+  };
+  const int number = blockIdx.x;
+  int span = -1;                                     // the last span that begins at this sixteen or before it
+  for (int s0 = 0; s0 < n_spans; s0 += kWave) {
+    const int s = min(s0 + lane, n_spans - 1);
+    const unsigned long long at = __ballot(s0 + lane < n_spans && span_start[s] / T + s <= number);
+    span += __popcll(at);
+    if (at != ~0ull) break;
+  }
+  const int t0 = span_start[span], t1 = span_start[span + 1];
+  const int t = t0 + (number - t0 / T - span) * T;
+  if (t >= t1) return;
+  const int nt = min(T, t1 - t), tok = t + min(low, nt - 1);
+  const bool there = low < nt;
+  const float* krow = kn + (long)tok * QK + (long)g * dk;
+  const float* qrow = qn + (long)tok * QK + (long)g * dk;
+  const float* grow = gb + (long)tok * 2 * H + g * per + min(wave, per - 1);
+  floatx4 k[NB], q[NB];
+#pragma unroll
+  for (int c = 0; c < NB; ++c) {
+    const int r = 16 * wave + 64 * c + 4 * high;
+    if constexpr (V4) {
+      k[c] = *reinterpret_cast<const floatx4*>(krow + min(r, dk - 4));
+      q[c] = *reinterpret_cast<const floatx4*>(qrow + min(r, dk - 4));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        k[c][e] = krow[min(r + e, dk - 1)];
+        q[c][e] = qrow[min(r + e, dk - 1)];
+      }
+    }
+  }
+  float d_low = grow[0], b_low = grow[H];
+  doublex4 kk = {0., 0., 0., 0.}, qk = {0., 0., 0., 0.};
+#pragma unroll
+  for (int c = 0; c < NB; ++c)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const bool ok = there && 16 * wave + 64 * c + 4 * high + e < dk;
+      k[c][e] = ok ? k[c][e] : 0.f;
+      q[c][e] = ok ? q[c][e] : 0.f;
+      const double kd = k[c][e], qd = q[c][e];
+      kk = __builtin_amdgcn_mfma_f64_16x16x4f64(kd, kd, kk, 0, 0, 0);
+      qk = __builtin_amdgcn_mfma_f64_16x16x4f64(qd, kd, qk, 0, 0, 0);
+    }
+  float* of_sixteen = factors + number * sixteen_floats(H, G, ROWS);
+  float* keys = of_sixteen + (long)g * 3 * T * ROWS;
+#pragma unroll
+  for (int c = 0; c < NB; ++c) {
+    const int quad = 4 * wave + 16 * c + high;
+    *reinterpret_cast<floatx4*>(keys + (quad * T + low) * 4) = k[c];
+    *reinterpret_cast<floatx4*>(keys + T * ROWS + (quad * T + low) * 4) = q[c];
+    transpose_four(k[c], lane);                    // tokens low / 4 * 4 .. + 3 of channel 4 quad + low % 4
+    *reinterpret_cast<floatx4*>(keys + 2 * T * ROWS + (low / 4 * ROWS + 4 * quad + low % 4) * 4) = k[c];
+  }
+  part[0][wave][lane] = kk;                        // element e of a result: row 4 e + high, column low
+  part[1][wave][lane] = qk;
+  __syncthreads();
+  for (int hh = wave; hh < per; hh += WAVES) {
+    const int h = g * per + hh;
+    if (hh > wave) {
+      d_low = gb[(long)tok * 2 * H + h];
+      b_low = gb[(long)tok * 2 * H + H + h];
+    }
+    double run = there ? (double)d_low : 1.;       // (a token that is not there decays nothing and writes nothing)
+    const double beta_low = there ? (double)b_low : 0.;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      runs[wave][p][low] = run;
+      const double before = __shfl(run, lane - (1 << p), kWave);
+      run *= low >= 1 << p ? before : 1.;
+    }
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_wave_barrier();
+    auto decays = [&](int upto, int count) {       // of the `count` tokens up to `upto`
+      double d = 1.;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const bool on = count >> p & 1;
+        const double v = runs[wave][p][max(upto, 0)];
+        d *= on ? v : 1.;
+        upto -= on ? 1 << p : 0;
+      }
+      return d;
+    };
+    float* f = of_sixteen + (long)G * 3 * T * ROWS + (long)h * kHeadFactors;
+    if (high == 0) *reinterpret_cast<float2*>(f + 2 * T * T + 2 * low) = float2{(float)run, (float)decays(T - 1, T - 1 - low)};
+    kk = part[0][0][lane];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) kk += part[0][w][lane];
+    qk = part[1][0][lane];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) qk += part[1][w][lane];
+    doublex4 L, LT, R;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int i = 4 * e + high, late = max(i, low);
+      const double between = decays(late, late - min(i, low)), beta = __shfl(beta_low, late, kWave);
+      double v = beta * between * kk[e];
+      if (!(fabs(v) < (double)INFINITY)) v = 0.;   // (x of a token that is not finite is not either: it needs no help from M)
+      L[e] = low < i ? v : 0.;
+      LT[e] = low > i ? v : 0.;
+      R[e] = (low == i ? 1. : 0.) - L[e];
+      f[T * T + low % 4 * 4 * T + low / 4 * T + i] = low <= i ? (float)(between * qk[e]) : 0.f;
+    }
+    const doublex4 zero = {0., 0., 0., 0.};
+    const doublex4 L2 = mul(LT, L, zero), L2T = mul(L, LT, zero);
+    R = mul(L2T, R, R);
+    const doublex4 L4 = mul(L2T, L2, zero), L4T = mul(L2, L2T, zero);
+    R = mul(L4T, R, R);
+    R = mul(mul(L4, L4T, zero), R, R);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) f[low / 4 * 4 * T + (4 * e + high) * 4 + low % 4] = (float)(R[e] * beta_low);
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// Workgroup (span, head, 16 columns), four waves: wave w holds the state's rows 64 c + 16 w ... + 15 as the results of
+// the 32-bit matrix instruction 16 x 16 x 4 (rows 4 (lane / 16) + e, column lane % 16), which are its right operands too:
+// which row a product covers is free.  The sums over the rows meet in LDS once a sixteen; x, u and the factors' products are
+// every wave's own, the outputs' are shared out.  Operands come from memory two sixteens ahead, in whole kilobytes; values
+// of tokens that are not there are out of a buffer's range: zeros.
+template <int NB>
+__global__ __launch_bounds__(kRecThreads, NB <= 3 ? 2 : 1) void gated_delta_sixteens_kernel(
+    const float* __restrict__ vv, const float* __restrict__ factors, float* __restrict__ o_out,
+    float* __restrict__ state, long slot_stride, const int* __restrict__ slots, const int* __restrict__ span_start,
+    const int* __restrict__ span_pos, int H, int G, int dk, int dv) {
+  constexpr int WAVES = kRecThreads / kWave, T = kSixteen, ROWS = 64 * NB;
+  __shared__ floatx4 met[2][WAVES][kWave];           // the waves' shares of S^T k
+  __shared__ float outs[2][WAVES][4][kWave];         // and of the outputs
+  __shared__ float slow[WAVES][T][T + 1];
+  const int span = blockIdx.x, h = blockIdx.y, lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int g = h / (H / G), low = lane % 16, high = lane / 16;
+  const int j = blockIdx.z * 16 + low;
+  const long t0 = span_start[span];
+  const int len = (int)(span_start[span + 1] - t0);
+  const bool fresh = span_pos[span] == 0;
+  float* S = state + (long)slots[span] * slot_stride + (long)h * dk * dv;
+  floatx4 s[NB];
+#pragma unroll
+  for (int c = 0; c < NB; ++c)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int r = 64 * c + 16 * wave + 4 * high + e;
+      s[c][e] = (j < dv && r < dk && !fresh) ? S[(long)r * dv + j] : 0.f;
+    }
+  const int HV = H * dv;
+  auto range = [&](const float* base) {              // the span's rows, dv numbers of the last one
+    return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, len > 0 ? (int)((((long)len - 1) * HV + dv) * 4) : 0, 0x00020000);
+  };
+  const auto v_rows = range(vv + t0 * HV + (long)h * dv), o_rows = range(o_out + t0 * HV + (long)h * dv);
+  constexpr unsigned kNowhere = 0x80000000u;         // out of every range (see the host's check)
+  const unsigned v_at = j < dv ? (unsigned)(4 * high * HV + j) * 4 : kNowhere;
+  const unsigned o_at = j < dv ? (unsigned)((4 * high + wave) * HV + j) * 4 : kNowhere;
+  const long stride = sixteen_floats(H, G, ROWS);
+  const float* of_span = factors + (t0 / T + span) * stride;
+  const float* of_keys = of_span + (long)g * 3 * T * ROWS;
+  const float* of_head = of_span + (long)G * 3 * T * ROWS + (long)h * kHeadFactors;
+  const int last = len > 0 ? (len - 1) / T : 0;
+  auto f32 = [](unsigned x) { return __builtin_bit_cast(float, x); };
+  struct Operands {
+    floatx4 k[NB], q[NB], kt[NB], v, m;
+    float b, all, upto, behind;                      // (decays: of token 4 high + lane % 4)
+  };
+  // The operands of the sixteen at t, a piece at a time, to be asked for between the products.  (Of a sixteen behind the
+  // last one: the last one's again, not used.)
+  constexpr int PIECES = 3 * NB + 8;
+  auto ask = [&](int piece, int t, Operands& P) {
+    const long at = min(t / T, last) * stride;
+    auto four = [](const float* p) { return *reinterpret_cast<const floatx4*>(p); };
+    const int quad = 4 * wave + high;
+    if (piece < NB) {
+      P.k[piece] = four(of_keys + at + ((quad + 16 * piece) * T + low) * 4);
+    } else if (piece < 2 * NB) {
+      P.q[piece - NB] = four(of_keys + at + T * ROWS + ((quad + 16 * (piece - NB)) * T + low) * 4);
+    } else if (piece == 2 * NB) {
+      const float2 d = *reinterpret_cast<const float2*>(of_head + at + 2 * T * T + 2 * (4 * high + lane % 4));
+      P.upto = d.x;
+      P.behind = d.y;
+    } else if (piece < 2 * NB + 5) {
+      const unsigned e = piece - 2 * NB - 1;
+      P.v[e] = f32(__builtin_amdgcn_raw_buffer_load_b32(v_rows, v_at + ((unsigned)t + e) * HV * 4, 0, 0));
+    } else if (piece == 2 * NB + 5) {
+      P.m = four(of_head + at + (high * T + low) * 4);
+    } else if (piece == 2 * NB + 6) {
+      P.b = of_head[at + T * T + (wave * 4 + high) * T + low];
+    } else if (piece < 3 * NB + 7) {
+      const int c = piece - 2 * NB - 7;
+      P.kt[c] = four(of_keys + at + 2 * T * ROWS + (high * ROWS + 64 * c + 16 * wave + low) * 4);
+    } else {
+      P.all = of_head[at + 2 * T * T + 2 * (T - 1)];
+    }
+  };
+  auto mfma = [](float a, float b, floatx4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); };
+  auto lds_barrier = [&]() {   // orders LDS traffic only: loads from memory stay in flight
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  auto write_out = [&](int t, int buf) {             // tokens t + 4 high + wave
+    float o = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) o += outs[buf][w][wave][lane];
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, o), o_rows, o_at + (unsigned)t * HV * 4, 0, 0);
+  };
+  // The sixteen at t; meanwhile the operands of the one at `then` are asked for.
+  auto sixteen = [&](const Operands& P, int t, int buf, Operands& next, int then) {
+    constexpr int FIRST = (NB + 1) / 2;
+    const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+    int piece = 0;
+    auto feed = [&]() {
+      if (piece < PIECES) ask(piece++, then, next);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    floatx4 a[NB], o[NB];                            // (a chain of sixteen products each: the sums' error, not their time)
+#pragma unroll
+    for (int c = 0; c < NB; ++c) {
+      a[c] = zero;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        a[c] = mfma(P.k[c][e], s[c][e], a[c]);
+        feed();
+      }
+    }
+#pragma unroll
+    for (int c = 1; c < NB; ++c) a[0] += a[c];
+    met[buf][wave][lane] = a[0];
+    __builtin_amdgcn_sched_barrier(0);
+    auto queries = [&](int c) {
+      o[c] = zero;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        o[c] = mfma(P.q[c][e], s[c][e], o[c]);
+        feed();
+      }
+    };
+#pragma unroll
+    for (int c = 0; c < FIRST; ++c) queries(c);      // while the sums are on their way
+    lds_barrier();
+    floatx4 x = met[buf][0][lane], others[WAVES - 1];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) others[w - 1] = met[buf][w][lane];
+    if (t > 0) write_out(t - T, buf ^ 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = FIRST; c < NB; ++c) queries(c);
+    floatx4 upto, behind;
+    upto[0] = dpp_moved<0x00>(P.upto), upto[1] = dpp_moved<0x55>(P.upto);      // (a four's lane 0, 1, 2, 3 to all of it)
+    upto[2] = dpp_moved<0xAA>(P.upto), upto[3] = dpp_moved<0xFF>(P.upto);
+    behind[0] = dpp_moved<0x00>(P.behind), behind[1] = dpp_moved<0x55>(P.behind);
+    behind[2] = dpp_moved<0xAA>(P.behind), behind[3] = dpp_moved<0xFF>(P.behind);
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) x += others[w - 1];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = fmaf(-upto[e], x[e], P.v[e]);
+    floatx4 u = zero;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      u = mfma(P.m[e], x[e], u);
+      feed();
+    }
+#pragma unroll
+    for (int c = 1; c < NB; ++c) o[0] += o[c];
+    floatx4 out = o[0] * upto;
+    const bool odd = !(fabsf(u[0]) < INFINITY && fabsf(u[1]) < INFINITY && fabsf(u[2]) < INFINITY && fabsf(u[3]) < INFINITY);
+    if (__builtin_expect(__any(odd), 0)) {
+      // A token that is not finite is to leave those before it alone: products with the zeros above the diagonals are
+      // left out, and tokens that are not there write nothing.
+      const float* f = of_head + t / T * stride;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) slow[wave][4 * high + e][low] = x[e];
+      __builtin_amdgcn_s_waitcnt(0xC07F);
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+      for (int e = 0; e < 4; ++e) {
+        const int i = 4 * high + e;
+        float v = 0.f;
+        for (int l = 0; l <= i; ++l) v = fmaf(f[(l / 4 * T + i) * 4 + l % 4], slow[wave][l][low], v);
+        if (t + i >= len) v = 0.f;
+        if (e == 0) u[0] = v; else if (e == 1) u[1] = v; else if (e == 2) u[2] = v; else u[3] = v;
+      }
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int e = 0; e < 4; ++e) slow[wave][4 * high + e][low] = u[e];
+      __builtin_amdgcn_s_waitcnt(0xC07F);
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+      for (int e = 0; e < 4; ++e) {
+        const int i = 4 * high + e;
+        float v = 0.f;
+        for (int l = wave; l <= i; l += 4) v = fmaf(f[T * T + (l % 4 * 4 + l / 4) * T + i], slow[wave][l][low], v);
+        if (e == 0) out[0] += v; else if (e == 1) out[1] += v; else if (e == 2) out[2] += v; else out[3] += v;
+      }
+      __builtin_amdgcn_wave_barrier();
+    } else {
+      out = mfma(P.b, wave == 0 ? u[0] : wave == 1 ? u[1] : wave == 2 ? u[2] : u[3], out);
+    }
+    u *= behind;
+#pragma unroll
+    for (int c = 0; c < NB; ++c) {
+      floatx4 more = zero;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        more = mfma(P.kt[c][e], u[e], more);
+        feed();
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[c][e] = fmaf(P.all, s[c][e], more[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) outs[buf][wave][e][lane] = out[e];
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) feed();
+  };
+  Operands P[3];                                     // (two sixteens ahead)
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) ask(i, 0, P[0]);
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) ask(i, T, P[1]);
+  int t = 0, buf = 0;
+  for (; t + 2 * T < len; t += 3 * T, buf ^= 1) {    // (three a turn: operands in three sets of registers)
+    sixteen(P[0], t, buf, P[2], t + 2 * T);
+    sixteen(P[1], t + T, buf ^ 1, P[0], t + 3 * T);
+    sixteen(P[2], t + 2 * T, buf, P[1], t + 4 * T);
+  }
+  if (t < len) sixteen(P[0], t, buf, P[2], t + 2 * T);
+  if (t + T < len) sixteen(P[1], t + T, buf ^ 1, P[0], t + 3 * T);
+  lds_barrier();
+  if (len > 0) write_out((len - 1) / T * T, (len - 1) / T & 1);
+#pragma unroll
+  for (int c = 0; c < NB; ++c)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int r = 64 * c + 16 * wave + 4 * high + e;
+      if (j < dv && r < dk) S[(long)r * dv + j] = s[c][e];
+    }
+}
+
 // ---------------------------------------------------------------------------- gated linear recurrence
 
 constexpr int kGateTile = 16;                 // tokens, and output channels, of a matrix instruction
@@ -704,18 +1108,67 @@ extern "C" int kllm_gated_delta_prep(const float* proj, int nsplit, long split_s
 
 extern "C" int kllm_gated_delta_max_dim(void) { return 16 * kDeltaParts; }
 
+extern "C" int kllm_gated_delta_factor_floats(int H, int G, int dk) {
+  if (H <= 0 || G <= 0 || dk <= 0 || dk > 16 * kDeltaParts) return -1;
+  const long floats = sixteen_floats(H, G, ceil_div(dk, 64) * 64);
+  return floats < 0x7fffffffL ? (int)floats : -1;
+}
+
+extern "C" int kllm_gated_delta_factors(const float* qn, const float* kn, const float* gb, const int* span_start,
+                                        float* factors, int n, int n_spans, int H, int G, int dk, hipStream_t stream) {
+  KLLM_REQUIRE(qn && kn && gb && span_start && factors, "gated_delta_factors: null pointer");
+  KLLM_REQUIRE(n > 0 && n_spans > 0 && H > 0 && G > 0 && G <= 65535 && H % G == 0 && dk > 0 && dk <= 16 * kDeltaParts,
+               "gated_delta_factors: bad sizes n=%d spans=%d H=%d G=%d dk=%d (keys of up to %d)", n, n_spans, H, G, dk,
+               16 * kDeltaParts);
+  KLLM_REQUIRE(((uintptr_t)factors & 15) == 0, "gated_delta_factors: the factors' place is not aligned to 16 bytes");
+  const int nb = ceil_div(dk, 64);
+  const bool v4 = dk % 4 == 0 && (((uintptr_t)qn | (uintptr_t)kn) & 15) == 0;
+#define KLLM_GDF(NB, V4)                                                                                              \
+  hipLaunchKernelGGL((gated_delta_factors_kernel<NB, V4>), dim3(ceil_div(n, kSixteen) + n_spans, G),                     \
+                     dim3(kRecThreads), 0, stream, qn, kn, gb, span_start, factors, n_spans, H, G, dk)
+#define KLLM_GDFN(NB)               \
+  do {                              \
+    if (v4) KLLM_GDF(NB, true);     \
+    else KLLM_GDF(NB, false);       \
+  } while (0)
+  if (nb <= 1) KLLM_GDFN(1);
+  else if (nb <= 2) KLLM_GDFN(2);
+  else if (nb <= 3) KLLM_GDFN(3);
+  else KLLM_GDFN(4);
+#undef KLLM_GDFN
+#undef KLLM_GDF
+  KLLM_CHECK_LAUNCH("gated_delta_factors");
+  return 0;
+}
+
 extern "C" int kllm_gated_delta_scan(const float* qn, const float* kn, const float* vv, const float* gb, float* o_out,
                                      float* state, long slot_stride, const int* slots, const int* span_start,
-                                     const int* span_pos, int n_spans, int H, int G, int dk, int dv, const float* dec,
-                                     hipStream_t stream) {
+                                     const int* span_pos, int n, int n_spans, int H, int G, int dk, int dv,
+                                     const float* dec, const float* factors, hipStream_t stream) {
   KLLM_REQUIRE(qn && kn && vv && gb && o_out && state && slots && span_start && span_pos,
                "gated_delta_scan: null pointer");
-  KLLM_REQUIRE(n_spans > 0 && H > 0 && H <= 65535 && G > 0 && H % G == 0 && dk > 0 && dk <= 16 * kDeltaParts && dv > 0,
+  KLLM_REQUIRE(n > 0 && n_spans > 0 && H > 0 && H <= 65535 && G > 0 && H % G == 0 && dk > 0 && dk <= 16 * kDeltaParts && dv > 0,
                "gated_delta_scan: bad sizes spans=%d H=%d G=%d dk=%d dv=%d (keys of up to %d)", n_spans, H, G, dk, dv,
                16 * kDeltaParts);
   const dim3 grid(n_spans, H, ceil_div(dv, kDeltaCols));
   KLLM_REQUIRE(grid.z <= 65535, "gated_delta_scan: values too wide for the grid");
   const int nb = ceil_div(dk, 64);
+  if (factors) {
+    KLLM_REQUIRE(!dec, "gated_delta_scan: factors of tokens with decays per key channel");
+    KLLM_REQUIRE(((long)n + 4 * kSixteen) * H * dv < 1L << 29, "gated_delta_scan: %d rows of %d values are beyond 2 GiB, not"
+                 " built with factors", n, H * dv);
+    KLLM_REQUIRE(((uintptr_t)factors & 15) == 0, "gated_delta_scan: the factors are not aligned to 16 bytes");
+#define KLLM_GDX(NB)                                                                                                   \
+  hipLaunchKernelGGL((gated_delta_sixteens_kernel<NB>), grid, dim3(kRecThreads), 0, stream, vv, factors, o_out, state, \
+                     slot_stride, slots, span_start, span_pos, H, G, dk, dv)
+    if (nb <= 1) KLLM_GDX(1);
+    else if (nb <= 2) KLLM_GDX(2);
+    else if (nb <= 3) KLLM_GDX(3);
+    else KLLM_GDX(4);
+#undef KLLM_GDX
+    KLLM_CHECK_LAUNCH("gated_delta_scan");
+    return 0;
+  }
 #define KLLM_GDS(NB)                                                                                                   \
   do {                                                                                                                 \
     if (dec)                                                                                                           \

@@ -154,7 +154,9 @@ def _declare(lib):
         "kllm_gated_delta_prep": [P, I, L, P, I, P, L, P, P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, F, I, P, I, L, I, P, I, L,
                                   I, I, P, P],
         "kllm_gated_delta_max_dim": [],
-        "kllm_gated_delta_scan": [P, P, P, P, P, P, L, P, P, P, I, I, I, I, I, P, P],
+        "kllm_gated_delta_factor_floats": [I, I, I],
+        "kllm_gated_delta_factors": [P, P, P, P, P, I, I, I, I, I, P],
+        "kllm_gated_delta_scan": [P, P, P, P, P, P, L, P, P, P, I, I, I, I, I, I, P, P, P],
         "kllm_linear_recurrence_prep": [P, I, L, P, P, P, I, P, L, P, P, P, P, P, P, P, P, P, P, P, I, I, I, P],
         "kllm_linear_recurrence_scan": [P, P, P, I, L, P, P, L, P, P, P, P, I, I, I, I, I, P],
         "kllm_scaled_sum": [P, P, I, L, F, P, I, L, F, L, P],
@@ -199,7 +201,8 @@ LAUNCHING = ("kllm_embed", "kllm_add_rmsnorm", "kllm_rope_tables", "kllm_rope_ap
              "kllm_group_norm_add", "kllm_qk_norm_append", "kllm_delta_prep", "kllm_delta_scan", "kllm_delta_out",
              "kllm_norm_residual", "kllm_rope_tables_freq", "kllm_qkv_norm_append", "kllm_gate_bias", "kllm_moe_route",
              "kllm_moe_plan", "kllm_moe_expert", "kllm_moe_expert_rows", "kllm_moe_combine",
-             "kllm_conv_state_update", "kllm_gated_delta_prep", "kllm_gated_delta_scan", "kllm_linear_recurrence_prep",
+             "kllm_conv_state_update", "kllm_gated_delta_prep", "kllm_gated_delta_factors", "kllm_gated_delta_scan",
+             "kllm_linear_recurrence_prep",
              "kllm_linear_recurrence_scan", "kllm_latent_kv_append", "kllm_latent_norm", "kllm_latent_query", "kllm_attn_latent",
              "kllm_latent_out", "kllm_scaled_sum", "kllm_normed_sum", "kllm_qkv_conv_append", "kllm_decayed_prep",
              "kllm_decayed_scan", "kllm_decayed_out", "kllm_decayed_step", "kllm_token_gate", "kllm_soft_cap")
@@ -1767,25 +1770,52 @@ def gated_delta_prep(proj, conv_w, taps, state, conv_offset, a_log, dt_bias, spa
             a_ptr, a_ns, a_st, a_row, g_ptr, g_ns, g_st, g_row, 1 if gate_sigmoid else 0, _ptr(decays, "gated_delta decays", F32, True), _stream())
 
 
+def gated_delta_factor_floats(n, n_spans, heads, kv_heads, dim) -> int:
+    """Numbers that ``gated_delta_factors`` needs for a step of n tokens."""
+    per = int(library().kllm_gated_delta_factor_floats(int(heads), int(kv_heads), int(dim)))
+    if per < 0:
+        raise KernelError(f"gated_delta_factors: {heads} heads, {kv_heads} key heads of {dim} are not built")
+    return ((n + 15) // 16 + int(n_spans)) * per
+
+
+def gated_delta_factors(qn, kn, gb, span_start, n_spans, factors, heads, kv_heads, dim):
+    """What ``gated_delta_scan`` needs of every sixteen tokens of a span besides the state and the values: keys
+    and queries in the order that it reads them, their products with the decays between them, and the inverse that
+    turns v - S^T k into u; ``factors`` float32 with ``gated_delta_factor_floats`` numbers."""
+    n = qn.shape[0]
+    if (tuple(qn.shape) != (n, kv_heads * dim) or tuple(kn.shape) != tuple(qn.shape) or tuple(gb.shape) != (n, 2, heads)
+            or factors.numel() < gated_delta_factor_floats(n, n_spans, heads, kv_heads, dim)
+            or span_start.numel() < n_spans + 1):
+        raise KernelError("gated_delta_factors: shapes do not fit")
+    F32, I32 = torch.float32, torch.int32
+    _launch("kllm_gated_delta_factors", "gated_delta_factors", _ptr(qn, "gated_delta qn", F32),
+            _ptr(kn, "gated_delta kn", F32), _ptr(gb, "gated_delta gb", F32),
+            _ptr(span_start, "gated_delta span_start", I32), _ptr(factors, "gated_delta factors", F32), n, int(n_spans),
+            int(heads), int(kv_heads), int(dim), _stream())
+
+
 def gated_delta_scan(qn, kn, vv, gb, o_out, state, offset, slots, span_start, span_pos, n_spans, heads, kv_heads, dim,
-                     vdim, decays=None):
+                     vdim, decays=None, factors=None):
     """S <- g S; u = beta (v - S^T k); S <- S + k u^T; o = S^T q, each request through its state
     ([heads, dim, vdim] float32 at ``offset`` floats into its slot; zero where a span's position is 0).
-    ``decays`` [n, heads * dim]: g has one number per head and key channel (a row of S each)."""
+    ``decays`` [n, heads * dim]: g has one number per head and key channel (a row of S each).
+    ``factors``: what ``gated_delta_factors`` made of these tokens; the kernel then takes sixteen at a time."""
     n = qn.shape[0]
     addr, per_slot = _field(state, offset, "gated_delta_scan")
     if (tuple(o_out.shape) != (n, heads * vdim) or tuple(vv.shape) != (n, heads * vdim)
             or tuple(qn.shape) != (n, kv_heads * dim) or tuple(kn.shape) != tuple(qn.shape)
             or tuple(gb.shape) != (n, 2, heads) or offset + heads * dim * vdim > per_slot
             or (decays is not None and tuple(decays.shape) != (n, heads * dim))
+            or (factors is not None and (decays is not None
+                                         or factors.numel() < gated_delta_factor_floats(n, n_spans, heads, kv_heads, dim)))
             or slots.numel() < n_spans or span_start.numel() < n_spans + 1 or span_pos.numel() < n_spans):
         raise KernelError("gated_delta_scan: shapes do not fit")
     F32, I32 = torch.float32, torch.int32
     _launch("kllm_gated_delta_scan", "gated_delta_scan", _ptr(qn, "gated_delta qn", F32), _ptr(kn, "gated_delta kn", F32),
             _ptr(vv, "gated_delta v", F32), _ptr(gb, "gated_delta gb", F32), _ptr(o_out, "gated_delta o", F32), addr,
             per_slot, _ptr(slots, "gated_delta slots", I32), _ptr(span_start, "gated_delta span_start", I32),
-            _ptr(span_pos, "gated_delta span_pos", I32), int(n_spans), int(heads), int(kv_heads), int(dim), int(vdim),
-            _ptr(decays, "gated_delta decays", F32, True), _stream())
+            _ptr(span_pos, "gated_delta span_pos", I32), n, int(n_spans), int(heads), int(kv_heads), int(dim), int(vdim),
+            _ptr(decays, "gated_delta decays", F32, True), _ptr(factors, "gated_delta factors", F32, True), _stream())
 
 
 def linear_recurrence_prep(proj, x_bias, conv_w, conv_b, taps, state, conv_offset, wr_t, wi_t, br, bi, rate,

@@ -192,3 +192,77 @@ def test_recurrence_chain_with_empty_spans(lens):
         state[int(slots[s])] = S
     close(out, want)
     close(dev_state, state)
+
+
+SIXTEENS = [[1], [16], [17, 1, 33], [48, 15, 0, 16], [100, 3], [1] * 70 + [64]]
+
+
+def delta_inputs(dk, dv, lens, fresh, seed):
+    g = torch.Generator().manual_seed(seed)
+    n, H, G = sum(lens), 4, 2
+    unit = lambda t: t / t.norm(dim=-1, keepdim=True)
+    k, q = (unit(torch.randn(n, G, dk, generator=g)) for _ in range(2))
+    v, beta = torch.randn(n, H, dv, generator=g), torch.rand(n, H, generator=g)
+    decay = torch.rand(n, H, generator=g) ** 0.25
+    decay[-1, 0] = 0.0                                                     # forgets everything
+    state = torch.randn(len(lens) + 1, 8 + H * dk * dv, generator=g)
+    return H, G, k, q, v, beta, decay, state, spans_of(lens, fresh)
+
+
+def run_delta(dk, dv, lens, H, G, k, q, v, beta, decay, state, spans, sixteens):
+    n, (_, _, span_start, span_pos, slots) = sum(lens), spans
+    f = lambda t: t.to(DEV).contiguous()
+    dev_state, out = f(state), torch.full((n, H * dv), float("nan"), device=DEV)
+    q, k, gb, factors = f(q).view(n, -1), f(k).view(n, -1), f(torch.stack([decay, beta], dim=1)), None
+    if sixteens:
+        floats = K().gated_delta_factor_floats(n, len(lens), H, G, dk)
+        factors = torch.full((floats,), float("nan"), device=DEV)
+        K().gated_delta_factors(q, k, gb, span_start, len(lens), factors, H, G, dk)
+    K().gated_delta_scan(q, k, f(v).view(n, -1), gb, out, dev_state, 8, slots, span_start, span_pos, len(lens), H, G, dk, dv,
+                         factors=factors)
+    return out.cpu().view(n, H, dv), dev_state.cpu()
+
+
+@pytest.mark.parametrize("dk,dv", [(8, 24), (64, 16), (65, 17), (128, 40), (136, 16), (200, 8), (256, 33)])
+@pytest.mark.parametrize("lens", SIXTEENS, ids=len)
+def test_delta_scan_by_sixteens(dk, dv, lens):
+    """Spans that end inside a sixteen, at its end and behind it, single tokens among them, more spans than a wave's lanes;
+    4e-5 of the largest number is what sums of 256 + 16 rounded products of a sum near one may be off by."""
+    fresh = [i % 2 for i in range(len(lens))]
+    H, G, k, q, v, beta, decay, state, spans = delta_inputs(dk, dv, lens, fresh, dk + dv)
+    out, after = run_delta(dk, dv, lens, H, G, k, q, v, beta, decay, state, spans, True)
+    start, slots = spans[0], spans[4]
+    want, want_state = torch.zeros(sum(lens), H, dv, dtype=F64), state.double()
+    for s in range(len(lens)):
+        slot = int(slots[s])
+        S = want_state[slot, 8:].view(H, dk, dv).clone() * (0.0 if fresh[s] else 1.0)
+        for t in range(start[s], start[s + 1]):
+            kk, qq = (x[t].double().repeat_interleave(H // G, 0) for x in (k, q))
+            S = S * decay[t].double()[:, None, None]
+            u = beta[t].double()[:, None] * (v[t].double() - (S * kk[:, :, None]).sum(1))
+            S = S + kk[:, :, None] * u[:, None, :]
+            want[t] = (S * qq[:, :, None]).sum(1)
+        want_state[slot, 8:] = S.reshape(-1)
+    close(out.to(DEV), want)
+    close(after.to(DEV), want_state)
+
+
+@pytest.mark.parametrize("what", ["v", "k", "q", "beta", "decay", "state"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_delta_scan_by_sixteens_of_numbers_that_are_not_finite(what, value):
+    """They reach what they reach when tokens are taken one by one: nothing before them, no other head of values, and behind a
+    span's end no state that was finite."""
+    dk, dv, lens = 72, 20, [37, 20]
+    H, G, k, q, v, beta, decay, state, spans = delta_inputs(dk, dv, lens, [0, 0], 5)
+    if what == "state":
+        state[int(spans[4][1]), 8 + dk * dv + 3] = value                   # (second span, head 1, row 0, column 3)
+    else:
+        x = {"v": v, "k": k, "q": q, "beta": beta, "decay": decay}[what]
+        x[21, 1] = value if x.ndim == 2 else x[21, 1]
+        if x.ndim == 3:
+            x[21, 1, 2] = value
+    one, one_state = run_delta(dk, dv, lens, H, G, k, q, v, beta, decay, state, spans, False)
+    out, after = run_delta(dk, dv, lens, H, G, k, q, v, beta, decay, state, spans, True)
+    assert torch.equal(out.isfinite(), one.isfinite()) and torch.equal(after.isfinite(), one_state.isfinite())
+    close(out.nan_to_num(0, 0, 0).to(DEV), one.nan_to_num(0, 0, 0).double())
+    close(after.nan_to_num(0, 0, 0).to(DEV), one_state.nan_to_num(0, 0, 0).double())
