@@ -362,7 +362,8 @@ int kllm_delta_out(const float* o, const float* gate, const float* weight, float
  * new rows instead: the norm in front of the next sub-layer.  `delta_scale` [n] (or null) is a
  * factor per row on delta's slices.  With `pair_b` ([pair_nb][n][d]) the sums are those of two
  * sub-layers side by side, each normed before they are added: pair_sa * pair_wa * N(delta) +
- * pair_sb * pair_wb * N(pair_b) stands where delta's slices stood.
+ * pair_sb * pair_wb * N(pair_b) stands where delta's slices stood; without pair_wa and pair_wb
+ * pair_sa * delta + pair_sb * pair_b does.
  * The sums may also be those of a routed feed-forward's chosen experts, not yet added up
  * (`chosen_y` [n * top][d], null: none): then the row is the sum over the token's choices of
  * chosen_wgt * (chosen_idx < E ? chosen_y : chosen_x, the feed-forward's input [n][d]) + delta's
@@ -481,11 +482,13 @@ int kllm_gated_delta_factors(const float* qn, const float* kn, const float* gb, 
                              int n, int n_spans, int H, int G, int dk, hipStream_t stream);
 /* The recurrence: state [H][dk][dv] per slot, o_out [n][H dv].  `dec` (or null): decays per head and
  * key channel [n][H dk], which then take the place of gb's decay.  `factors` (or null, and always
- * null with `dec`): what kllm_gated_delta_factors made of the same tokens; sixteen tokens are then taken at a time. */
+ * null with `dec`): what kllm_gated_delta_factors made of the same tokens; sixteen tokens are then taken at a time.  With `conv_state`
+ * (or null) the launch also does what kllm_conv_state_update does for the columns 0 .. conv_channels of conv_proj. */
 int kllm_gated_delta_scan(const float* qn, const float* kn, const float* vv, const float* gb, float* o_out,
                           float* state, long slot_stride, const int* slots, const int* span_start,
                           const int* span_pos, int n, int n_spans, int H, int G, int dk, int dv, const float* dec,
-                          const float* factors, hipStream_t stream);
+                          const float* factors, const float* conv_proj, int conv_nsplit, long conv_stride,
+                          int conv_cols, int conv_channels, float* conv_state, int taps, hipStream_t stream);
 /* Gated linear recurrence.  proj columns: y (W) | x (W).  wr_t, wi_t: the gates' block-diagonal matrices
  * [blocks][in][out]; rate [W] = 8 softplus(lambda).  Writes a and the added term, [n][W] each. */
 int kllm_linear_recurrence_prep(const float* proj, int nsplit, long split_stride, const float* x_bias,
@@ -495,11 +498,13 @@ int kllm_linear_recurrence_prep(const float* proj, int nsplit, long split_stride
                                 const int* span_start, const int* span_pos, float* a_out, float* b_out, int n, int W,
                                 int blocks, hipStream_t stream);
 /* S <- a S + b per span and channel (state [W] per slot); out [n][W] = S * gelu_tanh(y + y_bias).
- * longest: tokens of the longest span, or 0 if the caller does not know; only the split of the work goes by it. */
+ * longest: tokens of the longest span, or 0 if the caller does not know; only the split of the work goes by it.
+ * With `conv_state` (or null) the launch also does what kllm_conv_state_update does for the columns of x. */
 int kllm_linear_recurrence_scan(const float* a_in, const float* b_in, const float* proj, int nsplit,
                                 long split_stride, const float* y_bias, float* state, long slot_stride,
                                 const int* slots, const int* span_start, const int* span_pos, void* out, int n,
-                                int n_spans, int longest, int W, int dtype, hipStream_t stream);
+                                int n_spans, int longest, int W, int dtype, float* conv_state, const float* conv_bias,
+                                int taps, hipStream_t stream);
 
 /* out[i] = sa * sum over a's slices + sb * sum over b's slices (float32, `count` elements a slice). */
 int kllm_scaled_sum(float* out, const float* a, int na, long stride_a, float sa, const float* b, int nb,

@@ -2,9 +2,10 @@
 //
 // A short causal convolution per channel: y_t = sum_j w[c][j] x_(t - taps + 1 + j), zeros before
 // position 0.  Its inputs of the last taps - 1 positions are part of a request's state: the
-// kernels that convolve read them for the first tokens of a span, and `conv_state_update`, a
-// launch of its own behind them, writes the span's last inputs there (one thread per request
-// and channel reads the old entries before it writes the new ones).
+// kernels that convolve read them for the first tokens of a span, and a launch behind them (the scan, or
+// `conv_state_update`) writes the span's last inputs there (one thread per request and channel reads the
+// old entries before it writes the new ones).  In the scan's launch it costs 1.4 us (8 single tokens, 2,048 channels; 5 of a
+// chain of 1,500 tokens) where a launch of its own takes 4.7, and the gap in front of it.
 //
 // The gated delta rule, per head with a state S [key channel][value channel]:
 //
@@ -35,23 +36,20 @@ namespace kllm {
 constexpr int kRecThreads = 256;
 
 __global__ __launch_bounds__(kRecThreads) void conv_state_update_kernel(
-    const float* __restrict__ proj, int nsplit, long split_stride, long cols, int col0, int C,
-    const float* __restrict__ in_bias, float* __restrict__ state, long slot_stride, int taps,
-    const int* __restrict__ slots, const int* __restrict__ span_start, const int* __restrict__ span_pos) {
+    const ConvTail tail, long slot_stride, const int* __restrict__ slots, const int* __restrict__ span_start,
+    const int* __restrict__ span_pos) {
   const int c = blockIdx.x * kRecThreads + threadIdx.x;
-  if (c >= C) return;
+  if (c >= tail.C) return;
   const int span = blockIdx.y;
-  const int K = taps - 1;
-  const long t0 = span_start[span], t1 = span_start[span + 1];
-  const long len = t1 - t0;
-  const bool fresh = span_pos[span] == 0;
-  float* st = state + (long)slots[span] * slot_stride + (long)c * K;
-  float old[kMaxTaps];
-  for (int j = 0; j < K; ++j) old[j] = fresh ? 0.f : st[j];
-  for (int j = 0; j < K; ++j) {
-    const long row = t1 - K + j;
-    st[j] = row >= t0 ? conv_input(proj, nsplit, split_stride, cols, col0 + c, in_bias, row) : old[j + len];
-  }
+  conv_tail(tail, slot_stride, c, slots[span], span_start[span], span_start[span + 1], span_pos[span] == 0);
+}
+
+// The same in the launch of a scan whose workgroups (span, head, block of columns) share the channels out.
+__device__ __forceinline__ void conv_tail_of_span(const ConvTail& tail, long slot_stride, int slot, long t0, long t1,
+                                                  bool fresh) {
+  const int threads = gridDim.y * gridDim.z * kRecThreads;
+  for (int c = (blockIdx.y * gridDim.z + blockIdx.z) * kRecThreads + threadIdx.x; tail.taps > 1 && c < tail.C; c += threads)
+    conv_tail(tail, slot_stride, c, slot, t0, t1, fresh);
 }
 
 // ---------------------------------------------------------------------------- gated delta rule
@@ -161,7 +159,7 @@ __global__ __launch_bounds__(kRecThreads) void gated_delta_scan_kernel(
     const float* __restrict__ qn, const float* __restrict__ kn, const float* __restrict__ vv,
     const float* __restrict__ gb, float* __restrict__ o_out, float* __restrict__ state, long slot_stride,
     const int* __restrict__ slots, const int* __restrict__ span_start, const int* __restrict__ span_pos, int H, int G,
-    int dk, int dv, const float* __restrict__ dec) {
+    int dk, int dv, const float* __restrict__ dec, const ConvTail tail) {
   constexpr int ROW = 64 * NB;                       // a token's row in LDS
   constexpr int NV = VEC ? 3 : 2;                    // vectors of a token: k, q and the decays
   __shared__ __attribute__((aligned(16))) float rows[NV][kDeltaBlock][ROW];
@@ -183,6 +181,7 @@ __global__ __launch_bounds__(kRecThreads) void gated_delta_scan_kernel(
       const int r = 64 * b + 4 * p + e;
       s[b][e] = (col && r < dk && !fresh) ? S[(long)r * dv + j] : 0.f;
     }
+  conv_tail_of_span(tail, slot_stride, slots[span], t0, t1, fresh);
   const int QK = G * dk, HV = H * dv;
   // A thread's pieces of a block of tokens: of each vector the elements tid % 64 + 64 i of tokens
   // tid / 64 + 4 q, one of v, one of g and beta.  They are asked for one block ahead and wait in
@@ -347,8 +346,9 @@ __device__ __forceinline__ void transpose_four(floatx4& x, int lane) {
 }
 
 // Workgroup (sixteen, head of keys).  The sums go by the 64-bit matrix instruction (wave w takes the channels 16 w + 64 i),
-// then a wave makes a head's factors.  L to the power of 16 is zero, so that (1 + L)^-1 = (1 + L^8) (1 + L^4) (1 + L^2) (1 - L); an operand on the left is read from its transpose in the
-// layout of a result, so every power is made with its transpose.  Everything is 64-bit until it is written.
+// then a wave makes a head's factors.  L to the power of 16 is zero, so that (1 + L)^-1 = (1 + L^8) (1 + L^4) (1 + L^2)
+// (1 - L); an operand on the left is read from its transpose in the layout of a result, so every power is made with
+// its transpose.  Everything is 64-bit until it is written.
 template <int NB, bool V4>
 __global__ __launch_bounds__(kRecThreads, NB <= 2 && V4 ? 4 : 2) void gated_delta_factors_kernel(
     const float* __restrict__ qn, const float* __restrict__ kn, const float* __restrict__ gb,
@@ -489,7 +489,7 @@ template <int NB>
 __global__ __launch_bounds__(kRecThreads, NB <= 3 ? 2 : 1) void gated_delta_sixteens_kernel(
     const float* __restrict__ vv, const float* __restrict__ factors, float* __restrict__ o_out,
     float* __restrict__ state, long slot_stride, const int* __restrict__ slots, const int* __restrict__ span_start,
-    const int* __restrict__ span_pos, int H, int G, int dk, int dv) {
+    const int* __restrict__ span_pos, int H, int G, int dk, int dv, const ConvTail tail) {
   constexpr int WAVES = kRecThreads / kWave, T = kSixteen, ROWS = 64 * NB;
   __shared__ floatx4 met[2][WAVES][kWave];           // the waves' shares of S^T k
   __shared__ float outs[2][WAVES][4][kWave];         // and of the outputs
@@ -510,6 +510,7 @@ __global__ __launch_bounds__(kRecThreads, NB <= 3 ? 2 : 1) void gated_delta_sixt
       const int r = 64 * c + 16 * wave + 4 * high + e;
       s[c][e] = (j < dv && r < dk && !fresh) ? S[(long)r * dv + j] : 0.f;
     }
+  conv_tail_of_span(tail, slot_stride, slots[span], t0, t0 + len, fresh);
   const int HV = H * dv;
   auto range = [&](const float* base) {              // the span's rows, dv numbers of the last one
     return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, len > 0 ? (int)((((long)len - 1) * HV + dv) * 4) : 0, 0x00020000);
@@ -934,7 +935,7 @@ __global__ __launch_bounds__(CH * SEGS) void linear_recurrence_scan_kernel(
     const float* __restrict__ a_in, const float* __restrict__ b_in, const float* __restrict__ proj, int nsplit,
     long split_stride, const float* __restrict__ y_bias, float* __restrict__ state, long slot_stride,
     const int* __restrict__ slots, const int* __restrict__ span_start, const int* __restrict__ span_pos,
-    T* __restrict__ out, int W) {
+    T* __restrict__ out, int W, const ConvTail tail) {
   __shared__ float seg_a[SEGS][CH], seg_b[SEGS][CH];
   const int lane = threadIdx.x % CH, seg = threadIdx.x / CH;
   const int c = min((int)blockIdx.x * CH + lane, W - 1);
@@ -947,6 +948,7 @@ __global__ __launch_bounds__(CH * SEGS) void linear_recurrence_scan_kernel(
   const bool cut = SEGS > 1 && len > LEAST;
   const long a0 = min(t1, t0 + seg * per), a1 = min(t1, a0 + per);
   float* st = state + (long)slots[span] * slot_stride + c;
+  if (tail.taps > 1 && ok && seg == 0) conv_tail(tail, slot_stride, c, slots[span], t0, t1, span_pos[span] == 0);
   if (!cut && seg > 0) return;                            // (nobody meets)
   float S = span_pos[span] == 0 ? 0.f : *st;
   if (cut) {
@@ -1069,9 +1071,9 @@ extern "C" int kllm_conv_state_update(const float* proj, int nsplit, long split_
                "conv_state_update: bad sizes cols=%d col0=%d C=%d spans=%d", cols, col0, C, n_spans);
   KLLM_REQUIRE(taps >= 1 && taps <= kMaxTaps, "conv_state_update: %d taps (1 to %d)", taps, kMaxTaps);
   if (taps == 1) return 0;
-  hipLaunchKernelGGL(conv_state_update_kernel, dim3(ceil_div(C, kRecThreads), n_spans), dim3(kRecThreads), 0, stream,
-                     proj, nsplit, split_stride, (long)cols, col0, C, in_bias ? in_bias - col0 : nullptr, state,
-                     slot_stride, taps, slots, span_start, span_pos);
+  const ConvTail tail = {proj, split_stride, cols, in_bias, state, nsplit, col0, C, taps};
+  hipLaunchKernelGGL(conv_state_update_kernel, dim3(ceil_div(C, kRecThreads), n_spans), dim3(kRecThreads), 0, stream, tail,
+                     slot_stride, slots, span_start, span_pos);
   KLLM_CHECK_LAUNCH("conv_state_update");
   return 0;
 }
@@ -1144,12 +1146,20 @@ extern "C" int kllm_gated_delta_factors(const float* qn, const float* kn, const 
 extern "C" int kllm_gated_delta_scan(const float* qn, const float* kn, const float* vv, const float* gb, float* o_out,
                                      float* state, long slot_stride, const int* slots, const int* span_start,
                                      const int* span_pos, int n, int n_spans, int H, int G, int dk, int dv,
-                                     const float* dec, const float* factors, hipStream_t stream) {
+                                     const float* dec, const float* factors, const float* conv_proj, int conv_nsplit,
+                                     long conv_stride, int conv_cols, int conv_channels, float* conv_state, int taps,
+                                     hipStream_t stream) {
   KLLM_REQUIRE(qn && kn && vv && gb && o_out && state && slots && span_start && span_pos,
                "gated_delta_scan: null pointer");
   KLLM_REQUIRE(n > 0 && n_spans > 0 && H > 0 && H <= 65535 && G > 0 && H % G == 0 && dk > 0 && dk <= 16 * kDeltaParts && dv > 0,
                "gated_delta_scan: bad sizes spans=%d H=%d G=%d dk=%d dv=%d (keys of up to %d)", n_spans, H, G, dk, dv,
                16 * kDeltaParts);
+  KLLM_REQUIRE(!conv_state || (conv_proj && conv_nsplit >= 1 && conv_channels > 0 && conv_channels <= conv_cols &&
+                               taps >= 1 && taps <= kMaxTaps),
+               "gated_delta_scan: the convolution's inputs do not fit (%d channels of %d columns, %d taps)", conv_channels,
+               conv_cols, taps);
+  ConvTail tail = {conv_proj, conv_stride, conv_cols, nullptr, conv_state, conv_nsplit, 0, conv_channels, taps};
+  if (!conv_state) tail.taps = 0;
   const dim3 grid(n_spans, H, ceil_div(dv, kDeltaCols));
   KLLM_REQUIRE(grid.z <= 65535, "gated_delta_scan: values too wide for the grid");
   const int nb = ceil_div(dk, 64);
@@ -1160,7 +1170,7 @@ extern "C" int kllm_gated_delta_scan(const float* qn, const float* kn, const flo
     KLLM_REQUIRE(((uintptr_t)factors & 15) == 0, "gated_delta_scan: the factors are not aligned to 16 bytes");
 #define KLLM_GDX(NB)                                                                                                   \
   hipLaunchKernelGGL((gated_delta_sixteens_kernel<NB>), grid, dim3(kRecThreads), 0, stream, vv, factors, o_out, state, \
-                     slot_stride, slots, span_start, span_pos, H, G, dk, dv)
+                     slot_stride, slots, span_start, span_pos, H, G, dk, dv, tail)
     if (nb <= 1) KLLM_GDX(1);
     else if (nb <= 2) KLLM_GDX(2);
     else if (nb <= 3) KLLM_GDX(3);
@@ -1173,10 +1183,10 @@ extern "C" int kllm_gated_delta_scan(const float* qn, const float* kn, const flo
   do {                                                                                                                 \
     if (dec)                                                                                                           \
       hipLaunchKernelGGL((gated_delta_scan_kernel<NB, true>), grid, dim3(kRecThreads), 0, stream, qn, kn, vv, gb,      \
-                         o_out, state, slot_stride, slots, span_start, span_pos, H, G, dk, dv, dec);                   \
+                         o_out, state, slot_stride, slots, span_start, span_pos, H, G, dk, dv, dec, tail);             \
     else                                                                                                               \
       hipLaunchKernelGGL((gated_delta_scan_kernel<NB, false>), grid, dim3(kRecThreads), 0, stream, qn, kn, vv, gb,     \
-                         o_out, state, slot_stride, slots, span_start, span_pos, H, G, dk, dv, dec);                   \
+                         o_out, state, slot_stride, slots, span_start, span_pos, H, G, dk, dv, dec, tail);             \
   } while (0)
   if (nb <= 1) KLLM_GDS(1);
   else if (nb <= 2) KLLM_GDS(2);
@@ -1226,21 +1236,24 @@ extern "C" int kllm_linear_recurrence_prep(const float* proj, int nsplit, long s
 extern "C" int kllm_linear_recurrence_scan(const float* a_in, const float* b_in, const float* proj, int nsplit,
                                            long split_stride, const float* y_bias, float* state, long slot_stride,
                                            const int* slots, const int* span_start, const int* span_pos, void* out,
-                                           int n, int n_spans, int longest, int W, int dtype, hipStream_t stream) {
+                                           int n, int n_spans, int longest, int W, int dtype, float* conv_state,
+                                           const float* conv_bias, int taps, hipStream_t stream) {
   KLLM_REQUIRE(a_in && b_in && proj && y_bias && state && slots && span_start && span_pos && out,
                "linear_recurrence_scan: null pointer");
   KLLM_REQUIRE(n > 0 && n_spans > 0 && n_spans <= 65535 && W > 0 && nsplit >= 1,
                "linear_recurrence_scan: bad sizes n=%d spans=%d W=%d", n, n_spans, W);
   KLLM_REQUIRE(dtype == DT_F32 || dtype == DT_BF16, "linear_recurrence_scan: unknown dtype %d", dtype);
+  KLLM_REQUIRE(!conv_state || (taps >= 1 && taps <= kMaxTaps), "linear_recurrence_scan: %d taps (1 to %d)", taps, kMaxTaps);
+  const ConvTail tail = {proj, split_stride, 2L * W, conv_bias, conv_state, nsplit, W, W, conv_state ? taps : 0};      // (of x)
 #define KLLM_LRS(CH, SEGS)                                                                                               \
   do {                                                                                                                  \
     const dim3 grid(ceil_div(W, CH), n_spans), wg(CH * SEGS);                                                           \
     if (dtype == DT_F32)                                                                                                \
       hipLaunchKernelGGL((linear_recurrence_scan_kernel<float, CH, SEGS>), grid, wg, 0, stream, a_in, b_in, proj,       \
-                         nsplit, split_stride, y_bias, state, slot_stride, slots, span_start, span_pos, (float*)out, W); \
+                         nsplit, split_stride, y_bias, state, slot_stride, slots, span_start, span_pos, (float*)out, W, tail); \
     else                                                                                                                \
       hipLaunchKernelGGL((linear_recurrence_scan_kernel<bf16_t, CH, SEGS>), grid, wg, 0, stream, a_in, b_in, proj,      \
-                         nsplit, split_stride, y_bias, state, slot_stride, slots, span_start, span_pos, (bf16_t*)out, W); \
+                         nsplit, split_stride, y_bias, state, slot_stride, slots, span_start, span_pos, (bf16_t*)out, W, tail); \
   } while (0)
   // The longest span's chain bounds the time, and every span, however short, takes workgroups.  Up to 16 tokens there
   // is nothing to cut.  A long chain takes 64 segments of 16 channels where the tokens are those of few

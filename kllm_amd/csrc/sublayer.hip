@@ -37,10 +37,12 @@ struct ChosenSums {
 };
 
 // Two sub-layers side by side whose outputs are each normed before they are added: the row is
-// sa * wa * N(delta's slices) + sb * wb * N(b's slices) in place of delta's slices.
+// sa * wa * N(delta's slices) + sb * wb * N(b's slices) in place of delta's slices.  Without the weights they are
+// added as they are, sa * delta + sb * b (a launch of its own for that sum took 4 us a layer of a decode step and 16 at 1,500
+// tokens of 2,048 channels).
 struct NormedPair {
   const float* b;        // [nb][n][d], null: no such pair
-  const float* wa;       // [d]
+  const float* wa;       // [d], or null (and wb too)
   const float* wb;       // [d]
   long stride_b;
   int nb;
@@ -120,25 +122,30 @@ __global__ __launch_bounds__(kRowThreads) void norm_residual_kernel(
 #pragma unroll
           for (int j = 0; j < PER; ++j) {
             bv[j] = 0.f;
-            wa[j] = pair.wa[at[j]];
-            wb[j] = pair.wb[at[j]];
+            wa[j] = pair.wa ? pair.wa[at[j]] : 0.f;
+            wb[j] = pair.wa ? pair.wb[at[j]] : 0.f;
           }
           for (int s = 0; s < pair.nb; ++s) {
             const float* src = pair.b + s * pair.stride_b + r * d;
 #pragma unroll
             for (int j = 0; j < PER; ++j) bv[j] += src[at[j]];
           }
-          float ssa = 0.f, ssb = 0.f;
+          if (!pair.wa) {
 #pragma unroll
-          for (int j = 0; j < PER; ++j) {
-            if (threadIdx.x + kRowThreads * j >= d) dv[j] = bv[j] = 0.f;
-            ssa = fmaf(dv[j], dv[j], ssa);
-            ssb = fmaf(bv[j], bv[j], ssb);
+            for (int j = 0; j < PER; ++j) dv[j] = fmaf(pair.sa, dv[j], pair.sb * bv[j]);
+          } else {
+            float ssa = 0.f, ssb = 0.f;
+#pragma unroll
+            for (int j = 0; j < PER; ++j) {
+              if (threadIdx.x + kRowThreads * j >= d) dv[j] = bv[j] = 0.f;
+              ssa = fmaf(dv[j], dv[j], ssa);
+              ssb = fmaf(bv[j], bv[j], ssb);
+            }
+            const float ra = pair.sa / sqrtf(block_sum(ssa, red) / (float)d + eps);
+            const float rb = pair.sb / sqrtf(block_sum(ssb, red) / (float)d + eps);
+#pragma unroll
+            for (int j = 0; j < PER; ++j) dv[j] = fmaf(dv[j] * ra, wa[j], bv[j] * rb * wb[j]);
           }
-          const float ra = pair.sa / sqrtf(block_sum(ssa, red) / (float)d + eps);
-          const float rb = pair.sb / sqrtf(block_sum(ssb, red) / (float)d + eps);
-#pragma unroll
-          for (int j = 0; j < PER; ++j) dv[j] = fmaf(dv[j] * ra, wa[j], bv[j] * rb * wb[j]);
         }
 #pragma unroll
         for (int j = 0; j < PER; ++j) v[j] = fmaf(dscale, dv[j], v[j]);
@@ -194,8 +201,10 @@ __global__ __launch_bounds__(kRowThreads) void norm_residual_kernel(
       ssa = fmaf(a, a, ssa);
       ssb = fmaf(b, b, ssb);
     }
-    ra = pair.sa / sqrtf(block_sum(ssa, red) / (float)d + eps);
-    rb = pair.sb / sqrtf(block_sum(ssb, red) / (float)d + eps);
+    if (pair.wa) {
+      ra = pair.sa / sqrtf(block_sum(ssa, red) / (float)d + eps);
+      rb = pair.sb / sqrtf(block_sum(ssb, red) / (float)d + eps);
+    }
   }
   float ss = 0.f;
   for (int i = threadIdx.x; i < d; i += kRowThreads) {
@@ -203,7 +212,8 @@ __global__ __launch_bounds__(kRowThreads) void norm_residual_kernel(
     if (sums) {
       v = chosen.y ? chosen_at(i) : 0.f;
       if (pair.b) {
-        v = fmaf(dscale, fmaf(row_lds[i] * ra, pair.wa[i], row_lds[d + i] * rb * pair.wb[i]), v);
+        v = fmaf(dscale, pair.wa ? fmaf(row_lds[i] * ra, pair.wa[i], row_lds[d + i] * rb * pair.wb[i])
+                                 : fmaf(pair.sa, row_lds[i], pair.sb * row_lds[d + i]), v);
       } else if (delta) {
         float dsum = 0.f;
         for (int s = 0; s < nsplit; ++s) dsum += delta[s * split_stride + r * d + i];
@@ -391,8 +401,8 @@ extern "C" int kllm_norm_residual(float* x, const float* delta, int nsplit, long
                                   const float* pair_wa, const float* pair_wb, float pair_sa, float pair_sb,
                                   hipStream_t stream) {
   KLLM_REQUIRE(x && weight, "norm_residual: null pointer");
-  KLLM_REQUIRE(!pair_b || (delta && pair_wa && pair_wb && pair_nb >= 1 && !chosen_y),
-               "norm_residual: two normed sums come with both sums and both weights, and without chosen experts");
+  KLLM_REQUIRE(!pair_b || (delta && (pair_wa == nullptr) == (pair_wb == nullptr) && pair_nb >= 1 && !chosen_y),
+               "norm_residual: two sums side by side come with both sums and both weights or none, and without chosen experts");
   NormedPair pair;
   pair.b = pair_b; pair.wa = pair_wa; pair.wb = pair_wb; pair.stride_b = pair_stride; pair.nb = pair_nb;
   pair.sa = pair_sa; pair.sb = pair_sb;

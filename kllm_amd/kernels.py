@@ -156,9 +156,9 @@ def _declare(lib):
         "kllm_gated_delta_max_dim": [],
         "kllm_gated_delta_factor_floats": [I, I, I],
         "kllm_gated_delta_factors": [P, P, P, P, P, I, I, I, I, I, P],
-        "kllm_gated_delta_scan": [P, P, P, P, P, P, L, P, P, P, I, I, I, I, I, I, P, P, P],
+        "kllm_gated_delta_scan": [P, P, P, P, P, P, L, P, P, P, I, I, I, I, I, I, P, P, P, I, L, I, I, P, I, P],
         "kllm_linear_recurrence_prep": [P, I, L, P, P, P, I, P, L, P, P, P, P, P, P, P, P, P, P, P, I, I, I, P],
-        "kllm_linear_recurrence_scan": [P, P, P, I, L, P, P, L, P, P, P, P, I, I, I, I, I, P],
+        "kllm_linear_recurrence_scan": [P, P, P, I, L, P, P, L, P, P, P, P, I, I, I, I, I, P, P, I, P],
         "kllm_scaled_sum": [P, P, I, L, F, P, I, L, F, L, P],
         "kllm_normed_sum": [P, P, I, L, F, P, P, I, L, F, P, I, I, F, P],
         "kllm_qkv_conv_append": [P, I, L, I, I, P, I, P, L, I, P, P, I, I, F, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, I, P, P],
@@ -1458,7 +1458,8 @@ def delta_out(o, gate, weight, eps, out, heads, head_dim):
 class NormedPair:
     """What two sub-layers that ran side by side leave for the norm behind them: ``scale_a *
     weight_a * N(a) + scale_b * weight_b * N(b)``, each of the float32 sums ``a`` and ``b`` ([n, d] or
-    [slices, n, d]) normed over the row (with the eps of the norm that takes the pair)."""
+    [slices, n, d]) normed over the row (with the eps of the norm that takes the pair).  With both weights None:
+    ``scale_a * a + scale_b * b``."""
 
     def __init__(self, a, scale_a, weight_a, b, scale_b, weight_b):
         self.a, self.scale_a, self.weight_a, self.b, self.scale_b, self.weight_b = a, float(scale_a), weight_a, b, float(scale_b), weight_b
@@ -1493,7 +1494,8 @@ def norm_residual(x, weight, delta=None, bias=None, out=None, eps=0.0, mult=1.0,
     elif isinstance(delta, NormedPair):
         pair, delta = delta, delta.a
         pair_nb, pair_stride = _splits(pair.b, n, d, "norm_residual pair")
-        if pair.weight_a.numel() != d or pair.weight_b.numel() != d:
+        if (pair.weight_a is None) != (pair.weight_b is None) or (
+                pair.weight_a is not None and (pair.weight_a.numel() != d or pair.weight_b.numel() != d)):
             raise KernelError("norm_residual: the pair's weights do not fit")
     nsplit, stride = (1, 0) if delta is None else _splits(delta, n, d, "norm_residual")
     if weight.numel() != d or (bias is not None and bias.numel() != d) or (out is not None and tuple(out.shape) != (n, d)):
@@ -1513,8 +1515,8 @@ def norm_residual(x, weight, delta=None, bias=None, out=None, eps=0.0, mult=1.0,
             chosen.experts if chosen else 0, float(mult), _ptr(next_weight, "norm_residual next weight", F32, True),
             _ptr(delta_scale, "norm_residual delta scale", F32, True),
             _ptr(pair.b, "norm_residual pair b", F32) if pair else 0, pair_nb if pair else 0, pair_stride if pair else 0,
-            _ptr(pair.weight_a, "norm_residual pair weight", F32) if pair else 0,
-            _ptr(pair.weight_b, "norm_residual pair weight", F32) if pair else 0, pair.scale_a if pair else 0.0,
+            _ptr(pair.weight_a, "norm_residual pair weight", F32, True) if pair else 0,
+            _ptr(pair.weight_b, "norm_residual pair weight", F32, True) if pair else 0, pair.scale_a if pair else 0.0,
             pair.scale_b if pair else 0.0, _stream())
 
 
@@ -1795,11 +1797,12 @@ def gated_delta_factors(qn, kn, gb, span_start, n_spans, factors, heads, kv_head
 
 
 def gated_delta_scan(qn, kn, vv, gb, o_out, state, offset, slots, span_start, span_pos, n_spans, heads, kv_heads, dim,
-                     vdim, decays=None, factors=None):
+                     vdim, decays=None, factors=None, conv=None):
     """S <- g S; u = beta (v - S^T k); S <- S + k u^T; o = S^T q, each request through its state
     ([heads, dim, vdim] float32 at ``offset`` floats into its slot; zero where a span's position is 0).
     ``decays`` [n, heads * dim]: g has one number per head and key channel (a row of S each).
-    ``factors``: what ``gated_delta_factors`` made of these tokens; the kernel then takes sixteen at a time."""
+    ``factors``: what ``gated_delta_factors`` made of these tokens; the kernel then takes sixteen at a time.
+    ``conv`` (proj, channels, taps, offset): what ``conv_state_update`` does for the first ``channels`` columns, in this launch."""
     n = qn.shape[0]
     addr, per_slot = _field(state, offset, "gated_delta_scan")
     if (tuple(o_out.shape) != (n, heads * vdim) or tuple(vv.shape) != (n, heads * vdim)
@@ -1815,7 +1818,21 @@ def gated_delta_scan(qn, kn, vv, gb, o_out, state, offset, slots, span_start, sp
             _ptr(vv, "gated_delta v", F32), _ptr(gb, "gated_delta gb", F32), _ptr(o_out, "gated_delta o", F32), addr,
             per_slot, _ptr(slots, "gated_delta slots", I32), _ptr(span_start, "gated_delta span_start", I32),
             _ptr(span_pos, "gated_delta span_pos", I32), n, int(n_spans), int(heads), int(kv_heads), int(dim), int(vdim),
-            _ptr(decays, "gated_delta decays", F32, True), _ptr(factors, "gated_delta factors", F32, True), _stream())
+            _ptr(decays, "gated_delta decays", F32, True), _ptr(factors, "gated_delta factors", F32, True),
+            *_conv_args(conv, n, state), _stream())
+
+
+def _conv_args(conv, n, state):
+    """A scan's arguments for the convolution whose inputs it leaves in the state."""
+    if conv is None:
+        return 0, 1, 0, 0, 0, 0, 0
+    proj, channels, taps, offset = conv
+    cols = proj.shape[-1]
+    nsplit, stride = _splits(proj, n, cols, "conv")
+    addr, per_slot = _field(state, offset, "conv")
+    if offset + channels * (taps - 1) > per_slot or channels > cols:
+        raise KernelError("gated_delta_scan: the convolution's inputs do not fit")
+    return _ptr(proj, "conv proj", torch.float32), nsplit, stride, cols, int(channels), addr if taps > 1 else 0, int(taps)
 
 
 def linear_recurrence_prep(proj, x_bias, conv_w, conv_b, taps, state, conv_offset, wr_t, wi_t, br, bi, rate,
@@ -1842,14 +1859,19 @@ def linear_recurrence_prep(proj, x_bias, conv_w, conv_b, taps, state, conv_offse
             _ptr(a_out, "recurrence a", F32), _ptr(b_out, "recurrence b", F32), n, W, int(blocks), _stream())
 
 
-def linear_recurrence_scan(a_in, b_in, proj, y_bias, state, offset, slots, span_start, span_pos, n_spans, out, longest=0):
+def linear_recurrence_scan(a_in, b_in, proj, y_bias, state, offset, slots, span_start, span_pos, n_spans, out, longest=0,
+                           conv=None):
     """S <- a S + b along every span (state [W] float32 at ``offset`` floats into the slot); out
     [n, W] = S * gelu_tanh(y + y_bias), y the first W columns of the sums ``proj`` [nsplit, n, 2 W].
-    ``longest``: tokens of the longest span, if the caller knows it; the split of the work goes by it."""
+    ``longest``: tokens of the longest span, if the caller knows it; the split of the work goes by it.  ``conv`` (x_bias,
+    taps, offset): what ``conv_state_update`` does for the last W columns, in this launch."""
     n, W = a_in.shape
+    x_bias, taps, conv_offset = conv or (None, 1, 0)
+    conv_addr, _ = _field(state, conv_offset, "linear_recurrence_scan") if taps > 1 else (0, 0)
     nsplit, stride = _splits(proj, n, 2 * W, "linear_recurrence_scan")
     addr, per_slot = _field(state, offset, "linear_recurrence_scan")
     if (tuple(b_in.shape) != (n, W) or tuple(out.shape) != (n, W) or y_bias.numel() != W or offset + W > per_slot
+            or conv_offset + W * (taps - 1) > per_slot or (x_bias is not None and x_bias.numel() != W)
             or slots.numel() < n_spans or span_start.numel() < n_spans + 1 or span_pos.numel() < n_spans):
         raise KernelError("linear_recurrence_scan: shapes do not fit")
     F32, I32 = torch.float32, torch.int32
@@ -1857,7 +1879,8 @@ def linear_recurrence_scan(a_in, b_in, proj, y_bias, state, offset, slots, span_
             _ptr(b_in, "recurrence b", F32), _ptr(proj, "recurrence proj", F32), nsplit, stride,
             _ptr(y_bias, "recurrence y bias", F32), addr, per_slot, _ptr(slots, "recurrence slots", I32),
             _ptr(span_start, "recurrence span_start", I32), _ptr(span_pos, "recurrence span_pos", I32),
-            _ptr(out, "recurrence out"), n, int(n_spans), int(longest), W, dtype_code(out.dtype), _stream())
+            _ptr(out, "recurrence out"), n, int(n_spans), int(longest), W, dtype_code(out.dtype), conv_addr,
+            _ptr(x_bias, "recurrence x bias", F32, True), int(taps), _stream())
 
 
 def scaled_sum(out, a, scale_a, b, scale_b):

@@ -295,7 +295,9 @@ class SublayerNormBlock(Part):
         if pending is not None:
             raise ValueError("sublayer_norm: the layer in front of it left sums pending, which it has no norm for")
         xin = stream_copy(ctx, x)
-        delta = call_part(self.mixer, self.mixer.forward, ctx, xin, cache)
+        # two mixers side by side are added in the norm's launch
+        more = {"pair_ok": True} if getattr(self.mixer, "leaves_pair", False) else {}
+        delta = call_part(self.mixer, self.mixer.forward, ctx, xin, cache, **more)
         out = stream_copy(ctx, x, fill=False)
         K.norm_residual(x, self.norm_mixer.weight, delta, bias=getattr(self.mixer, "out_bias", None), out=out,
                         eps=self.norm_mixer.eps)

@@ -177,17 +177,16 @@ class GatedDeltaMixer(Part):
                            cache.slots, ctx.span_start, ctx.span_pos, qn, kn, vv, gb, gate, self.heads, self.kv_heads,
                            self.head_dim, self.value_dim, self.unit_eps, a_sums=a_sums, decays=decays,
                            low_sums=low_sums, gate_sigmoid=self.gate_sigmoid)
-        # (behind the launch that read the earlier inputs: the span's last ones take their place)
-        K.conv_state_update(proj, 0, self.channels, self.taps, cache.state, conv_at, cache.slots, ctx.span_start,
-                            ctx.span_pos, ctx.n_spans)
         o = ctx.buf("gdelta.o", (n, self.hv), f32)
         factors = None
         if not self.channel_decay and ctx.max_span_len >= SIXTEENS_FROM and (n + 64) * self.hv < 2 ** 29:
             floats = K.gated_delta_factor_floats(n, ctx.n_spans, self.heads, self.kv_heads, self.head_dim)
             factors = ctx.buf("gdelta.factors", (floats,), f32)
             K.gated_delta_factors(qn, kn, gb, ctx.span_start, ctx.n_spans, factors, self.heads, self.kv_heads, self.head_dim)
+        # (a launch behind the one that read the convolution's earlier inputs: the span's last ones take their place)
         K.gated_delta_scan(qn, kn, vv, gb, o, cache.state, 0, cache.slots, ctx.span_start, ctx.span_pos, ctx.n_spans,
-                           self.heads, self.kv_heads, self.head_dim, self.value_dim, decays=decays, factors=factors)
+                           self.heads, self.kv_heads, self.head_dim, self.value_dim, decays=decays, factors=factors,
+                           conv=(proj, self.channels, self.taps, conv_at))
         out = ctx.buf("gdelta.out", (n, self.hv), self.runtime.dtype)
         K.delta_out(o, gate, self.norm_weight, self.eps, out, self.heads, self.value_dim)
         return decode_linear(ctx, out, self.w_o, "gdelta.o_proj", self._tiled.get("o"))
@@ -259,11 +258,9 @@ class LinearRecurrenceMixer(Part):
         K.linear_recurrence_prep(proj, self.x_bias, self.conv, self.conv_bias, self.taps, cache.state, W, self.gate_r,
                                  self.gate_i, self.gate_r_bias, self.gate_i_bias, self.rate, ctx.span_of_token,
                                  cache.slots, ctx.span_start, ctx.span_pos, a, b, self.blocks)
-        K.conv_state_update(proj, W, W, self.taps, cache.state, W, cache.slots, ctx.span_start, ctx.span_pos,
-                            ctx.n_spans, in_bias=self.x_bias)
         out = ctx.buf("rec.out", (n, W), self.runtime.dtype)
         K.linear_recurrence_scan(a, b, proj, self.y_bias, cache.state, 0, cache.slots, ctx.span_start, ctx.span_pos,
-                                 ctx.n_spans, out, longest=ctx.max_span_len)
+                                 ctx.n_spans, out, longest=ctx.max_span_len, conv=(self.x_bias, self.taps, W))
         return decode_linear(ctx, out, self.w_o, "rec.o_proj", self._tiled.get("o"))
 
 
@@ -361,7 +358,13 @@ class MixerSum(Part):
     def leaves_sums(self):
         return self.folded
 
-    def forward(self, ctx, xn, cache, pair_eps=None, sums_ok=False):
+    # Without norms: the two outputs, not yet added, to a norm behind the mixer that adds them in its own
+    # launch (``pair_ok``: the caller takes a ``kernels.NormedPair`` without weights).
+    @property
+    def leaves_pair(self):
+        return self.norm_eps is None
+
+    def forward(self, ctx, xn, cache, pair_eps=None, sums_ok=False, pair_ok=False):
         views = list(cache) if isinstance(cache, (list, tuple)) else [cache]
 
         def take(m):       # a half with several needs gets them as a tuple, as a mixer alone does
@@ -382,6 +385,9 @@ class MixerSum(Part):
             return ScaledSum([left, right])
         if self.norm_eps is not None and pair_eps == self.norm_eps:
             return K.NormedPair(left, self.left_scale, self.left_norm, right, self.right_scale, self.right_norm)
+        if pair_ok and self.norm_eps is None:
+            scales = (1.0, 1.0) if self.folded else (self.left_scale, self.right_scale)
+            return K.NormedPair(left, scales[0], None, right, scales[1], None)
         out = ctx.buf("mixer_sum.out", (xn.shape[0], left.shape[-1]), torch.float32)
         if self.norm_eps is not None:
             K.normed_sum(out, left, self.left_scale, self.left_norm, right, self.right_scale, self.right_norm, self.norm_eps)

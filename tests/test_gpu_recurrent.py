@@ -266,3 +266,58 @@ def test_delta_scan_by_sixteens_of_numbers_that_are_not_finite(what, value):
     assert torch.equal(out.isfinite(), one.isfinite()) and torch.equal(after.isfinite(), one_state.isfinite())
     close(out.nan_to_num(0, 0, 0).to(DEV), one.nan_to_num(0, 0, 0).double())
     close(after.nan_to_num(0, 0, 0).to(DEV), one_state.nan_to_num(0, 0, 0).double())
+
+
+@pytest.mark.parametrize("taps", [1, 2, 4, 5])
+@pytest.mark.parametrize("sixteens", [False, True])
+def test_scans_leave_the_convolutions_inputs(taps, sixteens):
+    """In a scan's launch as in the launch of their own: spans of 0 to more tokens than the state holds, from position 0 and
+    behind earlier tokens; whole numbers are copied, so the states are the same."""
+    dk, dv, lens, fresh = 24, 20, [1, 2, 0, 3, 4, 0, 9, 1], [0, 1, 0, 0, 1, 1, 0, 1]
+    H, G, k, q, v, beta, decay, state, spans = delta_inputs(dk, dv, lens, fresh, 3)
+    n, C, (_, _, span_start, span_pos, slots) = sum(lens), 2 * G * dk + H * dv, spans
+    at = 8 + H * dk * dv
+    state = torch.cat([state, torch.randn(len(lens) + 1, C * (taps - 1))], dim=1)
+    proj = torch.randn(2, n, C + 7, device=DEV)
+    f = lambda t: t.to(DEV).contiguous()
+    want, got, out = f(state), f(state), torch.empty(n, H * dv, device=DEV)
+    gb, factors = f(torch.stack([decay, beta], dim=1)), None
+    if sixteens:
+        factors = torch.empty(K().gated_delta_factor_floats(n, len(lens), H, G, dk), device=DEV)
+        K().gated_delta_factors(f(q).view(n, -1), f(k).view(n, -1), gb, span_start, len(lens), factors, H, G, dk)
+    K().conv_state_update(proj, 0, C, taps, want, at, slots, span_start, span_pos, len(lens))
+    K().gated_delta_scan(f(q).view(n, -1), f(k).view(n, -1), f(v).view(n, -1), gb, out, got, 8, slots, span_start, span_pos,
+                         len(lens), H, G, dk, dv, factors=factors, conv=(proj, C, taps, at))
+    assert torch.equal(got[:, at:], want[:, at:])
+
+
+@pytest.mark.parametrize("taps", [1, 2, 4, 5])
+@pytest.mark.parametrize("longest", [9, 40, 200])                      # (one segment a span, sixteen and more)
+def test_linear_scan_leaves_the_convolutions_inputs(taps, longest):
+    W, lens, fresh = 40, [1, 2, 0, 3, 4, longest, 0, 1], [0, 1, 0, 0, 1, 0, 1, 1]
+    n = sum(lens)
+    _, _, span_start, span_pos, slots = spans_of(lens, fresh)
+    state = torch.randn(len(lens) + 1, W * taps + 3, device=DEV)
+    proj, bias, y_bias = torch.randn(2, n, 2 * W, device=DEV), torch.randn(W, device=DEV), torch.randn(W, device=DEV)
+    a, b, out = torch.rand(n, W, device=DEV), torch.randn(n, W, device=DEV), torch.empty(n, W, device=DEV)
+    want, got = state.clone(), state.clone()
+    K().conv_state_update(proj, W, W, taps, want, W + 3, slots, span_start, span_pos, len(lens), in_bias=bias)
+    K().linear_recurrence_scan(a, b, proj, y_bias, got, 3, slots, span_start, span_pos, len(lens), out, longest=longest,
+                               conv=(bias, taps, W + 3))
+    assert torch.equal(got[:, W + 3:], want[:, W + 3:])
+
+
+@pytest.mark.parametrize("d", [200, 1024, 2048, 4096, 5000])
+@pytest.mark.parametrize("slices", [(1, 1), (2, 3)])
+def test_norm_of_two_sums_without_weights(d, slices):
+    """The sum in the norm's launch is the sum of a launch in front of it, rounding for rounding."""
+    g = torch.Generator(device=DEV).manual_seed(d)
+    r = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    n, x, w = 5, r(5, d), r(d)
+    a, b, both = r(slices[0], n, d), r(slices[1], n, d), torch.empty(n, d, device=DEV)
+    K().scaled_sum(both, a, 0.75, b, -1.5)
+    want, got = x.clone(), x.clone()
+    out, out_want = torch.empty(n, d, device=DEV, dtype=torch.bfloat16), torch.empty(n, d, device=DEV, dtype=torch.bfloat16)
+    K().norm_residual(want, w, both, out=out_want, eps=1e-5)
+    K().norm_residual(got, w, K().NormedPair(a, 0.75, None, b, -1.5, None), out=out, eps=1e-5)
+    assert torch.equal(got, want) and torch.equal(out, out_want)
