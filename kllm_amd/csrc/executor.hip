@@ -28,6 +28,7 @@ static const Op kOps[] = {
     KLLM_CMD_OP(kllm_gemv_resid),
     KLLM_CMD_OP(kllm_gemv_rope_append),
     KLLM_CMD_OP(kllm_fused_linear),
+    KLLM_CMD_OP(kllm_linear_rows),
     KLLM_CMD_OP(kllm_attn_generic),
     KLLM_CMD_OP(kllm_attn_decode),
     KLLM_CMD_OP(kllm_attn_prefill),

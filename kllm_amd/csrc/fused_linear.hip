@@ -41,6 +41,7 @@
 #include <math.h>
 
 #include "common.hpp"
+#include "fused_linear.hpp"
 #include "kllm_kernels.h"
 
 namespace kllm {
@@ -79,34 +80,8 @@ __device__ __forceinline__ floatx4 fl_sum(floatx4 (&acc)[16]) {
     for (int e = 0; e < d; ++e) acc[e] += acc[e + d];
   return acc[0];
 }
-constexpr int FL_SS_LOADS = 4;     // 16-byte loads per lane of a row's partial sums of squares: 16 lanes a row
-constexpr int FL_SS_MAX = 16 * 4 * FL_SS_LOADS;   // partial sums of squares per row at most
 constexpr int FL_LDS_MAX = 160 * 1024;
 constexpr int FL_TILE = 16 * 17;    // floats of one wave's partial tile in LDS: [x row][w row], padded
-
-enum : int { FL_PARTS = 0, FL_RESID = 1, FL_SWIGLU = 2, FL_ROPE = 3 };
-// FL_PARTS with act >= FL_UNARY: y is [n][m] in the storage type = unary_act(sums, act - FL_UNARY), the
-// activation's learned constants (if it has any) behind norm_w.
-constexpr int FL_UNARY = 16;
-
-struct FlOut {
-  void* y;
-  const float* cos_t;
-  const float* sin_t;
-  void* cache;
-  const int* positions;
-  const int* span_of_token;
-  const int* block_table;
-  int max_pages, page_size, H, KV, hd;
-  int act;                      // the gate's activation (FL_SWIGLU)
-  float* resid;                 // FL_RESID: the residual stream [n][m]; y receives resid * norm_w in the storage type
-  const float* norm_w;          // FL_RESID: weight [m] of the norm behind the addition
-  float* ss_out;                // FL_RESID: [n][workgroups rounded up to 4] sums of squares of the new rows
-  const float* ss_in;           // SCALED: [n][ss_parts rounded up to 4], what a FL_RESID product left
-  int ss_parts;
-  float eps;
-  int tiled;                    // W is the copy that fl_tile_kernel made for this epilogue (see there)
-};
 
 // Row of W behind MFMA row c of a tile, or -1.  Pair epilogues: unit = pair.
 template <int EP>
@@ -128,15 +103,6 @@ __device__ __forceinline__ long fl_row(int tile, int c, int m, const FlOut& o) {
   }
   const long e = 2 * (long)(pair - rot_pairs);
   return (long)(o.H + o.KV) * o.hd + e + (second ? 1 : 0);
-}
-
-// A workgroup barrier for data in LDS.  Unlike __syncthreads it does not wait for loads from
-// memory: the weights asked for ahead stay in flight while the waves meet.
-__device__ __forceinline__ void fl_lds_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0xC07F);        // lgkmcnt(0): this wave's LDS operations are done
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
 }
 
 // NW waves share a tile's K; SCALED: the sums are multiplied by a row scale made from out.ss_in;
@@ -483,29 +449,7 @@ __global__ __launch_bounds__(64 * NW) void fused_linear_kernel(const T* __restri
           T* h = reinterpret_cast<T*>(out.y);
           h[(long)xr * pairs + pair] = from_f32<T>(gate_act(a, out.act) * b);
         } else {
-          const int half = out.hd / 2;
-          const int q_pairs = out.H * half, k_pairs = out.cache ? out.KV * half : 0;
-          const int region = pair < q_pairs ? 0 : pair < q_pairs + k_pairs ? 1 : 2;
-          const int page = ep_page[t], slot = ep_slot[t];
-          const long block = (long)out.page_size * out.hd;
-          if (region < 2) {
-            const int p = region ? pair - q_pairs : pair;
-            const int head = p / half, j = p % half;
-            const float cc = ep_cos[t], sn = ep_sin[t];
-            const float ra = a * cc - b * sn, rb = b * cc + a * sn;
-            T* o = region == 0
-                            ? reinterpret_cast<T*>(out.y) + ((long)xr * out.H + head) * out.hd
-                            : reinterpret_cast<T*>(out.cache) +
-                                  (((long)page * 2 + 0) * out.KV + head) * block + (long)slot * out.hd;
-            o[j] = from_f32<T>(ra);
-            o[j + half] = from_f32<T>(rb);
-          } else {
-            const int e = 2 * (pair - q_pairs - k_pairs);
-            const int head = e / out.hd, j = e % out.hd;
-            T* v = reinterpret_cast<T*>(out.cache) + (((long)page * 2 + 1) * out.KV + head) * block;
-            v[(long)j * out.page_size + slot] = from_f32<T>(a);
-            v[(long)(j + 1) * out.page_size + slot] = from_f32<T>(b);
-          }
+          fl_rope_store<T>(out, xr, pair, a, b, ep_cos[t], ep_sin[t], ep_page[t], ep_slot[t]);
         }
       }
     }

@@ -190,8 +190,16 @@ typedef struct {
   float eps;
   int tiled;            /* w is the copy that kllm_fused_linear_tile made of the weights for this kind */
   int f32;              /* x, w, y (but PARTS) and the cache are float32, not bfloat16; up to 16 rows */
+  int x_tiled;          /* kllm_linear_rows: x is what a product with y_tiled left */
+  int y_tiled;          /* kllm_linear_rows, RESID and SWIGLU: y goes out in the order the next such product's lanes read */
 } KllmLinearOut;
 long kllm_fused_linear_lds_bytes(int n, int k, int nsplit, int dtype);
+/* The RESID, SWIGLU and ROPE products of 17 to 64 rows (any n up to 64 is taken), bfloat16, K a multiple of 32,
+ * w the tiled copy.  RESID leaves kllm_linear_rows_parts(m) sums of squares a row (0: m is not taken).  Tiled rows
+ * (y_tiled, x_tiled; columns a multiple of 32): [row / 16][column / 32][column % 32 / 8][row % 16][8]; with more than 16 rows
+ * those up to the next multiple of 16 are there and hold anything, with fewer only the rows are. */
+int kllm_linear_rows(const void* x, int x_stride, const KllmLinearOut* y, const void* w, int n, int m, int k, hipStream_t stream);
+int kllm_linear_rows_parts(int m);
 /* Where that is more than LDS holds, the rows are staged and multiplied in passes over K, with
  * one tile to a workgroup (tiles_per_wg = 1): how many passes a call needs (1: all at once; 0:
  * the kernel does not take the sizes). */

@@ -1,0 +1,397 @@
+// Products of up to 64 rows of X (decode batches, short prompts) on MFMA in bfloat16, with the step after
+// the product in the same launch: the outputs of fused_linear.hpp, the weights in the lanes' order.
+//
+// What bounds such a product is the weights' way from memory and the rows' way from L2 into the CUs.  With tiles
+// whose operands both pass through LDS (gemm_ring.hip) 64 rows are one row of tiles, K has to go in
+// slices to fill the chip, and a second kernel adds the slices: norm, rotation and gate are launches of
+// their own, about 4.7 us each at these sizes.  fused_linear.hip stages all rows in LDS first, and more than 32 rows of
+// 2,048 do not fit.  Here nothing is staged: the waves of a workgroup share K, so no two of them want
+// the same element of X, and each loads its fragments of the rows (from L2) and of the weights (from memory)
+// straight into registers, four to eight steps of K in flight.  The waves meet once, when their sums
+// are complete, and the epilogue runs on the whole sums.  (Sixteen waves, or twelve steps in flight: up to 30 % slower.)
+//
+// A workgroup owns TW tiles of 16 rows of W and NT tiles of 16 rows of X.  Every workgroup reads its rows
+// of X whole, so TW is what divides the traffic from L2.  Two workgroups may share a tile of W and take half of the rows each;
+// they sit on one XCD, so that the weights come from memory once.
+//
+// Alone in a replayed graph, 8 / 64 rows, us: 2,048 x 2,048 4.6 / 7.2 (rows as attention leaves them); 2,048 x 5,632 9.9 / 12.2; 2 x
+// 5,632 x 2,048 11.0 / 14.5; 2,560 x 2,048 4.6 / 6.8; 4,096 x 14,336 23.4 / 41.0 (117 MB: 5.0 TB/s at 8 rows).  A decode step at
+// 1.1B sizes and contexts of 600, with fused_linear.hip's products and the tiles' and with these: 1 token 914 -> 888 us, 8 971
+// -> 937, 16 1,080 -> 1,031, 32 1,377 -> 1,155, 64 1,663 -> 1,370.
+#include <math.h>
+
+#include "common.hpp"
+#include "fused_linear.hpp"
+#include "kllm_kernels.h"
+
+namespace kllm {
+
+typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
+
+constexpr int LR_ROWS = 64;             // rows of X at most
+constexpr int LR_LD = 20;               // floats from one x row of a partial tile to the next: 16 and padding, whole 16 bytes
+constexpr int LR_TILE = 16 * LR_LD;
+
+// Element (row, column) of n rows of `cols` columns that go out in the lanes' order (out.y_tiled): [16 rows][32 columns][8
+// columns][row], so that a load of the next product's is one contiguous kilobyte, or less where there are fewer rows than 16.  From rows as
+// they are, its sixteen lanes with one K lie in sixteen rows, and a CU takes in 16 bytes a clock (64 rows of 5,632
+// against 2,048 columns: 15.8 -> 12.1 us; 16 rows 11.2 -> 10.1).
+__device__ __forceinline__ long lr_at(const FlOut& out, int row, int col, int n, int cols) {
+  if (!out.y_tiled) return (long)row * cols + col;
+  const int side = min(n, 16);
+  return (((long)(row / 16) * (cols / 32) + col / 32) * 4 + col % 32 / 8) * (8 * side) + row % 16 * 8 + col % 8;
+}
+
+// Steps of K in each of the two buffers a wave fills in turn: what 128 registers hold, four at most.
+constexpr int lr_ahead(int nt, int tw) { return nt + tw <= 4 ? 4 : nt + tw == 5 ? 3 : 2; }
+
+template <int NT, int TW, int EP, bool SCALED, int NW>
+__global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __restrict__ X, FlOut out,
+                                                              const bf16_t* __restrict__ W, int n, int m, int k, int tiles,
+                                                              int halves, int x_stride) {
+  constexpr int A = lr_ahead(NT, TW);
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+  float* part = reinterpret_cast<float*>(lds_raw);               // [NW][TW][NT][x row 16][LR_LD]
+  float* row_scale = part + NW * TW * NT * LR_TILE;              // [16 NT]
+  const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int g = lane / 16, c = lane % 16;
+  const int groups = (tiles + TW - 1) / TW;                      // workgroups side by side over W
+  // Blocks go to the XCDs in turn: two workgroups of one group of tiles are eight blocks apart.
+  const int group = halves == 1 ? (int)blockIdx.x : (int)(blockIdx.x / 16) * 8 + (int)(blockIdx.x % 8);
+  const int row0 = halves == 1 ? 0 : (int)(blockIdx.x / 8 % 2) * (16 * NT);
+  if (group >= groups || row0 >= n) return;                      // the whole workgroup
+  const int steps = k / 32;                                      // (k is a multiple of 32)
+  const int per = (steps + NW - 1) / NW;
+  const int s_beg = min(wave * per, steps);
+  const int mine = min(per, steps - s_beg);                      // steps of this wave, possibly none
+
+  // ---- what the epilogue needs is asked for first (loads return in order): the rotation's page and
+  // slot, the residual stream's old values
+  const int half = EP == FL_ROPE ? out.hd / 2 : 1;
+  constexpr int RR = 4 * NW;                               // rows that the threads take at a time, sixteen to a row
+  constexpr int RU = (16 * NT + RR - 1) / RR;                    // turns
+  constexpr int PU = EP == FL_ROPE ? (16 * NT + 2 * RR - 1) / (2 * RR) : 1;
+  int ep_pos[PU], ep_span[PU], ep_page[PU];
+  float ep_cos[PU], ep_sin[PU], res_old[RU], res_w = 0.f;
+  if (EP == FL_ROPE) {         // thread (pair tid % 8, row tid / 8, and 2 RR on)
+    const int pair = group * 8 + tid % 8;
+    const bool turns = out.cos_t && pair < (out.H + (out.cache ? out.KV : 0)) * half;
+#pragma unroll
+    for (int u = 0; u < PU; ++u) {
+      const int xr = min(row0 + tid / 8 + 2 * RR * u, n - 1);
+      ep_pos[u] = out.cache ? out.positions[xr] : 0;
+      ep_span[u] = out.cache ? out.span_of_token[xr] : 0;
+      ep_cos[u] = turns ? out.cos_t[(long)xr * half + pair % half] : 1.f;
+      ep_sin[u] = turns ? out.sin_t[(long)xr * half + pair % half] : 0.f;
+    }
+  }
+  if (EP == FL_RESID) {        // thread (w row tid % 16, x row tid / 16 and RR on)
+    const int col = min(group * 16 + tid % 16, m - 1);
+    res_w = out.norm_w[col];
+#pragma unroll
+    for (int u = 0; u < RU; ++u) res_old[u] = out.resid[(long)min(row0 + tid / 16 + RR * u, n - 1) * m + col];
+  }
+  constexpr int SU = RU;
+  floatx4 ssv[SCALED ? SU : 1][FL_SS_LOADS];
+  if (SCALED) {
+    const int stride = (out.ss_parts + 3) / 4 * 4;
+#pragma unroll
+    for (int u = 0; u < SU; ++u)
+#pragma unroll
+      for (int i = 0; i < FL_SS_LOADS; ++i) {
+        const int at = 4 * (tid % 16 + 16 * i);
+        ssv[u][i] = *reinterpret_cast<const floatx4*>(out.ss_in + (long)min(row0 + tid / 16 + RR * u, n - 1) * stride +
+                                                      (at < stride ? at : 0));
+      }
+  }
+
+  // ---- operands: offsets in bytes from descriptors that all lanes share, so that a step costs a scalar
+  // addition.  A step that does not exist reads the wave's last (or K's last) again and is not multiplied; a
+  // tile or a row of X beyond the last one reads the last, and its sums are not stored.
+  const int tile0 = group * TW;
+  const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<char*>(reinterpret_cast<const char*>(W)) + (long)tile0 * steps * 1024, 0,
+      min(TW, tiles - tile0) * steps * 1024, 0x00020000);
+  const int row_tiles = (n + 15) / 16, side = min(n, 16), x_step = out.x_tiled ? 64 * side : 64;
+  const __amdgpu_buffer_rsrc_t xr_ = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<bf16_t*>(X), 0, out.x_tiled ? row_tiles * steps * x_step : 2 * ((n - 1) * x_stride + k), 0x00020000);
+  int wo[TW], xo[NT];
+#pragma unroll
+  for (int j = 0; j < TW; ++j) wo[j] = min(j, tiles - tile0 - 1) * steps * 1024;
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+    xo[t] = out.x_tiled ? min(row0 / 16 + t, row_tiles - 1) * steps * x_step + (g * side + min(c, side - 1)) * 16
+                        : 2 * (min(row0 + t * 16 + c, n - 1) * x_stride + 8 * g);
+  const int s_last = min(s_beg + max(mine, 1), steps) - 1;
+  auto fill = [&](uintx4 (&wb)[A][TW], uintx4 (&xb)[A][NT], int s0) {
+#pragma unroll
+    for (int i = 0; i < A; ++i) {
+      const int s = min(s_beg + s0 + i, s_last);
+#pragma unroll
+      for (int j = 0; j < TW; ++j)
+        wb[i][j] = __builtin_amdgcn_raw_buffer_load_b128(wr, lane * 16, wo[j] + s * 1024, 0);
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        xb[i][t] = __builtin_amdgcn_raw_buffer_load_b128(xr_, xo[t], s * x_step, 0);
+    }
+    // Loads and products stay on their sides of this line: left to itself the compiler moves half of the
+    // loads to where their values are used.
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  floatx4 acc[TW][NT];
+#pragma unroll
+  for (int j = 0; j < TW; ++j)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[j][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto step = [&](const uintx4 (&wb)[TW], const uintx4 (&xb)[NT]) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int j = 0; j < TW; ++j)
+        acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wb[j]), __builtin_bit_cast(bf16x8, xb[t]),
+                                                            acc[j][t], 0, 0, 0);
+  };
+  // (whole words: as bfloat16 vectors the compiler puts the halves together again behind each load, and waits for it)
+  uintx4 wa[A][TW], xa[A][NT], wb[A][TW], xb[A][NT];
+  fill(wa, xa, 0);
+  if (EP == FL_ROPE)
+#pragma unroll
+    for (int u = 0; u < PU; ++u)
+      ep_page[u] = out.cache ? out.block_table[(long)ep_span[u] * out.max_pages + ep_pos[u] / out.page_size] : 0;
+  if (SCALED) {      // the rows' scales, before the second buffer needs the registers: sums in a fixed order, then across sixteen lanes
+#pragma unroll
+    for (int u = 0; u < SU; ++u) {
+      float v = 0.f;
+#pragma unroll
+      for (int i = 0; i < FL_SS_LOADS; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v += 4 * (tid % 16 + 16 * i) + e < out.ss_parts ? ssv[u][i][e] : 0.f;
+      v = parts_sum<16>(v);
+      if (tid % 16 == 0 && tid / 16 + RR * u < 16 * NT) row_scale[tid / 16 + RR * u] = rsqrtf(v / (float)k + out.eps);
+    }
+  }
+  fill(wb, xb, A);
+  int s = 0;
+  for (; mine - s > 2 * A; s += 2 * A) {
+#pragma unroll
+    for (int i = 0; i < A; ++i) step(wa[i], xa[i]);
+    __builtin_amdgcn_sched_barrier(0);
+    fill(wa, xa, s + 2 * A);
+#pragma unroll
+    for (int i = 0; i < A; ++i) step(wb[i], xb[i]);
+    __builtin_amdgcn_sched_barrier(0);
+    fill(wb, xb, s + 3 * A);
+  }
+#pragma unroll
+  for (int i = 0; i < A; ++i)
+    if (s + i < mine) step(wa[i], xa[i]);
+#pragma unroll
+  for (int i = 0; i < A; ++i)
+    if (s + A + i < mine) step(wb[i], xb[i]);
+
+  // ---- the waves meet: lane (g, c) holds w rows 4 g ... 4 g + 3 of x row c
+#pragma unroll
+  for (int j = 0; j < TW; ++j)
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      *reinterpret_cast<floatx4*>(&part[((wave * TW + j) * NT + t) * LR_TILE + c * LR_LD + 4 * g]) = acc[j][t];
+  fl_lds_barrier();
+  auto sum_of = [&](int j, int t, int xc, int r) {               // in a fixed order
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) v += part[((w * TW + j) * NT + t) * LR_TILE + xc * LR_LD + r];
+    return v;
+  };
+  if (EP == FL_RESID) {
+    const int col = group * 16 + tid % 16, stride = (groups + 3) / 4 * 4;
+#pragma unroll
+    for (int u = 0; u < RU; ++u) {
+      const int r = tid / 16 + RR * u, xr = row0 + r;
+      const bool live = r < 16 * NT && xr < n && col < m;
+      float x = 0.f;
+      if (live) {
+        x = res_old[u] + sum_of(0, r / 16, r % 16, tid % 16);
+        out.resid[(long)xr * m + col] = x;
+        reinterpret_cast<bf16_t*>(out.y)[lr_at(out, xr, col, n, m)] = from_f32<bf16_t>(x * res_w);
+      }
+      const float ss = parts_sum<16>(x * x);
+      if (tid % 16 == 0 && r < 16 * NT && xr < n) out.ss_out[(long)xr * stride + group] = ss;
+    }
+    return;
+  }
+  if (EP == FL_SWIGLU || EP == FL_ROPE) {
+    constexpr int P = 8 * TW;                                    // pairs of a row in the workgroup
+    const int pairs = m / 2;
+    auto pair_out = [&](int u) {
+      const int idx = tid + 64 * NW * u;
+      const int p = idx % P, r = idx / P, xr = row0 + r, pair = group * P + p;
+      if (r >= 16 * NT || pair >= pairs || xr >= n) return;
+      float a = sum_of(p / 8, r / 16, r % 16, p % 8), b = sum_of(p / 8, r / 16, r % 16, p % 8 + 8);
+      if (SCALED) {
+        a *= row_scale[r];
+        b *= row_scale[r];
+      }
+      if (EP == FL_SWIGLU) {
+        reinterpret_cast<bf16_t*>(out.y)[lr_at(out, xr, pair, n, pairs)] = from_f32<bf16_t>(gate_act(a, out.act) * b);
+      } else {
+        const int e = EP == FL_ROPE ? u : 0;
+        fl_rope_store<bf16_t>(out, xr, pair, a, b, ep_cos[e], ep_sin[e], ep_page[e], out.cache ? ep_pos[e] % out.page_size : 0);
+      }
+    };
+    if (EP == FL_ROPE) {
+#pragma unroll
+      for (int u = 0; u < PU; ++u) pair_out(u);
+    } else {                           // (one copy of the code: it is read cold at every launch)
+#pragma unroll 1
+      for (int u = 0; u < (16 * NT * P + 64 * NW - 1) / (64 * NW); ++u) pair_out(u);
+    }
+  }
+}
+
+static size_t lr_lds_bytes(int nt, int tw, int nw) { return (size_t)(nw * tw * nt * LR_TILE + LR_ROWS) * sizeof(float); }
+
+template <int NT, int TW, int EP, bool SCALED, int NW>
+static int lr_launch_waves(const void* x, const FlOut& out, const void* w, int n, int m, int k, int tiles, int halves,
+                     int x_stride, hipStream_t stream) {
+  const size_t lds = lr_lds_bytes(NT, TW, NW);
+  if (lds > 64 * 1024) {
+    static const hipError_t e = hipFuncSetAttribute((const void*)linear_rows_kernel<NT, TW, EP, SCALED, NW>,
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    if (e != hipSuccess) KLLM_FAIL((int)e, "linear_rows: cannot raise the LDS limit: %s", hipGetErrorString(e));
+  }
+  const int groups = ceil_div(tiles, TW);
+  const int blocks = halves == 1 ? groups : ceil_div(groups, 8) * 16;
+  hipLaunchKernelGGL((linear_rows_kernel<NT, TW, EP, SCALED, NW>), dim3(blocks), dim3(64 * NW), lds, stream,
+                     (const bf16_t*)x, out, (const bf16_t*)w, n, m, k, tiles, halves, x_stride);
+  return 0;
+}
+
+template <int NT, int TW, int EP, bool SCALED>
+static int lr_launch(const void* x, const FlOut& out, const void* w, int n, int m, int k, int tiles, int halves,
+                     int x_stride, hipStream_t stream) {
+  // Four waves a workgroup where a CU has several of them (4,096 -> 6,144: 14.7 us with eight, 13.3 with four), eight where it
+  // has one (a step of one token at 1.1B sizes 0.3 % shorter, of 64 tokens 1.2 %).
+  if constexpr (EP != FL_SWIGLU || TW == 3)
+    if ((long)halves * ceil_div(tiles, TW) > device_cus())
+      return lr_launch_waves<NT, TW, EP, SCALED, 4>(x, out, w, n, m, k, tiles, halves, x_stride, stream);
+  return lr_launch_waves<NT, TW, EP, SCALED, 8>(x, out, w, n, m, k, tiles, halves, x_stride, stream);
+}
+
+template <int NT, int TW>
+static int lr_launch_ep(int ep, bool scaled, const void* x, const FlOut& out, const void* w, int n, int m, int k,
+                        int tiles, int halves, int xs, hipStream_t st) {
+  if (ep == FL_SWIGLU)
+    return scaled ? lr_launch<NT, TW, FL_SWIGLU, true>(x, out, w, n, m, k, tiles, halves, xs, st)
+                  : lr_launch<NT, TW, FL_SWIGLU, false>(x, out, w, n, m, k, tiles, halves, xs, st);
+  if constexpr (TW == 1) {
+    if (ep == FL_RESID) return lr_launch<NT, 1, FL_RESID, false>(x, out, w, n, m, k, tiles, halves, xs, st);
+    return scaled ? lr_launch<NT, 1, FL_ROPE, true>(x, out, w, n, m, k, tiles, halves, xs, st)
+                  : lr_launch<NT, 1, FL_ROPE, false>(x, out, w, n, m, k, tiles, halves, xs, st);
+  }
+  KLLM_FAIL(ERR_STATE, "linear_rows: no kernel for output kind %d and %d tiles", ep, TW);
+}
+
+template <int NT>
+static int lr_launch_tw(int tw, int ep, bool scaled, const void* x, const FlOut& out, const void* w, int n, int m, int k,
+                        int tiles, int halves, int xs, hipStream_t st) {
+  if (tw == 1) return lr_launch_ep<NT, 1>(ep, scaled, x, out, w, n, m, k, tiles, halves, xs, st);
+  if (tw == 2) return lr_launch_ep<NT, 2>(ep, scaled, x, out, w, n, m, k, tiles, halves, xs, st);
+  return lr_launch_ep<NT, 3>(ep, scaled, x, out, w, n, m, k, tiles, halves, xs, st);
+}
+
+}  // namespace kllm
+
+using namespace kllm;
+
+static int lr_tiles(int kind, int m) { return kind == FL_RESID ? ceil_div(m, 16) : ceil_div(m / 2, 8); }
+
+extern "C" int kllm_linear_rows_parts(int m) { return m > 0 && lr_tiles(FL_RESID, m) <= FL_SS_MAX ? lr_tiles(FL_RESID, m) : 0; }
+
+extern "C" int kllm_linear_rows(const void* x, int x_stride, const KllmLinearOut* yout, const void* w, int n, int m, int k,
+                                hipStream_t stream) {
+  KLLM_REQUIRE(x && yout && w && yout->y, "linear_rows: null pointer");
+  const int ep = yout->kind;
+  KLLM_REQUIRE(ep == FL_RESID || ep == FL_SWIGLU || ep == FL_ROPE, "linear_rows: output kind %d is not built", ep);
+  KLLM_REQUIRE(n > 0 && n <= LR_ROWS, "linear_rows: n=%d is outside [1, %d]", n, LR_ROWS);
+  KLLM_REQUIRE(m > 0 && k > 0 && k % 32 == 0, "linear_rows: bad sizes m=%d k=%d (K must be a multiple of 32)", m, k);
+  KLLM_REQUIRE(k <= (1 << 20) && m < (1 << 30), "linear_rows: sizes overflow");
+  KLLM_REQUIRE(yout->tiled && !yout->f32 && yout->nsplit <= 1,
+               "linear_rows: takes bfloat16, the tiled copy of the weights and all of K");
+  KLLM_REQUIRE((((uintptr_t)x | (uintptr_t)w) & 15) == 0, "linear_rows: operands must be 16-byte aligned");
+  if (x_stride <= 0) x_stride = k;
+  KLLM_REQUIRE(x_stride >= k && x_stride % 8 == 0 && x_stride < (1 << 23), "linear_rows: row stride %d of x does not fit K=%d",
+               x_stride, k);
+  FlOut out = {};
+  out.y = yout->y;
+  out.act = yout->act;
+  out.tiled = 1;
+  out.x_tiled = yout->x_tiled != 0;
+  out.y_tiled = yout->y_tiled != 0;
+  KLLM_REQUIRE(!out.y_tiled || (ep == FL_RESID && m % 32 == 0) || (ep == FL_SWIGLU && m % 64 == 0),
+               "linear_rows: no tiled output of kind %d and m=%d", ep, m);
+  const int tiles = lr_tiles(ep, m);
+  const bool scaled = yout->ss_in != nullptr;
+  if (scaled) {
+    KLLM_REQUIRE(ep != FL_RESID, "linear_rows: only the gate and the rotation epilogues scale their rows");
+    KLLM_REQUIRE(yout->ss_parts >= 1 && yout->ss_parts <= FL_SS_MAX && ((uintptr_t)yout->ss_in & 15) == 0 && yout->eps >= 0.f,
+                 "linear_rows: %d partial sums of squares per row are outside [1, %d], or they are not 16-byte aligned",
+                 yout->ss_parts, FL_SS_MAX);
+    out.ss_in = yout->ss_in;
+    out.ss_parts = yout->ss_parts;
+    out.eps = yout->eps;
+  }
+  if (ep == FL_RESID) {
+    KLLM_REQUIRE(yout->resid && yout->norm_w && yout->ss_out, "linear_rows: the residual epilogue needs the stream, "
+                 "the norm's weight and room for the sums of squares");
+    KLLM_REQUIRE(kllm_linear_rows_parts(m) > 0, "linear_rows: %d columns leave more than %d sums of squares per row", m,
+                 FL_SS_MAX);
+    out.resid = yout->resid;
+    out.norm_w = yout->norm_w;
+    out.ss_out = yout->ss_out;
+  } else {
+    KLLM_REQUIRE(m % 2 == 0, "linear_rows: m=%d must be even for a pair epilogue", m);
+  }
+  KLLM_REQUIRE(ep != FL_SWIGLU || (out.act >= 0 && out.act < ACT_COUNT), "linear_rows: unknown activation %d", out.act);
+  if (ep == FL_ROPE) {
+    const int H = yout->H, KV = yout->KV, hd = yout->hd;
+    KLLM_REQUIRE(H > 0 && hd > 0 && hd % 2 == 0, "linear_rows: bad heads H=%d hd=%d", H, hd);
+    KLLM_REQUIRE((yout->cos_t == nullptr) == (yout->sin_t == nullptr), "linear_rows: cos and sin go together");
+    if (yout->cache)
+      KLLM_REQUIRE(KV > 0 && yout->positions && yout->span_of_token && yout->block_table && yout->max_pages > 0 &&
+                       yout->page_size > 0,
+                   "linear_rows: bad cache arguments");
+    KLLM_REQUIRE(m == H * hd + (yout->cache ? 2 * KV * hd : 0), "linear_rows: m=%d does not fit the heads", m);
+    out.cos_t = yout->cos_t;
+    out.sin_t = yout->sin_t;
+    out.cache = yout->cache;
+    out.positions = yout->positions;
+    out.span_of_token = yout->span_of_token;
+    out.block_table = yout->block_table;
+    out.max_pages = yout->max_pages;
+    out.page_size = yout->page_size;
+    out.H = H;
+    out.KV = KV;
+    out.hd = hd;
+  }
+  const int cus = device_cus();
+  // Tiles a workgroup: the least that leaves one round of the chip, three at most (2 x 5,632 x 2,048, 8 / 64 rows: 12.1 / 17.5 us with two, 11.0
+  // / 14.9 with three, 13.3 / 16.4 with four; 2 x 14,336 x 4,096, 16 / 64 rows: 48.5 / 62.0, 46.5 / 59.3, 54.5 / 59.6).
+  int tw = 1;
+  if (ep == FL_SWIGLU)
+    while (tw < 3 && ceil_div(tiles, tw) > cus) ++tw;
+  const int row_tiles = ceil_div(n, 16);
+  // Halves of the rows where the busiest CU then has fewer tiles of rows to take (or as many, of workgroups that share it
+  // anyway): 64 rows against 2,048 x 5,632 (128 tiles) 17.6 -> 12.2 us, 6,144 x 4,096 (384) 25.4 -> 21.2, 48 rows 21.3 -> 18.8; not
+  // 4,096 x 14,336 (256) 41.0 -> 46.7, nor 2,560 x 2,048 (160) at 32 rows 5.0 -> 5.5.
+  const int whole = ceil_div(tiles, cus) * row_tiles, halved = ceil_div(2L * tiles, cus) * ceil_div(row_tiles, 2);
+  const int halves = ep != FL_SWIGLU && (halved < whole || (halved == whole && tiles > cus)) ? 2 : 1;
+  const int nt = ceil_div(row_tiles, halves);
+  const int rc = nt == 1 ? lr_launch_tw<1>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream)
+               : nt == 2 ? lr_launch_tw<2>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream)
+               : nt == 3 ? lr_launch_tw<3>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream)
+                         : lr_launch_tw<4>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream);
+  if (rc) return rc;
+  KLLM_CHECK_LAUNCH("linear_rows");
+  return 0;
+}

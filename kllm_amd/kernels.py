@@ -21,7 +21,7 @@ import torch
 DT_F32, DT_BF16 = 0, 1
 GEMM_PLAIN, GEMM_TILED_F32, GEMM_MFMA_BF16, GEMM_SKINNY_BF16, GEMM_GEMV, GEMM_GEMV_LDS, GEMM_MFMA_F32 = 0, 1, 2, 3, 4, 5, 6
 GEMV_BEST_ROWS = 0         # rows up to which they beat the MFMA kernels in bfloat16: none (a step at 1.1B sizes, one token: 1.036 against 0.963 ms)
-ABI_VERSION = 18
+ABI_VERSION = 19
 
 
 class KernelError(RuntimeError):
@@ -106,6 +106,8 @@ def _declare(lib):
         "kllm_gemv_resid_parts": [I],
         "kllm_fused_linear": [P, I, P, P, I, I, I, I, P],
         "kllm_fused_linear_resid_parts": [I, I],
+        "kllm_linear_rows": [P, I, P, P, I, I, I, P],
+        "kllm_linear_rows_parts": [I],
         "kllm_fused_linear_passes": [I, I, I, I],
         "kllm_fused_linear_tile": [P, P, I, I, I, I, I, I, I, I, P],
         "kllm_command_op": [c_char_p],
@@ -196,7 +198,7 @@ def _declare(lib):
 # which of their arguments are pointers to structures that travel with the command.
 LAUNCHING = ("kllm_embed", "kllm_add_rmsnorm", "kllm_rope_tables", "kllm_rope_append", "kllm_silu_mul",
              "kllm_sum_splits", "kllm_gemm", "kllm_gemm_swiglu", "kllm_gemv_plain", "kllm_gemv_swiglu",
-             "kllm_gemv_resid", "kllm_gemv_rope_append", "kllm_fused_linear", "kllm_attn_generic",
+             "kllm_gemv_resid", "kllm_gemv_rope_append", "kllm_fused_linear", "kllm_linear_rows", "kllm_attn_generic",
              "kllm_attn_decode", "kllm_attn_prefill", "kllm_sample", "kllm_gemm_act", "kllm_add_sinusoid", "kllm_unary_act",
              "kllm_group_norm_add", "kllm_qk_norm_append", "kllm_delta_prep", "kllm_delta_scan", "kllm_delta_out",
              "kllm_norm_residual", "kllm_rope_tables_freq", "kllm_qkv_norm_append", "kllm_gate_bias", "kllm_moe_route",
@@ -208,7 +210,7 @@ LAUNCHING = ("kllm_embed", "kllm_add_rmsnorm", "kllm_rope_tables", "kllm_rope_ap
              "kllm_decayed_scan", "kllm_decayed_out", "kllm_decayed_step", "kllm_token_gate", "kllm_soft_cap")
 DYNAMIC_ARGS = {"kllm_attn_prefill": (19, 20)}     # arguments that may be a StepValue
 STRUCT_ARGS = {"kllm_gemv_plain": (7,), "kllm_gemv_swiglu": (8,), "kllm_gemv_rope_append": (17,),
-               "kllm_fused_linear": (2,)}
+               "kllm_fused_linear": (2,), "kllm_linear_rows": (2,)}
 
 
 def _check(rc: int, what: str):
@@ -832,7 +834,7 @@ class _LinearOut(ctypes.Structure):
                 ("kind", c_int), ("nsplit", c_int), ("max_pages", c_int), ("page_size", c_int),
                 ("H", c_int), ("KV", c_int), ("hd", c_int), ("act", c_int),
                 ("resid", c_void_p), ("norm_w", c_void_p), ("ss_out", c_void_p), ("ss_in", c_void_p),
-                ("ss_parts", c_int), ("eps", c_float), ("tiled", c_int), ("f32", c_int)]
+                ("ss_parts", c_int), ("eps", c_float), ("tiled", c_int), ("f32", c_int), ("x_tiled", c_int), ("y_tiled", c_int)]
 
 
 FUSED_LINEAR_MAX_ROWS = 32
@@ -970,8 +972,61 @@ class Rope:
 FUSED_LINEAR_UNARY = 16    # LINEAR_PARTS with act = this + an activation without a gate: see fused_linear
 
 
+class TiledRows:
+    """Rows [n, k] (k a multiple of 32) as ``linear_rows`` leaves them for the next such product: ``data`` [``stored(n)``, k]
+    in the order that product's lanes read, not row by row."""
+
+    @staticmethod
+    def stored(n):
+        return n if n <= 16 else -(-n // 16) * 16
+
+    def __init__(self, data, n):
+        self.data, self.shape = data, (int(n), int(data.shape[1]))
+
+    @property
+    def dtype(self):
+        return self.data.dtype
+
+
+LINEAR_ROWS_MAX = 64
+LINEAR_ROWS_BYTES = 380_000
+
+
+@functools.lru_cache(maxsize=4096)
+def linear_rows_best(kind, n, m, k, dtype=torch.bfloat16, tiled_x=True) -> bool:
+    """Whether ``linear_rows`` takes the product of n rows against the tiled copy of w [m, k] and is the fastest way.
+    Up to 16 rows it always is (a step in us, the decode-batch kernel's products against these: 1 / 4 / 8 / 16 tokens at 1.1B sizes 914 /
+    939 / 971 / 1,080 against 888 / 906 / 937 / 1,031; 4 / 8 / 16 at 8B sizes 3,580 / 3,795 / 4,065 against 3,397 / 3,506 / 3,750).
+    Beyond, while the rows that the busiest CU reads in all its workgroups stay below ``LINEAR_ROWS_BYTES`` (rows that are not
+    ``TiledRows`` take a CU longer and count twice): 2,048 x 5,632 at 64 rows has it read 360 KB, 12.1 us against 10.9 and 4.7 for K
+    in slices and the norm that adds them; 4,096 x 4,096 at 48 rows 390 KB, 16.4 against 15 (17 / 32 / 48 / 64 tokens at 1.1B
+    sizes 1,201 / 1,377 / 1,559 / 1,663 against 1,067 / 1,155 / 1,246 / 1,370; with all products at 8B sizes 64 tokens
+    4,902 against 6,146)."""
+    if dtype != torch.bfloat16 or not 1 <= n <= LINEAR_ROWS_MAX or k % 32 or k > 1 << 20:
+        return False
+    if kind == LINEAR_RESID and library().kllm_linear_rows_parts(int(m)) == 0:
+        return False
+    if n <= 16:
+        return True
+    tiles, cus, row_tiles = -(-m // 16), device_cus(), -(-n // 16)
+    busiest = -(-tiles // (3 * cus)) * row_tiles if kind == LINEAR_SWIGLU else min(
+        -(-tiles // cus) * row_tiles, -(-2 * tiles // cus) * -(-row_tiles // 2))
+    return 32 * k * busiest * (1 if tiled_x else 2) <= LINEAR_ROWS_BYTES
+
+
+def linear_rows(w, y, kind, x, rope=None, act=ACT_SILU, resid=None, norm_weight=None, ss_out=None):
+    """``fused_linear`` for up to 64 rows of bfloat16, K a multiple of 32: LINEAR_RESID, LINEAR_SWIGLU and
+    LINEAR_ROPE from the tiled copy ``w`` of the weights, nothing staged in LDS.  ``x`` (also inside a ``ScaledRows``) may be
+    ``TiledRows``, and so may ``y`` of the first two."""
+    if not isinstance(w, TiledWeights):
+        raise KernelError("linear_rows: takes the tiled copy of the weights")
+    if kind not in (LINEAR_RESID, LINEAR_SWIGLU, LINEAR_ROPE):
+        raise KernelError(f"linear_rows: output kind {kind} is not built")
+    fused_linear(w, y, kind, x, rope=rope, act=act, resid=resid, norm_weight=norm_weight, ss_out=ss_out, _rows=True)
+
+
 def fused_linear(w, y, kind, x, nsplit=1, tiles_per_wg=1, rope=None, act=ACT_SILU, resid=None, norm_weight=None,
-                 ss_out=None, unary=None):
+                 ss_out=None, unary=None, _rows=False):
     """One launch for a decode batch's product of x [n, k] (bfloat16, or float32 up to 16 rows; a view
     with a row stride is taken) with w [m, k], and the step after it, by
     ``kind`` (bfloat16 below is the operands' type): LINEAR_PARTS y float32 [nsplit, n, m]; LINEAR_SWIGLU y bfloat16
@@ -1002,6 +1057,15 @@ def fused_linear(w, y, kind, x, nsplit=1, tiles_per_wg=1, rope=None, act=ACT_SIL
         lo.ss_in, lo.ss_parts, lo.eps = _ptr(sr.ss, "fused_linear ss", torch.float32), sr.parts, sr.eps
     n = x.shape[0]
     lo.kind, lo.nsplit, lo.act = kind, nsplit, int(act)
+    for name, t in (("x", x), ("y", y)):
+        if isinstance(t, TiledRows):
+            if (not _rows or (name == "y" and kind == LINEAR_ROPE) or t.dtype != typ or not t.data.is_contiguous()
+                    or t.shape[1] % 32 or t.data.shape[0] != TiledRows.stored(n) or (name == "x" and t.shape[1] != k)):
+                raise KernelError(f"linear_rows: tiled rows {t.shape} do not fit {name}, or the kernel takes none")
+    if isinstance(x, TiledRows):
+        lo.x_tiled, x = 1, x.data[:n]
+    if isinstance(y, TiledRows):
+        lo.y_tiled, y = 1, y.data[:n]
     if x.dim() != 2 or x.shape[1] != k or x.dtype != typ or x.stride(1) != 1 or not x.is_cuda:
         raise KernelError(f"fused_linear: x {tuple(x.shape)} {x.dtype} does not fit w {tuple(w.shape)}")
     x_ptr, x_stride = x.data_ptr(), (x.stride(0) if n > 1 else k)
@@ -1052,6 +1116,9 @@ def fused_linear(w, y, kind, x, nsplit=1, tiles_per_wg=1, rope=None, act=ACT_SIL
     if tuple(y.shape) != want or y.dtype != dt:
         raise KernelError(f"fused_linear: output {tuple(y.shape)} {y.dtype}, expected {want} {dt}")
     lo.y = _ptr(y, "fused_linear y")
+    if _rows:
+        _launch("kllm_linear_rows", "linear_rows", x_ptr, x_stride, lo, _ptr(w, "linear_rows w"), n, m, k, _stream())
+        return
     _launch("kllm_fused_linear", "fused_linear", x_ptr, x_stride, lo, _ptr(w, "fused_linear w"), n, m, k,
                                        tiles_per_wg, _stream())
 

@@ -30,7 +30,7 @@ import torch
 
 from .. import kernels as K
 from .base import Normed, Part, register_part
-from .linear import decode_linear, fused_f32, linear, linear_into, tiled_copy
+from .linear import decode_linear, fused_f32, linear, linear_into, rows_kernel, tiled_copy
 from .spec import CacheNeed, WeightSpec
 
 
@@ -190,6 +190,15 @@ class CausalSelfAttention(Part):
             raise ValueError(f"attention: pages of {page_size} tokens are not built "
                              f"(1 to {K.GENERIC_MAX_PAGE_SIZE})")
 
+    def rows_input(self):
+        """(kind, rows, columns) of the input projections, where their tiled copy is there (``K.linear_rows_best``)."""
+        return (K.LINEAR_ROPE, *self.w_in.shape) if self._tiled.get("in") is not None else None
+
+    def _rows(self, n, x):
+        """Whether the input projections of the rows x run on ``K.linear_rows``."""
+        return self.plain_rotation and rows_kernel(self.runtime, K.LINEAR_ROPE, n, self.w_in, self._tiled.get("in"),
+                                                   isinstance(getattr(x, "xw", x), K.TiledRows))
+
     def _fused_tiles(self, n):
         """Tiles per workgroup of the decode-batch kernel for the input projections of n
         tokens, or 0 where it is not taken."""
@@ -206,7 +215,8 @@ class CausalSelfAttention(Part):
             opts = self.runtime.options
             gemv = (K.gemv_fits(n, self.w_in.shape[0], self.hidden, dtype) and n <= K.normed_max_rows()
                     and not opts.get("no_fused_gemv") and self.plain_rotation and xn.xw is None)
-            scaled = (not gemv and xn.xw is not None and self._fused_tiles(n) > 0)
+            scaled = (not gemv and xn.xw is not None
+                      and (self._rows(n, xn) or (self._fused_tiles(n) > 0 and not isinstance(xn.xw, K.TiledRows))))
             # the small-batch kernel below normalises while it stages its input, the decode-batch
             # kernel scales its sums by the row
             xn = xn.kernel_input() if gemv else xn.scaled_rows() if scaled else xn.materialize(ctx)
@@ -227,6 +237,10 @@ class CausalSelfAttention(Part):
             K.gemv_rope_append(xn, self.w_in, q, cos, sin, pages, ctx.positions, ctx.span_of_token,
                                cache.block_table, cache.page_size, self.heads, self.kv_heads,
                                self.head_dim)
+        elif self._rows(n, xn):
+            K.linear_rows(self._tiled["in"], q, K.LINEAR_ROPE, xn,
+                          rope=K.Rope(cos, sin, pages, ctx.positions, ctx.span_of_token, cache.block_table,
+                                      cache.page_size, self.heads, self.kv_heads, self.head_dim))
         elif self._fused_tiles(n) > 0:
             # a decode batch: the same on the matrix cores
             K.fused_linear(self._tiled.get("in") or self.w_in, q, K.LINEAR_ROPE, x=xn,

@@ -44,6 +44,9 @@ class PreNormBlock(Part):
     def bind(self, weights):
         for p in self.parts():
             p.bind(weights)
+        # what a residual product may leave its rows in the order of
+        for norm, consumer in ((self.norm_mixer, self.mixer), (self.norm_ff, self.feed_forward)):
+            norm.feeds = consumer.rows_input() if consumer.takes_normed and hasattr(consumer, "rows_input") else None
 
     def cache_need(self):
         return self.mixer.cache_need()

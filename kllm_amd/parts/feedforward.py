@@ -13,7 +13,7 @@ import torch
 
 from .. import kernels as K
 from .base import Normed, Part, register_part
-from .linear import decode_batch_fits, decode_linear, fused_f32, linear, linear_into, tiled_copy
+from .linear import decode_batch_fits, decode_linear, fused_f32, linear, linear_into, rows_kernel, sink_takes_rows, tiled_copy
 from .spec import WeightSpec
 
 
@@ -49,6 +49,10 @@ class GatedFeedForward(Part):
         self._tiled = {"gu": tiled_copy(self.runtime, self.w_gu, K.LINEAR_SWIGLU),
                        "down": tiled_copy(self.runtime, self.w_down, K.LINEAR_PARTS)}
 
+    def rows_input(self):
+        """(kind, rows, columns) of the gate and up product, where its tiled copy is there (``K.linear_rows_best``)."""
+        return (K.LINEAR_SWIGLU, *self.w_gu.shape) if self._tiled.get("gu") is not None else None
+
     def _gate_in_tiles(self, n, dtype):
         """Decode batches whose gate runs in the tiled product's epilogue: more than 32 rows
         where the tiles of 64 gate columns give three fifths of the CUs a workgroup, more
@@ -68,14 +72,22 @@ class GatedFeedForward(Part):
         tiles = K.fused_linear_tiles(n, 2 * self.intermediate, self.hidden, dtype) if best else 0
         if gemv and (isinstance(xn, Normed) and xn.xw is not None or dtype == torch.float32 and tiles > 0):
             gemv = False       # the producer was the decode-batch kernel: its consumer is, too
-        fused = not gemv and tiles > 0 and not opts.get("no_fused_linear")
+        rows = not gemv and rows_kernel(self.runtime, K.LINEAR_SWIGLU, n, self.w_gu, self._tiled.get("gu"),
+                                           isinstance(getattr(xn, "xw", xn), K.TiledRows))
+        fused = not gemv and not rows and tiles > 0 and not opts.get("no_fused_linear")
         if isinstance(xn, Normed):     # the small-batch kernel below normalises while it stages its input,
             # the decode-batch kernel scales its sums by the row
             xn = (xn.kernel_input() if gemv and n <= K.normed_max_rows()
-                  else xn.scaled_rows() if fused and xn.xw is not None else xn.materialize(ctx))
-        h = ctx.buf("ffn.h", (n, self.intermediate), dtype)
+                  else xn.scaled_rows() if xn.xw is not None and (rows or fused and not isinstance(xn.xw, K.TiledRows))
+                  else xn.materialize(ctx))
+        if rows and sink_takes_rows(self.runtime, sink, n, self.w_down, self._tiled.get("down")):
+            h = K.TiledRows(ctx.buf("ffn.ht", (K.TiledRows.stored(n), self.intermediate), dtype), n)
+        else:
+            h = ctx.buf("ffn.h", (n, self.intermediate), dtype)
         if gemv:
             K.gemv_swiglu(xn, self.w_gu, h, self.act)   # few tokens: both products and the gate in one launch
+        elif rows:
+            K.linear_rows(self._tiled["gu"], h, K.LINEAR_SWIGLU, xn, act=self.act)
         elif fused:
             # a decode batch: the same on the matrix cores
             K.fused_linear(self._tiled.get("gu") or self.w_gu, h, K.LINEAR_SWIGLU, x=xn, act=self.act,

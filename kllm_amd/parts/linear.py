@@ -5,6 +5,7 @@ it returns partial sums [nsplit, n, m] that the consuming kernel adds (norm,
 rotary + append, SiLU gate); with the compute dtype as result it returns
 [n, m].  Which kernel runs depends only on the dtype and on n:
 
+  (a product whose epilogue does the step after it, up to 64 rows of bfloat16: ``K.linear_rows``)
   n <= 8    float32: gemv with X in LDS and the whole of K in one wave (no
             partial sums), if the sizes fit, and from five rows on the decode-batch kernel
             (``fused_f32``) where its epilogue or one whole result is wanted; bfloat16 up to 4 rows: the streaming
@@ -191,6 +192,24 @@ def fused_f32(rt, n):
             and opts.get("gemm_algo") is None)
 
 
+def rows_kernel(rt, kind, n, w, w_tiled, tiled_x):
+    """Whether a product of n rows (``TiledRows``: ``tiled_x``) with the step after it runs on ``K.linear_rows``."""
+    return (w_tiled is not None and not rt.options.get("no_fused_linear") and rt.options.get("gemm_algo") is None
+            and rt.options.get("gemm") != "library" and K.linear_rows_best(kind, n, w.shape[0], w.shape[1], w_tiled.dtype, tiled_x))
+
+
+def _sink_fits(rt, sink, n, m):
+    opts, norm = rt.options, sink.norm
+    return not (opts.get("no_fused_norm") or opts.get("gemm_algo") is not None or opts.get("no_fused_gemv")
+                or tuple(sink.x.shape) != (n, m) or norm.weight is None or norm.weight.numel() != m)
+
+
+def sink_takes_rows(rt, sink, n, w, w_tiled):
+    """Whether ``linear_into`` will run the product of ``TiledRows`` on ``K.linear_rows``."""
+    return (sink is not None and _sink_fits(rt, sink, n, w.shape[0])
+            and rows_kernel(rt, K.LINEAR_RESID, n, w, w_tiled, True))
+
+
 def linear_into(ctx, x, w, sink, tag, w_tiled=None):
     """x . w^T added to the residual stream of ``sink`` in the product's own
     epilogue: returns the ``Normed`` that stands for the norm behind the addition, or None
@@ -202,19 +221,25 @@ def linear_into(ctx, x, w, sink, tag, w_tiled=None):
     n, k = x.shape
     m = w.shape[0]
     rt = ctx.runtime
-    if rt.options.get("no_fused_norm") or rt.options.get("gemm_algo") is not None:
-        return None
-    if rt.options.get("no_fused_gemv"):
+    if not _sink_fits(rt, sink, n, m):
         return None
     norm = sink.norm
-    if tuple(sink.x.shape) != (n, m) or norm.weight is None or norm.weight.numel() != m:
-        return None
     f32 = x.dtype == torch.float32
     parts = 0 if f32 and fused_f32(rt, n) else K.resid_parts(n, m, k, x.dtype)
     if parts:
         ss = ctx.buf(tag + ".ss", (n, -(-parts // 4) * 4), torch.float32)
         K.linear_resid(x, w, sink.x, ss)
         return Normed(sink.x, ss, parts, norm)
+    if rows_kernel(rt, K.LINEAR_RESID, n, w, w_tiled, isinstance(x, K.TiledRows)):
+        parts = -(-m // 16)
+        ss = ctx.buf(tag + ".ss", (n, -(-parts // 4) * 4), torch.float32)
+        feeds = getattr(norm, "feeds", None)
+        if feeds is not None and K.linear_rows_best(feeds[0], n, feeds[1], feeds[2], x.dtype):
+            xw = K.TiledRows(ctx.buf(tag + ".xt", (K.TiledRows.stored(n), m), x.dtype), n)     # for the product behind the norm
+        else:
+            xw = ctx.buf(tag + ".xw", (n, m), x.dtype)
+        K.linear_rows(w_tiled, xw, K.LINEAR_RESID, x, resid=sink.x, norm_weight=norm.weight, ss_out=ss)
+        return Normed(sink.x, ss, parts, norm, xw=xw)
     if not (fused_f32(rt, n) if f32 else n <= K.FUSED_NORM_BEST_ROWS) or rt.options.get("no_fused_linear"):
         return None
     # a decode batch on the matrix cores: all of K in a workgroup, the addition in the epilogue, and

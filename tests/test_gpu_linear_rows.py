@@ -1,0 +1,135 @@
+"""Products of 17 to 64 rows with the step after them (``kernels.linear_rows``) against float64 references: row
+tiles that are whole and not, one and two halves of the rows, one to three tiles a workgroup, K that gives the eight
+waves unequal shares or none."""
+
+import pytest
+import torch
+
+import plain_llama as P
+from test_gpu_kernels import DEV, K, _bf, read_cache, rnd
+
+pytestmark = pytest.mark.gpu
+
+
+# Tiles of W at most half the CUs: two workgroups share the rows (2,048 and below); more: one (4,096).
+@pytest.mark.parametrize("n,m,k", [(1, 16, 32), (17, 48, 96), (5, 64, 2048), (8, 2048, 5632), (33, 72, 288), (45, 2048, 2048), (48, 100, 5632),
+                                   (64, 2048, 5632), (64, 4096, 1056), (50, 4096, 4096), (32, 1000, 736), (63, 4090, 160)])
+def test_resid_then_scaled_consumers(n, m, k):
+    """The product added to the residual stream, what the norm behind it needs left beside it, and the two
+    consumers that scale their sums.  Bounds as for the decode-batch kernel's test: sums of k products of 16-bit
+    operands in 32 bits, xw and the consumers' results rounded to 16 bits."""
+    k_, eps = K(), 1e-5
+    x, w = _bf(n, k, seed=1, scale=0.5), _bf(m, k, seed=2, scale=0.1)
+    resid, nw = rnd(n, m, seed=3, scale=2.0), 1 + 0.2 * rnd(m, seed=4)
+    parts = -(-m // 16)
+    ss = torch.full((n, -(-parts // 4) * 4), float("nan"), device=DEV)
+    xw = torch.full((n, m), float("nan"), dtype=torch.bfloat16, device=DEV)
+    stream = resid.clone()
+    k_.linear_rows(k_.fused_linear_tile(w, k_.LINEAR_PARTS), xw, k_.LINEAR_RESID, x, resid=stream, norm_weight=nw, ss_out=ss)
+    want_x = resid.double() + x.double() @ w.double().T
+    assert (stream.double() - want_x).abs().max() < 1e-3 * k ** 0.5 * 0.05 + 1e-4
+    assert (xw.double() - want_x * nw.double()).abs().max() < 0.005 * want_x.abs().max() * 1.2 + 1e-3
+    got_ss = ss[:, :parts].double().sum(1)
+    assert ((got_ss - (want_x ** 2).sum(1)).abs() / (want_x ** 2).sum(1)).max() < 1e-4
+    if m % 32:
+        return
+    want_n = P.rmsnorm(want_x, nw.double(), eps)
+    # the same rows in the order that the next product's lanes read them: the same bits
+    xt = k_.TiledRows(torch.full((k_.TiledRows.stored(n), m), float("nan"), dtype=torch.bfloat16, device=DEV), n)
+    stream2, ss2 = resid.clone(), torch.zeros_like(ss)
+    k_.linear_rows(k_.fused_linear_tile(w, k_.LINEAR_PARTS), xt, k_.LINEAR_RESID, x, resid=stream2, norm_weight=nw, ss_out=ss2)
+    assert torch.equal(stream2, stream) and torch.equal(ss2[:, :parts], ss[:, :parts])
+    sr, st = k_.ScaledRows(xw, ss, parts, eps), k_.ScaledRows(xt, ss, parts, eps)
+    for f in (32, 40, 2056, 3080):      # one tile to a workgroup (4 and 5 of them), two (257 x 2), two (385)
+        wg = _bf(2 * f, m, seed=5, scale=0.1)
+        h = torch.full((n, f), float("nan"), dtype=torch.bfloat16, device=DEV)
+        k_.linear_rows(k_.fused_linear_tile(wg, k_.LINEAR_SWIGLU), h, k_.LINEAR_SWIGLU, sr)
+        g = want_n @ wg[:f].double().T
+        want = g * torch.sigmoid(g) * (want_n @ wg[f:].double().T)
+        assert (h.double() - want).abs().max() < 0.01 * want.abs().max() + 2e-3
+        h2 = torch.full_like(h, float("nan"))
+        k_.linear_rows(k_.fused_linear_tile(wg, k_.LINEAR_SWIGLU), h2, k_.LINEAR_SWIGLU, st)
+        assert torch.equal(h2, h)
+        if f % 32 == 0:                 # a tiled output as the next product's input
+            wn = _bf(96, f, seed=9, scale=0.1)
+            ht = k_.TiledRows(torch.full((k_.TiledRows.stored(n), f), float("nan"), dtype=torch.bfloat16, device=DEV), n)
+            k_.linear_rows(k_.fused_linear_tile(wg, k_.LINEAR_SWIGLU), ht, k_.LINEAR_SWIGLU, st)
+            got = []
+            for hin in (h, ht):
+                z, y, zs = torch.zeros(n, 96, device=DEV), torch.empty(n, 96, dtype=torch.bfloat16, device=DEV), torch.empty(n, 8, device=DEV)
+                k_.linear_rows(k_.fused_linear_tile(wn, k_.LINEAR_PARTS), y, k_.LINEAR_RESID, hin, resid=z,
+                               norm_weight=torch.ones(96, device=DEV), ss_out=zs)
+                got.append((z, y))
+            assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    H, hd = 2, 16
+    wq = _bf(H * hd, m, seed=6, scale=0.1)
+    pos = torch.arange(5, 5 + n, dtype=torch.int32, device=DEV)
+    cos, sin = torch.empty(n, hd // 2, device=DEV), torch.empty(n, hd // 2, device=DEV)
+    k_.rope_tables(cos, sin, pos, hd, 10000.0)
+    q = torch.full((n, H * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+    rope = k_.Rope(cos, sin, None, None, None, None, 16, H, 1, hd)
+    k_.linear_rows(k_.fused_linear_tile(wq, k_.LINEAR_ROPE, rope), q, k_.LINEAR_ROPE, sr, rope=rope)
+    want_q = P.rope((want_n @ wq.double().T).cpu(), pos.cpu().tolist(), H, hd, 10000.0)
+    assert (q.cpu().double() - want_q).abs().max() < 0.01 * want_q.abs().max() + 2e-3
+
+
+@pytest.mark.parametrize("n,f,k", [(64, 5632, 2048), (45, 5632, 512), (33, 24, 64), (17, 3000, 1024), (61, 4104, 320),
+                                   (31, 6000, 96)])
+def test_swiglu_of_a_strided_view(n, f, k):
+    """Up to three tiles a workgroup (5,632 and 6,000: 704 and 750 tiles), the last group not whole."""
+    k_ = K()
+    x, w = _bf(n, k + 24, seed=7, scale=0.5)[:, 8:8 + k], _bf(2 * f, k, seed=8, scale=0.1)
+    h = torch.full((n, f), float("nan"), dtype=torch.bfloat16, device=DEV)
+    k_.linear_rows(k_.fused_linear_tile(w, k_.LINEAR_SWIGLU), h, k_.LINEAR_SWIGLU, x, act=k_.ACT_GELU_TANH)
+    xd, wd = x.double(), w.double()
+    want = torch.nn.functional.gelu(xd @ wd[:f].T, approximate="tanh") * (xd @ wd[f:].T)
+    assert (h.double() - want).abs().max() < 0.01 * want.abs().max() + 1e-3
+
+
+@pytest.mark.parametrize("H,KV,hd,ps,d", [(4, 2, 16, 16, 64), (5, 5, 48, 32, 96), (32, 4, 64, 16, 2048), (3, 3, 80, 16, 128)])
+def test_rope_append(H, KV, hd, ps, d):
+    """Projections, rotation and append of 40 tokens of four requests."""
+    k_, theta = K(), 10000.0
+    spans = [(ps - 3, 13), (0, 9), (ps - 1, 1), (5, 17)]
+    n = sum(l for _, l in spans)
+    pos = torch.tensor([p0 + i for p0, l in spans for i in range(l)], dtype=torch.int32, device=DEV)
+    sot = torch.tensor([s for s, (_, l) in enumerate(spans) for _ in range(l)], dtype=torch.int32, device=DEV)
+    tables = [[9, 4], [2, 1], [7, -1], [3, 0]]
+    bt = torch.tensor(tables, dtype=torch.int32, device=DEV)
+    qd, kvd = H * hd, KV * hd
+    x, w = _bf(n, d, seed=3, scale=0.5), _bf(qd + 2 * kvd, d, seed=4, scale=0.1)
+    cos, sin = torch.empty(n, hd // 2, device=DEV), torch.empty(n, hd // 2, device=DEV)
+    k_.rope_tables(cos, sin, pos, hd, theta)
+    cache = torch.full((12, 2, KV, ps * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+    q_out = torch.full((n, qd), float("nan"), dtype=torch.bfloat16, device=DEV)
+    rope = k_.Rope(cos, sin, cache, pos, sot, bt, ps, H, KV, hd)
+    k_.linear_rows(k_.fused_linear_tile(w, k_.LINEAR_ROPE, rope), q_out, k_.LINEAR_ROPE, x, rope=rope)
+    full = P.linear(x.cpu().double(), w.cpu().double())
+    want_q = P.rope(full[:, :qd], pos.cpu().tolist(), H, hd, theta)
+    want_k = P.rope(full[:, qd:qd + kvd], pos.cpu().tolist(), KV, hd, theta)
+    t = 0.01 * full.abs().max() + 1e-3
+    assert (q_out.cpu().double() - want_q).abs().max() < t
+    off = 0
+    for s, (p0, l) in enumerate(spans):
+        ks, vs = read_cache(cache, tables[s], p0 + l, KV, hd, ps)
+        assert (ks[p0:].double() - want_k[off:off + l]).abs().max() < t
+        assert (vs[p0:].double() - full[off:off + l, qd + kvd:]).abs().max() < t
+        assert torch.isnan(ks[:p0]).all() and torch.isnan(vs[:p0]).all()
+        off += l
+
+
+def test_refusals():
+    k_ = K()
+    w = _bf(64, 96, seed=1, scale=0.1)
+    tiled = k_.fused_linear_tile(w, k_.LINEAR_SWIGLU)
+    h = torch.empty(20, 32, dtype=torch.bfloat16, device=DEV)
+    with pytest.raises(k_.KernelError, match="tiled copy"):
+        k_.linear_rows(w, h, k_.LINEAR_SWIGLU, _bf(20, 96, seed=2, scale=1.0))
+    with pytest.raises(k_.KernelError, match="outside"):
+        k_.linear_rows(tiled, torch.empty(65, 32, dtype=torch.bfloat16, device=DEV), k_.LINEAR_SWIGLU, _bf(65, 96, seed=2, scale=1.0))
+    with pytest.raises(k_.KernelError, match="multiple of 32"):
+        k_.linear_rows(k_.fused_linear_tile(_bf(64, 40, seed=1, scale=0.1), k_.LINEAR_SWIGLU), h, k_.LINEAR_SWIGLU,
+                       _bf(20, 40, seed=2, scale=1.0))
+    with pytest.raises(k_.KernelError, match="not built"):
+        k_.linear_rows(k_.fused_linear_tile(w, k_.LINEAR_PARTS), torch.empty(1, 20, 64, device=DEV), k_.LINEAR_PARTS,
+                       _bf(20, 96, seed=2, scale=1.0))
