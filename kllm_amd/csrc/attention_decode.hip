@@ -54,7 +54,8 @@ __device__ __forceinline__ float group4_sum(float v) {
 }
 
 // KEPT: kept first positions behind the window (an instance of its own: the others carry none of it)
-template <int HDT, int kDecodeWaves, bool BIASED = false, bool KEPT = false>  // head_dim = 16 * HDT; BIASED: scores lose slope * distance
+// TILED: the output's rows in the next product's order (gate.side; one instance for both cost the plain one 2 us of 49, in scalar registers)
+template <int HDT, int kDecodeWaves, bool BIASED = false, bool KEPT = false, bool TILED = false>  // head_dim = 16 * HDT; BIASED: scores lose slope * distance
 __global__ __launch_bounds__(64 * kDecodeWaves) void attn_decode_mfma_kernel(
     const bf16_t* __restrict__ q, bf16_t* __restrict__ final_out, float* __restrict__ part,
     const bf16_t* __restrict__ cache,
@@ -287,7 +288,8 @@ __global__ __launch_bounds__(64 * kDecodeWaves) void attn_decode_mfma_kernel(
       bf16x4 o;
 #pragma unroll
       for (int i = 0; i < 4; ++i) o[i] = (bf16_t)(v[i] * inv * og[i]);
-      *reinterpret_cast<bf16x4*>(final_out + ((long)t * H + head_o) * hd + d4) = o;
+      *reinterpret_cast<bf16x4*>(final_out + (TILED ? rows_at(gate.side, t, head_o * hd + d4, H * hd)
+                                                     : ((long)t * H + head_o) * hd + d4)) = o;
     } else {
       float* out = part + (((long)t * H + head_o) * gridDim.z + blockIdx.z) * (hd + 2);   // 8-byte rows
       *reinterpret_cast<floatx2*>(out + d4) = floatx2{v[0], v[1]};
@@ -337,6 +339,20 @@ static int launch_decode(dim3 grid, hipStream_t stream, const void* q, void* out
       raised_kept = 1;
     }
     hipLaunchKernelGGL((attn_decode_mfma_kernel<HDT, W, false, true>), grid, dim3(64 * W), lds, stream,
+                       (const bf16_t*)q, (bf16_t*)out, part, (const bf16_t*)cache, positions, span_of_token,
+                       block_table, max_pages, page_size, H, KV, window, chunk, sinks, keep_first, scale, slopes, head_tiles, token_list, gate);
+    return 0;
+  }
+  if (W == decode_waves_whole(HDT) && grid.z == 1 && gate.side) {
+    static int raised_tiled = 0;
+    if (lds > 64 * 1024 && !raised_tiled) {
+      hipError_t e = hipFuncSetAttribute((const void*)attn_decode_mfma_kernel<HDT, W, false, false, W == decode_waves_whole(HDT)>,
+                                         hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         W * 16 * (16 * HDT + 4) * (int)sizeof(float));
+      if (e != hipSuccess) KLLM_FAIL((int)e, "attn_decode: cannot raise the LDS limit: %s", hipGetErrorString(e));
+      raised_tiled = 1;
+    }
+    hipLaunchKernelGGL((attn_decode_mfma_kernel<HDT, W, false, false, W == decode_waves_whole(HDT)>), grid, dim3(64 * W), lds, stream,
                        (const bf16_t*)q, (bf16_t*)out, part, (const bf16_t*)cache, positions, span_of_token,
                        block_table, max_pages, page_size, H, KV, window, chunk, sinks, keep_first, scale, slopes, head_tiles, token_list, gate);
     return 0;
@@ -449,6 +465,9 @@ static int attn_decode_run(const char* who, const void* q, void* out, float* par
                            int dtype, const int* token_list, int n_listed, const OutGate& gate, hipStream_t stream) {
   KLLM_REQUIRE(!gate.sums || (gate.nsplit >= 1 && gate.width > 0 && gate.width <= hd && gate.row >= (long)H * gate.width),
                "%s: a gate of %d columns a head for heads of %d, rows of %ld", who, gate.width, hd, gate.row);
+  KLLM_REQUIRE(!gate.side || (!slopes && keep_first == 0), "%s: tiled rows go without a distance bias and kept first positions", who);
+  KLLM_REQUIRE(!gate.side || (dtype == DT_BF16 && gate.side == (n < 16 ? n : 16) && (long)H * hd % 32 == 0),
+               "%s: an output with sides of %d rows, n=%d H=%d head_dim=%d", who, gate.side, n, H, hd);
   KLLM_REQUIRE(q && out && part && cache && positions && span_of_token && block_table,
                "%s: null pointer", who);
   KLLM_REQUIRE(dtype == DT_BF16 || dtype == DT_F32, "%s: unknown dtype %d", who, dtype);
@@ -515,8 +534,8 @@ extern "C" int kllm_attn_decode(const void* q, void* out, float* part, long part
                                 const int* block_table, int max_pages, int page_size, int n, int H,
                                 int KV, int hd, int window, int chunk, const float* sinks, int keep_first, float scale, const float* slopes,
                                 int nslices, int dtype, const int* token_list, int n_listed, const float* gate_sums,
-                                int gate_nsplit, long gate_stride, long gate_row, int gate_width, hipStream_t stream) {
-  const OutGate gate = {gate_sums, gate_nsplit, gate_width, gate_stride, gate_row};
+                                int gate_nsplit, long gate_stride, long gate_row, int gate_width, int out_side, hipStream_t stream) {
+  const OutGate gate = {gate_sums, gate_nsplit, gate_width, gate_stride, gate_row, out_side};
   return attn_decode_run("attn_decode", q, out, part, part_floats, cache, positions, span_of_token,
                          block_table, max_pages, page_size, n, H, KV, hd, window, chunk, sinks, keep_first, scale, slopes, nslices, dtype,
                          token_list, n_listed, gate, stream);

@@ -55,7 +55,7 @@ __device__ __forceinline__ void attn_merge_one(T* __restrict__ out, const float*
 #pragma unroll
   for (int v = 0; v < DV; ++v)
     if (lane + 64 * v < hd)
-      out[((long)t * H + h) * hd + lane + 64 * v] = from_f32<T>(o[v] / denom * out_gate(gate, t, h, lane + 64 * v));
+      out[rows_at(gate.side, t, h * hd + lane + 64 * v, H * hd)] = from_f32<T>(o[v] / denom * out_gate(gate, t, h, lane + 64 * v));
 }
 
 // The same for up to 64 slices and heads of up to 128 in one trip to memory instead of one per
@@ -95,7 +95,7 @@ __device__ __forceinline__ void attn_merge_wide(T* __restrict__ out, const float
 #pragma unroll
   for (int v = 0; v < DV; ++v)
     if (lane + 64 * v < hd)
-      out[((long)t * H + h) * hd + lane + 64 * v] = from_f32<T>(o[v] / denom * out_gate(gate, t, h, lane + 64 * v));
+      out[rows_at(gate.side, t, h * hd + lane + 64 * v, H * hd)] = from_f32<T>(o[v] / denom * out_gate(gate, t, h, lane + 64 * v));
 }
 
 template <typename T, int DV, int R>

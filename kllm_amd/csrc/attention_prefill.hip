@@ -460,7 +460,8 @@ __global__ __launch_bounds__(64 * kPrefillWaves * PAR) __attribute__((amdgpu_wav
     return;
   }
   const float inv = 1.f / l;                                  // finite: a query reads its own key
-  bf16_t* orow = out + ((long)tq * H + h) * hd;
+  const int side = gate.side ? gate.side : 1;                 // (eights of columns lie side times as far apart)
+  bf16_t* orow = out + rows_at(gate.side, tq, h * hd + 4 * g, H * hd);
 #pragma unroll
   for (int r = 0; r < HDT; ++r)
 #pragma unroll
@@ -469,7 +470,7 @@ __global__ __launch_bounds__(64 * kPrefillWaves * PAR) __attribute__((amdgpu_wav
       bf16x4 v;
 #pragma unroll
       for (int j = 0; j < 4; ++j) v[j] = (bf16_t)(acc[r][4 * b + j] * inv * og[j]);
-      *reinterpret_cast<bf16x4*>(orow + 32 * r + 8 * b + 4 * g) = v;
+      *reinterpret_cast<bf16x4*>(orow + (32 * r + 8 * b) * side) = v;
     }
 }
 
@@ -751,7 +752,8 @@ __global__ __launch_bounds__(64 * kPrefillWaves) __attribute__((amdgpu_waves_per
     l += ww[w] * red[(w * kRows + HDT * 16 + 1) * kWave + lane];
   }
   const float inv = 1.f / l;
-  bf16_t* orow = out + ((long)tq * H + h) * hd;
+  const int side = gate.side ? gate.side : 1;                 // (eights of columns lie side times as far apart)
+  bf16_t* orow = out + rows_at(gate.side, tq, h * hd + 4 * g, H * hd);
 #pragma unroll
   for (int r = 0; r < HDT; ++r)
 #pragma unroll
@@ -766,7 +768,7 @@ __global__ __launch_bounds__(64 * kPrefillWaves) __attribute__((amdgpu_waves_per
         for (int w = 0; w < kPrefillWaves - 1; ++w) o += ww[w] * red[(w * kRows + 16 * r + i) * kWave + lane];
         v[j] = (bf16_t)(o * inv * og[j]);
       }
-      *reinterpret_cast<bf16x4*>(orow + 32 * r + 8 * b + 4 * g) = v;
+      *reinterpret_cast<bf16x4*>(orow + (32 * r + 8 * b) * side) = v;
     }
 }
 
@@ -886,8 +888,10 @@ extern "C" int kllm_attn_prefill(const void* q, void* out, const void* cache, co
                                  const int* block_table, int max_pages, int page_size, int H, int KV,
                                  int hd, int window, int chunk, const float* sinks, int keep_first, float scale, const float* slopes, long keys_total, int keys_longest,
                                  float* part, long part_floats, int nslices, int n_rows, int dtype, const float* gate_sums, int gate_nsplit,
-                                 long gate_stride, long gate_row, int gate_width, hipStream_t stream) {
-  const OutGate gate = {gate_sums, gate_nsplit, gate_width, gate_stride, gate_row};
+                                 long gate_stride, long gate_row, int gate_width, int out_side, hipStream_t stream) {
+  const OutGate gate = {gate_sums, gate_nsplit, gate_width, gate_stride, gate_row, out_side};
+  KLLM_REQUIRE(!out_side || (dtype == DT_BF16 && n_rows > 0 && out_side == (n_rows < 16 ? n_rows : 16)),
+               "attn_prefill: an output with sides of %d rows, n_rows=%d", out_side, n_rows);
   KLLM_REQUIRE(!gate_sums || (gate_nsplit >= 1 && gate_width > 0 && gate_width <= hd && gate_row >= (long)H * gate_width),
                "attn_prefill: a gate of %d columns a head for heads of %d, rows of %ld", gate_width, hd, gate_row);
   KLLM_REQUIRE(q && out && cache && query_tiles && span_start && span_pos && block_table,

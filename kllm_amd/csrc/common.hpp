@@ -82,11 +82,22 @@ __device__ __forceinline__ float sigmoid_f32(float v) { return 1.f / (1.f + expf
 // function of a sum of its own, taken where the output is written.  `sums` (null: no gate) points to
 // the gate's first column of float32 sums [nsplit][tokens][row]; a head has `width` columns, and
 // elements beyond them (padding, zero anyway) are not gated.
+// `side`: how the output's rows are stored (see rows_at).
 struct OutGate {
   const float* sums;
   int nsplit, width;
   long split_stride, row;
+  int side;
 };
+
+// Element (row, col) of rows of `cols` columns: row by row (side 0), or in the order that the products of up to 64 rows read
+// them: [16 rows][32 columns][8 columns][side rows][8], side the lesser of 16 and the number of rows.  The row's place and the
+// column's add up; column 8 i + j of a row lies 8 i times the side further on.
+__device__ __forceinline__ long rows_base(int side, int row, int cols) {
+  return side ? (long)(row / 16) * cols * side + row % 16 * 8 : (long)row * cols;
+}
+__device__ __forceinline__ int rows_col(int side, int col) { return (col & ~7) * (side ? side : 1) + (col & 7); }
+__device__ __forceinline__ long rows_at(int side, int row, int col, int cols) { return rows_base(side, row, cols) + rows_col(side, col); }
 
 __device__ __forceinline__ float out_gate(const OutGate& g, long t, int h, int d) {
   if (!g.sums || d >= g.width) return 1.f;

@@ -249,13 +249,13 @@ int kllm_attn_decode_slices(int n, int KV, int H, int hd, int dtype, int max_key
 /* Whether the float32 attention on the matrix cores takes this head size and page size. */
 int kllm_attn_f32_fits(int hd, int page_size);
 /* `chunk`, `sinks`, `keep_first` and the gate in kllm_attn_decode and kllm_attn_prefill: as in kllm_attn_generic
- * (kept first positions: bfloat16 only). */
+ * (kept first positions: bfloat16 only).  out_side: 0, or min(rows of q, 16): the output as tiled rows (kllm_linear_rows). */
 int kllm_attn_decode(const void* q, void* out, float* part, long part_floats, const void* cache,
                      const int* positions, const int* span_of_token, const int* block_table,
                      int max_pages, int page_size, int n, int H, int KV, int hd, int window,
                      int chunk, const float* sinks, int keep_first, float scale, const float* slopes, int nslices, int dtype,
                      const int* token_list, int n_listed, const float* gate_sums, int gate_nsplit, long gate_stride,
-                     long gate_row, int gate_width, hipStream_t stream);
+                     long gate_row, int gate_width, int out_side, hipStream_t stream);
 
 /* kllm_attn_decode without a workspace argument and without any allocation: for callers
  * that cannot allocate device memory (code under HIP graph capture, tight serving loops,
@@ -290,7 +290,7 @@ int kllm_attn_prefill(const void* q, void* out, const void* cache, const int* qu
                       int window, int chunk, const float* sinks, int keep_first, float scale, const float* slopes, long keys_total,
                       int keys_longest, float* part, long part_floats, int nslices, int n_rows, int dtype,
                       const float* gate_sums, int gate_nsplit, long gate_stride, long gate_row, int gate_width,
-                      hipStream_t stream);
+                      int out_side, hipStream_t stream);
 /* nslices of kllm_attn_prefill: how many workgroups share out the keys of a block and head
  * (1: none; more where few blocks of a large head would leave CUs idle; taken only when
  * keys_longest says that the longest block reads 1,280 keys or more).  With more than one,

@@ -14,6 +14,10 @@
 // of X whole, so TW is what divides the traffic from L2.  Two workgroups may share a tile of W and take half of the rows each;
 // they sit on one XCD, so that the weights come from memory once.
 //
+// Rows that go from one such product to the next are stored in the order its lanes read (rows_at): a load is then one contiguous
+// kilobyte, or less where there are fewer rows than 16.  From rows as they are, its sixteen lanes with one K lie in sixteen
+// rows, and a CU takes in 16 bytes a clock (64 rows of 5,632 against 2,048 columns: 15.8 -> 12.1 us; 16 rows 11.2 -> 10.1).
+//
 // Alone in a replayed graph, 8 / 64 rows, us: 2,048 x 2,048 4.6 / 7.2 (rows as attention leaves them); 2,048 x 5,632 9.9 / 12.2; 2 x
 // 5,632 x 2,048 11.0 / 14.5; 2,560 x 2,048 4.6 / 6.8; 4,096 x 14,336 23.4 / 41.0 (117 MB: 5.0 TB/s at 8 rows).  A decode step at
 // 1.1B sizes and contexts of 600, with fused_linear.hip's products and the tiles' and with these: 1 token 914 -> 888 us, 8 971
@@ -31,16 +35,6 @@ typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 constexpr int LR_ROWS = 64;             // rows of X at most
 constexpr int LR_LD = 20;               // floats from one x row of a partial tile to the next: 16 and padding, whole 16 bytes
 constexpr int LR_TILE = 16 * LR_LD;
-
-// Element (row, column) of n rows of `cols` columns that go out in the lanes' order (out.y_tiled): [16 rows][32 columns][8
-// columns][row], so that a load of the next product's is one contiguous kilobyte, or less where there are fewer rows than 16.  From rows as
-// they are, its sixteen lanes with one K lie in sixteen rows, and a CU takes in 16 bytes a clock (64 rows of 5,632
-// against 2,048 columns: 15.8 -> 12.1 us; 16 rows 11.2 -> 10.1).
-__device__ __forceinline__ long lr_at(const FlOut& out, int row, int col, int n, int cols) {
-  if (!out.y_tiled) return (long)row * cols + col;
-  const int side = min(n, 16);
-  return (((long)(row / 16) * (cols / 32) + col / 32) * 4 + col % 32 / 8) * (8 * side) + row % 16 * 8 + col % 8;
-}
 
 // Steps of K in each of the two buffers a wave fills in turn: what 128 registers hold, four at most.
 constexpr int lr_ahead(int nt, int tw) { return nt + tw <= 4 ? 4 : nt + tw == 5 ? 3 : 2; }
@@ -213,7 +207,7 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __re
       if (live) {
         x = res_old[u] + sum_of(0, r / 16, r % 16, tid % 16);
         out.resid[(long)xr * m + col] = x;
-        reinterpret_cast<bf16_t*>(out.y)[lr_at(out, xr, col, n, m)] = from_f32<bf16_t>(x * res_w);
+        reinterpret_cast<bf16_t*>(out.y)[rows_at(out.y_tiled ? min(n, 16) : 0, xr, col, m)] = from_f32<bf16_t>(x * res_w);
       }
       const float ss = parts_sum<16>(x * x);
       if (tid % 16 == 0 && r < 16 * NT && xr < n) out.ss_out[(long)xr * stride + group] = ss;
@@ -233,7 +227,7 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __re
         b *= row_scale[r];
       }
       if (EP == FL_SWIGLU) {
-        reinterpret_cast<bf16_t*>(out.y)[lr_at(out, xr, pair, n, pairs)] = from_f32<bf16_t>(gate_act(a, out.act) * b);
+        reinterpret_cast<bf16_t*>(out.y)[rows_at(out.y_tiled ? min(n, 16) : 0, xr, pair, pairs)] = from_f32<bf16_t>(gate_act(a, out.act) * b);
       } else {
         const int e = EP == FL_ROPE ? u : 0;
         fl_rope_store<bf16_t>(out, xr, pair, a, b, ep_cos[e], ep_sin[e], ep_page[e], out.cache ? ep_pos[e] % out.page_size : 0);

@@ -21,7 +21,7 @@ import torch
 DT_F32, DT_BF16 = 0, 1
 GEMM_PLAIN, GEMM_TILED_F32, GEMM_MFMA_BF16, GEMM_SKINNY_BF16, GEMM_GEMV, GEMM_GEMV_LDS, GEMM_MFMA_F32 = 0, 1, 2, 3, 4, 5, 6
 GEMV_BEST_ROWS = 0         # rows up to which they beat the MFMA kernels in bfloat16: none (a step at 1.1B sizes, one token: 1.036 against 0.963 ms)
-ABI_VERSION = 19
+ABI_VERSION = 20
 
 
 class KernelError(RuntimeError):
@@ -139,8 +139,8 @@ def _declare(lib):
         "kllm_calibrate_read": [P, L, P, P],
         "kllm_calibrate_read_workgroups": [],
         "kllm_calibrate_mfma": [I, I, P, P, P],
-        "kllm_attn_decode": [P, P, P, L, P, P, P, P, I, I, I, I, I, I, I, I, P, I, F, P, I, I, P, I, P, I, L, L, I, P],
-        "kllm_attn_prefill": [P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, P, I, F, P, L, I, P, L, I, I, I, P, I, L, L, I, P],
+        "kllm_attn_decode": [P, P, P, L, P, P, P, P, I, I, I, I, I, I, I, I, P, I, F, P, I, I, P, I, P, I, L, L, I, I, P],
+        "kllm_attn_prefill": [P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, P, I, F, P, L, I, P, L, I, I, I, P, I, L, L, I, I, P],
         "kllm_attn_prefill_slices": [I, I, I],
         "kllm_gemm_act": [P, P, P, I, I, I, I, I, P, P],
         "kllm_add_sinusoid": [P, P, I, I, D, P],
@@ -1264,10 +1264,20 @@ def attn_prefill_slices(n_tiles, n_heads, head_dim, dtype=torch.bfloat16) -> int
     return int(library().kllm_attn_prefill_slices(int(n_tiles), int(n_heads), int(head_dim)))
 
 
+def _rows_side(out, who):
+    """(``out_side`` of the call, its tensor) for an output that may be ``TiledRows``."""
+    if not isinstance(out, TiledRows):
+        return 0, out
+    n, cols = out.shape
+    if cols % 32 or out.data.shape[0] != TiledRows.stored(n) or not out.data.is_contiguous():
+        raise KernelError(f"{who}: tiled rows {out.shape} do not fit")
+    return min(n, 16), out.data
+
+
 def attn_prefill(q, out, cache, query_tiles, n_tiles, span_start, span_pos, block_table, page_size,
                  n_heads, n_kv_heads, head_dim, window, scale, keys_total=0, keys_longest=0, part=None,
                  nslices=None, slopes=None, chunk=0, sink=False, keep_first=0, gate=None):
-    """query_tiles [n_tiles, 2] int32: (first token row, span) of each block of up to
+    """(``out`` may be ``TiledRows``, in bfloat16.)  query_tiles [n_tiles, 2] int32: (first token row, span) of each block of up to
     PREFILL_QUERY_BLOCK consecutive tokens of one span.  ``keys_total`` and
     ``keys_longest``: how many keys the blocks read, all together and the longest block
     alone, if the caller knows (the kernel is chosen by them).  ``part``: float32 room for the
@@ -1285,6 +1295,7 @@ def attn_prefill(q, out, cache, query_tiles, n_tiles, span_start, span_pos, bloc
     if (tuple(q.shape) != (n, n_heads * head_dim) or tuple(out.shape) != tuple(q.shape)
             or q.dtype != cache.dtype or out.dtype != q.dtype):
         raise KernelError("attn_prefill: q/out shapes or dtypes do not fit")
+    side, out = _rows_side(out, "attn_prefill")
     if tuple(cache.shape[1:]) != (2, n_kv_heads, page_size * head_dim):
         raise KernelError(f"attn_prefill: cache {tuple(cache.shape)} does not fit")
     if query_tiles.numel() < 2 * n_tiles:
@@ -1298,7 +1309,7 @@ def attn_prefill(q, out, cache, query_tiles, n_tiles, span_start, span_pos, bloc
         keys_total if type(keys_total) is StepValue else int(keys_total),
         keys_longest if type(keys_longest) is StepValue else int(keys_longest),
         _ptr(part, "attn part", torch.float32, True) if nslices > 1 else 0, need, nslices, n,
-        dtype_code(q.dtype), *_out_gate(gate, n, n_heads, head_dim, "attn_prefill"), _stream())
+        dtype_code(q.dtype), *_out_gate(gate, n, n_heads, head_dim, "attn_prefill"), side, _stream())
 
 
 def attn_decode(q, out, part, cache, positions, span_of_token, block_table, page_size, n_heads,
@@ -1308,6 +1319,7 @@ def attn_decode(q, out, part, cache, positions, span_of_token, block_table, page
     if (tuple(q.shape) != (n, n_heads * head_dim) or tuple(out.shape) != tuple(q.shape)
             or q.dtype != cache.dtype or out.dtype != q.dtype):
         raise KernelError("attn_decode: q/out shapes or dtypes do not fit")
+    side, out = _rows_side(out, "attn_decode")
     if tuple(cache.shape[1:]) != (2, n_kv_heads, page_size * head_dim):
         raise KernelError(f"attn_decode: cache {tuple(cache.shape)} does not fit")
     if positions.numel() < n or span_of_token.numel() < n:
@@ -1320,7 +1332,7 @@ def attn_decode(q, out, part, cache, positions, span_of_token, block_table, page
         int(keep_first), float(scale), _slopes(slopes, n_heads, "attn_decode"),
         int(nslices), dtype_code(q.dtype),
         _ptr(token_list, "attn token_list", torch.int32, True), int(n_listed),
-        *_out_gate(gate, n, n_heads, head_dim, "attn_decode"), _stream())
+        *_out_gate(gate, n, n_heads, head_dim, "attn_decode"), side, _stream())
 
 
 def sample(out, logits, temperature=None, uniform=None):

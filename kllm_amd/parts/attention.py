@@ -30,7 +30,7 @@ import torch
 
 from .. import kernels as K
 from .base import Normed, Part, register_part
-from .linear import decode_linear, fused_f32, linear, linear_into, rows_kernel, tiled_copy
+from .linear import decode_linear, fused_f32, linear, linear_into, rows_kernel, sink_takes_rows, tiled_copy
 from .spec import CacheNeed, WeightSpec
 
 
@@ -252,13 +252,31 @@ class CausalSelfAttention(Part):
             K.rope_append(qkv, q, cos, sin, pages, ctx.positions, ctx.span_of_token,
                           cache.block_table, cache.page_size, self.heads, self.kv_heads,
                           self.head_dim, self.rotary_dim, self.interleaved)
-        out = ctx.buf("attn.out", (n, self.q_dim), dtype)
+        if (self.q_dim % 32 == 0 and self.slopes is None and not self.keep_first and self._fast(dtype, cache.page_size)[0]
+                and sink_takes_rows(self.runtime, sink, n, self.w_o, self._tiled.get("o"))):
+            out = K.TiledRows(ctx.buf("attn.out", (K.TiledRows.stored(n), self.q_dim), dtype), n)
+        else:
+            out = ctx.buf("attn.out", (n, self.q_dim), dtype)
         self.attend(ctx, q, out, cache)
         if sink is not None:
             normed = linear_into(ctx, out, self.w_o, sink, "attn.proj", w_tiled=self._tiled.get("o"))
             if normed is not None:
                 return normed
         return linear(ctx, out, self.w_o, "attn.proj")
+
+    def _fast(self, dtype, page_size):
+        """Whether attention runs on the matrix cores: decode tokens, prompts."""
+        if dtype == torch.bfloat16:
+            fast = page_size % 16 == 0 and self.head_dim in K.DECODE_HEAD_DIMS
+            prompt_ok = self.head_dim in K.PREFILL_HEAD_DIMS
+        else:
+            fast = prompt_ok = K.attn_f32_fits(self.head_dim, page_size)
+        # the kernels on the matrix cores take keys and values of one width; the 32-bit ones one run of
+        # keys a query (no kept first positions)
+        fast = (fast and self.runtime.options.get("attention", "auto") != "generic" and self.value_dim == self.head_dim
+                and not self.FAST_KERNELS_OFF
+                and not (self.keep_first and (dtype != torch.bfloat16 or self.slopes is not None)))
+        return fast, prompt_ok
 
     def attend(self, ctx, q, out, cache, gate=None):
         """Choose the attention kernels by the spans' lengths: tokens of short
@@ -267,16 +285,7 @@ class CausalSelfAttention(Part):
         (both on the matrix cores, in bfloat16 or with 32-bit operands); sizes
         those kernels do not take go to the kernel that takes every size.  ``gate``
         (``K.Columns`` of sums): its logistic function multiplies the output."""
-        mode = self.runtime.options.get("attention", "auto")
-        if q.dtype == torch.bfloat16:
-            fast = cache.page_size % 16 == 0 and self.head_dim in K.DECODE_HEAD_DIMS
-            prompt_ok = self.head_dim in K.PREFILL_HEAD_DIMS
-        else:
-            fast = prompt_ok = K.attn_f32_fits(self.head_dim, cache.page_size)
-        # the kernels on the matrix cores take keys and values of one width; the 32-bit ones one run of
-        # keys a query (no kept first positions)
-        fast = (fast and mode != "generic" and self.value_dim == self.head_dim and not self.FAST_KERNELS_OFF
-                and not (self.keep_first and (q.dtype != torch.bfloat16 or self.slopes is not None)))
+        fast, prompt_ok = self._fast(q.dtype, cache.page_size)
         if not fast:
             K.attn_generic(q, out, cache.pages, ctx.positions, ctx.span_of_token, cache.block_table,
                            cache.page_size, self.heads, self.kv_heads, self.head_dim, self.window,

@@ -81,7 +81,7 @@ class GatedFeedForward(Part):
                   else xn.scaled_rows() if xn.xw is not None and (rows or fused and not isinstance(xn.xw, K.TiledRows))
                   else xn.materialize(ctx))
         if rows and sink_takes_rows(self.runtime, sink, n, self.w_down, self._tiled.get("down")):
-            h = K.TiledRows(ctx.buf("ffn.ht", (K.TiledRows.stored(n), self.intermediate), dtype), n)
+            h = K.TiledRows(ctx.buf("ffn.h", (K.TiledRows.stored(n), self.intermediate), dtype), n)
         else:
             h = ctx.buf("ffn.h", (n, self.intermediate), dtype)
         if gemv:

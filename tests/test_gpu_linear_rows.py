@@ -133,3 +133,46 @@ def test_refusals():
     with pytest.raises(k_.KernelError, match="not built"):
         k_.linear_rows(k_.fused_linear_tile(w, k_.LINEAR_PARTS), torch.empty(1, 20, 64, device=DEV), k_.LINEAR_PARTS,
                        _bf(20, 96, seed=2, scale=1.0))
+
+
+def _rowwise(t):
+    """TiledRows as plain rows."""
+    n, k = t.shape
+    side = min(n, 16)
+    v = t.data.reshape(-1, k // 32, 4, side, 8)[: -(-n // 16)]
+    return v.permute(0, 3, 1, 2, 4).reshape(-1, k)[:n]
+
+
+@pytest.mark.parametrize("H,KV,hd,ps", [(8, 2, 16, 16), (32, 4, 64, 16), (6, 6, 128, 32)])
+@pytest.mark.parametrize("slices", [1, 4, 33])
+def test_attention_writes_tiled_rows(H, KV, hd, ps, slices):
+    """Decode attention (one workgroup and merged slices) and prompt attention write the same numbers in the
+    order that the output projection's lanes read."""
+    k_ = K()
+    for spans in ([(9, 1), (70, 1), (300, 1)], [(5, 1)] * 16, [(0, 37), (130, 3)]):
+        n = sum(l for _, l in spans)
+        pages = [-(-(p0 + l) // ps) for p0, l in spans]
+        bt = torch.zeros(len(spans), max(pages), dtype=torch.int32)
+        at = 0
+        for i, c in enumerate(pages):
+            bt[i, :c] = torch.arange(at, at + c)
+            at += c
+        bt = bt.to(DEV)
+        cache, q = _bf(at, 2, KV, ps * hd, seed=1, scale=1.0), _bf(n, H * hd, seed=2, scale=1.0)
+        pos = torch.tensor([p0 + i for p0, l in spans for i in range(l)], dtype=torch.int32, device=DEV)
+        sot = torch.tensor([s for s, (_, l) in enumerate(spans) for _ in range(l)], dtype=torch.int32, device=DEV)
+        part = torch.empty(n * H * slices * (hd + 2), device=DEV)
+        out = torch.empty(n, H * hd, dtype=torch.bfloat16, device=DEV)
+        tiled = k_.TiledRows(torch.zeros(k_.TiledRows.stored(n), H * hd, dtype=torch.bfloat16, device=DEV), n)
+        for o in (out, tiled):
+            k_.attn_decode(q, o, part, cache, pos, sot, bt, ps, H, KV, hd, 0, hd ** -0.5, slices)
+        assert torch.equal(_rowwise(tiled), out)
+        if hd in k_.PREFILL_HEAD_DIMS and slices == 1:
+            start = torch.tensor([0] + torch.tensor([l for _, l in spans]).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
+            tiles = torch.tensor([[int(start[s]), s] for s in range(len(spans))], dtype=torch.int32, device=DEV)
+            span_pos = torch.tensor([p0 for p0, _ in spans], dtype=torch.int32, device=DEV)
+            for keys in (0, 10 ** 6):            # both kernels
+                for o in (out, tiled):
+                    k_.attn_prefill(q, o, cache, tiles, len(spans), start, span_pos, bt, ps, H, KV, hd, 0, hd ** -0.5,
+                                    keys, keys)
+                assert torch.equal(_rowwise(tiled), out)
