@@ -195,11 +195,11 @@ typedef struct {
 } KllmLinearOut;
 long kllm_fused_linear_lds_bytes(int n, int k, int nsplit, int dtype);
 /* The RESID, SWIGLU and ROPE products of 17 to 64 rows (any n up to 64 is taken), bfloat16, K a multiple of 32,
- * w the tiled copy.  RESID leaves kllm_linear_rows_parts(m) sums of squares a row (0: m is not taken).  Tiled rows
+ * w the tiled copy.  RESID leaves kllm_linear_rows_parts(n, m, k) sums of squares a row (0: the sizes are not taken).  Tiled rows
  * (y_tiled, x_tiled; columns a multiple of 32): [row / 16][column / 32][column % 32 / 8][row % 16][8]; with more than 16 rows
  * those up to the next multiple of 16 are there and hold anything, with fewer only the rows are. */
 int kllm_linear_rows(const void* x, int x_stride, const KllmLinearOut* y, const void* w, int n, int m, int k, hipStream_t stream);
-int kllm_linear_rows_parts(int m);
+int kllm_linear_rows_parts(int n, int m, int k);
 /* Where that is more than LDS holds, the rows are staged and multiplied in passes over K, with
  * one tile to a workgroup (tiles_per_wg = 1): how many passes a call needs (1: all at once; 0:
  * the kernel does not take the sizes). */

@@ -39,7 +39,12 @@ constexpr int LR_TILE = 16 * LR_LD;
 // Steps of K in each of the two buffers a wave fills in turn: what 128 registers hold, four at most.
 constexpr int lr_ahead(int nt, int tw) { return nt + tw <= 4 ? 4 : nt + tw == 5 ? 3 : 2; }
 
-template <int NT, int TW, int EP, bool SCALED, int NW>
+// SPLIT (FL_RESID, up to 16 rows): a workgroup takes eight rows of W, each twice in a matrix instruction: K's first half in its rows
+// 0-7, the second half in rows 8-15, so that a load still brings a kilobyte.  Up to eight rows of X lie in the operand's columns the
+// same way (NT 1); more take an instruction for each half of K (NT 2).  What pairs a half with the other's X is not used.  A CU streams
+// about 20 GB/s of weights from memory whatever a workgroup has in flight, so a product on half the CUs takes half as long again:
+// a step at 1.1B sizes, 1 / 8 / 16 tokens 894 / 939 / 1,032 us without, 882 / 920 / 1,026 with.
+template <int NT, int TW, int EP, bool SCALED, int NW, bool SPLIT>
 __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __restrict__ X, FlOut out,
                                                               const bf16_t* __restrict__ W, int n, int m, int k, int tiles,
                                                               int halves, int x_stride) {
@@ -51,19 +56,23 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __re
   const int g = lane / 16, c = lane % 16;
   const int groups = (tiles + TW - 1) / TW;                      // workgroups side by side over W
   // Blocks go to the XCDs in turn: two workgroups of one group of tiles are eight blocks apart.
-  const int group = halves == 1 ? (int)blockIdx.x : (int)(blockIdx.x / 16) * 8 + (int)(blockIdx.x % 8);
+  const int group = SPLIT ? (int)blockIdx.x / 2
+                    : halves == 1 ? (int)blockIdx.x : (int)(blockIdx.x / 16) * 8 + (int)(blockIdx.x % 8);
+  const int half_tile = SPLIT ? (int)blockIdx.x % 2 : 0;         // which eight rows of W
   const int row0 = halves == 1 ? 0 : (int)(blockIdx.x / 8 % 2) * (16 * NT);
   if (group >= groups || row0 >= n) return;                      // the whole workgroup
   const int steps = k / 32;                                      // (k is a multiple of 32)
-  const int per = (steps + NW - 1) / NW;
-  const int s_beg = min(wave * per, steps);
-  const int mine = min(per, steps - s_beg);                      // steps of this wave, possibly none
+  const int walk = SPLIT ? steps / 2 : steps;                    // steps that the waves share
+  const int per = (walk + NW - 1) / NW;
+  const int s_beg = min(wave * per, walk);
+  const int mine = min(per, walk - s_beg);                       // steps of this wave, possibly none
 
   // ---- what the epilogue needs is asked for first (loads return in order): the rotation's page and
   // slot, the residual stream's old values
   const int half = EP == FL_ROPE ? out.hd / 2 : 1;
-  constexpr int RR = 4 * NW;                               // rows that the threads take at a time, sixteen to a row
-  constexpr int RU = (16 * NT + RR - 1) / RR;                    // turns
+  constexpr int RC = SPLIT ? 8 : 16;                             // columns of a workgroup's output tile, and threads to a row
+  constexpr int RR = 64 * NW / RC;                               // rows that the threads take at a time
+  constexpr int RU = ((SPLIT ? 16 : 16 * NT) + RR - 1) / RR;                    // turns
   constexpr int PU = EP == FL_ROPE ? (16 * NT + 2 * RR - 1) / (2 * RR) : 1;
   int ep_pos[PU], ep_span[PU], ep_page[PU];
   float ep_cos[PU], ep_sin[PU], res_old[RU], res_w = 0.f;
@@ -79,11 +88,11 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __re
       ep_sin[u] = turns ? out.sin_t[(long)xr * half + pair % half] : 0.f;
     }
   }
-  if (EP == FL_RESID) {        // thread (w row tid % 16, x row tid / 16 and RR on)
-    const int col = min(group * 16 + tid % 16, m - 1);
+  if (EP == FL_RESID) {        // thread (w row tid % RC, x row tid / RC and RR on)
+    const int col = min(group * 16 + 8 * half_tile + tid % RC, m - 1);
     res_w = out.norm_w[col];
 #pragma unroll
-    for (int u = 0; u < RU; ++u) res_old[u] = out.resid[(long)min(row0 + tid / 16 + RR * u, n - 1) * m + col];
+    for (int u = 0; u < RU; ++u) res_old[u] = out.resid[(long)min(row0 + tid / RC + RR * u, n - 1) * m + col];
   }
   constexpr int SU = RU;
   floatx4 ssv[SCALED ? SU : 1][FL_SS_LOADS];
@@ -116,14 +125,24 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __re
   for (int t = 0; t < NT; ++t)
     xo[t] = out.x_tiled ? min(row0 / 16 + t, row_tiles - 1) * steps * x_step + (g * side + min(c, side - 1)) * 16
                         : 2 * (min(row0 + t * 16 + c, n - 1) * x_stride + 8 * g);
-  const int s_last = min(s_beg + max(mine, 1), steps) - 1;
+  int wl = lane * 16;                                            // this lane's place in a step of W
+  if (SPLIT) {
+    const int later = c < 8 ? 0 : walk;                          // steps on, for the lanes of the second half of K
+    wl = later * 1024 + (16 * g + 8 * half_tile + c % 8) * 16;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int row = min(NT == 1 ? c % 8 : c, n - 1);
+      xo[t] = (NT == 1 ? later : t * walk) * x_step + (out.x_tiled ? (g * side + row) * 16 : 2 * (row * x_stride + 8 * g));
+    }
+  }
+  const int s_last = min(s_beg + max(mine, 1), walk) - 1;
   auto fill = [&](uintx4 (&wb)[A][TW], uintx4 (&xb)[A][NT], int s0) {
 #pragma unroll
     for (int i = 0; i < A; ++i) {
       const int s = min(s_beg + s0 + i, s_last);
 #pragma unroll
       for (int j = 0; j < TW; ++j)
-        wb[i][j] = __builtin_amdgcn_raw_buffer_load_b128(wr, lane * 16, wo[j] + s * 1024, 0);
+        wb[i][j] = __builtin_amdgcn_raw_buffer_load_b128(wr, wl, wo[j] + s * 1024, 0);
 #pragma unroll
       for (int t = 0; t < NT; ++t)
         xb[i][t] = __builtin_amdgcn_raw_buffer_load_b128(xr_, xo[t], s * x_step, 0);
@@ -194,23 +213,28 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __re
   auto sum_of = [&](int j, int t, int xc, int r) {               // in a fixed order
     float v = 0.f;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) v += part[((w * TW + j) * NT + t) * LR_TILE + xc * LR_LD + r];
+    for (int w = 0; w < NW; ++w) {
+      const float* of = part + ((w * TW + j) * NT + t) * LR_TILE + xc * LR_LD + r;
+      v += of[0];
+      if (SPLIT) v += NT == 1 ? of[8 * LR_LD + 8] : of[LR_TILE + 8];       // the second half of K
+    }
     return v;
   };
   if (EP == FL_RESID) {
-    const int col = group * 16 + tid % 16, stride = (groups + 3) / 4 * 4;
+    const int col = group * 16 + 8 * half_tile + tid % RC;
+    const int parts = SPLIT ? 2 * groups : groups, stride = (parts + 3) / 4 * 4;
 #pragma unroll
     for (int u = 0; u < RU; ++u) {
-      const int r = tid / 16 + RR * u, xr = row0 + r;
+      const int r = tid / RC + RR * u, xr = row0 + r;
       const bool live = r < 16 * NT && xr < n && col < m;
       float x = 0.f;
       if (live) {
-        x = res_old[u] + sum_of(0, r / 16, r % 16, tid % 16);
+        x = res_old[u] + sum_of(0, SPLIT ? 0 : r / 16, r % 16, tid % RC);
         out.resid[(long)xr * m + col] = x;
         reinterpret_cast<bf16_t*>(out.y)[rows_at(out.y_tiled ? min(n, 16) : 0, xr, col, m)] = from_f32<bf16_t>(x * res_w);
       }
-      const float ss = parts_sum<16>(x * x);
-      if (tid % 16 == 0 && r < 16 * NT && xr < n) out.ss_out[(long)xr * stride + group] = ss;
+      const float ss = parts_sum<RC>(x * x);
+      if (tid % RC == 0 && r < 16 * NT && xr < n) out.ss_out[(long)xr * stride + (SPLIT ? (int)blockIdx.x : group)] = ss;
     }
     return;
   }
@@ -245,18 +269,18 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __re
 
 static size_t lr_lds_bytes(int nt, int tw, int nw) { return (size_t)(nw * tw * nt * LR_TILE + LR_ROWS) * sizeof(float); }
 
-template <int NT, int TW, int EP, bool SCALED, int NW>
+template <int NT, int TW, int EP, bool SCALED, int NW, bool SPLIT = false>
 static int lr_launch_waves(const void* x, const FlOut& out, const void* w, int n, int m, int k, int tiles, int halves,
                      int x_stride, hipStream_t stream) {
   const size_t lds = lr_lds_bytes(NT, TW, NW);
   if (lds > 64 * 1024) {
-    static const hipError_t e = hipFuncSetAttribute((const void*)linear_rows_kernel<NT, TW, EP, SCALED, NW>,
+    static const hipError_t e = hipFuncSetAttribute((const void*)linear_rows_kernel<NT, TW, EP, SCALED, NW, SPLIT>,
                                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     if (e != hipSuccess) KLLM_FAIL((int)e, "linear_rows: cannot raise the LDS limit: %s", hipGetErrorString(e));
   }
   const int groups = ceil_div(tiles, TW);
-  const int blocks = halves == 1 ? groups : ceil_div(groups, 8) * 16;
-  hipLaunchKernelGGL((linear_rows_kernel<NT, TW, EP, SCALED, NW>), dim3(blocks), dim3(64 * NW), lds, stream,
+  const int blocks = SPLIT ? 2 * groups : halves == 1 ? groups : ceil_div(groups, 8) * 16;
+  hipLaunchKernelGGL((linear_rows_kernel<NT, TW, EP, SCALED, NW, SPLIT>), dim3(blocks), dim3(64 * NW), lds, stream,
                      (const bf16_t*)x, out, (const bf16_t*)w, n, m, k, tiles, halves, x_stride);
   return 0;
 }
@@ -300,7 +324,14 @@ using namespace kllm;
 
 static int lr_tiles(int kind, int m) { return kind == FL_RESID ? ceil_div(m, 16) : ceil_div(m / 2, 8); }
 
-extern "C" int kllm_linear_rows_parts(int m) { return m > 0 && lr_tiles(FL_RESID, m) <= FL_SS_MAX ? lr_tiles(FL_RESID, m) : 0; }
+// Whether a residual product takes eight rows of W a workgroup (SPLIT): up to 16 rows of X and no more tiles than half the CUs.
+static bool lr_split(int n, int m, int k) { return n <= 16 && k % 64 == 0 && 2 * lr_tiles(FL_RESID, m) <= device_cus(); }
+
+extern "C" int kllm_linear_rows_parts(int n, int m, int k) {
+  if (n <= 0 || m <= 0 || k <= 0) return 0;
+  const int parts = lr_split(n, m, k) ? 2 * lr_tiles(FL_RESID, m) : lr_tiles(FL_RESID, m);
+  return parts <= FL_SS_MAX ? parts : 0;
+}
 
 extern "C" int kllm_linear_rows(const void* x, int x_stride, const KllmLinearOut* yout, const void* w, int n, int m, int k,
                                 hipStream_t stream) {
@@ -338,7 +369,7 @@ extern "C" int kllm_linear_rows(const void* x, int x_stride, const KllmLinearOut
   if (ep == FL_RESID) {
     KLLM_REQUIRE(yout->resid && yout->norm_w && yout->ss_out, "linear_rows: the residual epilogue needs the stream, "
                  "the norm's weight and room for the sums of squares");
-    KLLM_REQUIRE(kllm_linear_rows_parts(m) > 0, "linear_rows: %d columns leave more than %d sums of squares per row", m,
+    KLLM_REQUIRE(kllm_linear_rows_parts(n, m, k) > 0, "linear_rows: %d columns leave more than %d sums of squares per row", m,
                  FL_SS_MAX);
     out.resid = yout->resid;
     out.norm_w = yout->norm_w;
@@ -381,7 +412,10 @@ extern "C" int kllm_linear_rows(const void* x, int x_stride, const KllmLinearOut
   const int whole = ceil_div(tiles, cus) * row_tiles, halved = ceil_div(2L * tiles, cus) * ceil_div(row_tiles, 2);
   const int halves = ep != FL_SWIGLU && (halved < whole || (halved == whole && tiles > cus)) ? 2 : 1;
   const int nt = ceil_div(row_tiles, halves);
-  const int rc = nt == 1 ? lr_launch_tw<1>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream)
+  const int rc = ep == FL_RESID && lr_split(n, m, k)
+                     ? (n <= 8 ? lr_launch_waves<1, 1, FL_RESID, false, 8, true>(x, out, w, n, m, k, tiles, 1, x_stride, stream)
+                               : lr_launch_waves<2, 1, FL_RESID, false, 8, true>(x, out, w, n, m, k, tiles, 1, x_stride, stream))
+               : nt == 1 ? lr_launch_tw<1>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream)
                : nt == 2 ? lr_launch_tw<2>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream)
                : nt == 3 ? lr_launch_tw<3>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream)
                          : lr_launch_tw<4>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream);

@@ -107,7 +107,7 @@ def _declare(lib):
         "kllm_fused_linear": [P, I, P, P, I, I, I, I, P],
         "kllm_fused_linear_resid_parts": [I, I],
         "kllm_linear_rows": [P, I, P, P, I, I, I, P],
-        "kllm_linear_rows_parts": [I],
+        "kllm_linear_rows_parts": [I, I, I],
         "kllm_fused_linear_passes": [I, I, I, I],
         "kllm_fused_linear_tile": [P, P, I, I, I, I, I, I, I, I, P],
         "kllm_command_op": [c_char_p],
@@ -988,6 +988,12 @@ class TiledRows:
         return self.data.dtype
 
 
+@functools.lru_cache(maxsize=4096)
+def linear_rows_parts(n, m, k) -> int:
+    """Partial sums of squares per row that a LINEAR_RESID product on ``linear_rows`` leaves, or 0 where it takes none such."""
+    return int(library().kllm_linear_rows_parts(int(n), int(m), int(k)))
+
+
 LINEAR_ROWS_MAX = 64
 LINEAR_ROWS_BYTES = 380_000
 
@@ -1004,7 +1010,7 @@ def linear_rows_best(kind, n, m, k, dtype=torch.bfloat16, tiled_x=True) -> bool:
     4,902 against 6,146)."""
     if dtype != torch.bfloat16 or not 1 <= n <= LINEAR_ROWS_MAX or k % 32 or k > 1 << 20:
         return False
-    if kind == LINEAR_RESID and library().kllm_linear_rows_parts(int(m)) == 0:
+    if kind == LINEAR_RESID and linear_rows_parts(n, m, k) == 0:
         return False
     if n <= 16:
         return True
@@ -1080,7 +1086,7 @@ def fused_linear(w, y, kind, x, nsplit=1, tiles_per_wg=1, rope=None, act=ACT_SIL
         want, dt = (nsplit, n, m), torch.float32
     elif kind == LINEAR_RESID:
         want, dt = (n, m), typ
-        parts = library().kllm_fused_linear_resid_parts(int(m), int(tiles_per_wg))
+        parts = linear_rows_parts(n, m, k) if _rows else library().kllm_fused_linear_resid_parts(int(m), int(tiles_per_wg))
         if (resid is None or norm_weight is None or ss_out is None or tuple(resid.shape) != (n, m)
                 or norm_weight.numel() != m or tuple(ss_out.shape) != (n, -(-parts // 4) * 4)):
             raise KernelError(f"fused_linear: the residual epilogue needs resid [{n}, {m}], the norm's weight [{m}] "

@@ -242,8 +242,9 @@ def linear_into(ctx, x, w, sink, tag, w_tiled=None):
         K.linear_resid(x, w, sink.x, ss)
         return Normed(sink.x, ss, parts, norm)
     if _resid_rows(rt, norm, n, w, w_tiled, isinstance(x, K.TiledRows)):
-        parts = -(-m // 16)
-        ss = ctx.buf(tag + ".ss", (n, -(-parts // 4) * 4), torch.float32)
+        parts = K.linear_rows_parts(n, m, k)
+        stride = -(-parts // 4) * 4          # (room for eight columns to a sum whatever n is: a smaller step must not ask for more)
+        ss = ctx.buf(tag + ".ss", (n * max(stride, -(-m // 32) * 4),), torch.float32)[:n * stride].view(n, stride)
         if _feeds_rows(norm, n):
             xw = K.TiledRows(ctx.buf(tag + ".xw", (K.TiledRows.stored(n), m), x.dtype), n)     # for the product behind the norm
         else:

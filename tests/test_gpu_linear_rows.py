@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 # Tiles of W at most half the CUs: two workgroups share the rows (2,048 and below); more: one (4,096).
-@pytest.mark.parametrize("n,m,k", [(1, 16, 32), (17, 48, 96), (5, 64, 2048), (8, 2048, 5632), (33, 72, 288), (45, 2048, 2048), (48, 100, 5632),
+@pytest.mark.parametrize("n,m,k", [(1, 16, 32), (17, 48, 96), (5, 64, 2048), (8, 2048, 5632), (3, 72, 448), (9, 40, 64), (16, 2048, 2048), (12, 1000, 1152), (16, 4096, 320), (33, 72, 288), (45, 2048, 2048), (48, 100, 5632),
                                    (64, 2048, 5632), (64, 4096, 1056), (50, 4096, 4096), (32, 1000, 736), (63, 4090, 160)])
 def test_resid_then_scaled_consumers(n, m, k):
     """The product added to the residual stream, what the norm behind it needs left beside it, and the two
@@ -21,7 +21,7 @@ def test_resid_then_scaled_consumers(n, m, k):
     k_, eps = K(), 1e-5
     x, w = _bf(n, k, seed=1, scale=0.5), _bf(m, k, seed=2, scale=0.1)
     resid, nw = rnd(n, m, seed=3, scale=2.0), 1 + 0.2 * rnd(m, seed=4)
-    parts = -(-m // 16)
+    parts = k_.linear_rows_parts(n, m, k)
     ss = torch.full((n, -(-parts // 4) * 4), float("nan"), device=DEV)
     xw = torch.full((n, m), float("nan"), dtype=torch.bfloat16, device=DEV)
     stream = resid.clone()
@@ -56,7 +56,8 @@ def test_resid_then_scaled_consumers(n, m, k):
             k_.linear_rows(k_.fused_linear_tile(wg, k_.LINEAR_SWIGLU), ht, k_.LINEAR_SWIGLU, st)
             got = []
             for hin in (h, ht):
-                z, y, zs = torch.zeros(n, 96, device=DEV), torch.empty(n, 96, dtype=torch.bfloat16, device=DEV), torch.empty(n, 8, device=DEV)
+                z, y, zs = torch.zeros(n, 96, device=DEV), torch.empty(n, 96, dtype=torch.bfloat16, device=DEV), None
+                zs = torch.empty(n, -(-k_.linear_rows_parts(n, 96, f) // 4) * 4, device=DEV)
                 k_.linear_rows(k_.fused_linear_tile(wn, k_.LINEAR_PARTS), y, k_.LINEAR_RESID, hin, resid=z,
                                norm_weight=torch.ones(96, device=DEV), ss_out=zs)
                 got.append((z, y))
