@@ -194,7 +194,7 @@ typedef struct {
   int y_tiled;          /* kllm_linear_rows, RESID and SWIGLU: y goes out in the order the next such product's lanes read */
 } KllmLinearOut;
 long kllm_fused_linear_lds_bytes(int n, int k, int nsplit, int dtype);
-/* The RESID, SWIGLU and ROPE products of 17 to 64 rows (any n up to 64 is taken), bfloat16, K a multiple of 32,
+/* The same products of up to 64 rows, bfloat16, all of K (a multiple of 32) in a workgroup and nothing staged,
  * w the tiled copy.  RESID leaves kllm_linear_rows_parts(n, m, k) sums of squares a row (0: the sizes are not taken).  Tiled rows
  * (y_tiled, x_tiled; columns a multiple of 32): [row / 16][column / 32][column % 32 / 8][row % 16][8]; with more than 16 rows
  * those up to the next multiple of 16 are there and hold anything, with fewer only the rows are. */

@@ -39,7 +39,7 @@ constexpr int LR_TILE = 16 * LR_LD;
 // Steps of K in each of the two buffers a wave fills in turn: what 128 registers hold, four at most.
 constexpr int lr_ahead(int nt, int tw) { return nt + tw <= 4 ? 4 : nt + tw == 5 ? 3 : 2; }
 
-// SPLIT (FL_RESID, up to 16 rows): a workgroup takes eight rows of W, each twice in a matrix instruction: K's first half in its rows
+// SPLIT (FL_RESID and FL_PARTS, up to 16 rows): a workgroup takes eight rows of W, each twice in a matrix instruction: K's first half in its rows
 // 0-7, the second half in rows 8-15, so that a load still brings a kilobyte.  Up to eight rows of X lie in the operand's columns the
 // same way (NT 1); more take an instruction for each half of K (NT 2).  What pairs a half with the other's X is not used.  A CU streams
 // about 20 GB/s of weights from memory whatever a workgroup has in flight, so a product on half the CUs takes half as long again:
@@ -238,6 +238,27 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __re
     }
     return;
   }
+  if (EP == FL_PARTS) {                // the sums, or an activation of them in 16 bits
+    constexpr int C = SPLIT ? 8 : 16 * TW, ROWS = SPLIT ? 16 : 16 * NT;
+#pragma unroll 1
+    for (int u = 0; u < (ROWS * C + 64 * NW - 1) / (64 * NW); ++u) {
+      const int idx = tid + 64 * NW * u;
+      const int cc = idx % C, r = idx / C, xr = row0 + r, col = group * (16 * TW) + 8 * half_tile + cc;
+      if (r >= ROWS || xr >= n || col >= m) continue;
+      const float v = sum_of(SPLIT ? 0 : cc / 16, SPLIT ? 0 : r / 16, r % 16, SPLIT ? cc : cc % 16);
+      if (out.act >= FL_UNARY) {
+        float a_pos = 0.f, a_neg = 0.f;
+        if (out.act - FL_UNARY == ACT_XIELU) {
+          a_pos = softplus_f32(out.norm_w[0]);
+          a_neg = softplus_f32(out.norm_w[1]);
+        }
+        reinterpret_cast<bf16_t*>(out.y)[(long)xr * m + col] = from_f32<bf16_t>(unary_act(v, out.act - FL_UNARY, a_pos, a_neg));
+      } else {
+        reinterpret_cast<float*>(out.y)[(long)xr * m + col] = v;
+      }
+    }
+    return;
+  }
   if (EP == FL_SWIGLU || EP == FL_ROPE) {
     constexpr int P = 8 * TW;                                    // pairs of a row in the workgroup
     const int pairs = m / 2;
@@ -290,7 +311,7 @@ static int lr_launch(const void* x, const FlOut& out, const void* w, int n, int 
                      int x_stride, hipStream_t stream) {
   // Four waves a workgroup where a CU has several of them (4,096 -> 6,144: 14.7 us with eight, 13.3 with four), eight where it
   // has one (a step of one token at 1.1B sizes 0.3 % shorter, of 64 tokens 1.2 %).
-  if constexpr (EP != FL_SWIGLU || TW == 3)
+  if constexpr ((EP != FL_SWIGLU && EP != FL_PARTS) || TW == 3)
     if ((long)halves * ceil_div(tiles, TW) > device_cus())
       return lr_launch_waves<NT, TW, EP, SCALED, 4>(x, out, w, n, m, k, tiles, halves, x_stride, stream);
   return lr_launch_waves<NT, TW, EP, SCALED, 8>(x, out, w, n, m, k, tiles, halves, x_stride, stream);
@@ -302,6 +323,7 @@ static int lr_launch_ep(int ep, bool scaled, const void* x, const FlOut& out, co
   if (ep == FL_SWIGLU)
     return scaled ? lr_launch<NT, TW, FL_SWIGLU, true>(x, out, w, n, m, k, tiles, halves, xs, st)
                   : lr_launch<NT, TW, FL_SWIGLU, false>(x, out, w, n, m, k, tiles, halves, xs, st);
+  if (ep == FL_PARTS) return lr_launch<NT, TW, FL_PARTS, false>(x, out, w, n, m, k, tiles, halves, xs, st);
   if constexpr (TW == 1) {
     if (ep == FL_RESID) return lr_launch<NT, 1, FL_RESID, false>(x, out, w, n, m, k, tiles, halves, xs, st);
     return scaled ? lr_launch<NT, 1, FL_ROPE, true>(x, out, w, n, m, k, tiles, halves, xs, st)
@@ -322,9 +344,9 @@ static int lr_launch_tw(int tw, int ep, bool scaled, const void* x, const FlOut&
 
 using namespace kllm;
 
-static int lr_tiles(int kind, int m) { return kind == FL_RESID ? ceil_div(m, 16) : ceil_div(m / 2, 8); }
+static int lr_tiles(int kind, int m) { return kind == FL_RESID || kind == FL_PARTS ? ceil_div(m, 16) : ceil_div(m / 2, 8); }
 
-// Whether a residual product takes eight rows of W a workgroup (SPLIT): up to 16 rows of X and no more tiles than half the CUs.
+// Whether a product that splits takes eight rows of W a workgroup (SPLIT): up to 16 rows of X and no more tiles than half the CUs.
 static bool lr_split(int n, int m, int k) { return n <= 16 && k % 64 == 0 && 2 * lr_tiles(FL_RESID, m) <= device_cus(); }
 
 extern "C" int kllm_linear_rows_parts(int n, int m, int k) {
@@ -337,7 +359,7 @@ extern "C" int kllm_linear_rows(const void* x, int x_stride, const KllmLinearOut
                                 hipStream_t stream) {
   KLLM_REQUIRE(x && yout && w && yout->y, "linear_rows: null pointer");
   const int ep = yout->kind;
-  KLLM_REQUIRE(ep == FL_RESID || ep == FL_SWIGLU || ep == FL_ROPE, "linear_rows: output kind %d is not built", ep);
+  KLLM_REQUIRE(ep == FL_PARTS || ep == FL_RESID || ep == FL_SWIGLU || ep == FL_ROPE, "linear_rows: unknown output kind %d", ep);
   KLLM_REQUIRE(n > 0 && n <= LR_ROWS, "linear_rows: n=%d is outside [1, %d]", n, LR_ROWS);
   KLLM_REQUIRE(m > 0 && k > 0 && k % 32 == 0, "linear_rows: bad sizes m=%d k=%d (K must be a multiple of 32)", m, k);
   KLLM_REQUIRE(k <= (1 << 20) && m < (1 << 30), "linear_rows: sizes overflow");
@@ -358,7 +380,7 @@ extern "C" int kllm_linear_rows(const void* x, int x_stride, const KllmLinearOut
   const int tiles = lr_tiles(ep, m);
   const bool scaled = yout->ss_in != nullptr;
   if (scaled) {
-    KLLM_REQUIRE(ep != FL_RESID, "linear_rows: only the gate and the rotation epilogues scale their rows");
+    KLLM_REQUIRE(ep != FL_RESID && ep != FL_PARTS, "linear_rows: only the gate and the rotation epilogues scale their rows");
     KLLM_REQUIRE(yout->ss_parts >= 1 && yout->ss_parts <= FL_SS_MAX && ((uintptr_t)yout->ss_in & 15) == 0 && yout->eps >= 0.f,
                  "linear_rows: %d partial sums of squares per row are outside [1, %d], or they are not 16-byte aligned",
                  yout->ss_parts, FL_SS_MAX);
@@ -374,6 +396,10 @@ extern "C" int kllm_linear_rows(const void* x, int x_stride, const KllmLinearOut
     out.resid = yout->resid;
     out.norm_w = yout->norm_w;
     out.ss_out = yout->ss_out;
+  } else if (ep == FL_PARTS) {
+    KLLM_REQUIRE(out.act < FL_UNARY + UNARY_ACT_COUNT, "linear_rows: unknown activation %d on the sums", out.act - FL_UNARY);
+    KLLM_REQUIRE(out.act - FL_UNARY != ACT_XIELU || yout->norm_w, "linear_rows: this activation needs its two constants");
+    out.norm_w = yout->norm_w;
   } else {
     KLLM_REQUIRE(m % 2 == 0, "linear_rows: m=%d must be even for a pair epilogue", m);
   }
@@ -403,22 +429,24 @@ extern "C" int kllm_linear_rows(const void* x, int x_stride, const KllmLinearOut
   // Tiles a workgroup: the least that leaves one round of the chip, three at most (2 x 5,632 x 2,048, 8 / 64 rows: 12.1 / 17.5 us with two, 11.0
   // / 14.9 with three, 13.3 / 16.4 with four; 2 x 14,336 x 4,096, 16 / 64 rows: 48.5 / 62.0, 46.5 / 59.3, 54.5 / 59.6).
   int tw = 1;
-  if (ep == FL_SWIGLU)
+  if (ep == FL_SWIGLU || ep == FL_PARTS)
     while (tw < 3 && ceil_div(tiles, tw) > cus) ++tw;
   const int row_tiles = ceil_div(n, 16);
   // Halves of the rows where the busiest CU then has fewer tiles of rows to take (or as many, of workgroups that share it
   // anyway): 64 rows against 2,048 x 5,632 (128 tiles) 17.6 -> 12.2 us, 6,144 x 4,096 (384) 25.4 -> 21.2, 48 rows 21.3 -> 18.8; not
   // 4,096 x 14,336 (256) 41.0 -> 46.7, nor 2,560 x 2,048 (160) at 32 rows 5.0 -> 5.5.
   const int whole = ceil_div(tiles, cus) * row_tiles, halved = ceil_div(2L * tiles, cus) * ceil_div(row_tiles, 2);
-  const int halves = ep != FL_SWIGLU && (halved < whole || (halved == whole && tiles > cus)) ? 2 : 1;
+  const int halves = ep != FL_SWIGLU && tw == 1 && (halved < whole || (halved == whole && tiles > cus)) ? 2 : 1;
   const int nt = ceil_div(row_tiles, halves);
-  const int rc = ep == FL_RESID && lr_split(n, m, k)
-                     ? (n <= 8 ? lr_launch_waves<1, 1, FL_RESID, false, 8, true>(x, out, w, n, m, k, tiles, 1, x_stride, stream)
-                               : lr_launch_waves<2, 1, FL_RESID, false, 8, true>(x, out, w, n, m, k, tiles, 1, x_stride, stream))
+#define KLLM_LRS(NT, EP) lr_launch_waves<NT, 1, EP, false, 8, true>(x, out, w, n, m, k, tiles, 1, x_stride, stream)
+  const bool split = (ep == FL_RESID || ep == FL_PARTS) && lr_split(n, m, k);
+  const int rc = split     ? (ep == FL_RESID ? (n <= 8 ? KLLM_LRS(1, FL_RESID) : KLLM_LRS(2, FL_RESID))
+                                             : (n <= 8 ? KLLM_LRS(1, FL_PARTS) : KLLM_LRS(2, FL_PARTS)))
                : nt == 1 ? lr_launch_tw<1>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream)
                : nt == 2 ? lr_launch_tw<2>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream)
                : nt == 3 ? lr_launch_tw<3>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream)
                          : lr_launch_tw<4>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream);
+#undef KLLM_LRS
   if (rc) return rc;
   KLLM_CHECK_LAUNCH("linear_rows");
   return 0;

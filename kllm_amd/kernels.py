@@ -1015,20 +1015,18 @@ def linear_rows_best(kind, n, m, k, dtype=torch.bfloat16, tiled_x=True) -> bool:
     if n <= 16:
         return True
     tiles, cus, row_tiles = -(-m // 16), device_cus(), -(-n // 16)
-    busiest = -(-tiles // (3 * cus)) * row_tiles if kind == LINEAR_SWIGLU else min(
+    busiest = -(-tiles // (3 * cus)) * row_tiles if kind == LINEAR_SWIGLU or (kind == LINEAR_PARTS and tiles > cus) else min(
         -(-tiles // cus) * row_tiles, -(-2 * tiles // cus) * -(-row_tiles // 2))
     return 32 * k * busiest * (1 if tiled_x else 2) <= LINEAR_ROWS_BYTES
 
 
-def linear_rows(w, y, kind, x, rope=None, act=ACT_SILU, resid=None, norm_weight=None, ss_out=None):
-    """``fused_linear`` for up to 64 rows of bfloat16, K a multiple of 32: LINEAR_RESID, LINEAR_SWIGLU and
-    LINEAR_ROPE from the tiled copy ``w`` of the weights, nothing staged in LDS.  ``x`` (also inside a ``ScaledRows``) may be
-    ``TiledRows``, and so may ``y`` of the first two."""
+def linear_rows(w, y, kind, x, rope=None, act=ACT_SILU, resid=None, norm_weight=None, ss_out=None, unary=None):
+    """``fused_linear`` for up to 64 rows of bfloat16, K a multiple of 32, in one slice,
+    from the tiled copy ``w`` of the weights, nothing staged in LDS.  ``x`` (also inside a ``ScaledRows``) may be
+    ``TiledRows``, and so may ``y`` of LINEAR_RESID and LINEAR_SWIGLU."""
     if not isinstance(w, TiledWeights):
         raise KernelError("linear_rows: takes the tiled copy of the weights")
-    if kind not in (LINEAR_RESID, LINEAR_SWIGLU, LINEAR_ROPE):
-        raise KernelError(f"linear_rows: output kind {kind} is not built")
-    fused_linear(w, y, kind, x, rope=rope, act=act, resid=resid, norm_weight=norm_weight, ss_out=ss_out, _rows=True)
+    fused_linear(w, y, kind, x, rope=rope, act=act, resid=resid, norm_weight=norm_weight, ss_out=ss_out, unary=unary, _rows=True)
 
 
 def fused_linear(w, y, kind, x, nsplit=1, tiles_per_wg=1, rope=None, act=ACT_SILU, resid=None, norm_weight=None,
@@ -1065,7 +1063,7 @@ def fused_linear(w, y, kind, x, nsplit=1, tiles_per_wg=1, rope=None, act=ACT_SIL
     lo.kind, lo.nsplit, lo.act = kind, nsplit, int(act)
     for name, t in (("x", x), ("y", y)):
         if isinstance(t, TiledRows):
-            if (not _rows or (name == "y" and kind == LINEAR_ROPE) or t.dtype != typ or not t.data.is_contiguous()
+            if (not _rows or (name == "y" and kind in (LINEAR_ROPE, LINEAR_PARTS)) or t.dtype != typ or not t.data.is_contiguous()
                     or t.shape[1] % 32 or t.data.shape[0] != TiledRows.stored(n) or (name == "x" and t.shape[1] != k)):
                 raise KernelError(f"linear_rows: tiled rows {t.shape} do not fit {name}, or the kernel takes none")
     if isinstance(x, TiledRows):

@@ -13,7 +13,7 @@ import torch
 
 from .. import kernels as K
 from .base import Normed, Part, register_part
-from .linear import decode_batch_fits, decode_linear, fused_f32, linear, linear_into, rows_kernel, sink_takes_rows, tiled_copy
+from .linear import decode_batch_fits, decode_linear, fused_f32, linear, linear_into, parts_rows, rows_kernel, sink_takes_rows, tiled_copy
 from .spec import WeightSpec
 
 
@@ -160,7 +160,8 @@ def dense_hidden(ctx, xn, w_up, tag, tiled, act, params=None):
     if (n > 128 and opts.get("gemm") != "library" and opts.get("gemm_algo") is None
             and xn.shape[1] % (8 if xn.dtype == torch.bfloat16 else 4) == 0):
         K.gemm_act(xn, w_up, h, act, params)      # prompts
-    elif decode_batch_fits(ctx.runtime, xn) and not opts.get("no_fused_linear") and opts.get("gemm_algo") is None:
+    elif parts_rows(ctx.runtime, n, w_up, tiled) or (decode_batch_fits(ctx.runtime, xn) and not opts.get("no_fused_linear")
+                                                     and opts.get("gemm_algo") is None):
         h = decode_linear(ctx, xn, w_up, tag + ".h", tiled, unary=(act, params))      # decode batches
     else:
         K.unary_act(decode_linear(ctx, xn, w_up, tag + ".up", tiled), h, act, params)

@@ -323,14 +323,25 @@ def decode_batch_fits(rt, x):
     return n <= 16 and K.fused_linear_fits(n, k, 1, x.dtype)
 
 
+def parts_rows(rt, n, w, w_tiled):
+    """Whether ``decode_linear`` runs on ``K.linear_rows``: not 9 to 16 rows, which the decode-batch kernel has in LDS while this one reads
+    sixteen of them a load (a step at Natenex sizes, without and with: 1 token 674 / 655 us, 8 785 / 785, 16 898 / 903; beyond 16 it takes
+    the place of K in slices: 24 1,123 / 894, 48 1,268 / 1,192, 64 1,538 / 1,524, a prompt of 20 1,004 / 761, of 60 1,146 / 1,131)."""
+    return w.shape[0] < 16384 and not 9 <= n <= 16 and rows_kernel(rt, K.LINEAR_PARTS, n, w, w_tiled, False)
+
+
 def decode_linear(ctx, x, w, tag, w_tiled=None, unary=None):
     """``linear`` for a consumer that takes float32 sums either whole or in slices: decode
     batches of up to 16 rows run on the decode-batch kernel with all of K in a workgroup (one
     result, from the tiled copy of w where there is one); everything else as ``linear`` cuts it.
-    ``unary`` = (activation without a gate, its constants): only where ``decode_batch_fits``;
+    ``unary`` = (activation without a gate, its constants): only where ``decode_batch_fits`` or ``parts_rows``;
     the result is then the activation of the sums in the compute dtype."""
     n, m = x.shape[0], w.shape[0]
     rt = ctx.runtime
+    if parts_rows(rt, n, w, w_tiled):
+        y = ctx.buf(tag, (n, m) if unary is not None else (1, n, m), x.dtype if unary is not None else torch.float32)
+        K.linear_rows(w_tiled, y, K.LINEAR_PARTS, x, unary=unary)
+        return y if unary is not None else y[0]
     if decode_batch_fits(rt, x) and not rt.options.get("no_fused_linear") and rt.options.get("gemm_algo") is None:
         tiles = 4 if m >= 16384 else 1
         if unary is not None:

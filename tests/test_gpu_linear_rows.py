@@ -131,9 +131,27 @@ def test_refusals():
     with pytest.raises(k_.KernelError, match="multiple of 32"):
         k_.linear_rows(k_.fused_linear_tile(_bf(64, 40, seed=1, scale=0.1), k_.LINEAR_SWIGLU), h, k_.LINEAR_SWIGLU,
                        _bf(20, 40, seed=2, scale=1.0))
-    with pytest.raises(k_.KernelError, match="not built"):
-        k_.linear_rows(k_.fused_linear_tile(w, k_.LINEAR_PARTS), torch.empty(1, 20, 64, device=DEV), k_.LINEAR_PARTS,
-                       _bf(20, 96, seed=2, scale=1.0))
+
+
+@pytest.mark.parametrize("n,m,k", [(1, 40, 64), (8, 2048, 2048), (5, 72, 96), (13, 2048, 1536), (16, 5632, 2048), (20, 5632, 512),
+                                   (33, 4096, 1056), (64, 2048, 5632), (45, 12300, 160), (3, 9000, 544)])
+def test_sums_and_activations_of_them(n, m, k):
+    """Plain sums, and an activation of them in 16 bits: half tiles of W, whole ones, two and three a workgroup."""
+    k_ = K()
+    x, w = _bf(n, k, seed=1, scale=0.5), _bf(m, k, seed=2, scale=0.1)
+    tiled = k_.fused_linear_tile(w, k_.LINEAR_PARTS)
+    want = x.double() @ w.double().T
+    y = torch.full((1, n, m), float("nan"), device=DEV)
+    k_.linear_rows(tiled, y, k_.LINEAR_PARTS, x)
+    assert (y[0].double() - want).abs().max() < 1e-3 * k ** 0.5 * 0.05 + 1e-4      # (as for the decode-batch kernel's sums)
+    h = torch.full((n, m), float("nan"), dtype=torch.bfloat16, device=DEV)
+    k_.linear_rows(tiled, h, k_.LINEAR_PARTS, x, unary=(k_.ACT_RELU_SQ, None))
+    want = want.clamp(min=0) ** 2
+    assert (h.double() - want).abs().max() < 0.01 * want.abs().max() + 1e-3
+    params = torch.tensor([0.3, -0.2], device=DEV)
+    k_.linear_rows(tiled, h, k_.LINEAR_PARTS, x, unary=(k_.ACT_XIELU, params))
+    k_.unary_act(y, h2 := torch.empty_like(h), k_.ACT_XIELU, params)
+    assert torch.equal(h, h2)
 
 
 def _rowwise(t):
