@@ -722,7 +722,7 @@ constexpr int kGateChunk = 1024;              // inputs of a block that LDS hold
 // the matrices' way from memory bounds the time, and it needs workgroups (16 channels each) and short
 // chains; a prompt has tiles enough and is bound by its products.
 // 1,500 tokens x 2,048 channels in blocks of 256: 140 -> 63 us (FMA on eight tokens at a time, 790 MB of matrices
-// through L2); 8 tokens: 18 -> 11 us, in a step, where the matrices come from memory, 28.8 -> 16.9 (32 workgroups then, 128 now).
+// through L2); 8 tokens: 18 -> 11 us, in a step, where the matrices come from memory, 28.8 -> 16.9 (32 workgroups then, 128 now) -> 14.0.
 // TAPS: the convolution's where it is 4, 8 for any number up to 8, 0 for more.  ONE: a block's inputs fit into LDS at
 // once; the sums then begin behind the convolution and take no registers in it (72 instead of 89, three workgroups a CU).
 template <int NT, int KS, int OW, int TAPS, bool ONE>
@@ -763,6 +763,7 @@ __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel
 #pragma unroll
   for (int t = 0; t < NT; ++t) ar[t] = ai[t] = own[t] = floatx4{0.f, 0.f, 0.f, 0.f};
   constexpr int CHAIN = 4;                    // steps of a chain
+  constexpr int AHEAD = KS > 1 ? CHAIN : 1;   // steps asked for ahead
   __shared__ int4 spans[TT];                  // the tokens' spans
   if (tid < nt) {
     const int span = span_of_token[tfirst + tid];
@@ -771,7 +772,15 @@ __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel
   int k0 = 0;
   do {
     __syncthreads();
-    if (TAPS > 0 && nt > 1) {
+    const int steps = (min(chunk, bs - k0) + 15) / 16;
+    const int per = (steps + KS - 1) / KS, s0 = ks * per, s1 = min(steps, s0 + per);
+    // The first of this wave's share of the matrices: a decode batch's whole chain (they come from memory, and nothing
+    // in them waits for the convolution), a prompt's first step.
+    Pair w[AHEAD];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i)
+      if (KS > 1) w[i] = fetch(k0 + 16 * min(s0 + i, steps - 1));
+    if (TAPS > 0 && (nt > 1 || KS > 1)) {
       // A thread takes a channel for a run of RUN tokens and asks for the run's inputs at once, each
       // for all the taps it meets, instead of for every tap of every token on its own.
       constexpr int MOST = TAPS > 0 ? TAPS : 1, RUN = 8;
@@ -791,6 +800,24 @@ __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel
           for (int j = 0; j < MOST; ++j) wt[j] = conv_w[(long)c * taps + min(j, K)];
         }
         const float cb = there ? conv_b[c] : 0.f;
+        // A decode batch's tokens are spans of their own and find all but one input in the requests' states: a run of
+        // tokens with a span's start in it asks for all their entries at once (in a prompt, where such runs are few, one by one: the
+        // entries' registers would cost a workgroup a CU).  8 tokens of 2,048 channels, in a step: 17.5 -> 15.6 us, 14.0 with the matrices asked for ahead.
+        constexpr bool AT_ONCE = KS > 1 && TAPS > 1;
+        float st[AT_ONCE ? RUN : 1][AT_ONCE ? TAPS - 1 : 1];
+        if constexpr (AT_ONCE) {
+          bool starts = false;
+#pragma unroll
+          for (int q = 0; q < RUN; ++q) starts |= there && tt0 + q < nt && tfirst + tt0 + q - K < spans[min(tt0 + q, nt - 1)].x;
+          if (starts) {
+#pragma unroll
+            for (int q = 0; q < RUN; ++q) {                 // (tokens that are not there: the last one's, not used)
+              const float* from = state + (long)spans[min(tt0 + q, nt - 1)].y * slot_stride + (long)c * K;
+#pragma unroll
+              for (int j = 0; j < TAPS - 1; ++j) st[q][j] = from[min(j, K - 1)];
+            }
+          }
+        }
 #pragma unroll
         for (int q = 0; q < RUN; ++q) {
           float v = 0.f;
@@ -802,7 +829,16 @@ __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel
               if (j > K) break;
               const int back = (int)(t - K + j) - sp.x;      // rows behind the span's first
               float in = x[q + j];
-              if (back < 0) in = sp.z ? 0.f : state[(long)sp.y * slot_stride + (long)c * K + K + back];
+              if (back < 0) {
+                if constexpr (AT_ONCE) {
+                  in = st[q][0];                      // entry K + back, by choice: the entries stay in registers
+#pragma unroll
+                  for (int i = 1; i < TAPS - 1; ++i) in = i == K + back ? st[q][i] : in;
+                  in = sp.z ? 0.f : in;
+                } else {
+                  in = sp.z ? 0.f : state[(long)sp.y * slot_stride + (long)c * K + K + back];
+                }
+              }
               v = fmaf(wt[j], in, v);
             }
             v += cb;
@@ -823,9 +859,7 @@ __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel
         us[tt * ld + e - k0] = v;
       }
     }
-    const int steps = (min(chunk, bs - k0) + 15) / 16;
-    const int per = (steps + KS - 1) / KS, s0 = ks * per, s1 = min(steps, s0 + per);
-    Pair w = fetch(k0 + 16 * min(s0, steps - 1));
+    if (KS == 1) w[0] = fetch(k0 + 16 * min(s0, steps - 1));
     __syncthreads();
     if (o >= k0 && o < k0 + chunk)
 #pragma unroll
@@ -836,9 +870,7 @@ __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel
       floatx4 cr[NT], ci[NT];
 #pragma unroll
       for (int t = 0; t < NT; ++t) cr[t] = ci[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-      for (int s = c0; s < min(s1, c0 + CHAIN); ++s) {
-        const Pair next = fetch(k0 + 16 * min(s + 1, steps - 1));
+      auto step = [&](int s, const Pair& w) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
           const floatx4 u = *reinterpret_cast<const floatx4*>(&us[(t * kGateTile + col) * ld + 16 * s + 4 * quad]);
@@ -848,7 +880,21 @@ __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel
             ci[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(u[e], w.i[e], ci[t], 0, 0, 0);
           }
         }
-        w = next;
+      };
+      if constexpr (KS > 1) {
+#pragma unroll
+        for (int i = 0; i < CHAIN; ++i)
+          if (c0 + i < s1) step(c0 + i, w[i]);
+        if (c0 + CHAIN < s1)
+#pragma unroll
+          for (int i = 0; i < CHAIN; ++i) w[i] = fetch(k0 + 16 * min(c0 + CHAIN + i, steps - 1));
+      } else {
+#pragma unroll 1
+        for (int s = c0; s < min(s1, c0 + CHAIN); ++s) {
+          const Pair next = fetch(k0 + 16 * min(s + 1, steps - 1));
+          step(s, w[0]);
+          w[0] = next;
+        }
       }
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
