@@ -83,28 +83,6 @@ __device__ __forceinline__ floatx4 fl_sum(floatx4 (&acc)[16]) {
 constexpr int FL_LDS_MAX = 160 * 1024;
 constexpr int FL_TILE = 16 * 17;    // floats of one wave's partial tile in LDS: [x row][w row], padded
 
-// Row of W behind MFMA row c of a tile, or -1.  Pair epilogues: unit = pair.
-template <int EP>
-__device__ __forceinline__ long fl_row(int tile, int c, int m, const FlOut& o) {
-  if (EP == FL_PARTS || EP == FL_RESID) {
-    const long r = (long)tile * 16 + c;
-    return r < m ? r : -1;
-  }
-  const int pair = tile * 8 + (c & 7);          // m < 2^31, so pairs and tiles fit an int
-  const int pairs = m / 2;
-  if (pair >= pairs) return -1;
-  const bool second = c >= 8;
-  if (EP == FL_SWIGLU) return second ? pairs + pair : pair;
-  const int half = o.hd / 2;
-  const int rot_pairs = (o.H + (o.cache ? o.KV : 0)) * half;
-  if (pair < rot_pairs) {
-    const long a = (long)(pair / half) * o.hd + pair % half;   // q and k rows follow each other in W
-    return second ? a + half : a;
-  }
-  const long e = 2 * (long)(pair - rot_pairs);
-  return (long)(o.H + o.KV) * o.hd + e + (second ? 1 : 0);
-}
-
 // NW waves share a tile's K; SCALED: the sums are multiplied by a row scale made from out.ss_in;
 // PASSES: the rows of X do not fit into LDS at once and go in passes of kpass of K (a kernel of
 // its own, so that the one for rows that fit carries none of it).

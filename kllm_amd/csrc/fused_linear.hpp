@@ -34,6 +34,28 @@ struct FlOut {
   int x_tiled, y_tiled;         // linear_rows: rows in the lanes' order
 };
 
+// Row of W behind MFMA row c of a tile, or -1.  Pair epilogues: unit = pair.
+template <int EP>
+__device__ __forceinline__ long fl_row(int tile, int c, int m, const FlOut& o) {
+  if (EP == FL_PARTS || EP == FL_RESID) {
+    const long r = (long)tile * 16 + c;
+    return r < m ? r : -1;
+  }
+  const int pair = tile * 8 + (c & 7);          // m < 2^31, so pairs and tiles fit an int
+  const int pairs = m / 2;
+  if (pair >= pairs) return -1;
+  const bool second = c >= 8;
+  if (EP == FL_SWIGLU) return second ? pairs + pair : pair;
+  const int half = o.hd / 2;
+  const int rot_pairs = (o.H + (o.cache ? o.KV : 0)) * half;
+  if (pair < rot_pairs) {
+    const long a = (long)(pair / half) * o.hd + pair % half;   // q and k rows follow each other in W
+    return second ? a + half : a;
+  }
+  const long e = 2 * (long)(pair - rot_pairs);
+  return (long)(o.H + o.KV) * o.hd + e + (second ? 1 : 0);
+}
+
 // A workgroup barrier for data in LDS.  Unlike __syncthreads it does not wait for loads from
 // memory: the weights asked for ahead stay in flight while the waves meet.
 __device__ __forceinline__ void fl_lds_barrier() {

@@ -44,10 +44,26 @@ constexpr int lr_ahead(int nt, int tw) { return nt + tw <= 4 ? 4 : nt + tw == 5 
 // same way (NT 1); more take an instruction for each half of K (NT 2).  What pairs a half with the other's X is not used.  A CU streams
 // about 20 GB/s of weights from memory whatever a workgroup has in flight, so a product on half the CUs takes half as long again:
 // a step at 1.1B sizes, 1 / 8 / 16 tokens 894 / 939 / 1,032 us without, 882 / 920 / 1,026 with.
-template <int NT, int TW, int EP, bool SCALED, int NW, bool SPLIT>
-__global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __restrict__ X, FlOut out,
-                                                              const bf16_t* __restrict__ W, int n, int m, int k, int tiles,
-                                                              int halves, int x_stride) {
+// float32 (up to 16 rows): four instructions of 4 to a step, true 32-bit.  A sum's products go in 64 or 128 chains, no fewer than in the
+// decode-batch kernel: 16 a wave, or 8 where eight waves take the place of its four (the gate, plain sums).
+template <typename T, int EP> constexpr int lr_chains() { return sizeof(T) == 2 ? 1 : EP == FL_RESID || EP == FL_ROPE ? 16 : 8; }
+__device__ __forceinline__ void lr_mma(uintx4 w, uintx4 x, floatx4 (&acc)[1], int, bf16_t) {
+  acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, x), acc[0], 0, 0, 0);
+}
+template <int CH>
+__device__ __forceinline__ void lr_mma(uintx4 w, uintx4 x, floatx4 (&acc)[CH], int i, float) {
+  const floatx4 a = __builtin_bit_cast(floatx4, w), b = __builtin_bit_cast(floatx4, x);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    floatx4& c = acc[(4 * i + e) % CH];
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
+  }
+}
+
+template <typename T, int NT, int TW, int EP, bool SCALED, int NW, bool SPLIT>
+__global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const T* __restrict__ X, FlOut out, const T* __restrict__ W, int n,
+                                                              int m, int k, int tiles, int halves, int x_stride) {
+  constexpr int ES = (int)sizeof(T), CH = lr_chains<T, EP>();
   constexpr int A = lr_ahead(NT, TW);
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   float* part = reinterpret_cast<float*>(lds_raw);               // [NW][TW][NT][x row 16][LR_LD]
@@ -61,7 +77,7 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __re
   const int half_tile = SPLIT ? (int)blockIdx.x % 2 : 0;         // which eight rows of W
   const int row0 = halves == 1 ? 0 : (int)(blockIdx.x / 8 % 2) * (16 * NT);
   if (group >= groups || row0 >= n) return;                      // the whole workgroup
-  const int steps = k / 32;                                      // (k is a multiple of 32)
+  const int steps = k / (64 / ES);                               // of 64 bytes of a row (k is a multiple of 32)
   const int walk = SPLIT ? steps / 2 : steps;                    // steps that the waves share
   const int per = (walk + NW - 1) / NW;
   const int s_beg = min(wave * per, walk);
@@ -112,27 +128,34 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __re
   // addition.  A step that does not exist reads the wave's last (or K's last) again and is not multiplied; a
   // tile or a row of X beyond the last one reads the last, and its sums are not stored.
   const int tile0 = group * TW;
+  // (float32 also takes the weights as they are, row by row: the sums are the same bits, so that a card with no room for
+  // the tiled copy gives the same results)
+  const bool tiled = ES == 2 || out.tiled;
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<char*>(reinterpret_cast<const char*>(W)) + (long)tile0 * steps * 1024, 0,
-      min(TW, tiles - tile0) * steps * 1024, 0x00020000);
+      const_cast<char*>(reinterpret_cast<const char*>(W)) + (tiled ? (long)tile0 * steps * 1024 : 0), 0,
+      tiled ? min(TW, tiles - tile0) * steps * 1024 : m * k * ES, 0x00020000);
+  const int w_step = tiled ? 1024 : 64;
   const int row_tiles = (n + 15) / 16, side = min(n, 16), x_step = out.x_tiled ? 64 * side : 64;
   const __amdgpu_buffer_rsrc_t xr_ = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<bf16_t*>(X), 0, out.x_tiled ? row_tiles * steps * x_step : 2 * ((n - 1) * x_stride + k), 0x00020000);
+      const_cast<T*>(X), 0, out.x_tiled ? row_tiles * steps * x_step : ES * ((n - 1) * x_stride + k), 0x00020000);
+  const int later = SPLIT && c >= 8 ? walk : 0;                  // steps on, for the lanes of the second half of K
+  const int wc = SPLIT ? 8 * half_tile + c % 8 : c;              // this lane's row of a tile
   int wo[TW], xo[NT];
 #pragma unroll
-  for (int j = 0; j < TW; ++j) wo[j] = min(j, tiles - tile0 - 1) * steps * 1024;
+  for (int j = 0; j < TW; ++j) {
+    const int tile = min(j, tiles - tile0 - 1);
+    wo[j] = tile * steps * 1024 + later * 1024 + (16 * g + wc) * 16;
+    if (!tiled) wo[j] = (int)max(fl_row<EP>(tile0 + tile, wc, m, out), 0L) * k * ES + later * 64 + 16 * g;
+  }
 #pragma unroll
   for (int t = 0; t < NT; ++t)
     xo[t] = out.x_tiled ? min(row0 / 16 + t, row_tiles - 1) * steps * x_step + (g * side + min(c, side - 1)) * 16
-                        : 2 * (min(row0 + t * 16 + c, n - 1) * x_stride + 8 * g);
-  int wl = lane * 16;                                            // this lane's place in a step of W
+                        : ES * min(row0 + t * 16 + c, n - 1) * x_stride + 16 * g;
   if (SPLIT) {
-    const int later = c < 8 ? 0 : walk;                          // steps on, for the lanes of the second half of K
-    wl = later * 1024 + (16 * g + 8 * half_tile + c % 8) * 16;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const int row = min(NT == 1 ? c % 8 : c, n - 1);
-      xo[t] = (NT == 1 ? later : t * walk) * x_step + (out.x_tiled ? (g * side + row) * 16 : 2 * (row * x_stride + 8 * g));
+      xo[t] = (NT == 1 ? later : t * walk) * x_step + (out.x_tiled ? (g * side + row) * 16 : ES * row * x_stride + 16 * g);
     }
   }
   const int s_last = min(s_beg + max(mine, 1), walk) - 1;
@@ -142,7 +165,7 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __re
       const int s = min(s_beg + s0 + i, s_last);
 #pragma unroll
       for (int j = 0; j < TW; ++j)
-        wb[i][j] = __builtin_amdgcn_raw_buffer_load_b128(wr, wl, wo[j] + s * 1024, 0);
+        wb[i][j] = __builtin_amdgcn_raw_buffer_load_b128(wr, wo[j], s * w_step, 0);
 #pragma unroll
       for (int t = 0; t < NT; ++t)
         xb[i][t] = __builtin_amdgcn_raw_buffer_load_b128(xr_, xo[t], s * x_step, 0);
@@ -152,18 +175,18 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __re
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
   };
-  floatx4 acc[TW][NT];
+  floatx4 acc[TW][NT][CH];
 #pragma unroll
   for (int j = 0; j < TW; ++j)
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[j][t] = floatx4{0.f, 0.f, 0.f, 0.f};
-  auto step = [&](const uintx4 (&wb)[TW], const uintx4 (&xb)[NT]) {
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int e = 0; e < CH; ++e) acc[j][t][e] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto step = [&](const uintx4 (&wb)[TW], const uintx4 (&xb)[NT], int i) {
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int j = 0; j < TW; ++j)
-        acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wb[j]), __builtin_bit_cast(bf16x8, xb[t]),
-                                                            acc[j][t], 0, 0, 0);
+      for (int j = 0; j < TW; ++j) lr_mma(wb[j], xb[t], acc[j][t], i, T());
   };
   // (whole words: as bfloat16 vectors the compiler puts the halves together again behind each load, and waits for it)
   uintx4 wa[A][TW], xa[A][NT], wb[A][TW], xb[A][NT];
@@ -188,37 +211,46 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __re
   int s = 0;
   for (; mine - s > 2 * A; s += 2 * A) {
 #pragma unroll
-    for (int i = 0; i < A; ++i) step(wa[i], xa[i]);
+    for (int i = 0; i < A; ++i) step(wa[i], xa[i], i);
     __builtin_amdgcn_sched_barrier(0);
     fill(wa, xa, s + 2 * A);
 #pragma unroll
-    for (int i = 0; i < A; ++i) step(wb[i], xb[i]);
+    for (int i = 0; i < A; ++i) step(wb[i], xb[i], i);
     __builtin_amdgcn_sched_barrier(0);
     fill(wb, xb, s + 3 * A);
   }
 #pragma unroll
   for (int i = 0; i < A; ++i)
-    if (s + i < mine) step(wa[i], xa[i]);
+    if (s + i < mine) step(wa[i], xa[i], i);
 #pragma unroll
   for (int i = 0; i < A; ++i)
-    if (s + A + i < mine) step(wb[i], xb[i]);
+    if (s + A + i < mine) step(wb[i], xb[i], i);
 
   // ---- the waves meet: lane (g, c) holds w rows 4 g ... 4 g + 3 of x row c
 #pragma unroll
   for (int j = 0; j < TW; ++j)
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
-      *reinterpret_cast<floatx4*>(&part[((wave * TW + j) * NT + t) * LR_TILE + c * LR_LD + 4 * g]) = acc[j][t];
+    for (int t = 0; t < NT; ++t) {
+#pragma unroll
+      for (int d = CH / 2; d > 0; d >>= 1)                       // (the chains, in pairs)
+#pragma unroll
+        for (int e = 0; e < d; ++e) acc[j][t][e] += acc[j][t][e + d];
+      *reinterpret_cast<floatx4*>(&part[((wave * TW + j) * NT + t) * LR_TILE + c * LR_LD + 4 * g]) = acc[j][t][0];
+    }
   fl_lds_barrier();
-  auto sum_of = [&](int j, int t, int xc, int r) {               // in a fixed order
-    float v = 0.f;
+  auto sum_of = [&](int j, int t, int xc, int r) {               // in pairs
+    float v[NW];
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
       const float* of = part + ((w * TW + j) * NT + t) * LR_TILE + xc * LR_LD + r;
-      v += of[0];
-      if (SPLIT) v += NT == 1 ? of[8 * LR_LD + 8] : of[LR_TILE + 8];       // the second half of K
+      v[w] = of[0];
+      if (SPLIT) v[w] += NT == 1 ? of[8 * LR_LD + 8] : of[LR_TILE + 8];    // the second half of K
     }
-    return v;
+#pragma unroll
+    for (int d = NW / 2; d > 0; d >>= 1)
+#pragma unroll
+      for (int w = 0; w < d; ++w) v[w] += v[w + d];
+    return v[0];
   };
   if (EP == FL_RESID) {
     const int col = group * 16 + 8 * half_tile + tid % RC;
@@ -231,7 +263,7 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __re
       if (live) {
         x = res_old[u] + sum_of(0, SPLIT ? 0 : r / 16, r % 16, tid % RC);
         out.resid[(long)xr * m + col] = x;
-        reinterpret_cast<bf16_t*>(out.y)[rows_at(out.y_tiled ? min(n, 16) : 0, xr, col, m)] = from_f32<bf16_t>(x * res_w);
+        reinterpret_cast<T*>(out.y)[rows_at(out.y_tiled ? min(n, 16) : 0, xr, col, m)] = from_f32<T>(x * res_w);
       }
       const float ss = parts_sum<RC>(x * x);
       if (tid % RC == 0 && r < 16 * NT && xr < n) out.ss_out[(long)xr * stride + (SPLIT ? (int)blockIdx.x : group)] = ss;
@@ -252,7 +284,7 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __re
           a_pos = softplus_f32(out.norm_w[0]);
           a_neg = softplus_f32(out.norm_w[1]);
         }
-        reinterpret_cast<bf16_t*>(out.y)[(long)xr * m + col] = from_f32<bf16_t>(unary_act(v, out.act - FL_UNARY, a_pos, a_neg));
+        reinterpret_cast<T*>(out.y)[(long)xr * m + col] = from_f32<T>(unary_act(v, out.act - FL_UNARY, a_pos, a_neg));
       } else {
         reinterpret_cast<float*>(out.y)[(long)xr * m + col] = v;
       }
@@ -272,10 +304,10 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __re
         b *= row_scale[r];
       }
       if (EP == FL_SWIGLU) {
-        reinterpret_cast<bf16_t*>(out.y)[rows_at(out.y_tiled ? min(n, 16) : 0, xr, pair, pairs)] = from_f32<bf16_t>(gate_act(a, out.act) * b);
+        reinterpret_cast<T*>(out.y)[rows_at(out.y_tiled ? min(n, 16) : 0, xr, pair, pairs)] = from_f32<T>(gate_act(a, out.act) * b);
       } else {
         const int e = EP == FL_ROPE ? u : 0;
-        fl_rope_store<bf16_t>(out, xr, pair, a, b, ep_cos[e], ep_sin[e], ep_page[e], out.cache ? ep_pos[e] % out.page_size : 0);
+        fl_rope_store<T>(out, xr, pair, a, b, ep_cos[e], ep_sin[e], ep_page[e], out.cache ? ep_pos[e] % out.page_size : 0);
       }
     };
     if (EP == FL_ROPE) {
@@ -290,54 +322,54 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const bf16_t* __re
 
 static size_t lr_lds_bytes(int nt, int tw, int nw) { return (size_t)(nw * tw * nt * LR_TILE + LR_ROWS) * sizeof(float); }
 
-template <int NT, int TW, int EP, bool SCALED, int NW, bool SPLIT = false>
+template <typename T, int NT, int TW, int EP, bool SCALED, int NW, bool SPLIT = false>
 static int lr_launch_waves(const void* x, const FlOut& out, const void* w, int n, int m, int k, int tiles, int halves,
                      int x_stride, hipStream_t stream) {
   const size_t lds = lr_lds_bytes(NT, TW, NW);
   if (lds > 64 * 1024) {
-    static const hipError_t e = hipFuncSetAttribute((const void*)linear_rows_kernel<NT, TW, EP, SCALED, NW, SPLIT>,
+    static const hipError_t e = hipFuncSetAttribute((const void*)linear_rows_kernel<T, NT, TW, EP, SCALED, NW, SPLIT>,
                                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     if (e != hipSuccess) KLLM_FAIL((int)e, "linear_rows: cannot raise the LDS limit: %s", hipGetErrorString(e));
   }
   const int groups = ceil_div(tiles, TW);
   const int blocks = SPLIT ? 2 * groups : halves == 1 ? groups : ceil_div(groups, 8) * 16;
-  hipLaunchKernelGGL((linear_rows_kernel<NT, TW, EP, SCALED, NW, SPLIT>), dim3(blocks), dim3(64 * NW), lds, stream,
-                     (const bf16_t*)x, out, (const bf16_t*)w, n, m, k, tiles, halves, x_stride);
+  hipLaunchKernelGGL((linear_rows_kernel<T, NT, TW, EP, SCALED, NW, SPLIT>), dim3(blocks), dim3(64 * NW), lds, stream,
+                     (const T*)x, out, (const T*)w, n, m, k, tiles, halves, x_stride);
   return 0;
 }
 
-template <int NT, int TW, int EP, bool SCALED>
+template <typename T, int NT, int TW, int EP, bool SCALED>
 static int lr_launch(const void* x, const FlOut& out, const void* w, int n, int m, int k, int tiles, int halves,
                      int x_stride, hipStream_t stream) {
   // Four waves a workgroup where a CU has several of them (4,096 -> 6,144: 14.7 us with eight, 13.3 with four), eight where it
   // has one (a step of one token at 1.1B sizes 0.3 % shorter, of 64 tokens 1.2 %).
-  if constexpr ((EP != FL_SWIGLU && EP != FL_PARTS) || TW == 3)
+  if constexpr ((EP != FL_SWIGLU && EP != FL_PARTS) || (TW == 3 && sizeof(T) == 2))
     if ((long)halves * ceil_div(tiles, TW) > device_cus())
-      return lr_launch_waves<NT, TW, EP, SCALED, 4>(x, out, w, n, m, k, tiles, halves, x_stride, stream);
-  return lr_launch_waves<NT, TW, EP, SCALED, 8>(x, out, w, n, m, k, tiles, halves, x_stride, stream);
+      return lr_launch_waves<T, NT, TW, EP, SCALED, 4>(x, out, w, n, m, k, tiles, halves, x_stride, stream);
+  return lr_launch_waves<T, NT, TW, EP, SCALED, 8>(x, out, w, n, m, k, tiles, halves, x_stride, stream);
 }
 
-template <int NT, int TW>
+template <typename T, int NT, int TW>
 static int lr_launch_ep(int ep, bool scaled, const void* x, const FlOut& out, const void* w, int n, int m, int k,
                         int tiles, int halves, int xs, hipStream_t st) {
   if (ep == FL_SWIGLU)
-    return scaled ? lr_launch<NT, TW, FL_SWIGLU, true>(x, out, w, n, m, k, tiles, halves, xs, st)
-                  : lr_launch<NT, TW, FL_SWIGLU, false>(x, out, w, n, m, k, tiles, halves, xs, st);
-  if (ep == FL_PARTS) return lr_launch<NT, TW, FL_PARTS, false>(x, out, w, n, m, k, tiles, halves, xs, st);
+    return scaled ? lr_launch<T, NT, TW, FL_SWIGLU, true>(x, out, w, n, m, k, tiles, halves, xs, st)
+                  : lr_launch<T, NT, TW, FL_SWIGLU, false>(x, out, w, n, m, k, tiles, halves, xs, st);
+  if (ep == FL_PARTS) return lr_launch<T, NT, TW, FL_PARTS, false>(x, out, w, n, m, k, tiles, halves, xs, st);
   if constexpr (TW == 1) {
-    if (ep == FL_RESID) return lr_launch<NT, 1, FL_RESID, false>(x, out, w, n, m, k, tiles, halves, xs, st);
-    return scaled ? lr_launch<NT, 1, FL_ROPE, true>(x, out, w, n, m, k, tiles, halves, xs, st)
-                  : lr_launch<NT, 1, FL_ROPE, false>(x, out, w, n, m, k, tiles, halves, xs, st);
+    if (ep == FL_RESID) return lr_launch<T, NT, 1, FL_RESID, false>(x, out, w, n, m, k, tiles, halves, xs, st);
+    return scaled ? lr_launch<T, NT, 1, FL_ROPE, true>(x, out, w, n, m, k, tiles, halves, xs, st)
+                  : lr_launch<T, NT, 1, FL_ROPE, false>(x, out, w, n, m, k, tiles, halves, xs, st);
   }
   KLLM_FAIL(ERR_STATE, "linear_rows: no kernel for output kind %d and %d tiles", ep, TW);
 }
 
-template <int NT>
+template <typename T, int NT>
 static int lr_launch_tw(int tw, int ep, bool scaled, const void* x, const FlOut& out, const void* w, int n, int m, int k,
                         int tiles, int halves, int xs, hipStream_t st) {
-  if (tw == 1) return lr_launch_ep<NT, 1>(ep, scaled, x, out, w, n, m, k, tiles, halves, xs, st);
-  if (tw == 2) return lr_launch_ep<NT, 2>(ep, scaled, x, out, w, n, m, k, tiles, halves, xs, st);
-  return lr_launch_ep<NT, 3>(ep, scaled, x, out, w, n, m, k, tiles, halves, xs, st);
+  if (tw == 1) return lr_launch_ep<T, NT, 1>(ep, scaled, x, out, w, n, m, k, tiles, halves, xs, st);
+  if (tw == 2) return lr_launch_ep<T, NT, 2>(ep, scaled, x, out, w, n, m, k, tiles, halves, xs, st);
+  return lr_launch_ep<T, NT, 3>(ep, scaled, x, out, w, n, m, k, tiles, halves, xs, st);
 }
 
 }  // namespace kllm
@@ -360,19 +392,21 @@ extern "C" int kllm_linear_rows(const void* x, int x_stride, const KllmLinearOut
   KLLM_REQUIRE(x && yout && w && yout->y, "linear_rows: null pointer");
   const int ep = yout->kind;
   KLLM_REQUIRE(ep == FL_PARTS || ep == FL_RESID || ep == FL_SWIGLU || ep == FL_ROPE, "linear_rows: unknown output kind %d", ep);
-  KLLM_REQUIRE(n > 0 && n <= LR_ROWS, "linear_rows: n=%d is outside [1, %d]", n, LR_ROWS);
+  const bool f32 = yout->f32 != 0;
+  KLLM_REQUIRE(n > 0 && n <= (f32 ? 16 : LR_ROWS), "linear_rows: n=%d is outside [1, %d]", n, f32 ? 16 : LR_ROWS);
   KLLM_REQUIRE(m > 0 && k > 0 && k % 32 == 0, "linear_rows: bad sizes m=%d k=%d (K must be a multiple of 32)", m, k);
   KLLM_REQUIRE(k <= (1 << 20) && m < (1 << 30), "linear_rows: sizes overflow");
-  KLLM_REQUIRE(yout->tiled && !yout->f32 && yout->nsplit <= 1,
-               "linear_rows: takes bfloat16, the tiled copy of the weights and all of K");
+  KLLM_REQUIRE((yout->tiled || f32) && yout->nsplit <= 1, "linear_rows: takes the tiled copy of the weights and all of K");
+  KLLM_REQUIRE(yout->tiled || (long)m * k < (1L << 29), "linear_rows: %d x %d weights need their tiled copy", m, k);
+  KLLM_REQUIRE(!f32 || (!yout->x_tiled && !yout->y_tiled), "linear_rows: tiled rows are bfloat16");
   KLLM_REQUIRE((((uintptr_t)x | (uintptr_t)w) & 15) == 0, "linear_rows: operands must be 16-byte aligned");
   if (x_stride <= 0) x_stride = k;
-  KLLM_REQUIRE(x_stride >= k && x_stride % 8 == 0 && x_stride < (1 << 23), "linear_rows: row stride %d of x does not fit K=%d",
+  KLLM_REQUIRE(x_stride >= k && x_stride % (f32 ? 4 : 8) == 0 && x_stride < (1 << 23), "linear_rows: row stride %d of x does not fit K=%d",
                x_stride, k);
   FlOut out = {};
   out.y = yout->y;
   out.act = yout->act;
-  out.tiled = 1;
+  out.tiled = yout->tiled ? 1 : 0;
   out.x_tiled = yout->x_tiled != 0;
   out.y_tiled = yout->y_tiled != 0;
   KLLM_REQUIRE(!out.y_tiled || (ep == FL_RESID && m % 32 == 0) || (ep == FL_SWIGLU && m % 64 == 0),
@@ -431,6 +465,7 @@ extern "C" int kllm_linear_rows(const void* x, int x_stride, const KllmLinearOut
   int tw = 1;
   if (ep == FL_SWIGLU || ep == FL_PARTS)
     while (tw < 3 && ceil_div(tiles, tw) > cus) ++tw;
+  if (f32 && tiles > 3 * cus) tw = 1;      // (many rounds: whole ones of one tile, two workgroups a CU; 8B sizes, 2 tokens 6,519 -> 6,166 us a step)
   const int row_tiles = ceil_div(n, 16);
   // Halves of the rows where the busiest CU then has fewer tiles of rows to take (or as many, of workgroups that share it
   // anyway): 64 rows against 2,048 x 5,632 (128 tiles) 17.6 -> 12.2 us, 6,144 x 4,096 (384) 25.4 -> 21.2, 48 rows 21.3 -> 18.8; not
@@ -438,14 +473,17 @@ extern "C" int kllm_linear_rows(const void* x, int x_stride, const KllmLinearOut
   const int whole = ceil_div(tiles, cus) * row_tiles, halved = ceil_div(2L * tiles, cus) * ceil_div(row_tiles, 2);
   const int halves = ep != FL_SWIGLU && tw == 1 && (halved < whole || (halved == whole && tiles > cus)) ? 2 : 1;
   const int nt = ceil_div(row_tiles, halves);
-#define KLLM_LRS(NT, EP) lr_launch_waves<NT, 1, EP, false, 8, true>(x, out, w, n, m, k, tiles, 1, x_stride, stream)
+#define KLLM_LRS(NT, EP)                                                                                        \
+  (f32 ? lr_launch_waves<float, NT, 1, EP, false, 8, true>(x, out, w, n, m, k, tiles, 1, x_stride, stream)      \
+       : lr_launch_waves<bf16_t, NT, 1, EP, false, 8, true>(x, out, w, n, m, k, tiles, 1, x_stride, stream))
   const bool split = (ep == FL_RESID || ep == FL_PARTS) && lr_split(n, m, k);
   const int rc = split     ? (ep == FL_RESID ? (n <= 8 ? KLLM_LRS(1, FL_RESID) : KLLM_LRS(2, FL_RESID))
                                              : (n <= 8 ? KLLM_LRS(1, FL_PARTS) : KLLM_LRS(2, FL_PARTS)))
-               : nt == 1 ? lr_launch_tw<1>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream)
-               : nt == 2 ? lr_launch_tw<2>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream)
-               : nt == 3 ? lr_launch_tw<3>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream)
-                         : lr_launch_tw<4>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream);
+               : f32     ? lr_launch_tw<float, 1>(tw, ep, scaled, x, out, w, n, m, k, tiles, 1, x_stride, stream)
+               : nt == 1 ? lr_launch_tw<bf16_t, 1>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream)
+               : nt == 2 ? lr_launch_tw<bf16_t, 2>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream)
+               : nt == 3 ? lr_launch_tw<bf16_t, 3>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream)
+                         : lr_launch_tw<bf16_t, 4>(tw, ep, scaled, x, out, w, n, m, k, tiles, halves, x_stride, stream);
 #undef KLLM_LRS
   if (rc) return rc;
   KLLM_CHECK_LAUNCH("linear_rows");

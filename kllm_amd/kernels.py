@@ -1008,7 +1008,9 @@ def linear_rows_best(kind, n, m, k, dtype=torch.bfloat16, tiled_x=True) -> bool:
     in slices and the norm that adds them; 4,096 x 4,096 at 48 rows 390 KB, 16.4 against 15 (17 / 32 / 48 / 64 tokens at 1.1B
     sizes 1,201 / 1,377 / 1,559 / 1,663 against 1,067 / 1,155 / 1,246 / 1,370; with all products at 8B sizes 64 tokens
     4,902 against 6,146)."""
-    if dtype != torch.bfloat16 or not 1 <= n <= LINEAR_ROWS_MAX or k % 32 or k > 1 << 20:
+    if not 1 <= n <= (LINEAR_ROWS_MAX if dtype == torch.bfloat16 else 16) or k % 32 or k > 1 << 20:
+        return False
+    if dtype == torch.float32 and m * k >= 1 << 29:        # (2 GiB: only the tiled copy could be read, and there may be none)
         return False
     if kind == LINEAR_RESID and linear_rows_parts(n, m, k) == 0:
         return False
@@ -1021,10 +1023,10 @@ def linear_rows_best(kind, n, m, k, dtype=torch.bfloat16, tiled_x=True) -> bool:
 
 
 def linear_rows(w, y, kind, x, rope=None, act=ACT_SILU, resid=None, norm_weight=None, ss_out=None, unary=None):
-    """``fused_linear`` for up to 64 rows of bfloat16, K a multiple of 32, in one slice,
-    from the tiled copy ``w`` of the weights, nothing staged in LDS.  ``x`` (also inside a ``ScaledRows``) may be
+    """``fused_linear`` for up to 64 rows of bfloat16 or 16 of float32, K a multiple of 32, in one slice,
+    from the tiled copy ``w`` of the weights (float32: or from the matrix, with the same bits), nothing staged in LDS.  ``x`` (also inside a ``ScaledRows``) may be
     ``TiledRows``, and so may ``y`` of LINEAR_RESID and LINEAR_SWIGLU."""
-    if not isinstance(w, TiledWeights):
+    if not isinstance(w, TiledWeights) and w.dtype != torch.float32:
         raise KernelError("linear_rows: takes the tiled copy of the weights")
     fused_linear(w, y, kind, x, rope=rope, act=act, resid=resid, norm_weight=norm_weight, ss_out=ss_out, unary=unary, _rows=True)
 
@@ -1063,7 +1065,7 @@ def fused_linear(w, y, kind, x, nsplit=1, tiles_per_wg=1, rope=None, act=ACT_SIL
     lo.kind, lo.nsplit, lo.act = kind, nsplit, int(act)
     for name, t in (("x", x), ("y", y)):
         if isinstance(t, TiledRows):
-            if (not _rows or (name == "y" and kind in (LINEAR_ROPE, LINEAR_PARTS)) or t.dtype != typ or not t.data.is_contiguous()
+            if (not _rows or typ != torch.bfloat16 or (name == "y" and kind in (LINEAR_ROPE, LINEAR_PARTS)) or t.dtype != typ or not t.data.is_contiguous()
                     or t.shape[1] % 32 or t.data.shape[0] != TiledRows.stored(n) or (name == "x" and t.shape[1] != k)):
                 raise KernelError(f"linear_rows: tiled rows {t.shape} do not fit {name}, or the kernel takes none")
     if isinstance(x, TiledRows):

@@ -238,7 +238,7 @@ class CausalSelfAttention(Part):
                                cache.block_table, cache.page_size, self.heads, self.kv_heads,
                                self.head_dim)
         elif self._rows(n, xn):
-            K.linear_rows(self._tiled["in"], q, K.LINEAR_ROPE, xn,
+            K.linear_rows(self._tiled.get("in") or self.w_in, q, K.LINEAR_ROPE, xn,
                           rope=K.Rope(cos, sin, pages, ctx.positions, ctx.span_of_token, cache.block_table,
                                       cache.page_size, self.heads, self.kv_heads, self.head_dim))
         elif self._fused_tiles(n) > 0:

@@ -87,7 +87,7 @@ class GatedFeedForward(Part):
         if gemv:
             K.gemv_swiglu(xn, self.w_gu, h, self.act)   # few tokens: both products and the gate in one launch
         elif rows:
-            K.linear_rows(self._tiled["gu"], h, K.LINEAR_SWIGLU, xn, act=self.act)
+            K.linear_rows(self._tiled.get("gu") or self.w_gu, h, K.LINEAR_SWIGLU, xn, act=self.act)
         elif fused:
             # a decode batch: the same on the matrix cores
             K.fused_linear(self._tiled.get("gu") or self.w_gu, h, K.LINEAR_SWIGLU, x=xn, act=self.act,

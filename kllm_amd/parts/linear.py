@@ -180,22 +180,24 @@ def tiled_copy(runtime, w, kind, rope=None):
 
 
 def fused_f32(rt, n):
-    """Whether a float32 decode batch of n tokens runs on the decode-batch kernel: up to four rows the
-    gemv with the same epilogues has the rows in registers and is the faster one (a step in ms, gemv
-    against this kernel, of 3 / 4 tokens at 1.1B sizes: 1.69 against 1.68, 1.70 against 1.64; of 4 at 8B sizes:
-    6.70 against 6.97); from five on its work per weight grows with the rows and the matrix cores' does not
-    (5 / 8 tokens at 1.1B sizes: 2.07 against 1.73, 2.14 against 1.70; 8 at 8B sizes: 8.41 against 7.82), and
-    from nine on K went in slices whose sums other kernels added (10 / 16 tokens: 2.93 against 1.66, 3.06
-    against 1.83; 16 at 8B sizes: 14.6 against 9.7)."""
+    """Whether a float32 decode batch of n tokens runs on the matrix cores, with the step after a product in its launch
+    (``K.linear_rows``, or the decode-batch kernel for sizes that one does not take).  One row stays with the gemv, which has the same epilogues
+    and the row in registers (a step in us, gemv against the matrix cores, of 1 / 2 / 4 tokens at 1.1B sizes: 1,436 / 1,516 / 1,708
+    against 1,381 / 1,404 / 1,434, without room for the copies of the weights 2 / 4 tokens 1,535 / 1,723 against 1,494 / 1,495; at 8B
+    sizes 6,103 / 6,262 / 6,610 against 6,392 / 6,166 / 6,197).  Its work per weight grows with the rows and the matrix cores' does
+    not, and from nine on K went in slices whose sums other kernels added (16 at 8B sizes: 14.6 ms against 9.7 on the
+    decode-batch kernel; 12: 9.1 there, 7.0 now)."""
     opts = rt.options
-    return (5 <= n <= 16 and not opts.get("no_fused_linear") and not opts.get("no_mfma_f32")
+    return (2 <= n <= 16 and not opts.get("no_fused_linear") and not opts.get("no_mfma_f32")
             and opts.get("gemm_algo") is None)
 
 
 def rows_kernel(rt, kind, n, w, w_tiled, tiled_x):
     """Whether a product of n rows (``TiledRows``: ``tiled_x``) with the step after it runs on ``K.linear_rows``."""
-    return (w_tiled is not None and not rt.options.get("no_fused_linear") and rt.options.get("gemm_algo") is None
-            and rt.options.get("gemm") != "library" and K.linear_rows_best(kind, n, w.shape[0], w.shape[1], w_tiled.dtype, tiled_x))
+    f32 = w.dtype == torch.float32
+    return ((fused_f32(rt, n) if f32 else w_tiled is not None and rt.options.get("gemm") != "library")
+            and not rt.options.get("no_fused_linear") and rt.options.get("gemm_algo") is None
+            and K.linear_rows_best(kind, n, w.shape[0], w.shape[1], w.dtype, tiled_x))
 
 
 def _sink_fits(rt, sink, n, m):
@@ -207,7 +209,7 @@ def _sink_fits(rt, sink, n, m):
 def _feeds_rows(norm, n):
     """Whether the product behind ``norm`` runs on ``K.linear_rows`` and reads ``TiledRows``."""
     feeds = getattr(norm, "feeds", None)
-    return feeds is not None and K.linear_rows_best(feeds[0], n, feeds[1], feeds[2])
+    return feeds is not None and norm.runtime.dtype == torch.bfloat16 and K.linear_rows_best(feeds[0], n, feeds[1], feeds[2])
 
 
 def _resid_rows(rt, norm, n, w, w_tiled, tiled_x):
@@ -218,7 +220,7 @@ def _resid_rows(rt, norm, n, w, w_tiled, tiled_x):
 
 def sink_takes_rows(rt, sink, n, w, w_tiled):
     """Whether ``linear_into`` will run the product of ``TiledRows`` on ``K.linear_rows``."""
-    return sink is not None and _sink_fits(rt, sink, n, w.shape[0]) and _resid_rows(rt, sink.norm, n, w, w_tiled, True)
+    return sink is not None and w.dtype == torch.bfloat16 and _sink_fits(rt, sink, n, w.shape[0]) and _resid_rows(rt, sink.norm, n, w, w_tiled, True)
 
 
 def linear_into(ctx, x, w, sink, tag, w_tiled=None):
@@ -249,7 +251,7 @@ def linear_into(ctx, x, w, sink, tag, w_tiled=None):
             xw = K.TiledRows(ctx.buf(tag + ".xw", (K.TiledRows.stored(n), m), x.dtype), n)     # for the product behind the norm
         else:
             xw = ctx.buf(tag + ".xw", (n, m), x.dtype)
-        K.linear_rows(w_tiled, xw, K.LINEAR_RESID, x, resid=sink.x, norm_weight=norm.weight, ss_out=ss)
+        K.linear_rows(w_tiled or w, xw, K.LINEAR_RESID, x, resid=sink.x, norm_weight=norm.weight, ss_out=ss)
         return Normed(sink.x, ss, parts, norm, xw=xw)
     if not (fused_f32(rt, n) if f32 else n <= K.FUSED_NORM_BEST_ROWS) or rt.options.get("no_fused_linear"):
         return None
@@ -340,7 +342,7 @@ def decode_linear(ctx, x, w, tag, w_tiled=None, unary=None):
     rt = ctx.runtime
     if parts_rows(rt, n, w, w_tiled):
         y = ctx.buf(tag, (n, m) if unary is not None else (1, n, m), x.dtype if unary is not None else torch.float32)
-        K.linear_rows(w_tiled, y, K.LINEAR_PARTS, x, unary=unary)
+        K.linear_rows(w_tiled or w, y, K.LINEAR_PARTS, x, unary=unary)
         return y if unary is not None else y[0]
     if decode_batch_fits(rt, x) and not rt.options.get("no_fused_linear") and rt.options.get("gemm_algo") is None:
         tiles = 4 if m >= 16384 else 1

@@ -195,3 +195,56 @@ def test_attention_writes_tiled_rows(H, KV, hd, ps, slices):
                     k_.attn_prefill(q, o, cache, tiles, len(spans), start, span_pos, bt, ps, H, KV, hd, 0, hd ** -0.5,
                                     keys, keys)
                 assert torch.equal(_rowwise(tiled), out)
+
+
+@pytest.mark.parametrize("n,m,k", [(5, 64, 64), (8, 2048, 2048), (8, 2048, 5632), (13, 72, 448), (16, 2048, 5632), (16, 4096, 4096),
+                                   (7, 4096, 1056), (1, 40, 32)])
+def test_float32(n, m, k):
+    """True 32-bit products and the steps after them: sums as close to 64 bits as the decode-batch kernel's."""
+    k_, f32, eps = K(), torch.float32, 1e-5
+    x, w = rnd(n, k, seed=1, scale=0.5), rnd(m, k, seed=2, scale=0.1)
+    tiled = k_.fused_linear_tile(w, k_.LINEAR_PARTS)
+    want = x.double() @ w.double().T
+    y, y2 = torch.full((1, n, m), float("nan"), device=DEV), torch.empty(1, n, m, device=DEV)
+    k_.linear_rows(tiled, y, k_.LINEAR_PARTS, x)
+    k_.fused_linear(tiled, y2, k_.LINEAR_PARTS, x)
+    k_.linear_rows(w, y3 := torch.empty_like(y), k_.LINEAR_PARTS, x)
+    assert torch.equal(y3, y)                       # from the matrix itself
+    # products of 0.5 x 0.1 added k at a time: 32-bit chains of at most k / 64 and 64 of them in a tree
+    bound = 0.05 * k ** 0.5 * 2.0 ** -24 * 8
+    assert (y[0].double() - want).norm() <= 1.1 * (y2[0].double() - want).norm() + 1e-12
+    assert (y[0].double() - want).abs().max() < 6 * bound + 1e-7
+    resid, nw = rnd(n, m, seed=3, scale=2.0), 1 + 0.2 * rnd(m, seed=4)
+    parts = k_.linear_rows_parts(n, m, k)
+    ss = torch.full((n, -(-parts // 4) * 4), float("nan"), device=DEV)
+    stream, xw = resid.clone(), torch.empty(n, m, device=DEV)
+    k_.linear_rows(tiled, xw, k_.LINEAR_RESID, x, resid=stream, norm_weight=nw, ss_out=ss)
+    want_x = resid.double() + want
+    assert (stream.double() - want_x).abs().max() < 6 * bound + 1e-6
+    assert torch.equal(xw, stream * nw)
+    k_.linear_rows(w, xw, k_.LINEAR_RESID, x, resid=(stream2 := resid.clone()), norm_weight=nw, ss_out=ss)
+    assert torch.equal(stream2, stream)
+    assert ((ss[:, :parts].double().sum(1) - (want_x ** 2).sum(1)).abs() / (want_x ** 2).sum(1)).max() < 1e-5
+    if m % 32:
+        return
+    want_n, sr = P.rmsnorm(want_x, nw.double(), eps), k_.ScaledRows(xw, ss, parts, eps)
+    for f in (40, 2056, 3080):
+        wg = rnd(2 * f, m, seed=5, scale=0.1)
+        h = torch.full((n, f), float("nan"), device=DEV)
+        k_.linear_rows(k_.fused_linear_tile(wg, k_.LINEAR_SWIGLU), h, k_.LINEAR_SWIGLU, sr)
+        k_.linear_rows(wg, h2 := torch.empty_like(h), k_.LINEAR_SWIGLU, sr)
+        assert torch.equal(h2, h)
+        g = want_n @ wg[:f].double().T
+        assert ((h.double() - g * torch.sigmoid(g) * (want_n @ wg[f:].double().T)).abs().max()
+                < 1e-5 * (g.abs().max() ** 2 + 1))
+    H, hd = 2, 16
+    wq = rnd(H * hd, m, seed=6, scale=0.1)
+    pos = torch.arange(5, 5 + n, dtype=torch.int32, device=DEV)
+    cos, sin = torch.empty(n, hd // 2, device=DEV), torch.empty(n, hd // 2, device=DEV)
+    k_.rope_tables(cos, sin, pos, hd, 10000.0)
+    rope, q = k_.Rope(cos, sin, None, None, None, None, 16, H, 1, hd), torch.full((n, H * hd), float("nan"), device=DEV)
+    k_.linear_rows(k_.fused_linear_tile(wq, k_.LINEAR_ROPE, rope), q, k_.LINEAR_ROPE, sr, rope=rope)
+    k_.linear_rows(wq, q2 := torch.empty_like(q), k_.LINEAR_ROPE, sr, rope=rope)
+    assert torch.equal(q2, q)
+    want_q = P.rope((want_n @ wq.double().T).cpu(), pos.cpu().tolist(), H, hd, 10000.0)
+    assert (q.cpu().double() - want_q).abs().max() < 1e-5 * (want_q.abs().max() + 1)
