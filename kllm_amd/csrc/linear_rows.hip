@@ -465,7 +465,9 @@ extern "C" int kllm_linear_rows(const void* x, int x_stride, const KllmLinearOut
   int tw = 1;
   if (ep == FL_SWIGLU || ep == FL_PARTS)
     while (tw < 3 && ceil_div(tiles, tw) > cus) ++tw;
-  if (f32 && tiles > 3 * cus) tw = 1;      // (many rounds: whole ones of one tile, two workgroups a CU; 8B sizes, 2 tokens 6,519 -> 6,166 us a step)
+  // Many rounds: one tile, whose rounds are whole (2 x 14,336 columns: seven, where three tiles are 2.3) and of which a CU holds two workgroups
+  // (a step at 8B sizes, 1 / 8 / 16 tokens 3,298 / 3,568 / 3,833 us with three, 3,146 / 3,407 / 3,694 with one; float32, 2 tokens 6,519, 6,166).
+  if (tiles > 3 * cus) tw = 1;
   const int row_tiles = ceil_div(n, 16);
   // Halves of the rows where the busiest CU then has fewer tiles of rows to take (or as many, of workgroups that share it
   // anyway): 64 rows against 2,048 x 5,632 (128 tiles) 17.6 -> 12.2 us, 6,144 x 4,096 (384) 25.4 -> 21.2, 48 rows 21.3 -> 18.8; not

@@ -1017,8 +1017,9 @@ def linear_rows_best(kind, n, m, k, dtype=torch.bfloat16, tiled_x=True) -> bool:
     if n <= 16:
         return True
     tiles, cus, row_tiles = -(-m // 16), device_cus(), -(-n // 16)
-    busiest = -(-tiles // (3 * cus)) * row_tiles if kind == LINEAR_SWIGLU or (kind == LINEAR_PARTS and tiles > cus) else min(
-        -(-tiles // cus) * row_tiles, -(-2 * tiles // cus) * -(-row_tiles // 2))
+    busiest = ((1 if tiles <= 3 * cus else -(-tiles // cus)) * row_tiles
+               if kind == LINEAR_SWIGLU or (kind == LINEAR_PARTS and tiles > cus) else min(
+        -(-tiles // cus) * row_tiles, -(-2 * tiles // cus) * -(-row_tiles // 2)))
     return 32 * k * busiest * (1 if tiled_x else 2) <= LINEAR_ROWS_BYTES
 
 
