@@ -1,4 +1,4 @@
-// What the decode-batch products (fused_linear.hip) and the products of 17 to 64 rows
+// What the decode-batch products (fused_linear.hip) and the products of up to 64 rows without staging
 // (linear_rows.hip) share: the output's description, its kinds and the rotation's stores.
 #pragma once
 

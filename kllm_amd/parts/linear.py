@@ -3,12 +3,12 @@
 ``linear`` computes x . w^T for x [n, k] and w [m, k].  With a float32 result
 it returns partial sums [nsplit, n, m] that the consuming kernel adds (norm,
 rotary + append, SiLU gate); with the compute dtype as result it returns
-[n, m].  Which kernel runs depends only on the dtype and on n:
+[n, m].  Which kernel runs depends only on the dtype and on n (products with the step after
+them in their launch, and ``decode_linear``, have the tiled copy of the weights and go to ``K.linear_rows``
+first: up to 64 rows of bfloat16, 2 to 16 of float32, see ``K.linear_rows_best``):
 
-  (a product whose epilogue does the step after it, up to 64 rows of bfloat16: ``K.linear_rows``)
   n <= 8    float32: gemv with X in LDS and the whole of K in one wave (no
-            partial sums), if the sizes fit, and from five rows on the decode-batch kernel
-            (``fused_f32``) where its epilogue or one whole result is wanted; bfloat16 up to 4 rows: the streaming
+            partial sums), if the sizes fit; bfloat16 up to 4 rows: the streaming
             gemv, K cut into slices for long rows (measured faster than the
             former for a plain product; the fused epilogues are another matter)
   float32   else: MFMA tiles with 32-bit operands (true 32-bit; K in slices for
@@ -169,8 +169,8 @@ def tiled_copy(runtime, w, kind, rope=None):
     does not take, or ``EngineOptions.extra["no_tiled_weights"]`` (the copies double the
     memory of the weights they are made of; decode batches of 2 to 16 tokens stream them 20 to
     30 % faster than the row-major matrix).  float32: only where the engine found room for all of them behind
-    its cache (``Runtime.second_copies``); without them 5 to 16 tokens at 1.1B sizes take 1.76 to 1.97 ms a step, with
-    them 1.66 to 1.83, and the sums are the same."""
+    its cache (``Runtime.second_copies``); without them 2 / 4 / 8 tokens at 1.1B sizes take 1,494 / 1,495 / 1,562 us a step, with
+    them 1,404 / 1,434 / 1,534, and the sums are the same."""
     if (w is None or not w.is_cuda or w.shape[1] % (4 if w.dtype == torch.float32 else 8)
             or runtime.options.get("no_tiled_weights") or runtime.options.get("no_fused_linear")):
         return None
@@ -333,7 +333,8 @@ def parts_rows(rt, n, w, w_tiled):
 
 
 def decode_linear(ctx, x, w, tag, w_tiled=None, unary=None):
-    """``linear`` for a consumer that takes float32 sums either whole or in slices: decode
+    """``linear`` for a consumer that takes float32 sums either whole or in slices: ``K.linear_rows`` where it is the
+    faster (``parts_rows``); else decode
     batches of up to 16 rows run on the decode-batch kernel with all of K in a workgroup (one
     result, from the tiled copy of w where there is one); everything else as ``linear`` cuts it.
     ``unary`` = (activation without a gate, its constants): only where ``decode_batch_fits`` or ``parts_rows``;

@@ -77,3 +77,23 @@ def test_slices_of_short_contexts_in_float32(n, KV, H, hd, keys, slices):
     """One workgroup's four slices where they are the faster: not for a single tile of keys, nor for two where
     its merge is long or the groups are many."""
     assert K.attn_decode_slices(n, KV, H, hd, F32, keys) == slices
+
+
+@pytest.mark.parametrize("kind,n,m,k,dtype,want", [
+    (K.LINEAR_RESID, 64, 2048, 5632, torch.bfloat16, True), (K.LINEAR_SWIGLU, 64, 11264, 2048, torch.bfloat16, True),
+    (K.LINEAR_ROPE, 64, 2560, 2048, torch.bfloat16, True), (K.LINEAR_RESID, 65, 2048, 5632, torch.bfloat16, False),
+    (K.LINEAR_RESID, 16, 4096, 14336, torch.bfloat16, True), (K.LINEAR_RESID, 17, 4096, 14336, torch.bfloat16, False),
+    (K.LINEAR_SWIGLU, 16, 28672, 4096, torch.bfloat16, True), (K.LINEAR_SWIGLU, 17, 28672, 4096, torch.bfloat16, False),
+    (K.LINEAR_RESID, 8, 4112, 4096, torch.bfloat16, False), (K.LINEAR_RESID, 8, 2048, 2040, torch.bfloat16, False),
+    (K.LINEAR_PARTS, 8, 2048, 2048, torch.float32, True), (K.LINEAR_PARTS, 17, 2048, 2048, torch.float32, False),
+    (K.LINEAR_SWIGLU, 8, 131072, 4096, torch.float32, False)])
+def test_products_without_staging_are_taken_by_size(kind, n, m, k, dtype, want):
+    """256 CUs: up to 16 rows always, beyond while the busiest CU's rows stay below 380 KB; sums of squares for 4,096 columns at
+    most, K in whole steps, float32 weights below 2 GiB (they are read without their copy too)."""
+    assert K.linear_rows_best(kind, n, m, k, dtype) is want
+
+
+def test_half_tiles_of_weights_only_where_half_the_cus_are_idle():
+    assert K.linear_rows_parts(16, 2048, 2048) == 256 and K.linear_rows_parts(17, 2048, 2048) == 128
+    assert K.linear_rows_parts(8, 2064, 2048) == 129 and K.linear_rows_parts(8, 2048, 2080) == 128
+    assert K.linear_rows_parts(8, 4096, 4096) == 256 and K.linear_rows_parts(8, 4112, 4096) == 0
