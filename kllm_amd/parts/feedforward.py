@@ -50,8 +50,9 @@ class GatedFeedForward(Part):
                        "down": tiled_copy(self.runtime, self.w_down, K.LINEAR_PARTS)}
 
     def rows_input(self):
-        """(kind, rows, columns) of the gate and up product, where its tiled copy is there (``K.linear_rows_best``)."""
-        return (K.LINEAR_SWIGLU, *self.w_gu.shape) if self._tiled.get("gu") is not None else None
+        """(kind, rows, columns) of the gate and up product, where ``K.linear_rows`` may take it (``K.linear_rows_best``): in
+        bfloat16 from its tiled copy only."""
+        return (K.LINEAR_SWIGLU, *self.w_gu.shape) if self._tiled.get("gu") is not None or self.w_gu.dtype == torch.float32 else None
 
     def _gate_in_tiles(self, n, dtype):
         """Decode batches whose gate runs in the tiled product's epilogue: more than 32 rows
@@ -68,12 +69,13 @@ class GatedFeedForward(Part):
         dtype, opts = self.runtime.dtype, self.runtime.options
         n = xn.rows if isinstance(xn, Normed) else xn.shape[0]
         gemv = K.gemv_fits(n, 2 * self.intermediate, self.hidden, dtype) and not opts.get("no_fused_gemv")
-        best = fused_f32(self.runtime, n) if dtype == torch.float32 else n <= K.FUSED_SWIGLU_BEST_ROWS
+        best = fused_f32(self.runtime, n, 2 * self.intermediate) if dtype == torch.float32 else n <= K.FUSED_SWIGLU_BEST_ROWS
         tiles = K.fused_linear_tiles(n, 2 * self.intermediate, self.hidden, dtype) if best else 0
-        if gemv and (isinstance(xn, Normed) and xn.xw is not None or dtype == torch.float32 and tiles > 0):
-            gemv = False       # the producer was the decode-batch kernel: its consumer is, too
-        rows = not gemv and rows_kernel(self.runtime, K.LINEAR_SWIGLU, n, self.w_gu, self._tiled.get("gu"),
-                                           isinstance(getattr(xn, "xw", xn), K.TiledRows))
+        rows = rows_kernel(self.runtime, K.LINEAR_SWIGLU, n, self.w_gu, self._tiled.get("gu"),
+                           isinstance(getattr(xn, "xw", xn), K.TiledRows))
+        if gemv and (xn.xw is not None if isinstance(xn, Normed) else dtype == torch.float32 and (rows or tiles > 0)):
+            gemv = False       # the producer was a kernel for decode batches: its consumer is, too
+        rows = rows and not gemv
         fused = not gemv and not rows and tiles > 0 and not opts.get("no_fused_linear")
         if isinstance(xn, Normed):     # the small-batch kernel below normalises while it stages its input,
             # the decode-batch kernel scales its sums by the row
@@ -160,7 +162,7 @@ def dense_hidden(ctx, xn, w_up, tag, tiled, act, params=None):
     if (n > 128 and opts.get("gemm") != "library" and opts.get("gemm_algo") is None
             and xn.shape[1] % (8 if xn.dtype == torch.bfloat16 else 4) == 0):
         K.gemm_act(xn, w_up, h, act, params)      # prompts
-    elif parts_rows(ctx.runtime, n, w_up, tiled) or (decode_batch_fits(ctx.runtime, xn) and not opts.get("no_fused_linear")
+    elif parts_rows(ctx.runtime, n, w_up, tiled) or (decode_batch_fits(ctx.runtime, xn, w_up.shape[0]) and not opts.get("no_fused_linear")
                                                      and opts.get("gemm_algo") is None):
         h = decode_linear(ctx, xn, w_up, tag + ".h", tiled, unary=(act, params))      # decode batches
     else:

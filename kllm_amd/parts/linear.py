@@ -179,17 +179,20 @@ def tiled_copy(runtime, w, kind, rope=None):
     return K.fused_linear_tile(w, kind, rope)
 
 
-def fused_f32(rt, n):
+def fused_f32(rt, n, m=None):
     """Whether a float32 decode batch of n tokens runs on the matrix cores, with the step after a product in its launch
-    (``K.linear_rows``, or the decode-batch kernel for sizes that one does not take).  One row stays with the gemv, which has the same epilogues
+    (``K.linear_rows``, or the decode-batch kernel for sizes that one does not take: ``m``, the product's columns).  One row stays with the
+    gemv, which has the same epilogues
     and the row in registers (a step in us, gemv against the matrix cores, of 1 / 2 / 4 tokens at 1.1B sizes: 1,436 / 1,516 / 1,708
     against 1,381 / 1,404 / 1,434, without room for the copies of the weights 2 / 4 tokens 1,535 / 1,723 against 1,494 / 1,495; at 8B
     sizes 6,103 / 6,262 / 6,610 against 6,392 / 6,166 / 6,197).  Its work per weight grows with the rows and the matrix cores' does
     not, and from nine on K went in slices whose sums other kernels added (16 at 8B sizes: 14.6 ms against 9.7 on the
-    decode-batch kernel; 12: 9.1 there, 7.0 now)."""
+    decode-batch kernel; 12: 9.1 there, 7.0 now).  The decode-batch kernel stages all rows first: two rows stay with the gemv, too, where it
+    has fewer tiles than there are CUs (a step, gemv / decode-batch kernel, 2 / 3 / 4 tokens: width 2,040 x 8 layers 716 / 884 / 896 us against
+    735 / 836 / 850; width 4,112 x 4 layers 896 / 912 / 929 against 864 / 850 / 898)."""
     opts = rt.options
-    return (2 <= n <= 16 and not opts.get("no_fused_linear") and not opts.get("no_mfma_f32")
-            and opts.get("gemm_algo") is None)
+    return (2 <= n <= 16 and (n > 2 or m is None or m >= 16 * K.device_cus()) and not opts.get("no_fused_linear")
+            and not opts.get("no_mfma_f32") and opts.get("gemm_algo") is None)
 
 
 def rows_kernel(rt, kind, n, w, w_tiled, tiled_x):
@@ -214,8 +217,14 @@ def _feeds_rows(norm, n):
 
 def _resid_rows(rt, norm, n, w, w_tiled, tiled_x):
     """Whether a residual product runs on ``K.linear_rows``: beyond 16 rows only where the next product does, too (a step of 32
-    tokens at 8B sizes, whose gate product does not, 4,234 us without and 4,370 with the output projection here)."""
-    return rows_kernel(rt, K.LINEAR_RESID, n, w, w_tiled, tiled_x) and (n <= 16 or _feeds_rows(norm, n))
+    tokens at 8B sizes, whose gate product does not, 4,234 us without and 4,370 with the output projection here); two rows of float32
+    not where the next product stays with the gemv, which makes its rows' norm itself and has no use for scaled ones."""
+    if not rows_kernel(rt, K.LINEAR_RESID, n, w, w_tiled, tiled_x):
+        return False
+    if w.dtype == torch.float32:
+        feeds = getattr(norm, "feeds", None)
+        return feeds is None or fused_f32(rt, n, feeds[1]) or K.linear_rows_best(feeds[0], n, feeds[1], feeds[2], torch.float32)
+    return n <= 16 or _feeds_rows(norm, n)
 
 
 def sink_takes_rows(rt, sink, n, w, w_tiled):
@@ -238,12 +247,13 @@ def linear_into(ctx, x, w, sink, tag, w_tiled=None):
         return None
     norm = sink.norm
     f32 = x.dtype == torch.float32
-    parts = 0 if f32 and fused_f32(rt, n) else K.resid_parts(n, m, k, x.dtype)
+    rows = _resid_rows(rt, norm, n, w, w_tiled, isinstance(x, K.TiledRows))
+    parts = 0 if f32 and (rows or fused_f32(rt, n, m)) else K.resid_parts(n, m, k, x.dtype)
     if parts:
         ss = ctx.buf(tag + ".ss", (n, -(-parts // 4) * 4), torch.float32)
         K.linear_resid(x, w, sink.x, ss)
         return Normed(sink.x, ss, parts, norm)
-    if _resid_rows(rt, norm, n, w, w_tiled, isinstance(x, K.TiledRows)):
+    if rows:
         parts = K.linear_rows_parts(n, m, k)
         stride = -(-parts // 4) * 4          # (room for eight columns to a sum whatever n is: a smaller step must not ask for more)
         ss = ctx.buf(tag + ".ss", (n * max(stride, -(-m // 32) * 4),), torch.float32)[:n * stride].view(n, stride)
@@ -253,7 +263,7 @@ def linear_into(ctx, x, w, sink, tag, w_tiled=None):
             xw = ctx.buf(tag + ".xw", (n, m), x.dtype)
         K.linear_rows(w_tiled or w, xw, K.LINEAR_RESID, x, resid=sink.x, norm_weight=norm.weight, ss_out=ss)
         return Normed(sink.x, ss, parts, norm, xw=xw)
-    if not (fused_f32(rt, n) if f32 else n <= K.FUSED_NORM_BEST_ROWS) or rt.options.get("no_fused_linear"):
+    if not (fused_f32(rt, n, m) if f32 else n <= K.FUSED_NORM_BEST_ROWS) or rt.options.get("no_fused_linear"):
         return None
     # a decode batch on the matrix cores: all of K in a workgroup, the addition in the epilogue, and
     # beside the stream its rows times the norm's weight in the compute dtype for a consumer that scales its sums
@@ -316,11 +326,11 @@ def linear(ctx, x, w, tag, out_dtype=torch.float32, split=True, w_tiled=None):
     return y
 
 
-def decode_batch_fits(rt, x):
-    """Whether a product of these rows runs on the decode-batch kernel (up to 16 rows, all of K
+def decode_batch_fits(rt, x, m):
+    """Whether a product of these rows with m columns runs on the decode-batch kernel (up to 16 rows, all of K
     in a workgroup; float32 see ``fused_f32``)."""
     n, k = x.shape
-    if x.dtype == torch.float32 and not fused_f32(rt, n):
+    if x.dtype == torch.float32 and not fused_f32(rt, n, m):
         return False
     return n <= 16 and K.fused_linear_fits(n, k, 1, x.dtype)
 
@@ -345,7 +355,7 @@ def decode_linear(ctx, x, w, tag, w_tiled=None, unary=None):
         y = ctx.buf(tag, (n, m) if unary is not None else (1, n, m), x.dtype if unary is not None else torch.float32)
         K.linear_rows(w_tiled or w, y, K.LINEAR_PARTS, x, unary=unary)
         return y if unary is not None else y[0]
-    if decode_batch_fits(rt, x) and not rt.options.get("no_fused_linear") and rt.options.get("gemm_algo") is None:
+    if decode_batch_fits(rt, x, m) and not rt.options.get("no_fused_linear") and rt.options.get("gemm_algo") is None:
         tiles = 4 if m >= 16384 else 1
         if unary is not None:
             y = ctx.buf(tag, (n, m), x.dtype)

@@ -6,6 +6,8 @@ import torch
 
 from kllm_amd import kernels as K
 from kllm_amd.engine.engine import room_for_copies
+from kllm_amd.parts import linear as products
+from kllm_amd.parts.base import ResidualSink
 from kllm_amd.parts.linear import choose
 
 BF16, F32 = torch.bfloat16, torch.float32
@@ -97,3 +99,34 @@ def test_half_tiles_of_weights_only_where_half_the_cus_are_idle():
     assert K.linear_rows_parts(16, 2048, 2048) == 256 and K.linear_rows_parts(17, 2048, 2048) == 128
     assert K.linear_rows_parts(8, 2064, 2048) == 129 and K.linear_rows_parts(8, 2048, 2080) == 128
     assert K.linear_rows_parts(8, 4096, 4096) == 256 and K.linear_rows_parts(8, 4112, 4096) == 0
+
+
+class _Recorder:
+    """Stands for the context, the runtime and the norm of a product whose launch is only asked for."""
+
+    def __init__(self, dtype, feeds=None, **options):
+        self.runtime, self.options, self.dtype, self.feeds = self, options, dtype, feeds
+
+    def buf(self, tag, shape, dtype):
+        return torch.empty(shape, dtype=dtype)
+
+
+@pytest.mark.parametrize("n,m,k,feeds,kernel", [
+    (2, 2040, 2040, None, "gemv"), (3, 2040, 2040, None, "decode_batch"), (2, 4112, 4112, None, "decode_batch"),
+    (2, 2048, 5632, (K.LINEAR_ROPE, 2560, 2048), "rows"), (2, 2040, 5632, (K.LINEAR_ROPE, 2856, 2040), "gemv"),
+    (3, 2040, 5632, (K.LINEAR_ROPE, 2856, 2040), "rows"), (2, 2040, 5632, (K.LINEAR_SWIGLU, 11264, 2040), "rows"),
+    (1, 2048, 2048, None, "gemv"), (5, 2040, 2040, None, "decode_batch")])
+def test_few_rows_of_float32_leave_the_gemv_where_that_is_the_faster_way(n, m, k, feeds, kernel, monkeypatch):
+    """Two rows whose K is in no whole steps stay with the gemv unless the decode-batch kernel has a tile for every CU; so do those
+    whose scaled rows the product behind the norm would not take."""
+    went = []
+    monkeypatch.setattr(K, "linear_resid", lambda *a, **b: went.append("gemv"))
+    monkeypatch.setattr(K, "linear_rows", lambda *a, **b: went.append("rows"))
+    monkeypatch.setattr(K, "fused_linear", lambda *a, **b: went.append("decode_batch"))
+    rt = _Recorder(F32, feeds)
+    rt.weight = torch.empty(m)
+    rt.eps = 1e-5
+    x, w = torch.empty(n, k), torch.empty(m, k)
+    normed = products.linear_into(rt, x, w, ResidualSink(torch.empty(n, m), rt), "t")
+    assert went == [kernel] and (normed.xw is None) == (kernel == "gemv")
+    assert products.decode_batch_fits(rt, x, m) == (n > 2 or n == 2 and m >= 4096)
