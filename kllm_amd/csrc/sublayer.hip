@@ -49,7 +49,12 @@ struct NormedPair {
   float sa, sb;
 };
 
-template <typename TOUT, int PER>
+// What stands beside delta's slices: nothing, a pair whose two sums are each normed, or one whose sums are added as they are.  Instances of
+// their own: with the choice at run time a row without a pair took 5.6 us for 5.4 (8 rows of 4,096), one with two norms 7.5 for 7.3, and an added
+// pair wider than 4,096 waited in LDS as two rows.  With the stores of the stream behind all of its elements' sums 4.7 and 6.5.
+enum : int { PAIR_NONE = 0, PAIR_NORMED = 1, PAIR_ADDED = 2 };
+
+template <typename TOUT, int PER, int PAIR>
 __global__ __launch_bounds__(kRowThreads) void norm_residual_kernel(
     float* __restrict__ x, const float* __restrict__ delta, int nsplit, long split_stride,
     const float* __restrict__ bias, const float* __restrict__ w, TOUT* __restrict__ out, int d, float eps,
@@ -117,35 +122,41 @@ __global__ __launch_bounds__(kRowThreads) void norm_residual_kernel(
 #pragma unroll
           for (int j = 0; j < PER; ++j) dv[j] += src[at[j]];
         }
-        if (pair.b) {       // each of the two normed over the row before they are added
+        if constexpr (PAIR == PAIR_ADDED) {
+          float bv[PER];
+#pragma unroll
+          for (int j = 0; j < PER; ++j) bv[j] = 0.f;
+          for (int s = 0; s < pair.nb; ++s) {
+            const float* src = pair.b + s * pair.stride_b + r * d;
+#pragma unroll
+            for (int j = 0; j < PER; ++j) bv[j] += src[at[j]];
+          }
+#pragma unroll
+          for (int j = 0; j < PER; ++j) dv[j] = fmaf(pair.sa, dv[j], pair.sb * bv[j]);
+        } else if constexpr (PAIR == PAIR_NORMED) {       // each of the two normed over the row before they are added
           float bv[PER], wa[PER], wb[PER];
 #pragma unroll
           for (int j = 0; j < PER; ++j) {
             bv[j] = 0.f;
-            wa[j] = pair.wa ? pair.wa[at[j]] : 0.f;
-            wb[j] = pair.wa ? pair.wb[at[j]] : 0.f;
+            wa[j] = pair.wa[at[j]];
+            wb[j] = pair.wb[at[j]];
           }
           for (int s = 0; s < pair.nb; ++s) {
             const float* src = pair.b + s * pair.stride_b + r * d;
 #pragma unroll
             for (int j = 0; j < PER; ++j) bv[j] += src[at[j]];
           }
-          if (!pair.wa) {
+          float ssa = 0.f, ssb = 0.f;
 #pragma unroll
-            for (int j = 0; j < PER; ++j) dv[j] = fmaf(pair.sa, dv[j], pair.sb * bv[j]);
-          } else {
-            float ssa = 0.f, ssb = 0.f;
-#pragma unroll
-            for (int j = 0; j < PER; ++j) {
-              if (threadIdx.x + kRowThreads * j >= d) dv[j] = bv[j] = 0.f;
-              ssa = fmaf(dv[j], dv[j], ssa);
-              ssb = fmaf(bv[j], bv[j], ssb);
-            }
-            const float ra = pair.sa / sqrtf(block_sum(ssa, red) / (float)d + eps);
-            const float rb = pair.sb / sqrtf(block_sum(ssb, red) / (float)d + eps);
-#pragma unroll
-            for (int j = 0; j < PER; ++j) dv[j] = fmaf(dv[j] * ra, wa[j], bv[j] * rb * wb[j]);
+          for (int j = 0; j < PER; ++j) {
+            if (threadIdx.x + kRowThreads * j >= d) dv[j] = bv[j] = 0.f;
+            ssa = fmaf(dv[j], dv[j], ssa);
+            ssb = fmaf(bv[j], bv[j], ssb);
           }
+          const float ra = pair.sa / sqrtf(block_sum(ssa, red) / (float)d + eps);
+          const float rb = pair.sb / sqrtf(block_sum(ssb, red) / (float)d + eps);
+#pragma unroll
+          for (int j = 0; j < PER; ++j) dv[j] = fmaf(dv[j] * ra, wa[j], bv[j] * rb * wb[j]);
         }
 #pragma unroll
         for (int j = 0; j < PER; ++j) v[j] = fmaf(dscale, dv[j], v[j]);
@@ -171,9 +182,12 @@ __global__ __launch_bounds__(kRowThreads) void norm_residual_kernel(
       const int i = threadIdx.x + kRowThreads * j;
       const float y = v[j] * rstd * wv[j];
       v[j] = i < d ? (sums ? fmaf(mult, y, xv[j]) : y) : 0.f;
-      if (i < d) xr[i] = v[j];
       ss2 = fmaf(v[j], v[j], ss2);
     }
+    // (behind all of them: between them a wait for the next element's loads would wait for the stores too)
+#pragma unroll
+    for (int j = 0; j < PER; ++j)
+      if (threadIdx.x + kRowThreads * j < d) xr[threadIdx.x + kRowThreads * j] = v[j];
     if (!out) return;
     if (next_w) {       // the norm in front of the next sub-layer, of the row that is still in registers
 #pragma unroll
@@ -190,7 +204,7 @@ __global__ __launch_bounds__(kRowThreads) void norm_residual_kernel(
     return;
   }
   float ra = 1.f, rb = 0.f;
-  if (pair.b) {       // a pass of its own for the two sums of squares; the sums wait in LDS
+  if (PAIR == PAIR_NORMED) {       // a pass of its own for the two sums of squares; the sums wait in LDS
     float ssa = 0.f, ssb = 0.f;
     for (int i = threadIdx.x; i < d; i += kRowThreads) {
       float a = 0.f, b = 0.f;
@@ -201,22 +215,24 @@ __global__ __launch_bounds__(kRowThreads) void norm_residual_kernel(
       ssa = fmaf(a, a, ssa);
       ssb = fmaf(b, b, ssb);
     }
-    if (pair.wa) {
-      ra = pair.sa / sqrtf(block_sum(ssa, red) / (float)d + eps);
-      rb = pair.sb / sqrtf(block_sum(ssb, red) / (float)d + eps);
-    }
+    ra = pair.sa / sqrtf(block_sum(ssa, red) / (float)d + eps);
+    rb = pair.sb / sqrtf(block_sum(ssb, red) / (float)d + eps);
   }
   float ss = 0.f;
   for (int i = threadIdx.x; i < d; i += kRowThreads) {
     float v;
     if (sums) {
       v = chosen.y ? chosen_at(i) : 0.f;
-      if (pair.b) {
-        v = fmaf(dscale, pair.wa ? fmaf(row_lds[i] * ra, pair.wa[i], row_lds[d + i] * rb * pair.wb[i])
-                                 : fmaf(pair.sa, row_lds[i], pair.sb * row_lds[d + i]), v);
+      if (PAIR == PAIR_NORMED) {
+        v = fmaf(dscale, fmaf(row_lds[i] * ra, pair.wa[i], row_lds[d + i] * rb * pair.wb[i]), v);
       } else if (delta) {
         float dsum = 0.f;
         for (int s = 0; s < nsplit; ++s) dsum += delta[s * split_stride + r * d + i];
+        if (PAIR == PAIR_ADDED) {
+          float bsum = 0.f;
+          for (int s = 0; s < pair.nb; ++s) bsum += pair.b[s * pair.stride_b + r * d + i];
+          dsum = fmaf(pair.sa, dsum, pair.sb * bsum);
+        }
         v = fmaf(dscale, dsum, v);
       }
       if (bias) v += bias[i];
@@ -418,10 +434,16 @@ extern "C" int kllm_norm_residual(float* x, const float* delta, int nsplit, long
   KLLM_REQUIRE(!delta || nsplit >= 1, "norm_residual: nsplit %d", nsplit);
   KLLM_REQUIRE(delta || chosen_y || !bias, "norm_residual: a bias goes with sums");
   KLLM_REQUIRE(out_dtype == DT_F32 || out_dtype == DT_BF16, "norm_residual: unknown dtype %d", out_dtype);
-#define KLLM_NR(TOUT, PER)                                                                                    \
-  hipLaunchKernelGGL((norm_residual_kernel<TOUT, PER>), dim3(n), dim3(kRowThreads),                           \
-                     PER ? 0 : (size_t)d * sizeof(float) * (pair_b ? 2 : 1), stream, x, delta, nsplit, split_stride, \
+#define KLLM_NRP(TOUT, PER, PAIR)                                                                             \
+  hipLaunchKernelGGL((norm_residual_kernel<TOUT, PER, PAIR>), dim3(n), dim3(kRowThreads),                     \
+                     PER ? 0 : (size_t)d * sizeof(float) * (PAIR == PAIR_NORMED ? 2 : 1), stream, x, delta, nsplit, split_stride, \
                      bias, weight, (TOUT*)out, d, eps, chosen, mult, next_weight, delta_scale, pair)
+#define KLLM_NR(TOUT, PER)                                  \
+  do {                                                      \
+    if (!pair_b) KLLM_NRP(TOUT, PER, PAIR_NONE);            \
+    else if (pair_wa) KLLM_NRP(TOUT, PER, PAIR_NORMED);     \
+    else KLLM_NRP(TOUT, PER, PAIR_ADDED);                   \
+  } while (0)
   const bool bf = out && out_dtype == DT_BF16;
   if (d <= 4 * kRowThreads) {
     if (bf) KLLM_NR(bf16_t, 4); else KLLM_NR(float, 4);
@@ -433,6 +455,7 @@ extern "C" int kllm_norm_residual(float* x, const float* delta, int nsplit, long
     if (bf) KLLM_NR(bf16_t, 0); else KLLM_NR(float, 0);
   }
 #undef KLLM_NR
+#undef KLLM_NRP
   KLLM_CHECK_LAUNCH("norm_residual");
   return 0;
 }

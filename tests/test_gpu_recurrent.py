@@ -321,3 +321,9 @@ def test_norm_of_two_sums_without_weights(d, slices):
     K().norm_residual(want, w, both, out=out_want, eps=1e-5)
     K().norm_residual(got, w, K().NormedPair(a, 0.75, None, b, -1.5, None), out=out, eps=1e-5)
     assert torch.equal(got, want) and torch.equal(out, out_want)
+
+
+@pytest.mark.parametrize("d", [8200, 16384])
+def test_norm_of_two_sums_without_weights_of_wide_rows(d):
+    """Rows of which two do not fit into a launch's 64 KB of LDS: the two sums are added on the way there."""
+    test_norm_of_two_sums_without_weights(d, (2, 1))
