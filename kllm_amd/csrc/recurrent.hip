@@ -975,7 +975,10 @@ static int recurrence_prep_launch(int bs, A... args) {
 // those before a segment are folded into its starting state and it runs once more, now writing.  A
 // chain of n steps becomes two of n / SEGS.
 // CH channels and SEGS segments a workgroup (see kllm_linear_recurrence_scan); a span of up to LEAST tokens is one
-// segment, and the others' threads leave at once.
+// segment, and the others' threads leave at once.  The convolution's inputs are left by workgroups of their own, behind those of
+// a span's channels: in front of a chain they held it up (us, before and now, 2,048 channels: 480 tokens beside 20 single ones 23.1 / 17.1,
+// 1,500 tokens 36.0 / 31.9, 8 single tokens 5.2 / 4.5).  Where single tokens have twelve workgroups a CU the chain's threads do it, as
+// before (64 tokens, 4,096 channels: 8.2 us; 8.9 with workgroups of their own; at 2,048 channels 6.5 and 6.3).
 template <typename T, int CH, int SEGS>
 __global__ __launch_bounds__(CH * SEGS) void linear_recurrence_scan_kernel(
     const float* __restrict__ a_in, const float* __restrict__ b_in, const float* __restrict__ proj, int nsplit,
@@ -988,13 +991,20 @@ __global__ __launch_bounds__(CH * SEGS) void linear_recurrence_scan_kernel(
   const bool ok = blockIdx.x * CH + lane < W;
   const int span = blockIdx.y;
   const long t0 = span_start[span], t1 = span_start[span + 1];
+  const int own = (W + CH - 1) / CH;                      // workgroups of the chain
+  if (SEGS == 1 && (int)gridDim.x == own && tail.taps > 1 && ok)
+    conv_tail(tail, slot_stride, c, slots[span], t0, t1, span_pos[span] == 0);
+  if ((int)blockIdx.x >= own) {
+    const int cc = ((int)blockIdx.x - own) * CH * SEGS + (int)threadIdx.x;
+    if (cc < W) conv_tail(tail, slot_stride, cc, slots[span], t0, t1, span_pos[span] == 0);
+    return;
+  }
   const long len = t1 - t0;
   constexpr int U = 8, LEAST = 4;                         // tokens asked for at a time, of a segment at least
   const long per = SEGS > 1 ? max((long)LEAST, (len + SEGS - 1) / SEGS) : len;
   const bool cut = SEGS > 1 && len > LEAST;
   const long a0 = min(t1, t0 + seg * per), a1 = min(t1, a0 + per);
   float* st = state + (long)slots[span] * slot_stride + c;
-  if (tail.taps > 1 && ok && seg == 0) conv_tail(tail, slot_stride, c, slots[span], t0, t1, span_pos[span] == 0);
   if (!cut && seg > 0) return;                            // (nobody meets)
   float S = span_pos[span] == 0 ? 0.f : *st;
   if (cut) {
@@ -1293,7 +1303,8 @@ extern "C" int kllm_linear_recurrence_scan(const float* a_in, const float* b_in,
   const ConvTail tail = {proj, split_stride, 2L * W, conv_bias, conv_state, nsplit, W, W, conv_state ? taps : 0};      // (of x)
 #define KLLM_LRS(CH, SEGS)                                                                                               \
   do {                                                                                                                  \
-    const dim3 grid(ceil_div(W, CH), n_spans), wg(CH * SEGS);                                                           \
+    const bool apart = tail.taps > 1 && (SEGS > 1 || (long)n_spans * ceil_div(W, CH) <= 12L * device_cus());            \
+    const dim3 grid(ceil_div(W, CH) + (apart ? ceil_div(W, CH * SEGS) : 0), n_spans), wg(CH * SEGS);                    \
     if (dtype == DT_F32)                                                                                                \
       hipLaunchKernelGGL((linear_recurrence_scan_kernel<float, CH, SEGS>), grid, wg, 0, stream, a_in, b_in, proj,       \
                          nsplit, split_stride, y_bias, state, slot_stride, slots, span_start, span_pos, (float*)out, W, tail); \

@@ -327,3 +327,22 @@ def test_norm_of_two_sums_without_weights(d, slices):
 def test_norm_of_two_sums_without_weights_of_wide_rows(d):
     """Rows of which two do not fit into a launch's 64 KB of LDS: the two sums are added on the way there."""
     test_norm_of_two_sums_without_weights(d, (2, 1))
+
+
+@pytest.mark.parametrize("W,spans", [(70, 3), (1100, 3), (2048, 97)])
+@pytest.mark.parametrize("longest", [1, 30, 150])
+def test_linear_scan_leaves_the_inputs_of_more_channels_than_a_workgroup(W, spans, longest):
+    """Workgroups of 64 to 1,024 threads for the convolution's inputs, the last one not whole; 97 single tokens of 2,048 channels
+    (more than twelve workgroups a CU) leave them by the chain's own threads."""
+    lens = [1] * (spans - 1) + [longest]
+    fresh, taps, n = [i % 2 for i in range(spans)], 4, sum(lens)
+    _, _, span_start, span_pos, slots = spans_of(lens, fresh)
+    state = torch.randn(spans + 1, W * taps, device=DEV)
+    proj, bias, y_bias = torch.randn(1, n, 2 * W, device=DEV), torch.randn(W, device=DEV), torch.randn(W, device=DEV)
+    a, b, out = torch.rand(n, W, device=DEV), torch.randn(n, W, device=DEV), torch.empty(n, W, device=DEV)
+    want, got, alone = state.clone(), state.clone(), torch.empty(n, W, device=DEV)
+    K().conv_state_update(proj, W, W, taps, want, W, slots, span_start, span_pos, spans, in_bias=bias)
+    K().linear_recurrence_scan(a, b, proj, y_bias, want, 0, slots, span_start, span_pos, spans, alone, longest=longest)
+    K().linear_recurrence_scan(a, b, proj, y_bias, got, 0, slots, span_start, span_pos, spans, out, longest=longest,
+                               conv=(bias, taps, W))
+    assert torch.equal(got, want) and torch.equal(out, alone)
