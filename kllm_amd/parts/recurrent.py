@@ -50,6 +50,17 @@ MAX_TAPS = 16
 SIXTEENS_FROM = 64
 
 
+def takes_sixteens(lens, head_dim):
+    """Whether a step with spans of these lengths takes the gated delta rule's tokens sixteen at a time.  A single token costs a whole
+    sixteen's operands there, so every span shorter than sixteen beyond the first eight asks for two more tokens of the
+    longest.  Token by token / sixteen at a time, in us, a prompt's portion beside single tokens, 16 heads of 128: 64 beside 8
+    25 / 21, beside 32 45 / 48, beside 200 187 / 221; 256 beside 64 113 / 98, beside 200 224 / 242; 32 heads, 256 beside 64 175 / 170; 8 heads of
+    64, 256 beside 128 1.14 times as long, of 256, 192 beside 64 0.94.  Keys of 129 to 192 channels are the faster sixteen at
+    a time beside any number (64 beside 64 104 / 92, beside 256 0.97), which stand in three of the token kernel's four blocks of 64."""
+    short = 0 if 128 < head_dim <= 192 else sum(n < 16 for n in lens)
+    return max(lens) >= SIXTEENS_FROM + 2 * max(0, short - 8)
+
+
 @register_part("mixer", "gated_delta")
 class GatedDeltaMixer(Part):
     graph_safe = True
@@ -179,7 +190,7 @@ class GatedDeltaMixer(Part):
                            low_sums=low_sums, gate_sigmoid=self.gate_sigmoid)
         o = ctx.buf("gdelta.o", (n, self.hv), f32)
         factors = None
-        if not self.channel_decay and ctx.max_span_len >= SIXTEENS_FROM and (n + 64) * self.hv < 2 ** 29:
+        if not self.channel_decay and takes_sixteens(ctx.h_span_len, self.head_dim) and (n + 64) * self.hv < 2 ** 29:
             floats = K.gated_delta_factor_floats(n, ctx.n_spans, self.heads, self.kv_heads, self.head_dim)
             factors = ctx.buf("gdelta.factors", (floats,), f32)
             K.gated_delta_factors(qn, kn, gb, ctx.span_start, ctx.n_spans, factors, self.heads, self.kv_heads, self.head_dim)

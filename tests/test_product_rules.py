@@ -9,6 +9,7 @@ from kllm_amd.engine.engine import room_for_copies
 from kllm_amd.parts import linear as products
 from kllm_amd.parts.base import ResidualSink
 from kllm_amd.parts.linear import choose
+from kllm_amd.parts.recurrent import takes_sixteens
 
 BF16, F32 = torch.bfloat16, torch.float32
 LONG = 1 << 23          # from this K on a lane's offset takes 64 bits
@@ -130,3 +131,11 @@ def test_few_rows_of_float32_leave_the_gemv_where_that_is_the_faster_way(n, m, k
     normed = products.linear_into(rt, x, w, ResidualSink(torch.empty(n, m), rt), "t")
     assert went == [kernel] and (normed.xw is None) == (kernel == "gemv")
     assert products.decode_batch_fits(rt, x, m) == (n > 2 or n == 2 and m >= 4096)
+
+
+@pytest.mark.parametrize("lens,head_dim,want", [
+    ([64], 128, True), ([63], 128, False), ([64] + [1] * 8, 128, True), ([64] + [1] * 9, 128, False), ([112] + [1] * 32, 128, True),
+    ([111] + [1] * 32, 128, False), ([100] * 70, 128, True), ([480] + [1] * 200, 64, True), ([256] + [15] * 200, 64, False),
+    ([64] + [1] * 200, 192, True), ([64] + [1] * 200, 129, True), ([64] + [1] * 200, 193, False), ([1] * 8, 192, False)])
+def test_sixteen_tokens_at_a_time_only_where_short_spans_are_few(lens, head_dim, want):
+    assert takes_sixteens(lens, head_dim) is want
