@@ -162,7 +162,7 @@ def dense_hidden(ctx, xn, w_up, tag, tiled, act, params=None):
     if (n > 128 and opts.get("gemm") != "library" and opts.get("gemm_algo") is None
             and xn.shape[1] % (8 if xn.dtype == torch.bfloat16 else 4) == 0):
         K.gemm_act(xn, w_up, h, act, params)      # prompts
-    elif parts_rows(ctx.runtime, n, w_up, tiled) or (decode_batch_fits(ctx.runtime, xn, w_up.shape[0]) and not opts.get("no_fused_linear")
+    elif parts_rows(ctx.runtime, n, w_up, tiled, True) or (decode_batch_fits(ctx.runtime, xn, w_up.shape[0]) and not opts.get("no_fused_linear")
                                                      and opts.get("gemm_algo") is None):
         h = decode_linear(ctx, xn, w_up, tag + ".h", tiled, unary=(act, params))      # decode batches
     else:

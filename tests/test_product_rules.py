@@ -139,3 +139,18 @@ def test_few_rows_of_float32_leave_the_gemv_where_that_is_the_faster_way(n, m, k
     ([64] + [1] * 200, 192, True), ([64] + [1] * 200, 129, True), ([64] + [1] * 200, 193, False), ([1] * 8, 192, False)])
 def test_sixteen_tokens_at_a_time_only_where_short_spans_are_few(lens, head_dim, want):
     assert takes_sixteens(lens, head_dim) is want
+
+
+@pytest.mark.parametrize("n,m,k,dtype,unary,want", [
+    (1, 2048, 1024, BF16, False, False), (1, 2048, 1056, BF16, False, True), (6, 2048, 2048, BF16, False, True),
+    (7, 2048, 2048, BF16, False, False), (7, 2048, 2080, BF16, False, True), (8, 2064, 2048, BF16, False, True), (8, 1024, 1056, BF16, True, True), (8, 1024, 1024, BF16, True, False),
+    (9, 2048, 2048, BF16, False, False), (16, 2048, 2048, BF16, True, False), (17, 2048, 160, BF16, False, True),
+    (17, 2048, 128, BF16, False, False), (17, 2048, 128, BF16, True, True), (32, 2048, 2816, BF16, False, True),
+    (33, 2048, 2080, BF16, False, False), (33, 2048, 2048, BF16, False, True), (64, 5632, 1024, BF16, True, True),
+    (32, 12304, 512, BF16, True, False), (32, 12288, 512, BF16, True, True), (8, 16384, 4096, BF16, False, False),
+    (5, 64, 64, F32, False, True), (6, 64, 64, F32, False, False), (8, 2816, 64, F32, False, True), (8, 64, 544, F32, False, True),
+    (9, 2816, 2816, F32, False, False)])
+def test_plain_sums_without_staging_by_size(n, m, k, dtype, unary, want):
+    """The lines of the rule, both sides of each."""
+    rt, w = _Recorder(dtype), torch.empty(m, k, dtype=dtype)
+    assert products.parts_rows(rt, n, w, object(), unary) is want
