@@ -339,7 +339,7 @@ def _parts_best(n, m, k, dtype, unary):
     """Whether ``K.linear_rows`` is the fastest way to plain sums, or (``unary``) an activation of them, of n rows that are read row by row.
     The decode-batch kernel has the rows in LDS, this one reads up to sixteen of them a load: up to eight rows it is the faster one where
     K is long enough, of 9 to 16 not (a step of Nusilix layers of 1,024 columns, there / here, with K of 1,024 here, too: 1 token 601 / 608 us, 2
-    606 / 617, 8 678 / 714; us a product: 8 rows 2,048 x 1,024 3.8 / 4.6, 2,048 x 4,096 6.8 / 6.2, 1,024 x 2,048 4.6 / 4.5, 2,048 x 2,048 4.9 /
+    606 / 617, 8 678 / 714; us a product: 8 rows 2,048 x 1,024 3.8 / 4.6, 2,048 x 4,096 6.8 / 6.2, 1,024 x 1,408 in a step 3.9 / 5.3, 2,048 x 2,048 4.9 /
     5.2; a step at Natenex sizes, 16 rows 898 / 903).  Beyond 16 rows it takes the place of K in slices from the tiles, which the consumer adds, and
     of an activation's launch (a step at Natenex sizes, without and with: 24 tokens 1,123 / 894, 48 1,268 / 1,192, 64 1,538 / 1,524, a
     prompt of 20 1,004 / 761, of 60 1,146 / 1,131), but for sums of little K and, beyond 32 rows, of long K (a product and a
@@ -348,7 +348,7 @@ def _parts_best(n, m, k, dtype, unary):
     if dtype == torch.float32:
         return n <= 5 or n <= 8 and (k > 512 or m > 2048)      # (8 rows, 2,048 x 512: 4.5 us there, 4.8 here; 2,816 x 512 5.2 / 5.0)
     if n <= 8:
-        return k > 1024 and (n <= 6 or k > 2048 or not 1024 < m <= 2048)
+        return k > 1024 and (n <= 6 or k > 2048 or m > 2048)
     if n <= 16 or m > 48 * K.device_cus():
         return False
     return unary or (k > 128 and (n <= 32 or k <= 2048))

@@ -143,7 +143,7 @@ def test_sixteen_tokens_at_a_time_only_where_short_spans_are_few(lens, head_dim,
 
 @pytest.mark.parametrize("n,m,k,dtype,unary,want", [
     (1, 2048, 1024, BF16, False, False), (1, 2048, 1056, BF16, False, True), (6, 2048, 2048, BF16, False, True),
-    (7, 2048, 2048, BF16, False, False), (7, 2048, 2080, BF16, False, True), (8, 2064, 2048, BF16, False, True), (8, 1024, 1056, BF16, True, True), (8, 1024, 1024, BF16, True, False),
+    (7, 2048, 2048, BF16, False, False), (7, 2048, 2080, BF16, False, True), (8, 2064, 2048, BF16, False, True), (8, 1024, 1056, BF16, True, False), (8, 4096, 1056, BF16, True, True), (8, 1024, 1024, BF16, True, False),
     (9, 2048, 2048, BF16, False, False), (16, 2048, 2048, BF16, True, False), (17, 2048, 160, BF16, False, True),
     (17, 2048, 128, BF16, False, False), (17, 2048, 128, BF16, True, True), (32, 2048, 2816, BF16, False, True),
     (33, 2048, 2080, BF16, False, False), (33, 2048, 2048, BF16, False, True), (64, 5632, 1024, BF16, True, True),
