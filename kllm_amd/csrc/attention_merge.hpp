@@ -17,7 +17,8 @@ namespace kllm {
 template <typename T, int DV, int R = 16>   // DV: elements of a head per lane (head size up to 64 DV); R: slices a round
 __device__ __forceinline__ void attn_merge_one(T* __restrict__ out, const float* __restrict__ part, int t, int h, int H,
                                                int hd, int nslices, int lane, const OutGate& gate) {
-  const int stride = hd + 2;
+  const int stride = hd + 2, side = gate.side;
+  asm volatile("" ::"s"(side));        // (with the other arguments: in front of the stores it was a trip to memory of its own)
   const float* p = part + ((long)t * H + h) * nslices * stride;
   float M = -INFINITY, denom = 0.f, o[DV];
 #pragma unroll
@@ -55,7 +56,7 @@ __device__ __forceinline__ void attn_merge_one(T* __restrict__ out, const float*
 #pragma unroll
   for (int v = 0; v < DV; ++v)
     if (lane + 64 * v < hd)
-      out[rows_at(gate.side, t, h * hd + lane + 64 * v, H * hd)] = from_f32<T>(o[v] / denom * out_gate(gate, t, h, lane + 64 * v));
+      out[rows_at(side, t, h * hd + lane + 64 * v, H * hd)] = from_f32<T>(o[v] / denom * out_gate(gate, t, h, lane + 64 * v));
 }
 
 // The same for up to 64 slices and heads of up to 128 in one trip to memory instead of one per
@@ -65,7 +66,8 @@ __device__ __forceinline__ void attn_merge_one(T* __restrict__ out, const float*
 template <typename T, int DV, int R>   // R: 16, 32 or 64, at least the number of slices
 __device__ __forceinline__ void attn_merge_wide(T* __restrict__ out, const float* __restrict__ part, int t, int h, int H,
                                                 int hd, int nslices, int lane, const OutGate& gate) {
-  const int stride = hd + 2;
+  const int stride = hd + 2, side = gate.side;
+  asm volatile("" ::"s"(side));        // (as above)
   const float* p = part + ((long)t * H + h) * nslices * stride;
   float os[DV][R];
 #pragma unroll
@@ -95,7 +97,7 @@ __device__ __forceinline__ void attn_merge_wide(T* __restrict__ out, const float
 #pragma unroll
   for (int v = 0; v < DV; ++v)
     if (lane + 64 * v < hd)
-      out[rows_at(gate.side, t, h * hd + lane + 64 * v, H * hd)] = from_f32<T>(o[v] / denom * out_gate(gate, t, h, lane + 64 * v));
+      out[rows_at(side, t, h * hd + lane + 64 * v, H * hd)] = from_f32<T>(o[v] / denom * out_gate(gate, t, h, lane + 64 * v));
 }
 
 template <typename T, int DV, int R>

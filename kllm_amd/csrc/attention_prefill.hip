@@ -460,18 +460,22 @@ __global__ __launch_bounds__(64 * kPrefillWaves * PAR) __attribute__((amdgpu_wav
     return;
   }
   const float inv = 1.f / l;                                  // finite: a query reads its own key
-  const int side = gate.side ? gate.side : 1;                 // (eights of columns lie side times as far apart)
   bf16_t* orow = out + rows_at(gate.side, tq, h * hd + 4 * g, H * hd);
+  auto store = [&](auto side) {                               // (eights of columns lie side times as far apart)
 #pragma unroll
-  for (int r = 0; r < HDT; ++r)
+    for (int r = 0; r < HDT; ++r)
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const floatx4 og = out_gate4(gate, tq, h, 32 * r + 8 * b + 4 * g);
-      bf16x4 v;
+      for (int b = 0; b < 4; ++b) {
+        const floatx4 og = out_gate4(gate, tq, h, 32 * r + 8 * b + 4 * g);
+        bf16x4 v;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = (bf16_t)(acc[r][4 * b + j] * inv * og[j]);
-      *reinterpret_cast<bf16x4*>(orow + (32 * r + 8 * b) * side) = v;
-    }
+        for (int j = 0; j < 4; ++j) v[j] = (bf16_t)(acc[r][4 * b + j] * inv * og[j]);
+        *reinterpret_cast<bf16x4*>(orow + (32 * r + 8 * b) * side) = v;
+      }
+  };
+  // (rows as they are with the distances in the instructions: 8 heads of 256, 512 / 480 behind 480 tokens 49.5 / 82.6 us without, 48.6 / 81.3)
+  if (gate.side) store(gate.side);
+  else store(std::integral_constant<int, 1>());
 }
 
 // The merge of the slices' results, one wave per (query, head); a block's queries are the
