@@ -200,6 +200,8 @@ long kllm_fused_linear_lds_bytes(int n, int k, int nsplit, int dtype);
  * those up to the next multiple of 16 are there and hold anything, with fewer only the rows are. */
 int kllm_linear_rows(const void* x, int x_stride, const KllmLinearOut* y, const void* w, int n, int m, int k, hipStream_t stream);
 int kllm_linear_rows_parts(int n, int m, int k);
+/* Tiles of 16 rows of X that the busiest CU reads in all its workgroups. */
+int kllm_linear_rows_row_tiles(int kind, int n, int m, int k);
 /* Where that is more than LDS holds, the rows are staged and multiplied in passes over K, with
  * one tile to a workgroup (tiles_per_wg = 1): how many passes a call needs (1: all at once; 0:
  * the kernel does not take the sizes). */

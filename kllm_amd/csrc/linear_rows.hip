@@ -381,6 +381,42 @@ static int lr_tiles(int kind, int m) { return kind == FL_RESID || kind == FL_PAR
 // Whether a product that splits takes eight rows of W a workgroup (SPLIT): up to 16 rows of X and no more tiles than half the CUs.
 static bool lr_split(int n, int m, int k) { return n <= 16 && k % 64 == 0 && 2 * lr_tiles(FL_RESID, m) <= device_cus(); }
 
+// Tiles of W a workgroup, workgroups that share the rows out, tiles of rows a workgroup.
+struct LrPlan {
+  int tw, halves, nt;
+};
+
+static LrPlan lr_plan(int ep, int n, int m, int k, bool f32, bool x_tiled) {
+  const int cus = device_cus(), tiles = lr_tiles(ep, m);
+  LrPlan p = {1, 1, ceil_div(n, 16)};
+  if (ep == FL_SWIGLU || ep == FL_PARTS) {
+    // Tiles a workgroup: the least that leaves one round of the chip, three at most (2 x 5,632 x 2,048, 8 / 64 rows: 12.1 / 17.5 us with two, 11.0
+    // / 14.9 with three, 13.3 / 16.4 with four; 2 x 14,336 x 4,096, 16 / 64 rows: 48.5 / 62.0, 46.5 / 59.3, 54.5 / 59.6).
+    while (p.tw < 3 && ceil_div(tiles, p.tw) > cus) ++p.tw;
+    // Many rounds: one tile, of which a CU holds two workgroups, where K is long; two where a workgroup is short, or where many
+    // rows that lie as they are (slow to read) are read once for both.  us with one / two / three: 2 x 14,336 x 4,096, 8 rows 41.4 / 45.6 / 45.9, 16 rows
+    // 45.2 / 47.0 / 47.5, as they are 9 42.0 / 46.6, 12 44.5 / 46.4, 16 49.1 / 46.8 / 48.3; 2 x 13,824 x 5,120, 12 rows as they are 61.7 / 57.8 / 58.9; 2 x 8,192 x 3,072, 16 rows 23.4 / 20.9 / 23.7; x 2,048, 1 row
+    // 13.7 / 14.1 / 15.6; 2 x 11,008 x 1,024, 8 rows 14.0 / 11.9 / 10.5.  float32, whose rows are as they are: 2 x 8,192 x 2,048, 8 / 16 rows 25.6
+    // / 29.9 with one, 28.5 / 29.2 with two; 2 x 7,168 x 1,536 21.5 / 26.6, 21.3 / 23.6.
+    if (tiles > 3 * cus) p.tw = n > 16 ? 1 : n <= 8 ? (f32 || k >= 2048 ? 1 : 2) : f32 ? (k >= 2048 ? 1 : 2) : (k >= 4096 && (x_tiled || n * k <= 49152) ? 1 : 2);
+  }
+  // Halves of the rows where the busiest CU then has fewer tiles of rows to take (or as many, of workgroups that share it
+  // anyway): 64 rows against 2,048 x 5,632 (128 tiles) 17.6 -> 12.2 us, 6,144 x 4,096 (384) 25.4 -> 21.2, 48 rows 21.3 -> 18.8; not
+  // 4,096 x 14,336 (256) 41.0 -> 46.7, nor 2,560 x 2,048 (160) at 32 rows 5.0 -> 5.5.
+  const int whole = ceil_div(tiles, cus) * p.nt, halved = ceil_div(2L * tiles, cus) * ceil_div(p.nt, 2);
+  if (ep != FL_SWIGLU && p.tw == 1 && (halved < whole || (halved == whole && tiles > cus))) {
+    p.halves = 2;
+    p.nt = ceil_div(p.nt, 2);
+  }
+  return p;
+}
+
+extern "C" int kllm_linear_rows_row_tiles(int kind, int n, int m, int k) {
+  if (n <= 0 || m <= 0 || k <= 0) return 0;
+  const LrPlan p = lr_plan(kind, n, m, k, false, true);
+  return ceil_div((long)ceil_div(lr_tiles(kind, m), p.tw) * p.halves, device_cus()) * p.nt;
+}
+
 extern "C" int kllm_linear_rows_parts(int n, int m, int k) {
   if (n <= 0 || m <= 0 || k <= 0) return 0;
   const int parts = lr_split(n, m, k) ? 2 * lr_tiles(FL_RESID, m) : lr_tiles(FL_RESID, m);
@@ -459,22 +495,8 @@ extern "C" int kllm_linear_rows(const void* x, int x_stride, const KllmLinearOut
     out.KV = KV;
     out.hd = hd;
   }
-  const int cus = device_cus();
-  // Tiles a workgroup: the least that leaves one round of the chip, three at most (2 x 5,632 x 2,048, 8 / 64 rows: 12.1 / 17.5 us with two, 11.0
-  // / 14.9 with three, 13.3 / 16.4 with four; 2 x 14,336 x 4,096, 16 / 64 rows: 48.5 / 62.0, 46.5 / 59.3, 54.5 / 59.6).
-  int tw = 1;
-  if (ep == FL_SWIGLU || ep == FL_PARTS)
-    while (tw < 3 && ceil_div(tiles, tw) > cus) ++tw;
-  // Many rounds: one tile, whose rounds are whole (2 x 14,336 columns: seven, where three tiles are 2.3) and of which a CU holds two workgroups
-  // (a step at 8B sizes, 1 / 8 / 16 tokens 3,298 / 3,568 / 3,833 us with three, 3,146 / 3,407 / 3,694 with one; float32, 2 tokens 6,519, 6,166).
-  if (tiles > 3 * cus) tw = 1;
-  const int row_tiles = ceil_div(n, 16);
-  // Halves of the rows where the busiest CU then has fewer tiles of rows to take (or as many, of workgroups that share it
-  // anyway): 64 rows against 2,048 x 5,632 (128 tiles) 17.6 -> 12.2 us, 6,144 x 4,096 (384) 25.4 -> 21.2, 48 rows 21.3 -> 18.8; not
-  // 4,096 x 14,336 (256) 41.0 -> 46.7, nor 2,560 x 2,048 (160) at 32 rows 5.0 -> 5.5.
-  const int whole = ceil_div(tiles, cus) * row_tiles, halved = ceil_div(2L * tiles, cus) * ceil_div(row_tiles, 2);
-  const int halves = ep != FL_SWIGLU && tw == 1 && (halved < whole || (halved == whole && tiles > cus)) ? 2 : 1;
-  const int nt = ceil_div(row_tiles, halves);
+  const LrPlan plan = lr_plan(ep, n, m, k, f32, out.x_tiled);
+  const int tw = plan.tw, halves = plan.halves, nt = plan.nt;
 #define KLLM_LRS(NT, EP)                                                                                        \
   (f32 ? lr_launch_waves<float, NT, 1, EP, false, 8, true>(x, out, w, n, m, k, tiles, 1, x_stride, stream)      \
        : lr_launch_waves<bf16_t, NT, 1, EP, false, 8, true>(x, out, w, n, m, k, tiles, 1, x_stride, stream))

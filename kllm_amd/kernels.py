@@ -21,7 +21,7 @@ import torch
 DT_F32, DT_BF16 = 0, 1
 GEMM_PLAIN, GEMM_TILED_F32, GEMM_MFMA_BF16, GEMM_SKINNY_BF16, GEMM_GEMV, GEMM_GEMV_LDS, GEMM_MFMA_F32 = 0, 1, 2, 3, 4, 5, 6
 GEMV_BEST_ROWS = 0         # rows up to which they beat the MFMA kernels in bfloat16: none (a step at 1.1B sizes, one token: 1.036 against 0.963 ms)
-ABI_VERSION = 20
+ABI_VERSION = 21
 
 
 class KernelError(RuntimeError):
@@ -108,6 +108,7 @@ def _declare(lib):
         "kllm_fused_linear_resid_parts": [I, I],
         "kllm_linear_rows": [P, I, P, P, I, I, I, P],
         "kllm_linear_rows_parts": [I, I, I],
+        "kllm_linear_rows_row_tiles": [I, I, I, I],
         "kllm_fused_linear_passes": [I, I, I, I],
         "kllm_fused_linear_tile": [P, P, I, I, I, I, I, I, I, I, P],
         "kllm_command_op": [c_char_p],
@@ -1007,7 +1008,8 @@ def linear_rows_best(kind, n, m, k, dtype=torch.bfloat16, tiled_x=True) -> bool:
     ``TiledRows`` take a CU longer and count twice): 2,048 x 5,632 at 64 rows has it read 360 KB, 12.1 us against 10.9 and 4.7 for K
     in slices and the norm that adds them; 4,096 x 4,096 at 48 rows 390 KB, 16.4 against 15 (17 / 32 / 48 / 64 tokens at 1.1B
     sizes 1,201 / 1,377 / 1,559 / 1,663 against 1,067 / 1,155 / 1,246 / 1,370; with all products at 8B sizes 64 tokens
-    4,902 against 6,146)."""
+    4,902 against 6,146), and not with more than three tiles of columns a CU, which workgroups would take one by one (32 rows 14,336 x 1,024 with an
+    activation 12.3 us from the tiles, 18.7 here)."""
     if not 1 <= n <= (LINEAR_ROWS_MAX if dtype == torch.bfloat16 else 16) or k % 32 or k > 1 << 20:
         return False
     if dtype == torch.float32 and m * k >= 1 << 29:        # (2 GiB: only the tiled copy could be read, and there may be none)
@@ -1016,10 +1018,9 @@ def linear_rows_best(kind, n, m, k, dtype=torch.bfloat16, tiled_x=True) -> bool:
         return False
     if n <= 16:
         return True
-    tiles, cus, row_tiles = -(-m // 16), device_cus(), -(-n // 16)
-    busiest = ((1 if tiles <= 3 * cus else -(-tiles // cus)) * row_tiles
-               if kind == LINEAR_SWIGLU or (kind == LINEAR_PARTS and tiles > cus) else min(
-        -(-tiles // cus) * row_tiles, -(-2 * tiles // cus) * -(-row_tiles // 2)))
+    if kind in (LINEAR_SWIGLU, LINEAR_PARTS) and m > 48 * device_cus():
+        return False
+    busiest = int(library().kllm_linear_rows_row_tiles(int(kind), int(n), int(m), int(k)))
     return 32 * k * busiest * (1 if tiled_x else 2) <= LINEAR_ROWS_BYTES
 
 

@@ -87,6 +87,32 @@ def test_swiglu_of_a_strided_view(n, f, k):
     assert (h.double() - want).abs().max() < 0.01 * want.abs().max() + 1e-3
 
 
+@pytest.mark.parametrize("n,f,k,dtype", [(8, 6200, 96, "bfloat16"), (3, 6200, 2048, "bfloat16"), (13, 6200, 2080, "bfloat16"),
+                                         (16, 6152, 4096, "bfloat16"), (33, 6200, 64, "bfloat16"), (2, 6152, 96, "float32"),
+                                         (11, 6200, 96, "float32"), (16, 6152, 2048, "float32")])
+def test_swiglu_of_more_than_three_tiles_a_cu(n, f, k, dtype):
+    """769 and 775 tiles: two a workgroup, one where K is long, the last group not whole; rows as they are and in the lanes' order
+    (16 rows of 4,096 go one tile a workgroup only there) give the same bits.  Bounds: 16-bit results of 32-bit sums; in float32
+    a sum of k products of 0.05 has an error of 2^-24 sqrt(k) of its size, and the gate multiplies two of them."""
+    k_, dt = K(), getattr(torch, dtype)
+    x, w = rnd(n, k, seed=1, scale=0.5).to(dt), rnd(2 * f, k, seed=2, scale=0.1).to(dt)
+    tiled = k_.fused_linear_tile(w, k_.LINEAR_SWIGLU)
+    h = torch.full((n, f), float("nan"), dtype=dt, device=DEV)
+    k_.linear_rows(tiled, h, k_.LINEAR_SWIGLU, x)
+    g = x.double() @ w[:f].double().T
+    want = g * torch.sigmoid(g) * (x.double() @ w[f:].double().T)
+    if dtype == "float32":
+        assert (h.double() - want).abs().max() < 1e-5 * (g.abs().max() ** 2 + 1)
+        return
+    assert (h.double() - want).abs().max() < 0.01 * want.abs().max() + 2e-3
+    xt = k_.TiledRows(torch.zeros(k_.TiledRows.stored(n), k, dtype=dt, device=DEV), n)
+    for r in range(n):
+        for_row = xt.data.view(-1, k // 32, 4, min(n, 16), 8)[r // 16, :, :, r % 16]
+        for_row.copy_(x[r].view(k // 32, 4, 8))
+    k_.linear_rows(tiled, h2 := torch.full_like(h, float("nan")), k_.LINEAR_SWIGLU, xt)
+    assert torch.equal(h2, h)
+
+
 @pytest.mark.parametrize("H,KV,hd,ps,d", [(4, 2, 16, 16, 64), (5, 5, 48, 32, 96), (32, 4, 64, 16, 2048), (3, 3, 80, 16, 128)])
 def test_rope_append(H, KV, hd, ps, d):
     """Projections, rotation and append of 40 tokens of four requests."""

@@ -154,3 +154,14 @@ def test_plain_sums_without_staging_by_size(n, m, k, dtype, unary, want):
     """The lines of the rule, both sides of each."""
     rt, w = _Recorder(dtype), torch.empty(m, k, dtype=dtype)
     assert products.parts_rows(rt, n, w, object(), unary) is want
+
+
+@pytest.mark.parametrize("kind,n,m,tiles", [
+    (K.LINEAR_SWIGLU, 64, 11264, 4), (K.LINEAR_SWIGLU, 64, 4096, 4), (K.LINEAR_ROPE, 64, 2560, 4), (K.LINEAR_ROPE, 64, 6144, 6),
+    (K.LINEAR_RESID, 64, 2048, 2), (K.LINEAR_RESID, 33, 4096, 3), (K.LINEAR_PARTS, 48, 4112, 3), (K.LINEAR_PARTS, 48, 2048, 2)])
+def test_rows_that_the_busiest_cu_reads(kind, n, m, tiles):
+    """As the launch shares the tiles of columns and the halves of the rows out; beyond three tiles of columns a CU the products are not
+    taken with more than 16 rows."""
+    assert K.library().kllm_linear_rows_row_tiles(kind, n, m, 2048) == tiles
+    assert K.linear_rows_best(K.LINEAR_SWIGLU, 17, 12288, 512) and not K.linear_rows_best(K.LINEAR_SWIGLU, 17, 12304, 512)
+    assert K.linear_rows_best(K.LINEAR_SWIGLU, 16, 12304, 512)
