@@ -1017,7 +1017,10 @@ def linear_rows_best(kind, n, m, k, dtype=torch.bfloat16, tiled_x=True) -> bool:
     if kind == LINEAR_RESID and linear_rows_parts(n, m, k) == 0:
         return False
     if n <= 16:
-        return True
+        # Half tiles of a residual product read their rows in twice as many workgroups: not more than four rows that lie as they are
+        # (us, decode-batch kernel / here: 4 rows 2,048 x 2,048 4.9 / 5.3, 16 rows 5.5 / 7.3; a step of 16 tokens of layers of 1,024 columns whose
+        # attention leaves such rows 995 / 1,008).
+        return kind != LINEAR_RESID or tiled_x or n <= 4 or dtype == torch.float32 or linear_rows_parts(n, m, k) == -(-m // 16)
     if kind in (LINEAR_SWIGLU, LINEAR_PARTS) and m > 48 * device_cus():
         return False
     busiest = int(library().kllm_linear_rows_row_tiles(int(kind), int(n), int(m), int(k)))

@@ -165,3 +165,10 @@ def test_rows_that_the_busiest_cu_reads(kind, n, m, tiles):
     assert K.library().kllm_linear_rows_row_tiles(kind, n, m, 2048) == tiles
     assert K.linear_rows_best(K.LINEAR_SWIGLU, 17, 12288, 512) and not K.linear_rows_best(K.LINEAR_SWIGLU, 17, 12304, 512)
     assert K.linear_rows_best(K.LINEAR_SWIGLU, 16, 12304, 512)
+
+
+@pytest.mark.parametrize("n,m,k,dtype,want", [(4, 2048, 2048, BF16, True), (5, 2048, 2048, BF16, False), (16, 512, 1024, BF16, False),
+                                              (16, 2064, 2048, BF16, True), (16, 2048, 2080, BF16, True), (16, 2048, 2048, F32, True)])
+def test_half_tiles_of_weights_want_rows_in_the_lanes_order(n, m, k, dtype, want):
+    assert K.linear_rows_best(K.LINEAR_RESID, n, m, k, dtype, False) is want
+    assert K.linear_rows_best(K.LINEAR_RESID, n, m, k, dtype, True)
