@@ -143,6 +143,8 @@ def _shape(obj, names: _Names):
         return ("t", obj.data_ptr(), tuple(obj.shape), tuple(obj.stride()), obj.dtype)
     if obj is None or isinstance(obj, (bool, int, float, str)):
         return obj
+    if type(obj) is K.TiledRows:
+        return ("r", obj.data.data_ptr(), obj.shape, obj.dtype)
     if isinstance(obj, _OPAQUE):
         raise _Unnamed()
     if isinstance(obj, Part):
@@ -162,7 +164,7 @@ def _shape(obj, names: _Names):
 def _moved(obj, src: _Names, dst: _Names):
     """``obj`` (made by a run with the parts ``src``) as the run with the parts ``dst`` would
     have made it: the same tensors and numbers, that run's parts."""
-    if obj is None or isinstance(obj, (torch.Tensor, bool, int, float, str)):
+    if obj is None or isinstance(obj, (torch.Tensor, bool, int, float, str, K.TiledRows)):
         return obj
     if isinstance(obj, Part):
         return dst.parts[src.path_of[id(obj)]]

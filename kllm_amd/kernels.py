@@ -982,24 +982,31 @@ class TiledRows:
         return n if n <= 16 else -(-n // 16) * 16
 
     def __init__(self, data, n):
-        self.data, self.shape = data, (int(n), int(data.shape[1]))
+        stored, cols = data.shape
+        self.data, self.shape, self.dtype = data, (n, cols), data.dtype
+        self.whole = cols % 32 == 0 and stored == TiledRows.stored(n) and data.is_contiguous() and data.dtype == torch.bfloat16
 
-    @property
-    def dtype(self):
-        return self.data.dtype
+    def pointer(self, name, n):
+        """Address for the kernels, where these are n rows as the kernels store them."""
+        if not self.whole or self.shape[0] != n:
+            raise KernelError(f"linear_rows: tiled rows {self.shape} do not fit {name}, or the kernel takes none")
+        return _ptr(self.data, "linear_rows " + name)
 
 
 @functools.lru_cache(maxsize=4096)
+def _linear_rows_parts(n, m, k) -> int:
+    return int(library().kllm_linear_rows_parts(int(n), int(m), int(k)))
+
+
 def linear_rows_parts(n, m, k) -> int:
     """Partial sums of squares per row that a LINEAR_RESID product on ``linear_rows`` leaves, or 0 where it takes none such."""
-    return int(library().kllm_linear_rows_parts(int(n), int(m), int(k)))
+    return _linear_rows_parts(16 if n <= 16 else 64, m, k)        # (a step of a new size finds the answer of another)
 
 
 LINEAR_ROWS_MAX = 64
 LINEAR_ROWS_BYTES = 380_000
 
 
-@functools.lru_cache(maxsize=4096)
 def linear_rows_best(kind, n, m, k, dtype=torch.bfloat16, tiled_x=True) -> bool:
     """Whether ``linear_rows`` takes the product of n rows against the tiled copy of w [m, k] and is the fastest way.
     Up to 16 rows it always is (a step in us, the decode-batch kernel's products against these: 1 / 4 / 8 / 16 tokens at 1.1B sizes 914 /
@@ -1010,7 +1017,13 @@ def linear_rows_best(kind, n, m, k, dtype=torch.bfloat16, tiled_x=True) -> bool:
     sizes 1,201 / 1,377 / 1,559 / 1,663 against 1,067 / 1,155 / 1,246 / 1,370; with all products at 8B sizes 64 tokens
     4,902 against 6,146), and not with more than three tiles of columns a CU, which workgroups would take one by one (32 rows 14,336 x 1,024 with an
     activation 12.3 us from the tiles, 18.7 here)."""
-    if not 1 <= n <= (LINEAR_ROWS_MAX if dtype == torch.bfloat16 else 16) or k % 32 or k > 1 << 20:
+    # (by tiles of rows, so that a step of a new size finds the answer of another)
+    return 1 <= n <= LINEAR_ROWS_MAX and _linear_rows_best(kind, 4 if n <= 4 else -(-n // 16) * 16, m, k, dtype, tiled_x)
+
+
+@functools.lru_cache(maxsize=4096)
+def _linear_rows_best(kind, n, m, k, dtype, tiled_x):
+    if n > (LINEAR_ROWS_MAX if dtype == torch.bfloat16 else 16) or k % 32 or k > 1 << 20:
         return False
     if dtype == torch.float32 and m * k >= 1 << 29:        # (2 GiB: only the tiled copy could be read, and there may be none)
         return False
@@ -1068,18 +1081,14 @@ def fused_linear(w, y, kind, x, nsplit=1, tiles_per_wg=1, rope=None, act=ACT_SIL
         lo.ss_in, lo.ss_parts, lo.eps = _ptr(sr.ss, "fused_linear ss", torch.float32), sr.parts, sr.eps
     n = x.shape[0]
     lo.kind, lo.nsplit, lo.act = kind, nsplit, int(act)
-    for name, t in (("x", x), ("y", y)):
-        if isinstance(t, TiledRows):
-            if (not _rows or typ != torch.bfloat16 or (name == "y" and kind in (LINEAR_ROPE, LINEAR_PARTS)) or t.dtype != typ or not t.data.is_contiguous()
-                    or t.shape[1] % 32 or t.data.shape[0] != TiledRows.stored(n) or (name == "x" and t.shape[1] != k)):
-                raise KernelError(f"linear_rows: tiled rows {t.shape} do not fit {name}, or the kernel takes none")
-    if isinstance(x, TiledRows):
-        lo.x_tiled, x = 1, x.data[:n]
-    if isinstance(y, TiledRows):
-        lo.y_tiled, y = 1, y.data[:n]
-    if x.dim() != 2 or x.shape[1] != k or x.dtype != typ or x.stride(1) != 1 or not x.is_cuda:
-        raise KernelError(f"fused_linear: x {tuple(x.shape)} {x.dtype} does not fit w {tuple(w.shape)}")
-    x_ptr, x_stride = x.data_ptr(), (x.stride(0) if n > 1 else k)
+    if type(x) is TiledRows:
+        if not _rows or x.shape[1] != k or typ != x.dtype:
+            raise KernelError(f"linear_rows: tiled rows {x.shape} do not fit x, or the kernel takes none")
+        lo.x_tiled, x_ptr, x_stride = 1, x.pointer("x", n), k
+    else:
+        if x.dim() != 2 or x.shape[1] != k or x.dtype != typ or x.stride(1) != 1 or not x.is_cuda:
+            raise KernelError(f"fused_linear: x {tuple(x.shape)} {x.dtype} does not fit w {tuple(w.shape)}")
+        x_ptr, x_stride = x.data_ptr(), (x.stride(0) if n > 1 else k)
     if kind == LINEAR_PARTS and unary is not None:
         code, params = unary
         if nsplit != 1 or (code == ACT_XIELU and (params is None or params.numel() != 2)):
@@ -1126,7 +1135,12 @@ def fused_linear(w, y, kind, x, nsplit=1, tiles_per_wg=1, rope=None, act=ACT_SIL
         raise KernelError(f"fused_linear: unknown output kind {kind}")
     if tuple(y.shape) != want or y.dtype != dt:
         raise KernelError(f"fused_linear: output {tuple(y.shape)} {y.dtype}, expected {want} {dt}")
-    lo.y = _ptr(y, "fused_linear y")
+    if type(y) is TiledRows:
+        if not _rows or kind in (LINEAR_ROPE, LINEAR_PARTS):
+            raise KernelError(f"linear_rows: tiled rows {y.shape} do not fit y, or the kernel takes none")
+        lo.y_tiled, lo.y = 1, y.pointer("y", n)
+    else:
+        lo.y = _ptr(y, "fused_linear y")
     if _rows:
         _launch("kllm_linear_rows", "linear_rows", x_ptr, x_stride, lo, _ptr(w, "linear_rows w"), n, m, k, _stream())
         return
@@ -1279,10 +1293,9 @@ def _rows_side(out, who):
     """(``out_side`` of the call, its tensor) for an output that may be ``TiledRows``."""
     if not isinstance(out, TiledRows):
         return 0, out
-    n, cols = out.shape
-    if cols % 32 or out.data.shape[0] != TiledRows.stored(n) or not out.data.is_contiguous():
+    if not out.whole:
         raise KernelError(f"{who}: tiled rows {out.shape} do not fit")
-    return min(n, 16), out.data
+    return min(out.shape[0], 16), out.data
 
 
 def attn_prefill(q, out, cache, query_tiles, n_tiles, span_start, span_pos, block_table, page_size,

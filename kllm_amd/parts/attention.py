@@ -211,13 +211,18 @@ class CausalSelfAttention(Part):
 
     def forward(self, ctx, xn, cache, sink=None):
         dtype = self.runtime.dtype
+        rows = None                 # whether ``K.linear_rows`` takes the input projections, once it is known
         if isinstance(xn, Normed):
             n = xn.rows
             opts = self.runtime.options
             gemv = (K.gemv_fits(n, self.w_in.shape[0], self.hidden, dtype) and n <= K.normed_max_rows()
                     and not opts.get("no_fused_gemv") and self.plain_rotation and xn.xw is None)
-            scaled = (not gemv and xn.xw is not None
-                      and (self._rows(n, xn) or (self._fused_tiles(n) > 0 and not isinstance(xn.xw, K.TiledRows))))
+            scaled = False
+            if not gemv and xn.xw is not None:
+                rows = self._rows(n, xn)
+                scaled = rows or (self._fused_tiles(n) > 0 and not isinstance(xn.xw, K.TiledRows))
+                if not scaled:
+                    rows = None     # (the rows that the norm makes lie as they are)
             # the small-batch kernel below normalises while it stages its input, the decode-batch
             # kernel scales its sums by the row
             xn = xn.kernel_input() if gemv else xn.scaled_rows() if scaled else xn.materialize(ctx)
@@ -238,7 +243,7 @@ class CausalSelfAttention(Part):
             K.gemv_rope_append(xn, self.w_in, q, cos, sin, pages, ctx.positions, ctx.span_of_token,
                                cache.block_table, cache.page_size, self.heads, self.kv_heads,
                                self.head_dim)
-        elif self._rows(n, xn):
+        elif self._rows(n, xn) if rows is None else rows:
             K.linear_rows(self._tiled.get("in") or self.w_in, q, K.LINEAR_ROPE, xn,
                           rope=K.Rope(cos, sin, pages, ctx.positions, ctx.span_of_token, cache.block_table,
                                       cache.page_size, self.heads, self.kv_heads, self.head_dim))
@@ -253,8 +258,8 @@ class CausalSelfAttention(Part):
             K.rope_append(qkv, q, cos, sin, pages, ctx.positions, ctx.span_of_token,
                           cache.block_table, cache.page_size, self.heads, self.kv_heads,
                           self.head_dim, self.rotary_dim, self.interleaved)
-        if (self.q_dim % 32 == 0 and self.slopes is None and not self.keep_first and self._fast(dtype, cache.page_size)[0]
-                and sink_takes_rows(self.runtime, sink, n, self.w_o, self._tiled.get("o"))):
+        if (sink is not None and n <= K.LINEAR_ROWS_MAX and self.q_dim % 32 == 0 and self.slopes is None and not self.keep_first
+                and sink_takes_rows(self.runtime, sink, n, self.w_o, self._tiled.get("o")) and self._fast(dtype, cache.page_size)[0]):
             out = K.TiledRows(ctx.buf("attn.out", (K.TiledRows.stored(n), self.q_dim), dtype), n)
         else:
             out = ctx.buf("attn.out", (n, self.q_dim), dtype)

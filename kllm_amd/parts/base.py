@@ -46,6 +46,7 @@ from typing import Any, Callable, Dict, List, Optional, Tuple
 
 import torch
 
+from .. import kernels as K
 from .spec import CacheNeed, PartSpec, WeightSpec
 
 CATEGORIES = ("norm", "position", "mixer", "feed_forward", "stream", "block", "embedding", "head")
@@ -107,7 +108,6 @@ class Workspace:
         buf = self._bufs.get(key)
         if buf is None or buf.numel() < numel:
             if buf is not None:
-                from .. import kernels as K
                 K.flush_recorded()   # launches recorded with the old buffer's address run before it goes
                 self.generation += 1
             buf = torch.empty(max(numel, 1), dtype=dtype, device=self.device)
@@ -204,11 +204,9 @@ class Normed:
         return self.x.shape[0]
 
     def kernel_input(self):
-        from .. import kernels as K
         return K.NormedInput(self.x, self.norm.weight, self.ss, self.parts, self.norm.eps)
 
     def scaled_rows(self):
-        from .. import kernels as K
         return K.ScaledRows(self.xw, self.ss, self.parts, self.norm.eps)
 
     def materialize(self, ctx):
@@ -281,7 +279,6 @@ def stream_copy(ctx, x, fill=True):
     read the stream itself: x where the compute dtype is float32; otherwise a buffer that
     whoever last changed x filled in the same launch (``fill`` False: the caller is about to;
     it hands the buffer to its kernel, or None where none is needed), or that is filled here."""
-    from .. import kernels as K
     if ctx.runtime.dtype == torch.float32:
         return x if fill else None
     held = ctx.scratch.get("stream.copy")
@@ -298,7 +295,6 @@ def call_part(part, fn, *args, **kwargs):
     """Call ``fn`` (a method of ``part``) so that its work reaches the stream in program order:
     as it is for a part that records its launches, otherwise with the recorded launches run
     first and recording switched off inside."""
-    from .. import kernels as K
     if getattr(part, "records_launches", False) or not K.recording():
         return fn(*args, **kwargs)
     with K.direct_launches():

@@ -195,12 +195,21 @@ def fused_f32(rt, n, m=None):
             and not opts.get("no_mfma_f32") and opts.get("gemm_algo") is None)
 
 
+def _rows_options(rt, n, f32, w_tiled):
+    """Whether the engine's options and the copy of the weights (for bfloat16) leave n rows to ``K.linear_rows``."""
+    if f32:
+        return fused_f32(rt, n)
+    opts = rt.options
+    return (w_tiled is not None and opts.get("gemm") != "library" and not opts.get("no_fused_linear")
+            and opts.get("gemm_algo") is None)
+
+
 def rows_kernel(rt, kind, n, w, w_tiled, tiled_x):
     """Whether a product of n rows (``TiledRows``: ``tiled_x``) with the step after it runs on ``K.linear_rows``."""
-    f32 = w.dtype == torch.float32
-    return ((fused_f32(rt, n) if f32 else w_tiled is not None and rt.options.get("gemm") != "library")
-            and not rt.options.get("no_fused_linear") and rt.options.get("gemm_algo") is None
-            and K.linear_rows_best(kind, n, w.shape[0], w.shape[1], w.dtype, tiled_x))
+    if n > K.LINEAR_ROWS_MAX:
+        return False
+    dtype, (m, k) = w.dtype, w.shape
+    return K.linear_rows_best(kind, n, m, k, dtype, tiled_x) and _rows_options(rt, n, dtype == torch.float32, w_tiled)
 
 
 def _sink_fits(rt, sink, n, m):
@@ -229,7 +238,7 @@ def _resid_rows(rt, norm, n, w, w_tiled, tiled_x):
 
 def sink_takes_rows(rt, sink, n, w, w_tiled):
     """Whether ``linear_into`` will run the product of ``TiledRows`` on ``K.linear_rows``."""
-    return sink is not None and w.dtype == torch.bfloat16 and _sink_fits(rt, sink, n, w.shape[0]) and _resid_rows(rt, sink.norm, n, w, w_tiled, True)
+    return sink is not None and n <= K.LINEAR_ROWS_MAX and w.dtype == torch.bfloat16 and _sink_fits(rt, sink, n, w.shape[0]) and _resid_rows(rt, sink.norm, n, w, w_tiled, True)
 
 
 def linear_into(ctx, x, w, sink, tag, w_tiled=None):
@@ -243,11 +252,12 @@ def linear_into(ctx, x, w, sink, tag, w_tiled=None):
     n, k = x.shape
     m = w.shape[0]
     rt = ctx.runtime
-    if not _sink_fits(rt, sink, n, m):
+    rows = isinstance(x, K.TiledRows)            # (``sink_takes_rows`` said so)
+    if not rows and not _sink_fits(rt, sink, n, m):
         return None
     norm = sink.norm
     f32 = x.dtype == torch.float32
-    rows = _resid_rows(rt, norm, n, w, w_tiled, isinstance(x, K.TiledRows))
+    rows = rows or _resid_rows(rt, norm, n, w, w_tiled, False)
     parts = 0 if f32 and (rows or fused_f32(rt, n, m)) else K.resid_parts(n, m, k, x.dtype)
     if parts:
         ss = ctx.buf(tag + ".ss", (n, -(-parts // 4) * 4), torch.float32)
@@ -256,7 +266,8 @@ def linear_into(ctx, x, w, sink, tag, w_tiled=None):
     if rows:
         parts = K.linear_rows_parts(n, m, k)
         stride = -(-parts // 4) * 4          # (room for eight columns to a sum whatever n is: a smaller step must not ask for more)
-        ss = ctx.buf(tag + ".ss", (n * max(stride, -(-m // 32) * 4),), torch.float32)[:n * stride].view(n, stride)
+        ctx.buf(tag + ".ss", (n * max(stride, -(-m // 32) * 4),), torch.float32)
+        ss = ctx.buf(tag + ".ss", (n, stride), torch.float32)
         if _feeds_rows(norm, n):
             xw = K.TiledRows(ctx.buf(tag + ".xw", (K.TiledRows.stored(n), m), x.dtype), n)     # for the product behind the norm
         else:
@@ -335,6 +346,7 @@ def decode_batch_fits(rt, x, m):
     return n <= 16 and K.fused_linear_fits(n, k, 1, x.dtype)
 
 
+@functools.lru_cache(maxsize=4096)
 def _parts_best(n, m, k, dtype, unary):
     """Whether ``K.linear_rows`` is the fastest way to plain sums, or (``unary``) an activation of them, of n rows that are read row by row.
     The decode-batch kernel has the rows in LDS, this one reads up to sixteen of them a load: up to eight rows it is the faster one where
@@ -345,6 +357,8 @@ def _parts_best(n, m, k, dtype, unary):
     prompt of 20 1,004 / 761, of 60 1,146 / 1,131), but for sums of little K and, beyond 32 rows, of long K (a product and a
     kernel that adds the slices, there / here: 48 rows 1,024 x 64 6.1 / 7.6, 1,024 x 2,816 8.9 / 12.3), nor for more than three
     tiles of columns a CU (32 rows 14,336 x 1,024 with the activation 12.3 / 18.7)."""
+    if m >= 16384 or not K.linear_rows_best(K.LINEAR_PARTS, n, m, k, dtype, False):
+        return False
     if dtype == torch.float32:
         return n <= 5 or n <= 8 and (k > 512 or m > 2048)      # (8 rows, 2,048 x 512: 4.5 us there, 4.8 here; 2,816 x 512 5.2 / 5.0)
     if n <= 8:
@@ -356,8 +370,10 @@ def _parts_best(n, m, k, dtype, unary):
 
 def parts_rows(rt, n, w, w_tiled, unary=False):
     """Whether ``decode_linear`` runs on ``K.linear_rows`` (``_parts_best``)."""
-    return (w.shape[0] < 16384 and _parts_best(n, w.shape[0], w.shape[1], w.dtype, unary)
-            and rows_kernel(rt, K.LINEAR_PARTS, n, w, w_tiled, False))
+    if n > K.LINEAR_ROWS_MAX:
+        return False
+    dtype, (m, k) = w.dtype, w.shape
+    return _parts_best(n if n <= 8 else -(-n // 16) * 16, m, k, dtype, unary) and _rows_options(rt, n, dtype == torch.float32, w_tiled)
 
 
 def decode_linear(ctx, x, w, tag, w_tiled=None, unary=None):
