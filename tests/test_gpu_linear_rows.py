@@ -1,6 +1,7 @@
-"""Products of 17 to 64 rows with the step after them (``kernels.linear_rows``) against float64 references: row
-tiles that are whole and not, one and two halves of the rows, one to three tiles a workgroup, K that gives the eight
-waves unequal shares or none."""
+"""Products of 1 to 64 rows with the step after them (``kernels.linear_rows``) against float64 references: row
+tiles that are whole and not, one and two halves of the rows, half tiles of the weights (up to 16 rows, where tiles are few), one to
+three tiles a workgroup, K that gives the eight waves unequal shares or none, bfloat16 and (up to 16 rows) float32; and the
+attention kernels that write their rows in the order these products read."""
 
 import pytest
 import torch
@@ -11,7 +12,8 @@ from test_gpu_kernels import DEV, K, _bf, read_cache, rnd
 pytestmark = pytest.mark.gpu
 
 
-# Tiles of W at most half the CUs: two workgroups share the rows (2,048 and below); more: one (4,096).
+# Tiles of W at most half the CUs (2,048 columns and below): two workgroups share the rows beyond 16, or a tile of the weights up to
+# 16 rows; more (4,096): one, or two halves of the rows.
 @pytest.mark.parametrize("n,m,k", [(1, 16, 32), (17, 48, 96), (5, 64, 2048), (8, 2048, 5632), (3, 72, 448), (9, 40, 64), (16, 2048, 2048), (12, 1000, 1152), (16, 4096, 320), (33, 72, 288), (45, 2048, 2048), (48, 100, 5632),
                                    (64, 2048, 5632), (64, 4096, 1056), (50, 4096, 4096), (32, 1000, 736), (63, 4090, 160)])
 def test_resid_then_scaled_consumers(n, m, k):
@@ -160,9 +162,11 @@ def test_refusals():
 
 
 @pytest.mark.parametrize("n,m,k", [(1, 40, 64), (8, 2048, 2048), (5, 72, 96), (13, 2048, 1536), (16, 5632, 2048), (20, 5632, 512),
-                                   (33, 4096, 1056), (64, 2048, 5632), (45, 12300, 160), (3, 9000, 544)])
+                                   (33, 4096, 1056), (64, 2048, 5632), (45, 12300, 160), (3, 9000, 544), (45, 12200, 160),
+                                   (20, 8400, 96), (64, 12288, 64)])
 def test_sums_and_activations_of_them(n, m, k):
-    """Plain sums, and an activation of them in 16 bits: half tiles of W, whole ones, two and three a workgroup."""
+    """Plain sums, and an activation of them in 16 bits: half tiles of W, whole ones, two (5,632 columns) and three (8,400 to 12,288)
+    a workgroup, and one of 769 tiles (12,300)."""
     k_ = K()
     x, w = _bf(n, k, seed=1, scale=0.5), _bf(m, k, seed=2, scale=0.1)
     tiled = k_.fused_linear_tile(w, k_.LINEAR_PARTS)
@@ -221,6 +225,17 @@ def test_attention_writes_tiled_rows(H, KV, hd, ps, slices):
                     k_.attn_prefill(q, o, cache, tiles, len(spans), start, span_pos, bt, ps, H, KV, hd, 0, hd ** -0.5,
                                     keys, keys)
                 assert torch.equal(_rowwise(tiled), out)
+            most = k_.attn_prefill_slices(len(spans), H, hd)
+            assert (most > 1) == (hd == 128)
+            if most > 1:                         # the blocks' keys in slices, merged in the same call
+                part = torch.full((n * H * most * (hd + 2),), float("nan"), device=DEV)
+                out2 = torch.zeros_like(out)
+                tiled.data.zero_()
+                for o in (out2, tiled):
+                    k_.attn_prefill(q, o, cache, tiles, len(spans), start, span_pos, bt, ps, H, KV, hd, 0, hd ** -0.5,
+                                    10 ** 6, 10 ** 6, part=part, nslices=most)
+                # (16-bit results, the slices' sums in 32: one rounding apart)
+                assert torch.equal(_rowwise(tiled), out2) and (out2 - out).abs().max() <= 2.0 ** -7 * out.abs().max()
 
 
 @pytest.mark.parametrize("n,m,k", [(5, 64, 64), (8, 2048, 2048), (8, 2048, 5632), (13, 72, 448), (16, 2048, 5632), (16, 4096, 4096),
