@@ -191,9 +191,10 @@ class CausalSelfAttention(Part):
                              f"(1 to {K.GENERIC_MAX_PAGE_SIZE})")
 
     def rows_input(self):
-        """(kind, rows, columns) of the input projections, where ``K.linear_rows`` may take them (``K.linear_rows_best``): in
-        bfloat16 from their tiled copy only."""
-        return (K.LINEAR_ROPE, *self.w_in.shape) if self._tiled.get("in") is not None or self.w_in.dtype == torch.float32 else None
+        """(kind, rows, columns, whether there is a tiled copy) of the input projections, where ``K.linear_rows`` may take them
+        (``K.linear_rows_best``): in bfloat16 from the copy only."""
+        copied = self._tiled.get("in") is not None
+        return (K.LINEAR_ROPE, *self.w_in.shape, copied) if copied or self.w_in.dtype == torch.float32 else None
 
     def _rows(self, n, x):
         """Whether the input projections of the rows x run on ``K.linear_rows``."""
@@ -204,7 +205,7 @@ class CausalSelfAttention(Part):
         """Tiles per workgroup of the decode-batch kernel for the input projections of n
         tokens, or 0 where it is not taken."""
         rt = self.runtime
-        best = fused_f32(rt, n, self.w_in.shape[0]) if rt.dtype == torch.float32 else n <= K.FUSED_ROPE_BEST_ROWS
+        best = fused_f32(rt, n, *self.w_in.shape, self._tiled.get("in") is not None) if rt.dtype == torch.float32 else n <= K.FUSED_ROPE_BEST_ROWS
         if not best or not self.plain_rotation or rt.options.get("no_fused_linear"):
             return 0
         return K.fused_linear_tiles(n, self.w_in.shape[0], self.hidden, rt.dtype)

@@ -50,9 +50,10 @@ class GatedFeedForward(Part):
                        "down": tiled_copy(self.runtime, self.w_down, K.LINEAR_PARTS)}
 
     def rows_input(self):
-        """(kind, rows, columns) of the gate and up product, where ``K.linear_rows`` may take it (``K.linear_rows_best``): in
-        bfloat16 from its tiled copy only."""
-        return (K.LINEAR_SWIGLU, *self.w_gu.shape) if self._tiled.get("gu") is not None or self.w_gu.dtype == torch.float32 else None
+        """(kind, rows, columns, whether there is a tiled copy) of the gate and up product, where ``K.linear_rows`` may take it
+        (``K.linear_rows_best``): in bfloat16 from the copy only."""
+        copied = self._tiled.get("gu") is not None
+        return (K.LINEAR_SWIGLU, *self.w_gu.shape, copied) if copied or self.w_gu.dtype == torch.float32 else None
 
     def _gate_in_tiles(self, n, dtype):
         """Decode batches whose gate runs in the tiled product's epilogue: more than 32 rows
@@ -69,7 +70,8 @@ class GatedFeedForward(Part):
         dtype, opts = self.runtime.dtype, self.runtime.options
         n = xn.rows if isinstance(xn, Normed) else xn.shape[0]
         gemv = K.gemv_fits(n, 2 * self.intermediate, self.hidden, dtype) and not opts.get("no_fused_gemv")
-        best = fused_f32(self.runtime, n, 2 * self.intermediate) if dtype == torch.float32 else n <= K.FUSED_SWIGLU_BEST_ROWS
+        best = (fused_f32(self.runtime, n, *self.w_gu.shape, self._tiled.get("gu") is not None) if dtype == torch.float32
+                else n <= K.FUSED_SWIGLU_BEST_ROWS)
         tiles = K.fused_linear_tiles(n, 2 * self.intermediate, self.hidden, dtype) if best else 0
         rows = rows_kernel(self.runtime, K.LINEAR_SWIGLU, n, self.w_gu, self._tiled.get("gu"),
                            isinstance(getattr(xn, "xw", xn), K.TiledRows))
@@ -162,7 +164,7 @@ def dense_hidden(ctx, xn, w_up, tag, tiled, act, params=None):
     if (n > 128 and opts.get("gemm") != "library" and opts.get("gemm_algo") is None
             and xn.shape[1] % (8 if xn.dtype == torch.bfloat16 else 4) == 0):
         K.gemm_act(xn, w_up, h, act, params)      # prompts
-    elif parts_rows(ctx.runtime, n, w_up, tiled, True) or (decode_batch_fits(ctx.runtime, xn, w_up.shape[0]) and not opts.get("no_fused_linear")
+    elif parts_rows(ctx.runtime, n, w_up, tiled, True) or (decode_batch_fits(ctx.runtime, xn, w_up.shape[0], tiled is not None) and not opts.get("no_fused_linear")
                                                      and opts.get("gemm_algo") is None):
         h = decode_linear(ctx, xn, w_up, tag + ".h", tiled, unary=(act, params))      # decode batches
     else:

@@ -179,7 +179,7 @@ def tiled_copy(runtime, w, kind, rope=None):
     return K.fused_linear_tile(w, kind, rope)
 
 
-def fused_f32(rt, n, m=None):
+def fused_f32(rt, n, m=None, k=None, copied=True):
     """Whether a float32 decode batch of n tokens runs on the matrix cores, with the step after a product in its launch
     (``K.linear_rows``, or the decode-batch kernel for sizes that one does not take: ``m``, the product's columns).  One row stays with the
     gemv, which has the same epilogues
@@ -189,16 +189,19 @@ def fused_f32(rt, n, m=None):
     not, and from nine on K went in slices whose sums other kernels added (16 at 8B sizes: 14.6 ms against 9.7 on the
     decode-batch kernel; 12: 9.1 there, 7.0 now).  The decode-batch kernel stages all rows first: two rows stay with the gemv, too, where it
     has fewer tiles than there are CUs (a step, gemv / decode-batch kernel, 2 / 3 / 4 tokens: width 2,040 x 8 layers 716 / 884 / 896 us against
-    735 / 836 / 850; width 4,112 x 4 layers 896 / 912 / 929 against 864 / 850 / 898)."""
+    735 / 836 / 850; width 4,112 x 4 layers 896 / 912 / 929 against 864 / 850 / 898).  Without the copy of the weights (not
+    ``copied``) two rows leave the gemv, which reads the weights in whole rows, only for ``K.linear_rows`` with ``k`` beyond 1,024 (a product alone
+    1,024 x 1,024 3.9 / 4.9 us; a step of 2 tokens, layers of 1,024 columns, 692 / 739, of 2,048 839 / 797; of 5,120, whose residual products
+    went to the decode-batch kernel, 1,173 / 1,264)."""
     opts = rt.options
-    return (2 <= n <= 16 and (n > 2 or m is None or m >= 16 * K.device_cus()) and not opts.get("no_fused_linear")
-            and not opts.get("no_mfma_f32") and opts.get("gemm_algo") is None)
+    return (2 <= n <= 16 and (n > 2 or ((copied or k is None or k > 1024) if m is None else copied and m >= 16 * K.device_cus()))
+            and not opts.get("no_fused_linear") and not opts.get("no_mfma_f32") and opts.get("gemm_algo") is None)
 
 
-def _rows_options(rt, n, f32, w_tiled):
-    """Whether the engine's options and the copy of the weights (for bfloat16) leave n rows to ``K.linear_rows``."""
+def _rows_options(rt, n, k, f32, w_tiled):
+    """Whether the engine's options and the copy of the weights leave n rows of k to ``K.linear_rows``."""
     if f32:
-        return fused_f32(rt, n)
+        return fused_f32(rt, n, None, k, w_tiled is not None)
     opts = rt.options
     return (w_tiled is not None and opts.get("gemm") != "library" and not opts.get("no_fused_linear")
             and opts.get("gemm_algo") is None)
@@ -209,7 +212,7 @@ def rows_kernel(rt, kind, n, w, w_tiled, tiled_x):
     if n > K.LINEAR_ROWS_MAX:
         return False
     dtype, (m, k) = w.dtype, w.shape
-    return K.linear_rows_best(kind, n, m, k, dtype, tiled_x) and _rows_options(rt, n, dtype == torch.float32, w_tiled)
+    return K.linear_rows_best(kind, n, m, k, dtype, tiled_x) and _rows_options(rt, n, k, dtype == torch.float32, w_tiled)
 
 
 def _sink_fits(rt, sink, n, m):
@@ -224,15 +227,21 @@ def _feeds_rows(norm, n):
     return feeds is not None and norm.runtime.dtype == torch.bfloat16 and K.linear_rows_best(feeds[0], n, feeds[1], feeds[2])
 
 
+def _feeds_f32(rt, norm, n):
+    """Whether the float32 product behind ``norm`` has a use for scaled rows: not where it stays with the gemv, which makes its rows'
+    norm itself."""
+    feeds = getattr(norm, "feeds", None)
+    if feeds is None:
+        return True
+    kind, m, k, copied = feeds
+    return fused_f32(rt, n, None if K.linear_rows_best(kind, n, m, k, torch.float32) else m, k, copied)
+
+
 def _resid_rows(rt, norm, n, w, w_tiled, tiled_x):
     """Whether a residual product runs on ``K.linear_rows``: beyond 16 rows only where the next product does, too (a step of 32
-    tokens at 8B sizes, whose gate product does not, 4,234 us without and 4,370 with the output projection here); two rows of float32
-    not where the next product stays with the gemv, which makes its rows' norm itself and has no use for scaled ones."""
+    tokens at 8B sizes, whose gate product does not, 4,234 us without and 4,370 with the output projection here)."""
     if not rows_kernel(rt, K.LINEAR_RESID, n, w, w_tiled, tiled_x):
         return False
-    if w.dtype == torch.float32:
-        feeds = getattr(norm, "feeds", None)
-        return feeds is None or fused_f32(rt, n, feeds[1]) or K.linear_rows_best(feeds[0], n, feeds[1], feeds[2], torch.float32)
     return n <= 16 or _feeds_rows(norm, n)
 
 
@@ -257,8 +266,9 @@ def linear_into(ctx, x, w, sink, tag, w_tiled=None):
         return None
     norm = sink.norm
     f32 = x.dtype == torch.float32
-    rows = rows or _resid_rows(rt, norm, n, w, w_tiled, False)
-    parts = 0 if f32 and (rows or fused_f32(rt, n, m)) else K.resid_parts(n, m, k, x.dtype)
+    rows = rows or ((not f32 or _feeds_f32(rt, norm, n)) and _resid_rows(rt, norm, n, w, w_tiled, False))
+    fused = f32 and (rows or fused_f32(rt, n, m, k, w_tiled is not None) and _feeds_f32(rt, norm, n))
+    parts = 0 if fused else K.resid_parts(n, m, k, x.dtype)
     if parts:
         ss = ctx.buf(tag + ".ss", (n, -(-parts // 4) * 4), torch.float32)
         K.linear_resid(x, w, sink.x, ss)
@@ -274,7 +284,7 @@ def linear_into(ctx, x, w, sink, tag, w_tiled=None):
             xw = ctx.buf(tag + ".xw", (n, m), x.dtype)
         K.linear_rows(w_tiled or w, xw, K.LINEAR_RESID, x, resid=sink.x, norm_weight=norm.weight, ss_out=ss)
         return Normed(sink.x, ss, parts, norm, xw=xw)
-    if not (fused_f32(rt, n, m) if f32 else n <= K.FUSED_NORM_BEST_ROWS) or rt.options.get("no_fused_linear"):
+    if not (fused if f32 else n <= K.FUSED_NORM_BEST_ROWS) or rt.options.get("no_fused_linear"):
         return None
     # a decode batch on the matrix cores: all of K in a workgroup, the addition in the epilogue, and
     # beside the stream its rows times the norm's weight in the compute dtype for a consumer that scales its sums
@@ -337,17 +347,17 @@ def linear(ctx, x, w, tag, out_dtype=torch.float32, split=True, w_tiled=None):
     return y
 
 
-def decode_batch_fits(rt, x, m):
+def decode_batch_fits(rt, x, m, copied=True):
     """Whether a product of these rows with m columns runs on the decode-batch kernel (up to 16 rows, all of K
     in a workgroup; float32 see ``fused_f32``)."""
     n, k = x.shape
-    if x.dtype == torch.float32 and not fused_f32(rt, n, m):
+    if x.dtype == torch.float32 and not fused_f32(rt, n, m, k, copied):
         return False
     return n <= 16 and K.fused_linear_fits(n, k, 1, x.dtype)
 
 
 @functools.lru_cache(maxsize=4096)
-def _parts_best(n, m, k, dtype, unary):
+def _parts_best(n, m, k, dtype, unary, copied=True):
     """Whether ``K.linear_rows`` is the fastest way to plain sums, or (``unary``) an activation of them, of n rows that are read row by row.
     The decode-batch kernel has the rows in LDS, this one reads up to sixteen of them a load: up to eight rows it is the faster one where
     K is long enough, of 9 to 16 not (a step of Nusilix layers of 1,024 columns, there / here, with K of 1,024 here, too: 1 token 601 / 608 us, 2
@@ -360,6 +370,8 @@ def _parts_best(n, m, k, dtype, unary):
     if m >= 16384 or not K.linear_rows_best(K.LINEAR_PARTS, n, m, k, dtype, False):
         return False
     if dtype == torch.float32:
+        if not copied and (n == 2 and k <= 2048 or n > 5 and k <= 1024):
+            return False          # (without the copy, 8 rows 1,024 x 1,024 5.1 us by the gemv, 5.4 here)
         return n <= 5 or n <= 8 and (k > 512 or m > 2048)      # (8 rows, 2,048 x 512: 4.5 us there, 4.8 here; 2,816 x 512 5.2 / 5.0)
     if n <= 8:
         return k > 1024 and (n <= 6 or k > 2048 or m > 2048)
@@ -373,7 +385,7 @@ def parts_rows(rt, n, w, w_tiled, unary=False):
     if n > K.LINEAR_ROWS_MAX:
         return False
     dtype, (m, k) = w.dtype, w.shape
-    return _parts_best(n if n <= 8 else -(-n // 16) * 16, m, k, dtype, unary) and _rows_options(rt, n, dtype == torch.float32, w_tiled)
+    return _parts_best(n if n <= 8 else -(-n // 16) * 16, m, k, dtype, unary, w_tiled is not None) and _rows_options(rt, n, k, dtype == torch.float32, w_tiled)
 
 
 def decode_linear(ctx, x, w, tag, w_tiled=None, unary=None):
@@ -389,7 +401,7 @@ def decode_linear(ctx, x, w, tag, w_tiled=None, unary=None):
         y = ctx.buf(tag, (n, m) if unary is not None else (1, n, m), x.dtype if unary is not None else torch.float32)
         K.linear_rows(w_tiled or w, y, K.LINEAR_PARTS, x, unary=unary)
         return y if unary is not None else y[0]
-    if decode_batch_fits(rt, x, m) and not rt.options.get("no_fused_linear") and rt.options.get("gemm_algo") is None:
+    if decode_batch_fits(rt, x, m, w_tiled is not None) and not rt.options.get("no_fused_linear") and rt.options.get("gemm_algo") is None:
         tiles = 4 if m >= 16384 else 1
         if unary is not None:
             y = ctx.buf(tag, (n, m), x.dtype)

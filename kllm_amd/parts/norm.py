@@ -23,7 +23,7 @@ class RMSNorm(Part):
     graph_safe = True
     records_launches = True
     fusable = True     # a product's epilogue may do the addition, its consumer the row scale
-    feeds = None       # (output kind, rows and columns of the weights) of the product behind it, if that has a tiled copy of them
+    feeds = None       # the product behind it that may take its rows in the lanes' order or scaled: see ``rows_input`` of the parts
 
     def __init__(self, spec, runtime):
         super().__init__(spec, runtime)

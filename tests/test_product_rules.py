@@ -116,21 +116,29 @@ class _Recorder:
     (2, 2040, 2040, None, "gemv"), (3, 2040, 2040, None, "decode_batch"), (2, 4112, 4112, None, "decode_batch"),
     (2, 2048, 5632, (K.LINEAR_ROPE, 2560, 2048), "rows"), (2, 2040, 5632, (K.LINEAR_ROPE, 2856, 2040), "gemv"),
     (3, 2040, 5632, (K.LINEAR_ROPE, 2856, 2040), "rows"), (2, 2040, 5632, (K.LINEAR_SWIGLU, 11264, 2040), "rows"),
-    (1, 2048, 2048, None, "gemv"), (5, 2040, 2040, None, "decode_batch")])
-def test_few_rows_of_float32_leave_the_gemv_where_that_is_the_faster_way(n, m, k, feeds, kernel, monkeypatch):
+    (1, 2048, 2048, None, "gemv"), (5, 2040, 2040, None, "decode_batch"), (4, 1024, 1024, None, "rows"),
+    (4, 1024, 2816, (K.LINEAR_ROPE, 1536, 1024), "rows"), (2, 1024, 2816, (K.LINEAR_ROPE, 1536, 1024), "rows")])
+@pytest.mark.parametrize("copied", [True, False])
+def test_few_rows_of_float32_leave_the_gemv_where_that_is_the_faster_way(n, m, k, feeds, kernel, copied, monkeypatch):
     """Two rows whose K is in no whole steps stay with the gemv unless the decode-batch kernel has a tile for every CU; so do those
-    whose scaled rows the product behind the norm would not take."""
+    whose scaled rows the product behind the norm would not take.  Without the copy of the weights two rows leave it only where nothing
+    is staged and K is beyond 1,024."""
     went = []
+    if not copied and n == 2 and not (m == 2048 and feeds):
+        kernel = "gemv"
     monkeypatch.setattr(K, "linear_resid", lambda *a, **b: went.append("gemv"))
     monkeypatch.setattr(K, "linear_rows", lambda *a, **b: went.append("rows"))
     monkeypatch.setattr(K, "fused_linear", lambda *a, **b: went.append("decode_batch"))
-    rt = _Recorder(F32, feeds)
+    rt = _Recorder(F32, feeds and (*feeds, copied))
     rt.weight = torch.empty(m)
     rt.eps = 1e-5
     x, w = torch.empty(n, k), torch.empty(m, k)
-    normed = products.linear_into(rt, x, w, ResidualSink(torch.empty(n, m), rt), "t")
-    assert went == [kernel] and (normed.xw is None) == (kernel == "gemv")
-    assert products.decode_batch_fits(rt, x, m) == (n > 2 or n == 2 and m >= 4096)
+    normed = products.linear_into(rt, x, w, ResidualSink(torch.empty(n, m), rt), "t", object() if copied else None)
+    if kernel == "gemv" and K.resid_parts(n, m, k, F32) == 0:       # (more columns than its sums of squares are read for)
+        assert normed is None and not went
+    else:
+        assert went == [kernel] and (normed.xw is None) == (kernel == "gemv")
+    assert products.decode_batch_fits(rt, x, m, copied) == (n > 2 or n == 2 and m >= 4096 and copied)
 
 
 @pytest.mark.parametrize("lens,head_dim,want", [
