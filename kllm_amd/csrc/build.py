@@ -22,10 +22,12 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_NAME = "libkllm_hip.so"
 ARCH = "gfx950"
-# Packed 32-bit float instructions are switched off for all device code.
+# Packed 32-bit float instructions are switched off for all device code.  A kernel's first arguments (fourteen words at most, up
+# to the first struct) are in scalar registers when a wave starts, instead of a trip to memory away: a decode step of 140 launches
+# at 1.1B sizes 874 -> 856 us by that alone.
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-         "-Wno-unused-result"]
+         "-mllvm", "-amdgpu-kernarg-preload-count=16", "-Wno-unused-result"]
 
 
 class BuildError(RuntimeError):

@@ -18,10 +18,16 @@
 // kilobyte, or less where there are fewer rows than 16.  From rows as they are, its sixteen lanes with one K lie in sixteen
 // rows, and a CU takes in 16 bytes a clock (64 rows of 5,632 against 2,048 columns: 15.8 -> 12.1 us; 16 rows 11.2 -> 10.1).
 //
-// Alone in a replayed graph, 8 / 64 rows, us: 2,048 x 2,048 4.6 / 7.2 (rows as attention leaves them); 2,048 x 5,632 9.9 / 12.2; 2 x
-// 5,632 x 2,048 11.0 / 14.5; 2,560 x 2,048 4.6 / 6.8; 4,096 x 14,336 23.4 / 41.0 (117 MB: 5.0 TB/s at 8 rows).  A decode step at
-// 1.1B sizes and contexts of 600, with fused_linear.hip's products and the tiles' and with these: 1 token 914 -> 888 us, 8 971
-// -> 937, 16 1,080 -> 1,031, 32 1,377 -> 1,155, 64 1,663 -> 1,370.
+// At a few rows a launch is mostly its own beginning and end: of 4.9 us for 2,048 x 2,048 at one row the weights take 1.6.  So what the
+// loads of the weights need comes with the launch (the first fourteen words of the arguments lie in scalar registers when a wave starts; a trip
+// to the arguments is 0.3 us in a cold cache, and there were three in a row), they are the first thing that a wave asks for, and
+// what only the epilogue needs comes behind them.
+//
+// Alone in a replayed graph, 1 / 8 / 16 / 64 rows (tiled, but for 2,048 x 2,048), us, before that and now: 2,048 x 2,048 4.9 / 5.8 /
+// 7.3 / 7.7, 3.7 / 4.2 / 5.0 / 7.0; 2,048 x 5,632 7.5 / 8.0 / 9.4 / 12.0, 6.4 / 6.8 / 8.0 / 11.2; 2 x 5,632 x 2,048 10.9 / 11.0 / 11.3 / 14.1, 10.1 /
+// 10.2 / 10.6 / 13.9; plain sums 2,560 x 2,048 4.6 / 4.8 / 5.2 / 8.6, 3.9 / 4.2 / 4.5 / 8.0; 4,096 x 4,096 8.9 / 9.2 / 9.3 / 14.6, 7.9 / 8.1 / 8.3
+// / 13.8; 4,096 x 14,336 23.5 / 24.1 / 25.9 / 44.7, 22.8 / 23.1 / 25.0 / 42.6 (117 MB: 5.1 TB/s).  A decode step at 1.1B sizes, 1 / 8 / 64 tokens
+// 874 / 945 / 1,575 -> 794 / 868 / 1,530 us, 45 tokens of prompt 1,027 -> 958, 8B sizes at 16 tokens 3,980 -> 3,855, float32 at 8 1,565 -> 1,510.
 #include <math.h>
 
 #include "common.hpp"
@@ -39,6 +45,7 @@ constexpr int LR_TILE = 16 * LR_LD;
 // Steps of K in each of the two buffers a wave fills in turn: what 128 registers hold, four at most.
 constexpr int lr_ahead(int nt, int tw) { return nt + tw <= 4 ? 4 : nt + tw == 5 ? 3 : 2; }
 
+// A: steps of K in each of the two buffers.
 // SPLIT (FL_RESID and FL_PARTS, up to 16 rows): a workgroup takes eight rows of W, each twice in a matrix instruction: K's first half in its rows
 // 0-7, the second half in rows 8-15, so that a load still brings a kilobyte.  Up to eight rows of X lie in the operand's columns the
 // same way (NT 1); more take an instruction for each half of K (NT 2).  What pairs a half with the other's X is not used.  A CU streams
@@ -60,84 +67,62 @@ __device__ __forceinline__ void lr_mma(uintx4 w, uintx4 x, floatx4 (&acc)[CH], i
   }
 }
 
-template <typename T, int NT, int TW, int EP, bool SCALED, int NW, bool SPLIT>
-__global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const T* __restrict__ X, FlOut out, const T* __restrict__ W, int n,
-                                                              int m, int k, int tiles, int halves, int x_stride) {
-  constexpr int ES = (int)sizeof(T), CH = lr_chains<T, EP>();
-  constexpr int A = lr_ahead(NT, TW);
+enum : unsigned { LR_HALVES = 1, LR_X_TILED = 2, LR_W_TILED = 4 };
+
+template <typename T, int NT, int TW, int EP, bool SCALED, int NW, bool SPLIT, int A>
+__global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const T* __restrict__ W, const T* __restrict__ X, int m, int k,
+                                                              int x_stride, unsigned how, const int* __restrict__ positions,
+                                                              const int* __restrict__ span_of_token, const float* __restrict__ ss_in,
+                                                              FlOut out) {
+  const int n = how >> 8 & 0xFF, ss_parts = how >> 16;
+  constexpr int ES = (int)sizeof(T), CH = lr_chains<T, EP>();    // (n and ss_parts share a word with the flags: all of it in fourteen)
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   float* part = reinterpret_cast<float*>(lds_raw);               // [NW][TW][NT][x row 16][LR_LD]
   float* row_scale = part + NW * TW * NT * LR_TILE;              // [16 NT]
   const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int g = lane / 16, c = lane % 16;
-  const int groups = (tiles + TW - 1) / TW;                      // workgroups side by side over W
+  const int tiles = EP == FL_RESID || EP == FL_PARTS ? (int)((unsigned)(m + 15) / 16) : (int)((unsigned)(m / 2 + 7) / 8);
+  const int groups = (int)((unsigned)(tiles + TW - 1) / TW);     // workgroups side by side over W
+  const bool halved = how & LR_HALVES;
   // Blocks go to the XCDs in turn: two workgroups of one group of tiles are eight blocks apart.
-  const int group = SPLIT ? (int)blockIdx.x / 2
-                    : halves == 1 ? (int)blockIdx.x : (int)(blockIdx.x / 16) * 8 + (int)(blockIdx.x % 8);
-  const int half_tile = SPLIT ? (int)blockIdx.x % 2 : 0;         // which eight rows of W
-  const int row0 = halves == 1 ? 0 : (int)(blockIdx.x / 8 % 2) * (16 * NT);
+  const int group = SPLIT ? (int)(blockIdx.x / 2) : !halved ? (int)blockIdx.x : (int)(blockIdx.x / 16) * 8 + (int)(blockIdx.x % 8);
+  const int half_tile = SPLIT ? (int)(blockIdx.x % 2) : 0;       // which eight rows of W
+  const int row0 = halved ? (int)(blockIdx.x / 8 % 2) * (16 * NT) : 0;
   if (group >= groups || row0 >= n) return;                      // the whole workgroup
-  const int steps = k / (64 / ES);                               // of 64 bytes of a row (k is a multiple of 32)
+  const int steps = (int)((unsigned)k / (64 / ES));              // of 64 bytes of a row (k is a multiple of 32)
   const int walk = SPLIT ? steps / 2 : steps;                    // steps that the waves share
-  const int per = (walk + NW - 1) / NW;
+  const int per = (int)((unsigned)(walk + NW - 1) / NW);
   const int s_beg = min(wave * per, walk);
   const int mine = min(per, walk - s_beg);                       // steps of this wave, possibly none
 
-  // ---- what the epilogue needs is asked for first (loads return in order): the rotation's page and
-  // slot, the residual stream's old values
+  // ---- loads return in order: a rotation's page takes two trips, so its position goes first, and so do the sums of squares,
+  // which are added while the weights are on their way (behind the weights: up to 3 % of a step slower)
   const int half = EP == FL_ROPE ? out.hd / 2 : 1;
   constexpr int RC = SPLIT ? 8 : 16;                             // columns of a workgroup's output tile, and threads to a row
   constexpr int RR = 64 * NW / RC;                               // rows that the threads take at a time
   constexpr int RU = ((SPLIT ? 16 : 16 * NT) + RR - 1) / RR;                    // turns
   constexpr int PU = EP == FL_ROPE ? (16 * NT + 2 * RR - 1) / (2 * RR) : 1;
   int ep_pos[PU], ep_span[PU], ep_page[PU];
-  float ep_cos[PU], ep_sin[PU], res_old[RU], res_w = 0.f;
   if (EP == FL_ROPE) {         // thread (pair tid % 8, row tid / 8, and 2 RR on)
-    const int pair = group * 8 + tid % 8;
-    const bool turns = out.cos_t && pair < (out.H + (out.cache ? out.KV : 0)) * half;
 #pragma unroll
     for (int u = 0; u < PU; ++u) {
       const int xr = min(row0 + tid / 8 + 2 * RR * u, n - 1);
-      ep_pos[u] = out.cache ? out.positions[xr] : 0;
-      ep_span[u] = out.cache ? out.span_of_token[xr] : 0;
-      ep_cos[u] = turns ? out.cos_t[(long)xr * half + pair % half] : 1.f;
-      ep_sin[u] = turns ? out.sin_t[(long)xr * half + pair % half] : 0.f;
+      ep_pos[u] = positions ? positions[xr] : 0;
+      ep_span[u] = positions ? span_of_token[xr] : 0;
     }
-  }
-  if (EP == FL_RESID) {        // thread (w row tid % RC, x row tid / RC and RR on)
-    const int col = min(group * 16 + 8 * half_tile + tid % RC, m - 1);
-    res_w = out.norm_w[col];
-#pragma unroll
-    for (int u = 0; u < RU; ++u) res_old[u] = out.resid[(long)min(row0 + tid / RC + RR * u, n - 1) * m + col];
-  }
-  constexpr int SU = RU;
-  floatx4 ssv[SCALED ? SU : 1][FL_SS_LOADS];
-  if (SCALED) {
-    const int stride = (out.ss_parts + 3) / 4 * 4;
-#pragma unroll
-    for (int u = 0; u < SU; ++u)
-#pragma unroll
-      for (int i = 0; i < FL_SS_LOADS; ++i) {
-        const int at = 4 * (tid % 16 + 16 * i);
-        ssv[u][i] = *reinterpret_cast<const floatx4*>(out.ss_in + (long)min(row0 + tid / 16 + RR * u, n - 1) * stride +
-                                                      (at < stride ? at : 0));
-      }
   }
 
   // ---- operands: offsets in bytes from descriptors that all lanes share, so that a step costs a scalar
-  // addition.  A step that does not exist reads the wave's last (or K's last) again and is not multiplied; a
+  // addition; the weights of a buffer before its rows, which come from nearer.  A step that does not exist reads the wave's last (or K's last) again and is not multiplied; a
   // tile or a row of X beyond the last one reads the last, and its sums are not stored.
   const int tile0 = group * TW;
   // (float32 also takes the weights as they are, row by row: the sums are the same bits, so that a card with no room for
   // the tiled copy gives the same results)
-  const bool tiled = ES == 2 || out.tiled;
+  const bool tiled = ES == 2 || (how & LR_W_TILED), x_tiled = how & LR_X_TILED;
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<char*>(reinterpret_cast<const char*>(W)) + (tiled ? (long)tile0 * steps * 1024 : 0), 0,
       tiled ? min(TW, tiles - tile0) * steps * 1024 : m * k * ES, 0x00020000);
   const int w_step = tiled ? 1024 : 64;
-  const int row_tiles = (n + 15) / 16, side = min(n, 16), x_step = out.x_tiled ? 64 * side : 64;
-  const __amdgpu_buffer_rsrc_t xr_ = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<T*>(X), 0, out.x_tiled ? row_tiles * steps * x_step : ES * ((n - 1) * x_stride + k), 0x00020000);
   const int later = SPLIT && c >= 8 ? walk : 0;                  // steps on, for the lanes of the second half of K
   const int wc = SPLIT ? 8 * half_tile + c % 8 : c;              // this lane's row of a tile
   int wo[TW], xo[NT];
@@ -147,29 +132,38 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const T* __restric
     wo[j] = tile * steps * 1024 + later * 1024 + (16 * g + wc) * 16;
     if (!tiled) wo[j] = (int)max(fl_row<EP>(tile0 + tile, wc, m, out), 0L) * k * ES + later * 64 + 16 * g;
   }
+  const int s_last = min(s_beg + max(mine, 1), walk) - 1;
+  auto fill_w = [&](uintx4 (&wb)[A][TW], int s0) {
+#pragma unroll
+    for (int i = 0; i < A; ++i)
+#pragma unroll
+      for (int j = 0; j < TW; ++j)
+        wb[i][j] = __builtin_amdgcn_raw_buffer_load_b128(wr, wo[j], min(s_beg + s0 + i, s_last) * w_step, 0);
+  };
+  const int row_tiles = (n + 15) / 16, side = min(n, 16), x_step = x_tiled ? 64 * side : 64;
+  const __amdgpu_buffer_rsrc_t xr_ = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<T*>(X), 0, x_tiled ? row_tiles * steps * x_step : ES * ((n - 1) * x_stride + k), 0x00020000);
 #pragma unroll
   for (int t = 0; t < NT; ++t)
-    xo[t] = out.x_tiled ? min(row0 / 16 + t, row_tiles - 1) * steps * x_step + (g * side + min(c, side - 1)) * 16
-                        : ES * min(row0 + t * 16 + c, n - 1) * x_stride + 16 * g;
+    xo[t] = x_tiled ? min(row0 / 16 + t, row_tiles - 1) * steps * x_step + (g * side + min(c, side - 1)) * 16
+                    : ES * min(row0 + t * 16 + c, n - 1) * x_stride + 16 * g;
   if (SPLIT) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const int row = min(NT == 1 ? c % 8 : c, n - 1);
-      xo[t] = (NT == 1 ? later : t * walk) * x_step + (out.x_tiled ? (g * side + row) * 16 : ES * row * x_stride + 16 * g);
+      xo[t] = (NT == 1 ? later : t * walk) * x_step + (x_tiled ? (g * side + row) * 16 : ES * row * x_stride + 16 * g);
     }
   }
-  const int s_last = min(s_beg + max(mine, 1), walk) - 1;
-  auto fill = [&](uintx4 (&wb)[A][TW], uintx4 (&xb)[A][NT], int s0) {
+  auto fill_x = [&](uintx4 (&xb)[A][NT], int s0) {
 #pragma unroll
-    for (int i = 0; i < A; ++i) {
-      const int s = min(s_beg + s0 + i, s_last);
-#pragma unroll
-      for (int j = 0; j < TW; ++j)
-        wb[i][j] = __builtin_amdgcn_raw_buffer_load_b128(wr, wo[j], s * w_step, 0);
+    for (int i = 0; i < A; ++i)
 #pragma unroll
       for (int t = 0; t < NT; ++t)
-        xb[i][t] = __builtin_amdgcn_raw_buffer_load_b128(xr_, xo[t], s * x_step, 0);
-    }
+        xb[i][t] = __builtin_amdgcn_raw_buffer_load_b128(xr_, xo[t], min(s_beg + s0 + i, s_last) * x_step, 0);
+  };
+  auto fill = [&](uintx4 (&wb)[A][TW], uintx4 (&xb)[A][NT], int s0) {
+    fill_w(wb, s0);
+    fill_x(xb, s0);
     // Loads and products stay on their sides of this line: left to itself the compiler moves half of the
     // loads to where their values are used.
     asm volatile("" ::: "memory");
@@ -190,11 +184,33 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const T* __restric
   };
   // (whole words: as bfloat16 vectors the compiler puts the halves together again behind each load, and waits for it)
   uintx4 wa[A][TW], xa[A][NT], wb[A][TW], xb[A][NT];
-  fill(wa, xa, 0);
-  if (EP == FL_ROPE)
+  constexpr int SU = RU;
+  floatx4 ssv[SCALED ? SU : 1][FL_SS_LOADS];
+  if (SCALED) {
+    const int stride = (ss_parts + 3) / 4 * 4;
 #pragma unroll
-    for (int u = 0; u < PU; ++u)
+    for (int u = 0; u < SU; ++u)
+#pragma unroll
+      for (int i = 0; i < FL_SS_LOADS; ++i) {
+        const int at = 4 * (tid % 16 + 16 * i);
+        ssv[u][i] = *reinterpret_cast<const floatx4*>(ss_in + (long)min(row0 + tid / 16 + RR * u, n - 1) * stride +
+                                                      (at < stride ? at : 0));
+      }
+  }
+  fill(wa, xa, 0);
+  // ---- what the epilogue needs: behind the first operands
+  float ep_cos[PU], ep_sin[PU], res_old[RU], res_w = 0.f;
+  if (EP == FL_ROPE) {
+    const int pair = group * 8 + tid % 8;
+    const bool turns = out.cos_t && pair < (out.H + (out.cache ? out.KV : 0)) * half;
+#pragma unroll
+    for (int u = 0; u < PU; ++u) {
+      const int xr = min(row0 + tid / 8 + 2 * RR * u, n - 1);
+      ep_cos[u] = turns ? out.cos_t[(long)xr * half + pair % half] : 1.f;
+      ep_sin[u] = turns ? out.sin_t[(long)xr * half + pair % half] : 0.f;
       ep_page[u] = out.cache ? out.block_table[(long)ep_span[u] * out.max_pages + ep_pos[u] / out.page_size] : 0;
+    }
+  }
   if (SCALED) {      // the rows' scales, before the second buffer needs the registers: sums in a fixed order, then across sixteen lanes
 #pragma unroll
     for (int u = 0; u < SU; ++u) {
@@ -202,29 +218,44 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const T* __restric
 #pragma unroll
       for (int i = 0; i < FL_SS_LOADS; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v += 4 * (tid % 16 + 16 * i) + e < out.ss_parts ? ssv[u][i][e] : 0.f;
+        for (int e = 0; e < 4; ++e) v += 4 * (tid % 16 + 16 * i) + e < ss_parts ? ssv[u][i][e] : 0.f;
       v = parts_sum<16>(v);
       if (tid % 16 == 0 && tid / 16 + RR * u < 16 * NT) row_scale[tid / 16 + RR * u] = rsqrtf(v / (float)k + out.eps);
     }
   }
-  fill(wb, xb, A);
-  int s = 0;
-  for (; mine - s > 2 * A; s += 2 * A) {
+  auto ask_stream = [&] {
+    if (EP != FL_RESID) return;  // thread (w row tid % RC, x row tid / RC and RR on)
+    const int col = min(group * 16 + 8 * half_tile + tid % RC, m - 1);
+    res_w = out.norm_w[col];
 #pragma unroll
-    for (int i = 0; i < A; ++i) step(wa[i], xa[i], i);
-    __builtin_amdgcn_sched_barrier(0);
-    fill(wa, xa, s + 2 * A);
+    for (int u = 0; u < RU; ++u) res_old[u] = out.resid[(long)min(row0 + tid / RC + RR * u, n - 1) * m + col];
+  };
+  if (SPLIT && ES == 2 && per <= A) {      // (K of up to 2,048: one buffer is all a wave has)
+    ask_stream();
 #pragma unroll
-    for (int i = 0; i < A; ++i) step(wb[i], xb[i], i);
-    __builtin_amdgcn_sched_barrier(0);
-    fill(wb, xb, s + 3 * A);
+    for (int i = 0; i < A; ++i)
+      if (i < mine) step(wa[i], xa[i], i);
+  } else {
+    fill(wb, xb, A);
+    ask_stream();
+    int s = 0;
+    for (; mine - s > 2 * A; s += 2 * A) {
+#pragma unroll
+      for (int i = 0; i < A; ++i) step(wa[i], xa[i], i);
+      __builtin_amdgcn_sched_barrier(0);
+      fill(wa, xa, s + 2 * A);
+#pragma unroll
+      for (int i = 0; i < A; ++i) step(wb[i], xb[i], i);
+      __builtin_amdgcn_sched_barrier(0);
+      fill(wb, xb, s + 3 * A);
+    }
+#pragma unroll
+    for (int i = 0; i < A; ++i)
+      if (s + i < mine) step(wa[i], xa[i], i);
+#pragma unroll
+    for (int i = 0; i < A; ++i)
+      if (s + A + i < mine) step(wb[i], xb[i], i);
   }
-#pragma unroll
-  for (int i = 0; i < A; ++i)
-    if (s + i < mine) step(wa[i], xa[i], i);
-#pragma unroll
-  for (int i = 0; i < A; ++i)
-    if (s + A + i < mine) step(wb[i], xb[i], i);
 
   // ---- the waves meet: lane (g, c) holds w rows 4 g ... 4 g + 3 of x row c
 #pragma unroll
@@ -322,19 +353,22 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const T* __restric
 
 static size_t lr_lds_bytes(int nt, int tw, int nw) { return (size_t)(nw * tw * nt * LR_TILE + LR_ROWS) * sizeof(float); }
 
-template <typename T, int NT, int TW, int EP, bool SCALED, int NW, bool SPLIT = false>
+template <typename T, int NT, int TW, int EP, bool SCALED, int NW, bool SPLIT = false, int A = lr_ahead(NT, TW)>
 static int lr_launch_waves(const void* x, const FlOut& out, const void* w, int n, int m, int k, int tiles, int halves,
                      int x_stride, hipStream_t stream) {
   const size_t lds = lr_lds_bytes(NT, TW, NW);
   if (lds > 64 * 1024) {
-    static const hipError_t e = hipFuncSetAttribute((const void*)linear_rows_kernel<T, NT, TW, EP, SCALED, NW, SPLIT>,
+    static const hipError_t e = hipFuncSetAttribute((const void*)linear_rows_kernel<T, NT, TW, EP, SCALED, NW, SPLIT, A>,
                                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     if (e != hipSuccess) KLLM_FAIL((int)e, "linear_rows: cannot raise the LDS limit: %s", hipGetErrorString(e));
   }
   const int groups = ceil_div(tiles, TW);
   const int blocks = SPLIT ? 2 * groups : halves == 1 ? groups : ceil_div(groups, 8) * 16;
-  hipLaunchKernelGGL((linear_rows_kernel<T, NT, TW, EP, SCALED, NW, SPLIT>), dim3(blocks), dim3(64 * NW), lds, stream,
-                     (const T*)x, out, (const T*)w, n, m, k, tiles, halves, x_stride);
+  hipLaunchKernelGGL((linear_rows_kernel<T, NT, TW, EP, SCALED, NW, SPLIT, A>), dim3(blocks), dim3(64 * NW), lds, stream,
+                     (const T*)w, (const T*)x, m, k, x_stride,
+                     (halves == 2 ? LR_HALVES : 0u) | (out.x_tiled ? LR_X_TILED : 0u) | (out.tiled ? LR_W_TILED : 0u) |
+                         (unsigned)n << 8 | (unsigned)out.ss_parts << 16,
+                     out.cache ? out.positions : nullptr, out.cache ? out.span_of_token : nullptr, out.ss_in, out);
   return 0;
 }
 
@@ -380,6 +414,15 @@ static int lr_tiles(int kind, int m) { return kind == FL_RESID || kind == FL_PAR
 
 // Whether a product that splits takes eight rows of W a workgroup (SPLIT): up to 16 rows of X and no more tiles than half the CUs.
 static bool lr_split(int n, int m, int k) { return n <= 16 && k % 64 == 0 && 2 * lr_tiles(FL_RESID, m) <= device_cus(); }
+
+// Whether a SPLIT product's waves fill their buffers three steps at a time instead of four: a wave asks for whole turns of both
+// buffers, and what is beyond its last step is read again for nothing.  2,048 x 5,632 (eleven steps a wave, sixteen asked
+// for in fours, twelve in threes), 1 / 8 rows alone in a replayed graph: 6.7 / 8.2 us in fours, 6.5 / 7.5 in threes, 6.4 / 7.7 in sixes;
+// 2,048 x 2,048 (four steps: one buffer) 3.6 / 4.2, 3.8 / 4.7, 3.8 / 4.5.
+static bool lr_threes(int k) {
+  const int per = ceil_div(k / 64, 8);
+  return per > 4 && ceil_div(per, 6) * 6 < ceil_div(per, 8) * 8;
+}
 
 // Tiles of W a workgroup, workgroups that share the rows out, tiles of rows a workgroup.
 struct LrPlan {
@@ -498,8 +541,9 @@ extern "C" int kllm_linear_rows(const void* x, int x_stride, const KllmLinearOut
   const LrPlan plan = lr_plan(ep, n, m, k, f32, out.x_tiled);
   const int tw = plan.tw, halves = plan.halves, nt = plan.nt;
 #define KLLM_LRS(NT, EP)                                                                                        \
-  (f32 ? lr_launch_waves<float, NT, 1, EP, false, 8, true>(x, out, w, n, m, k, tiles, 1, x_stride, stream)      \
-       : lr_launch_waves<bf16_t, NT, 1, EP, false, 8, true>(x, out, w, n, m, k, tiles, 1, x_stride, stream))
+  (f32           ? lr_launch_waves<float, NT, 1, EP, false, 8, true>(x, out, w, n, m, k, tiles, 1, x_stride, stream)       \
+   : lr_threes(k) ? lr_launch_waves<bf16_t, NT, 1, EP, false, 8, true, 3>(x, out, w, n, m, k, tiles, 1, x_stride, stream)   \
+                 : lr_launch_waves<bf16_t, NT, 1, EP, false, 8, true, 4>(x, out, w, n, m, k, tiles, 1, x_stride, stream))
   const bool split = (ep == FL_RESID || ep == FL_PARTS) && lr_split(n, m, k);
   const int rc = split     ? (ep == FL_RESID ? (n <= 8 ? KLLM_LRS(1, FL_RESID) : KLLM_LRS(2, FL_RESID))
                                              : (n <= 8 ? KLLM_LRS(1, FL_PARTS) : KLLM_LRS(2, FL_PARTS)))
