@@ -1270,6 +1270,21 @@ def test_attention_generic(H, KV, hd, ps, dtype, window):
         assert err < (2e-5 if dtype == torch.float32 else 2e-2), (kernel, float(err))
 
 
+@pytest.mark.parametrize("H,KV,hd,ps", [(2, 1, 64, 16), (4, 1, 48, 48), (1, 1, 128, 80), (18, 1, 16, 112), (2, 2, 112, 32)])
+@pytest.mark.parametrize("window", [0, 333])
+def test_attention_decode_places(H, KV, hd, ps, window):
+    """Decode attention's tiles of 32 keys in halves of a page each, in pages of odd multiples of sixteen; waves with none, one, two and
+    three tiles, and with more than the 32 tiles whose pages are looked up at once (a wave of one workgroup of eight
+    takes 1,056 to 1,152 of 8,450 and 9,200 keys); a slice of the keys cut in 1, 3 and 16.  Slots that hold no key are NaN.  A score
+    and a weight are 32-bit sums: what differs from the reference is the rounding of the probabilities and of the output, 2^-8 each."""
+    for spans, slices in (([(8449, 1), (9199, 1)], (1, 3)), ([(0, 1), (30, 1), (31, 1), (47, 1), (95, 1), (511, 1), (1055, 1), (2047, 1)], (1, 3, 16))):
+        c = attention_case(H, KV, hd, ps, torch.bfloat16, window, spans, seed=3)
+        for ns in slices:
+            out = run_attention("decode", c["q"], c["cache"], c["pos"], c["sot"], c["bt"], ps, H, KV, hd, window, c["scale"], nslices=ns)
+            err = (out.cpu().double() - c["want"]).abs().max()
+            assert torch.isfinite(out).all() and err < 2 ** -7 * c["want"].abs().max(), (ns, float(err))
+
+
 @pytest.mark.parametrize("H,KV,hd,ps", [(4, 2, 32, 16), (3, 1, 64, 16), (8, 2, 64, 32), (5, 5, 96, 16),
                                         (2, 1, 128, 16), (2, 2, 192, 16), (2, 1, 256, 16), (32, 4, 64, 16),
                                         (4, 2, 64, 48), (2, 1, 128, 48), (2, 2, 192, 80), (12, 4, 128, 16),
