@@ -59,37 +59,59 @@ __device__ __forceinline__ void attn_merge_one(T* __restrict__ out, const float*
       out[rows_at(side, t, h * hd + lane + 64 * v, H * hd)] = from_f32<T>(o[v] / denom * out_gate(gate, t, h, lane + 64 * v));
 }
 
+// The greatest of the first R lanes' values (-infinity in the others), the same in every lane.
+template <int CTRL>
+__device__ __forceinline__ float dpp_max(float v) {
+  return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true)));
+}
+template <int R>
+__device__ __forceinline__ float first_lanes_max(float v) {
+  v = dpp_max<0xB1>(v);     // quad_perm [1,0,3,2]
+  v = dpp_max<0x4E>(v);     // quad_perm [2,3,0,1]
+  v = dpp_max<0x141>(v);    // row_half_mirror
+  v = dpp_max<0x140>(v);    // row_mirror
+  if (R > 16) v = fmaxf(v, __shfl_xor(v, 16, kWave));
+  if (R > 32) v = fmaxf(v, __shfl_xor(v, 32, kWave));
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+
 // The same for up to 64 slices and heads of up to 128 in one trip to memory instead of one per
-// sixteen slices, with fewer loads a lane: every output element of every slice is asked for at once (64 DV
-// loads a lane), lane s fetches slice s's maximum and sum and works out its weight, and the
-// weights go from lane to lane while the sums are added in the order of the slices.
+// sixteen slices, with fewer loads a lane: lane s fetches slice s's maximum and sum and works out its weight, every output element
+// of every slice is asked for behind them (R DV loads a lane; beyond the last slice the descriptor ends and a load brings
+// zeros from nowhere), and the weights go from lane to lane while the sums are added in the order of the slices.  t and h are a wave's.
 template <typename T, int DV, int R>   // R: 16, 32 or 64, at least the number of slices
 __device__ __forceinline__ void attn_merge_wide(T* __restrict__ out, const float* __restrict__ part, int t, int h, int H,
                                                 int hd, int nslices, int lane, const OutGate& gate) {
-  const int stride = hd + 2, side = gate.side;
-  asm volatile("" ::"s"(side));        // (as above)
-  const float* p = part + ((long)t * H + h) * nslices * stride;
+  t = __builtin_amdgcn_readfirstlane(t);
+  h = __builtin_amdgcn_readfirstlane(h);
+  const int row = (hd + 2) * (int)sizeof(float);
+  const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<char*>(reinterpret_cast<const char*>(part)) + ((long)t * H + h) * nslices * row, 0, nslices * row, 0x00020000);
+  auto load = [&](int at, int slice_at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rows, at, slice_at, 0)); };
+  const float ms0 = load(lane * row + 4 * hd, 0), ls = load(lane * row + 4 * hd + 4, 0);
   float os[DV][R];
 #pragma unroll
-  for (int j = 0; j < R; ++j) {
-    const float* q = p + (long)(j < nslices ? j : 0) * stride;      // beyond the last slice: a valid address
+  for (int j = 0; j < R; ++j)
 #pragma unroll
-    for (int v = 0; v < DV; ++v) os[v][j] = q[lane + 64 * v < hd ? lane + 64 * v : 0];
-  }
-  const bool mine = lane < nslices;
-  const float* q = p + (long)(mine ? lane : 0) * stride;
-  const float ms = mine ? q[hd] : -INFINITY, ls = mine ? q[hd + 1] : 0.f;
-  float M = ms;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
+    for (int v = 0; v < DV; ++v) os[v][j] = load(4 * (lane + 64 * v < hd ? lane + 64 * v : 0), j * row);
+  __builtin_amdgcn_sched_barrier(0);
+  const int side = gate.side;
+  asm volatile("" ::"s"(side), "s"(gate.sums), "s"(gate.width), "s"(H));     // (now: in front of the stores it was a trip to memory of its own)
+  const float ms = lane < nslices ? ms0 : -INFINITY;
+  const float M = first_lanes_max<R>(ms);
   // (M is finite: some slice holds the token's own key)
   const float w = (ms == -INFINITY) ? 0.f : expf(ms - M);
+#pragma unroll
+  for (int j = 0; j < R; ++j)
+#pragma unroll
+    for (int v = 0; v < DV; ++v) asm volatile("" : "+v"(os[v][j]));     // (needed here: left alone they are asked for in the branch around the stores)
   float denom = 0.f, o[DV];
 #pragma unroll
   for (int v = 0; v < DV; ++v) o[v] = 0.f;
+  auto lane_of = [](float v, int j) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), j)); };
 #pragma unroll
   for (int j = 0; j < R; ++j) {
-    const float wj = __shfl(w, j, 64), lj = __shfl(ls, j, 64);     // 0 beyond the last slice
+    const float wj = lane_of(w, j), lj = lane_of(ls, j);     // 0 beyond the last slice
     denom += wj * lj;
 #pragma unroll
     for (int v = 0; v < DV; ++v) o[v] += wj * os[v][j];
@@ -101,10 +123,11 @@ __device__ __forceinline__ void attn_merge_wide(T* __restrict__ out, const float
 }
 
 template <typename T, int DV, int R>
-__global__ __launch_bounds__(64) void attn_merge_wide_kernel(T* __restrict__ out, const float* __restrict__ part, int H,
-                                                             int hd, int nslices, const int* __restrict__ token_list,
-                                                             const OutGate gate) {
-  const int t = token_list ? token_list[blockIdx.x] : blockIdx.x;
+__global__ __launch_bounds__(64) void attn_merge_wide_kernel(const float* __restrict__ part, const int* __restrict__ token_list,
+                                                             T* __restrict__ out, int H, int hd, int nslices, const OutGate gate) {
+  int t = blockIdx.x;
+  asm volatile("" : "+v"(t));          // (a vector load: a scalar one would wait for the other arguments with it)
+  if (token_list) t = token_list[t];
   attn_merge_wide<T, DV, R>(out, part, t, blockIdx.y, H, hd, nslices, threadIdx.x, gate);
 }
 
@@ -127,7 +150,7 @@ inline void launch_attn_merge(T* out, const float* part, int count, int H, int h
     // numbers instead of slices x (2 + DV); 64 slices of a head of 64: the merge 10 us -> 6,
     // 16 slices: a microsecond less)
 #define KLLM_MERGE_WIDE(DV, R) \
-    hipLaunchKernelGGL((attn_merge_wide_kernel<T, DV, R>), grid, block, 0, stream, out, part, H, hd, nslices, token_list, gate)
+    hipLaunchKernelGGL((attn_merge_wide_kernel<T, DV, R>), grid, block, 0, stream, part, token_list, out, H, hd, nslices, gate)
     if (hd <= 64) {
       if (nslices <= 16) KLLM_MERGE_WIDE(1, 16); else if (nslices <= 32) KLLM_MERGE_WIDE(1, 32); else KLLM_MERGE_WIDE(1, 64);
     } else {
