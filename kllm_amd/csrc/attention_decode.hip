@@ -49,32 +49,6 @@ namespace kllm {
 // 4,096 keys 220 / 195; 32 tokens x 32 KV heads of 128 at 2,048 keys 221 / 208.
 constexpr int kDecodeWavesShared = 4;
 constexpr int decode_waves_whole(int hdt) { return hdt <= 8 ? 8 : 4; }
-// Over lanes c, c + 16, c + 32, c + 48, without a trip through LDS: a swap of rows of sixteen (of halves) of a value with itself
-// leaves every lane its own and its partner's.
-__device__ __forceinline__ float group4_max(float v) {
-  unsigned u = __builtin_bit_cast(unsigned, v);
-  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  u = __builtin_bit_cast(unsigned, fmaxf(__builtin_bit_cast(float, (unsigned)a[0]), __builtin_bit_cast(float, (unsigned)a[1])));
-  const auto b = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return fmaxf(__builtin_bit_cast(float, (unsigned)b[0]), __builtin_bit_cast(float, (unsigned)b[1]));
-}
-__device__ __forceinline__ float group4_sum(float v) {
-  unsigned u = __builtin_bit_cast(unsigned, v);
-  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  u = __builtin_bit_cast(unsigned, __builtin_bit_cast(float, (unsigned)a[0]) + __builtin_bit_cast(float, (unsigned)a[1]));
-  const auto b = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return __builtin_bit_cast(float, (unsigned)b[0]) + __builtin_bit_cast(float, (unsigned)b[1]);
-}
-// x / d and what is left, with magic = 2^32 / d rounded down (2^32 - 1 for d = 1): the product is the quotient or one less.
-__device__ __forceinline__ unsigned divided(unsigned x, unsigned d, unsigned magic, unsigned& left) {
-  unsigned r = __umulhi(x, magic);
-  left = x - r * d;
-  const bool more = left >= d;
-  left = more ? left - d : left;
-  return more ? r + 1 : r;
-}
-constexpr float kLog2E = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
-
 // KEPT: kept first positions behind the window (an instance of its own: the others carry none of it)
 // TILED: the output's rows in the next product's order (gate.side; one instance for both cost the plain one 2 us of 49, in scalar registers)
 // G: query heads of a KV head; page16: page size / 16; page_magic and slice_magic: see divided(), of page16 and of the slices (waves).

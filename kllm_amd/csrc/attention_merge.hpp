@@ -59,22 +59,6 @@ __device__ __forceinline__ void attn_merge_one(T* __restrict__ out, const float*
       out[rows_at(side, t, h * hd + lane + 64 * v, H * hd)] = from_f32<T>(o[v] / denom * out_gate(gate, t, h, lane + 64 * v));
 }
 
-// The greatest of the first R lanes' values (-infinity in the others), the same in every lane.
-template <int CTRL>
-__device__ __forceinline__ float dpp_max(float v) {
-  return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true)));
-}
-template <int R>
-__device__ __forceinline__ float first_lanes_max(float v) {
-  v = dpp_max<0xB1>(v);     // quad_perm [1,0,3,2]
-  v = dpp_max<0x4E>(v);     // quad_perm [2,3,0,1]
-  v = dpp_max<0x141>(v);    // row_half_mirror
-  v = dpp_max<0x140>(v);    // row_mirror
-  if (R > 16) v = fmaxf(v, __shfl_xor(v, 16, kWave));
-  if (R > 32) v = fmaxf(v, __shfl_xor(v, 32, kWave));
-  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
-}
-
 // The same for up to 64 slices and heads of up to 128 in one trip to memory instead of one per
 // sixteen slices, with fewer loads a lane: lane s fetches slice s's maximum and sum and works out its weight, every output element
 // of every slice is asked for behind them (R DV loads a lane; beyond the last slice the descriptor ends and a load brings

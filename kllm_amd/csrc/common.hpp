@@ -229,4 +229,46 @@ __device__ __forceinline__ float parts_sum(float v) {
   return v;
 }
 
+// Over lanes c, c + 16, c + 32, c + 48, without a trip through LDS: a swap of rows of sixteen (of halves) of a value with itself
+// leaves every lane its own and its partner's.
+__device__ __forceinline__ float group4_max(float v) {
+  unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  u = __builtin_bit_cast(unsigned, fmaxf(__builtin_bit_cast(float, (unsigned)a[0]), __builtin_bit_cast(float, (unsigned)a[1])));
+  const auto b = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return fmaxf(__builtin_bit_cast(float, (unsigned)b[0]), __builtin_bit_cast(float, (unsigned)b[1]));
+}
+__device__ __forceinline__ float group4_sum(float v) {
+  unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  u = __builtin_bit_cast(unsigned, __builtin_bit_cast(float, (unsigned)a[0]) + __builtin_bit_cast(float, (unsigned)a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __builtin_bit_cast(float, (unsigned)b[0]) + __builtin_bit_cast(float, (unsigned)b[1]);
+}
+// x / d and what is left, with magic = 2^32 / d rounded down (2^32 - 1 for d = 1): the product is the quotient or one less.
+__device__ __forceinline__ unsigned divided(unsigned x, unsigned d, unsigned magic, unsigned& left) {
+  unsigned r = __umulhi(x, magic);
+  left = x - r * d;
+  const bool more = left >= d;
+  left = more ? left - d : left;
+  return more ? r + 1 : r;
+}
+constexpr float kLog2E = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
+
+// The greatest of the first R lanes' values (-infinity in the others), the same in every lane.
+template <int CTRL>
+__device__ __forceinline__ float dpp_max(float v) {
+  return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true)));
+}
+template <int R>
+__device__ __forceinline__ float first_lanes_max(float v) {
+  v = dpp_max<0xB1>(v);     // quad_perm [1,0,3,2]
+  v = dpp_max<0x4E>(v);     // quad_perm [2,3,0,1]
+  v = dpp_max<0x141>(v);    // row_half_mirror
+  v = dpp_max<0x140>(v);    // row_mirror
+  if (R > 16) v = fmaxf(v, __shfl_xor(v, 16, kWave));
+  if (R > 32) v = fmaxf(v, __shfl_xor(v, 32, kWave));
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+
 }  // namespace kllm

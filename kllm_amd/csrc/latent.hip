@@ -224,227 +224,280 @@ __global__ __launch_bounds__(kLatThreads) void attn_latent_kernel(
   }
 }
 
-// attn_latent on the matrix cores (bfloat16).  A workgroup takes one token and up to 16 heads;
-// its four waves take the token's keys in tiles of 32, round robin, and meet in LDS.  All heads
-// read the same keys, so the 16 heads are the columns of one product:
+// attn_latent on the matrix cores (bfloat16).  A workgroup takes one token, up to 16 heads and, round by round, 128 of the token's
+// keys.  All heads read the same keys, so the 16 heads are the columns of one product:
 // MFMA 16x16x32 (lane l: g = l/16, c = l%16): A[c][8g..8g+7], B[8g..8g+7][c], D[4g+i][c].
-// Scores: A = 16 keys x 32 elements of their rows (one row per lane, straight from the page),
-// B = the folded queries of the 16 heads, D[key 4g+i][head c].  Weighted sum: the 32 slots that
-// are summed over are the keys (4g+j) of the tile's first half for j < 4 and of its second half for
-// j >= 4, which is how a lane holds its probabilities; A = latents [element c][those keys], two
-// 8-byte reads from the transposed copy.  NR: 16-element pieces of the latent a lane accumulates.
+// Scores: each of the four waves takes a tile of 32 keys, A = 16 of them x 32 elements of their rows (one row per lane, straight from the page),
+// B = the folded queries of the 16 heads.  Which key stands in which row is free: key 8 (c / 4) + 4 u + c % 4 in row c of the u-th of two
+// instructions, so that a lane's probabilities are those of eight neighbouring keys.  They meet in LDS (the heads' maxima first), and each
+// wave takes a quarter of the weighted sum's elements for all four tiles: A = latents [element c][8 keys], 16 bytes from the transposed copy.
+//
+// What bounds a decode step's launch are its trips to memory (position and span; pages; rows and latents, all of a round asked for
+// at once) and its code, which is read cold.  A wave that keeps all elements for its own keys needs four times the accumulators and
+// a merge of them in LDS that leaves a CU one workgroup: 28 KB of code, 25 us for 8 tokens, 32 heads and 1,400 keys with rank 512 in 32 slices, most of them
+// empty but writing their zeros; so 14, of which the rows and latents, 24 MB, take five at the rate of a large read.
+// NR: 16-element pieces of the latent, KS: steps of 32 over a row that a lane asks for at once (0: four at a time, for rows longer
+// than the built sizes).  The queries lie in LDS: in registers, with the round's keys and latents there, they were spilt.
 constexpr int kLatWaves = 4;
 
-// KS: steps of 32 over a row whose pieces of the query a lane keeps in registers (0: it asks for
-// them at every tile, for rows longer than the built sizes).
 template <int NR, int KS>
 __global__ __launch_bounds__(64 * kLatWaves) void attn_latent_mfma_kernel(
-    const bf16_t* __restrict__ q, bf16_t* __restrict__ out, const bf16_t* __restrict__ cache,
-    const int* __restrict__ positions, const int* __restrict__ span_of_token, const int* __restrict__ block_table,
-    int max_pages, int page_size, unsigned page_magic, int H, int row, int rank, float scale, int window,
-    float* __restrict__ part) {
-  extern __shared__ float lat_red[];            // [kLatWaves][NR * 4 + 2][64]
+    const bf16_t* __restrict__ cache, const int* __restrict__ positions, const int* __restrict__ span_of_token,
+    const int* __restrict__ block_table, const bf16_t* __restrict__ q, int max_pages, int page16, int H, int row, int rank, unsigned page_magic,
+    float scale, int window, int nslices, bf16_t* __restrict__ out, float* __restrict__ part) {
+  constexpr int PER = NR / kLatWaves;           // pieces of a wave: wave, wave + 4, ...
+  constexpr int PLD = 32 * kLatWaves + 8;       // probabilities of a head's 128 keys in LDS, and a shift of banks
+  __shared__ __attribute__((aligned(16))) bf16_t probs[2][16 * PLD];
+  constexpr int QLD = (KS > 0 ? 32 * KS : kLatMaxRow) + 8;
+  __shared__ __attribute__((aligned(16))) bf16_t queries[16 * QLD];
+  __shared__ float meet[2][kLatWaves][16];
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int g = lane / 16, c = lane % 16;
-  const int t = blockIdx.x, h0 = blockIdx.y * 16;
+  const int t = blockIdx.x, h0 = blockIdx.y * 16, slice = blockIdx.z;
+  int at = t;
+  asm volatile("" : "+v"(at));                  // (vector loads, as in decode attention: they go out together)
+  const int pos_v = positions[at], span_v = span_of_token[at];
+  asm volatile("" ::"s"(rank), "s"(page_magic), "s"(scale), "s"(window), "s"(nslices), "s"(out), "s"(part));
+  const int page_size = 16 * page16;
   const int head = min(h0 + c, H - 1);
   const bool head_ok = h0 + c < H;
-  const int len = positions[t] + 1;
+  int len = __builtin_amdgcn_readfirstlane(pos_v) + 1, span = __builtin_amdgcn_readfirstlane(span_v);
+  asm volatile("" : "+s"(len), "+s"(span));
   const int lo = first_key(len - 1, window, 0);        // the first key that is read
-  const int* table = block_table + (long)span_of_token[t] * max_pages;
-  const long page_elems = (long)page_size * (row + rank);
-  const int ksteps = (row + 31) / 32, nr = rank / 16;
-  const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-  const bf16_t* qrow = q + ((long)t * H + head) * row;
-  bf16x8 qreg[KS > 0 ? KS : 1];
+  const int tile0 = lo / 32, rounds = (len - 32 * tile0 + 127) / 128;
+  float* prow = part + (((long)t * H + head) * nslices + slice) * (rank + 2);     // (of several slices) rows of rank + 2 floats
+  if (slice >= rounds) {                               // no keys: a maximum of -inf, and the merge reads no more of it
+    if (wave == 0 && g == 0 && head_ok) *reinterpret_cast<floatx2*>(prow + rank) = floatx2{-INFINITY, 0.f};
+    return;
+  }
+  const int* table = block_table + (long)span * max_pages;
+  const long page_bytes = 2L * page_size * (row + rank);
+  const float scale2 = scale * kLog2E;
+  auto bits = [](int from, int to) -> unsigned {       // from ... to - 1 of 32
+    return to <= 0 || from >= 32 ? 0u : (~0u >> (32 - min(to, 32))) & (~0u << max(from, 0));
+  };
+  // Where the 64 halves of eight rounds from r0 on lie, a half (16 keys in one page) to a lane: their pages are one load.
+  // A half that is not read (its page may be gone) reads page 0.
+  struct Places {
+    unsigned mask;                              // of the half's tile: which keys are read
+    int slot;
+    long base;                                  // bytes from the cache's first to the half's page
+  };
+  auto lookup = [&](int r0) -> Places {
+    Places P;
+    const int kb = 32 * (tile0 + 4 * (r0 + lane / 8 * nslices) + lane % 8 / 2);
+    P.mask = bits(lo - kb, len - kb);
+    const bool live = (P.mask >> (16 * (lane % 2))) & 0xFFFFu;
+    unsigned left;
+    const int index = (int)divided(live ? (unsigned)kb / 16 + lane % 2 : 0u, (unsigned)page16, page_magic, left);
+    P.slot = live ? (int)left * 16 : -1;
+    P.base = table[index];
+    return P;
+  };
+  auto placed = [&](Places P) -> Places {              // once the pages are there
+    P.base = (long)(P.slot >= 0 ? (int)P.base : 0) * page_bytes;
+    P.slot = max(P.slot, 0);
+    return P;
+  };
+  auto half_at = [&](const Places& P, int i) {
+    const unsigned low = __builtin_amdgcn_readlane((int)P.base, i);
+    return reinterpret_cast<const char*>(cache) +
+           (long)((unsigned long)(unsigned)__builtin_amdgcn_readlane((int)(P.base >> 32), i) << 32 | low);
+  };
+  auto slot_at = [&](const Places& P, int i) { return __builtin_amdgcn_readlane(P.slot, i); };
+  auto mask_at = [&](const Places& P, int i) -> unsigned { return __builtin_amdgcn_readlane((int)P.mask, i); };
+  // A tile without keys reads the round's first one again: its scores are masked and its sums left out.
+  auto key_row = [&](const Places& P, int i) {         // this lane's row of the wave's tile of the i-th round
+    const int j = 8 * i + (mask_at(P, 8 * i + 2 * wave) ? 2 * wave : 0);
+    const char* k0 = half_at(P, j) + (long)slot_at(P, j) * (2 * row);
+    const char* k1 = half_at(P, j + 1) + (long)slot_at(P, j + 1) * (2 * row);
+    return (c < 8 ? k0 : k1) + ((8 * (c / 4 % 2) + c % 4) * row + 8 * g) * 2;
+  };
+  auto k_at = [&](const char* kl, int kk, int u) {
+    return *reinterpret_cast<const bf16x8*>(kl + 8 * u * row + (32 * kk + 8 * g < row ? 64 * kk : -16 * g));
+  };
+  struct Values {
+    bf16x8 v[PER];
+  };
+  auto v_fetch = [&](const Places& P, int i, int w) -> Values {       // tile w of the i-th round
+    Values V;
+    const int j = 8 * i + (mask_at(P, 8 * i + 2 * w) ? 2 * w : 0);
+    const char* v0 = half_at(P, j) + 2L * page_size * row + 2 * slot_at(P, j);
+    const char* v1 = half_at(P, j + 1) + 2L * page_size * row + 2 * slot_at(P, j + 1);
+    const char* vl = (g < 2 ? v0 : v1) + ((16 * wave + c) * page_size + 8 * (g % 2)) * 2;
 #pragma unroll
-  for (int kk = 0; kk < KS; ++kk) {
-    const int d0 = 32 * kk + 8 * g;
-    qreg[kk] = (d0 < row && head_ok) ? *reinterpret_cast<const bf16x8*>(qrow + d0) : zero8;
+    for (int r = 0; r < PER; ++r)
+      V.v[r] = *reinterpret_cast<const bf16x8*>(vl + (16 * (4 * r + wave) < rank ? 128L * r * page_size : -32L * wave * page_size));
+    return V;
+  };
+
+  Places first = lookup(slice);
+  // The heads' queries go to LDS, zeros behind a row up to whole steps (there a key's row brings another piece of itself): asked for
+  // behind the pages, written once the first keys are on their way.
+  const int steps = KS > 0 ? KS : (row + 31) / 32;
+  auto q_load = [&](int i) {
+    const int h = i / (4 * steps), d0 = 8 * (i % (4 * steps));
+    return *reinterpret_cast<const bf16x8*>(q + ((long)t * H + min(h0 + h, H - 1)) * row + (d0 < row ? d0 : 0));
+  };
+  auto q_store = [&](int i, bf16x8 v) {
+    const int h = i / (4 * steps), d0 = 8 * (i % (4 * steps));
+    if (d0 >= row) v = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    *reinterpret_cast<bf16x8*>(&queries[h * QLD + d0]) = v;
+  };
+  auto q_at = [&](int kk) { return *reinterpret_cast<const bf16x8*>(&queries[c * QLD + 32 * kk + 8 * g]); };
+  constexpr int QN = KS > 0 ? (64 * KS + 64 * kLatWaves - 1) / (64 * kLatWaves) : 1;
+  bf16x8 qv[QN];
+  if constexpr (KS > 0) {
+#pragma unroll
+    for (int j = 0; j < QN; ++j) qv[j] = q_load(min((int)threadIdx.x + 64 * kLatWaves * j, 64 * KS - 1));
+    __builtin_amdgcn_sched_barrier(0);
   }
 
   float m = -INFINITY, l = 0.f;
-  floatx4 acc[NR];
+  floatx4 acc[PER];
 #pragma unroll
-  for (int r = 0; r < NR; ++r) acc[r] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-  // The tiles go in turn to the slices (workgroups of the same token and heads, blockIdx.z: where
-  // tokens and heads alone leave CUs idle) and, within a slice, to the waves.
-  const int nslices = gridDim.z, slice = blockIdx.z;
-  const int tiles = (len + 31) / 32;
-  const unsigned k_lane = c * row + 8 * g, v_lane = c * page_size + 4 * g;       // this lane's place in a half's rows and latents
-  for (int tile = lo / 32 + slice * kLatWaves + wave; tile < tiles; tile += kLatWaves * nslices) {
-    const int kb = tile * 32;
-    // A half (16 keys) lies in one page (pages hold a multiple of 16 slots).  Loads carry no branch,
-    // so that many are in flight: a half that is not read takes page 0, whose rows make scores that
-    // are masked (a row is one key's alone) and whose latents are replaced by zeros.
-    const bf16_t* pbase[2];
-    int slot0[2];
-    bool live[2];
+  for (int r = 0; r < PER; ++r) acc[r] = floatx4{0.f, 0.f, 0.f, 0.f};
+  int parity = 0;
+  for (int r0 = slice; r0 < rounds; r0 += 8 * nslices) {
+    if (r0 != slice) first = lookup(r0);
+    const Places P = placed(first);
+    bf16x8 kr[KS > 0 ? KS : 1][2];
+    auto k_fetch = [&](int i) {
+      const char* kl = key_row(P, i);
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int k0 = kb + 16 * u;
-      live[u] = k0 < len && k0 + 16 > lo;                    // (a half behind the window may lie in a page that is gone)
-      const int pi = live[u] ? (int)(__umulhi((unsigned)k0, page_magic) >> 3) : 0;   // k0 / page_size (see the launch)
-      // (the same in every lane: said so explicitly, which keeps the addresses on the scalar unit)
-      const int page = __builtin_amdgcn_readfirstlane(table[pi]);
-      pbase[u] = cache + (long)(live[u] ? page : 0) * page_elems;
-      slot0[u] = live[u] ? k0 - pi * page_size : 0;
-    }
-    const bf16_t* krow[2] = {pbase[0] + (long)slot0[0] * row, pbase[1] + (long)slot0[1] * row};      // + this lane's place
-    const bf16_t* vt[2] = {pbase[0] + (long)page_size * row + slot0[0], pbase[1] + (long)page_size * row + slot0[1]};
-    // ---- the latents' pieces, RB at a time: the first asked for behind the scores' products
-    constexpr int RB = NR < 16 ? NR : 16;
-    struct Piece {
-      bf16x4 v[RB][2];
+      for (int kk = 0; kk < KS; ++kk)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) kr[kk][u] = k_at(kl, kk, u);
+      __builtin_amdgcn_sched_barrier(0);
     };
-    auto v_fetch = [&](int r0) -> Piece {
-      Piece P;
+    k_fetch(0);
+    if (r0 == slice) {
+      if constexpr (KS > 0) {
 #pragma unroll
-      for (int r = 0; r < RB; ++r)
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-          P.v[r][u] = *reinterpret_cast<const bf16x4*>(vt[u] + (long)(16 * min(r0 + r, nr - 1)) * page_size + v_lane);
-      return P;
-    };
-    floatx4 s[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
-    if constexpr (KS > 0) {
-      // the keys' pieces, KB steps at a time and one group ahead of the products
-      constexpr int KB = KS % 6 == 0 ? 6 : KS % 5 == 0 ? 5 : 4;
-      static_assert(KS % KB == 0, "whole groups of steps");
-      bf16x8 a[2][KB][2];
-      auto k_fetch = [&](bf16x8 (&dst)[KB][2], int j0) {
-#pragma unroll
-        for (int j = 0; j < KB; ++j)
-#pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            const int d0 = 32 * (j0 + j) + 8 * g;
-            dst[j][u] = *reinterpret_cast<const bf16x8*>(krow[u] + k_lane + (unsigned)(d0 < row ? 32 * (j0 + j) : 0));
-          }
-      };
-      k_fetch(a[0], 0);
-#pragma unroll
-      for (int j0 = 0; j0 < KS; j0 += KB) {
-        if (j0 + KB < KS) k_fetch(a[(j0 / KB + 1) % 2], j0 + KB);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int j = 0; j < KB; ++j)
-#pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            const bool in = 32 * (j0 + j) + 8 * g < row;     // beyond a row: another slot's, anything
-            s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(in ? a[j0 / KB % 2][j][u] : zero8, qreg[j0 + j], s[u], 0, 0, 0);
-          }
-        __builtin_amdgcn_sched_barrier(0);
+        for (int j = 0; j < QN; ++j) q_store(min((int)threadIdx.x + 64 * kLatWaves * j, 64 * KS - 1), qv[j]);
+      } else {
+        for (int i = threadIdx.x; i < 64 * steps; i += 64 * kLatWaves) q_store(i, q_load(i));
       }
-    } else {
-      for (int ks = 0; ks < ksteps; ++ks) {
-        const int d0 = 32 * ks + 8 * g, da = d0 < row ? d0 : 0;
-        const bf16x8 qv = *reinterpret_cast<const bf16x8*>(qrow + da);
-        const bf16x8 qb = (d0 < row && head_ok) ? qv : zero8;
+      // (what is in LDS, not what is on its way from memory: __syncthreads would wait for the keys)
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(0xC07F);
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
+#pragma unroll 1
+    for (int i = 0; i < 8 && r0 + i * nslices < rounds; ++i, parity ^= 1) {
+      Values V[kLatWaves];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const bf16x8 a = *reinterpret_cast<const bf16x8*>(krow[u] + c * row + da);
-          s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d0 < row ? a : zero8, qb, s[u], 0, 0, 0);
+      for (int w = 0; w < kLatWaves; ++w) V[w] = v_fetch(P, i, w);
+      __builtin_amdgcn_sched_barrier(0);
+      floatx4 s[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+      if constexpr (KS > 0) {
+        constexpr int QB = KS % 6 == 0 ? 6 : 4;        // pieces of the query, a group ahead of the products
+        static_assert(KS % QB == 0, "whole groups of steps");
+        bf16x8 qb[2][QB];
+#pragma unroll
+        for (int kk = 0; kk < QB; ++kk) qb[0][kk] = q_at(kk);
+#pragma unroll
+        for (int k0 = 0; k0 < KS; k0 += QB) {
+#pragma unroll
+          for (int kk = 0; kk < QB; ++kk)
+            if (k0 + QB < KS) qb[(k0 / QB + 1) % 2][kk] = q_at(k0 + QB + kk);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int kk = 0; kk < QB; ++kk)
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+              s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kr[k0 + kk][u], qb[k0 / QB % 2][kk], s[u], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (i < 7 && r0 + (i + 1) * nslices < rounds) k_fetch(i + 1);
+      } else {
+        const char* kl = key_row(P, i);
+        for (int k0 = 0; k0 < steps; k0 += 4) {
+          bf16x8 kv[4][2];
+#pragma unroll
+          for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) kv[kk][u] = k_at(kl, min(k0 + kk, steps - 1), u);
+#pragma unroll
+          for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+              if (k0 + kk < steps) s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv[kk][u], q_at(k0 + kk), s[u], 0, 0, 0);
         }
       }
-    }
-    Piece piece = v_fetch(0);
-    __builtin_amdgcn_sched_barrier(0);
-    // ---- online softmax for this lane's head over its 8 keys, then over the 4 lanes of the column
-    float tmax = -INFINITY;
+      // ---- online softmax, in units of log2(e): the heads' maxima over the round's four tiles first
+      const unsigned mine = mask_at(P, 8 * i + 2 * wave) >> (8 * g);
+      float sc[8], tmax = -INFINITY;
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int key = kb + 16 * u + 4 * g + i;
-        s[u][i] = (key < len && key >= lo) ? s[u][i] * scale : -INFINITY;
-        tmax = fmaxf(tmax, s[u][i]);
+      for (int e = 0; e < 8; ++e) {
+        sc[e] = (mine >> e) & 1u ? s[e / 4][e % 4] * scale2 : -INFINITY;
+        tmax = fmaxf(tmax, sc[e]);
       }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, kWave));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
-    const float m_new = fmaxf(m, tmax);                    // finite: every tile holds a key that is read
-    const float alpha = expf(m - m_new);
-    bf16x8 pb;
-    float psum = 0.f;
+      tmax = group4_max(tmax);
+      if (g == 0) meet[parity][wave][c] = tmax;
+      __syncthreads();
+      float m_new = m;
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+      for (int w = 0; w < kLatWaves; ++w) m_new = fmaxf(m_new, meet[parity][w][c]);     // finite: every round holds a key that is read
+      const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+      bf16x8 pb;
+      float psum = 0.f;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float p = (s[u][i] == -INFINITY) ? 0.f : expf(s[u][i] - m_new);
-        const bf16_t pr = (bf16_t)p;
-        pb[4 * u + i] = pr;
-        psum += (float)pr;
+      for (int e = 0; e < 8; ++e) {
+        pb[e] = (bf16_t)__builtin_amdgcn_exp2f(sc[e] - m_new);
+        psum += (float)pb[e];
       }
-    l = l * alpha + psum;
-    m = m_new;
-    // ---- the weighted sum of the latents: slots beyond the last key may hold anything
-    const bool edge = !live[0] || kb + 32 > len;
+      *reinterpret_cast<bf16x8*>(&probs[parity][c * PLD + 32 * wave + 8 * g]) = pb;
+      l = l * alpha + psum;
+      if (__builtin_amdgcn_ballot_w64(m_new > m)) {
 #pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      if (r < nr) {
-        acc[r] *= alpha;
-        bf16x8 a;
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            a[4 * u + i] = (!edge || (live[u] && kb + 16 * u + 4 * g + i < len)) ? piece.v[r % RB][u][i] : (bf16_t)0.f;
-        acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb, acc[r], 0, 0, 0);
+        for (int r = 0; r < PER; ++r) acc[r] *= alpha;
       }
-      if (r % RB == RB - 1 && r + 1 < NR) {
-        piece = v_fetch(r + 1);
-        __builtin_amdgcn_sched_barrier(0);
+      m = m_new;
+      __syncthreads();
+      // ---- the weighted sum of the latents: slots of keys that are not read may hold anything
+#pragma unroll
+      for (int w = 0; w < kLatWaves; ++w) {
+        const unsigned mask = mask_at(P, 8 * i + 2 * w);
+        if (mask != ~0u) {
+          typedef unsigned uint4_t __attribute__((ext_vector_type(4)));
+          const unsigned own = mask >> (8 * g);
+          uint4_t keep;
+#pragma unroll
+          for (int d = 0; d < 4; ++d) keep[d] = ((own >> (2 * d)) & 1u ? 0xFFFFu : 0u) | ((own >> (2 * d + 1)) & 1u ? 0xFFFF0000u : 0u);
+#pragma unroll
+          for (int r = 0; r < PER; ++r) V[w].v[r] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(uint4_t, V[w].v[r]) & keep);
+        }
+        const bf16x8 pw = *reinterpret_cast<const bf16x8*>(&probs[parity][c * PLD + 32 * w + 8 * g]);
+#pragma unroll
+        for (int r = 0; r < PER; ++r) acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(V[w].v[r], pw, acc[r], 0, 0, 0);
       }
     }
   }
-  l += __shfl_xor(l, 16, kWave);
-  l += __shfl_xor(l, 32, kWave);
-
-  // ---- the waves meet: each leaves maximum, sum and output in LDS (lane-contiguous), then adds its share
-  // of the elements of all of them in a fixed order with weights exp(m_w - max m) and writes
-  constexpr int kRows = NR * 4 + 2;
-  float* mine = lat_red + (long)wave * kRows * kWave + lane;
-#pragma unroll
-  for (int r = 0; r < NR; ++r)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) mine[(4 * r + i) * kWave] = acc[r][i];
-  mine[(NR * 4) * kWave] = m;
-  mine[(NR * 4 + 1) * kWave] = l;
+  l = group4_sum(l);
+  if (g == 0) meet[parity][wave][c] = l;
   __syncthreads();
+  float L = 0.f;
+#pragma unroll
+  for (int w = 0; w < kLatWaves; ++w) L += meet[parity][w][c];
   if (!head_ok) return;
-  const float* all = lat_red + lane;
-  float ww[kLatWaves], M = -INFINITY, L = 0.f;
-#pragma unroll
-  for (int w = 0; w < kLatWaves; ++w) M = fmaxf(M, all[(w * kRows + NR * 4) * kWave]);
-#pragma unroll
-  for (int w = 0; w < kLatWaves; ++w) {
-    const float mw = all[(w * kRows + NR * 4) * kWave];
-    ww[w] = (mw == -INFINITY) ? 0.f : expf(mw - M);        // (a slice beyond the token's keys has none)
-    L += ww[w] * all[(w * kRows + NR * 4 + 1) * kWave];
-  }
-  // of a slice the sums as they are, with its maximum and its sum of probabilities: rows of rank + 2
-  // floats; a slice without a key leaves a maximum of -inf and zeros
-  float* prow = nslices > 1 ? part + (((long)t * H + head) * nslices + slice) * (rank + 2) : nullptr;
-  const float inv = nslices > 1 ? 1.f : 1.f / L;
+  // of a slice the sums as they are, with its maximum (in units of log2(e)) and its sum of probabilities
+  const float inv = 1.f / L;
   bf16_t* orow = out + ((long)t * H + head) * rank;
 #pragma unroll
-  for (int j = 0; j < NR / kLatWaves; ++j) {
-    const int r = wave * (NR / kLatWaves) + j;
-    if (r >= nr) continue;
-    floatx4 o = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int w = 0; w < kLatWaves; ++w)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = fmaf(ww[w], all[(w * kRows + 4 * r + i) * kWave], o[i]);
+  for (int j = 0; j < PER; ++j) {
+    const int r = 4 * j + wave;
+    if (16 * r >= rank) continue;
     if (nslices > 1) {                                       // (rows are 8-byte aligned)
-      *reinterpret_cast<floatx2*>(prow + 16 * r + 4 * g) = floatx2{o[0], o[1]};
-      *reinterpret_cast<floatx2*>(prow + 16 * r + 4 * g + 2) = floatx2{o[2], o[3]};
+      *reinterpret_cast<floatx2*>(prow + 16 * r + 4 * g) = floatx2{acc[j][0], acc[j][1]};
+      *reinterpret_cast<floatx2*>(prow + 16 * r + 4 * g + 2) = floatx2{acc[j][2], acc[j][3]};
     } else {
       *reinterpret_cast<bf16x4*>(orow + 16 * r + 4 * g) =
-          bf16x4{(bf16_t)(o[0] * inv), (bf16_t)(o[1] * inv), (bf16_t)(o[2] * inv), (bf16_t)(o[3] * inv)};
+          bf16x4{(bf16_t)(acc[j][0] * inv), (bf16_t)(acc[j][1] * inv), (bf16_t)(acc[j][2] * inv), (bf16_t)(acc[j][3] * inv)};
     }
   }
-  if (nslices > 1 && wave == 0 && g == 0) *reinterpret_cast<floatx2*>(prow + rank) = floatx2{M, L};
+  if (nslices > 1 && wave == 0 && g == 0) *reinterpret_cast<floatx2*>(prow + rank) = floatx2{m, L};
 }
 
 // The same for steps of many tokens: a workgroup takes four consecutive tokens of the step and up
@@ -944,35 +997,42 @@ static int launch_latent_columns(const void* q, void* out, const void* cache, co
   return 0;
 }
 
-// The slices' results of one (token, head) become its output: weights exp(m_s - max m).  A lane takes one
-// slice's maximum and sum (up to 64 slices) and works out its weight; the weights wait in LDS while
-// eight slices' outputs at a time are asked for.
-__global__ __launch_bounds__(kLatThreads) void attn_latent_merge_kernel(const float* __restrict__ part,
-                                                                        bf16_t* __restrict__ out, int rank, int nslices) {
-  __shared__ float weight[kWave];
+// The slices' results of one (token, head) become its output: weights exp2(m_s - max m).  Lane s takes slice s's maximum and sum and works
+// out its weight, each wave for itself; every slice's outputs are asked for behind them, so that all of it is one trip to memory (weights
+// first and then eight slices at a time: 9.6 us for 8 tokens, 32 heads and 32 slices of 512; so 4.9 with 16).  R: at least the number of slices.
+template <int R>
+__global__ __launch_bounds__(kLatThreads) void attn_latent_merge_kernel(const float* __restrict__ part, int rank, int nslices,
+                                                                        bf16_t* __restrict__ out) {
+  const int lane = threadIdx.x % kWave, bytes = (rank + 2) * (int)sizeof(float);
   const long th = blockIdx.x;
-  const long stride = rank + 2;
-  const float* rows = part + th * nslices * stride;
-  const int lane = threadIdx.x % kWave;
-  const bool there = lane < nslices;
-  const float ms = there ? rows[lane * stride + rank] : -INFINITY;
-  const float ls = there ? rows[lane * stride + rank + 1] : 0.f;
-  const float M = wave_max(ms);                               // finite: some slice holds the token's own key
-  const float w = ms == -INFINITY ? 0.f : expf(ms - M);
-  const float inv = 1.f / wave_sum(w * ls);
-  if (threadIdx.x < kWave) weight[lane] = w * inv;            // 0 for a slice without a key
-  __syncthreads();
-  for (int e = threadIdx.x; e < rank; e += kLatThreads) {
+  const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<char*>(reinterpret_cast<const char*>(part)) + th * nslices * bytes, 0, nslices * bytes, 0x00020000);
+  auto load = [&](int at, int slice_at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rows, at, slice_at, 0)); };
+  const float m0 = load(lane * bytes + 4 * rank, 0), ls = load(lane * bytes + 4 * rank + 4, 0);      // (beyond the last slice zeros, from nowhere)
+  float v[2][R];
+#pragma unroll
+  for (int j = 0; j < R; ++j)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) v[e][j] = load(4 * min((int)threadIdx.x + e * kLatThreads, rank - 1), j * bytes);
+  __builtin_amdgcn_sched_barrier(0);
+  const float ms = lane < nslices ? m0 : -INFINITY;
+  const float M = first_lanes_max<R>(ms);                     // finite: some slice holds the token's own key
+  const float w = ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - M);
+  const float wn = w / wave_sum(w * ls);                      // 0 for a slice without a key, whose outputs may be anything
+#pragma unroll
+  for (int j = 0; j < R; ++j)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) asm volatile("" : "+v"(v[e][j]));
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
     float o = 0.f;
-    for (int s0 = 0; s0 < nslices; s0 += 8) {
-      float v[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = rows[min(s0 + j, nslices - 1) * stride + e];
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (s0 + j < nslices && weight[s0 + j] != 0.f) o = fmaf(weight[s0 + j], v[j], o);
+    for (int j = 0; j < R; ++j) {
+      const float wj = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wn), j));
+      o = fmaf(wj, wj == 0.f ? 0.f : v[e][j], o);
     }
-    out[th * rank + e] = (bf16_t)o;
+    const int at = threadIdx.x + e * kLatThreads;
+    if (at < rank) out[th * rank + at] = (bf16_t)o;
   }
 }
 
@@ -980,14 +1040,8 @@ template <int NR, int KS>
 static void launch_latent_mfma(const void* q, void* out, const void* cache, const int* positions, const int* span_of_token,
                                const int* block_table, int max_pages, int page_size, int n, int H, int row, int rank,
                                float scale, int window, float* part, int nslices, int redo, hipStream_t stream) {
-  const size_t lds = (size_t)kLatWaves * (NR * 4 + 2) * kWave * sizeof(float);
-  const unsigned page_magic = (unsigned)(((1ull << 35) + page_size - 1) / page_size);
-  static int raised = 0;
-  if (lds > 64 * 1024 && !raised) {
-    (void)hipFuncSetAttribute((const void*)attn_latent_mfma_kernel<NR, KS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    raised = 1;
-  }
   if (nslices == 0) {       // steps of many tokens: four tokens a workgroup, their keys through LDS
+    const unsigned page_magic = (unsigned)(((1ull << 35) + page_size - 1) / page_size);
     const size_t tiles = ((size_t)32 * (row + 8) + (size_t)rank * 36) * sizeof(bf16_t);
     static size_t raised_to = 64 * 1024;
     if (tiles > raised_to) {
@@ -999,11 +1053,15 @@ static void launch_latent_mfma(const void* q, void* out, const void* cache, cons
                        block_table, max_pages, page_size, page_magic, n, H, row, rank, scale, window, redo);
     return;
   }
-  hipLaunchKernelGGL((attn_latent_mfma_kernel<NR, KS>), dim3(n, (H + 15) / 16, nslices), dim3(64 * kLatWaves), lds, stream,
-                     (const bf16_t*)q, (bf16_t*)out, (const bf16_t*)cache, positions, span_of_token, block_table, max_pages,
-                     page_size, page_magic, H, row, rank, scale, window, part);
-  if (nslices > 1)
-    hipLaunchKernelGGL(attn_latent_merge_kernel, dim3(n * H), dim3(kLatThreads), 0, stream, part, (bf16_t*)out, rank, nslices);
+  const unsigned page16 = page_size / 16, magic16 = page16 == 1 ? 0xFFFFFFFFu : (unsigned)((1ull << 32) / page16);
+  hipLaunchKernelGGL((attn_latent_mfma_kernel<NR, KS>), dim3(n, (H + 15) / 16, nslices), dim3(64 * kLatWaves), 0, stream,
+                     (const bf16_t*)cache, positions, span_of_token, block_table, (const bf16_t*)q, max_pages, (int)page16, H, row, rank,
+                     magic16, scale, window, nslices, (bf16_t*)out, part);
+#define KLLM_LATM(R) hipLaunchKernelGGL(attn_latent_merge_kernel<R>, dim3(n * H), dim3(kLatThreads), 0, stream, part, rank, nslices, (bf16_t*)out)
+  if (nslices > 32) KLLM_LATM(64);
+  else if (nslices > 16) KLLM_LATM(32);
+  else if (nslices > 1) KLLM_LATM(16);
+#undef KLLM_LATM
 }
 
 // attended: [n][H][rank]; w_uv [H * dv][rank]; gate: [nsplit][n][H * dv] sums ([H] with by_head) or null.

@@ -2315,21 +2315,24 @@ def latent_query(q, w_uk, cos, sin, out, heads, dim, rot_dim, rank, transposed=F
 LATENT_BLOCK_FROM = 64      # tokens of a step from which four tokens share a workgroup and its tiles of keys
 
 
-def attn_latent_slices(n, heads, rank, dtype=torch.bfloat16, window=0) -> int:
+def attn_latent_slices(n, heads, rank, dtype=torch.bfloat16, window=0, max_keys=0) -> int:
     """Workgroups that share out the keys of a token and 16 heads (their results are merged in
-    the same call): as many as bring a step's workgroups to about two a CU, for steps of few
+    the same call): as many as bring a step's workgroups to about one a CU, which holds one (a step of 9 tokens at 2,600 keys with half as
+    many 795 us, 761, with twice as many 765; 24 tokens at 1,000 890, 863, 866), for steps of few
     tokens; 1 where the kernel on the matrix cores does not run; 0 for steps of many tokens: there
-    a workgroup takes four tokens, whose keys pass through LDS once for the four.  A ``window`` bounds a
-    token's keys: a slice has 128 of them at least.  Does not depend on any context
-    length, so a recorded step can be replayed as contexts grow."""
+    a workgroup takes four tokens, whose keys pass through LDS once for the four.  A slice has 128 keys at least, what a workgroup
+    takes at a time: ``max_keys`` (0: not known), the most keys of a token, and a ``window`` bound them.  Does not depend on any context
+    length beyond ``max_keys``, so a recorded step can be replayed as contexts grow."""
     if dtype != torch.bfloat16 or rank % 16 or rank > 512:
         return 1
     if n >= LATENT_BLOCK_FROM:
         return 0
     groups = n * ((heads + 15) // 16)
     slices = 1
-    most = min(32, -(-(window + 31) // 128)) if window else 32
-    while slices < most and groups * slices * 2 <= 2 * device_cus():
+    most = min(64, -(-(window + 31) // 128)) if window else 64
+    if max_keys:
+        most = min(most, -(-max_keys // 128))
+    while slices < most and groups * slices * 2 <= device_cus():
         slices *= 2
     return slices
 

@@ -130,8 +130,11 @@ class LatentAttention(Part):
             K.latent_query(q, self.w_uk, cos, sin, qa, self.heads, self.head_dim, self.rot_dim, self.kv_rank)
         attended = ctx.buf("latent.att", (n, self.heads * self.kv_rank), dtype)
         plain = self.runtime.options.get("attention", "auto") == "generic"
-        slices = 1 if plain or self.row % 8 or cache.page_size % 16 else K.attn_latent_slices(n, self.heads, self.kv_rank, dtype,
-                                                                                                           self.window)
+        pages = 8                # (the table's width, rounded up as recorded steps round theirs: see attention)
+        while pages < cache.block_table.shape[1]:
+            pages *= 2
+        slices = 1 if plain or self.row % 8 or cache.page_size % 16 else K.attn_latent_slices(
+            n, self.heads, self.kv_rank, dtype, self.window, pages * cache.page_size)
         part = ctx.buf("latent.part", (n * self.heads * slices * (self.kv_rank + 2),), torch.float32) if slices > 1 else None
         K.attn_latent(qa, attended, cache.pages, ctx.positions, ctx.span_of_token, cache.block_table, cache.page_size,
                       self.heads, self.row, self.kv_rank, self.scale, plain=plain, part=part, nslices=slices, window=self.window)

@@ -330,6 +330,48 @@ def test_attention_over_cached_latents(H, rank, dr, dtype):
         assert rel(got, want) < tol, (plain, slices)
 
 
+@pytest.mark.parametrize("H,row,rank,page", [(20, 544, 512, 16), (3, 104, 80, 48), (17, 640, 512, 32), (2, 704, 512, 16), (16, 288, 256, 80)])
+@pytest.mark.parametrize("window", [0, 150])
+def test_attention_through_latents_round_by_round(H, row, rank, page, window):
+    """Decode's kernel takes 128 keys a round: tokens with one key, with a round's edge on either side, and with more than the
+    eight rounds whose pages are looked up at once (2,321 keys in one slice are nineteen), rows that are no whole steps of 32, the sizes
+    whose steps are asked for four at a time, and slices without keys.  Slots and columns that hold nothing are NaN.  Probabilities and
+    output are rounded to 2^-9 each."""
+    from kllm_amd import kernels as K
+    g = torch.Generator().manual_seed(row + page)
+    lens = [1, 127, 128, 129, 2321]
+    maxp = -(-max(lens) // page)
+    table = torch.full((len(lens), maxp), -1, dtype=torch.int32)
+    cache = torch.full((sum(-(-n // page) for n in lens) + 1, page * (row + rank)), float("nan"))
+    keys, used = [], 1
+    for s, n in enumerate(lens):
+        kk = torch.randn(n, row, generator=g).bfloat16().float()
+        keys.append(kk.double())
+        for p in range(-(-n // page)):
+            here = kk[p * page:(p + 1) * page]
+            cache[used, :page * row].view(page, row)[:len(here)] = here
+            cache[used, page * row:].view(rank, page)[:, :len(here)] = here[:, :rank].T
+            table[s, p] = used
+            used += 1
+    q = (torch.randn(len(lens), H, row, generator=g) * 2).bfloat16()
+    scale = row ** -0.5
+    want = torch.zeros(len(lens), H, rank, dtype=F64)
+    for s, n in enumerate(lens):
+        kk = keys[s][max(0, n - window) if window else 0:]
+        want[s] = torch.softmax(q[s].double() @ kk.T * scale, -1) @ kk[:, :rank]
+    dev = lambda t: t.to("cuda")
+    args = (dev(cache.bfloat16()), dev(torch.tensor([n - 1 for n in lens], dtype=torch.int32)),
+            torch.arange(len(lens), dtype=torch.int32, device="cuda"), dev(table), page, H, row, rank, scale)
+    for slices in (1, 2, 16, 64):
+        out = torch.full((len(lens), H * rank), float("nan"), dtype=torch.bfloat16, device="cuda")
+        part = torch.full((len(lens) * H * slices * (rank + 2),), float("nan"), device="cuda") if slices > 1 else None
+        K.attn_latent(dev(q.view(len(lens), H * row)), out, *args, part=part, nslices=slices, window=window)
+        got = out.float().cpu().view(len(lens), H, rank)
+        assert torch.isfinite(got).all()
+        for s in range(len(lens)):
+            assert rel(got[s], want[s]) < 2 ** -7, (slices, s, rel(got[s], want[s]))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("n,H,d,dr,dv,rank", [(1, 3, 16, 8, 20, 40), (37, 6, 64, 32, 64, 160), (130, 3, 128, 64, 128, 448),
                                               (5, 20, 32, 16, 24, 96), (70, 2, 96, 8, 200, 64)])
