@@ -136,20 +136,45 @@ __device__ __forceinline__ float gated(float g, float u, int act, float limit, f
   return gate_act(g, act) * u;
 }
 
+// Lanes exchange within a row of sixteen by moves that cost an instruction each, and between rows by swaps of rows (of halves) of a value with
+// itself, which leave every lane its own and its partner's: nothing here goes through LDS (six exchanges in a row there were 0.3 us of a
+// short launch's norm).
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+  const int moved = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true);   // (every lane has a source: the move folds into the add)
+  return v + __builtin_bit_cast(float, moved);
+}
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_max(float v) {
+  return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true)));
+}
+// Over lanes c, c + 16, c + 32, c + 48.
+__device__ __forceinline__ float group4_max(float v) {
+  unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  u = __builtin_bit_cast(unsigned, fmaxf(__builtin_bit_cast(float, (unsigned)a[0]), __builtin_bit_cast(float, (unsigned)a[1])));
+  const auto b = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return fmaxf(__builtin_bit_cast(float, (unsigned)b[0]), __builtin_bit_cast(float, (unsigned)b[1]));
+}
+__device__ __forceinline__ float group4_sum(float v) {
+  unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  u = __builtin_bit_cast(unsigned, __builtin_bit_cast(float, (unsigned)a[0]) + __builtin_bit_cast(float, (unsigned)a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __builtin_bit_cast(float, (unsigned)b[0]) + __builtin_bit_cast(float, (unsigned)b[1]);
+}
+
+// Over all lanes; every lane has the same bits.
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
-  return v;
+  return group4_sum(dpp_add<0x140>(dpp_add<0x141>(dpp_add<0x4E>(dpp_add<0xB1>(v)))));
 }
 
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, kWave));
-  return v;
+  return group4_max(dpp_max<0x140>(dpp_max<0x141>(dpp_max<0x4E>(dpp_max<0xB1>(v)))));
 }
 
-// Sum over a workgroup of up to 1024 threads. `red` is LDS of at least 16
-// floats. Every thread gets the result; the order of additions is fixed.
+// Over a workgroup of up to sixteen waves: their results are one read of LDS, a result to a lane of each row.
 __device__ __forceinline__ float block_sum(float v, float* red) {
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int nwaves = (blockDim.x + kWave - 1) / kWave;
@@ -157,9 +182,9 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   __syncthreads();  // red may still be read from an earlier call
   if (lane == 0) red[wave] = v;
   __syncthreads();
-  float total = 0.f;
-  for (int w = 0; w < nwaves; ++w) total += red[w];
-  return total;
+  v = red[lane % 16 < nwaves ? lane % 16 : 0];
+  v = lane % 16 < nwaves ? v : 0.f;
+  return dpp_add<0x140>(dpp_add<0x141>(dpp_add<0x4E>(dpp_add<0xB1>(v))));
 }
 
 __device__ __forceinline__ float block_max(float v, float* red) {
@@ -169,9 +194,8 @@ __device__ __forceinline__ float block_max(float v, float* red) {
   __syncthreads();
   if (lane == 0) red[wave] = v;
   __syncthreads();
-  float total = red[0];
-  for (int w = 1; w < nwaves; ++w) total = fmaxf(total, red[w]);
-  return total;
+  v = red[lane % 16 < nwaves ? lane % 16 : 0];
+  return dpp_max<0x140>(dpp_max<0x141>(dpp_max<0x4E>(dpp_max<0xB1>(v))));
 }
 
 // ---- errors ---------------------------------------------------------------
@@ -212,39 +236,17 @@ inline int ceil_div(long a, long b) { return (int)((a + b - 1) / b); }
 // lane getting the sum: within a row of 16 lanes by data-parallel moves (neighbour, other pair,
 // mirrored half row, mirrored row), which cost an instruction each; across the two rows of a
 // group of 32 by a lane exchange.
-template <int CTRL>
-__device__ __forceinline__ float dpp_add(float v) {
-  const int moved = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true);   // (every lane has a source: the move folds into the add)
-  return v + __builtin_bit_cast(float, moved);
-}
-
 template <int PARTS>
 __device__ __forceinline__ float parts_sum(float v) {
   if (PARTS >= 2) v = dpp_add<0xB1>(v);     // quad_perm [1,0,3,2]
   if (PARTS >= 4) v = dpp_add<0x4E>(v);     // quad_perm [2,3,0,1]
   if (PARTS >= 8) v = dpp_add<0x141>(v);    // row_half_mirror
   if (PARTS >= 16) v = dpp_add<0x140>(v);   // row_mirror
-  if (PARTS >= 32) v += __shfl_xor(v, 16, kWave);
-  if (PARTS >= 64) v += __shfl_xor(v, 32, kWave);
+  if (PARTS == 32) v += __shfl_xor(v, 16, kWave);
+  if (PARTS >= 64) v = group4_sum(v);
   return v;
 }
 
-// Over lanes c, c + 16, c + 32, c + 48, without a trip through LDS: a swap of rows of sixteen (of halves) of a value with itself
-// leaves every lane its own and its partner's.
-__device__ __forceinline__ float group4_max(float v) {
-  unsigned u = __builtin_bit_cast(unsigned, v);
-  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  u = __builtin_bit_cast(unsigned, fmaxf(__builtin_bit_cast(float, (unsigned)a[0]), __builtin_bit_cast(float, (unsigned)a[1])));
-  const auto b = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return fmaxf(__builtin_bit_cast(float, (unsigned)b[0]), __builtin_bit_cast(float, (unsigned)b[1]));
-}
-__device__ __forceinline__ float group4_sum(float v) {
-  unsigned u = __builtin_bit_cast(unsigned, v);
-  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  u = __builtin_bit_cast(unsigned, __builtin_bit_cast(float, (unsigned)a[0]) + __builtin_bit_cast(float, (unsigned)a[1]));
-  const auto b = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return __builtin_bit_cast(float, (unsigned)b[0]) + __builtin_bit_cast(float, (unsigned)b[1]);
-}
 // x / d and what is left, with magic = 2^32 / d rounded down (2^32 - 1 for d = 1): the product is the quotient or one less.
 __device__ __forceinline__ unsigned divided(unsigned x, unsigned d, unsigned magic, unsigned& left) {
   unsigned r = __umulhi(x, magic);
@@ -256,10 +258,6 @@ __device__ __forceinline__ unsigned divided(unsigned x, unsigned d, unsigned mag
 constexpr float kLog2E = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
 
 // The greatest of the first R lanes' values (-infinity in the others), the same in every lane.
-template <int CTRL>
-__device__ __forceinline__ float dpp_max(float v) {
-  return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true)));
-}
 template <int R>
 __device__ __forceinline__ float first_lanes_max(float v) {
   v = dpp_max<0xB1>(v);     // quad_perm [1,0,3,2]

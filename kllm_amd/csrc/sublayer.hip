@@ -54,18 +54,41 @@ struct NormedPair {
 // pair wider than 4,096 waited in LDS as two rows.  With the stores of the stream behind all of its elements' sums 4.7 and 6.5.
 enum : int { PAIR_NONE = 0, PAIR_NORMED = 1, PAIR_ADDED = 2 };
 
-template <typename TOUT, int PER, int PAIR>
+// Element i of the j-th of a thread's PER: one in kRowThreads, or (VEC: rows and pointers of whole 16 bytes) four in a row.
+template <bool VEC>
+__device__ __forceinline__ int row_at(int j) {
+  return VEC ? 4 * (int)threadIdx.x + 4 * kRowThreads * (j / 4) + j % 4 : (int)threadIdx.x + kRowThreads * j;
+}
+template <int PER, bool VEC>
+__device__ __forceinline__ void row_load(float (&v)[PER], const float* __restrict__ src, int d) {
+  if constexpr (VEC) {
+#pragma unroll
+    for (int j = 0; j < PER; j += 4) {
+      const int i = row_at<VEC>(j);
+      const floatx4 q = *reinterpret_cast<const floatx4*>(src + (i < d ? i : 0));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[j + e] = q[e];
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < PER; ++j) v[j] = src[row_at<VEC>(j) < d ? row_at<VEC>(j) : 0];
+  }
+}
+
+// CHOSEN: with the sums of chosen experts (an instance of its own: the others carry none of it).  The first fourteen words of the
+// arguments, all that the loads need, lie in registers when a wave starts.  At a few rows a launch is its trips to memory and its row
+// sums: with loads behind branches, element by element, the next weight asked for at the end and sums through LDS exchanges a step of Natenex
+// layers (16 such launches) took 668 us at 8 tokens, so 655; 1,500 rows of 2,048 11.8 us a launch, so 11.0.
+template <typename TOUT, int PER, int PAIR, bool CHOSEN, bool VEC>
 __global__ __launch_bounds__(kRowThreads) void norm_residual_kernel(
-    float* __restrict__ x, const float* __restrict__ delta, int nsplit, long split_stride,
-    const float* __restrict__ bias, const float* __restrict__ w, TOUT* __restrict__ out, int d, float eps,
-    const ChosenSums chosen, float mult, const float* __restrict__ next_w, const float* __restrict__ delta_scale,
-    const NormedPair pair) {
+    const float* __restrict__ delta, float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ next_w, int d, int nsplit,
+    long split_stride, float eps, float mult, TOUT* __restrict__ out, const float* __restrict__ bias,
+    const float* __restrict__ delta_scale, const NormedPair pair, const ChosenSums chosen) {
   extern __shared__ float row_lds[];      // [d] (PER == 0; twice that with a pair)
   __shared__ float red[16];
   const long r = blockIdx.x;
-  const float dscale = delta_scale ? delta_scale[r] : 1.f;      // a factor of the row's delta (a gate of a shared expert)
   float* xr = x + r * d;
-  const bool sums = delta || chosen.y;    // otherwise the stream itself is normalised
+  const bool sums = delta || (CHOSEN && chosen.y);    // otherwise the stream itself is normalised
   auto chosen_at = [&](int i) {
     float t = 0.f;
     for (int s = 0; s < chosen.top; ++s) {
@@ -81,128 +104,132 @@ __global__ __launch_bounds__(kRowThreads) void norm_residual_kernel(
     return t;
   };
   if constexpr (PER > 0) {
-    // Loops over slices and choices stand outside the loop over a thread's elements, whose
-    // loads then go out together (a load behind a loop of unknown length is waited for at once).
-    float v[PER], xv[PER], wv[PER];
-    int at[PER];
-#pragma unroll
-    for (int j = 0; j < PER; ++j) {
-      const int i = threadIdx.x + kRowThreads * j;
-      at[j] = i < d ? i : 0;
-      xv[j] = xr[at[j]];
-      wv[j] = w[at[j]];
-      v[j] = 0.f;
+    // Everything that the row needs goes out before the first use, the norms' weights too: a row costs one trip to memory (a second one per
+    // further slice; a load behind a loop of unknown length is waited for at once).
+    float v[PER], xv[PER], wv[PER], nv[PER], dv[PER];
+    row_load<PER, VEC>(dv, delta ? delta + r * d : xr, d);
+    row_load<PER, VEC>(xv, xr, d);
+    row_load<PER, VEC>(wv, w, d);
+    row_load<PER, VEC>(nv, next_w ? next_w : w, d);
+    float bv[PER], wa[PER], wb[PER];
+    if constexpr (PAIR != PAIR_NONE) row_load<PER, VEC>(bv, pair.b + r * d, d);
+    if constexpr (PAIR == PAIR_NORMED) {
+      row_load<PER, VEC>(wa, pair.wa, d);
+      row_load<PER, VEC>(wb, pair.wb, d);
     }
-    if (sums) {
-      if (chosen.y) {
+    const float dscale = delta_scale ? delta_scale[r] : 1.f;      // a factor of the row's delta (a gate of a shared expert)
+#pragma unroll
+    for (int j = 0; j < PER; ++j) v[j] = 0.f;
+    if (!CHOSEN || sums) {
+      if (CHOSEN && chosen.y) {
         for (int s = 0; s < chosen.top; ++s) {
           const long entry = r * chosen.top + s;
           const float weight = chosen.wgt[entry];
+          float t[PER];
           if (chosen.idx[entry] < chosen.E) {
-            const float* src = chosen.y + entry * d;
-#pragma unroll
-            for (int j = 0; j < PER; ++j) v[j] = fmaf(weight, src[at[j]], v[j]);
+            row_load<PER, VEC>(t, chosen.y + entry * d, d);
           } else if (chosen.xin_dtype == DT_BF16) {
             const bf16_t* src = reinterpret_cast<const bf16_t*>(chosen.xin) + r * d;
 #pragma unroll
-            for (int j = 0; j < PER; ++j) v[j] = fmaf(weight, to_f32(src[at[j]]), v[j]);
+            for (int j = 0; j < PER; ++j) t[j] = to_f32(src[row_at<VEC>(j) < d ? row_at<VEC>(j) : 0]);
           } else {
-            const float* src = reinterpret_cast<const float*>(chosen.xin) + r * d;
-#pragma unroll
-            for (int j = 0; j < PER; ++j) v[j] = fmaf(weight, src[at[j]], v[j]);
+            row_load<PER, VEC>(t, reinterpret_cast<const float*>(chosen.xin) + r * d, d);
           }
+#pragma unroll
+          for (int j = 0; j < PER; ++j) v[j] = fmaf(weight, t[j], v[j]);
         }
       }
       if (delta) {
-        float dv[PER];
+        for (int s = 1; s < nsplit; ++s) {
+          float t[PER];
+          row_load<PER, VEC>(t, delta + s * split_stride + r * d, d);
 #pragma unroll
-        for (int j = 0; j < PER; ++j) dv[j] = 0.f;
-        for (int s = 0; s < nsplit; ++s) {
-          const float* src = delta + s * split_stride + r * d;
-#pragma unroll
-          for (int j = 0; j < PER; ++j) dv[j] += src[at[j]];
+          for (int j = 0; j < PER; ++j) dv[j] += t[j];
         }
-        if constexpr (PAIR == PAIR_ADDED) {
-          float bv[PER];
+      }
+      if constexpr (PAIR != PAIR_NONE) {
+        for (int s = 1; s < pair.nb; ++s) {
+          float t[PER];
+          row_load<PER, VEC>(t, pair.b + s * pair.stride_b + r * d, d);
 #pragma unroll
-          for (int j = 0; j < PER; ++j) bv[j] = 0.f;
-          for (int s = 0; s < pair.nb; ++s) {
-            const float* src = pair.b + s * pair.stride_b + r * d;
-#pragma unroll
-            for (int j = 0; j < PER; ++j) bv[j] += src[at[j]];
-          }
-#pragma unroll
-          for (int j = 0; j < PER; ++j) dv[j] = fmaf(pair.sa, dv[j], pair.sb * bv[j]);
-        } else if constexpr (PAIR == PAIR_NORMED) {       // each of the two normed over the row before they are added
-          float bv[PER], wa[PER], wb[PER];
-#pragma unroll
-          for (int j = 0; j < PER; ++j) {
-            bv[j] = 0.f;
-            wa[j] = pair.wa[at[j]];
-            wb[j] = pair.wb[at[j]];
-          }
-          for (int s = 0; s < pair.nb; ++s) {
-            const float* src = pair.b + s * pair.stride_b + r * d;
-#pragma unroll
-            for (int j = 0; j < PER; ++j) bv[j] += src[at[j]];
-          }
-          float ssa = 0.f, ssb = 0.f;
-#pragma unroll
-          for (int j = 0; j < PER; ++j) {
-            if (threadIdx.x + kRowThreads * j >= d) dv[j] = bv[j] = 0.f;
-            ssa = fmaf(dv[j], dv[j], ssa);
-            ssb = fmaf(bv[j], bv[j], ssb);
-          }
-          const float ra = pair.sa / sqrtf(block_sum(ssa, red) / (float)d + eps);
-          const float rb = pair.sb / sqrtf(block_sum(ssb, red) / (float)d + eps);
-#pragma unroll
-          for (int j = 0; j < PER; ++j) dv[j] = fmaf(dv[j] * ra, wa[j], bv[j] * rb * wb[j]);
+          for (int j = 0; j < PER; ++j) bv[j] += t[j];
         }
+      }
+      if constexpr (PAIR == PAIR_ADDED) {
+#pragma unroll
+        for (int j = 0; j < PER; ++j) dv[j] = fmaf(pair.sa, dv[j], pair.sb * bv[j]);
+      } else if constexpr (PAIR == PAIR_NORMED) {         // each of the two normed over the row before they are added
+        float ssa = 0.f, ssb = 0.f;
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+          if (row_at<VEC>(j) >= d) dv[j] = bv[j] = 0.f;
+          ssa = fmaf(dv[j], dv[j], ssa);
+          ssb = fmaf(bv[j], bv[j], ssb);
+        }
+        const float ra = pair.sa / sqrtf(block_sum(ssa, red) / (float)d + eps);
+        const float rb = pair.sb / sqrtf(block_sum(ssb, red) / (float)d + eps);
+#pragma unroll
+        for (int j = 0; j < PER; ++j) dv[j] = fmaf(dv[j] * ra, wa[j], bv[j] * rb * wb[j]);
+      }
+      if (!CHOSEN || delta) {
 #pragma unroll
         for (int j = 0; j < PER; ++j) v[j] = fmaf(dscale, dv[j], v[j]);
       }
       if (bias) {
+        float t[PER];
+        row_load<PER, VEC>(t, bias, d);
 #pragma unroll
-        for (int j = 0; j < PER; ++j) v[j] += bias[at[j]];
+        for (int j = 0; j < PER; ++j) v[j] += t[j];
       }
     } else {
 #pragma unroll
       for (int j = 0; j < PER; ++j) v[j] = xv[j];
     }
-#pragma unroll
-    for (int j = 0; j < PER; ++j)
-      if (threadIdx.x + kRowThreads * j >= d) v[j] = 0.f;
     float ss = 0.f;
 #pragma unroll
-    for (int j = 0; j < PER; ++j) ss = fmaf(v[j], v[j], ss);
+    for (int j = 0; j < PER; ++j) {
+      if (row_at<VEC>(j) >= d) v[j] = 0.f;
+      ss = fmaf(v[j], v[j], ss);
+    }
     const float rstd = 1.f / sqrtf(block_sum(ss, red) / (float)d + eps);
     float ss2 = 0.f;
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-      const int i = threadIdx.x + kRowThreads * j;
       const float y = v[j] * rstd * wv[j];
-      v[j] = i < d ? (sums ? fmaf(mult, y, xv[j]) : y) : 0.f;
+      v[j] = row_at<VEC>(j) < d ? (sums ? fmaf(mult, y, xv[j]) : y) : 0.f;
       ss2 = fmaf(v[j], v[j], ss2);
     }
     // (behind all of them: between them a wait for the next element's loads would wait for the stores too)
+    if constexpr (VEC) {
 #pragma unroll
-    for (int j = 0; j < PER; ++j)
-      if (threadIdx.x + kRowThreads * j < d) xr[threadIdx.x + kRowThreads * j] = v[j];
+      for (int j = 0; j < PER; j += 4)
+        if (row_at<VEC>(j) < d) *reinterpret_cast<floatx4*>(xr + row_at<VEC>(j)) = floatx4{v[j], v[j + 1], v[j + 2], v[j + 3]};
+    } else {
+#pragma unroll
+      for (int j = 0; j < PER; ++j)
+        if (row_at<VEC>(j) < d) xr[row_at<VEC>(j)] = v[j];
+    }
     if (!out) return;
     if (next_w) {       // the norm in front of the next sub-layer, of the row that is still in registers
-#pragma unroll
-      for (int j = 0; j < PER; ++j) wv[j] = next_w[at[j]];
       const float rstd2 = 1.f / sqrtf(block_sum(ss2, red) / (float)d + eps);
 #pragma unroll
-      for (int j = 0; j < PER; ++j) v[j] = v[j] * rstd2 * wv[j];
+      for (int j = 0; j < PER; ++j) v[j] = v[j] * rstd2 * nv[j];
     }
+    if constexpr (VEC) {
+      typedef TOUT out4 __attribute__((ext_vector_type(4)));
 #pragma unroll
-    for (int j = 0; j < PER; ++j) {
-      const int i = threadIdx.x + kRowThreads * j;
-      if (i < d) out[r * d + i] = from_f32<TOUT>(v[j]);
+      for (int j = 0; j < PER; j += 4)
+        if (row_at<VEC>(j) < d)
+          *reinterpret_cast<out4*>(out + r * d + row_at<VEC>(j)) =
+              out4{from_f32<TOUT>(v[j]), from_f32<TOUT>(v[j + 1]), from_f32<TOUT>(v[j + 2]), from_f32<TOUT>(v[j + 3])};
+    } else {
+#pragma unroll
+      for (int j = 0; j < PER; ++j)
+        if (row_at<VEC>(j) < d) out[r * d + row_at<VEC>(j)] = from_f32<TOUT>(v[j]);
     }
     return;
   }
+  const float dscale = delta_scale ? delta_scale[r] : 1.f;
   float ra = 1.f, rb = 0.f;
   if (PAIR == PAIR_NORMED) {       // a pass of its own for the two sums of squares; the sums wait in LDS
     float ssa = 0.f, ssb = 0.f;
@@ -222,7 +249,7 @@ __global__ __launch_bounds__(kRowThreads) void norm_residual_kernel(
   for (int i = threadIdx.x; i < d; i += kRowThreads) {
     float v;
     if (sums) {
-      v = chosen.y ? chosen_at(i) : 0.f;
+      v = CHOSEN && chosen.y ? chosen_at(i) : 0.f;
       if (PAIR == PAIR_NORMED) {
         v = fmaf(dscale, fmaf(row_lds[i] * ra, pair.wa[i], row_lds[d + i] * rb * pair.wb[i]), v);
       } else if (delta) {
@@ -434,15 +461,24 @@ extern "C" int kllm_norm_residual(float* x, const float* delta, int nsplit, long
   KLLM_REQUIRE(!delta || nsplit >= 1, "norm_residual: nsplit %d", nsplit);
   KLLM_REQUIRE(delta || chosen_y || !bias, "norm_residual: a bias goes with sums");
   KLLM_REQUIRE(out_dtype == DT_F32 || out_dtype == DT_BF16, "norm_residual: unknown dtype %d", out_dtype);
-#define KLLM_NRP(TOUT, PER, PAIR)                                                                             \
-  hipLaunchKernelGGL((norm_residual_kernel<TOUT, PER, PAIR>), dim3(n), dim3(kRowThreads),                     \
-                     PER ? 0 : (size_t)d * sizeof(float) * (PAIR == PAIR_NORMED ? 2 : 1), stream, x, delta, nsplit, split_stride, \
-                     bias, weight, (TOUT*)out, d, eps, chosen, mult, next_weight, delta_scale, pair)
-#define KLLM_NR(TOUT, PER)                                  \
-  do {                                                      \
-    if (!pair_b) KLLM_NRP(TOUT, PER, PAIR_NONE);            \
-    else if (pair_wa) KLLM_NRP(TOUT, PER, PAIR_NORMED);     \
-    else KLLM_NRP(TOUT, PER, PAIR_ADDED);                   \
+  // whole 16 bytes a load where rows and pointers allow it (the output in bfloat16: 8)
+  const bool vec = d % 4 == 0 && split_stride % 4 == 0 && pair_stride % 4 == 0 &&
+                   (((uintptr_t)x | (uintptr_t)delta | (uintptr_t)weight | (uintptr_t)next_weight | (uintptr_t)bias | (uintptr_t)pair_b |
+                     (uintptr_t)pair_wa | (uintptr_t)pair_wb | (uintptr_t)out | (uintptr_t)chosen_y | (uintptr_t)chosen_x) & 15) == 0;
+#define KLLM_NRP(TOUT, PER, PAIR, CHOSEN, VEC)                                                                \
+  hipLaunchKernelGGL((norm_residual_kernel<TOUT, PER, PAIR, CHOSEN, VEC>), dim3(n), dim3(kRowThreads),        \
+                     PER ? 0 : (size_t)d * sizeof(float) * (PAIR == PAIR_NORMED ? 2 : 1), stream, delta, x, weight, next_weight, d, \
+                     nsplit, split_stride, eps, mult, (TOUT*)out, bias, delta_scale, pair, chosen)
+#define KLLM_NRV(TOUT, PER, PAIR, CHOSEN)                                                            \
+  do {                                                                                               \
+    if (PER > 0 && vec) KLLM_NRP(TOUT, PER, PAIR, CHOSEN, (PER > 0)); else KLLM_NRP(TOUT, PER, PAIR, CHOSEN, false); \
+  } while (0)
+#define KLLM_NR(TOUT, PER)                                        \
+  do {                                                            \
+    if (chosen_y) KLLM_NRV(TOUT, PER, PAIR_NONE, true);           \
+    else if (!pair_b) KLLM_NRV(TOUT, PER, PAIR_NONE, false);      \
+    else if (pair_wa) KLLM_NRV(TOUT, PER, PAIR_NORMED, false);    \
+    else KLLM_NRV(TOUT, PER, PAIR_ADDED, false);                  \
   } while (0)
   const bool bf = out && out_dtype == DT_BF16;
   if (d <= 4 * kRowThreads) {
@@ -455,6 +491,7 @@ extern "C" int kllm_norm_residual(float* x, const float* delta, int nsplit, long
     if (bf) KLLM_NR(bf16_t, 0); else KLLM_NR(float, 0);
   }
 #undef KLLM_NR
+#undef KLLM_NRV
 #undef KLLM_NRP
   KLLM_CHECK_LAUNCH("norm_residual");
   return 0;

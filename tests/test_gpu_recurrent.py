@@ -346,3 +346,32 @@ def test_linear_scan_leaves_the_inputs_of_more_channels_than_a_workgroup(W, span
     K().linear_recurrence_scan(a, b, proj, y_bias, got, 0, slots, span_start, span_pos, spans, out, longest=longest,
                                conv=(bias, taps, W))
     assert torch.equal(got, want) and torch.equal(out, alone)
+
+
+@pytest.mark.parametrize("d", [4, 7, 1020, 1026, 2048, 2046, 3000, 4093])
+@pytest.mark.parametrize("slices,paired", [(1, 0), (3, 0), (2, 1), (1, 2)])
+def test_norm_behind_a_sub_layer_whole_and_odd_rows(d, slices, paired):
+    """Rows that are read sixteen bytes at a time and rows (by their length, or by where they start) that are not, over the edges of a
+    thread's elements; slices, two sums side by side as they are (1) or normed (2), and the next norm's rows.  Sums of up to 4,093
+    squares in 32 bits: 1e-6 of the result."""
+    k = K()
+    g = torch.Generator().manual_seed(d + slices)
+    n, eps = 3, 1e-5
+    odd = 1 if d in (1020, 3000) else 0            # a first element that is not on 16 bytes
+    def dev(t):
+        flat = torch.empty(t.numel() + odd, device="cuda")
+        flat[odd:] = t.flatten().cuda()
+        return flat[odd:].view(t.shape)
+    x, w, w2 = torch.randn(n, d, generator=g), torch.randn(d, generator=g), torch.randn(d, generator=g)
+    a, b = torch.randn(slices, n, d, generator=g), torch.randn(2, n, d, generator=g)
+    wa, wb = torch.randn(d, generator=g), torch.randn(d, generator=g)
+    norm = lambda v: v / torch.sqrt((v * v).mean(-1, keepdim=True) + eps)
+    A, B = a.double().sum(0), b.double().sum(0)
+    delta = A if paired == 0 else 0.75 * A - 1.5 * B if paired == 1 else 0.75 * wa.double() * norm(A) - 1.5 * wb.double() * norm(B)
+    want = x.double() + 0.6 * w.double() * norm(delta)
+    xd, out = dev(x), torch.empty(n, d, device="cuda")
+    arg = dev(a) if paired == 0 else k.NormedPair(dev(a), 0.75, dev(wa) if paired == 2 else None, dev(b), -1.5, dev(wb) if paired == 2 else None)
+    k.norm_residual(xd, dev(w), arg, out=out, eps=eps, mult=0.6, next_weight=dev(w2))
+    for got, ref in ((xd, want), (out, norm(want) * w2.double())):
+        err = (got.double().cpu() - ref).norm() / ref.norm()
+        assert err < 1e-6, float(err)
