@@ -358,7 +358,8 @@ def decode_batch_fits(rt, x, m, copied=True):
 
 @functools.lru_cache(maxsize=4096)
 def _parts_best(n, m, k, dtype, unary, copied=True):
-    """Whether ``K.linear_rows`` is the fastest way to plain sums, or (``unary``) an activation of them, of n rows that are read row by row.
+    """Whether ``K.linear_rows`` is the fastest way to plain sums, or (``unary``) an activation of them, of n rows that are read row by row
+    (for bfloat16 up to 16 rows where the decode-batch kernel does not run: what it would run of those, ``_unstaged`` sends there as well).
     The decode-batch kernel has the rows in LDS, this one reads up to sixteen of them a load: up to eight rows it is the faster one where
     K is long enough, of 9 to 16 not (a step of Nusilix layers of 1,024 columns, there / here, with K of 1,024 here, too: 1 token 601 / 608 us, 2
     606 / 617, 8 678 / 714; us a product: 8 rows 2,048 x 1,024 3.8 / 4.6, 2,048 x 4,096 6.8 / 6.2, 1,024 x 1,408 in a step 3.9 / 5.3, 2,048 x 2,048 4.9 /
@@ -388,9 +389,22 @@ def parts_rows(rt, n, w, w_tiled, unary=False):
     return _parts_best(n if n <= 8 else -(-n // 16) * 16, m, k, dtype, unary, w_tiled is not None) and _rows_options(rt, n, k, dtype == torch.float32, w_tiled)
 
 
+def _unstaged(rt, n, m, k, dtype, w_tiled):
+    """Whether plain sums, or an activation of them, of up to 16 rows of bfloat16 that ``_parts_best`` leaves to the decode-batch
+    kernel come from ``K.linear_rows`` all the same.  That rule's figures are from before this kernel asked for the weights first and had its
+    arguments with the launch; now it is the faster at every size tried (us a product, decode-batch kernel / this one, at 1, 8 and 16 rows:
+    512 x 64 3.1 / 2.0, 3.4 / 2.4, 3.7 / 3.3; 1,024 x 512 3.4 / 2.4, 3.6 / 3.0, 3.9 / 3.8; 1,024 x 1,408 4.1 / 2.9, 4.4 / 3.4, 4.9 / 4.2; 2,048 x
+    2,048 4.5 / 3.5, 4.9 / 3.9, 5.5 / 4.7; 4,096 x 512 3.6 / 3.3, 3.9 / 3.6, 4.2 / 4.2; 8,192 x 1,024 5.6 / 5.3, 6.2 / 5.6, 6.5 / 6.1; 2,048 x 5,632 9.2 /
+    6.1, 8.9 / 7.4, 11.0 / 10.0; with an activation the same; steps: Natenex sizes 8 tokens 643 / 632, 16 tokens 800 / 770, Puladra layers of 1,024
+    columns 1 token 1,063 / 969, Nusilix layers of 2,048 columns 12 tokens 518 / 495).  From 16,384 columns on and where K is no multiple of 32
+    the decode-batch kernel stays."""
+    return (dtype == torch.bfloat16 and w_tiled is not None and n <= 16 and k % 32 == 0 and m < 16384
+            and _rows_options(rt, n, k, False, w_tiled))
+
+
 def decode_linear(ctx, x, w, tag, w_tiled=None, unary=None):
     """``linear`` for a consumer that takes float32 sums either whole or in slices: ``K.linear_rows`` where it is the
-    faster (``parts_rows``); else decode
+    faster (``parts_rows``, ``_unstaged``); else decode
     batches of up to 16 rows run on the decode-batch kernel with all of K in a workgroup (one
     result, from the tiled copy of w where there is one); everything else as ``linear`` cuts it.
     ``unary`` = (activation without a gate, its constants): only where ``decode_batch_fits`` or ``parts_rows``;
@@ -402,14 +416,12 @@ def decode_linear(ctx, x, w, tag, w_tiled=None, unary=None):
         K.linear_rows(w_tiled or w, y, K.LINEAR_PARTS, x, unary=unary)
         return y if unary is not None else y[0]
     if decode_batch_fits(rt, x, m, w_tiled is not None) and not rt.options.get("no_fused_linear") and rt.options.get("gemm_algo") is None:
-        tiles = 4 if m >= 16384 else 1
-        if unary is not None:
-            y = ctx.buf(tag, (n, m), x.dtype)
-            K.fused_linear(w_tiled if w_tiled is not None else w, y, K.LINEAR_PARTS, x=x, tiles_per_wg=tiles, unary=unary)
-            return y
-        y = ctx.buf(tag, (1, n, m), torch.float32)
-        K.fused_linear(w_tiled if w_tiled is not None else w, y, K.LINEAR_PARTS, x=x, tiles_per_wg=tiles)
-        return y[0]
+        y = ctx.buf(tag, (n, m) if unary is not None else (1, n, m), x.dtype if unary is not None else torch.float32)
+        if _unstaged(rt, n, m, w.shape[1], x.dtype, w_tiled):
+            K.linear_rows(w_tiled, y, K.LINEAR_PARTS, x, unary=unary)
+        else:
+            K.fused_linear(w_tiled if w_tiled is not None else w, y, K.LINEAR_PARTS, x=x, tiles_per_wg=4 if m >= 16384 else 1, unary=unary)
+        return y if unary is not None else y[0]
     if unary is not None:
         raise ValueError("decode_linear: the activation goes with the decode-batch kernel only")
     return linear(ctx, x, w, tag)

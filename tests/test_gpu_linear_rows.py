@@ -289,3 +289,27 @@ def test_float32(n, m, k):
     assert torch.equal(q2, q)
     want_q = P.rope((want_n @ wq.double().T).cpu(), pos.cpu().tolist(), H, hd, 10000.0)
     assert (q.cpu().double() - want_q).abs().max() < 1e-5 * (want_q.abs().max() + 1)
+
+
+@pytest.mark.parametrize("m,k", [(16, 32), (100, 64), (513, 512), (2048, 2048), (1030, 1056), (16383, 96)])
+def test_plain_sums_of_a_decode_batch_by_either_kernel(m, k):
+    """``decode_linear`` up to 16 rows from the tiled copy, rows apart by more than K among them: against the decode-batch kernel
+    (the option that keeps products from the library leaves it that one) and the product in 64 bits.  A sum's error is at most K
+    units of the 32-bit rounding of the sum of magnitudes, either way; an activation rounds to bfloat16 behind it."""
+    from types import SimpleNamespace
+    from kllm_amd.parts import linear as products
+    k_ = K()
+    ctx = [SimpleNamespace(runtime=SimpleNamespace(options=o, dtype=torch.bfloat16),
+                           buf=lambda tag, shape, dtype: torch.full(shape, float("nan"), dtype=dtype, device=DEV)) for o in ({}, {"gemm": "library"})]
+    w = _bf(m, k, seed=3, scale=0.1)
+    tiled = k_.fused_linear_tile(w, k_.LINEAR_PARTS)
+    for n in (1, 2, 8, 9, 15, 16):
+        for x in (_bf(n, k, seed=n, scale=1.0), _bf(n, k + 40, seed=n, scale=1.0)[:, 8:k + 8]):
+            assert products._unstaged(ctx[0].runtime, n, m, k, x.dtype, tiled) and not products._unstaged(ctx[1].runtime, n, m, k, x.dtype, tiled)
+            ref = x.double() @ w.double().T
+            bound = k * 2.0 ** -23 * (x.double().abs() @ w.double().abs().T)
+            for c in ctx:
+                assert ((products.decode_linear(c, x, w, "y", tiled).double() - ref).abs() <= bound).all(), (n, x.stride(0))
+                h = products.decode_linear(c, x, w, "h", tiled, unary=(k_.ACT_RELU_SQ, None)).double()
+                want = ref.clamp_min(0) ** 2
+                assert ((h - want).abs() <= 2.0 ** -8 * want + (2 * ref.abs() + bound) * bound * 1.01).all(), (n, x.stride(0))
