@@ -1,5 +1,6 @@
 // Float32 attention over the paged cache on the matrix cores, for prompts and
-// for decode tokens: one kernel, two ways of filling its 32 columns.
+// for decode tokens: one kernel, two ways of filling its 32 columns, and behind it one of 16 columns
+// that most decode tokens run on.
 //
 // Operands, products and sums are 32-bit throughout (MFMA 32x32x2 with float32
 // inputs; expf; no reduced precision anywhere).  Formulas as in the generic
@@ -390,6 +391,247 @@ __global__ __launch_bounds__(64 * kF32Waves) void attn_f32_mfma_kernel(const Att
   }
 }
 
+// ---- Decode tokens with up to 16 query heads to a KV head, head sizes 32, 64, 96 and 128 and pages of a multiple of 16 slots:
+// one wave takes one slice of the keys for the group's heads as 16 columns (MFMA 16x16x4: A[c][g], B[g][c], D[4g + i][c] for lane
+// l, g = l / 16, c = l % 16), which is half the matrix instructions that 32 columns take.  Formulas and precision as above.
+//   scores  A = key row c, floats 16kk + 4g ... + 3 of head_dim, one 16-byte read for four instructions; B = the same floats of
+//           column c's query, in registers.  Row c of the u-th of two is key 8 (c / 4) + 4u + c % 4 of a tile of 32: the lane then holds
+//           the scores of keys 8g ... 8g + 7.
+//   values  A = values [head_dim row 16r + c][keys 8g ... 8g + 7], two 16-byte reads for eight instructions.
+// What bounds it: up to a few tiles a wave, three trips to memory in a row (position and span; all pages of the wave's tiles, a half of a tile to a
+// lane; keys and values) and the matrix instructions of its tiles; at many tokens the cache's bytes.  So the arguments come with the
+// launch (the first eight), nothing goes through LDS before the merge, the sums are rescaled only where a maximum moved, and the slices are
+// cut over the waves of the workgroups that a launch has, without 64-bit divisions.  us in a step, 32 columns before and 16 now: 8 tokens
+// at 1,400 keys, 4 KV heads of 64 16.0 -> 9.1, of which the multiplications of two tiles are 1.7 (on 32 columns 3.4); steps of 1.1B Llama sizes, 1 / 8 / 16 / 32 tokens
+// 1,394 / 1,502 / 1,701 / 2,860 -> 1,271 / 1,350 / 1,551 / 2,663, of 7B (2 tokens) 5,910 -> 5,665, of 8B (4) 6,470 -> 6,220.
+// An exponential is exp2 of the difference to the maximum times log2(e): the product's rounding, |x| 2^-24 for exp(x), x <= 0, weighs at most
+// x exp(x) < 0.4 of that in a sum.
+template <int HDT>   // head_dim = 16 * HDT
+__global__ __launch_bounds__(64 * kF32Waves) __attribute__((amdgpu_waves_per_eu(HDT <= 4 ? 2 : 1))) void attn_f32_decode_kernel(
+    const float* __restrict__ cache, const int* __restrict__ positions, const int* __restrict__ span_of_token, const int* __restrict__ block_table,
+    const int* __restrict__ token_list, const float* __restrict__ q, int max_pages, int KV, float* __restrict__ out, float* __restrict__ part, int H, int G,
+    int page16, int wgs, unsigned page_magic, unsigned slice_magic, int window, int chunk, const float* __restrict__ sinks, float scale,
+    const float* __restrict__ slopes, const OutGate gate) {
+  constexpr int hd = 16 * HDT;
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int g = lane / 16, c = lane % 16;
+  int at = blockIdx.x;                                       // (vector loads: scalar ones come one behind the other)
+  asm volatile("" : "+v"(at));
+  if (token_list) at = token_list[at];
+  const int pos_v = positions[at], span_v = span_of_token[at];
+  asm volatile("" ::"s"(H), "s"(G), "s"(page16), "s"(wgs), "s"(page_magic), "s"(slice_magic), "s"(window), "s"(chunk), "s"(sinks), "s"(scale),
+               "s"(slopes), "s"(out), "s"(part), "s"(gate.sums));
+  const int t = __builtin_amdgcn_readfirstlane(at), page_size = 16 * page16, kvh = blockIdx.y;
+  const int nslices = wgs * kF32Waves, slice = blockIdx.z * kF32Waves + wave;
+  const bool head_ok = c < G;
+  const int head = kvh * G + (head_ok ? c : 0);              // (a column without a head computes another's, and nothing comes of it)
+  const float slope = slopes ? slopes[head] : 0.f;
+  floatx4 qb[HDT];
+#pragma unroll
+  for (int kk = 0; kk < HDT; ++kk) qb[kk] = *reinterpret_cast<const floatx4*>(q + ((long)t * H + head) * hd + 16 * kk + 4 * g);
+
+  const int len = __builtin_amdgcn_readfirstlane(pos_v) + 1, span = __builtin_amdgcn_readfirstlane(span_v);
+  const int start = first_key(len - 1, window, chunk), first = start & ~31;
+  const int tiles = (len - first + 31) / 32;
+  unsigned left;
+  const int per = (int)divided((unsigned)(tiles + nslices - 1), (unsigned)nslices, slice_magic, left);
+  const int tile0 = slice * per, tile1 = min(tile0 + per, tiles);
+  const int* table = block_table + (long)span * max_pages;
+  const long block = (long)page_size * hd;
+
+  // A sink is where the running maximum and sum of the first slice start; one of a column's four lanes holds its term, 1.
+  const bool owns_sink = sinks && slice == 0;
+  float m = owns_sink ? sinks[head] : -INFINITY, l = (owns_sink && g == 0) ? 1.f : 0.f;
+  floatx4 acc[HDT];
+#pragma unroll
+  for (int r = 0; r < HDT; ++r) acc[r] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  struct Tile {
+    floatx4 k[2][HDT], v[HDT][2];
+    unsigned mask;             // which of its keys are read (0: there is no such tile)
+  };
+  auto bits = [](int lo, int hi) -> unsigned {               // lo ... hi - 1 of 32 (lo < hi)
+    return (~0u >> (32 - min(max(hi, 1), 32))) & (~0u << min(max(lo, 0), 31));
+  };
+  // Where the 64 halves (16 keys, of one page) of 32 tiles from b0 on lie, a half to a lane.  One that is not read (its page may be
+  // gone) reads page 0, whose keys and values nothing comes of.
+  struct Places {
+    unsigned mask;
+    int slot;
+    long base;               // floats from the cache's first to the page's keys of this head
+  };
+  auto lookup = [&](int b0) -> Places {
+    Places P;
+    const int tile = b0 + lane / 2, kb = first + tile * 32;
+    P.mask = tile < tile1 ? bits(start - kb, len - kb) : 0u;
+    const bool live = (P.mask >> (16 * (lane % 2))) & 0xFFFFu;
+    unsigned left;
+    const int index = (int)divided(live ? (unsigned)kb / 16 + lane % 2 : 0u, (unsigned)page16, page_magic, left);
+    const int page = table[index];
+    P.slot = (int)left * 16;
+    P.base = ((long)(live ? page : 0) * 2 * KV + kvh) * block;
+    return P;
+  };
+  const int k_lane = (8 * (c / 4 % 2) + c % 4) * hd + 4 * g;             // floats of this lane in a half's keys
+  const int v_lane = c * page_size + 8 * (g % 2);                        // ... and in a page's values
+  auto fetch = [&](const Places& P, int i) -> Tile {         // the i-th of those tiles
+    Tile T;
+    T.mask = __builtin_amdgcn_readlane(P.mask, 2 * i);
+    const float* kp[2];
+    const float* vp[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const unsigned lo = __builtin_amdgcn_readlane((int)P.base, 2 * i + h);
+      const long base = (long)((unsigned long)(unsigned)__builtin_amdgcn_readlane((int)(P.base >> 32), 2 * i + h) << 32 | lo);
+      const int slot = __builtin_amdgcn_readlane(P.slot, 2 * i + h);
+      kp[h] = cache + base + slot * hd;
+      vp[h] = cache + base + KV * block + slot;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const float* kl = (c < 8 ? kp[0] : kp[1]) + k_lane;
+    const float* vl = (g < 2 ? vp[0] : vp[1]) + v_lane;
+#pragma unroll
+    for (int kk = 0; kk < HDT; ++kk)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) T.k[u][kk] = *reinterpret_cast<const floatx4*>(kl + 4 * u * hd + 16 * kk);
+    __builtin_amdgcn_sched_barrier(0);     // (keys first: the scores wait for no values)
+#pragma unroll
+    for (int r = 0; r < HDT; ++r)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) T.v[r][h] = *reinterpret_cast<const floatx4*>(vl + (long)r * 16 * page_size + 4 * h);
+    __builtin_amdgcn_sched_barrier(0);
+    return T;
+  };
+  auto compute = [&](Tile& T, int tile) {
+    floatx4 s[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int kk = 0; kk < HDT; ++kk)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) s[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(T.k[u][kk][e], qb[kk][e], s[u], 0, 0, 0);
+    float sc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sc[e] = s[e / 4][e % 4] * scale;
+    if (slopes) {
+      const int far = len - 1 - (first + tile * 32) - 8 * g;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sc[e] -= slope * (float)(far - e);
+    }
+    if (T.mask != ~0u) {                                     // first and last tiles: what is not read may hold anything
+      const unsigned mine = T.mask >> (8 * g);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const bool ok = (mine >> e) & 1u;
+        sc[e] = ok ? sc[e] : -INFINITY;
+#pragma unroll
+        for (int r = 0; r < HDT; ++r) T.v[r][e / 4][e % 4] = ok ? T.v[r][e / 4][e % 4] : 0.f;
+      }
+    }
+    float tmax = sc[0];
+#pragma unroll
+    for (int e = 1; e < 8; ++e) tmax = fmaxf(tmax, sc[e]);
+    const float m_new = fmaxf(m, group4_max(tmax));
+    const float mref = m_new == -INFINITY ? 0.f : m_new;     // scores may have overflowed
+    const float alpha = __builtin_amdgcn_exp2f((m - mref) * kLog2E);
+    float psum = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      sc[e] = __builtin_amdgcn_exp2f((sc[e] - mref) * kLog2E);
+      psum += sc[e];
+    }
+    l = l * alpha + psum;
+    if (__builtin_amdgcn_ballot_w64(m_new > m)) {            // (after a few tiles the maximum rarely moves)
+#pragma unroll
+      for (int r = 0; r < HDT; ++r) acc[r] *= alpha;
+    }
+    m = m_new;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int r = 0; r < HDT; ++r) acc[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(T.v[r][e / 4][e % 4], sc[e], acc[r], 0, 0, 0);
+  };
+  // While a tile is multiplied the next one's operands are on their way, in two buffers by name.  Beyond the wave's last tile that
+  // one is asked for again.
+  for (int b0 = tile0; b0 < tile1; b0 += 32) {
+    const Places P = lookup(b0);
+    const int n = min(tile1 - b0, 32);
+    Tile A = fetch(P, 0), B;
+    if (n == 1) {            // (short contexts: nothing is asked for that is not read)
+      compute(A, b0);
+      break;
+    }
+#pragma unroll 1
+    for (int i = 0; i < n; i += 2) {
+      B = fetch(P, min(i + 1, n - 1));
+      compute(A, b0 + i);
+      A = fetch(P, min(i + 2, n - 1));
+      if (i + 1 < n) compute(B, b0 + i + 1);
+    }
+  }
+  l = group4_sum(l);
+
+  // ---- the waves' results meet in LDS; a thread merges, in the order of the waves, four elements of one head: the output itself
+  // where this workgroup had all the keys, else the workgroup's partial result
+  extern __shared__ __attribute__((aligned(16))) float red[];   // [waves][G][hd + 4]
+  constexpr int RS = hd + 4;
+  if (head_ok) {
+    float* mine = red + (wave * G + c) * RS;
+#pragma unroll
+    for (int r = 0; r < HDT; ++r) *reinterpret_cast<floatx4*>(mine + 16 * r + 4 * g) = acc[r];
+    if (g == 0) {
+      mine[hd] = m;                                          // -inf and 0 for a slice without keys
+      mine[hd + 1] = l;
+    }
+  }
+  __syncthreads();
+  constexpr int CH = hd / 4;
+  for (int idx = threadIdx.x; idx < G * CH; idx += 64 * kF32Waves) {
+    const int hc = idx / CH, d4 = (idx % CH) * 4;
+    const float* col = red + hc * RS;
+    float mj[kF32Waves], M = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < kF32Waves; ++j) {
+      mj[j] = col[j * G * RS + hd];
+      M = fmaxf(M, mj[j]);
+    }
+    floatx4 v = {0.f, 0.f, 0.f, 0.f};
+    float L = 0.f;
+#pragma unroll
+    for (int j = 0; j < kF32Waves; ++j) {
+      const float* w = col + j * G * RS;
+      const float wj = M != -INFINITY ? __builtin_amdgcn_exp2f((mj[j] - M) * kLog2E) : 0.f;
+      L += wj * w[hd + 1];
+      v += wj * *reinterpret_cast<const floatx4*>(w + d4);
+    }
+    const long row = (long)t * H + kvh * G + hc;
+    if (wgs == 1) {
+      const floatx4 og = out_gate4(gate, t, kvh * G + hc, d4);
+      const float inv = 1.f / L;                             // finite: a column reads its own key
+      floatx4 o;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] = v[j] * inv * og[j];
+      *reinterpret_cast<floatx4*>(out + row * hd + d4) = o;
+    } else {
+      float* prow = part + (row * wgs + blockIdx.z) * (hd + 2);   // 8-byte rows
+      *reinterpret_cast<floatx2*>(prow + d4) = floatx2{v[0], v[1]};
+      *reinterpret_cast<floatx2*>(prow + d4 + 2) = floatx2{v[2], v[3]};
+      if (d4 == 0) *reinterpret_cast<floatx2*>(prow + hd) = floatx2{M, L};
+    }
+  }
+}
+
+template <int HDT>
+static void launch_f32_decode(const AttnF32Args& a, int wgs, hipStream_t stream) {
+  const int G = a.H / a.KV;
+  const unsigned page16 = a.page_size / 16, slices = wgs * kF32Waves;
+  const unsigned page_magic = page16 == 1 ? 0xFFFFFFFFu : (unsigned)((1ull << 32) / page16), slice_magic = (unsigned)((1ull << 32) / slices);
+  hipLaunchKernelGGL(attn_f32_decode_kernel<HDT>, dim3(a.count, a.KV, wgs), dim3(64 * kF32Waves),
+                     (size_t)kF32Waves * G * (16 * HDT + 4) * sizeof(float), stream, a.cache, a.positions, a.span_of_token, a.block_table, a.token_list,
+                     a.q, a.max_pages, a.KV, a.out, a.part, a.H, G, (int)page16, wgs, page_magic, slice_magic, a.window, a.chunk, a.sinks, a.scale,
+                     a.slopes, a.gate);
+}
+
 template <int HDT, bool DECODE>
 static int launch_f32(const AttnF32Args& a, long items, hipStream_t stream) {
   const size_t lds = (size_t)kF32Waves * 32 * (a.hd + 4) * sizeof(float);
@@ -424,15 +666,17 @@ bool attn_f32_fits(int hd, int page_size) {
 extern "C" int kllm_attn_f32_fits(int hd, int page_size) { return attn_f32_fits(hd, page_size) ? 1 : 0; }
 
 int attn_f32_slices(int n, int KV, int H, int hd, int max_keys) {
-  // About four waves per CU across the chip (eight from one group per CU on, where partial
-  // results cost little beside the keys), shared out over tokens x KV heads x blocks of 32
-  // heads; a slice is one wave and should have 32 keys at least (measured: 64 tokens at 2,048
-  // keys 61 us with 8 slices against 68 with 4; one token at 32,768 keys 47 us with 256 against
-  // 69 with 64; 8 tokens at 512 keys 13 us with 16 against 15 with 32).
+  // About four waves per CU across the chip, shared out over tokens x KV heads x blocks of 32 heads; a slice is one wave and should have
+  // 32 keys at least (one token at 32,768 keys 47 us with 256 against 69 with 64, on 32 columns; on 16, in us with the merge in a replayed graph:
+  // 8 tokens x 4 KV heads of 64 at 1,000 keys 17.1 / 13.0 / 10.0 / 7.5 / 7.9 with 4 / 8 / 16 / 32 / 64; 16 x 8 of 128 41.6 / 30.9 / 37.3 / 35.2 / 40.1).
+  // From one group per CU on eight on 32 columns (64 tokens at 2,048 keys 61 us with 8 slices against 68 with 4) and on 16 the four of one workgroup,
+  // which leave nothing to merge (4 / 8 slices: 64 tokens x 4 KV heads of 64 at 1,000 keys 24.2 / 28.2, at 256 8.5 / 9.8; 8 x 32 of 128 at 1,000 50.2 / 57.4,
+  // at 256 20.4 / 19.4).
   const int col_blocks = (H / KV + 31) / 32;
   const long groups = (long)n * KV * col_blocks;
   const int cus = device_cus();
   long want = (groups >= cus ? 8L : 4L) * cus / (groups > 0 ? groups : 1);
+  if (groups >= cus && H / KV <= 16 && hd % 32 == 0 && hd <= 128 && want > kF32Waves) want = kF32Waves;
   long most = max_keys > 0 ? max_keys / 32 : 64;
   if (most > kAttnF32MaxSlices) most = kAttnF32MaxSlices;
   // Up to 128 keys (a tile of 32 a wave) the second kernel costs more than the keys: one workgroup's four
@@ -466,6 +710,21 @@ int attn_f32_decode(const float* q, float* out, float* part, const float* cache,
   a.block_table = block_table; a.count = count;
   a.max_pages = max_pages; a.page_size = page_size; a.H = H; a.KV = KV; a.hd = hd; a.window = window; a.chunk = chunk; a.sinks = sinks; a.gate = gate;
   a.scale = scale; a.slopes = slopes; a.nslices = nslices; a.col_blocks = (H / KV + 31) / 32;
+  // The kernel of 16 columns takes a workgroup's four slices at a time, whatever their number (no more partial results than
+  // the slices that ``part`` has room for).
+  const int wgs = (nslices + kF32Waves - 1) / kF32Waves;
+  if (H / KV <= 16 && hd % 32 == 0 && hd <= 128 && page_size % 16 == 0 && KV <= 65535) {
+    if (hd == 32) launch_f32_decode<2>(a, wgs, stream);
+    else if (hd == 64) launch_f32_decode<4>(a, wgs, stream);
+    else if (hd == 96) launch_f32_decode<6>(a, wgs, stream);
+    else launch_f32_decode<8>(a, wgs, stream);
+    KLLM_CHECK_LAUNCH("attn_decode float32");
+    if (wgs > 1) {
+      launch_attn_merge<float>(out, part, count, H, hd, wgs, token_list, gate, stream);
+      KLLM_CHECK_LAUNCH("attn_merge float32");
+    }
+    return 0;
+  }
   a.wg_merge = nslices % kF32Waves == 0;
   const long items = (long)count * KV * a.col_blocks * nslices;
   if (int rc = dispatch_f32<true>(a, items, stream)) return rc;

@@ -1622,3 +1622,16 @@ def test_sample_frequencies_follow_softmax():
     want = [1 / 8, 2 / 8, 5 / 8]
     chi2 = sum((counts[k] - n * want[k]) ** 2 / (n * want[k]) for k in range(3))
     assert chi2 < 13.8 and counts[3] == 0
+
+
+@pytest.mark.parametrize("H,KV,hd,ps", [(2, 1, 64, 16), (16, 1, 32, 48), (1, 1, 128, 80), (6, 2, 96, 112), (32, 4, 64, 16), (17, 1, 64, 16), (2, 1, 64, 20)])
+@pytest.mark.parametrize("window", [0, 333])
+def test_attention_decode_places_float32(H, KV, hd, ps, window):
+    """As ``test_attention_decode_places``: sixteen heads as columns and, beside it, what stays on thirty-two (17 heads; pages of 20 slots).
+    All is 32-bit: a score's rounding is hd 2^-24 of the sum of its magnitudes, and weights and sums add less than that over thousands of keys."""
+    for spans, slices in (([(8449, 1), (9199, 1)], (1, 3)), ([(0, 1), (30, 1), (31, 1), (47, 1), (95, 1), (511, 1), (1055, 1), (2047, 1)], (1, 3, 4, 6, 16))):
+        c = attention_case(H, KV, hd, ps, torch.float32, window, spans, seed=3)
+        for ns in slices:
+            out = run_attention("decode", c["q"], c["cache"], c["pos"], c["sot"], c["bt"], ps, H, KV, hd, window, c["scale"], nslices=ns)
+            err = (out.cpu().double() - c["want"]).abs().max()
+            assert torch.isfinite(out).all() and err < 2e-5, (ns, float(err))
