@@ -722,17 +722,19 @@ constexpr int kGateChunk = 1024;              // inputs of a block that LDS hold
 // the matrices' way from memory bounds the time, and it needs workgroups (16 channels each) and short
 // chains; a prompt has tiles enough and is bound by its products.
 // 1,500 tokens x 2,048 channels in blocks of 256: 140 -> 63 us (FMA on eight tokens at a time, 790 MB of matrices
-// through L2); 8 tokens: 18 -> 11 us, in a step, where the matrices come from memory, 28.8 -> 16.9 (32 workgroups then, 128 now) -> 14.0.
+// through L2) -> 56; 8 tokens: 18 -> 11 us, in a step, where the matrices come from memory, 28.8 -> 16.9 (32 workgroups then, 128 now) -> 14.0 -> 10.0: a
+// run's inputs are now asked for together whatever the number of the projection's slices (a loop over them for every input waited eleven
+// times), the tokens' spans, the gates' constants and the matrices in one go before anything is waited for, and the arguments they need
+// come with the launch.
 // TAPS: the convolution's where it is 4, 8 for any number up to 8, 0 for more.  ONE: a block's inputs fit into LDS at
 // once; the sums then begin behind the convolution and take no registers in it (72 instead of 89, three workgroups a CU).
 template <int NT, int KS, int OW, int TAPS, bool ONE>
 __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel(
-    const float* __restrict__ proj, int nsplit, long split_stride, const float* __restrict__ x_bias,
-    const float* __restrict__ conv_w, const float* __restrict__ conv_b, int taps, const float* __restrict__ state,
-    long slot_stride, const float* __restrict__ wr_t, const float* __restrict__ wi_t, const float* __restrict__ br,
-    const float* __restrict__ bi, const float* __restrict__ rate, const int* __restrict__ span_of_token,
-    const int* __restrict__ slots, const int* __restrict__ span_start, const int* __restrict__ span_pos,
-    float* __restrict__ a_out, float* __restrict__ b_out, int n, int W, int bs) {
+    const int* __restrict__ span_of_token, const int* __restrict__ span_start, const int* __restrict__ slots, const int* __restrict__ span_pos,
+    const float* __restrict__ proj, int n, int W, int bs, int taps, const float* __restrict__ conv_w, const float* __restrict__ conv_b,
+    int nsplit, const float* __restrict__ x_bias, const float* __restrict__ wr_t, const float* __restrict__ wi_t, long split_stride,
+    const float* __restrict__ state, long slot_stride, const float* __restrict__ br, const float* __restrict__ bi, const float* __restrict__ rate,
+    float* __restrict__ a_out, float* __restrict__ b_out) {
   constexpr int TT = NT * kGateTile, THREADS = kWave * KS * OW;
   extern __shared__ __attribute__((aligned(16))) float us[];
   const int b = blockIdx.y, tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
@@ -765,13 +767,23 @@ __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel
   constexpr int CHAIN = 4;                    // steps of a chain
   constexpr int AHEAD = KS > 1 ? CHAIN : 1;   // steps asked for ahead
   __shared__ int4 spans[TT];                  // the tokens' spans
-  if (tid < nt) {
-    const int span = span_of_token[tfirst + tid];
-    spans[tid] = int4{span_start[span], slots[span], span_pos[span] == 0, 0};
+  // A decode batch asks for the tokens' spans first and, before it waits for them, for all that needs none of them.
+  constexpr bool AT_ONCE = KS > 1 && TAPS > 1;
+  const int span = span_of_token[tfirst + min(tid, nt - 1)];
+  float rb = 0.f, ib = 0.f, rt = 0.f;
+  auto constants = [&] {
+    const int c = b * bs + oc;
+    rb = br[c], ib = bi[c], rt = rate[c];
+  };
+  if (AT_ONCE) {
+    asm volatile("" ::"s"(conv_w), "s"(conv_b), "s"(nsplit), "s"(x_bias), "s"(wr_t), "s"(wi_t), "s"(state), "s"(slot_stride), "s"(br), "s"(bi),
+                 "s"(rate), "s"(a_out), "s"(b_out));
+    constants();
   }
+  const int4 mine = int4{span_start[span], slots[span], span_pos[span] == 0, 0};
   int k0 = 0;
   do {
-    __syncthreads();
+    if (!ONE && k0 > 0) __syncthreads();
     const int steps = (min(chunk, bs - k0) + 15) / 16;
     const int per = (steps + KS - 1) / KS, s0 = ks * per, s1 = min(steps, s0 + per);
     // The first of this wave's share of the matrices: a decode batch's whole chain (they come from memory, and nothing
@@ -780,6 +792,10 @@ __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel
 #pragma unroll
     for (int i = 0; i < AHEAD; ++i)
       if (KS > 1) w[i] = fetch(k0 + 16 * min(s0 + i, steps - 1));
+    if (k0 == 0) {
+      if (tid < nt) spans[tid] = mine;
+      __syncthreads();
+    }
     if (TAPS > 0 && (nt > 1 || KS > 1)) {
       // A thread takes a channel for a run of RUN tokens and asks for the run's inputs at once, each
       // for all the taps it meets, instead of for every tap of every token on its own.
@@ -789,55 +805,64 @@ __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel
         const int r = i / chunk, e = k0 + i - r * chunk, c = b * bs + e, tt0 = r * RUN;
         const bool there = e < bs && tt0 < nt;
         float x[RUN + MOST - 1], wt[MOST];
+        const int cc = min(c, W - 1);
         if (there) {
+          auto row_at = [&](int q) { return proj + (long)min(max((int)tfirst + tt0 - K + q, 0), n - 1) * cols + W + cc; };
 #pragma unroll
           for (int q = 0; q < RUN + MOST - 1; ++q) {        // (rows that are not there: some row that is, not used)
             if (q >= RUN + K) break;
-            const long row = min(max(tfirst + tt0 - K + q, 0L), (long)n - 1);
-            x[q] = conv_input(proj, nsplit, split_stride, cols, W + c, x_bias - W, row);
+            x[q] = *row_at(q);
           }
 #pragma unroll
           for (int j = 0; j < MOST; ++j) wt[j] = conv_w[(long)c * taps + min(j, K)];
+          for (int sp = 1; sp < nsplit; ++sp)
+#pragma unroll
+            for (int q = 0; q < RUN + MOST - 1; ++q) {
+              if (q >= RUN + K) break;
+              x[q] += row_at(q)[sp * split_stride];
+            }
         }
-        const float cb = there ? conv_b[c] : 0.f;
+        const float cb = there ? conv_b[c] : 0.f, xb = there && x_bias ? x_bias[c] : 0.f;
+        int4 sp[RUN];                                       // first row, slot, whether the span starts at position 0
+#pragma unroll
+        for (int q = 0; q < RUN; ++q) sp[q] = spans[min(tt0 + q, nt - 1)];
         // A decode batch's tokens are spans of their own and find all but one input in the requests' states: a run of
         // tokens with a span's start in it asks for all their entries at once (in a prompt, where such runs are few, one by one: the
-        // entries' registers would cost a workgroup a CU).  8 tokens of 2,048 channels, in a step: 17.5 -> 15.6 us, 14.0 with the matrices asked for ahead.
-        constexpr bool AT_ONCE = KS > 1 && TAPS > 1;
+        // entries' registers would cost a workgroup a CU).
         float st[AT_ONCE ? RUN : 1][AT_ONCE ? TAPS - 1 : 1];
         if constexpr (AT_ONCE) {
           bool starts = false;
 #pragma unroll
-          for (int q = 0; q < RUN; ++q) starts |= there && tt0 + q < nt && tfirst + tt0 + q - K < spans[min(tt0 + q, nt - 1)].x;
-          if (starts) {
+          for (int q = 0; q < RUN; ++q) starts |= (int)tfirst + min(tt0 + q, nt - 1) - K < sp[q].x;
+          if (starts && there) {
 #pragma unroll
             for (int q = 0; q < RUN; ++q) {                 // (tokens that are not there: the last one's, not used)
-              const float* from = state + (long)spans[min(tt0 + q, nt - 1)].y * slot_stride + (long)c * K;
+              const float* from = state + (long)sp[q].y * slot_stride + (long)c * K;
 #pragma unroll
               for (int j = 0; j < TAPS - 1; ++j) st[q][j] = from[min(j, K - 1)];
             }
           }
         }
+        if (x_bias)                                         // the convolution's input carries the projection's bias
+#pragma unroll
+          for (int q = 0; q < RUN + MOST - 1; ++q) x[q] += xb;
 #pragma unroll
         for (int q = 0; q < RUN; ++q) {
           float v = 0.f;
           if (there && tt0 + q < nt) {
-            const long t = tfirst + tt0 + q;
-            const int4 sp = spans[tt0 + q];           // first row, slot, whether the span starts at position 0
+            const int t = (int)tfirst + tt0 + q;
 #pragma unroll
             for (int j = 0; j < MOST; ++j) {
               if (j > K) break;
-              const int back = (int)(t - K + j) - sp.x;      // rows behind the span's first
+              const int back = t - K + j - sp[q].x;         // rows behind the span's first
               float in = x[q + j];
-              if (back < 0) {
-                if constexpr (AT_ONCE) {
-                  in = st[q][0];                      // entry K + back, by choice: the entries stay in registers
+              if constexpr (AT_ONCE) {
+                float was = st[q][0];                       // entry K + back, by choice: the entries stay in registers
 #pragma unroll
-                  for (int i = 1; i < TAPS - 1; ++i) in = i == K + back ? st[q][i] : in;
-                  in = sp.z ? 0.f : in;
-                } else {
-                  in = sp.z ? 0.f : state[(long)sp.y * slot_stride + (long)c * K + K + back];
-                }
+                for (int i = 1; i < TAPS - 1; ++i) was = i == K + back ? st[q][i] : was;
+                in = back < 0 ? (sp[q].z ? 0.f : was) : in;
+              } else if (back < 0) {
+                in = sp[q].z ? 0.f : state[(long)sp[q].y * slot_stride + (long)c * K + K + back];
               }
               v = fmaf(wt[j], in, v);
             }
@@ -921,7 +946,7 @@ __global__ __launch_bounds__(kWave * KS * OW) void linear_recurrence_prep_kernel
   }
   if (o >= bs) return;
   const int c = b * bs + o;
-  const float rb = br[c], ib = bi[c], rt = rate[c];
+  if (!AT_ONCE) constants();
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -955,8 +980,8 @@ static int recurrence_prep_launch_chunks(const float* proj, int nsplit, long spl
   }
   hipLaunchKernelGGL((linear_recurrence_prep_kernel<NT, KS, OW, TAPS, ONE>),
                      dim3(ceil_div(n, NT * kGateTile), blocks, ceil_div(bs, OW * kGateTile)), dim3(kWave * KS * OW), lds,
-                     stream, proj, nsplit, split_stride, x_bias, conv_w, conv_b, taps, state, slot_stride, wr_t, wi_t, br,
-                     bi, rate, span_of_token, slots, span_start, span_pos, a_out, b_out, n, W, bs);
+                     stream, span_of_token, span_start, slots, span_pos, proj, n, W, bs, taps, conv_w, conv_b, nsplit, x_bias, wr_t, wi_t,
+                     split_stride, state, slot_stride, br, bi, rate, a_out, b_out);
   KLLM_CHECK_LAUNCH("linear_recurrence_prep");
   return 0;
 }
