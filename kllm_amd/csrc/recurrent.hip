@@ -237,23 +237,102 @@ constexpr int kDeltaBlock = 16;                              // tokens staged at
 // instead of one per head.
 template <int NB, bool VEC>
 __global__ __launch_bounds__(kRecThreads) void gated_delta_scan_kernel(
-    const float* __restrict__ qn, const float* __restrict__ kn, const float* __restrict__ vv,
-    const float* __restrict__ gb, float* __restrict__ o_out, float* __restrict__ state, long slot_stride,
-    const int* __restrict__ slots, const int* __restrict__ span_start, const int* __restrict__ span_pos, int H, int G,
-    int dk, int dv, const float* __restrict__ dec, const ConvTail tail) {
+    const int* __restrict__ span_start, const int* __restrict__ slots, const int* __restrict__ span_pos, float* __restrict__ state, int H, int G,
+    int dk, int dv, long slot_stride, const float* __restrict__ kn, const float* __restrict__ qn, const float* __restrict__ vv,
+    const float* __restrict__ gb, float* __restrict__ o_out, const float* __restrict__ dec, const ConvTail tail) {
   constexpr int ROW = 64 * NB;                       // a token's row in LDS
   constexpr int NV = VEC ? 3 : 2;                    // vectors of a token: k, q and the decays
   __shared__ __attribute__((aligned(16))) float rows[NV][kDeltaBlock][ROW];
   __shared__ float vs[kDeltaBlock][kDeltaCols], os[kDeltaBlock][kDeltaCols];
   __shared__ __attribute__((aligned(16))) float gs[kDeltaBlock][4];      // g, beta, k . q
-  const int span = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  int at = blockIdx.x;                               // (vector loads: scalar ones come one behind the other)
+  asm volatile("" : "+v"(at));
+  const int first_v = span_start[at], last_v = span_start[at + 1], slot_v = slots[at], pos_v = span_pos[at];
+  asm volatile("" ::"s"(kn), "s"(qn), "s"(vv), "s"(gb), "s"(o_out), "s"(dec), "s"(tail.proj), "s"(tail.split_stride), "s"(tail.cols), "s"(tail.in_bias),
+               "s"(tail.state), "s"(tail.nsplit), "s"(tail.col0), "s"(tail.C), "s"(tail.taps));
+  const int h = blockIdx.y, tid = threadIdx.x;
   const int g = h / (H / G);
   const int jl = tid / kDeltaParts, p = tid % kDeltaParts;
   const int j = blockIdx.z * kDeltaCols + jl;
   const bool col = j < dv;
-  const long t0 = span_start[span], t1 = span_start[span + 1];
-  const bool fresh = span_pos[span] == 0;
-  float* S = state + (long)slots[span] * slot_stride + (long)h * dk * dv;
+  const long t0 = __builtin_amdgcn_readfirstlane(first_v), t1 = __builtin_amdgcn_readfirstlane(last_v);
+  const int slot = __builtin_amdgcn_readfirstlane(slot_v);
+  const bool fresh = __builtin_amdgcn_readfirstlane(pos_v) == 0;
+  float* S = state + (long)slot * slot_stride + (long)h * dk * dv;
+  if (t1 - t0 == 1 && dv % 4 == 0 && (((unsigned long)S | (unsigned long)vv) & 15) == 0) {
+    // One token: the state's way from memory and back is all there is.  A thread takes four columns of every 64th row, 16 bytes a load,
+    // and the sums over the rows go over the wave's sixteen rows by lane exchanges and over the waves through LDS.  8 tokens, 16 heads of
+    // 128 x 128: 13.3 -> 7.2 us (17 MB; 16-byte pieces of four rows a load before, and a chain's staging for one token).
+    const int quad = tid % 4, rr = tid / 4;
+    const int j4 = blockIdx.z * kDeltaCols + 4 * quad, jc = j4 < dv ? j4 : 0;
+    const long key = t0 * G * dk + (long)g * dk, head = t0 * H + h;
+    floatx4 x[NB];
+    float k[NB], q[NB], d[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int r = min(64 * b + rr, dk - 1);
+      k[b] = kn[key + r];
+      q[b] = qn[key + r];
+      d[b] = VEC ? dec[head * dk + r] : 1.f;
+    }
+    const float decay = gb[2 * t0 * H + h], beta = gb[2 * t0 * H + H + h];
+    const floatx4 v = *reinterpret_cast<const floatx4*>(vv + head * dv + jc);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) x[b] = *reinterpret_cast<const floatx4*>(S + (long)min(64 * b + rr, dk - 1) * dv + jc);
+    conv_tail_of_span(tail, slot_stride, slot, t0, t1, fresh);
+    float kq = 0.f, dks[4] = {0.f, 0.f, 0.f, 0.f}, dqs[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const bool row = 64 * b + rr < dk;
+      k[b] = row ? k[b] : 0.f;
+      q[b] = row ? q[b] : 0.f;
+      kq = fmaf(k[b], q[b], kq);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[b][e] = row && !fresh ? x[b][e] * (VEC ? d[b] : decay) : 0.f;
+        dks[e] = fmaf(x[b][e], k[b], dks[e]);
+        dqs[e] = fmaf(x[b][e], q[b], dqs[e]);
+      }
+    }
+    auto over_rows = [](float v) { return group4_sum(dpp_add<0x128>(dpp_add<0x124>(v))); };      // row_ror 4 and 8: lanes of the same quad
+    floatx4(*meet)[4][4] = reinterpret_cast<floatx4(*)[4][4]>(&rows[0][0][0]);      // [wave][quad]: k . S, q . S, k . q
+    floatx4 dk4, dq4;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      dk4[e] = over_rows(dks[e]);
+      dq4[e] = over_rows(dqs[e]);
+    }
+    kq = over_rows(kq);
+    if (tid % kWave < 4) {
+      meet[tid / kWave][quad][0] = dk4;
+      meet[tid / kWave][quad][1] = dq4;
+      meet[tid / kWave][quad][2][0] = kq;
+    }
+    __syncthreads();
+    dk4 = meet[0][quad][0];
+    dq4 = meet[0][quad][1];
+    kq = meet[0][quad][2][0];
+#pragma unroll
+    for (int w = 1; w < kRecThreads / kWave; ++w) {
+      dk4 += meet[w][quad][0];
+      dq4 += meet[w][quad][1];
+      kq += meet[w][quad][2][0];
+    }
+    const floatx4 u = beta * (v - dk4);
+    if (j4 >= dv) return;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      if (64 * b + rr >= dk) break;
+      floatx4 y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = fmaf(k[b], u[e], x[b][e]);
+      *reinterpret_cast<floatx4*>(S + (long)(64 * b + rr) * dv + j4) = y;
+    }
+    if (tid < 4)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o_out[head * dv + j4 + e] = fmaf(kq, u[e], dq4[e]);
+    return;
+  }
   floatx4 s[NB];
 #pragma unroll
   for (int b = 0; b < NB; ++b)
@@ -262,7 +341,7 @@ __global__ __launch_bounds__(kRecThreads) void gated_delta_scan_kernel(
       const int r = 64 * b + 4 * p + e;
       s[b][e] = (col && r < dk && !fresh) ? S[(long)r * dv + j] : 0.f;
     }
-  conv_tail_of_span(tail, slot_stride, slots[span], t0, t1, fresh);
+  conv_tail_of_span(tail, slot_stride, slot, t0, t1, fresh);
   const int QK = G * dk, HV = H * dv;
   // A thread's pieces of a block of tokens: of each vector the elements tid % 64 + 64 i of tokens
   // tid / 64 + 4 q, one of v, one of g and beta.  They are asked for one block ahead and wait in
@@ -1343,11 +1422,11 @@ extern "C" int kllm_gated_delta_scan(const float* qn, const float* kn, const flo
 #define KLLM_GDS(NB)                                                                                                   \
   do {                                                                                                                 \
     if (dec)                                                                                                           \
-      hipLaunchKernelGGL((gated_delta_scan_kernel<NB, true>), grid, dim3(kRecThreads), 0, stream, qn, kn, vv, gb,      \
-                         o_out, state, slot_stride, slots, span_start, span_pos, H, G, dk, dv, dec, tail);             \
+      hipLaunchKernelGGL((gated_delta_scan_kernel<NB, true>), grid, dim3(kRecThreads), 0, stream, span_start, slots,         \
+                         span_pos, state, H, G, dk, dv, slot_stride, kn, qn, vv, gb, o_out, dec, tail);                \
     else                                                                                                               \
-      hipLaunchKernelGGL((gated_delta_scan_kernel<NB, false>), grid, dim3(kRecThreads), 0, stream, qn, kn, vv, gb,     \
-                         o_out, state, slot_stride, slots, span_start, span_pos, H, G, dk, dv, dec, tail);             \
+      hipLaunchKernelGGL((gated_delta_scan_kernel<NB, false>), grid, dim3(kRecThreads), 0, stream, span_start, slots,        \
+                         span_pos, state, H, G, dk, dv, slot_stride, kn, qn, vv, gb, o_out, dec, tail);                \
   } while (0)
   if (nb <= 1) KLLM_GDS(1);
   else if (nb <= 2) KLLM_GDS(2);

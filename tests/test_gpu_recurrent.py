@@ -375,3 +375,63 @@ def test_norm_behind_a_sub_layer_whole_and_odd_rows(d, slices, paired):
     for got, ref in ((xd, want), (out, norm(want) * w2.double())):
         err = (got.double().cpu() - ref).norm() / ref.norm()
         assert err < 1e-6, float(err)
+
+
+@pytest.mark.parametrize("dk,dv", [(8, 24), (64, 16), (65, 20), (128, 40), (136, 16), (200, 8), (256, 36)])
+@pytest.mark.parametrize("per_channel", [False, True])
+def test_delta_scan_of_single_tokens_where_rows_are_whole_pieces(dk, dv, per_channel):
+    """Spans of one token whose state lies on 16 bytes: against the same states four bytes further, which go token by token.  A sum of dk
+    products in another order, and what hangs on it, differs by dk 2^-23 of the magnitudes, here at most a few units."""
+    g = torch.Generator().manual_seed(dk * dv)
+    n, H, G = 5, 4, 2
+    unit = lambda t: (t / t.norm(dim=-1, keepdim=True)).view(n, -1).to(DEV).contiguous()
+    k, q = (unit(torch.randn(n, G, dk, generator=g)) for _ in range(2))
+    v, dec = torch.randn(n, H * dv, generator=g).to(DEV), torch.rand(n, H * dk, generator=g).to(DEV)
+    gb = torch.rand(n, 2, H, generator=g).to(DEV)
+    fill = torch.randn(n + 1, H * dk * dv, generator=g).to(DEV)
+    _, _, span_start, span_pos, slots = spans_of([1] * n, [0, 1, 0, 0, 1])
+    got = {}
+    for at in (4, 5):
+        state = torch.zeros(n + 1, 8 + H * dk * dv, device=DEV)
+        state[:, at:at + H * dk * dv] = fill
+        out = torch.full((n, H * dv), float("nan"), device=DEV)
+        K().gated_delta_scan(q, k, v, gb, out, state, at, slots, span_start, span_pos, n, H, G, dk, dv, dec if per_channel else None)
+        assert not state[:, :at].any() and not state[:, at + H * dk * dv:].any()
+        got[at] = out, state[:, at:at + H * dk * dv]
+    for one, other in zip(got[4], got[5]):
+        assert (one - other).abs().max() <= dk * 2.0 ** -23 * 8
+
+
+@pytest.mark.parametrize("dk,dv", [(64, 128), (128, 130), (200, 40), (256, 300)])
+@pytest.mark.parametrize("taps", [1, 4, 5])
+@pytest.mark.parametrize("nsplit", [1, 3])
+def test_delta_preparation(dk, dv, taps, nsplit):
+    """Convolution, SiLU and unit norms against 64 bits: spans that begin inside a token's window, behind earlier tokens and at position 0;
+    heads of one, of two and of more than two channels a lane."""
+    g = torch.Generator().manual_seed(dk + taps)
+    lens, fresh, H, G = [1, 1, 2, 5, 1], [0, 1, 0, 1, 0], 2, 1
+    n, QK, HV = sum(lens), G * dk, H * dv
+    C = 2 * QK + HV
+    start, token, span_start, span_pos, slots = spans_of(lens, fresh)
+    proj = torch.randn(nsplit, n, C + 2 * H + HV + 3, generator=g)
+    w, a_log, dt = torch.randn(C, taps, generator=g), torch.randn(H, generator=g), torch.randn(H, generator=g)
+    state = torch.randn(len(lens) + 1, 3 + C * (taps - 1), generator=g)
+    f = lambda t: t.to(DEV).contiguous()
+    qn, kn, vv, gate = (torch.full((n, m), float("nan"), device=DEV) for m in (QK, QK, HV, HV))
+    gb = torch.full((n, 2, H), float("nan"), device=DEV)
+    K().gated_delta_prep(f(proj), f(w), taps, f(state), 3, f(a_log), f(dt), token, slots, span_start, span_pos, qn, kn, vv, gb, gate, H, G, dk, dv)
+    x = proj.double().sum(0)
+    y = torch.zeros(n, C, dtype=F64)
+    for s in range(len(lens)):
+        before = state[int(slots[s]), 3:].double().view(C, taps - 1).T * (0.0 if fresh[s] else 1.0)
+        rows = torch.cat([before, x[start[s]:start[s + 1], :C]])
+        for t in range(lens[s]):
+            y[start[s] + t] = (rows[t:t + taps] * w.double().T).sum(0)
+    y = torch.nn.functional.silu(y)
+    unit = lambda t: t / (t.view(n, G, dk).norm(dim=-1, keepdim=True).square() + 1e-6).sqrt().expand(n, G, dk).reshape(n, QK)
+    close(qn, unit(y[:, :QK]) * dk ** -0.5)
+    close(kn, unit(y[:, QK:2 * QK]))
+    close(vv, y[:, 2 * QK:])
+    close(gate, torch.nn.functional.silu(x[:, C + 2 * H:C + 2 * H + HV]))
+    close(gb[:, 1], torch.sigmoid(x[:, C:C + H]))
+    close(gb[:, 0], torch.exp(-a_log.double().exp() * torch.nn.functional.softplus(x[:, C + H:C + 2 * H] + dt.double())))
