@@ -696,3 +696,35 @@ def test_the_command_line_programs_take_the_model(folders, tmp_path):
 def test_zz_the_worst_difference_seen():
     print("worst relative difference of logits:", WORST)
     assert all(WORST[d] < TOL[d] for d in WORST)
+
+
+@pytest.mark.parametrize("n,H,d,dr,rank,dv", [(1, 3, 32, 2, 32, 16), (15, 2, 96, 6, 288, 40), (16, 1, 160, 64, 544, 130), (17, 2, 256, 30, 1056, 64),
+                                              (8, 32, 128, 64, 512, 128)])
+@pytest.mark.parametrize("nsplit,by_head", [(1, False), (3, True)])
+def test_products_with_a_heads_own_matrix_of_a_few_tokens(n, H, d, dr, rank, dv, nsplit, by_head):
+    """A decode batch's two products: heads of one to eight steps, with steps asked for that are not there; ranks of less than a round of
+    512, a little more and two; sums in slices.  Against 64 bits; the queries' sums and the outputs are rounded to 2^-9 each."""
+    from kllm_amd import kernels as K
+    g = torch.Generator().manual_seed(n + d)
+    BF = torch.bfloat16
+    q = torch.randn(nsplit, n, H * (d + dr), generator=g)
+    w_uk = (torch.randn(H * d, rank, generator=g) * d ** -0.5).to(BF)
+    ang = torch.rand(n, dr // 2, generator=g) * 6.0
+    out = torch.full((n, H * (rank + dr)), float("nan"), dtype=BF, device="cuda")
+    w_t = w_uk.view(H, d, rank).transpose(1, 2).contiguous().view(H * rank, d)
+    K.latent_query(q.cuda(), w_t.cuda(), ang.cos().cuda(), ang.sin().cuda(), out, H, d, dr, rank, transposed=True)
+    qs = q.double().sum(0).view(n, H, d + dr)
+    got = out.double().cpu().view(n, H, rank + dr)
+    want = torch.einsum("nhi,hir->nhr", qs[..., :d], w_uk.double().view(H, d, rank))
+    assert rel(got[..., :rank], want) < 2.0 ** -7
+    a, b, c, s = qs[..., d:d + dr // 2], qs[..., d + dr // 2:], ang.cos().double()[:, None], ang.sin().double()[:, None]
+    assert rel(got[..., rank:], torch.cat([a * c - b * s, b * c + a * s], -1)) < 2.0 ** -8
+    att, w_uv = torch.randn(n, H * rank, generator=g).to(BF), (torch.randn(H * dv, rank, generator=g) * rank ** -0.5).to(BF)
+    gate = torch.randn(nsplit, n, 7 + (H if by_head else H * dv), generator=g)
+    want = torch.einsum("nhr,hjr->nhj", att.double().view(n, H, rank), w_uv.double().view(H, dv, rank))
+    out = torch.full((n, H * dv), float("nan"), dtype=BF, device="cuda")
+    K.latent_out(att.cuda(), w_uv.cuda(), out, H, dv, rank)
+    assert rel(out.double().cpu().view(n, H, dv), want) < 2.0 ** -8
+    K.latent_out(att.cuda(), w_uv.cuda(), out, H, dv, rank, gate=gate.cuda(), gate_column=7, **({"gate_by_head": True} if by_head else {}))
+    opened = torch.sigmoid(gate.double().sum(0)[:, 7:]).view(n, H, -1)
+    assert rel(out.double().cpu().view(n, H, dv), want * opened) < 2.0 ** -8
