@@ -698,12 +698,12 @@ def test_zz_the_worst_difference_seen():
     assert all(WORST[d] < TOL[d] for d in WORST)
 
 
-@pytest.mark.parametrize("n,H,d,dr,rank,dv", [(1, 3, 32, 2, 32, 16), (15, 2, 96, 6, 288, 40), (16, 1, 160, 64, 544, 130), (17, 2, 256, 30, 1056, 64),
+@pytest.mark.parametrize("n,H,d,dr,rank,dv", [(1, 3, 32, 2, 32, 16), (15, 2, 96, 6, 288, 40), (16, 1, 160, 64, 544, 130), (17, 2, 256, 30, 928, 64),
                                               (8, 32, 128, 64, 512, 128)])
 @pytest.mark.parametrize("nsplit,by_head", [(1, False), (3, True)])
 def test_products_with_a_heads_own_matrix_of_a_few_tokens(n, H, d, dr, rank, dv, nsplit, by_head):
     """A decode batch's two products: heads of one to eight steps, with steps asked for that are not there; ranks of less than a round of
-    512, a little more and two; sums in slices.  Against 64 bits; the queries' sums and the outputs are rounded to 2^-9 each."""
+    512, a little more and nearly two; sums in slices.  Against 64 bits; the queries' sums and the outputs are rounded to 2^-9 each."""
     from kllm_amd import kernels as K
     g = torch.Generator().manual_seed(n + d)
     BF = torch.bfloat16
