@@ -411,6 +411,102 @@ __global__ __launch_bounds__(256) void qkv_norm_append_kernel(
   }
 }
 
+// The same for heads of 32, 64, 128 and 256 in eight elements a lane, four neighbouring pairs (of halves) or, behind what turns, eight
+// that pass through: loads and stores of 16 bytes, L = dk / 8 lanes a head.  As rope_append's: workgroups are numbered so that a run of sixteen
+// neighbouring tokens stays on one XCD, `chunks` workgroups a token take its queries and keys and `vblocks` a run the values of its tokens, 64
+// elements of each with lanes of neighbouring tokens side by side, whose places in a page are neighbours too.
+// Bound by the sums' bytes for a prompt and by trips to memory for a decode batch: everything but the page is asked for at once.
+// 32 + 4 heads of 64 and as many of values, us, a pair a lane before and now: 1,500 tokens 24.3 -> 10.2, 8 tokens 5.3 -> 5.0 (a step of 8 tokens at Natenex sizes
+// 569 -> 563).
+constexpr int kNormRun = 16;
+template <typename T, int L>
+__global__ __launch_bounds__(256) void qkv_norm_append_vec_kernel(
+    const int* __restrict__ positions, const int* __restrict__ span_of_token, const float* __restrict__ qkv, int n, int H, int KV, int dv, int rot,
+    int chunks, int vblocks, int xcds, const float* __restrict__ cos_t, const float* __restrict__ sin_t, int nsplit, int unit_norm, float eps,
+    int max_pages, int page_size, long split_stride, const int* __restrict__ block_table, const float* __restrict__ bias,
+    const float* __restrict__ q_weight, const float* __restrict__ k_weight, T* __restrict__ q_out, T* __restrict__ cache) {
+  typedef T tx4 __attribute__((ext_vector_type(4)));
+  constexpr int dk = 8 * L;
+  const int xcd = blockIdx.x % xcds, seq = blockIdx.x / xcds, per_run = kNormRun * chunks + vblocks, at = seq % per_run;
+  const int t0 = (seq / per_run * xcds + xcd) * kNormRun, tid = threadIdx.x;
+  const long cols = (long)(H + KV) * dk + (long)KV * dv, kblock = (long)page_size * dk, vblock = (long)page_size * dv;
+  auto sums = [&](const float* src) {
+    floatx4 v = *reinterpret_cast<const floatx4*>(src);
+    for (int s = 1; s < nsplit; ++s) v += *reinterpret_cast<const floatx4*>(src + s * split_stride);
+    return v;
+  };
+  if (at >= kNormRun * chunks) {
+    // values: thread = (token of the run, four neighbouring elements)
+    const int t = t0 + tid % kNormRun, idx = (at - kNormRun * chunks) * (4 * 256 / kNormRun) + tid / kNormRun * 4;
+    if (t >= n || idx >= KV * dv) return;
+    const int pos = positions[t], span = span_of_token[t];
+    const long vcol = (long)(H + KV) * dk + idx;
+    floatx4 v = sums(qkv + t * cols + vcol);
+    if (bias) v += *reinterpret_cast<const floatx4*>(bias + vcol);
+    const long page = block_table[(long)span * max_pages + pos / page_size];
+    const int h = idx / dv, j = idx % dv;
+    T* dst = cache + page * KV * (kblock + vblock) + KV * kblock + h * vblock + pos % page_size;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) dst[(long)(j + e) * page_size] = from_f32<T>(v[e]);
+    return;
+  }
+  const int t = t0 + at % kNormRun;
+  if (t >= n) return;
+  int at_v = t;                                          // (vector loads: scalar ones come one behind the other)
+  asm volatile("" : "+v"(at_v));
+  const int pos_v = positions[at_v], span_v = span_of_token[at_v];
+  const int item = at / kNormRun * (256 / L) + tid / L, i = tid % L, it = min(item, H + KV - 1), rq = rot / 8;
+  const bool turns = i < rq, is_q = it < H;
+  const int ea = turns ? 4 * i : rot + 8 * (i - rq), eb = turns ? ea + rot / 2 : ea + 4;
+  const long base = (long)it * dk;                       // queries first, then keys, head after head
+  const float* src = qkv + t * cols + base;
+  floatx4 a = sums(src + ea), b = sums(src + eb), c = {1, 1, 1, 1}, sn = {0, 0, 0, 0};
+  if (turns && cos_t) {
+    c = *reinterpret_cast<const floatx4*>(cos_t + (long)t * (rot / 2) + 4 * i);
+    sn = *reinterpret_cast<const floatx4*>(sin_t + (long)t * (rot / 2) + 4 * i);
+  }
+  if (bias) {
+    a += *reinterpret_cast<const floatx4*>(bias + base + ea);
+    b += *reinterpret_cast<const floatx4*>(bias + base + eb);
+  }
+  const float* nw = is_q ? q_weight : k_weight;
+  auto squares = [&] {
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss += a[e] * a[e] + b[e] * b[e];
+    return 1.f / sqrtf(parts_sum<L>(ss) / (float)dk + eps);
+  };
+  if (nw) {                                              // a norm with weights in front of the rotation
+    const floatx4 wa = *reinterpret_cast<const floatx4*>(nw + ea), wb = *reinterpret_cast<const floatx4*>(nw + eb);
+    const float rs = squares();
+    a = a * rs * wa;
+    b = b * rs * wb;
+  }
+  const floatx4 ra = a * c - b * sn, rb = b * c + a * sn;
+  a = ra;
+  b = rb;
+  if (!nw && unit_norm) {
+    const float rs = squares();
+    a *= rs;
+    b *= rs;
+  }
+  if (item >= H + KV) return;
+  T* dst = q_out + (long)t * H * dk + base;
+  if (!is_q) {
+    const int pos = __builtin_amdgcn_readfirstlane(pos_v), span = __builtin_amdgcn_readfirstlane(span_v);
+    const long page = block_table[(long)span * max_pages + pos / page_size];
+    dst = cache + page * KV * (kblock + vblock) + (it - H) * kblock + (long)(pos % page_size) * dk;
+  }
+  tx4 lo, hi;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    lo[e] = from_f32<T>(a[e]);
+    hi[e] = from_f32<T>(b[e]);
+  }
+  *reinterpret_cast<tx4*>(dst + ea) = lo;
+  *reinterpret_cast<tx4*>(dst + eb) = hi;
+}
+
 template <typename TOUT>
 __global__ void gate_bias_kernel(const float* __restrict__ gu, int nsplit, long split_stride,
                                  const float* __restrict__ bias, TOUT* __restrict__ out, long count, int f, int act,
@@ -524,6 +620,31 @@ extern "C" int kllm_qkv_norm_append(const float* qkv, int nsplit, long split_str
   KLLM_REQUIRE((cos_t == nullptr) == (sin_t == nullptr), "qkv_norm_append: cos and sin go together");
   KLLM_REQUIRE(max_pages > 0 && page_size > 0, "qkv_norm_append: bad cache sizes");
   KLLM_REQUIRE(dtype == DT_F32 || dtype == DT_BF16, "qkv_norm_append: unknown dtype %d", dtype);
+  // Whole pieces of four numbers everywhere: the kernel with eight elements a lane.
+  const uintptr_t any = (uintptr_t)qkv | (uintptr_t)bias | (uintptr_t)cos_t | (uintptr_t)sin_t | (uintptr_t)q_weight | (uintptr_t)k_weight |
+                        (uintptr_t)q_out | (uintptr_t)cache;
+  const long cols = (long)(H + KV) * dk + (long)KV * dv;
+  const int runs0 = ceil_div(n, kNormRun), xcds = runs0 >= device_xcds() ? device_xcds() : 1, L = dk / 8;
+  if ((dk == 32 || dk == 64 || dk == 128 || dk == 256) && !interleaved && rot % 8 == 0 && dv % 4 == 0 && (any & 15) == 0 &&
+      (nsplit == 1 || split_stride % 4 == 0) && cols < (1L << 30)) {
+    const int chunks = ceil_div((H + KV) * L, 256), vblocks = ceil_div((long)KV * dv, 4 * 256 / kNormRun);
+    const long blocks = (long)ceil_div(runs0, xcds) * xcds * (kNormRun * chunks + vblocks);       // padded: every XCD gets as many runs
+    if (blocks < (1L << 31)) {
+#define KLLM_QV(T, L)                                                                                                        \
+  hipLaunchKernelGGL((qkv_norm_append_vec_kernel<T, L>), dim3(blocks), dim3(256), 0, stream, positions, span_of_token, qkv, n, \
+                     H, KV, dv, rot, chunks, vblocks, xcds, cos_t, sin_t, nsplit, unit_norm, eps, max_pages, page_size,      \
+                     split_stride, block_table, bias, q_weight, k_weight, (T*)q_out, (T*)cache)
+#define KLLM_QVS(T)                                                                                                          \
+  do {                                                                                                                       \
+    if (L == 4) KLLM_QV(T, 4); else if (L == 8) KLLM_QV(T, 8); else if (L == 16) KLLM_QV(T, 16); else KLLM_QV(T, 32);        \
+  } while (0)
+      if (dtype == DT_F32) KLLM_QVS(float); else KLLM_QVS(bf16_t);
+#undef KLLM_QVS
+#undef KLLM_QV
+      KLLM_CHECK_LAUNCH("qkv_norm_append");
+      return 0;
+    }
+  }
   const dim3 grid(n, ceil_div(H + 2 * KV, 4));
   if (dtype == DT_F32)
     hipLaunchKernelGGL(qkv_norm_append_kernel<float>, grid, dim3(256), 0, stream, qkv, nsplit, split_stride, bias, cos_t,

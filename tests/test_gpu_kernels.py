@@ -1635,3 +1635,44 @@ def test_attention_decode_places_float32(H, KV, hd, ps, window):
             out = run_attention("decode", c["q"], c["cache"], c["pos"], c["sot"], c["bt"], ps, H, KV, hd, window, c["scale"], nslices=ns)
             err = (out.cpu().double() - c["want"]).abs().max()
             assert torch.isfinite(out).all() and err < 2e-5, (ns, float(err))
+
+
+@pytest.mark.parametrize("dk,dv,rot", [(32, 36, 8), (64, 64, 32), (128, 128, 128), (256, 100, 0), (64, 12, 48)])
+@pytest.mark.parametrize("n,nsplit", [(1, 1), (17, 3), (700, 1)])
+@pytest.mark.parametrize("norm", ["unit", "weights", "none"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_qkv_norm_append_in_whole_pieces(dk, dv, rot, n, nsplit, norm, dtype):
+    """Eight elements a lane against a pair a lane (the same call with sums that lie beside a 16-byte border): parts of a head that
+    turn and that pass, a run of tokens that is not whole, runs over all XCDs and slots in pages of 24.  The norms' sums are added in other
+    orders, a few units of 2^-24 of a rotated pair's terms, which may cancel in the result and are no more than twice the greatest one; then
+    the results are rounded to the cache's type."""
+    k_ = K()
+    H, KV, ps = 5, 2, 24
+    g = torch.Generator().manual_seed(dk + n)
+    f = lambda *s: torch.randn(*s, generator=g).to(DEV)
+    cols = (H + KV) * dk + KV * dv
+    flat = f(nsplit * n * cols + 1)
+    sums, aside = flat[:-1].clone().view(nsplit, n, cols), flat.clone()
+    aside[1:] = flat[:-1]
+    pos = torch.arange(n, dtype=torch.int32, device=DEV) + 7
+    pages = (n + 7) // ps + 1
+    table = torch.randperm(pages, generator=g).to(torch.int32).view(1, -1).to(DEV)
+    span = torch.zeros(n, dtype=torch.int32, device=DEV)
+    ang = f(n, max(rot // 2, 1))
+    kw = dict(bias=f(cols), interleaved=False, unit_norm=norm == "unit", eps=1e-5)
+    if rot:
+        kw.update(cos=ang.cos(), sin=ang.sin(), rotary_dim=rot)
+    if norm == "weights":
+        kw.update(q_weight=f(dk), k_weight=f(dk))
+    got = []
+    for x in (sums, aside[1:].view(nsplit, n, cols)):
+        q = torch.full((n, H * dk), float("nan"), dtype=dtype, device=DEV)
+        cache = torch.zeros(pages, KV * ps * (dk + dv), dtype=dtype, device=DEV)
+        if dk == dv:
+            cache = cache.view(pages, 2, KV, ps * dk)
+        k_.qkv_norm_append(x, q, cache, pos, span, table, ps, H, KV, dk, dv, **kw)
+        got.append((q.double(), cache.double()))
+    assert sums.data_ptr() % 16 == 0 and aside[1:].data_ptr() % 16 == 4
+    for one, other in zip(*got):
+        assert torch.isfinite(one).all() and one.abs().max() > 0
+        assert ((one - other).abs() <= (2.0 ** -7 if dtype == torch.bfloat16 else 0.0) * other.abs() + 2.0 ** -21 * other.abs().max()).all()
