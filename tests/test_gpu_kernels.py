@@ -1676,3 +1676,26 @@ def test_qkv_norm_append_in_whole_pieces(dk, dv, rot, n, nsplit, norm, dtype):
     for one, other in zip(*got):
         assert torch.isfinite(one).all() and one.abs().max() > 0
         assert ((one - other).abs() <= (2.0 ** -7 if dtype == torch.bfloat16 else 0.0) * other.abs() + 2.0 ** -21 * other.abs().max()).all()
+
+
+@pytest.mark.parametrize("n,d", [(7, 2049), (300, 3001), (3, 9001), (7, 2048), (700, 2048), (300, 4100), (257, 16384), (3, 16388)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_rows_of_whole_pieces_and_odd_ones(n, d, dtype):
+    """The norm of one and two slices, with one, two and four pieces a thread, with rows whose length is no multiple of four and with ones too
+    long for it; and the embedding of such rows, some by a token that lies on the device.  Bounds as in ``test_add_rmsnorm``."""
+    x, w = rnd(n, d, seed=1, scale=3.0), (1 + 0.2 * rnd(d, seed=2))
+    for nsplit in (1, 2, 5):
+        delta, x1, out = rnd(nsplit, n, d, seed=3 + nsplit), x.clone(), torch.full((n, d), float("nan"), dtype=dtype, device=DEV)
+        K().add_rmsnorm(x1, delta=delta, weight=w, out=out, eps=1e-5)
+        want = x.double() + delta.double().sum(0)
+        assert (x1.double() - want).abs().max() < 2e-5
+        assert (out.double() - P.rmsnorm(want.cpu(), w.cpu().double(), 1e-5).to(DEV)).abs().max() < tol(dtype) * 3
+    table = rnd(131, d, dtype=dtype)
+    ids = torch.arange(n, dtype=torch.int32, device=DEV) % 131
+    from_, sampled = torch.full((n,), -1, dtype=torch.int32, device=DEV), torch.tensor([130, 4], dtype=torch.int32, device=DEV)
+    from_[0], from_[n - 1] = 1, 0
+    out, copy = torch.full((n, d), float("nan"), device=DEV), torch.full((n, d), float("nan"), dtype=dtype, device=DEV)
+    K().embed(out, table, ids, from_, sampled, scale=3.0, copy=copy)
+    ids[0], ids[n - 1] = 4, 130
+    want = table[ids.long()].float() * 3.0
+    assert torch.equal(out, want) and torch.equal(copy, want.to(dtype))
