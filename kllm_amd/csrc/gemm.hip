@@ -529,3 +529,24 @@ extern "C" int kllm_gemm_act(const void* x, const void* w, void* h, int n, int m
   KLLM_CHECK_LAUNCH("gemm_act");
   return 0;
 }
+
+// q = the rotated queries of x . w^T, keys and values into the pages: the product, the rotation and the append in one launch (RING_ROPE).
+extern "C" int kllm_gemm_rope(const void* x, const KllmLinearOut* y, const void* w, int n, int m, int k, hipStream_t stream) {
+  KLLM_REQUIRE(x && w && y && y->y && y->kind == KLLM_LINEAR_OUT_ROPE, "gemm_rope: null pointer, or another kind of output");
+  KLLM_REQUIRE(n > 0 && m > 0 && k > 0, "gemm_rope: bad sizes n=%d m=%d k=%d", n, m, k);
+  const int chunk = y->f32 ? 4 : 8, H = y->H, KV = y->KV, hd = y->hd;
+  KLLM_REQUIRE(k % chunk == 0 && k < (1 << 23) && (long)m * k * (16 / chunk) < (1L << 32) && aligned16(x) && aligned16(w),
+               "gemm_rope: K=%d must be a multiple of %d, the weights below 4 GiB and the operands 16-byte aligned", k, chunk);
+  KLLM_REQUIRE(H > 0 && hd > 0 && hd % 8 == 0 && (!y->cache || KV > 0) && m == H * hd + (y->cache ? 2 * KV * hd : 0),
+               "gemm_rope: m=%d does not fit %d and %d heads of %d (a multiple of 8)", m, H, KV, hd);
+  KLLM_REQUIRE((y->cos_t == nullptr) == (y->sin_t == nullptr), "gemm_rope: cos and sin go together");
+  KLLM_REQUIRE(aligned16(y->y) && aligned16(y->cache) && aligned16(y->cos_t) && aligned16(y->sin_t), "gemm_rope: unaligned pointer");
+  KLLM_REQUIRE(!y->cache || (y->positions && y->span_of_token && y->block_table && y->max_pages > 0 && y->page_size > 0),
+               "gemm_rope: the append needs positions, spans, a block table and pages");
+  KLLM_REQUIRE((long)n * m < (1L << 31), "gemm_rope: sizes overflow");
+  const RingRope rope = {y->cos_t, y->sin_t, y->cache, y->positions, y->span_of_token, y->block_table,
+                         y->max_pages, y->page_size, H, y->cache ? KV : 0, hd / 2};
+  if (int rc = gemm_ring(x, w, y->y, n, m / 2, k, 1, RING_ROPE, y->f32 != 0, y->f32 != 0, -1, nullptr, stream, rope)) return rc;
+  KLLM_CHECK_LAUNCH("gemm_rope");
+  return 0;
+}

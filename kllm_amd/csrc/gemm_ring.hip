@@ -104,8 +104,8 @@ template <typename T, typename TOUT, int MODE, int WR, int WC, int TM, int TN, i
 __global__ __launch_bounds__(512, sizeof(T) == 4 ? 6 : 2) void gemm_ring_kernel(const T* __restrict__ X, const T* __restrict__ W,
                                                            TOUT* __restrict__ Y, int n, int m, int k, int tiles_x,
                                                            int tiles_y, int kslice, int act,
-                                                           const float* __restrict__ act_params, int xcds) {
-  constexpr bool GATE = MODE == RING_GATE, TAIL = KIND != RING_WHOLE;
+                                                           const float* __restrict__ act_params, int xcds, const RingRope rope) {
+  constexpr bool ROPE = MODE == RING_ROPE, GATE = MODE == RING_GATE || ROPE, TAIL = KIND != RING_WHOLE;      // (GATE: columns in pairs)
   typedef typename RingOperand<T>::type op_t;
   typedef typename RingOffset<KIND == RING_LONG>::type off_t;
   constexpr int EPC = 16 / sizeof(T), STAGE = 8 * EPC;     // elements of a chunk of 16 bytes, of a stage
@@ -159,9 +159,14 @@ __global__ __launch_bounds__(512, sizeof(T) == 4 ? 6 : 2) void gemm_ring_kernel(
 #pragma unroll
     for (int h = 0; h < 2; ++h)       // GATE: the first half of a tile's rows of W are gates, the second their up rows
       woff[h][i] = (off_t)(min(col0 + (GATE ? 0 : h * WS) + r, m - 1) - col0) * (off_t)k * (off_t)sizeof(T) + wchunk[i] * 16u;
+    if constexpr (ROPE) {             // pair c is elements c % half and half + c % half of head c / half
+      const int c = min(col0 + r, m - 1);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) woff[h][i] = (off_t)(c + (c / rope.half + h) * rope.half) * (off_t)k * (off_t)sizeof(T) + wchunk[i] * 16u;
+    }
   }
   const T* const xbase = X + (long)row0 * k + kbeg;
-  const T* const wbase[2] = {W + (long)col0 * k + kbeg, W + ((long)col0 + (GATE ? m : 0)) * k + kbeg};
+  const T* const wbase[2] = {W + (ROPE ? 0 : (long)col0 * k) + kbeg, W + (ROPE ? 0 : ((long)col0 + (GATE ? m : 0)) * k) + kbeg};
 
   auto load = [&](const char* src, off_t& off, int chunk, int left, unsigned char* dst) {
     if (CHAINS > 1) asm volatile("" : "+v"(off));        // (or the loop keeps 64-bit addresses instead: eight registers, spills)
@@ -288,6 +293,91 @@ __global__ __launch_bounds__(512, sizeof(T) == 4 ? 6 : 2) void gemm_ring_kernel(
   auto sum = [&](int hx, int hw, int i, int j, int e) {
     return CHAINS == 1 ? acc[0][hx][hw][i][j][e] : acc[0][hx][hw][i][j][e] + acc[CHAINS - 1][hx][hw][i][j][e];
   };
+  if constexpr (ROPE) {
+    // A lane's four columns are four neighbouring pairs of a head.  The rows' pages are looked up where the tile has keys or values; a
+    // value's place is beside its neighbour token's, so sixteen lanes fill a sector, as in rope_append.  In place of the 32-bit sums' way out and
+    // back and rope_append's launch, in us: 2,048 x 2,560 x 2,048 33.0 + 9.0 and a gap -> 35.1; prompts of 2,048 at 1.1B Llama sizes 5,850 -> 5,720, of
+    // 1,999 at 8B sizes 25,310 -> 24,850; 500 to 1,300 tokens, and 32-bit, the same to 0.3 %.
+    typedef T tx4 __attribute__((ext_vector_type(4)));
+    const int half = rope.half, hd = 2 * half, H = rope.H, KV = rope.KV, qd = H * hd, page_size = rope.page_size;
+    const bool keys = rope.cache && col0 + WS > H * half;  // (a tile's columns may end behind the last pair)
+    int head[TN], at[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int c = col0 + (wc * TN + j) * 16 + 4 * lch;
+      head[j] = c / half;
+      at[j] = c - head[j] * half;
+      if (c >= m) head[j] = -1;
+    }
+    int page[2][TM] = {}, slot[2][TM] = {};
+    if (keys) {
+      int span[2][TM];
+#pragma unroll
+      for (int hx = 0; hx < 2; ++hx)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const int r = min(row0 + hx * XR + (wr * TM + i) * 16 + lrow, n - 1);
+          slot[hx][i] = rope.positions[r];
+          span[hx][i] = rope.span_of_token[r];
+        }
+#pragma unroll
+      for (int hx = 0; hx < 2; ++hx)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const int p = slot[hx][i] / page_size;
+          page[hx][i] = rope.block_table[(long)span[hx][i] * rope.max_pages + p];
+          slot[hx][i] -= p * page_size;
+        }
+    }
+    T* const cache = static_cast<T*>(rope.cache);
+    const long block = (long)page_size * hd;
+    // (the next row's turns are asked for while this one is stored; rows behind the last read that one's)
+    floatx4 cs[2][TN], sn[2][TN];
+    auto turn = [&](int t) {
+      const int r = min(row0 + t / TM * XR + (wr * TM + t % TM) * 16 + lrow, n - 1);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        cs[t % 2][j] = floatx4{1.f, 1.f, 1.f, 1.f};
+        sn[t % 2][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        if (rope.cos_t) {
+          cs[t % 2][j] = *reinterpret_cast<const floatx4*>(rope.cos_t + (long)r * half + at[j]);
+          sn[t % 2][j] = *reinterpret_cast<const floatx4*>(rope.sin_t + (long)r * half + at[j]);
+        }
+      }
+    };
+    turn(0);
+#pragma unroll
+    for (int t = 0; t < 2 * TM; ++t) {
+      const int hx = t / TM, i = t % TM, r = row0 + hx * XR + (wr * TM + i) * 16 + lrow;
+      if (t + 1 < 2 * TM) turn(t + 1);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        tx4 lo, hi;
+        const bool value = head[j] >= H + KV;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float a = sum(hx, 0, i, j, e), b = sum(hx, 1, i, j, e);
+          lo[e] = from_f32<T>(value ? a : a * cs[t % 2][j][e] - b * sn[t % 2][j][e]);
+          hi[e] = from_f32<T>(value ? b : b * cs[t % 2][j][e] + a * sn[t % 2][j][e]);
+        }
+        if (r >= n || head[j] < 0) continue;
+        if (!value) {
+          T* o = head[j] < H ? Y + (long)r * qd + head[j] * hd
+                             : cache + ((long)page[hx][i] * 2 * KV + head[j] - H) * block + (long)slot[hx][i] * hd;
+          *reinterpret_cast<tx4*>(o + at[j]) = lo;
+          *reinterpret_cast<tx4*>(o + at[j] + half) = hi;
+        } else {
+          T* v = cache + (((long)page[hx][i] * 2 + 1) * KV + head[j] - H - KV) * block + slot[hx][i];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            v[(long)(at[j] + e) * page_size] = lo[e];
+            v[(long)(at[j] + e + half) * page_size] = hi[e];
+          }
+        }
+      }
+    }
+    return;
+  }
   const bool vec = m % 4 == 0 && (reinterpret_cast<uintptr_t>(Y) & (4 * sizeof(TOUT) - 1)) == 0;
 #pragma unroll
   for (int hx = 0; hx < 2; ++hx)
@@ -424,8 +514,8 @@ static int ring_tile(bool f32, int n, int m, int k, int nsplit, bool gate, bool 
 
 template <typename T, typename TOUT, int MODE, int WR, int WC, int TM, int TN, int KIND>
 static int ring_launch(const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int act,
-                       const float* act_params, hipStream_t stream) {
-  constexpr int XR = WR * TM * 16, WS = WC * TN * 16, BM = 2 * XR, BN = MODE == RING_GATE ? WS : 2 * WS;
+                       const float* act_params, const RingRope& rope, hipStream_t stream) {
+  constexpr int XR = WR * TM * 16, WS = WC * TN * 16, BM = 2 * XR, BN = MODE == RING_GATE || MODE == RING_ROPE ? WS : 2 * WS;
   const int tx = ceil_div(m, BN), ty = ceil_div(n, BM), xcds = device_xcds();
   const dim3 grid(ceil_div((long)tx * ty, xcds) * xcds, nsplit);   // padded so that every XCD gets as many
   const size_t lds = (size_t)4 * (XR + WS) * 128;
@@ -438,48 +528,52 @@ static int ring_launch(const void* x, const void* w, void* y, int n, int m, int 
   }
   hipLaunchKernelGGL((gemm_ring_kernel<T, TOUT, MODE, WR, WC, TM, TN, KIND>), grid, dim3(512), lds, stream, (const T*)x,
                      (const T*)w, (TOUT*)y, n, m, k, tx, ty, ring_kslice(k, nsplit, 256 / (int)sizeof(T)), act,
-                     act_params, xcds);
+                     act_params, xcds, rope);
   return 0;
 }
 
 template <typename T, typename TOUT, int MODE, int KIND>
 static int ring_shape(int tile, const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int act,
-                      const float* ap, hipStream_t st) {
+                      const float* ap, const RingRope& rope, hipStream_t st) {
   if constexpr (sizeof(T) == 2 && KIND != RING_LONG) {
     switch (tile) {
-      case 0: return ring_launch<T, TOUT, MODE, 2, 4, 4, 2, KIND>(x, w, y, n, m, k, nsplit, act, ap, st);
-      case 1: return ring_launch<T, TOUT, MODE, 4, 2, 2, 3, KIND>(x, w, y, n, m, k, nsplit, act, ap, st);
-      case 2: return ring_launch<T, TOUT, MODE, 2, 4, 2, 2, KIND>(x, w, y, n, m, k, nsplit, act, ap, st);
-      case 3: return ring_launch<T, TOUT, MODE, 2, 4, 2, 1, KIND>(x, w, y, n, m, k, nsplit, act, ap, st);
-      case kRingWide: return ring_launch<T, TOUT, MODE, 2, 4, 1, 2, KIND>(x, w, y, n, m, k, nsplit, act, ap, st);
+      case 0: return ring_launch<T, TOUT, MODE, 2, 4, 4, 2, KIND>(x, w, y, n, m, k, nsplit, act, ap, rope, st);
+      case 1: return ring_launch<T, TOUT, MODE, 4, 2, 2, 3, KIND>(x, w, y, n, m, k, nsplit, act, ap, rope, st);
+      case 2: return ring_launch<T, TOUT, MODE, 2, 4, 2, 2, KIND>(x, w, y, n, m, k, nsplit, act, ap, rope, st);
+      case 3: return ring_launch<T, TOUT, MODE, 2, 4, 2, 1, KIND>(x, w, y, n, m, k, nsplit, act, ap, rope, st);
+      case kRingWide: return ring_launch<T, TOUT, MODE, 2, 4, 1, 2, KIND>(x, w, y, n, m, k, nsplit, act, ap, rope, st);
     }
   }
-  return ring_launch<T, TOUT, MODE, 2, 4, 1, 1, KIND>(x, w, y, n, m, k, nsplit, act, ap, st);
+  return ring_launch<T, TOUT, MODE, 2, 4, 1, 1, KIND>(x, w, y, n, m, k, nsplit, act, ap, rope, st);
 }
 
 template <typename T, typename TOUT, int MODE>
 static int ring_kind(int tile, const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int act,
-                     const float* ap, hipStream_t st) {
+                     const float* ap, const RingRope& rope, hipStream_t st) {
   constexpr int PAIR = 256 / sizeof(T);
-  if (k >= kRingLongK) return ring_shape<T, TOUT, MODE, RING_LONG>(tile, x, w, y, n, m, k, nsplit, act, ap, st);
+  if constexpr (MODE != RING_ROPE)
+    if (k >= kRingLongK) return ring_shape<T, TOUT, MODE, RING_LONG>(tile, x, w, y, n, m, k, nsplit, act, ap, rope, st);
   const int slice = ring_kslice(k, nsplit, PAIR);
   const bool whole = k % PAIR == 0 && slice % PAIR == 0;
-  return whole ? ring_shape<T, TOUT, MODE, RING_WHOLE>(tile, x, w, y, n, m, k, nsplit, act, ap, st)
-               : ring_shape<T, TOUT, MODE, RING_TAIL>(tile, x, w, y, n, m, k, nsplit, act, ap, st);
+  return whole ? ring_shape<T, TOUT, MODE, RING_WHOLE>(tile, x, w, y, n, m, k, nsplit, act, ap, rope, st)
+               : ring_shape<T, TOUT, MODE, RING_TAIL>(tile, x, w, y, n, m, k, nsplit, act, ap, rope, st);
 }
 
 int gemm_ring(const void* x, const void* w, void* y, int n, int m, int k, int nsplit, int mode, bool f32, bool f32_out,
-              int act, const float* act_params, hipStream_t stream) {
-  const int tile = ring_tile(f32, n, m, k, nsplit, mode == RING_GATE, f32_out);
+              int act, const float* act_params, hipStream_t stream, const RingRope& rope) {
+  const int tile = ring_tile(f32, n, m, k, nsplit, mode == RING_GATE || mode == RING_ROPE, f32_out);
+  if (mode == RING_ROPE)
+    return f32 ? ring_kind<float, float, RING_ROPE>(tile, x, w, y, n, m, k, 1, act, act_params, rope, stream)
+               : ring_kind<bf16_t, bf16_t, RING_ROPE>(tile, x, w, y, n, m, k, 1, act, act_params, rope, stream);
   if (f32) {
-    if (mode == RING_GATE) return ring_kind<float, float, RING_GATE>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
-    if (mode == RING_UNARY) return ring_kind<float, float, RING_UNARY>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
-    return ring_kind<float, float, RING_SUMS>(tile, x, w, y, n, m, k, nsplit, act, act_params, stream);
+    if (mode == RING_GATE) return ring_kind<float, float, RING_GATE>(tile, x, w, y, n, m, k, 1, act, act_params, rope, stream);
+    if (mode == RING_UNARY) return ring_kind<float, float, RING_UNARY>(tile, x, w, y, n, m, k, 1, act, act_params, rope, stream);
+    return ring_kind<float, float, RING_SUMS>(tile, x, w, y, n, m, k, nsplit, act, act_params, rope, stream);
   }
-  if (mode == RING_GATE) return ring_kind<bf16_t, bf16_t, RING_GATE>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
-  if (mode == RING_UNARY) return ring_kind<bf16_t, bf16_t, RING_UNARY>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
-  if (f32_out) return ring_kind<bf16_t, float, RING_SUMS>(tile, x, w, y, n, m, k, nsplit, act, act_params, stream);
-  return ring_kind<bf16_t, bf16_t, RING_SUMS>(tile, x, w, y, n, m, k, 1, act, act_params, stream);
+  if (mode == RING_GATE) return ring_kind<bf16_t, bf16_t, RING_GATE>(tile, x, w, y, n, m, k, 1, act, act_params, rope, stream);
+  if (mode == RING_UNARY) return ring_kind<bf16_t, bf16_t, RING_UNARY>(tile, x, w, y, n, m, k, 1, act, act_params, rope, stream);
+  if (f32_out) return ring_kind<bf16_t, float, RING_SUMS>(tile, x, w, y, n, m, k, nsplit, act, act_params, rope, stream);
+  return ring_kind<bf16_t, bf16_t, RING_SUMS>(tile, x, w, y, n, m, k, 1, act, act_params, rope, stream);
 }
 
 }  // namespace kllm

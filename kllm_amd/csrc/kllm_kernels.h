@@ -194,6 +194,9 @@ typedef struct {
   int y_tiled;          /* kllm_linear_rows, RESID and SWIGLU: y goes out in the order the next such product's lanes read */
 } KllmLinearOut;
 long kllm_fused_linear_lds_bytes(int n, int k, int nsplit, int dtype);
+/* A prompt's queries, keys and values with rotation and append: out->kind ROPE (H, KV, hd a multiple of 8, cos_t, sin_t, cache,
+ * ...), w [m][k] as stored, out->f32 as there; all of K in one slice. */
+int kllm_gemm_rope(const void* x, const KllmLinearOut* out, const void* w, int n, int m, int k, hipStream_t stream);
 /* The same products of up to 64 rows of bfloat16 or 16 of float32, all of K (a multiple of 32) in a workgroup and nothing staged,
  * w the tiled copy (float32: or the weights themselves, below 2 GiB; the same bits).  RESID leaves kllm_linear_rows_parts(n, m, k) sums of squares a row (0: the sizes are not taken).  Tiled rows
  * (y_tiled, x_tiled; columns a multiple of 32): [row / 16][column / 32][column % 32 / 8][row % 16][8]; with more than 16 rows

@@ -143,6 +143,7 @@ def _declare(lib):
         "kllm_attn_decode": [P, P, P, L, P, P, P, P, I, I, I, I, I, I, I, I, P, I, F, P, I, I, P, I, P, I, L, L, I, I, P],
         "kllm_attn_prefill": [P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, P, I, F, P, L, I, P, L, I, I, I, P, I, L, L, I, I, P],
         "kllm_attn_prefill_slices": [I, I, I],
+        "kllm_gemm_rope": [P, P, P, I, I, I, P],
         "kllm_gemm_act": [P, P, P, I, I, I, I, I, P, P],
         "kllm_add_sinusoid": [P, P, I, I, D, P],
         "kllm_unary_act": [P, I, L, I, P, I, I, I, I, P, P],
@@ -200,7 +201,7 @@ def _declare(lib):
 LAUNCHING = ("kllm_embed", "kllm_add_rmsnorm", "kllm_rope_tables", "kllm_rope_append", "kllm_silu_mul",
              "kllm_sum_splits", "kllm_gemm", "kllm_gemm_swiglu", "kllm_gemv_plain", "kllm_gemv_swiglu",
              "kllm_gemv_resid", "kllm_gemv_rope_append", "kllm_fused_linear", "kllm_linear_rows", "kllm_attn_generic",
-             "kllm_attn_decode", "kllm_attn_prefill", "kllm_sample", "kllm_gemm_act", "kllm_add_sinusoid", "kllm_unary_act",
+             "kllm_attn_decode", "kllm_attn_prefill", "kllm_sample", "kllm_gemm_act", "kllm_gemm_rope", "kllm_add_sinusoid", "kllm_unary_act",
              "kllm_group_norm_add", "kllm_qk_norm_append", "kllm_delta_prep", "kllm_delta_scan", "kllm_delta_out",
              "kllm_norm_residual", "kllm_rope_tables_freq", "kllm_qkv_norm_append", "kllm_gate_bias", "kllm_moe_route",
              "kllm_moe_plan", "kllm_moe_expert", "kllm_moe_expert_rows", "kllm_moe_combine",
@@ -211,7 +212,7 @@ LAUNCHING = ("kllm_embed", "kllm_add_rmsnorm", "kllm_rope_tables", "kllm_rope_ap
              "kllm_decayed_scan", "kllm_decayed_out", "kllm_decayed_step", "kllm_token_gate", "kllm_soft_cap")
 DYNAMIC_ARGS = {"kllm_attn_prefill": (19, 20)}     # arguments that may be a StepValue
 STRUCT_ARGS = {"kllm_gemv_plain": (7,), "kllm_gemv_swiglu": (8,), "kllm_gemv_rope_append": (17,),
-               "kllm_fused_linear": (2,), "kllm_linear_rows": (2,)}
+               "kllm_fused_linear": (2,), "kllm_linear_rows": (2,), "kllm_gemm_rope": (1,)}
 
 
 def _check(rc: int, what: str):
@@ -1040,6 +1041,27 @@ def _linear_rows_best(kind, n, m, k, dtype, tiled_x):
     return 32 * k * busiest * (1 if tiled_x else 2) <= LINEAR_ROWS_BYTES
 
 
+def _describe_rope(lo, rope, n, typ):
+    """The rotate-and-append epilogue's part of ``lo``, checked against n rows of ``typ``."""
+    half = rope.head_dim // 2
+    if rope.cos is not None and (tuple(rope.cos.shape) != (n, half) or tuple(rope.sin.shape) != (n, half)):
+        raise KernelError("fused_linear: cos/sin shapes do not fit")
+    lo.cos_t = _ptr(rope.cos, "fused_linear cos", torch.float32, True)
+    lo.sin_t = _ptr(rope.sin, "fused_linear sin", torch.float32, True)
+    if rope.cache is not None:
+        if (tuple(rope.cache.shape[1:]) != (2, rope.kv_heads, rope.page_size * rope.head_dim)
+                or rope.cache.dtype != typ):
+            raise KernelError(f"fused_linear: cache {tuple(rope.cache.shape)} {rope.cache.dtype} does not fit")
+        if rope.positions.numel() < n or rope.span_of_token.numel() < n:
+            raise KernelError("fused_linear: index arrays are too short")
+        lo.cache = _ptr(rope.cache, "fused_linear cache")
+        lo.positions = _ptr(rope.positions, "fused_linear positions", torch.int32)
+        lo.span_of_token = _ptr(rope.span_of_token, "fused_linear span_of_token", torch.int32)
+        lo.block_table = _ptr(rope.block_table, "fused_linear block_table", torch.int32)
+        lo.max_pages = rope.block_table.shape[1]
+    lo.page_size, lo.H, lo.KV, lo.hd = rope.page_size, rope.heads, rope.kv_heads, rope.head_dim
+
+
 def linear_rows(w, y, kind, x, rope=None, act=ACT_SILU, resid=None, norm_weight=None, ss_out=None, unary=None):
     """``fused_linear`` for up to 64 rows of bfloat16 or 16 of float32, K a multiple of 32, in one slice,
     from the tiled copy ``w`` of the weights (float32: or from the matrix, with the same bits), nothing staged in LDS.  ``x`` (also inside a ``ScaledRows``) may be
@@ -1114,23 +1136,7 @@ def fused_linear(w, y, kind, x, nsplit=1, tiles_per_wg=1, rope=None, act=ACT_SIL
         if rope is None:
             raise KernelError("fused_linear: the rope epilogue needs its description")
         want, dt = (n, rope.heads * rope.head_dim), typ
-        half = rope.head_dim // 2
-        if rope.cos is not None and (tuple(rope.cos.shape) != (n, half) or tuple(rope.sin.shape) != (n, half)):
-            raise KernelError("fused_linear: cos/sin shapes do not fit")
-        lo.cos_t = _ptr(rope.cos, "fused_linear cos", torch.float32, True)
-        lo.sin_t = _ptr(rope.sin, "fused_linear sin", torch.float32, True)
-        if rope.cache is not None:
-            if (tuple(rope.cache.shape[1:]) != (2, rope.kv_heads, rope.page_size * rope.head_dim)
-                    or rope.cache.dtype != typ):
-                raise KernelError(f"fused_linear: cache {tuple(rope.cache.shape)} {rope.cache.dtype} does not fit")
-            if rope.positions.numel() < n or rope.span_of_token.numel() < n:
-                raise KernelError("fused_linear: index arrays are too short")
-            lo.cache = _ptr(rope.cache, "fused_linear cache")
-            lo.positions = _ptr(rope.positions, "fused_linear positions", torch.int32)
-            lo.span_of_token = _ptr(rope.span_of_token, "fused_linear span_of_token", torch.int32)
-            lo.block_table = _ptr(rope.block_table, "fused_linear block_table", torch.int32)
-            lo.max_pages = rope.block_table.shape[1]
-        lo.page_size, lo.H, lo.KV, lo.hd = rope.page_size, rope.heads, rope.kv_heads, rope.head_dim
+        _describe_rope(lo, rope, n, typ)
     else:
         raise KernelError(f"fused_linear: unknown output kind {kind}")
     if tuple(y.shape) != want or y.dtype != dt:
@@ -1419,6 +1425,27 @@ def gemm_act(x, w, h, act, params=None):
         raise KernelError("gemm_act: xielu needs its two constants")
     _launch("kllm_gemm_act", "gemm_act", _ptr(x, "gemm_act x"), _ptr(w, "gemm_act w"), _ptr(h, "gemm_act h"), n, m, k,
             dtype_code(x.dtype), int(act), _ptr(params, "gemm_act params", torch.float32, True), _stream())
+
+
+def gemm_rope(x, w, q, rope):
+    """q [n, H head_dim] = the rotated queries of x . w^T on the MFMA tiles, keys and values of the other rows of w appended to the pages
+    (``Rope``), in the product's epilogue; where ``gemm_rope_fits``."""
+    n, k = x.shape
+    m = w.shape[0]
+    if (w.shape[1] != k or x.dtype != w.dtype or tuple(q.shape) != (n, rope.heads * rope.head_dim) or q.dtype != x.dtype
+            or not gemm_rope_fits(m, k, rope.head_dim, x.dtype)):
+        raise KernelError(f"gemm_rope: x {tuple(x.shape)}, w {tuple(w.shape)}, q {tuple(q.shape)} do not fit")
+    lo = _LinearOut()
+    lo.kind, lo.nsplit, lo.f32 = LINEAR_ROPE, 1, int(dtype_code(x.dtype) == DT_F32)
+    _describe_rope(lo, rope, n, x.dtype)
+    lo.y = _ptr(q, "gemm_rope q")
+    _launch("kllm_gemm_rope", "gemm_rope", _ptr(x, "gemm_rope x"), lo, _ptr(w, "gemm_rope w"), n, m, k, _stream())
+
+
+def gemm_rope_fits(m, k, head_dim, dtype):
+    """Whether ``gemm_rope`` takes weights [m, k] and heads of this size."""
+    size = 4 if dtype == torch.float32 else 2
+    return k % (16 // size) == 0 and k < 1 << 23 and m * k * size < 1 << 32 and head_dim % 8 == 0
 
 
 def group_norm_add(x, deltas=(), bias=None, mult=1.0, weight=None, out=None, rows=None, groups=1, eps=0.0,

@@ -30,7 +30,7 @@ import torch
 
 from .. import kernels as K
 from .base import Normed, Part, register_part
-from .linear import decode_linear, fused_f32, linear, linear_into, rows_kernel, sink_takes_rows, tiled_copy
+from .linear import decode_linear, fused_f32, linear, linear_into, one_slice, rows_kernel, sink_takes_rows, tiled_copy
 from .spec import CacheNeed, WeightSpec
 
 
@@ -254,6 +254,11 @@ class CausalSelfAttention(Part):
                            tiles_per_wg=self._fused_tiles(n),
                            rope=K.Rope(cos, sin, pages, ctx.positions, ctx.span_of_token, cache.block_table,
                                        cache.page_size, self.heads, self.kv_heads, self.head_dim))
+        elif (plain_rotation and type(xn) is torch.Tensor and xn.is_contiguous() and one_slice(self.runtime, n, self.w_in)
+              and K.gemm_rope_fits(*self.w_in.shape, self.head_dim, dtype)):
+            # a prompt whose product is one slice: the same on its tiles (slices go to rope_append, which adds them)
+            K.gemm_rope(xn, self.w_in, q, K.Rope(cos, sin, pages, ctx.positions, ctx.span_of_token, cache.block_table,
+                                                 cache.page_size, self.heads, self.kv_heads, self.head_dim))
         else:
             qkv = linear(ctx, xn, self.w_in, "attn.qkv")
             K.rope_append(qkv, q, cos, sin, pages, ctx.positions, ctx.span_of_token,

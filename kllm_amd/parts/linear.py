@@ -298,6 +298,11 @@ def linear_into(ctx, x, w, sink, tag, w_tiled=None):
     return Normed(sink.x, ss, parts, norm, xw=xw)
 
 
+def one_slice(rt, n, w):
+    """Whether a prompt's product (more than 64 rows) runs on the MFMA tiles with all of K in one slice."""
+    return n > 64 and choose(w.dtype, n, *w.shape, rt.options) in ((K.GEMM_MFMA_BF16, 1), (K.GEMM_MFMA_F32, 1))
+
+
 def linear(ctx, x, w, tag, out_dtype=torch.float32, split=True, w_tiled=None):
     """x [n, k] . w [m, k]^T.  With a float32 result and ``split``: partial
     sums [nsplit, n, m] for a consumer that adds them; otherwise one [n, m]

@@ -1699,3 +1699,42 @@ def test_rows_of_whole_pieces_and_odd_ones(n, d, dtype):
     ids[0], ids[n - 1] = 4, 130
     want = table[ids.long()].float() * 3.0
     assert torch.equal(out, want) and torch.equal(copy, want.to(dtype))
+
+
+@pytest.mark.parametrize("H,KV,hd,k", [(4, 2, 64, 256), (3, 1, 128, 192), (5, 5, 8, 72), (2, 1, 72, 1096), (17, 3, 40, 520), (32, 4, 64, 2048)])
+@pytest.mark.parametrize("n", [65, 140, 523, 2100])
+@pytest.mark.parametrize("turned,append", [(True, True), (False, True), (True, False)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_prompt_projections_with_rotation_and_append(H, KV, hd, k, n, turned, append, dtype):
+    """One launch against the product's sums, rotated and appended behind it: tiles of every size with heads across their borders, rows and columns
+    that end inside a tile, K that is no whole stage, two spans in shuffled pages of 24 slots; what is not written stays.  The sums are the same ones, so
+    that an element differs by the rounding of its own last step: a unit of the result's type, and of 32 bits of the pair's terms."""
+    k_ = K()
+    if n == 2100 and (H, KV) not in ((32, 4), (3, 1)):
+        pytest.skip("the large tiles: two of the sizes")
+    g = torch.Generator().manual_seed(hd + n)
+    m = (H + (2 * KV if append else 0)) * hd
+    x, w = torch.randn(n, k, generator=g).to(DEV, dtype), (torch.randn(m, k, generator=g) * k ** -0.5).to(DEV, dtype)
+    ps, first = 24, n // 3
+    pos = torch.cat([torch.arange(first) + 5, torch.arange(n - first)]).to(torch.int32).to(DEV)
+    span = torch.cat([torch.zeros(first), torch.ones(n - first)]).to(torch.int32).to(DEV)
+    per = (n + 5) // ps + 1
+    table = torch.randperm(2 * per, generator=g).to(torch.int32).view(2, per).to(DEV)
+    ang = torch.randn(n, hd // 2, generator=g).to(DEV)
+    cos, sin = (ang.cos(), ang.sin()) if turned else (None, None)
+    got = []
+    for fused in (True, False):
+        q = torch.full((n, H * hd), float("nan"), dtype=dtype, device=DEV)
+        cache = torch.full((2 * per, 2, KV, ps * hd), -7.0, dtype=dtype, device=DEV) if append else None
+        if fused:
+            assert k_.gemm_rope_fits(m, k, hd, dtype)
+            k_.gemm_rope(x, w, q, k_.Rope(cos, sin, cache, pos, span, table, ps, H, KV, hd))
+        else:
+            sums = torch.empty(1, n, m, device=DEV)
+            k_.gemm(x, w, sums, k_.GEMM_MFMA_F32 if dtype == torch.float32 else k_.GEMM_MFMA_BF16, 1)
+            k_.rope_append(sums, q, cos, sin, cache, pos, span, table, ps, H, KV, hd)
+        got.append((q, cache) if append else (q,))
+    for one, other in zip(*got):
+        one, other = one.double(), other.double()
+        assert torch.isfinite(one).all() and torch.equal(one == -7.0, other == -7.0)
+        assert ((one - other).abs() <= (2.0 ** -7 if dtype == torch.bfloat16 else 0.0) * other.abs() + 2.0 ** -21 * other.abs().max()).all()
