@@ -1305,49 +1305,123 @@ __global__ __launch_bounds__(kLatThreads) void latent_query_block_kernel(
   }
 }
 
-// A wave takes 32 outputs and 32 of the tokens, the rank in steps of 16, eight steps' pieces in flight.
-__global__ __launch_bounds__(kLatThreads) void latent_out_block_kernel(
-    const bf16_t* __restrict__ attended, const bf16_t* __restrict__ w_uv, const float* __restrict__ gate, int nsplit,
-    long split_stride, long gate_stride, int by_head, bf16_t* __restrict__ out, int n, int H, int dv, int rank) {
-  constexpr int kAhead = 8;
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  const int g = lane / 32, c = lane % 32;
-  const int h = blockIdx.x, t0 = blockIdx.y * kLatTokens + 32 * (wave % 2);
-  const int j0 = (2 * blockIdx.z + wave / 2) * 32;
-  if (j0 >= dv || t0 >= n) return;
-  const bf16_t* wrow = w_uv + ((long)h * dv + min(j0 + c, dv - 1)) * rank + 8 * g;
-  const bf16_t* arow = attended + ((long)min(t0 + c, n - 1) * H + h) * rank + 8 * g;
-  floatx16 acc = {};
-  const int steps = rank / 16;
-  for (int k0 = 0; k0 < steps; k0 += kAhead) {
-    bf16x8 a[kAhead], b[kAhead];
+// A workgroup takes 64 tokens of a head and 64 U of its outputs, a wave 16 U of those (U 2, or 1 where that leaves CUs without work).  The tokens' rows of up to 512 of the rank go into LDS, a row a load
+// instruction (they lie H rank apart: a matrix operand's lanes would ask for 32 bytes of 32 rows, 32 pages, a load; the tiles of all
+// products, which come back to a row for every 128 bytes, took 8 to 20 us more than that up to 200 tokens),
+// and a wave's weights into registers, all on their way at once.  Chunk j (16 bytes) of row r lies in slot j ^ (r % 16), so that sixteen rows' chunk
+// meets all banks.  Row c of the u-th of a wave's A operands is output 4 U (c / 4) + 4 u + c % 4: a lane then holds 4 U neighbouring
+// outputs of a token.  In us, 32 heads of 128, rank 512, with a gate in one slice, operands by lane before and now: 64 tokens 11.8 -> 9.1, 200 12.2 ->
+// 9.4, 260 21.0 -> 12.3, 400 21.5 -> 12.7, 700 31.1 -> 20.8, 1,500 60.4 -> 33.4, in four slices 17.1 -> 11.5, 17.9 -> 13.7, 31.0 -> 17.5, 31.8 -> 19.3, 48.1 ->
+// 29.9, 96.7 -> 47.7; U 2 / 1: 200 tokens 13.1 / 9.4, 400 13.6 / 12.7, 520 (288 workgroups of U 2) 16.1 / 19.8, 1,500 33.4 / 40.3.
+constexpr int kOutChunk = 512;
+template <int U>
+__global__ __launch_bounds__(kLatThreads, 2) void latent_out_block_kernel(
+    const bf16_t* __restrict__ attended, const bf16_t* __restrict__ w_uv, int n, int H, int dv, int rank, const float* __restrict__ gate, long gate_stride,
+    int nsplit, int by_head, long split_stride, bf16_t* __restrict__ out) {
+  constexpr int STEPS = kOutChunk / 32, TB = kLatTokens / 16;
+  __shared__ __attribute__((aligned(1024))) bf16_t rows[kLatTokens * kOutChunk];
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int g = lane / 16, c = lane % 16;
+  const int h = blockIdx.x, t0 = blockIdx.y * kLatTokens, j0 = 16 * U * (4 * blockIdx.z + wave);
+  const bf16_t* wrow[U];
 #pragma unroll
-    for (int k = 0; k < kAhead; ++k) {
-      const int at = 16 * min(k0 + k, steps - 1);
-      a[k] = *reinterpret_cast<const bf16x8*>(wrow + at);
-      b[k] = *reinterpret_cast<const bf16x8*>(arow + at);
+  for (int u = 0; u < U; ++u) wrow[u] = w_uv + ((long)h * dv + min(j0 + 4 * U * (c / 4) + 4 * u + c % 4, dv - 1)) * rank;
+  floatx4 acc[TB][U];
+#pragma unroll
+  for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc[tb][u] = floatx4{0.f, 0.f, 0.f, 0.f};
+  typedef float anywhere4 __attribute__((ext_vector_type(4), aligned(4)));
+  auto opened = [&](int s, floatx4 (&z)[TB][U]) {           // a slice of the gate's sums for this lane's outputs
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb) {
+      const float* at = gate + s * split_stride + min(t0 + 16 * tb + c, n - 1) * gate_stride;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (by_head) {
+          const float one = at[h];
+          z[tb][u] = floatx4{one, one, one, one};
+        } else {                                              // (pieces behind the head's outputs: its last one, not used)
+          const int j = j0 + 4 * U * g + 4 * u;
+          if (dv % 4 == 0) {
+            z[tb][u] = *reinterpret_cast<const anywhere4*>(at + (long)h * dv + min(j, dv - 4));
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) z[tb][u][e] = at[(long)h * dv + min(j + e, dv - 1)];
+          }
+        }
+      }
     }
+  };
+  floatx4 z[TB][U];
+  for (int k0 = 0; k0 < rank; k0 += kOutChunk) {
+    const int width = min(rank - k0, kOutChunk), chunks = width / 8;       // rank % 16 == 0 (the launch)
+    if (k0) __syncthreads();
 #pragma unroll
-    for (int k = 0; k < kAhead; ++k)
-      if (k0 + k < steps) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[k], b[k], acc, 0, 0, 0);
+    for (int i = 0; i < kLatTokens / 4; ++i) {
+      const int r = 4 * i + wave, chunk = lane ^ (r % 16);                // (chunks that are not there are never read)
+      const bf16_t* src = attended + ((long)min(t0 + r, n - 1) * H + h) * rank + k0 + 8 * (chunk < chunks ? chunk : 0);
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                       (__attribute__((address_space(3))) void*)(rows + r * kOutChunk), 16, 0, 0);
+    }
+    bf16x8 w[U][STEPS];
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+      for (int u = 0; u < U; ++u) w[u][s] = *reinterpret_cast<const bf16x8*>(wrow[u] + k0 + (32 * s + 8 * g < width ? 32 * s + 8 * g : 0));
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+      for (int u = 0; u < U; ++u) asm volatile("" : "+v"(w[u][s]));       // (here, not step by step behind the barrier)
+    if (U == 1 && gate && k0 == 0) opened(0, z);           // (two operands' weights leave no registers for it)
+    __syncthreads();                                       // (the rows are there: it waits for every load)
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+      if (32 * s >= width) break;
+      const bool there = 32 * s + 8 * g < width;             // (half a step where the rank is no multiple of 32: zeros)
+      const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+      for (int tb = 0; tb < TB; ++tb) {
+        const int r = 16 * tb + c;
+        bf16x8 b = *reinterpret_cast<const bf16x8*>(rows + r * kOutChunk + 8 * ((4 * s + g) ^ c));
+        b = there ? b : zero;
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc[tb][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(there ? w[u][s] : zero, b, acc[tb][u], 0, 0, 0);
+      }
+    }
   }
-  const int t = t0 + c;
-  if (t >= n) return;
+  constexpr int E = 4 * U;
+  if (j0 + E * g >= dv) return;
+  typedef bf16_t piece __attribute__((ext_vector_type(E)));
+  const bool whole = dv % E == 0 && ((unsigned long)out & (2 * E - 1)) == 0;
+  if (U > 1 && gate) opened(0, z);
+  for (int s = 1; gate && s < nsplit; ++s) {                  // (a slice's sums all together)
+    floatx4 more[TB][U];
+    opened(s, more);
 #pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    const int j = j0 + 8 * b + 4 * g;
-    if (j >= dv) continue;                                    // dv in steps of 4 (the launch)
-    float z[4] = {0.f, 0.f, 0.f, 0.f};
-    if (gate) {
-      const float* at = gate + t * gate_stride + (by_head ? h : (long)h * dv + j);
-      for (int s = 0; s < nsplit; ++s)
+    for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) z[e] += at[s * split_stride + (by_head ? 0 : e)];
+      for (int u = 0; u < U; ++u) z[tb][u] += more[tb][u];
+  }
+#pragma unroll
+  for (int tb = 0; tb < TB; ++tb) {
+    const int t = t0 + 16 * tb + c;
+    if (t >= n) continue;
+    piece v;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      float a = acc[tb][e / 4][e % 4];
+      if (gate) a *= sigmoid_f32(z[tb][e / 4][e % 4]);
+      v[e] = (bf16_t)a;
     }
-    bf16x4 v;
+    bf16_t* dst = out + ((long)t * H + h) * dv + j0 + E * g;
+    if (whole) {
+      *reinterpret_cast<piece*>(dst) = v;
+    } else {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = (bf16_t)(gate ? acc[4 * b + e] * sigmoid_f32(z[e]) : acc[4 * b + e]);
-    *reinterpret_cast<bf16x4*>(out + ((long)t * H + h) * dv + j) = v;
+      for (int e = 0; e < E; ++e)
+        if (j0 + E * g + e < dv) dst[e] = v[e];
+    }
   }
 }
 
@@ -1500,11 +1574,14 @@ extern "C" int kllm_latent_out(const void* attended, const void* w_uv, const flo
   KLLM_REQUIRE(n > 0 && H > 0 && H <= 65535 && dv > 0 && rank > 0 && rank <= 8192 && (!gate || nsplit >= 1),
                "latent_out: bad sizes n=%d H=%d dv=%d rank=%d", n, H, dv, rank);
   KLLM_REQUIRE(dtype == DT_F32 || dtype == DT_BF16, "latent_out: unknown dtype %d", dtype);
-  if (dtype == DT_BF16 && n >= kLatTokens && rank % 16 == 0 && dv % 4 == 0 && ((uintptr_t)attended & 15) == 0 &&
-      ((uintptr_t)w_uv & 15) == 0 && ((uintptr_t)out & 7) == 0 && (n + kLatTokens - 1) / kLatTokens <= 65535) {
-    hipLaunchKernelGGL(latent_out_block_kernel, dim3(H, (n + kLatTokens - 1) / kLatTokens, (dv + 63) / 64), dim3(kLatThreads), 0,
-                       stream, (const bf16_t*)attended, (const bf16_t*)w_uv, gate, nsplit, split_stride, gate_stride,
-                       gate_by_head, (bf16_t*)out, n, H, dv, rank);
+  if (dtype == DT_BF16 && n >= kLatTokens && rank % 16 == 0 && ((uintptr_t)attended & 15) == 0 && ((uintptr_t)w_uv & 15) == 0 &&
+      (n + kLatTokens - 1) / kLatTokens <= 65535 && (dv + 63) / 64 <= 65535) {
+    const dim3 grid(H, (n + kLatTokens - 1) / kLatTokens, (dv + 127) / 128), halves(H, grid.y, (dv + 63) / 64);
+#define KLLM_LO(U, G)                                                                                                             \
+  hipLaunchKernelGGL(latent_out_block_kernel<U>, G, dim3(kLatThreads), 0, stream, (const bf16_t*)attended, (const bf16_t*)w_uv, n, H, dv, \
+                     rank, gate, gate_stride, nsplit, gate_by_head, split_stride, (bf16_t*)out)
+    if ((long)H * grid.y * grid.z <= device_cus()) KLLM_LO(1, halves); else KLLM_LO(2, grid);
+#undef KLLM_LO
     KLLM_CHECK_LAUNCH("latent_out");
     return 0;
   }
