@@ -15,14 +15,9 @@ namespace kllm {
 constexpr int kSampleThreads = 1024;
 constexpr int kSampleWaves = kSampleThreads / kWave;
 
-// (value, index) with the larger value, the smaller index on equal values
-__device__ __forceinline__ void better(float& v, int& i, float ov, int oi) {
-  if (ov > v || (ov == v && oi < i)) {
-    v = ov;
-    i = oi;
-  }
-}
-
+// One workgroup a row: a row's logits come in one trip (up to 32,768; 128,256 in four), and what follows is a chain of lane exchanges, so
+// the maximum goes by data-parallel moves and its place by asking the lanes that have it: 8 rows of 32,000 8.9 -> 5.7 us (contiguous segments a
+// thread and twelve exchanges through LDS a wave before).
 __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
     int* __restrict__ out, const float* __restrict__ logits, const float* __restrict__ temperature,
     const float* __restrict__ uniform, int vocab) {
@@ -36,51 +31,52 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   // (asked for here, so that the trip to memory runs beside the logits')
   const float temp = temperature ? temperature[r] : 0.f;
   const float u = uniform ? uniform[r] : 0.f;
-  // Each thread owns one contiguous segment, so thread order is index order.
-  // Segments are multiples of four logits, so that a row whose length is one too is read
-  // in 16-byte pieces, eight of them in flight per thread.
+  // For the sums, and the maximum of a row in no whole pieces, each thread owns one contiguous segment, so thread order is index order.
   const int seg = (vocab + 4 * kSampleThreads - 1) / (4 * kSampleThreads) * 4;
   const int lo = min(tid * seg, vocab), hi = min(lo + seg, vocab);
 
+  // The greatest logit and the first place that has it (numbers only: a NaN is never chosen before one that is none).
   float bv = -INFINITY;
   int bi = vocab;  // "none": loses against every index
   if (vocab % 4 == 0 && ((uintptr_t)logits & 15) == 0) {
-    for (int i0 = lo; i0 < hi; i0 += 32) {
+    // pieces of 16 bytes, neighbouring threads side by side, eight of them in flight a thread
+    const int pieces = vocab / 4;
+    for (int p0 = tid; p0 < pieces; p0 += 8 * kSampleThreads) {
       floatx4 v[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        v[j] = i0 + 4 * j < hi ? *reinterpret_cast<const floatx4*>(row + i0 + 4 * j)
-                               : floatx4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const floatx4*>(row + 4 * min(p0 + j * kSampleThreads, pieces - 1));
 #pragma unroll
       for (int j = 0; j < 8; ++j)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int i = i0 + 4 * j + e;
-          if (i < hi && (bi == vocab || v[j][e] > bv)) { bv = v[j][e]; bi = i; }   // strict: the first maximum stays
+          const int i = 4 * (p0 + j * kSampleThreads) + e;
+          if (i < vocab && (v[j][e] > bv || (bi == vocab && v[j][e] == bv))) { bv = v[j][e]; bi = i; }   // strict: the first maximum stays
         }
     }
   } else {
     for (int i = lo; i < hi; ++i) {
       const float v = row[i];
-      if (bi == vocab || v > bv) { bv = v; bi = i; }
+      if (v > bv || (bi == vocab && v == bv)) { bv = v; bi = i; }
     }
   }
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) {
-    const float ov = __shfl_xor(bv, off, kWave);
-    const int oi = __shfl_xor(bi, off, kWave);
-    if (oi < vocab && (bi == vocab || ov > bv || (ov == bv && oi < bi))) { bv = ov; bi = oi; }
-  }
+  // Maxima by data-parallel moves; then the lanes that have it, mostly one, are asked for their places.
+  auto first_of = [&](float v, int i, float greatest) {
+    int best = vocab;
+    for (unsigned long m = __builtin_amdgcn_ballot_w64(v == greatest); m; m &= m - 1) best = min(best, __builtin_amdgcn_readlane(i, __builtin_ctzl(m)));
+    return best;
+  };
+  const float wm = wave_max(bv);
+  const int wi = first_of(bv, bi, wm);
   if (lane == 0) {
-    wave_val[wave] = bv;
-    wave_idx[wave] = bi;
+    wave_val[wave] = wm;
+    wave_idx[wave] = wi;
   }
   if (tid == 0) chosen = vocab - 1;
   __syncthreads();
-  float mx = wave_val[0];
-  int arg = wave_idx[0];
-  for (int w = 1; w < kSampleWaves; ++w)
-    if (wave_idx[w] < vocab && (arg == vocab || wave_val[w] > mx)) { mx = wave_val[w]; arg = wave_idx[w]; }
+  const float wv = wave_val[lane % kSampleWaves];
+  const float mx = wave_max(wv);
+  int arg = first_of(wv, wave_idx[lane % kSampleWaves], mx);
+  if (arg == vocab) arg = 0;      // nothing but NaN
   if (!(temp > 0.f)) {
     if (tid == 0) out[r] = arg;
     return;

@@ -1738,3 +1738,30 @@ def test_prompt_projections_with_rotation_and_append(H, KV, hd, k, n, turned, ap
         one, other = one.double(), other.double()
         assert torch.isfinite(one).all() and torch.equal(one == -7.0, other == -7.0)
         assert ((one - other).abs() <= (2.0 ** -7 if dtype == torch.bfloat16 else 0.0) * other.abs() + 2.0 ** -21 * other.abs().max()).all()
+
+
+@pytest.mark.parametrize("vocab", [1, 4, 63, 4096, 32000, 32003, 131072, 128256])
+def test_sample_greedy_places(vocab):
+    """The first of several equal maxima wherever they lie (one thread's pieces, a wave's, the workgroup's; whole pieces of four and not), the last
+    place, rows of the lowest value, of infinities, and NaN beside numbers: the first of the greatest numbers."""
+    g = torch.Generator().manual_seed(vocab)
+    rows, want = [], []
+    for k in range(12):
+        row = torch.randn(vocab, generator=g)
+        if k == 0:
+            row.fill_(-float("inf"))
+        elif k == 1:
+            row[vocab - 1] = 9.0
+        elif k == 2:
+            row[:] = float("inf")
+        elif k == 3:
+            row[torch.rand(vocab, generator=g) < 0.5] = float("nan")
+            row[vocab // 2] = 1.5
+        else:
+            row[torch.randint(0, vocab, (k,), generator=g)] = 7.0
+        rows.append(row)
+        m = row[~row.isnan()].max()
+        want.append(int((row == m).nonzero()[0]))
+    out = torch.full((12,), -1, dtype=torch.int32, device=DEV)
+    K().sample(out, torch.stack(rows).to(DEV))
+    assert out.tolist() == want
