@@ -1637,6 +1637,32 @@ def test_attention_decode_places_float32(H, KV, hd, ps, window):
             assert torch.isfinite(out).all() and err < 2e-5, (ns, float(err))
 
 
+@pytest.mark.parametrize("hd", [32, 64, 96, 128])
+@pytest.mark.parametrize("H", [1, 2, 17])
+@pytest.mark.parametrize("slices", [1, 4, 8])
+def test_attention_decode_weights_float32(hd, H, slices):
+    """Every weight of a float32 token to 32 bits, the small ones too: key j's score lies x_j (0 to -83, no rounding in it) from key 0's and its value is
+    1 in column j alone, so that an output is exp(x_j) over the sum.  What rounds, in units of 2^-24 of an element: two exponentials (of the wave's keys, of the waves or
+    slices), 4 each by their bound of 2 ulp; the sum, whose 32 largest terms are added one behind the other at most, no more than 8; the
+    reciprocal and four products 6.  In base 2, x_j log2(e) rounded once would be off by up to |x_j| of them."""
+    x = -(83.0 * torch.arange(hd) / hd).to(torch.float32)
+    scale, ps = 0.125, 16
+    pages = hd // ps
+    table = torch.arange(pages, dtype=torch.int32, device=DEV).flip(0).contiguous()
+    cache = torch.zeros(pages, 2, 1, ps * hd, device=DEV)
+    for j in range(hd):
+        page = int(table[j // ps])
+        cache[page, 0, 0].view(ps, hd)[j % ps, 0] = 8.0 * x[j]
+        cache[page, 1, 0].view(hd, ps)[j, j % ps] = 1.0
+    q = torch.zeros(1, H * hd, device=DEV)
+    q.view(H, hd)[:, 0] = 1.0
+    one = lambda v: torch.tensor([v], dtype=torch.int32, device=DEV)
+    out = run_attention("decode", q, cache, one(hd - 1), one(0), table.view(1, -1), ps, H, 1, hd, 0, scale, nslices=slices)
+    want = torch.softmax(x.double(), 0)
+    err = (out.cpu().double().view(H, hd) / want - 1).abs().max()
+    assert err < 24 * 2.0 ** -24, float(err) * 2 ** 24
+
+
 @pytest.mark.parametrize("dk,dv,rot", [(32, 36, 8), (64, 64, 32), (128, 128, 128), (256, 100, 0), (64, 12, 48)])
 @pytest.mark.parametrize("n,nsplit", [(1, 1), (17, 3), (700, 1)])
 @pytest.mark.parametrize("norm", ["unit", "weights", "none"])
