@@ -71,13 +71,14 @@ __device__ __forceinline__ void attn_merge_wide(T* __restrict__ out, const float
   const int row = (hd + 2) * (int)sizeof(float);
   const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<char*>(reinterpret_cast<const char*>(part)) + ((long)t * H + h) * nslices * row, 0, nslices * row, 0x00020000);
-  auto load = [&](int at, int slice_at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rows, at, slice_at, 0)); };
-  const float ms0 = load(lane * row + 4 * hd, 0), ls = load(lane * row + 4 * hd + 4, 0);
+  // (all of a place in the vector offset, which the descriptor's end is held against; a scalar one need not be)
+  auto load = [&](int at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rows, at, 0, 0)); };
+  const float ms0 = load(lane * row + 4 * hd), ls = load(lane * row + 4 * hd + 4);
   float os[DV][R];
 #pragma unroll
   for (int j = 0; j < R; ++j)
 #pragma unroll
-    for (int v = 0; v < DV; ++v) os[v][j] = load(4 * (lane + 64 * v < hd ? lane + 64 * v : 0), j * row);
+    for (int v = 0; v < DV; ++v) os[v][j] = load(4 * (lane + 64 * v < hd ? lane + 64 * v : 0) + j * row);
   __builtin_amdgcn_sched_barrier(0);
   const int side = gate.side;
   asm volatile("" ::"s"(side), "s"(gate.sums), "s"(gate.width), "s"(H));     // (now: in front of the stores it was a trip to memory of its own)

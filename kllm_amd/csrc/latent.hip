@@ -1031,13 +1031,14 @@ __global__ __launch_bounds__(kLatThreads) void attn_latent_merge_kernel(const fl
   const long th = blockIdx.x;
   const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<char*>(reinterpret_cast<const char*>(part)) + th * nslices * bytes, 0, nslices * bytes, 0x00020000);
-  auto load = [&](int at, int slice_at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rows, at, slice_at, 0)); };
-  const float m0 = load(lane * bytes + 4 * rank, 0), ls = load(lane * bytes + 4 * rank + 4, 0);      // (beyond the last slice zeros, from nowhere)
+  // (beyond the last slice zeros, from nowhere: all of a place is in the vector offset, which the descriptor's end is held against)
+  auto load = [&](int at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rows, at, 0, 0)); };
+  const float m0 = load(lane * bytes + 4 * rank), ls = load(lane * bytes + 4 * rank + 4);
   float v[2][R];
 #pragma unroll
   for (int j = 0; j < R; ++j)
 #pragma unroll
-    for (int e = 0; e < 2; ++e) v[e][j] = load(4 * min((int)threadIdx.x + e * kLatThreads, rank - 1), j * bytes);
+    for (int e = 0; e < 2; ++e) v[e][j] = load(4 * min((int)threadIdx.x + e * kLatThreads, rank - 1) + j * bytes);
   __builtin_amdgcn_sched_barrier(0);
   const float ms = lane < nslices ? m0 : -INFINITY;
   const float M = first_lanes_max<R>(ms);                     // finite: some slice holds the token's own key

@@ -1663,6 +1663,26 @@ def test_attention_decode_weights_float32(hd, H, slices):
     assert err < 24 * 2.0 ** -24, float(err) * 2 ** 24
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_attention_merge_reads_its_own_slices(hd, dtype):
+    """3, 17 and 33 workgroups' partial results to a head, which the merge asks for in 16, 32 and 64 rows: what lies behind a head's own, the next
+    head's (NaN here: its values are), the next token's or the room behind the last, leaves it as it is."""
+    H, KV, ps = 4, 2, 16
+    c = attention_case(H, KV, hd, ps, dtype, 0, [(699, 1), (520, 1), (650, 1)], seed=5)
+    cache, per = c["cache"].clone(), 4 if dtype == torch.float32 else 1      # (float32: four slices to a workgroup)
+    cache[c["tables"][0][:44], 1, 1] = float("nan")
+    cache[c["tables"][1][:33], 1] = float("nan")
+    for slices in (3 * per, 17 * per, 33 * per):
+        out = torch.full_like(c["q"], 7.0)
+        part = torch.full((3 * H * slices * (hd + 2) + 64 * (hd + 2),), float("nan"), device=DEV)
+        K().attn_decode(c["q"], out, part, cache, c["pos"], c["sot"], c["bt"], ps, H, KV, hd, 0, c["scale"], slices)
+        got = out.cpu().double()
+        assert got[0, 2 * hd:].isnan().all() and got[1].isnan().all()
+        for rows in ((0, slice(0, 2 * hd)), (2, slice(0, H * hd))):
+            assert (got[rows] - c["want"][rows]).abs().max() < attn_tol(dtype), (slices, rows)
+
+
 @pytest.mark.parametrize("dk,dv,rot", [(32, 36, 8), (64, 64, 32), (128, 128, 128), (256, 100, 0), (64, 12, 48)])
 @pytest.mark.parametrize("n,nsplit", [(1, 1), (17, 3), (700, 1)])
 @pytest.mark.parametrize("norm", ["unit", "weights", "none"])

@@ -372,6 +372,35 @@ def test_attention_through_latents_round_by_round(H, row, rank, page, window):
             assert rel(got[s], want[s]) < 2 ** -7, (slices, s, rel(got[s], want[s]))
 
 
+def test_the_merge_of_latent_slices_reads_its_own():
+    """Three tokens' partial results in 3, 17 and 33 slices, the second's keys NaN and room behind the last: the others are what they are alone."""
+    from kllm_amd import kernels as K
+    g = torch.Generator().manual_seed(3)
+    H, row, rank, page, lens = 3, 104, 96, 16, [300, 290, 270]
+    per = -(-max(lens) // page)
+    cache = torch.zeros(3 * per, page * (row + rank))
+    keys = []
+    for s, n in enumerate(lens):
+        keys.append(torch.randn(n, row, generator=g).bfloat16())
+        for p in range(-(-n // page)):
+            here = keys[s][p * page:(p + 1) * page].float()
+            cache[s * per + p, :page * row].view(page, row)[:len(here)] = here
+            cache[s * per + p, page * row:].view(rank, page)[:, :len(here)] = here[:, :rank].T
+    cache[per:2 * per] = float("nan")
+    q = torch.randn(3, H, row, generator=g).bfloat16()
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    for slices in (3, 17, 33):
+        out = torch.full((3, H * rank), 7.0, dtype=torch.bfloat16, device="cuda")
+        part = torch.full(((3 * H * slices + 64) * (rank + 2),), float("nan"), device="cuda")
+        K.attn_latent(q.view(3, -1).cuda(), out, cache.bfloat16().cuda(), i32([n - 1 for n in lens]), i32([0, 1, 2]),
+                      i32(list(range(3 * per))).view(3, per), page, H, row, rank, row ** -0.5, part=part, nslices=slices)
+        got = out.float().cpu().view(3, H, rank)
+        assert got[1].isnan().all()
+        for s in (0, 2):
+            want = torch.softmax(q[s].double() @ keys[s].double().T * row ** -0.5, -1) @ keys[s].double()[:, :rank]
+            assert rel(got[s], want) < 2 ** -7, (slices, s)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("n,H,d,dr,dv,rank", [(1, 3, 16, 8, 20, 40), (37, 6, 64, 32, 64, 160), (130, 3, 128, 64, 128, 448),
                                               (5, 20, 32, 16, 24, 96), (70, 2, 96, 8, 200, 64)])
