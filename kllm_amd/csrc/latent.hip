@@ -402,7 +402,7 @@ __global__ __launch_bounds__(64 * kLatWaves) void attn_latent_mfma_kernel(
       } else {
         for (int i = threadIdx.x; i < 64 * steps; i += 64 * kLatWaves) q_store(i, q_load(i));
       }
-      // (what is in LDS, not what is on its way from memory: __syncthreads would wait for the keys)
+      // (a wait for what goes to LDS and for nothing else, written out: the keys stay on their way)
       asm volatile("" ::: "memory");
       __builtin_amdgcn_s_waitcnt(0xC07F);
       __builtin_amdgcn_s_barrier();
@@ -1405,7 +1405,8 @@ __global__ __launch_bounds__(kLatThreads, 2) void latent_out_block_kernel(
 #pragma unroll
       for (int u = 0; u < U; ++u) asm volatile("" : "+v"(w[u][s]));       // (here, not step by step behind the barrier)
     if (U == 1 && gate && k0 == 0) opened(0, z);           // (two operands' weights leave no registers for it)
-    __syncthreads();                                       // (the rows are there: it waits for every load)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // this wave's rows are in LDS: a barrier alone waits for no load from memory
+    __syncthreads();
 #pragma unroll
     for (int s = 0; s < STEPS; ++s) {
       if (32 * s >= width) break;
