@@ -2,7 +2,9 @@
 
 import os
 import re
+import struct
 
+import msgpack
 import pytest
 
 from kllm_amd.csrc import build
@@ -20,3 +22,36 @@ def test_loads_into_lds_are_waited_for_in_front_of_a_barrier(name):
         barrier = re.search(r"__syncthreads\(\)|_barrier\(\)", rest)
         assert barrier is None or not barrier.group().startswith("__sync") or "s_waitcnt" in rest[:barrier.start()], \
             text[:load.start()].count("\n") + 1
+
+
+def kernels_of(library):
+    """What the compiler wrote about the kernels in the library (code objects in offload bundles, their notes): by mangled name."""
+    data, at, found = open(library, "rb").read(), -1, {}
+    while (at := data.find(b"__CLANG_OFFLOAD_BUNDLE__", at + 1)) >= 0:
+        place, (count,) = at + 32, struct.unpack_from("<Q", data, at + 24)
+        for _ in range(count if count < 8 else 0):               # (more: the name itself, in host code)
+            offset, size, length = struct.unpack_from("<QQQ", data, place)
+            target, place = data[place + 24:place + 24 + length], place + 24 + length
+            if b"gfx950" not in target:
+                continue
+            elf = data[at + offset:at + offset + size]
+            (sections,), (step, number) = struct.unpack_from("<Q", elf, 0x28), struct.unpack_from("<HH", elf, 0x3A)
+            for i in range(number):
+                kind, = struct.unpack_from("<I", elf, sections + i * step + 4)
+                note, end = struct.unpack_from("<QQ", elf, sections + i * step + 0x18)
+                end += note
+                while kind == 7 and note < end:                  # notes
+                    name, text, type_ = struct.unpack_from("<III", elf, note)
+                    note += 12 + (name + 3) // 4 * 4
+                    if type_ == 32:
+                        found.update((k[".name"], k) for k in msgpack.unpackb(elf[note:note + text])["amdhsa.kernels"])
+                    note += (text + 3) // 4 * 4
+    return found
+
+
+@pytest.mark.parametrize("kernel,instances", [("attn_latent_mfma_kernel", 7), ("attn_f32_decode_kernel", 4), ("attn_decode_mfma_kernel", 60)])
+def test_kernels_whose_registers_all_fit(kernel, instances):
+    """Instances that hold a round's operands in registers, up to all 512 of a lane: none of them goes by way of memory."""
+    own = [k for name, k in kernels_of(build.ensure_built()).items() if kernel in name]
+    assert len(own) >= instances
+    assert not [(k[".name"], k[".vgpr_spill_count"]) for k in own if k[".vgpr_spill_count"] or k[".private_segment_fixed_size"]]
