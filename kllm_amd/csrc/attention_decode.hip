@@ -408,9 +408,9 @@ static int decode_resident(int hdt, int heads, bool whole) {
 
 using namespace kllm;
 
-extern "C" int kllm_attn_decode_slices(int n, int KV, int H, int hd, int dtype, int max_keys) {
+extern "C" int kllm_attn_decode_slices(int n, int KV, int H, int hd, int dtype, int max_keys, int page_size) {
   if (KV <= 0 || H <= 0 || n <= 0 || hd <= 0) return 1;
-  if (dtype == DT_F32) return attn_f32_slices(n, KV, H, hd, max_keys);
+  if (dtype == DT_F32) return attn_f32_slices(n, KV, H, hd, max_keys, page_size);
   // Three quarters as many token x KV head x head tile groups as CUs, or more: one workgroup
   // takes all keys of its group and writes the output.  Otherwise workgroups of four waves
   // that each leave a partial result: about two per CU across the chip, their number per

@@ -666,18 +666,38 @@ bool attn_f32_fits(int hd, int page_size) {
 
 extern "C" int kllm_attn_f32_fits(int hd, int page_size) { return attn_f32_fits(hd, page_size) ? 1 : 0; }
 
-int attn_f32_slices(int n, int KV, int H, int hd, int max_keys) {
+// Whether a decode token's keys go by attn_f32_decode_kernel, on 16 columns.
+static bool f32_sixteen(int H, int KV, int hd, int page_size) {
+  return H / KV <= 16 && hd % 32 == 0 && hd <= 128 && page_size % 16 == 0 && KV <= 65535;
+}
+
+int attn_f32_slices(int n, int KV, int H, int hd, int max_keys, int page_size) {
   // About four waves per CU across the chip, shared out over tokens x KV heads x blocks of 32 heads; a slice is one wave and should have
   // 32 keys at least (one token at 32,768 keys 47 us with 256 against 69 with 64, on 32 columns; on 16, in us with the merge in a replayed graph:
   // 8 tokens x 4 KV heads of 64 at 1,000 keys 17.1 / 13.0 / 10.0 / 7.5 / 7.9 with 4 / 8 / 16 / 32 / 64; 16 x 8 of 128 41.6 / 30.9 / 37.3 / 35.2 / 40.1).
-  // From one group per CU on eight on 32 columns (64 tokens at 2,048 keys 61 us with 8 slices against 68 with 4) and on 16 the four of one workgroup,
-  // which leave nothing to merge (4 / 8 slices: 64 tokens x 4 KV heads of 64 at 1,000 keys 24.2 / 28.2, at 256 8.5 / 9.8; 8 x 32 of 128 at 1,000 50.2 / 57.4,
-  // at 256 20.4 / 19.4).
   const int col_blocks = (H / KV + 31) / 32;
   const long groups = (long)n * KV * col_blocks;
   const int cus = device_cus();
   long want = (groups >= cus ? 8L : 4L) * cus / (groups > 0 ? groups : 1);
-  if (groups >= cus && H / KV <= 16 && hd % 32 == 0 && hd <= 128 && want > kF32Waves) want = kF32Waves;
+  const long keys = max_keys > 0 ? max_keys : 2048;          // (of a table's width, up to twice the context's)
+  if (groups >= cus && f32_sixteen(H, KV, hd, page_size)) {
+    // From one group per CU on, on 16 columns, the four slices of one workgroup, which leave nothing to merge (4 / 8 slices: 64 tokens x 4 KV heads of 64 at 250
+    // keys 9.8 / 10.9, at 32,768 742 / 746; 8 x 32 of 128 at 250 19.9 / 20.7, at 6,000 282 / 286).  Unless the CUs' last round of workgroups is at least
+    // half empty and the keys are many: then eight, or sixteen, where that shortens it once more (4 / 8 / 16 slices, groups per CU 1 1/8, 1 1/2, 2 1/8, 3 1/2: heads of 64
+    // at 2,048 keys 70.7 / 60.6 / 56.0, 80.2 / 75.4 / 77.2, 120 / 110 / 107, 171 / 167 / 170, at 6,000 222 / 183 / 169, 238 / 211 / 212, 354 / 322 / 297,
+    // 501 / 481 / 464; of 128 at 2,048 169 / 143 / 139, 175 / 157 / 172, 265 / 246 / 254, 375 / 352 / 385, at 6,000 479 / 386 / 338, 499 / 424 / 420, 747 /
+    // 659 / 632, 1,035 / 967 / 989; 4 / 8 at 600 59.8 / 57.1, 61.6 / 64.1, 95.1 / 99.9, 136 / 152, at 1,000 85.8 / 79.2, 95.1 / 90.6, 143 / 141, 197 / 205).
+    auto rounds = [&](long workgroups) { return ceil_div(groups * workgroups, cus); };
+    const bool few = 4 * groups <= 5L * cus;                 // a quarter of a second round at most
+    want = kF32Waves;
+    if (groups <= 4L * cus && keys >= (few ? 1024 : 2048) && rounds(2) < 2 * rounds(1))
+      want = (keys >= (few ? 4096 : 8192) && rounds(4) < 2 * rounds(2) ? 4 : 2) * kF32Waves;
+  } else if (groups == cus && H / KV <= 16 && hd % 32 == 0 && hd <= 128 && (hd > 64 || keys <= 768)) {
+    // On 32 columns eight waves a CU (heads of 64, pages of 20 slots, 4 / 8 slices: at 1,000 keys 41.2 / 40.7, at 6,000 200 / 182; of 128, 1 1/8 groups per
+    // CU, 4 / 7: at 2,048 222 / 158), but in whole rounds four of large heads (128, one group per CU: at 600 46.0 / 63.4, at 6,000 321 / 335) and of few
+    // keys (64: at 250 16.4 / 19.2, at 600 28.2 / 31.9).
+    want = kF32Waves;
+  }
   long most = max_keys > 0 ? max_keys / 32 : 64;
   if (most > kAttnF32MaxSlices) most = kAttnF32MaxSlices;
   // Up to 128 keys (a tile of 32 a wave) the second kernel costs more than the keys: one workgroup's four
@@ -714,7 +734,7 @@ int attn_f32_decode(const float* q, float* out, float* part, const float* cache,
   // The kernel of 16 columns takes a workgroup's four slices at a time, whatever their number (no more partial results than
   // the slices that ``part`` has room for).
   const int wgs = (nslices + kF32Waves - 1) / kF32Waves;
-  if (H / KV <= 16 && hd % 32 == 0 && hd <= 128 && page_size % 16 == 0 && KV <= 65535) {
+  if (f32_sixteen(H, KV, hd, page_size)) {
     if (hd == 32) launch_f32_decode<2>(a, wgs, stream);
     else if (hd == 64) launch_f32_decode<4>(a, wgs, stream);
     else if (hd == 96) launch_f32_decode<6>(a, wgs, stream);

@@ -31,7 +31,7 @@ int attn_f32_prefill(const float* q, float* out, const float* cache, const int* 
                      const OutGate& gate, hipStream_t stream);
 
 // Slices proposed for a decode batch of n tokens whose longest request has at most max_keys
-// keys (0: unknown).
-int attn_f32_slices(int n, int KV, int H, int hd, int max_keys);
+// keys (0: unknown), in pages of page_size slots.
+int attn_f32_slices(int n, int KV, int H, int hd, int max_keys, int page_size);
 
 }  // namespace kllm

@@ -248,9 +248,9 @@ int kllm_attn_generic(const void* q, void* out, const void* cache, const int* po
  * n*H*nslices*(hd+2) elements (one slice, and in float32 four, write the output at once
  * and leave it untouched).  kllm_attn_decode_slices proposes nslices for a batch
  * whose longest request has at most max_keys keys (0: unknown, as for contexts
- * of 2,048).  With token_list only the n_listed tokens it names are computed (q,
+ * of 2,048), in pages of page_size slots.  With token_list only the n_listed tokens it names are computed (q,
  * out and part stay indexed by token row). */
-int kllm_attn_decode_slices(int n, int KV, int H, int hd, int dtype, int max_keys);
+int kllm_attn_decode_slices(int n, int KV, int H, int hd, int dtype, int max_keys, int page_size);
 /* Whether the float32 attention on the matrix cores takes this head size and page size. */
 int kllm_attn_f32_fits(int hd, int page_size);
 /* `chunk`, `sinks`, `keep_first` and the gate in kllm_attn_decode and kllm_attn_prefill: as in kllm_attn_generic

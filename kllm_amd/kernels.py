@@ -21,7 +21,7 @@ import torch
 DT_F32, DT_BF16 = 0, 1
 GEMM_PLAIN, GEMM_TILED_F32, GEMM_MFMA_BF16, GEMM_SKINNY_BF16, GEMM_GEMV, GEMM_GEMV_LDS, GEMM_MFMA_F32 = 0, 1, 2, 3, 4, 5, 6
 GEMV_BEST_ROWS = 0         # rows up to which they beat the MFMA kernels in bfloat16: none (a step at 1.1B sizes, one token: 1.036 against 0.963 ms)
-ABI_VERSION = 22
+ABI_VERSION = 23
 
 
 class KernelError(RuntimeError):
@@ -127,7 +127,7 @@ def _declare(lib):
         "kllm_moe_expert_rows": [P, P, P, P, I, I, I, I, I, I, I, F, F, I, P],
         "kllm_moe_combine": [P, P, P, P, P, I, L, P, I, I, I, I, I, P, I, P, P],
         "kllm_sample": [P, P, P, P, I, I, P],
-        "kllm_attn_decode_slices": [I, I, I, I, I, I],
+        "kllm_attn_decode_slices": [I, I, I, I, I, I, I],
         "kllm_device_cus": [],
         "kllm_device_xcds": [],
         "kllm_gemm_prompt_slices": [I, I, I, I],
@@ -1244,11 +1244,11 @@ DECODE_HEAD_DIMS = (16, 32, 48, 64, 80, 96, 112, 128, 192, 256)
 
 
 @functools.lru_cache(maxsize=4096)
-def attn_decode_slices(n, n_kv_heads, n_heads, head_dim, dtype=torch.bfloat16, max_keys=0) -> int:
+def attn_decode_slices(n, n_kv_heads, n_heads, head_dim, dtype=torch.bfloat16, max_keys=0, page_size=16) -> int:
     """Slices of keys for a decode batch of n tokens; ``max_keys`` bounds the keys of the
     longest request (block-table width x page size, or the window), 0 if unknown."""
     return library().kllm_attn_decode_slices(n, n_kv_heads, n_heads, int(head_dim), dtype_code(dtype),
-                                             int(max_keys))
+                                             int(max_keys), int(page_size))
 
 
 def attn_f32_fits(head_dim, page_size) -> bool:

@@ -350,7 +350,7 @@ class CausalSelfAttention(Part):
             max_keys = min(max_keys, self.window + self.keep_first + cache.page_size)
         if self.chunk:
             max_keys = min(max_keys, self.chunk)
-        nslices = K.attn_decode_slices(count, self.kv_heads, self.heads, self.head_dim, q.dtype, max_keys)
+        nslices = K.attn_decode_slices(count, self.kv_heads, self.heads, self.head_dim, q.dtype, max_keys, cache.page_size)
         part = ctx.buf("attn.part", (n * self.heads * nslices * (self.head_dim + 2),), torch.float32)
         K.attn_decode(q, out, part, cache.pages, ctx.positions, ctx.span_of_token, cache.block_table,
                       cache.page_size, self.heads, self.kv_heads, self.head_dim, self.window,

@@ -82,6 +82,17 @@ def test_slices_of_short_contexts_in_float32(n, KV, H, hd, keys, slices):
     assert K.attn_decode_slices(n, KV, H, hd, F32, keys) == slices
 
 
+@pytest.mark.parametrize("n,KV,H,hd,keys,page,slices", [
+    (64, 4, 32, 64, 2048, 20, 8), (64, 4, 32, 64, 2048, 24, 8), (72, 4, 32, 96, 8192, 20, 7), (20, 32, 32, 64, 4096, 12, 3),       # 32 columns: eight waves a CU
+    (8, 32, 32, 128, 2048, 20, 4), (9, 32, 32, 128, 2048, 20, 7), (64, 4, 32, 64, 640, 20, 4), (32, 8, 256, 64, 640, 16, 8), (64, 4, 128, 64, 2048, 16, 8),
+    (64, 4, 32, 64, 2048, 16, 4), (64, 4, 32, 64, 1 << 17, 48, 4), (14, 32, 32, 128, 16384, 16, 4), (16, 32, 32, 64, 8192, 32, 4),    # 16: whole last rounds
+    (9, 32, 32, 64, 512, 16, 4), (9, 32, 32, 64, 1024, 16, 8), (9, 32, 32, 64, 4096, 16, 16), (12, 32, 32, 64, 1024, 16, 4), (12, 32, 32, 64, 2048, 16, 8), (12, 32, 32, 128, 8192, 16, 8),
+    (17, 32, 32, 64, 8192, 16, 16), (72, 4, 32, 96, 4096, 16, 16), (72, 4, 32, 96, 2048, 16, 8), (28, 32, 32, 64, 2048, 16, 8), (100, 32, 32, 64, 8192, 16, 4)])
+def test_slices_of_many_groups_in_float32(n, KV, H, hd, keys, page, slices):
+    """From one group of heads per CU on: by the kernel that takes the pages, and on 16 columns by how full the last round of workgroups is."""
+    assert K.attn_decode_slices(n, KV, H, hd, F32, keys, page) == slices
+
+
 @pytest.mark.parametrize("kind,n,m,k,dtype,want", [
     (K.LINEAR_RESID, 64, 2048, 5632, torch.bfloat16, True), (K.LINEAR_SWIGLU, 64, 11264, 2048, torch.bfloat16, True),
     (K.LINEAR_ROPE, 64, 2560, 2048, torch.bfloat16, True), (K.LINEAR_RESID, 65, 2048, 5632, torch.bfloat16, False),
