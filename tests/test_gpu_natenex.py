@@ -265,6 +265,43 @@ def test_kept_first_positions_in_the_attention_kernels(H, KV, hd, window, keep):
                 assert rel(got[r], want[i]) < 2e-2, (firsts, total, longest, i)
 
 
+@pytest.mark.parametrize("H,KV,hd,page,window,keep,lens", [
+    (2, 1, 64, 48, 130, 40, [1, 41, 170, 171, 700, 2333]), (4, 1, 128, 80, 333, 100, [99, 433, 434, 1111]), (6, 2, 32, 80, 96, 17, [97, 113, 129, 640]),
+    (2, 1, 64, 48, 8500, 70, [8569, 8603, 9201]), (3, 1, 96, 80, 8640, 200, [8850, 12000])])
+def test_kept_first_positions_in_large_pages_and_many_tiles(H, KV, hd, page, window, keep, lens):
+    """Single tokens whose kept positions end inside a tile of 32 and a page of 48 or 80 slots, with no gap, a part of a tile and many pages between them and
+    the window, and with more than the 32 tiles of a wave whose pages are looked up at once (one slice of 8,700 and 8,840 keys).  Pages
+    of the gap and slots behind the last key are NaN.  Probabilities and output are rounded to 2^-9 each."""
+    from kllm_amd import kernels as K
+    g = torch.Generator().manual_seed(page + window)
+    per, scale, B = -(-max(lens) // page), hd ** -0.5, len(lens)
+    table = torch.randperm(B * per + 1, generator=g)[:B * per].view(B, per).to(torch.int32)
+    cache = torch.full((B * per + 1, 2, KV, page * hd), float("nan"))
+    q = (2 * torch.randn(B, H, hd, generator=g)).bfloat16()
+    want = torch.zeros(B, H, hd, dtype=F64)
+    for s, n in enumerate(lens):
+        k, v = torch.randn(n, KV, hd, generator=g).bfloat16(), torch.randn(n, KV, hd, generator=g).bfloat16()
+        for j in range(-(-n // page)):
+            if j * page >= keep and (j + 1) * page <= n - window:
+                continue
+            kk, vv = k[j * page:(j + 1) * page].float(), v[j * page:(j + 1) * page].float()
+            cache[table[s, j], 0].view(KV, page, hd)[:, :len(kk)] = kk.transpose(0, 1)
+            cache[table[s, j], 1].view(KV, hd, page)[..., :len(vv)] = vv.permute(1, 2, 0)
+        seen = [j for j in range(n) if j >= n - window or j < keep]
+        for h in range(H):
+            kv = h // (H // KV)
+            want[s, h] = torch.softmax(k[seen, kv].double() @ q[s, h].double() * scale, 0) @ v[seen, kv].double()
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    for slices in (1, 3, 16):
+        out = torch.full((B, H * hd), 7.0, dtype=torch.bfloat16, device="cuda")
+        part = torch.full((B * H * slices * (hd + 2),), float("nan"), device="cuda")
+        K.attn_decode(q.view(B, -1).cuda(), out, part, cache.bfloat16().cuda(), i32([n - 1 for n in lens]), i32(list(range(B))), table.cuda(), page, H, KV,
+                      hd, window, scale, slices, keep_first=keep)
+        got = out.float().cpu().view(B, H, hd)
+        for s in range(B):
+            assert rel(got[s], want[s]) < 2 ** -7, (slices, lens[s])
+
+
 LATENT_CASES = [(3, 40, 8), (6, 160, 32), (3, 448, 64), (20, 96, 32), (34, 128, 16), (2, 512, 64), (5, 200, 24), (4, 16, 8)]
 
 
