@@ -12,11 +12,11 @@ namespace kllm {
 // every read is a trip to memory: all reads of sixteen slices (maxima, sums and this lane's
 // DV elements of each output) go out together, and every lane works out the weights for
 // itself, so that sixteen slices cost one trip and no exchange between lanes.  Further
-// rounds of sixteen (long contexts) are merged with a running maximum.  (R: the slices of a
-// round, for callers with few.)
-template <typename T, int DV, int R = 16>   // DV: elements of a head per lane (head size up to 64 DV); R: slices a round
+// rounds of sixteen (long contexts) are merged with a running maximum.
+template <typename T, int DV>   // DV: elements of a head per lane (head size up to 64 DV)
 __device__ __forceinline__ void attn_merge_one(T* __restrict__ out, const float* __restrict__ part, int t, int h, int H,
                                                int hd, int nslices, int lane, const OutGate& gate) {
+  constexpr int R = 16;                // slices a round
   const int stride = hd + 2, side = gate.side;
   asm volatile("" ::"s"(side));        // (with the other arguments: in front of the stores it was a trip to memory of its own)
   const float* p = part + ((long)t * H + h) * nslices * stride;
@@ -131,9 +131,9 @@ inline void launch_attn_merge(T* out, const float* part, int count, int H, int h
                               const int* token_list, const OutGate& gate, hipStream_t stream) {
   const dim3 grid(count, H), block(64);
   if (nslices <= 64 && hd <= 128) {
-    // (one trip to memory whatever the number of slices, and a lane asks for 2 + slices x DV
-    // numbers instead of slices x (2 + DV); 64 slices of a head of 64: the merge 10 us -> 6,
-    // 16 slices: a microsecond less)
+    // (one trip to memory whatever the number of slices, and a lane asks for 2 + R DV numbers, those
+    // behind the last slice from nowhere, instead of R (2 + DV); 64 slices of a head of 64: the merge 10 us
+    // -> 6, 16 slices: a microsecond less)
 #define KLLM_MERGE_WIDE(DV, R) \
     hipLaunchKernelGGL((attn_merge_wide_kernel<T, DV, R>), grid, block, 0, stream, part, token_list, out, H, hd, nslices, gate)
     if (hd <= 64) {

@@ -1188,7 +1188,7 @@ __global__ __launch_bounds__(kLatThreads) void latent_query_mfma_kernel(
   const int tt = blockIdx.x * 16 + c;
   const float* in = q + ((long)t * H + h) * hw;
   const int r0 = (blockIdx.z * 4 + wave) * 16;
-  // Everything that a wave needs is asked for before anything is used, 64 of d at a time: weights, the heads' sums, and its
+  // Everything that a wave needs is asked for before anything is used, 128 of d at a time: weights, the heads' sums, and its
   // share of the rotated part (elements 4 piece + g and every 16 gridDim.z'th behind).
   typedef float anywhere4 __attribute__((ext_vector_type(4), aligned(4)));      // (rows of d + dr floats)
   const bf16_t* wrow = w_ukt + ((long)h * rank + min(r0 + c, rank - 1)) * d;
