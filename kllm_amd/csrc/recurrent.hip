@@ -65,6 +65,10 @@ __device__ __forceinline__ void conv_tail_of_span(const ConvTail& tail, long slo
 //
 // Bound by a decode batch's trips to memory in a row and, for a prompt, by the sums' bytes: with four taps a wave asks for its channels' rows,
 // weights and, where the span begins inside the window, entries at once, 128 channels at a time (tap after tap waited for each; 8 tokens, heads of 128: 8.6 -> 6.9 us, 1,500 tokens 55.7 -> 33.4).
+// UP: 4: four taps; 3: up to three, as the last of four; 0: more, a channel and a tap at a time.  R: channels a lane takes at a time, of heads up to 64
+// one.  us, 1,500 tokens: three taps, 16 heads of 64, tap after tap 17.3, and of 128 channels at a time, the head's or not, 22.5, so 16.6; 32 heads of 128 46.6, so
+// 34.3; four taps, 16 heads of 64, tap after tap 20.9, two channels a lane 15.2, one 14.7.
+template <int UP, int R>
 __global__ __launch_bounds__(kRecThreads) void gated_delta_prep_kernel(
     const int* __restrict__ span_of_token, const int* __restrict__ span_start, const int* __restrict__ span_pos, const int* __restrict__ slots,
     const float* __restrict__ proj, int H, int G, int dk, int dv, const float* __restrict__ conv_w, int taps, int nsplit, long cols, long split_stride,
@@ -83,10 +87,10 @@ __global__ __launch_bounds__(kRecThreads) void gated_delta_prep_kernel(
   const int lane = threadIdx.x % kWave;
   const int item = blockIdx.y * (kRecThreads / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   if (item >= 2 * G + H) return;
-  const int QK = G * dk, HV = H * dv, C = 2 * QK + HV, K = taps - 1;
+  const int QK = G * dk, HV = H * dv, C = 2 * QK + HV, K = UP == 4 ? 3 : taps - 1;
+  const int none = 3 - K;                                // of the window's four rows, how many the convolution does not have (UP)
   const int gate_col = C + (a_sums ? H : 2 * H);
   // y[r]: SiLU of the convolution of channel c0 + lane + 64 r, of `width` (beyond it some channel's, not used)
-  constexpr int R = 2;
   struct Ask {                                           // what four taps need, on its way
     float x[R][4], w[R][4];
   };
@@ -98,7 +102,7 @@ __global__ __launch_bounds__(kRecThreads) void gated_delta_prep_kernel(
 #pragma unroll
       for (int j = 0; j < 4; ++j) {                      // (rows that are not there: the step's first, not used)
         A.x[r][j] = proj[max(t - 3 + j, 0L) * cols + c];
-        A.w[r][j] = conv_w[(long)c * 4 + j];
+        A.w[r][j] = conv_w[(long)c * (K + 1) + max(j - none, 0)];
       }
     }
     return A;
@@ -107,26 +111,27 @@ __global__ __launch_bounds__(kRecThreads) void gated_delta_prep_kernel(
     const long t0 = __builtin_amdgcn_readfirstlane(first_v);
     const bool fresh = __builtin_amdgcn_readfirstlane(pos_v) == 0;
     const float* st = state + (long)__builtin_amdgcn_readfirstlane(slot_v) * slot_stride;
-    if (taps == 4) {
-      const int before = (int)min(max(t0 - t + 3, 0L), 3L);      // rows of the window before the span's first: entries 3 - before ... of the state
+    if constexpr (UP > 0) {
+      const int before = (int)min(max(t0 - t + 3, 0L), 3L);      // rows of the window before the span's first: entries of the state, the last K of three
       float was[R][3];
-      if (before > 0 && !fresh) {
+      if (before > 0 && !fresh && K > 0) {
 #pragma unroll
         for (int r = 0; r < R; ++r)
 #pragma unroll
-          for (int j = 0; j < 3; ++j) was[r][j] = st[(long)(c0 + min(e0 + lane + kWave * r, width - 1)) * 3 + j];
+          for (int j = 0; j < 3; ++j) was[r][j] = st[(long)(c0 + min(e0 + lane + kWave * r, width - 1)) * K + max(j - none, 0)];
       }
 #pragma unroll
       for (int r = 0; r < R; ++r) {
+        y[r] = 0.f;
         const int c = c0 + min(e0 + lane + kWave * r, width - 1);
         for (int s = 1; s < nsplit; ++s)
 #pragma unroll
           for (int j = 0; j < 4; ++j) A.x[r][j] += proj[s * split_stride + max(t - 3 + j, 0L) * cols + c];
-        y[r] = 0.f;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
+          if (j < none) continue;
           float in = A.x[r][j];
-          if (j < before) {                              // row t - 3 + j, before - j rows before the first: entry 3 - (before - j)
+          if (j < before) {                              // row t - 3 + j, before - j rows before the first: entry K - (before - j)
             in = 0.f;
             if (!fresh) in = before - j == 1 ? was[r][2] : before - j == 2 ? was[r][1] : was[r][0];
           }
@@ -136,8 +141,10 @@ __global__ __launch_bounds__(kRecThreads) void gated_delta_prep_kernel(
     } else {
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        const int c = c0 + min(e0 + lane + kWave * r, width - 1);
-        y[r] = conv_at(proj, nsplit, split_stride, cols, c, nullptr, conv_w + (long)c * taps, taps, st + (long)c * K, fresh, t, t0);
+        const int c = c0 + e0 + lane + kWave * r;
+        y[r] = 0.f;
+        if (c < c0 + width)
+          y[r] = conv_at(proj, nsplit, split_stride, cols, c, nullptr, conv_w + (long)c * taps, taps, st + (long)c * K, fresh, t, t0);
       }
     }
 #pragma unroll
@@ -148,11 +155,11 @@ __global__ __launch_bounds__(kRecThreads) void gated_delta_prep_kernel(
     float val[4] = {0.f, 0.f, 0.f, 0.f};
     float ss = 0.f;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < 4 / R; ++h) {
       if (h * R * kWave >= dk) break;
       float y[R];
       Ask A;
-      if (taps == 4) A = ask(c0, dk, h * R * kWave);
+      if (UP) A = ask(c0, dk, h * R * kWave);
       convolved(A, c0, dk, h * R * kWave, y);
 #pragma unroll
       for (int r = 0; r < R; ++r) val[R * h + r] = lane + kWave * (R * h + r) < dk ? y[r] : 0.f;
@@ -177,7 +184,7 @@ __global__ __launch_bounds__(kRecThreads) void gated_delta_prep_kernel(
   const float al = a_log[h], dt = dt_bias[own_decay ? h : 0];
   for (int e0 = 0; e0 < dv; e0 += R * kWave) {
     Ask A;
-    if (taps == 4) A = ask(2 * QK + h * dv, dv, e0);
+    if (UP) A = ask(2 * QK + h * dv, dv, e0);
     float g[R], y[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -1353,9 +1360,17 @@ extern "C" int kllm_gated_delta_prep(const float* proj, int nsplit, long split_s
                "gated_delta_prep: rows of %d and %d sums do not hold the decays and the gates", a_row, g_row);
   const int items = 2 * G + H, per_wg = kRecThreads / kWave;
   KLLM_REQUIRE(ceil_div(items, per_wg) <= 65535, "gated_delta_prep: %d heads are too many for the grid", items);
-  hipLaunchKernelGGL(gated_delta_prep_kernel, dim3(n, ceil_div(items, per_wg)), dim3(kRecThreads), 0, stream, span_of_token, span_start,
-                     span_pos, slots, proj, H, G, dk, dv, conv_w, taps, nsplit, (long)cols, split_stride, state, slot_stride, a_log, dt_bias, qn, kn, vv, gb,
-                     gate, unit_eps, a_sums, a_ns, a_stride, (long)a_row, gate_sums, g_ns, g_stride, (long)g_row, gate_sigmoid, dec);
+#define KLLM_GDP(UP, R)                                                                                                                  \
+  hipLaunchKernelGGL((gated_delta_prep_kernel<UP, R>), dim3(n, ceil_div(items, per_wg)), dim3(kRecThreads), 0, stream, span_of_token,         \
+                     span_start, span_pos, slots, proj, H, G, dk, dv, conv_w, taps, nsplit, (long)cols, split_stride, state, slot_stride,   \
+                     a_log, dt_bias, qn, kn, vv, gb, gate, unit_eps, a_sums, a_ns, a_stride, (long)a_row, gate_sums, g_ns, g_stride,       \
+                     (long)g_row, gate_sigmoid, dec)
+  const bool narrow = dk <= kWave && dv <= kWave;
+  if (taps > 4) KLLM_GDP(0, 2);
+  else if (taps == 4) { if (narrow) KLLM_GDP(4, 1); else KLLM_GDP(4, 2); }
+  else if (narrow) KLLM_GDP(3, 1);
+  else KLLM_GDP(3, 2);
+#undef KLLM_GDP
   KLLM_CHECK_LAUNCH("gated_delta_prep");
   return 0;
 }

@@ -403,7 +403,7 @@ def test_delta_scan_of_single_tokens_where_rows_are_whole_pieces(dk, dv, per_cha
 
 
 @pytest.mark.parametrize("dk,dv", [(64, 128), (128, 130), (200, 40), (256, 300)])
-@pytest.mark.parametrize("taps", [1, 4, 5])
+@pytest.mark.parametrize("taps", [1, 2, 3, 4, 5])
 @pytest.mark.parametrize("nsplit", [1, 3])
 def test_delta_preparation(dk, dv, taps, nsplit):
     """Convolution, SiLU and unit norms against 64 bits: spans that begin inside a token's window, behind earlier tokens and at position 0;
