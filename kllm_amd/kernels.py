@@ -2342,11 +2342,13 @@ def latent_query(q, w_uk, cos, sin, out, heads, dim, rot_dim, rank, transposed=F
 LATENT_BLOCK_FROM = 64      # tokens of a step from which four tokens share a workgroup and its tiles of keys
 
 
-def attn_latent_slices(n, heads, rank, dtype=torch.bfloat16, window=0, max_keys=0) -> int:
+def attn_latent_slices(n, heads, rank, dtype=torch.bfloat16, window=0, max_keys=0, row=0) -> int:
     """Workgroups that share out the keys of a token and 16 heads (their results are merged in
-    the same call): as many as bring a step's workgroups to about one a CU, which holds one (a step of 9 tokens at 2,600 keys with half as
-    many 795 us, 761, with twice as many 765; 24 tokens at 1,000 890, 863, 866), for steps of few
-    tokens; 1 where the kernel on the matrix cores does not run; 0 for steps of many tokens: there
+    the same call), for steps of few tokens: as many as bring a step's workgroups to what the chip holds at a time (us with half
+    as many, so, and with twice as many: ranks above 128, of which a CU holds one, a step of 9 tokens at 2,600 keys 795, 761, 765, 24 tokens at 1,000 890,
+    863, 866; ranks up to 128, and rows above 384 (0: not known) with ranks up to 256, of which it holds two, at 1,400 keys: 33 tokens x 16 heads, row 72 and
+    rank 64, 12.0, 10.3, 9.5, x 32 heads 19.0, 13.1, 12.8, 63 x 32 20.2, 17.9, 18.6, row 400 and rank 128, 33 x 32 43.1, 28.7, 27.4, row 424 and rank 256
+    47.6, 33.6, 33.0).  1 where the kernel on the matrix cores does not run; 0 for steps of many tokens: there
     a workgroup takes four tokens, whose keys pass through LDS once for the four.  A slice has 128 keys at least, what a workgroup
     takes at a time: ``max_keys`` (0: not known), the most keys of a token, and a ``window`` bound them.  Does not depend on any context
     length beyond ``max_keys``, so a recorded step can be replayed as contexts grow."""
@@ -2359,7 +2361,8 @@ def attn_latent_slices(n, heads, rank, dtype=torch.bfloat16, window=0, max_keys=
     most = min(64, -(-(window + 31) // 128)) if window else 64
     if max_keys:
         most = min(most, -(-max_keys // 128))
-    while slices < most and groups * slices * 2 <= device_cus():
+    held = 2 if rank <= 128 or (rank <= 256 and row > 384) else 1
+    while slices < most and groups * slices * 2 <= held * device_cus():
         slices *= 2
     return slices
 

@@ -134,7 +134,7 @@ class LatentAttention(Part):
         while pages < cache.block_table.shape[1]:
             pages *= 2
         slices = 1 if plain or self.row % 8 or cache.page_size % 16 else K.attn_latent_slices(
-            n, self.heads, self.kv_rank, dtype, self.window, pages * cache.page_size)
+            n, self.heads, self.kv_rank, dtype, self.window, pages * cache.page_size, self.row)
         part = ctx.buf("latent.part", (n * self.heads * slices * (self.kv_rank + 2),), torch.float32) if slices > 1 else None
         K.attn_latent(qa, attended, cache.pages, ctx.positions, ctx.span_of_token, cache.block_table, cache.page_size,
                       self.heads, self.row, self.kv_rank, self.scale, plain=plain, part=part, nslices=slices, window=self.window)

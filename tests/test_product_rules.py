@@ -93,6 +93,14 @@ def test_slices_of_many_groups_in_float32(n, KV, H, hd, keys, page, slices):
     assert K.attn_decode_slices(n, KV, H, hd, F32, keys, page) == slices
 
 
+@pytest.mark.parametrize("n,heads,row,rank,keys,window,slices", [
+    (8, 32, 576, 512, 1024, 0, 8), (8, 32, 576, 512, 4096, 0, 16), (33, 32, 576, 512, 4096, 0, 2), (33, 32, 288, 256, 4096, 0, 2), (33, 32, 704, 512, 4096, 0, 2),
+    (33, 32, 192, 128, 4096, 0, 4), (33, 16, 72, 64, 4096, 0, 8), (16, 128, 400, 128, 4096, 0, 4), (33, 32, 424, 256, 4096, 0, 4), (33, 32, 384, 256, 4096, 0, 2),
+    (4, 16, 72, 64, 300, 0, 4), (1, 16, 576, 512, 0, 100, 2), (64, 32, 576, 512, 4096, 0, 0)])
+def test_slices_of_latent_attention_by_what_a_cu_holds(n, heads, row, rank, keys, window, slices):
+    assert K.attn_latent_slices(n, heads, rank, BF16, window, keys, row) == slices
+
+
 @pytest.mark.parametrize("kind,n,m,k,dtype,want", [
     (K.LINEAR_RESID, 64, 2048, 5632, torch.bfloat16, True), (K.LINEAR_SWIGLU, 64, 11264, 2048, torch.bfloat16, True),
     (K.LINEAR_ROPE, 64, 2560, 2048, torch.bfloat16, True), (K.LINEAR_RESID, 65, 2048, 5632, torch.bfloat16, False),
