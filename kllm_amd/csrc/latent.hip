@@ -1347,13 +1347,14 @@ __global__ __launch_bounds__(kLatThreads) void latent_query_block_kernel(
 // outputs of a token.  In us, 32 heads of 128, rank 512, with a gate in one slice, operands by lane before and now: 64 tokens 11.8 -> 9.1, 200 12.2 ->
 // 9.4, 260 21.0 -> 12.3, 400 21.5 -> 12.7, 700 31.1 -> 20.8, 1,500 60.4 -> 33.4, in four slices 17.1 -> 11.5, 17.9 -> 13.7, 31.0 -> 17.5, 31.8 -> 19.3, 48.1 ->
 // 29.9, 96.7 -> 47.7; U 2 / 1: 200 tokens 13.1 / 9.4, 400 13.6 / 12.7, 520 (288 workgroups of U 2) 16.1 / 19.8, 1,500 33.4 / 40.3.
-constexpr int kOutChunk = 512;
-template <int U>
+// CHUNK: of the rank, in LDS and registers at a time.  With 512 whatever the rank, rows of 64 to 256 asked for what they do not have: us, operands by lane, 512, and
+// so: rank 64 (4 heads of 64, 200 tokens) 4.4, 6.1, 3.6; 96 (33 of 40, 1,500) 7.4, 12.6, 5.2; 256 (16 of 128, 500) 6.5, 7.2, 5.3.  Heads of up to 64 outputs take U 1.
+template <int U, int CHUNK>
 __global__ __launch_bounds__(kLatThreads, 2) void latent_out_block_kernel(
     const bf16_t* __restrict__ attended, const bf16_t* __restrict__ w_uv, int n, int H, int dv, int rank, const float* __restrict__ gate, long gate_stride,
     int nsplit, int by_head, long split_stride, bf16_t* __restrict__ out) {
-  constexpr int STEPS = kOutChunk / 32, TB = kLatTokens / 16;
-  __shared__ __attribute__((aligned(1024))) bf16_t rows[kLatTokens * kOutChunk];
+  constexpr int STEPS = CHUNK / 32, TB = kLatTokens / 16, SLOTS = CHUNK / 8;
+  __shared__ __attribute__((aligned(1024))) bf16_t rows[kLatTokens * CHUNK];
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int g = lane / 16, c = lane % 16;
   const int h = blockIdx.x, t0 = blockIdx.y * kLatTokens, j0 = 16 * U * (4 * blockIdx.z + wave);
@@ -1388,15 +1389,16 @@ __global__ __launch_bounds__(kLatThreads, 2) void latent_out_block_kernel(
     }
   };
   floatx4 z[TB][U];
-  for (int k0 = 0; k0 < rank; k0 += kOutChunk) {
-    const int width = min(rank - k0, kOutChunk), chunks = width / 8;       // rank % 16 == 0 (the launch)
+  for (int k0 = 0; k0 < rank; k0 += CHUNK) {
+    const int width = min(rank - k0, CHUNK), chunks = width / 8;       // rank % 16 == 0 (the launch)
     if (k0) __syncthreads();
 #pragma unroll
-    for (int i = 0; i < kLatTokens / 4; ++i) {
-      const int r = 4 * i + wave, chunk = lane ^ (r % 16);                // (chunks that are not there are never read)
+    for (int i = 0; i < kLatTokens / 4 / (kWave / SLOTS); ++i) {
+      const int r0 = (4 * i + wave) * (kWave / SLOTS), r = r0 + lane / SLOTS;
+      const int chunk = lane % SLOTS ^ (r % 16);                          // (chunks that are not there are never read)
       const bf16_t* src = attended + ((long)min(t0 + r, n - 1) * H + h) * rank + k0 + 8 * (chunk < chunks ? chunk : 0);
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                       (__attribute__((address_space(3))) void*)(rows + r * kOutChunk), 16, 0, 0);
+                                       (__attribute__((address_space(3))) void*)(rows + r0 * CHUNK), 16, 0, 0);
     }
     bf16x8 w[U][STEPS];
 #pragma unroll
@@ -1418,7 +1420,7 @@ __global__ __launch_bounds__(kLatThreads, 2) void latent_out_block_kernel(
 #pragma unroll
       for (int tb = 0; tb < TB; ++tb) {
         const int r = 16 * tb + c;
-        bf16x8 b = *reinterpret_cast<const bf16x8*>(rows + r * kOutChunk + 8 * ((4 * s + g) ^ c));
+        bf16x8 b = *reinterpret_cast<const bf16x8*>(rows + r * CHUNK + 8 * ((4 * s + g) ^ c));
         b = there ? b : zero;
 #pragma unroll
         for (int u = 0; u < U; ++u) acc[tb][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(there ? w[u][s] : zero, b, acc[tb][u], 0, 0, 0);
@@ -1612,11 +1614,16 @@ extern "C" int kllm_latent_out(const void* attended, const void* w_uv, const flo
   if (dtype == DT_BF16 && n >= kLatTokens && rank % 16 == 0 && ((uintptr_t)attended & 15) == 0 && ((uintptr_t)w_uv & 15) == 0 &&
       (n + kLatTokens - 1) / kLatTokens <= 65535 && (dv + 63) / 64 <= 65535) {
     const dim3 grid(H, (n + kLatTokens - 1) / kLatTokens, (dv + 127) / 128), halves(H, grid.y, (dv + 63) / 64);
-#define KLLM_LO(U, G)                                                                                                             \
-  hipLaunchKernelGGL(latent_out_block_kernel<U>, G, dim3(kLatThreads), 0, stream, (const bf16_t*)attended, (const bf16_t*)w_uv, n, H, dv, \
-                     rank, gate, gate_stride, nsplit, gate_by_head, split_stride, (bf16_t*)out)
-    if ((long)H * grid.y * grid.z <= device_cus()) KLLM_LO(1, halves); else KLLM_LO(2, grid);
+#define KLLM_LOC(U, CHUNK, G)                                                                                                     \
+  hipLaunchKernelGGL((latent_out_block_kernel<U, CHUNK>), G, dim3(kLatThreads), 0, stream, (const bf16_t*)attended, (const bf16_t*)w_uv, n, \
+                     H, dv, rank, gate, gate_stride, nsplit, gate_by_head, split_stride, (bf16_t*)out)
+#define KLLM_LO(U, G)                                                                                        \
+  do {                                                                                                       \
+    if (rank <= 128) KLLM_LOC(U, 128, G); else if (rank <= 256) KLLM_LOC(U, 256, G); else KLLM_LOC(U, 512, G); \
+  } while (0)
+    if (dv <= 64 || (long)H * grid.y * grid.z <= device_cus()) KLLM_LO(1, halves); else KLLM_LO(2, grid);
 #undef KLLM_LO
+#undef KLLM_LOC
     KLLM_CHECK_LAUNCH("latent_out");
     return 0;
   }

@@ -796,10 +796,10 @@ def test_products_with_a_heads_own_matrix_of_a_few_tokens(n, H, d, dr, rank, dv,
     assert rel(out.double().cpu().view(n, H, dv), want * opened) < 2.0 ** -8
 
 
-@pytest.mark.parametrize("n,H,dv,rank", [(64, 3, 130, 48), (65, 2, 36, 560), (200, 32, 128, 512), (330, 70, 64, 80), (700, 33, 72, 1040), (129, 300, 7, 16)])
+@pytest.mark.parametrize("n,H,dv,rank", [(64, 3, 130, 48), (65, 2, 36, 560), (200, 32, 128, 512), (330, 70, 64, 80), (700, 33, 72, 1040), (129, 300, 7, 16), (90, 5, 64, 240), (150, 6, 40, 304)])
 @pytest.mark.parametrize("nsplit,by_head", [(0, False), (1, False), (3, False), (2, True)])
 def test_latent_out_of_prompts(n, H, dv, rank, nsplit, by_head):
-    """64 tokens a workgroup, 64 or 128 outputs of a head: tokens, outputs and ranks (half a step of 32, less than a chunk of 512, a little more,
+    """64 tokens a workgroup, 64 or 128 outputs of a head: tokens, outputs and ranks (half a step of 32, less than a chunk of 128, 256 or 512, a little more,
     two) that end inside one, gates in slices, per output and per head.  Against 64 bits; the outputs are rounded to 2^-9."""
     from kllm_amd import kernels as K
     g = torch.Generator().manual_seed(n + dv)
