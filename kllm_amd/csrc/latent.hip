@@ -22,6 +22,8 @@
 // (token, head) in 32-bit arithmetic for every size and type, and, in bfloat16 for ranks in
 // steps of 16 and rows in steps of 8, one on the matrix cores (below).
 #include <math.h>
+
+#include <type_traits>
 #include <stdint.h>
 
 #include "common.hpp"
@@ -1260,10 +1262,10 @@ __global__ __launch_bounds__(kLatThreads) void latent_query_block_kernel(
   const int h = blockIdx.x, t0 = blockIdx.y * kLatTokens;
   const int hw = d + dr, half = dr / 2;
   const long row_out = (long)H * (rank + dr);
-  // A thread asks for a slice of its pieces together, eight at a time (one after the other, a trip to memory each: a prompt
+  // A thread asks for a slice of its pieces together, up to eight at a time (one after the other, a trip to memory each: a prompt
   // of 70 tokens at Natenex sizes 995 us, now 961, of 200 1,256 / 1,240; of 1,500, where other workgroups fill the wait, 34.9 / 33.5 of a layer).
   typedef float anywhere4 __attribute__((ext_vector_type(4), aligned(4)));
-  constexpr int PIECES = kLatTokens * (d / 4), MANY = 8;
+  constexpr int PIECES = kLatTokens * (d / 4), MANY = DS < 8 ? DS : 8;        // (DS pieces a thread)
 #pragma unroll 1
   for (int i0 = tid; i0 < PIECES; i0 += MANY * kLatThreads) {
     floatx4 v[MANY];
@@ -1283,37 +1285,41 @@ __global__ __launch_bounds__(kLatThreads) void latent_query_block_kernel(
       if (i < PIECES) *reinterpret_cast<bf16x4*>(qs + tt * LD + e) = bf16x4{(bf16_t)v[k][0], (bf16_t)v[k][1], (bf16_t)v[k][2], (bf16_t)v[k][3]};
     }
   }
-  // the rotated part beside it
+  // the rotated part beside it, as many pairs a thread at a time as there are
   const int pairs = kLatTokens * half;
+  auto rotated = [&](auto at_a_time) {
+    constexpr int PAIRS = decltype(at_a_time)::value;
 #pragma unroll 1
-  for (int i0 = tid; i0 < pairs; i0 += MANY * kLatThreads) {
-    float u[MANY], v[MANY], cs[MANY], sn[MANY];
+    for (int i0 = tid; i0 < pairs; i0 += PAIRS * kLatThreads) {
+      float u[PAIRS], v[PAIRS], cs[PAIRS], sn[PAIRS];
 #pragma unroll
-    for (int k = 0; k < MANY; ++k) {
-      const int i = min(i0 + k * kLatThreads, pairs - 1), tt = i / half, e = i - tt * half, t = min(t0 + tt, n - 1);
-      const float* in = q + ((long)t * H + h) * hw + d + e;
-      u[k] = in[0];
-      v[k] = in[half];
-      cs[k] = cos_t[(long)t * half + e];
-      sn[k] = sin_t[(long)t * half + e];
-    }
-    for (int s = 1; s < nsplit; ++s)
-#pragma unroll
-      for (int k = 0; k < MANY; ++k) {
+      for (int k = 0; k < PAIRS; ++k) {
         const int i = min(i0 + k * kLatThreads, pairs - 1), tt = i / half, e = i - tt * half, t = min(t0 + tt, n - 1);
-        const float* in = q + s * split_stride + ((long)t * H + h) * hw + d + e;
-        u[k] += in[0];
-        v[k] += in[half];
+        const float* in = q + ((long)t * H + h) * hw + d + e;
+        u[k] = in[0];
+        v[k] = in[half];
+        cs[k] = cos_t[(long)t * half + e];
+        sn[k] = sin_t[(long)t * half + e];
       }
+      for (int s = 1; s < nsplit; ++s)
 #pragma unroll
-    for (int k = 0; k < MANY; ++k) {
-      const int i = i0 + k * kLatThreads, tt = i / half, e = i - tt * half, t = t0 + tt;
-      if (i >= pairs || t >= n) continue;
-      bf16_t* dst = out + t * row_out + (long)h * (rank + dr) + rank + e;
-      dst[0] = (bf16_t)(u[k] * cs[k] - v[k] * sn[k]);
-      dst[half] = (bf16_t)(v[k] * cs[k] + u[k] * sn[k]);
+        for (int k = 0; k < PAIRS; ++k) {
+          const int i = min(i0 + k * kLatThreads, pairs - 1), tt = i / half, e = i - tt * half, t = min(t0 + tt, n - 1);
+          const float* in = q + s * split_stride + ((long)t * H + h) * hw + d + e;
+          u[k] += in[0];
+          v[k] += in[half];
+        }
+#pragma unroll
+      for (int k = 0; k < PAIRS; ++k) {
+        const int i = i0 + k * kLatThreads, tt = i / half, e = i - tt * half, t = t0 + tt;
+        if (i >= pairs || t >= n) continue;
+        bf16_t* dst = out + t * row_out + (long)h * (rank + dr) + rank + e;
+        dst[0] = (bf16_t)(u[k] * cs[k] - v[k] * sn[k]);
+        dst[half] = (bf16_t)(v[k] * cs[k] + u[k] * sn[k]);
+      }
     }
-  }
+  };
+  if (half <= 8) rotated(std::integral_constant<int, 2>()); else rotated(std::integral_constant<int, 8>());
   __syncthreads();
   for (int r0 = 32 * wave; r0 < rank; r0 += 32 * (kLatThreads / kWave)) {
     const bf16_t* wrow = w_ukt + ((long)h * rank + min(r0 + c, rank - 1)) * d + 8 * g;
