@@ -363,8 +363,10 @@ def decode_batch_fits(rt, x, m, copied=True):
 
 @functools.lru_cache(maxsize=4096)
 def _parts_best(n, m, k, dtype, unary, copied=True):
-    """Whether ``K.linear_rows`` is the fastest way to plain sums, or (``unary``) an activation of them, of n rows that are read row by row
-    (for bfloat16 up to 16 rows where the decode-batch kernel does not run: what it would run of those, ``_unstaged`` sends there as well).
+    """Whether ``K.linear_rows`` is the fastest way to plain sums, or (``unary``) an activation of them, of n rows that are read row by row.
+    For bfloat16 up to 16 rows this asks where it beats the kernels other than the decode-batch kernel: what that one would run, ``_unstaged`` sends to
+    ``K.linear_rows`` as well, so that the lines for those rows matter only where K is too long for its passes.  They, their figures below and the float32 lines
+    were measured before ``K.linear_rows`` asked for the weights first; its times are up to 1.5 us a product shorter now.
     The decode-batch kernel has the rows in LDS, this one reads up to sixteen of them a load: up to eight rows it is the faster one where
     K is long enough, of 9 to 16 not (a step of Nusilix layers of 1,024 columns, there / here, with K of 1,024 here, too: 1 token 601 / 608 us, 2
     606 / 617, 8 678 / 714; us a product: 8 rows 2,048 x 1,024 3.8 / 4.6, 2,048 x 4,096 6.8 / 6.2, 1,024 x 1,408 in a step 3.9 / 5.3, 2,048 x 2,048 4.9 /
