@@ -65,10 +65,10 @@ __device__ __forceinline__ void conv_tail_of_span(const ConvTail& tail, long slo
 //
 // Bound by a decode batch's trips to memory in a row and, for a prompt, by the sums' bytes: with four taps a wave asks for its channels' rows,
 // weights and, where the span begins inside the window, entries at once, 128 channels at a time (tap after tap waited for each; 8 tokens, heads of 128: 8.6 -> 6.9 us, 1,500 tokens 55.7 -> 33.4).
-// UP: 4: four taps; 3: up to three, as the last of four; 0: more, a channel and a tap at a time.  R: channels a lane takes at a time, of heads up to 64
-// one.  us, 1,500 tokens: three taps, 16 heads of 64, tap after tap 17.3, and of 128 channels at a time, the head's or not, 22.5, so 16.6; 32 heads of 128 46.6, so
-// 34.3; four taps, 16 heads of 64, tap after tap 20.9, two channels a lane 15.2, one 14.7.
-template <int UP, int R>
+// TAPS: their number up to four, 0 for more, which go a channel and a tap at a time.  R: channels a lane takes at a time, of heads up to 64 one.  us, 1,500 tokens:
+// three taps, 16 heads of 64, tap after tap 17.3, and of 128 channels at a time, the head's or not, 22.5, so 13.2; 32 heads of 128 46.6, so 27.9; four
+// taps, 16 heads of 64, tap after tap 20.9, two channels a lane 15.2, one 14.7.
+template <int TAPS, int R>
 __global__ __launch_bounds__(kRecThreads) void gated_delta_prep_kernel(
     const int* __restrict__ span_of_token, const int* __restrict__ span_start, const int* __restrict__ span_pos, const int* __restrict__ slots,
     const float* __restrict__ proj, int H, int G, int dk, int dv, const float* __restrict__ conv_w, int taps, int nsplit, long cols, long split_stride,
@@ -87,8 +87,8 @@ __global__ __launch_bounds__(kRecThreads) void gated_delta_prep_kernel(
   const int lane = threadIdx.x % kWave;
   const int item = blockIdx.y * (kRecThreads / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   if (item >= 2 * G + H) return;
-  const int QK = G * dk, HV = H * dv, C = 2 * QK + HV, K = UP == 4 ? 3 : taps - 1;
-  const int none = 3 - K;                                // of the window's four rows, how many the convolution does not have (UP)
+  const int QK = G * dk, HV = H * dv, C = 2 * QK + HV, K = TAPS ? TAPS - 1 : taps - 1;
+  constexpr int FROM = 4 - TAPS;                         // of four rows up to the token's, the first that the convolution has (TAPS)
   const int gate_col = C + (a_sums ? H : 2 * H);
   // y[r]: SiLU of the convolution of channel c0 + lane + 64 r, of `width` (beyond it some channel's, not used)
   struct Ask {                                           // what four taps need, on its way
@@ -100,9 +100,9 @@ __global__ __launch_bounds__(kRecThreads) void gated_delta_prep_kernel(
     for (int r = 0; r < R; ++r) {
       const int c = c0 + min(e0 + lane + kWave * r, width - 1);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {                      // (rows that are not there: the step's first, not used)
+      for (int j = FROM; j < 4; ++j) {                   // (rows that are not there: the step's first, not used)
         A.x[r][j] = proj[max(t - 3 + j, 0L) * cols + c];
-        A.w[r][j] = conv_w[(long)c * (K + 1) + max(j - none, 0)];
+        A.w[r][j] = conv_w[(long)c * TAPS + j - FROM];
       }
     }
     return A;
@@ -111,14 +111,14 @@ __global__ __launch_bounds__(kRecThreads) void gated_delta_prep_kernel(
     const long t0 = __builtin_amdgcn_readfirstlane(first_v);
     const bool fresh = __builtin_amdgcn_readfirstlane(pos_v) == 0;
     const float* st = state + (long)__builtin_amdgcn_readfirstlane(slot_v) * slot_stride;
-    if constexpr (UP > 0) {
+    if constexpr (TAPS > 0) {
       const int before = (int)min(max(t0 - t + 3, 0L), 3L);      // rows of the window before the span's first: entries of the state, the last K of three
       float was[R][3];
-      if (before > 0 && !fresh && K > 0) {
+      if (before > 0 && !fresh) {
 #pragma unroll
         for (int r = 0; r < R; ++r)
 #pragma unroll
-          for (int j = 0; j < 3; ++j) was[r][j] = st[(long)(c0 + min(e0 + lane + kWave * r, width - 1)) * K + max(j - none, 0)];
+          for (int j = FROM; j < 3; ++j) was[r][j] = st[(long)(c0 + min(e0 + lane + kWave * r, width - 1)) * K + j - FROM];
       }
 #pragma unroll
       for (int r = 0; r < R; ++r) {
@@ -126,10 +126,9 @@ __global__ __launch_bounds__(kRecThreads) void gated_delta_prep_kernel(
         const int c = c0 + min(e0 + lane + kWave * r, width - 1);
         for (int s = 1; s < nsplit; ++s)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) A.x[r][j] += proj[s * split_stride + max(t - 3 + j, 0L) * cols + c];
+          for (int j = FROM; j < 4; ++j) A.x[r][j] += proj[s * split_stride + max(t - 3 + j, 0L) * cols + c];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if (j < none) continue;
+        for (int j = FROM; j < 4; ++j) {
           float in = A.x[r][j];
           if (j < before) {                              // row t - 3 + j, before - j rows before the first: entry K - (before - j)
             in = 0.f;
@@ -159,7 +158,7 @@ __global__ __launch_bounds__(kRecThreads) void gated_delta_prep_kernel(
       if (h * R * kWave >= dk) break;
       float y[R];
       Ask A;
-      if (UP) A = ask(c0, dk, h * R * kWave);
+      if (TAPS) A = ask(c0, dk, h * R * kWave);
       convolved(A, c0, dk, h * R * kWave, y);
 #pragma unroll
       for (int r = 0; r < R; ++r) val[R * h + r] = lane + kWave * (R * h + r) < dk ? y[r] : 0.f;
@@ -184,7 +183,7 @@ __global__ __launch_bounds__(kRecThreads) void gated_delta_prep_kernel(
   const float al = a_log[h], dt = dt_bias[own_decay ? h : 0];
   for (int e0 = 0; e0 < dv; e0 += R * kWave) {
     Ask A;
-    if (UP) A = ask(2 * QK + h * dv, dv, e0);
+    if (TAPS) A = ask(2 * QK + h * dv, dv, e0);
     float g[R], y[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -1360,16 +1359,21 @@ extern "C" int kllm_gated_delta_prep(const float* proj, int nsplit, long split_s
                "gated_delta_prep: rows of %d and %d sums do not hold the decays and the gates", a_row, g_row);
   const int items = 2 * G + H, per_wg = kRecThreads / kWave;
   KLLM_REQUIRE(ceil_div(items, per_wg) <= 65535, "gated_delta_prep: %d heads are too many for the grid", items);
-#define KLLM_GDP(UP, R)                                                                                                                  \
-  hipLaunchKernelGGL((gated_delta_prep_kernel<UP, R>), dim3(n, ceil_div(items, per_wg)), dim3(kRecThreads), 0, stream, span_of_token,         \
+#define KLLM_GDP(TAPS, R)                                                                                                                \
+  hipLaunchKernelGGL((gated_delta_prep_kernel<TAPS, R>), dim3(n, ceil_div(items, per_wg)), dim3(kRecThreads), 0, stream, span_of_token,         \
                      span_start, span_pos, slots, proj, H, G, dk, dv, conv_w, taps, nsplit, (long)cols, split_stride, state, slot_stride,   \
                      a_log, dt_bias, qn, kn, vv, gb, gate, unit_eps, a_sums, a_ns, a_stride, (long)a_row, gate_sums, g_ns, g_stride,       \
                      (long)g_row, gate_sigmoid, dec)
-  const bool narrow = dk <= kWave && dv <= kWave;
-  if (taps > 4) KLLM_GDP(0, 2);
-  else if (taps == 4) { if (narrow) KLLM_GDP(4, 1); else KLLM_GDP(4, 2); }
-  else if (narrow) KLLM_GDP(3, 1);
-  else KLLM_GDP(3, 2);
+#define KLLM_GDT(TAPS)                                                              \
+  do {                                                                              \
+    if (dk <= kWave && dv <= kWave) KLLM_GDP(TAPS, 1); else KLLM_GDP(TAPS, 2);       \
+  } while (0)
+  if (taps == 1) KLLM_GDT(1);
+  else if (taps == 2) KLLM_GDT(2);
+  else if (taps == 3) KLLM_GDT(3);
+  else if (taps == 4) KLLM_GDT(4);
+  else KLLM_GDP(0, 2);
+#undef KLLM_GDT
 #undef KLLM_GDP
   KLLM_CHECK_LAUNCH("gated_delta_prep");
   return 0;
