@@ -1149,10 +1149,14 @@ __global__ __launch_bounds__(kWave) void latent_out_mfma_kernel(
   };
   ask(0, a[0], b[0]);
   if (rank > 32 * STEPS) ask(32 * STEPS, a[1], b[1]);
-  float gs[4] = {0.f, 0.f, 0.f, 0.f};
+  float gs[4] = {0.f, 0.f, 0.f, 0.f}, more[4] = {0.f, 0.f, 0.f, 0.f};      // two slices of the gate's sums
   if (gate)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) gs[i] = gate[t * gate_stride + (by_head ? h : (long)h * dv + min(j0 + 4 * g + i, dv - 1))];
+    for (int i = 0; i < 4; ++i) {
+      const float* at = gate + t * gate_stride + (by_head ? h : (long)h * dv + min(j0 + 4 * g + i, dv - 1));
+      gs[i] = at[0];
+      if (nsplit > 1) more[i] = at[split_stride];
+    }
   floatx4 acc = {0.f, 0.f, 0.f, 0.f};
   for (int k0 = 0; k0 < rank; k0 += 64 * STEPS) {
 #pragma unroll
@@ -1172,7 +1176,8 @@ __global__ __launch_bounds__(kWave) void latent_out_mfma_kernel(
     const long col = (long)h * dv + jj;
     float v = acc[i];
     if (gate) {
-      for (int s = 1; s < nsplit; ++s) gs[i] += gate[s * split_stride + tt * gate_stride + (by_head ? h : col)];
+      gs[i] += more[i];
+      for (int s = 2; s < nsplit; ++s) gs[i] += gate[s * split_stride + tt * gate_stride + (by_head ? h : col)];
       v *= sigmoid_f32(gs[i]);
     }
     out[(long)tt * H * dv + col] = (bf16_t)v;
