@@ -1256,7 +1256,7 @@ constexpr int kLatTokens = 64;
 // DS = d / 16.  The tokens' queries (their slices added, in the compute type) pass through LDS once
 // for all outputs; a wave takes every fourth piece of 32 outputs.
 template <int DS>
-__global__ __launch_bounds__(kLatThreads) void latent_query_block_kernel(
+__global__ __launch_bounds__(kLatThreads, DS <= 8 ? 4 : 2) void latent_query_block_kernel(
     const float* __restrict__ q, int nsplit, long split_stride, const bf16_t* __restrict__ w_ukt,
     const float* __restrict__ cos_t, const float* __restrict__ sin_t, bf16_t* __restrict__ out, int n, int H, int dr,
     int rank) {
