@@ -1,6 +1,6 @@
-// Prompt attention over the paged cache on the matrix cores (bfloat16), two
+// Prompt attention over the paged cache on the matrix cores (bfloat16), three
 // kernels with the same arithmetic; which one runs is decided per launch (see
-// launch_prefill at the end of this file).
+// launch_prefill at the end of this file).  attention_prompt.hpp has the one for heads of 32, 64 and 128 without a distance bias.
 //
 // Both read a request's keys from the first key any of a workgroup's queries
 // may read to the last -- earlier pages of the cache and the rows this step
@@ -11,7 +11,7 @@
 // probabilities are rounded to bfloat16 for the product with the values and
 // their sum is taken over the rounded numbers, as in the decode kernel.
 //
-// The first kernel (attn_prefill_mfma_kernel): a workgroup takes up to 128
+// The first kernel here (attn_prefill_mfma_kernel, other heads and distance biases): a workgroup takes up to 128
 // consecutive tokens of one request (a query block) and one head; each wave of
 // a group of four owns 32 of the queries.  Keys and values pass through LDS in
 // tiles of 64 keys (two blocks of 32; 32 keys for head sizes above 128, for
@@ -43,6 +43,7 @@
 
 #include "attention_f32.hpp"
 #include "attention_merge.hpp"
+#include "attention_prompt.hpp"
 #include "common.hpp"
 #include "kllm_kernels.h"
 
@@ -776,6 +777,33 @@ __global__ __launch_bounds__(64 * kPrefillWaves) __attribute__((amdgpu_waves_per
     }
 }
 
+template <int HDT>
+static void launch_prefill_merge(hipStream_t stream, void* out, const float* part, const int* query_tiles, int n_tiles, const int* span_start,
+                                 int H, int nslices, const OutGate& gate) {
+  if (nslices <= 1) return;
+  const dim3 grid(n_tiles * kQueryBlock, ceil_div(H, kMergeWaves));
+  hipLaunchKernelGGL((attn_prefill_merge_kernel<(HDT + 1) / 2>), grid, dim3(64 * kMergeWaves), 0, stream, (bf16_t*)out, part, query_tiles,
+                     span_start, H, 32 * HDT, nslices, gate);
+}
+
+constexpr bool prompt_kernel_takes(int hdt) { return hdt == 1 || hdt == 2 || hdt == 4; }
+
+template <int HDT, int PAR>
+static void launch_prompt(dim3 grid, hipStream_t stream, const void* q, void* out, const void* cache, const int* query_tiles, int n_tiles,
+                          const int* span_start, const int* span_pos, const int* block_table, int max_pages, int page_size, unsigned page_magic,
+                          int H, int KV, int window, int chunk, const float* sinks, int keep_first, float scale, const OutGate& gate, float* part) {
+  typedef PromptShape<HDT> S;
+  const size_t lds = (size_t)PAR * S::RING * 2 * S::TB;        // also holds the groups' merge
+  static int raised = 0;
+  if (lds > 64 * 1024 && !raised) {
+    (void)hipFuncSetAttribute((const void*)attn_prompt_kernel<HDT, PAR>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    raised = 1;
+  }
+  hipLaunchKernelGGL((attn_prompt_kernel<HDT, PAR>), grid, dim3(256 * PAR), lds, stream, (const bf16_t*)q, (bf16_t*)out, (const bf16_t*)cache,
+                     query_tiles, n_tiles, span_start, span_pos, block_table, max_pages, page_size, page_magic, H, KV, window, chunk, sinks,
+                     keep_first, scale, part, gate);
+}
+
 template <int HDT, int PAR>
 static void launch_prefill_par(int grid, hipStream_t stream, const void* q, void* out, const void* cache,
                                const int* query_tiles, int n_tiles, const int* span_start,
@@ -791,14 +819,16 @@ static void launch_prefill_par(int grid, hipStream_t stream, const void* q, void
     raised = 1;
   }
   const unsigned page_magic = (unsigned)(((1UL << 35) + page_size - 1) / page_size);   // ceil(2^35 / page_size)
+  if constexpr (prompt_kernel_takes(HDT))
+    if (!slopes) {
+      launch_prompt<HDT, PAR>(dim3(grid, nslices), stream, q, out, cache, query_tiles, n_tiles, span_start, span_pos, block_table, max_pages,
+                              page_size, page_magic, H, KV, window, chunk, sinks, keep_first, scale, gate, part);
+      return launch_prefill_merge<HDT>(stream, out, part, query_tiles, n_tiles, span_start, H, nslices, gate);
+    }
   hipLaunchKernelGGL((attn_prefill_mfma_kernel<HDT, PAR>), dim3(grid, nslices), dim3(64 * kPrefillWaves * PAR), lds, stream,
                      (const bf16_t*)q, (bf16_t*)out, (const bf16_t*)cache, query_tiles, n_tiles,
                      span_start, span_pos, block_table, max_pages, page_size, page_magic, H, KV, window, chunk, sinks, keep_first, scale, slopes, part, gate);
-  if (nslices > 1) {
-    const dim3 mgrid(n_tiles * kQueryBlock, ceil_div(H, kMergeWaves));
-    hipLaunchKernelGGL((attn_prefill_merge_kernel<(HDT + 1) / 2>), mgrid, dim3(64 * kMergeWaves), 0, stream,
-                       (bf16_t*)out, part, query_tiles, span_start, H, 32 * HDT, nslices, gate);
-  }
+  launch_prefill_merge<HDT>(stream, out, part, query_tiles, n_tiles, span_start, H, nslices, gate);
 }
 
 template <int HDT>
@@ -819,23 +849,40 @@ static void launch_prefill_split(int n_tiles, hipStream_t stream, const void* q,
                      span_start, span_pos, block_table, max_pages, page_size, H, KV, window, chunk, sinks, scale, slopes, gate);
 }
 
-// Which kernel.  One group of waves with the keys through LDS (three workgroups a CU) when
+// Groups of four waves to a block of attn_prompt_kernel.  One group: a CU holds up to three blocks, and the longest block's chain of tiles, or
+// the CU's share of all of them, follows on what a workgroup costs beside its tiles.  Two groups: a CU holds one block at a time, each with that
+// cost, but a chain is half as long.  In us, per 64 keys.  (One group / two, measured: heads of 64, 2,048 tokens of 32 heads 37 / 35, 1,500
+// 28 / 24, four prompts of 300 10.9 / 15.5, 17 blocks of three prompts 22 / 26, 8,192 tokens 341 / 342, 45 tokens 5.4 / 6.2; heads of 128, 2,048 59 / 51,
+// three prompts 32 / 35, 480 behind 480 27 / 21, four prompts of 300 16 / 22.)
+static int prompt_groups(int hdt, int grid, int H, long keys_total, int keys_longest) {
+  const int cus = device_cus();
+  if (keys_total <= 0 || keys_longest <= 0) return grid > 2 * cus ? 1 : 2;      // not known
+  const float longest = keys_longest / 64.f, share = (float)keys_total * H / (64.f * cus);
+  const bool wide = hdt > 2;
+  const float one = 5.f + fmaxf(longest * (wide ? 1.45f : 0.85f), share * (wide ? 1.1f : 0.65f));
+  const float two = 1.5f + 4.5f * ceil_div(grid, cus) + fmaxf(longest, share) * (wide ? 1.1f : 0.6f);
+  return two < one ? 2 : 1;
+}
+
+// Which kernel.  Heads of 32, 64 and 128 without a distance bias run on attn_prompt_kernel (prompt_groups says with how many groups), but for
+// a few blocks with short chains, whose keys the small workgroups of attn_prefill_split_kernel share out more finely: heads of 64, one to four tiles
+// of keys and more on a quarter of the CUs (100 tokens of 32 heads 6.4 us there, 6.8 here; 256 7.7 / 8.3; 100 behind 250 9.4 / 9.8; but 45
+// tokens 6.0 / 5.4, 100 behind 1,000 18.1 / 16.3, 300 tokens 10.4 / 8.6, six spans of 60 behind 200 13.0 / 9.1); heads of 32 on three
+// quarters of the CUs (16 heads, 1,024 tokens 10.8 / 11.5).
+// The others: one group of waves with the keys through LDS (three workgroups a CU) when
 // there are more than two query blocks per CU: the CUs are full and the traffic decides.  With
 // fewer, a block's chain of tiles takes about 2,700 cycles a tile whatever else the CU holds;
 // two groups of waves that take the tiles in turn (one workgroup a CU, longest blocks first)
 // bring a pair of tiles to 3,900 cycles.  That pays when the longest chain bounds the time:
-// whole prompts, whose later blocks read more keys (32 heads, one prompt, us with one group ->
-// two: head 64, 2,048 tokens 47.7 -> 42.9, 1,500 tokens 36.3 -> 27.9; 24 heads of 96, 2,048
-// tokens 60.7 -> 46.8; head 128, 2,048 tokens 74.4 -> 69.6), or one block per CU.  It does not
+// whole prompts, whose later blocks read more keys (24 heads of 96, 2,048
+// tokens, us with one group -> two: 60.7 -> 46.8), or one block per CU.  It does not
 // when every block has a long chain and a CU holds two of them, a portion of a prompt far into
 // its context: then the CU's tiles bound the time, and one group with its blocks side by side
-// takes fewer cycles a tile (32,768 tokens in portions of 2,048: 237 ms against 252).  The
+// takes fewer cycles a tile.  The
 // caller says how many keys the blocks read together and the longest block alone
 // (`keys_total`, `keys_longest`; 0: not known, the prompt is taken to start at its beginning).
 // For heads below 128 and no more blocks than three quarters of the CUs, the keys are shared
-// out over the waves of small workgroups instead (512 tokens: 11.2 us against 12.4 with two
-// groups; 8 heads, 2,048 tokens: 28.4 against 31.8; 1,024 tokens of 32 heads, one block per CU:
-// 22.6 against 20.0).
+// out over the waves of small workgroups instead.
 template <int HDT>
 static void launch_prefill(int grid, hipStream_t stream, const void* q, void* out, const void* cache,
                            const int* query_tiles, int n_tiles, const int* span_start,
@@ -852,6 +899,20 @@ static void launch_prefill(int grid, hipStream_t stream, const void* q, void* ou
                                                         keep_first, scale, slopes, gate, part, nslices);
     return;
   }
+  if constexpr (prompt_kernel_takes(HDT))
+    if (!slopes) {
+      const bool split = HDT <= 2 && keep_first == 0 && (HDT == 1 || keys_longest == 0 ? 4 * grid <= 3 * cus
+                                                                                        : 4 * grid <= cus && keys_longest > 64 && keys_longest <= 384);
+      if (!split) {
+        if (prompt_groups(HDT, grid, H, keys_total, keys_longest) == 2)
+          launch_prefill_par<HDT, 2>(grid, stream, q, out, cache, query_tiles, n_tiles, span_start, span_pos, block_table, max_pages, page_size,
+                                     H, KV, window, chunk, sinks, keep_first, scale, slopes, gate);
+        else
+          launch_prefill_par<HDT, 1>(grid, stream, q, out, cache, query_tiles, n_tiles, span_start, span_pos, block_table, max_pages, page_size,
+                                     H, KV, window, chunk, sinks, keep_first, scale, slopes, gate);
+        return;
+      }
+    }
   bool chain_bound = true;
   if (keys_total > 0 && keys_longest > 0)   // tiles of a CU's share of all blocks against the longest block's
     chain_bound = 5 * (keys_total * H / cus) < 6 * (long)keys_longest;

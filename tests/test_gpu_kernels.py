@@ -1320,6 +1320,52 @@ def test_attention_prefill(H, KV, hd, ps, window, dtype):
         assert (out2.cpu().double() - c["want"])[rows2].abs().max() < attn_tol(dtype)
 
 
+@pytest.mark.parametrize("hd", [32, 64, 128])
+@pytest.mark.parametrize("ps", [16, 48])
+@pytest.mark.parametrize("window,keep,chunk,sink", [(0, 0, 0, False), (70, 0, 0, False), (70, 20, 0, False), (0, 0, 96, True)])
+def test_attention_prompt_edges(hd, ps, window, keep, chunk, sink):
+    """The kernel for heads of 32, 64 and 128 with one and two groups of waves (chosen by the keys the caller names) and with slices: spans that end at
+    the edges of its tiles of 32 and 64 keys and of its 128 queries, windows, chunks and kept positions that begin inside a tile, and a chain
+    of more than 64 tiles a group, whose places are looked up in turns; pages that hold no key of the request are NaN.  Against 64 bits: the
+    probabilities and the result are rounded to bfloat16."""
+    k_ = K()
+    H, KV, n_new = 16, 4, [1, 31, 32, 33, 64, 65, 127, 128, 129, 3]
+    before = [0, 0, 1, 63, 64, 31, 129, 0, 200, 8400]
+    spans = list(zip(before, n_new))
+    c = attention_case(H, KV, hd, ps, torch.bfloat16, window, spans, seed=9)
+    lens, q = c["lens"], c["q"].double()
+    used = torch.zeros(c["cache"].shape[0], dtype=torch.bool, device=DEV)
+    used[c["bt"][c["bt"] >= 0].long()] = True
+    c["cache"][~used] = float("nan")
+    cache = c["cache"].double()
+    want = torch.empty(q.shape[0], H * hd, dtype=torch.float64, device=DEV)
+    for s, (a, b) in enumerate(spans):
+        pages = cache[c["bt"][s, :-(-lens[s] // ps)].long()]
+        kk = pages[:, 0].reshape(-1, KV, ps, hd).transpose(1, 2).reshape(-1, KV, hd)[:lens[s]].repeat_interleave(H // KV, 1)
+        vv = pages[:, 1].reshape(-1, KV, hd, ps).permute(0, 3, 1, 2).reshape(-1, KV, hd)[:lens[s]].repeat_interleave(H // KV, 1)
+        i, j = torch.arange(a, a + b, device=DEV)[:, None], torch.arange(lens[s], device=DEV)[None, :]
+        seen = j <= i
+        if window:
+            seen &= (i - j < window) | (j < keep)
+        if chunk:
+            seen &= j >= i // chunk * chunk
+        row0 = int(c["span_start"][s])
+        qs = q[row0:row0 + b].view(b, H, hd)
+        for h in range(H):
+            w = torch.exp((qs[:, h] @ kk[:, h].T.contiguous()) * c["scale"]) * seen
+            want[row0:row0 + b, h * hd:(h + 1) * hd] = (w @ vv[:, h]) / (w.sum(1, keepdim=True) + (1.0 if sink else 0.0))
+    tiles = [(t, s) for s, b in enumerate(n_new) for t in range(int(c["span_start"][s]), int(c["span_start"][s]) + b, k_.PREFILL_QUERY_BLOCK)]
+    qt = torch.tensor(tiles, dtype=torch.int32, device=DEV)
+    sinks = torch.zeros(H, dtype=torch.float32, device=DEV) if sink else False
+    slices = k_.attn_prefill_slices(len(tiles), H, hd)
+    for keys, nslices in (((1000, 64), 1), ((10 ** 9, 1000), 1), ((2000, 1000), 1), ((20000, 9000), slices)):
+        out = torch.full_like(c["q"], float("nan"))
+        k_.attn_prefill(c["q"], out, c["cache"], qt, len(tiles), c["span_start"], c["span_pos"], c["bt"], ps, H, KV, hd, window, c["scale"],
+                        *keys, nslices=nslices, chunk=chunk, sink=sinks, keep_first=keep)
+        assert torch.isfinite(out).all()
+        assert (out.double() - want).abs().max() < attn_tol(torch.bfloat16), keys
+
+
 def test_attention_prefill_refuses_tables_beyond_its_page_arithmetic():
     """The prompt kernel finds a key's page with a multiplication that is exact for
     requests of up to 2^24 tokens and pages of up to 2,048: a wider block table or a
