@@ -9,7 +9,8 @@
 // subtracted, online over tiles of 32 keys so that no score matrix exists.
 //
 // One wave is one work item with 32 columns:
-//   prompt   32 consecutive tokens of one request and one head: column c is
+//   prompt   (heads that are no multiple of 32 or above 128, pages that are no multiple of 16: the others run on attention_f32_prompt.hpp)
+//            32 consecutive tokens of one request and one head: column c is
 //            token t0 + c, each with its own causal bound
 //   decode   one token, one KV head and up to 32 query heads of its group:
 //            column c is head c, all with the token's bound; the token's keys
@@ -40,6 +41,7 @@
 #include <math.h>
 
 #include "attention_f32.hpp"
+#include "attention_f32_prompt.hpp"
 #include "attention_merge.hpp"
 #include "common.hpp"
 #include "kllm_kernels.h"
@@ -757,6 +759,23 @@ int attn_f32_decode(const float* q, float* out, float* part, const float* cache,
   return 0;
 }
 
+template <int HDT>
+static int launch_f32_prompt(const AttnF32Args& a, hipStream_t stream) {
+  const size_t lds = (size_t)kF32Waves * 2 * F32PromptShape<HDT>::TB;
+  static int raised = 0;
+  if (lds > 64 * 1024 && !raised) {
+    hipError_t e = hipFuncSetAttribute((const void*)attn_f32_prompt_kernel<HDT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) KLLM_FAIL((int)e, "attention float32: cannot raise the LDS limit: %s", hipGetErrorString(e));
+    raised = 1;
+  }
+  const long grid = (long)a.count * 4 * a.H;
+  KLLM_REQUIRE(grid < (1L << 31), "attention float32: %ld work items do not fit a grid", grid);
+  hipLaunchKernelGGL(attn_f32_prompt_kernel<HDT>, dim3((unsigned)grid), dim3(64 * kF32Waves), lds, stream, a.q, a.out, a.cache, a.query_tiles,
+                     a.count, a.span_start, a.span_pos, a.block_table, a.max_pages, a.page_size, a.H, a.KV, a.window, a.chunk, a.sinks, a.scale,
+                     a.slopes, a.gate);
+  return 0;
+}
+
 int attn_f32_prefill(const float* q, float* out, const float* cache, const int* query_tiles, int n_tiles,
                      const int* span_start, const int* span_pos, const int* block_table, int max_pages,
                      int page_size, int H, int KV, int hd, int window, int chunk, const float* sinks, float scale, const float* slopes,
@@ -770,6 +789,13 @@ int attn_f32_prefill(const float* q, float* out, const float* cache, const int* 
   a.block_table = block_table; a.count = n_tiles;
   a.max_pages = max_pages; a.page_size = page_size; a.H = H; a.KV = KV; a.hd = hd; a.window = window; a.chunk = chunk; a.sinks = sinks; a.gate = gate;
   a.scale = scale; a.slopes = slopes; a.nslices = 1; a.col_blocks = 1;
+  if (page_size % 16 == 0 && hd % 32 == 0 && hd <= 128) {
+    const int rc = hd == 32 ? launch_f32_prompt<1>(a, stream) : hd == 64 ? launch_f32_prompt<2>(a, stream)
+                 : hd == 96 ? launch_f32_prompt<3>(a, stream) : launch_f32_prompt<4>(a, stream);
+    if (rc) return rc;
+    KLLM_CHECK_LAUNCH("attn_prefill float32");
+    return 0;
+  }
   const long items = (long)n_tiles * 4 * H;
   if (int rc = dispatch_f32<false>(a, items, stream)) return rc;
   KLLM_CHECK_LAUNCH("attn_prefill float32");

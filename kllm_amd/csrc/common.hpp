@@ -257,6 +257,17 @@ __device__ __forceinline__ unsigned divided(unsigned x, unsigned d, unsigned mag
 }
 constexpr float kLog2E = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
 
+// e^x for x <= 0 (also -inf), to two units in the last place: the hardware's 2^p for p = x log2(e) as rounded, times 2^(what the rounding
+// left), which is small enough for two terms.  Half the instructions of expf, which has positive x and results below 2^-126 to look after
+// (here 0, beside a sum of at least 1).
+__device__ __forceinline__ float exp_negative(float x) {
+  x = fmaxf(x, -1e4f);
+  const float p = x * kLog2E;
+  const float rest = fmaf(x, 1.925963033e-8f, fmaf(x, kLog2E, -p));          // log2(e) is kLog2E (as rounded to 32 bits) + 1.926e-8
+  const float y = __builtin_amdgcn_exp2f(p);
+  return fmaf(y * kLn2, rest, y);
+}
+
 // The greatest of the first R lanes' values (-infinity in the others), the same in every lane.
 template <int R>
 __device__ __forceinline__ float first_lanes_max(float v) {

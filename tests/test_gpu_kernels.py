@@ -1709,6 +1709,44 @@ def test_attention_decode_weights_float32(hd, H, slices):
     assert err < 24 * 2.0 ** -24, float(err) * 2 ** 24
 
 
+@pytest.mark.parametrize("hd", [32, 64, 96, 128])
+def test_attention_prompt_weights_float32(hd):
+    """The same for the prompt kernel, whose waves take the tiles of 32 keys in turn: what rounds is as above, with the sum of a
+    column's two lanes and four waves."""
+    x = -(83.0 * torch.arange(hd) / hd).to(torch.float32)
+    H, scale, ps = 8, 0.125, 16
+    pages = hd // ps
+    table = torch.arange(pages, dtype=torch.int32, device=DEV).flip(0).contiguous()
+    cache = torch.zeros(pages, 2, 1, ps * hd, device=DEV)
+    for j in range(hd):
+        page = int(table[j // ps])
+        cache[page, 0, 0].view(ps, hd)[j % ps, 0] = 8.0 * x[j]
+        cache[page, 1, 0].view(hd, ps)[j, j % ps] = 1.0
+    q = torch.zeros(1, H * hd, device=DEV)
+    q.view(H, hd)[:, 0] = 1.0
+    ints = lambda *v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    out = torch.full_like(q, float("nan"))
+    K().attn_prefill(q, out, cache, ints(0, 0), 1, ints(0, 1), ints(hd - 1), table.view(1, -1), ps, H, 1, hd, 0, scale)
+    want = torch.softmax(x.double(), 0)
+    err = (out.cpu().double().view(H, hd) / want - 1).abs().max()
+    assert err < 24 * 2.0 ** -24, float(err) * 2 ** 24
+
+
+@pytest.mark.parametrize("H,KV,hd,ps", [(4, 2, 32, 16), (16, 4, 64, 48), (3, 3, 96, 32), (8, 1, 128, 16)])
+@pytest.mark.parametrize("window", [0, 70])
+def test_attention_prompt_edges_float32(H, KV, hd, ps, window):
+    """The float32 prompt kernel where its tiles of 32 keys and blocks of 32 tokens begin and end, with chains of more than 32 tiles a wave (a
+    wave's places are looked up 32 tiles at a time), pages that hold no key of the request NaN; sums in another order: 2e-5 as elsewhere here."""
+    spans = [(0, 1), (0, 31), (1, 32), (31, 33), (64, 64), (129, 65), (0, 129), (4200, 3)]
+    c = attention_case(H, KV, hd, ps, torch.float32, window, spans, seed=10)
+    used = torch.zeros(c["cache"].shape[0], dtype=torch.bool, device=DEV)
+    used[c["bt"][c["bt"] >= 0].long()] = True
+    c["cache"][~used] = float("nan")
+    out, rows = run_prefill(c)
+    assert rows.all() and torch.isfinite(out).all()
+    assert (out.cpu().double() - c["want"]).abs().max() < attn_tol(torch.float32)
+
+
 @pytest.mark.parametrize("hd", [64, 128])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_attention_merge_reads_its_own_slices(hd, dtype):
