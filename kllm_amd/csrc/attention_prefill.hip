@@ -52,10 +52,7 @@ namespace kllm {
 constexpr int kPrefillWaves = 4;
 constexpr int kQueryBlock = 32 * kPrefillWaves;   // queries of a workgroup
 // Limits of the division-free page arithmetic (page_magic in the first kernel).
-constexpr int kPrefillMaxPage = 2048;
-constexpr int kPrefillMaxKeys = 1 << 24;
 constexpr int kPrefillMaxSlices = 4;              // workgroups that may share out the keys of one block and head
-constexpr int kPrefillSliceFromKeys = 1280;       // ... when the longest block reads at least this many
 
 template <int HDT>
 struct PrefillShape {
@@ -847,21 +844,6 @@ static void launch_prefill_split(int n_tiles, hipStream_t stream, const void* q,
   hipLaunchKernelGGL(attn_prefill_split_kernel<HDT>, dim3(grid), dim3(64 * kPrefillWaves), lds, stream,
                      (const bf16_t*)q, (bf16_t*)out, (const bf16_t*)cache, query_tiles, n_tiles,
                      span_start, span_pos, block_table, max_pages, page_size, H, KV, window, chunk, sinks, scale, slopes, gate);
-}
-
-// Groups of four waves to a block of attn_prompt_kernel.  One group: a CU holds up to three blocks, and the longest block's chain of tiles, or
-// the CU's share of all of them, follows on what a workgroup costs beside its tiles.  Two groups: a CU holds one block at a time, each with that
-// cost, but a chain is half as long.  In us, per 64 keys.  (One group / two, measured: heads of 64, 2,048 tokens of 32 heads 37 / 35, 1,500
-// 28 / 24, four prompts of 300 10.9 / 15.5, 17 blocks of three prompts 22 / 26, 8,192 tokens 341 / 342, 45 tokens 5.4 / 6.2; heads of 128, 2,048 59 / 51,
-// three prompts 32 / 35, 480 behind 480 27 / 21, four prompts of 300 16 / 22.)
-static int prompt_groups(int hdt, int grid, int H, long keys_total, int keys_longest) {
-  const int cus = device_cus();
-  if (keys_total <= 0 || keys_longest <= 0) return grid > 2 * cus ? 1 : 2;      // not known
-  const float longest = keys_longest / 64.f, share = (float)keys_total * H / (64.f * cus);
-  const bool wide = hdt > 2;
-  const float one = 5.f + fmaxf(longest * (wide ? 1.45f : 0.85f), share * (wide ? 1.1f : 0.65f));
-  const float two = 1.5f + 4.5f * ceil_div(grid, cus) + fmaxf(longest, share) * (wide ? 1.1f : 0.6f);
-  return two < one ? 2 : 1;
 }
 
 // Which kernel.  Heads of 32, 64 and 128 without a distance bias run on attn_prompt_kernel (prompt_groups says with how many groups), but for

@@ -26,6 +26,10 @@
 
 namespace kllm {
 
+constexpr int kPrefillMaxPage = 2048;
+constexpr int kPrefillMaxKeys = 1 << 24;
+constexpr int kPrefillSliceFromKeys = 1280;       // the keys of a block go in slices when the longest block reads at least this many
+
 template <int HDT>
 struct PromptShape {
   static constexpr int hd = 32 * HDT;
@@ -39,12 +43,12 @@ struct PromptShape {
 };
 
 template <int HDT, int PAR>  // head_dim = 32 * HDT; PAR groups of four waves
-__global__ __launch_bounds__(256 * PAR) __attribute__((amdgpu_waves_per_eu(PAR == 1 && HDT <= 2 ? 3 : 2))) void attn_prompt_kernel(
+__device__ __forceinline__ void attn_prompt_block(
     const bf16_t* __restrict__ q, bf16_t* __restrict__ out, const bf16_t* __restrict__ cache,
     const int* __restrict__ query_tiles, int n_tiles, const int* __restrict__ span_start,
     const int* __restrict__ span_pos, const int* __restrict__ block_table, int max_pages,
     int page_size, unsigned page_magic, int H, int KV, int window, int chunk, const float* __restrict__ sinks, int keep_first,
-    float scale, float* __restrict__ part, const OutGate gate) {
+    float scale, float* __restrict__ part, const OutGate gate, int place, int slice, int nslices) {
   typedef PromptShape<HDT> S;
   constexpr int hd = S::hd, KS = S::KS, NB = S::NB, KT = S::KT, CH = S::CH, TB = S::TB, DI = S::DI, RING = S::RING;
   extern __shared__ __attribute__((aligned(1024))) unsigned char ring_lds[];   // [PAR][RING][keys, values][TB]
@@ -52,13 +56,13 @@ __global__ __launch_bounds__(256 * PAR) __attribute__((amdgpu_waves_per_eu(PAR =
   const int wave8 = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int par = wave8 / 4, wave = wave8 % 4;               // the group: tiles par, par + PAR, ...
   const int g = lane / 32, c = lane % 32;
-  const int item = blockIdx.x;                                // (block, head), head fastest
+  const int item = place;                                // (block, head), head fastest
   // Later blocks read more keys.  With several workgroups a CU (one group) the later half of the list starts first, longest block first, then
   // the earlier half, shortest first, so that a CU gets a long and a short one; with one workgroup a CU longest first throughout.
-  const int place = item / H, n_late = (n_tiles + 1) / 2;
+  const int turn = item / H, n_late = (n_tiles + 1) / 2;
   int h = item % H;
   if (H % 8 == 0) h = h % 8 * (H / 8) + h / 8;               // neighbouring heads, which share keys, on one XCD
-  const int blk = (PAR == 2 || place < n_late) ? n_tiles - 1 - place : place - n_late;
+  const int blk = (PAR == 2 || turn < n_late) ? n_tiles - 1 - turn : turn - n_late;
   const int kvh = h / (H / KV);
   const int t0 = __builtin_amdgcn_readfirstlane(query_tiles[2 * blk]);
   const int span = __builtin_amdgcn_readfirstlane(query_tiles[2 * blk + 1]);
@@ -86,12 +90,11 @@ __global__ __launch_bounds__(256 * PAR) __attribute__((amdgpu_waves_per_eu(PAR =
     qb[kk] = *reinterpret_cast<const bf16x8*>(q + ((long)tq * H + h) * hd + 16 * kk + 8 * g);
 
   // Kept first positions: the keys below kept_end (none of them in the tiles from kb0 on) come first, in n_kept tiles of their own from key
-  // 0; pages between them and kb0 may be gone.  The tiles go in turn to the slices (blockIdx.y) and, within a slice, to the groups.
+  // 0; pages between them and kb0 may be gone.  The tiles go in turn to the slices and, within a slice, to the groups.
   const int kb0 = lowest / 32 * 32;
   const int kept_end = min(keep_first, kb0);
   const int n_kept = (kept_end + KT - 1) / KT;
   const int ntiles_all = (blk_qmax - kb0) / KT + 1 + n_kept;
-  const int nslices = gridDim.y, slice = blockIdx.y;
   const int ntiles = (ntiles_all + PAR * nslices - 1) / (PAR * nslices);   // steps of the loop: the same for all
   auto tile_no = [&](int t) { return nslices * (PAR * t + par) + slice; };
   auto first_of = [&](int n) { return n < n_kept ? KT * n : kb0 + KT * (n - n_kept); };   // first key of a tile
@@ -354,6 +357,32 @@ __global__ __launch_bounds__(256 * PAR) __attribute__((amdgpu_waves_per_eu(PAR =
   if (gate.side) store(gate.side);
   else store(std::integral_constant<int, 1>());
 #undef KLLM_VM_WAIT
+}
+
+template <int HDT, int PAR>
+__global__ __launch_bounds__(256 * PAR) __attribute__((amdgpu_waves_per_eu(PAR == 1 && HDT <= 2 ? 3 : 2))) void attn_prompt_kernel(
+    const bf16_t* __restrict__ q, bf16_t* __restrict__ out, const bf16_t* __restrict__ cache,
+    const int* __restrict__ query_tiles, int n_tiles, const int* __restrict__ span_start,
+    const int* __restrict__ span_pos, const int* __restrict__ block_table, int max_pages,
+    int page_size, unsigned page_magic, int H, int KV, int window, int chunk, const float* __restrict__ sinks, int keep_first,
+    float scale, float* __restrict__ part, const OutGate gate) {
+  attn_prompt_block<HDT, PAR>(q, out, cache, query_tiles, n_tiles, span_start, span_pos, block_table, max_pages, page_size, page_magic, H, KV, window,
+                              chunk, sinks, keep_first, scale, part, gate, blockIdx.x, blockIdx.y, gridDim.y);
+}
+
+// Groups of four waves to a block of attn_prompt_kernel.  One group: a CU holds up to three blocks, and the longest block's chain of tiles, or
+// the CU's share of all of them, follows on what a workgroup costs beside its tiles.  Two groups: a CU holds one block at a time, each with that
+// cost, but a chain is half as long.  In us, per 64 keys.  (One group / two, measured: heads of 64, 2,048 tokens of 32 heads 37 / 35, 1,500
+// 28 / 24, four prompts of 300 10.9 / 15.5, 17 blocks of three prompts 22 / 26, 8,192 tokens 341 / 342, 45 tokens 5.4 / 6.2; heads of 128, 2,048 59 / 51,
+// three prompts 32 / 35, 480 behind 480 27 / 21, four prompts of 300 16 / 22.)
+inline int prompt_groups(int hdt, int grid, int H, long keys_total, int keys_longest) {
+  const int cus = device_cus();
+  if (keys_total <= 0 || keys_longest <= 0) return grid > 2 * cus ? 1 : 2;      // not known
+  const float longest = keys_longest / 64.f, share = (float)keys_total * H / (64.f * cus);
+  const bool wide = hdt > 2;
+  const float one = 5.f + fmaxf(longest * (wide ? 1.45f : 0.85f), share * (wide ? 1.1f : 0.65f));
+  const float two = 1.5f + 4.5f * ceil_div(grid, cus) + fmaxf(longest, share) * (wide ? 1.1f : 0.6f);
+  return two < one ? 2 : 1;
 }
 
 }  // namespace kllm

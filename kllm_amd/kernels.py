@@ -142,6 +142,7 @@ def _declare(lib):
         "kllm_calibrate_mfma": [I, I, P, P, P],
         "kllm_attn_decode": [P, P, P, L, P, P, P, P, I, I, I, I, I, I, I, I, P, I, F, P, I, I, P, I, P, I, L, L, I, I, P],
         "kllm_attn_prefill": [P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, P, I, F, P, L, I, P, L, I, I, I, P, I, L, L, I, I, P],
+        "kllm_attn_step": [P, P, P, L, P, P, P, P, I, I, I, I, I, I, I, I, P, I, F, P, I, I, P, I, P, I, P, P, L, I, P, L, I, P, I, L, L, I, I, P],
         "kllm_attn_prefill_slices": [I, I, I],
         "kllm_gemm_rope": [P, P, P, I, I, I, P],
         "kllm_gemm_act": [P, P, P, I, I, I, I, I, P, P],
@@ -201,7 +202,7 @@ def _declare(lib):
 LAUNCHING = ("kllm_embed", "kllm_add_rmsnorm", "kllm_rope_tables", "kllm_rope_append", "kllm_silu_mul",
              "kllm_sum_splits", "kllm_gemm", "kllm_gemm_swiglu", "kllm_gemv_plain", "kllm_gemv_swiglu",
              "kllm_gemv_resid", "kllm_gemv_rope_append", "kllm_fused_linear", "kllm_linear_rows", "kllm_attn_generic",
-             "kllm_attn_decode", "kllm_attn_prefill", "kllm_sample", "kllm_gemm_act", "kllm_gemm_rope", "kllm_add_sinusoid", "kllm_unary_act",
+             "kllm_attn_decode", "kllm_attn_prefill", "kllm_attn_step", "kllm_sample", "kllm_gemm_act", "kllm_gemm_rope", "kllm_add_sinusoid", "kllm_unary_act",
              "kllm_group_norm_add", "kllm_qk_norm_append", "kllm_delta_prep", "kllm_delta_scan", "kllm_delta_out",
              "kllm_norm_residual", "kllm_rope_tables_freq", "kllm_qkv_norm_append", "kllm_gate_bias", "kllm_moe_route",
              "kllm_moe_plan", "kllm_moe_expert", "kllm_moe_expert_rows", "kllm_moe_combine",
@@ -210,7 +211,7 @@ LAUNCHING = ("kllm_embed", "kllm_add_rmsnorm", "kllm_rope_tables", "kllm_rope_ap
              "kllm_linear_recurrence_scan", "kllm_latent_kv_append", "kllm_latent_norm", "kllm_latent_query", "kllm_attn_latent",
              "kllm_latent_out", "kllm_scaled_sum", "kllm_normed_sum", "kllm_qkv_conv_append", "kllm_decayed_prep",
              "kllm_decayed_scan", "kllm_decayed_out", "kllm_decayed_step", "kllm_token_gate", "kllm_soft_cap")
-DYNAMIC_ARGS = {"kllm_attn_prefill": (19, 20)}     # arguments that may be a StepValue
+DYNAMIC_ARGS = {"kllm_attn_prefill": (19, 20), "kllm_attn_step": (28, 29)}     # arguments that may be a StepValue
 STRUCT_ARGS = {"kllm_gemv_plain": (7,), "kllm_gemv_swiglu": (8,), "kllm_gemv_rope_append": (17,),
                "kllm_fused_linear": (2,), "kllm_linear_rows": (2,), "kllm_gemm_rope": (1,)}
 
@@ -1363,6 +1364,35 @@ def attn_decode(q, out, part, cache, positions, span_of_token, block_table, page
         int(nslices), dtype_code(q.dtype),
         _ptr(token_list, "attn token_list", torch.int32, True), int(n_listed),
         *_out_gate(gate, n, n_heads, head_dim, "attn_decode"), side, _stream())
+
+
+def attn_step(q, out, part, cache, positions, span_of_token, block_table, page_size, n_heads, n_kv_heads, head_dim, window, scale,
+              nslices, token_list, n_listed, query_tiles, n_tiles, span_start, span_pos, keys_total, keys_longest, block_part=None,
+              block_slices=1, slopes=None, chunk=0, sink=False, keep_first=0, gate=None):
+    """``attn_decode`` for the tokens of ``token_list`` and ``attn_prefill`` for the blocks of ``query_tiles`` in one call, and in one
+    launch where the library has one for the step (``block_part``, ``block_slices``: ``attn_prefill``'s ``part`` and ``nslices``)."""
+    n = q.shape[0]
+    if (tuple(q.shape) != (n, n_heads * head_dim) or tuple(out.shape) != tuple(q.shape)
+            or q.dtype != cache.dtype or out.dtype != q.dtype):
+        raise KernelError("attn_step: q/out shapes or dtypes do not fit")
+    side, out = _rows_side(out, "attn_step")
+    if tuple(cache.shape[1:]) != (2, n_kv_heads, page_size * head_dim):
+        raise KernelError(f"attn_step: cache {tuple(cache.shape)} does not fit")
+    if positions.numel() < n or span_of_token.numel() < n or token_list.numel() < n_listed or query_tiles.numel() < 2 * n_tiles:
+        raise KernelError("attn_step: index arrays are too short")
+    need = n * n_heads * block_slices * (head_dim + 2) if block_slices > 1 else 0
+    if need and (block_part is None or block_part.dtype != torch.float32 or block_part.numel() < need):
+        raise KernelError(f"attn_step: {block_slices} slices of the blocks' keys need {need} floats of room")
+    _launch("kllm_attn_step", "attn_step", _ptr(q, "attn q"), _ptr(out, "attn out"), _ptr(part, "attn part", torch.float32), part.numel(),
+            _ptr(cache, "attn cache"), _ptr(positions, "attn positions", torch.int32), _ptr(span_of_token, "attn span_of_token", torch.int32),
+            _ptr(block_table, "attn block_table", torch.int32), block_table.shape[1], page_size, n, n_heads, n_kv_heads, head_dim,
+            int(window), int(chunk), _sinks(sink, n_heads, q.device, "attn_step"), int(keep_first), float(scale),
+            _slopes(slopes, n_heads, "attn_step"), int(nslices), dtype_code(q.dtype), _ptr(token_list, "attn token_list", torch.int32),
+            int(n_listed), _ptr(query_tiles, "attn query_tiles", torch.int32), n_tiles, _ptr(span_start, "attn span_start", torch.int32),
+            _ptr(span_pos, "attn span_pos", torch.int32), keys_total if type(keys_total) is StepValue else int(keys_total),
+            keys_longest if type(keys_longest) is StepValue else int(keys_longest),
+            _ptr(block_part, "attn block_part", torch.float32, True) if need else 0, need, int(block_slices),
+            *_out_gate(gate, n, n_heads, head_dim, "attn_step"), side, _stream())
 
 
 def sample(out, logits, temperature=None, uniform=None):

@@ -312,20 +312,27 @@ class CausalSelfAttention(Part):
         if n_short + n_blocks == 0 or (n_blocks and not prompt_ok):   # a context built by hand may carry no lists
             self._decode(ctx, q, out, cache, None, n, gate)   # token by token
             return
-        if n_short:
+        if not n_blocks:
             self._decode(ctx, q, out, cache, None if n_short == n else short, n_short, gate)
-        if n_blocks:
-            total, longest = self._keys_read(ctx)
-            part = None
-            slices = (1 if self.runtime.options.get("no_attention_slices")
-                      else K.attn_prefill_slices(n_blocks, self.heads, self.head_dim, q.dtype))
-            if slices > 1:     # few blocks of a large head: their keys in slices over workgroups, merged in the same call
-                part = ctx.buf("attn.block_part", (n * self.heads * slices * (self.head_dim + 2),), torch.float32)
-            K.attn_prefill(q, out, cache.pages, blocks, n_blocks, ctx.span_start,
-                           ctx.span_pos, cache.block_table, cache.page_size, self.heads,
-                           self.kv_heads, self.head_dim, self.window, self.scale, total, longest, part=part,
-                           nslices=slices, slopes=self.slopes, chunk=self.chunk, sink=self.sinks,
-                           keep_first=self.keep_first, gate=gate)
+            return
+        total, longest = self._keys_read(ctx)
+        part = None
+        slices = (1 if self.runtime.options.get("no_attention_slices")
+                  else K.attn_prefill_slices(n_blocks, self.heads, self.head_dim, q.dtype))
+        if slices > 1:     # few blocks of a large head: their keys in slices over workgroups, merged in the same call
+            part = ctx.buf("attn.block_part", (n * self.heads * slices * (self.head_dim + 2),), torch.float32)
+        if n_short:        # both: in one launch where that is faster
+            nslices, token_part = self._decode_slices(ctx, q, cache, n_short)
+            K.attn_step(q, out, token_part, cache.pages, ctx.positions, ctx.span_of_token, cache.block_table, cache.page_size,
+                        self.heads, self.kv_heads, self.head_dim, self.window, self.scale, nslices, short, n_short, blocks, n_blocks,
+                        ctx.span_start, ctx.span_pos, total, longest, part, slices, slopes=self.slopes, chunk=self.chunk,
+                        sink=self.sinks, keep_first=self.keep_first, gate=gate)
+            return
+        K.attn_prefill(q, out, cache.pages, blocks, n_blocks, ctx.span_start,
+                       ctx.span_pos, cache.block_table, cache.page_size, self.heads,
+                       self.kv_heads, self.head_dim, self.window, self.scale, total, longest, part=part,
+                       nslices=slices, slopes=self.slopes, chunk=self.chunk, sink=self.sinks,
+                       keep_first=self.keep_first, gate=gate)
 
     def _keys_read(self, ctx):
         """The step's key counts (see ``step_values``), as the engine worked them out for this
@@ -336,8 +343,8 @@ class CausalSelfAttention(Part):
         own = self.step_values(ctx.h_span_start, ctx.h_span_len, ctx.h_span_pos)
         return own["keys_total"], own["keys_longest"]
 
-    def _decode(self, ctx, q, out, cache, token_list, count, gate=None):
-        n = q.shape[0]
+    def _decode_slices(self, ctx, q, cache, count):
+        """(slices of the keys of ``count`` tokens, room for their partial results)."""
         # The block table's width bounds the keys of the step's longest request.  It is rounded up
         # to a power of two of pages (from 8), as recorded steps round theirs: a step then cuts
         # the keys alike, and gives the same sums bit for bit, whether it runs directly or as
@@ -351,7 +358,10 @@ class CausalSelfAttention(Part):
         if self.chunk:
             max_keys = min(max_keys, self.chunk)
         nslices = K.attn_decode_slices(count, self.kv_heads, self.heads, self.head_dim, q.dtype, max_keys, cache.page_size)
-        part = ctx.buf("attn.part", (n * self.heads * nslices * (self.head_dim + 2),), torch.float32)
+        return nslices, ctx.buf("attn.part", (q.shape[0] * self.heads * nslices * (self.head_dim + 2),), torch.float32)
+
+    def _decode(self, ctx, q, out, cache, token_list, count, gate=None):
+        nslices, part = self._decode_slices(ctx, q, cache, count)
         K.attn_decode(q, out, part, cache.pages, ctx.positions, ctx.span_of_token, cache.block_table,
                       cache.page_size, self.heads, self.kv_heads, self.head_dim, self.window,
                       self.scale, nslices, token_list, count, slopes=self.slopes, chunk=self.chunk, sink=self.sinks,

@@ -1366,6 +1366,50 @@ def test_attention_prompt_edges(hd, ps, window, keep, chunk, sink):
         assert (out.double() - want).abs().max() < attn_tol(torch.bfloat16), keys
 
 
+@pytest.mark.parametrize("hd,H,KV", [(64, 16, 4), (64, 4, 4), (128, 32, 1), (128, 8, 8), (96, 4, 2)])
+@pytest.mark.parametrize("ps,window,chunk,sink,gated", [(16, 0, 0, False, False), (48, 70, 0, False, True), (16, 0, 96, True, False)])
+def test_attention_step_against_its_two_halves(hd, H, KV, ps, window, chunk, sink, gated):
+    """Tokens of short spans and blocks of longer ones in one call, where they share a launch (heads of 64 and 128; one workgroup to a token or
+    several, groups of more than 16 heads in two tiles) and where they do not (heads of 96): rows that either leaves out keep what they
+    hold, pages without a key of a request are NaN.  The same sums as in the launches of their own, but the keys may be cut
+    otherwise: both are the bfloat16 numbers next to sums whose probabilities were rounded to bfloat16."""
+    k_ = K()
+    spans = [(0, 1), (31, 1), (700, 3), (0, 33), (64, 1), (500, 129), (2000, 2), (3, 128), (12, 4), (0, 7)]
+    c = attention_case(H, KV, hd, ps, torch.bfloat16, window, spans, seed=11)
+    used = torch.zeros(c["cache"].shape[0], dtype=torch.bool, device=DEV)
+    used[c["bt"][c["bt"] >= 0].long()] = True
+    c["cache"][~used] = float("nan")
+    n = c["q"].shape[0]
+    starts = c["span_start"].tolist()
+    short = [t for s, (_, b) in enumerate(spans) if b <= 4 and s != 4 for t in range(starts[s], starts[s] + b)]       # (span 4 in neither list)
+    tiles = [(t, s) for s, (_, b) in enumerate(spans) if b > 4 for t in range(starts[s], starts[s] + b, k_.PREFILL_QUERY_BLOCK)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    tl, qt = i32(short), i32(tiles)
+    sinks = torch.zeros(H, dtype=torch.float32, device=DEV) if sink else False
+    sums = torch.randn(n, H * hd, device=DEV)
+    gate = k_.Columns(sums, 0, H * hd) if gated else None
+    kw = dict(chunk=chunk, sink=sinks, gate=gate)
+    common = (ps, H, KV, hd, window, c["scale"])
+    blocks = k_.attn_prefill_slices(len(tiles), H, hd)
+    bpart = torch.empty(n * H * blocks * (hd + 2), device=DEV) if blocks > 1 else None
+    for nslices, keys in ((1, (2000, 640)), (7, (2000, 640)), (12, (300, 40)), (2, (9000, 1300)), (3, (0, 0))):
+        want = torch.full_like(c["q"], float("nan"))
+        got = want.clone()
+        part = torch.empty(n * H * nslices * (hd + 2), device=DEV)
+        k_.attn_decode(c["q"], want, part, c["cache"], c["pos"], c["sot"], c["bt"], *common, nslices, tl, len(short), **kw)
+        k_.attn_prefill(c["q"], want, c["cache"], qt, len(tiles), c["span_start"], c["span_pos"], c["bt"], *common, *keys, part=bpart,
+                        nslices=blocks, **kw)
+        k_.attn_step(c["q"], got, part, c["cache"], c["pos"], c["sot"], c["bt"], *common, nslices, tl, len(short), qt, len(tiles),
+                     c["span_start"], c["span_pos"], *keys, bpart, blocks, **kw)
+        rows = torch.isfinite(want).all(1)
+        assert int(rows.sum()) == n - 1 and torch.equal(torch.isfinite(got), torch.isfinite(want))
+        # (a gate's factor is at most 1)
+        assert (got[rows].float() - want[rows].float()).abs().max() < attn_tol(torch.bfloat16), (nslices, keys)
+    with pytest.raises(k_.KernelError):          # what either refuses stays refused
+        k_.attn_step(c["q"], got, part[:8], c["cache"], c["pos"], c["sot"], c["bt"], *common, 3, tl, len(short), qt, len(tiles),
+                     c["span_start"], c["span_pos"], 2000, 640, bpart, blocks, **kw)
+
+
 def test_attention_prefill_refuses_tables_beyond_its_page_arithmetic():
     """The prompt kernel finds a key's page with a multiplication that is exact for
     requests of up to 2^24 tokens and pages of up to 2,048: a wider block table or a
