@@ -341,7 +341,7 @@ __global__ void silu_mul_kernel(const TIN* __restrict__ gu, int nsplit, long spl
     const TIN* row = gu + t * 2 * f;
     const float g = sum_splits(row + i, nsplit, split_stride);
     const float u = sum_splits(row + f + i, nsplit, split_stride);
-    out[idx] = from_f32<TOUT>(gate_act(g, act) * u);
+    out[idx] = from_f32<TOUT>(gate_act<TOUT>(g, act) * u);
   }
 }
 

@@ -380,7 +380,7 @@ __global__ __launch_bounds__(64 * NW) void fused_linear_kernel(const T* __restri
               a_pos = softplus_f32(out.norm_w[0]);
               a_neg = softplus_f32(out.norm_w[1]);
             }
-            reinterpret_cast<T*>(out.y)[(long)xr * m + row] = from_f32<T>(unary_act(v, out.act - FL_UNARY, a_pos, a_neg));
+            reinterpret_cast<T*>(out.y)[(long)xr * m + row] = from_f32<T>(unary_act<T>(v, out.act - FL_UNARY, a_pos, a_neg));
           } else {
             reinterpret_cast<float*>(out.y)[((long)blockIdx.y * n + xr) * m + row] = v;
           }
@@ -425,7 +425,7 @@ __global__ __launch_bounds__(64 * NW) void fused_linear_kernel(const T* __restri
         }
         if (EP == FL_SWIGLU) {
           T* h = reinterpret_cast<T*>(out.y);
-          h[(long)xr * pairs + pair] = from_f32<T>(gate_act(a, out.act) * b);
+          h[(long)xr * pairs + pair] = from_f32<T>(gate_act<T>(a, out.act) * b);
         } else {
           fl_rope_store<T>(out, xr, pair, a, b, ep_cos[t], ep_sin[t], ep_page[t], ep_slot[t]);
         }

@@ -52,6 +52,8 @@
 
 #include <math.h>
 
+#include <type_traits>
+
 #include "common.hpp"
 #include "kllm_kernels.h"
 
@@ -379,51 +381,68 @@ __global__ __launch_bounds__(512, sizeof(T) == 4 ? 6 : 2) void gemm_ring_kernel(
     return;
   }
   const bool vec = m % 4 == 0 && (reinterpret_cast<uintptr_t>(Y) & (4 * sizeof(TOUT) - 1)) == 0;
+  // KNOWN: the activation, where it has a copy of the stores of its own (-1: any).  In one copy for all, every gate of an element was worked out and one
+  // kept, and an activation went through the loop below (us, with that and now: gate of 2,048 x 11,264 x 2,048 81.1 / 80.0, of 1,999 x 28,672 x 4,096
+  // 367 / 357; 1,500 x 5,632 x 2,048 with the squared rectifier 45.8 / 37.9, with GELU 49.6 / 37.7; 1,500 x 5,632 x 1,024 33.6 / 25.3 and 37.2 / 25.3).
+  auto store = [&](auto known) __attribute__((always_inline)) {
+    constexpr int KNOWN = decltype(known)::value;
 #pragma unroll
-  for (int hx = 0; hx < 2; ++hx)
+    for (int hx = 0; hx < 2; ++hx)
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int r = row0 + hx * XR + (wr * TM + i) * 16 + lrow;
-      if (r >= n) continue;
+      for (int i = 0; i < TM; ++i) {
+        const int r = row0 + hx * XR + (wr * TM + i) * 16 + lrow;
+        if (r >= n) continue;
 #pragma unroll
-      for (int hw = 0; hw < (GATE ? 1 : 2); ++hw)
+        for (int hw = 0; hw < (GATE ? 1 : 2); ++hw)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const int c = col0 + hw * WS + (wc * TN + j) * 16 + 4 * lch;
-          typedef TOUT vec_t __attribute__((ext_vector_type(4)));
-          floatx4 q;
+          for (int j = 0; j < TN; ++j) {
+            const int c = col0 + hw * WS + (wc * TN + j) * 16 + 4 * lch;
+            typedef TOUT vec_t __attribute__((ext_vector_type(4)));
+            floatx4 q;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            q[e] = sum(hx, hw, i, j, e);
-            if (GATE) q[e] = gate_act(q[e], act) * sum(hx, 1, i, j, e);
-          }
-          if constexpr (MODE == RING_UNARY) {
-            // Larger tiles have one copy of the activations to four sums: with four the kernel's end alone is longer than the
-            // instruction cache, and at 256 x 256 its loops are no longer unrolled, so that the accumulators go through
-            // scratch memory (squared ReLU / tanh in us: 1,500 x 32,000 x 1,024 254 / 267 -> 130 / 162; 1,500 x 5,632 x 2,048 60 /
-            // 68 -> 46 / 55; 700 x 5,632 x 2,048 43 / 49 -> 35 / 40).  Tiles of 128 x 128 are faster with four (300 x 2,048
-            // x 2,048 24.2 / 28.5, with one 25.5 / 29.0).
-            if constexpr (TM * TN >= 4) {
+            for (int e = 0; e < 4; ++e) {
+              q[e] = sum(hx, hw, i, j, e);
+              if (GATE) q[e] = gate_act<TOUT>(q[e], KNOWN) * sum(hx, 1, i, j, e);
+            }
+            if constexpr (MODE == RING_UNARY) {
+              // Larger tiles have one copy of the other activations to four sums: with four the kernel's end alone is longer than the
+              // instruction cache, and at 256 x 256 its loops are no longer unrolled, so that the accumulators go through
+              // scratch memory (tanh in us: 1,500 x 32,000 x 1,024 267 -> 162; 1,500 x 5,632 x 2,048
+              // 68 -> 55; 700 x 5,632 x 2,048 49 -> 40).  Tiles of 128 x 128 are faster with four (300 x 2,048
+              // x 2,048 24.2 / 28.5, with one 25.5 / 29.0).
+              if constexpr (KNOWN < 0 && TM * TN >= 4) {
 #pragma unroll 1
-              for (int e = 0; e < 4; ++e) q = floatx4{q[1], q[2], q[3], unary_act(q[0], act, a_pos, a_neg)};
+                for (int e = 0; e < 4; ++e) q = floatx4{q[1], q[2], q[3], unary_act<TOUT>(q[0], act, a_pos, a_neg)};
+              } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) q[e] = unary_act<TOUT>(q[e], KNOWN < 0 ? act : KNOWN, a_pos, a_neg);
+              }
+            }
+            vec_t v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = from_f32<TOUT>(q[e]);
+            TOUT* dst = Y + (long)r * m + c;
+            if (vec && c + 3 < m) {
+              *reinterpret_cast<vec_t*>(dst) = v;
             } else {
 #pragma unroll
-              for (int e = 0; e < 4; ++e) q[e] = unary_act(q[e], act, a_pos, a_neg);
+              for (int e = 0; e < 4; ++e)
+                if (c + e < m) dst[e] = v[e];
             }
           }
-          vec_t v;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = from_f32<TOUT>(q[e]);
-          TOUT* dst = Y + (long)r * m + c;
-          if (vec && c + 3 < m) {
-            *reinterpret_cast<vec_t*>(dst) = v;
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (c + e < m) dst[e] = v[e];
-          }
-        }
-    }
+      }
+  };
+  if constexpr (MODE == RING_GATE) {
+    if (act == ACT_SILU) store(std::integral_constant<int, ACT_SILU>());
+    else store(std::integral_constant<int, ACT_GELU_TANH>());
+  } else if constexpr (MODE == RING_UNARY) {
+    if (act == ACT_RELU_SQ) store(std::integral_constant<int, ACT_RELU_SQ>());
+    else if (sizeof(TOUT) == 2 && act == ACT_GELU_TANH) store(std::integral_constant<int, ACT_GELU_TANH>());
+    else if (sizeof(TOUT) == 2 && act == ACT_SILU) store(std::integral_constant<int, ACT_SILU>());
+    else store(std::integral_constant<int, -1>());
+  } else {
+    store(std::integral_constant<int, -1>());
+  }
 }
 
 // ------------------------------------------------------------------ which tile, how many slices of K

@@ -290,7 +290,7 @@ __global__ __launch_bounds__(64 * GV_WAVES) void gemv_fused_kernel(
     y[(long)t * m + row_b] = mine_b;
   } else if (MODE == GV_SWIGLU) {
     T* h = reinterpret_cast<T*>(Y);
-    h[(long)t * f + pair] = from_f32<T>(gate_act(mine_a, rp.act) * mine_b);
+    h[(long)t * f + pair] = from_f32<T>(gate_act<T>(mine_a, rp.act) * mine_b);
   } else {
     const int half = rp.hd / 2;
     int page = 0, slot = 0;

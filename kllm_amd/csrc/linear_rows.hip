@@ -315,7 +315,7 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const T* __restric
           a_pos = softplus_f32(out.norm_w[0]);
           a_neg = softplus_f32(out.norm_w[1]);
         }
-        reinterpret_cast<T*>(out.y)[(long)xr * m + col] = from_f32<T>(unary_act(v, out.act - FL_UNARY, a_pos, a_neg));
+        reinterpret_cast<T*>(out.y)[(long)xr * m + col] = from_f32<T>(unary_act<T>(v, out.act - FL_UNARY, a_pos, a_neg));
       } else {
         reinterpret_cast<float*>(out.y)[(long)xr * m + col] = v;
       }
@@ -335,7 +335,7 @@ __global__ __launch_bounds__(64 * NW) void linear_rows_kernel(const T* __restric
         b *= row_scale[r];
       }
       if (EP == FL_SWIGLU) {
-        reinterpret_cast<T*>(out.y)[rows_at(out.y_tiled ? min(n, 16) : 0, xr, pair, pairs)] = from_f32<T>(gate_act(a, out.act) * b);
+        reinterpret_cast<T*>(out.y)[rows_at(out.y_tiled ? min(n, 16) : 0, xr, pair, pairs)] = from_f32<T>(gate_act<T>(a, out.act) * b);
       } else {
         const int e = EP == FL_ROPE ? u : 0;
         fl_rope_store<T>(out, xr, pair, a, b, ep_cos[e], ep_sin[e], ep_page[e], out.cache ? ep_pos[e] % out.page_size : 0);

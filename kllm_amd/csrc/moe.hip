@@ -319,9 +319,9 @@ __global__ __launch_bounds__(256) void moe_expert_kernel(const T* __restrict__ X
         if (row >= count) continue;
         const long dst = (long)sorted[start + row] * M + c;
         if (MODE == 0)
-          reinterpret_cast<T*>(out_)[dst] = from_f32<T>(gated(acc[a][b][0][e], acc[a][b][NB - 1][e], act, limit, alpha));
+          reinterpret_cast<T*>(out_)[dst] = from_f32<T>(gated<T>(acc[a][b][0][e], acc[a][b][NB - 1][e], act, limit, alpha));
         else if (MODE == 2)
-          reinterpret_cast<T*>(out_)[dst] = from_f32<T>(unary_act(acc[a][b][0][e], act, 0.f, 0.f));
+          reinterpret_cast<T*>(out_)[dst] = from_f32<T>(unary_act<T>(acc[a][b][0][e], act, 0.f, 0.f));
         else
           reinterpret_cast<float*>(out_)[dst] = acc[a][b][0][e];
       }
@@ -398,9 +398,9 @@ __global__ __launch_bounds__(256) void moe_gemv_kernel(const T* __restrict__ X, 
     if (c0 + c >= M) continue;
     const long dst = (long)entry * M + c0 + c;
     if (MODE == 0)
-      reinterpret_cast<T*>(out_)[dst] = from_f32<T>(gated(g[c], u[c], act, limit, alpha));
+      reinterpret_cast<T*>(out_)[dst] = from_f32<T>(gated<T>(g[c], u[c], act, limit, alpha));
     else if (MODE == 2)
-      reinterpret_cast<T*>(out_)[dst] = from_f32<T>(unary_act(g[c], act, 0.f, 0.f));
+      reinterpret_cast<T*>(out_)[dst] = from_f32<T>(unary_act<T>(g[c], act, 0.f, 0.f));
     else
       reinterpret_cast<float*>(out_)[dst] = g[c];
   }

@@ -41,7 +41,7 @@ __global__ void unary_act_kernel(const float* __restrict__ in, int nsplit, long 
   }
   float z = 0.f;
   for (int s = 0; s < nsplit; ++s) z += in[src + s * split_stride];
-  out[idx] = from_f32<TOUT>(unary_act(z, act, a_pos, a_neg));
+  out[idx] = from_f32<TOUT>(unary_act<TOUT>(z, act, a_pos, a_neg));
 }
 
 // out[t][j] = act(sums[t][j]) * table[id of token t][j], the table's rows `row_stride` elements apart.
@@ -60,7 +60,7 @@ __global__ void token_gate_kernel(const float* __restrict__ sums, int nsplit, lo
   const float e = to_f32(table[(long)id * row_stride + idx % f]);
   float z = 0.f;
   for (int s = 0; s < nsplit; ++s) z += sums[idx + s * split_stride];
-  out[idx] = from_f32<T>(gate_act(z, act) * e);
+  out[idx] = from_f32<T>(gate_act<T>(z, act) * e);
 }
 
 constexpr int kGroupNormThreads = 256;

@@ -1248,7 +1248,7 @@ __global__ __launch_bounds__(CH * SEGS) void linear_recurrence_scan_kernel(
     for (int q = 0; q < U; ++q) {
       if (tb + q >= a1) break;
       S = fmaf(a[q], S, b[q]);
-      const float gate = gate_act(y[q] + yb, ACT_GELU_TANH);
+      const float gate = gate_act<T>(y[q] + yb, ACT_GELU_TANH);
       if (ok) out[(long)(tb + q) * W + c] = from_f32<T>(S * gate);
     }
   }

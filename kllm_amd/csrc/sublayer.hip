@@ -525,7 +525,7 @@ __global__ void gate_bias_kernel(const float* __restrict__ gu, int nsplit, long 
     g += bias[j];
     u += bias[f + j];
   }
-  out[idx] = from_f32<TOUT>(gated(g, u, act, limit, alpha));
+  out[idx] = from_f32<TOUT>(gated<TOUT>(g, u, act, limit, alpha));
 }
 
 }  // namespace kllm

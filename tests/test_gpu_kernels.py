@@ -1912,6 +1912,28 @@ def test_prompt_projections_with_rotation_and_append(H, KV, hd, k, n, turned, ap
         assert ((one - other).abs() <= (2.0 ** -7 if dtype == torch.bfloat16 else 0.0) * other.abs() + 2.0 ** -21 * other.abs().max()).all()
 
 
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh", "sigmoid"])
+def test_gates_of_bfloat16_results(act):
+    """Over the whole range of a 32-bit number, infinities and NaN, against 64 bits: the rounding to bfloat16 (half a unit of eight bits, 2^-8 of the result at most), before it 2^-24 times what the
+    exponential is taken of (88 at most, where the result is not 0) and the rounding of a few products; results below 1e-35 may be 0."""
+    k_ = K()
+    z = torch.cat([torch.linspace(-120, 120, 20001), torch.logspace(-30, 38, 4000), -torch.logspace(-30, 38, 4000),
+                   torch.tensor([0.0, -0.0, float("inf"), -float("inf"), float("nan"), 3.4028234e38, -3.4028234e38])]).to(DEV)
+    out = torch.empty(1, z.numel(), dtype=torch.bfloat16, device=DEV)
+    k_.unary_act(z[None], out, k_.UNARY_ACTIVATIONS[act])
+    d = z.double()
+    e = d if act != "gelu_tanh" else 2 * math.sqrt(2 / math.pi) * (d + 0.044715 * d ** 3)
+    want = torch.sigmoid(e) * (1.0 if act == "sigmoid" else d)
+    got, unit = out[0].double(), 2.0 ** -8 + 88 * 2.0 ** -24 + 2.0 ** -20
+    inside = torch.isfinite(want) & (want.abs() < 3.38e38)
+    assert ((got - want).abs() <= unit * want.abs() + 1e-35)[inside].all()
+    assert torch.isnan(got[-3]) and got[-5] == want[-5]
+    if act != "sigmoid":
+        gated = torch.empty_like(out)
+        k_.silu_mul(torch.cat([z, torch.ones_like(z)])[None, None], gated, k_.ACTIVATIONS[act])
+        assert torch.equal(gated[0][inside], out[0][inside])
+
+
 @pytest.mark.parametrize("vocab", [1, 4, 63, 4096, 32000, 32003, 131072, 128256])
 def test_sample_greedy_places(vocab):
     """The first of several equal maxima wherever they lie (one thread's pieces, a wave's, the workgroup's; whole pieces of four and not), the last
