@@ -760,14 +760,15 @@ __global__ __launch_bounds__(64 * kLatWaves) void attn_latent_block_kernel(
 // The same for long steps of the common sizes (rank and rows in steps of 32): the (token, head) pairs of a
 // step in a row are columns, 128 to a workgroup and 32 to a wave, and the products are MFMA 32x32x16
 // (lane l: g = l/32, c = l%32: A[c][8g..8g+7], B[8g..8g+7][c], D[8(i/4) + 4g + i%4][c]).  Scores S^T =
-// K Q^T: A = 32 keys x 16 of their rows from LDS, B = the columns' folded queries, which stay in
-// registers; a lane holds 16 scores of one column, lane ^ 32 the other 16.  Weighted sum O^T += C^T P^T:
-// the 16 slots of MFMA u are the keys 16u + 8(j/4) + 4g + j%4, j = 0..7, which are the scores 8u + j a
-// lane holds; A = latents [element c][those keys], two 8-byte reads.
+// K Q^T: A = 32 keys x 16 of their rows from LDS, row r of it the key r with bits 2 and 3 exchanged, B = the columns' folded
+// queries, which stay in registers; a lane holds 16 scores of one column, lane ^ 32 the other 16: 8u + j that of key 16u + 8g + j.
+// Weighted sum O^T += C^T P^T: the 16 slots of MFMA u are those keys, A = latents [element c][eight neighbouring keys], one read of 16 bytes.
 //
 // A tile of 32 keys (rows, then latents with the keys side by side) goes from the pages straight into one of
 // two LDS buffers (global loads that write LDS: 16 bytes a lane, a wave's 64 pieces in a row), the
-// next tile's while this one is multiplied.  A wave cannot pad what it writes this way, so the 16-byte
+// next tile's while this one is multiplied, a load behind every two products of the scores: with a wave to a SIMD whatever is not a product stands in
+// line with them, and the loads all at once in front of the first reads from LDS kept those waiting.  Reads of 8 bytes and loads in
+// front -> now, us: 1,500 tokens of 32 heads, rank 512 156 -> 136, 700 82 -> 73, 4,000 of 16 heads 383 -> 333, 1,500 of 16 heads, rank 256 93 -> 85.  A wave cannot pad what it writes this way, so the 16-byte
 // pieces of a row change places: piece p of key row k lies at p ^ (k & row_mask), piece p of
 // element e's 32 keys at p ^ (e/4 % 4), which spreads a read over the banks.
 //
@@ -841,12 +842,12 @@ __global__ __launch_bounds__(64 * kLatWaves) __attribute__((amdgpu_waves_per_eu(
   const int v_piece = (lane % 4) ^ (lane / 16 % 4), v_half = v_piece / 2;
   const unsigned lds0 = lds_address(lat_tiles);
   // ... and where it reads them: four places each, the rest are constant distances
-  int k_at[4], v_at[4];
+  const int krow = (c & 19) | ((c & 4) << 1) | ((c & 8) >> 1);
+  int k_at[4], v_at[2];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    k_at[j] = c * row + 8 * ((2 * j + g) ^ (c & row_mask));
-    v_at[j] = c * 32 + 8 * (j ^ (c / 4 % 4)) + 4 * g;
-  }
+  for (int j = 0; j < 4; ++j) k_at[j] = krow * row + 8 * ((2 * j + g) ^ (krow & row_mask));
+#pragma unroll
+  for (int u = 0; u < 2; ++u) v_at[u] = c * 32 + 8 * ((2 * u + g) ^ (c / 4 % 4));
 
   bool over = false;
   for (int first = t_first; first <= t_last;) {
@@ -872,7 +873,11 @@ __global__ __launch_bounds__(64 * kLatWaves) __attribute__((amdgpu_waves_per_eu(
       }
       return P;
     };
-    auto fetch = [&](int kb, const Halves& P, int buf) {
+    struct Source {
+      const bf16_t *k[2], *v;                                 // the halves' rows; this lane's latents
+      unsigned lds;
+    };
+    auto source = [&](int kb, const Halves& P, int buf) -> Source {
       const bf16_t* base[2];
       int slot[2];
 #pragma unroll
@@ -883,38 +888,40 @@ __global__ __launch_bounds__(64 * kLatWaves) __attribute__((amdgpu_waves_per_eu(
         base[u] = cache + (long)(live ? page : 0) * page_elems;
         slot[u] = live ? k0 - page_index(k0) * page_size : 0;
       }
-      const unsigned k_lds = lds0 + (unsigned)(buf * buf_elems) * (unsigned)sizeof(bf16_t);
-      const unsigned v_lds = k_lds + (unsigned)(32 * row) * (unsigned)sizeof(bf16_t);
-#pragma unroll
-      for (int j = 0; j < KL; ++j) {
-        const int load = 4 * j + wave;                        // of KS
-        if (load >= KS) continue;
-        const int u = 2 * load >= KS;                         // the first KS / 2 loads are the first half's
-        load_to_lds(k_lds + 1024u * (unsigned)load, u ? base[1] + (long)slot[1] * row : base[0] + (long)slot[0] * row, k_off[j]);
-      }
       const bf16_t* v0 = base[0] + (long)page_size * row + slot[0];
       const bf16_t* v1 = base[1] + (long)page_size * row + slot[1];
-      const bf16_t* vsrc = (v_half ? v1 : v0) + 8 * (v_piece % 2) + (long)(lane / 4) * page_size;
-#pragma unroll
-      for (int j = 0; j < NB / 2; ++j) {
-        const int load = 4 * j + wave;                        // of 2 NB
-        load_to_lds(v_lds + 1024u * (unsigned)load, vsrc + (long)(16 * load) * page_size);
+      return {{base[0] + (long)slot[0] * row, base[1] + (long)slot[1] * row},
+              (v_half ? v1 : v0) + 8 * (v_piece % 2) + (long)(16 * wave + lane / 4) * page_size,
+              lds0 + (unsigned)(buf * buf_elems) * (unsigned)sizeof(bf16_t)};
+    };
+    constexpr int LOADS = KL + NB / 2;                        // of a wave for a tile: rows, then latents
+    auto fetch = [&](Source& F, int j) __attribute__((always_inline)) {
+      if (j < KL) {
+        const int load = 4 * j + wave;                        // of KS; the first KS / 2 are the first half's
+        if (KS % 4 == 0 || load < KS) load_to_lds(F.lds + 1024u * (unsigned)load, F.k[2 * load >= KS], k_off[j < KL ? j : 0]);
+      } else {
+        const int load = 4 * (j - KL) + wave;                 // of 2 NB
+        load_to_lds(F.lds + (unsigned)(32 * row) * (unsigned)sizeof(bf16_t) + 1024u * (unsigned)load, F.v);
+        F.v += 64 * (long)page_size;
+        asm volatile("" : "+v"(F.v));                         // (one address, not one for every load)
       }
     };
     const int kb0 = group_lo / 32 * 32;
     Halves pages = lookup(kb0);
     __syncthreads();                                          // the span before this one has been worked through
-    fetch(kb0, pages, 0);
+    {
+      Source F = source(kb0, pages, 0);
+#pragma unroll
+      for (int j = 0; j < LOADS; ++j) fetch(F, j);
+    }
     pages = lookup(kb0 + 32);
     int buf = 0;
     for (int kb = kb0; kb < group_len; kb += 32, buf ^= 1) {
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // this wave's part of the tile is in LDS, its reads of the last one are done
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      if (kb + 32 < group_len) {                              // (the same for all)
-        fetch(kb + 32, pages, buf ^ 1);
-        pages = lookup(kb + 64);
-      }
+      Source F = source(kb + 32, pages, buf ^ 1);       // (behind the last tile: halves that nobody reads)
+      pages = lookup(kb + 64);
       bf16_t* const ks = lat_tiles + buf * buf_elems;         // [32][row]
       bf16_t* const vs = ks + 32 * row;                       // [rank][32]
       if (kb + 32 > group_len || !half_live(kb)) {            // latents of slots that may hold anything become zeros
@@ -929,31 +936,43 @@ __global__ __launch_bounds__(64 * kLatWaves) __attribute__((amdgpu_waves_per_eu(
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
       }
-      if (!__any(mine && kb < len && kb + 32 > lo)) continue;
-      // ---- scores: this lane's key row is c
-      // (a group of pieces is read while the one before it is multiplied, and no more: registers)
-      constexpr int kGroup = 2;
+      // ---- scores: this lane's key row is krow; the next tile's loads between the products (all at once in front of them they kept
+      // the wave from its LDS reads)
+      // (kAhead groups of pieces are on their way from LDS while one is multiplied, and no more: registers; two took 156 us where one takes 136)
+      constexpr int kGroup = 2, kAhead = 1;
       floatx16 s0 = {}, s1 = {};
-      bf16x8 ka[2][kGroup];
+      bf16x8 ka[kAhead + 1][kGroup];
+      auto read_k = [&](int kk) __attribute__((always_inline)) {           // piece 2 kk + g of the row, at its swapped place
+        ka[kk / kGroup % (kAhead + 1)][kk % kGroup] = *reinterpret_cast<const bf16x8*>(ks + k_at[kk % 4] + 64 * (kk / 4));
+      };
 #pragma unroll
-      for (int j = 0; j < kGroup; ++j) ka[0][j] = *reinterpret_cast<const bf16x8*>(ks + k_at[j]);
+      for (int kk = 0; kk < kGroup * kAhead; ++kk)
+        if (kk < KS) read_k(kk);
 #pragma unroll
-      for (int k0 = 0; k0 < KS; k0 += kGroup) {               // piece 2 kk + g of the row, at its swapped place
+      for (int k0 = 0; k0 < KS; k0 += kGroup) {
 #pragma unroll
-        for (int j = 0; j < kGroup; ++j) {
-          const int kk = k0 + kGroup + j;
-          if (kk < KS) ka[(k0 / kGroup + 1) % 2][j] = *reinterpret_cast<const bf16x8*>(ks + k_at[kk % 4] + 64 * (kk / 4));
-        }
+        for (int j = 0; j < kGroup; ++j)
+          if (k0 + kGroup * kAhead + j < KS) read_k(k0 + kGroup * kAhead + j);
         __builtin_amdgcn_sched_barrier(0);
-        s0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[k0 / kGroup % 2][0], qreg[k0], s0, 0, 0, 0);
-        s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[k0 / kGroup % 2][1], qreg[k0 + 1], s1, 0, 0, 0);
+        s0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[k0 / kGroup % (kAhead + 1)][0], qreg[k0], s0, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[k0 / kGroup % (kAhead + 1)][1], qreg[k0 + 1], s1, 0, 0, 0);
+        if (k0 / kGroup < LOADS) fetch(F, k0 / kGroup);
         __builtin_amdgcn_sched_barrier(0);
       }
-      const int hi_e = mine ? len - 1 - kb - 4 * g : -1, lo_e = lo - kb - 4 * g;    // offsets that this lane's column reads
+      static_assert(LOADS <= KS / kGroup, "every load has its group");
+      bf16x8 va[kAhead + 1][2];
+      auto read_v = [&](int r) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) va[r % (kAhead + 1)][u] = *reinterpret_cast<const bf16x8*>(vs + v_at[u] + 1024 * r);
+      };
+#pragma unroll
+      for (int r = 0; r < kAhead; ++r)
+        if (r < NB) read_v(r);
+      const int hi_e = mine ? len - 1 - kb - 8 * g : -1, lo_e = lo - kb - 8 * g;    // offsets that this lane's column reads
       float tmax = -INFINITY;
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        const int e = 8 * (i / 4) + i % 4;
+        const int e = 16 * (i / 8) + i % 8;
         s0[i] = (e <= hi_e && e >= lo_e) ? (s0[i] + s1[i]) * c2 : -INFINITY;
         tmax = fmaxf(tmax, s0[i]);
       }
@@ -971,26 +990,16 @@ __global__ __launch_bounds__(64 * kLatWaves) __attribute__((amdgpu_waves_per_eu(
       }
       l += psum;
       // ---- the weighted sum of the latents
-      {
-        bf16x4 va[2][4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) va[0][j] = *reinterpret_cast<const bf16x4*>(vs + v_at[j]);
+      for (int r = 0; r < NB; ++r) {
+        if (r + kAhead < NB) read_v(r + kAhead);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int r = 0; r < NB; ++r) {
-          if (r + 1 < NB)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) va[(r + 1) % 2][j] = *reinterpret_cast<const bf16x4*>(vs + v_at[j] + 1024 * (r + 1));
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            const bf16x4 a0 = va[r % 2][2 * u], a1 = va[r % 2][2 * u + 1];
-            const bf16x8 a = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-            acc[r] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, pb[u], acc[r], 0, 0, 0);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
+        for (int u = 0; u < 2; ++u) acc[r] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[r % (kAhead + 1)][u], pb[u], acc[r], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // nothing more comes into LDS (the last tile's loads went to the other buffer)
     first = last + 1;
   }
   l += __shfl_xor(l, 32, kWave);
