@@ -23,7 +23,7 @@
 // Measured with the chip's counters: 2,271 cycles a stage of 256 x 256 where the matrix instructions
 // alone take 2,048 (90 %), whatever the caches hold.  With random operands on all CUs the chip then
 // lowers its clock (2.4 -> 1.7 GHz): power bounds the large products now, not operands.
-// Against the two-stage tiles before, in us: 2,048 x 28,672 x 4,096 (gate) 498 -> 369; 2,048 x 11,264 x
+// Against the two-stage tiles before, in us: 2,048 x 28,672 x 4,096 (gate) 498 -> 369 (357 since a gate takes less); 2,048 x 11,264 x
 // 2,048 (gate) 104 -> 79; 2,048 x 6,144 x 4,096 99 -> 78; 2,048 x 4,096 x 14,336 212 -> 167; 500 x
 // 22,016 x 4,096 (gate) 101 -> 79; 500 x 4,096 x 11,008 52 (8 slices) -> 43 (4); 1,500 x 5,632 x 2,048
 // 49 -> 39; 72 x 2,048 x 2,048 11.2 -> 8.4.  Matrix instructions of 32 x 32 in place of 16 x 16 take 2,630
@@ -433,6 +433,7 @@ __global__ __launch_bounds__(512, sizeof(T) == 4 ? 6 : 2) void gemm_ring_kernel(
       }
   };
   if constexpr (MODE == RING_GATE) {
+    static_assert(ACT_COUNT == 2, "a copy of the stores for every gate");
     if (act == ACT_SILU) store(std::integral_constant<int, ACT_SILU>());
     else store(std::integral_constant<int, ACT_GELU_TANH>());
   } else if constexpr (MODE == RING_UNARY) {
@@ -621,6 +622,22 @@ extern "C" int kllm_gemm_prompt_slices(int n, int m, int k, int dtype) {
     if (ns == 1 || us < least) least = us, best = ns;
   }
   return best;
+}
+
+// Whether the product of n rows with the queries', keys' and values' weights goes to kllm_gemm_rope (all of K in one slice, rotated and
+// appended in the product's end) or its slices to rope_append, which reads 4 bytes of each and writes 2 of every element.  Where the slices' estimate says
+// one, the former always: the same product without its sums' way out and back.  Else where it is an eighth faster by the estimates, which leave out
+// what the rotation costs the end of a tile (slices and append / one, us, and the estimates' share: 1,500 x 2,560 x 2,048 33.0 / 27.5, 0.82; 1,280
+// rows 29.0 / 26.5, 0.86; left alone: 1,024 rows 26.0 / 25.7, 0.94; 1,024 x 6,144 x 4,096 59.5 / 62.7, 0.92; 450 x 12,288 x 4,096 63.9 / 63.3, 0.96).
+extern "C" int kllm_gemm_rope_best(int n, int m, int k, int dtype) {
+  if (n <= 64 || m <= 0 || k <= 0 || k >= kRingLongK) return 0;
+  const int ns = kllm_gemm_prompt_slices(n, m, k, dtype);
+  if (ns == 1) return 1;
+  if (dtype == DT_F32) return 0;
+  float one = 0.f, apart = 0.f;
+  ring_tile(false, n, m / 2, k, 1, true, false, &one);
+  ring_tile(false, n, m, k, ns, false, true, &apart);
+  return one < 0.875f * (apart + fmaxf(4.5f, 0.2e-6f * (4 * ns + 2) * n * (float)m));
 }
 
 // Rows and columns of the tile that a product gets, as rows * 1000 + columns (of W's rows, gates included).

@@ -197,6 +197,8 @@ long kllm_fused_linear_lds_bytes(int n, int k, int nsplit, int dtype);
 /* A prompt's queries, keys and values with rotation and append: out->kind ROPE (H, KV, hd a multiple of 8, cos_t, sin_t, cache,
  * ...), w [m][k] as stored, out->f32 as there; all of K in one slice. */
 int kllm_gemm_rope(const void* x, const KllmLinearOut* out, const void* w, int n, int m, int k, hipStream_t stream);
+/* Whether a prompt's product (n > 64) of these sizes goes to kllm_gemm_rope rather than in slices of K to kllm_rope_append. */
+int kllm_gemm_rope_best(int n, int m, int k, int dtype);
 /* The same products of up to 64 rows of bfloat16 or 16 of float32, all of K (a multiple of 32) in a workgroup and nothing staged,
  * w the tiled copy (float32: or the weights themselves, below 2 GiB; the same bits).  RESID leaves kllm_linear_rows_parts(n, m, k) sums of squares a row (0: the sizes are not taken).  Tiled rows
  * (y_tiled, x_tiled; columns a multiple of 32): [row / 16][column / 32][column % 32 / 8][row % 16][8]; with more than 16 rows

@@ -145,6 +145,7 @@ def _declare(lib):
         "kllm_attn_step": [P, P, P, L, P, P, P, P, I, I, I, I, I, I, I, I, P, I, F, P, I, I, P, I, P, I, P, P, L, I, P, L, I, P, I, L, L, I, I, P],
         "kllm_attn_prefill_slices": [I, I, I],
         "kllm_gemm_rope": [P, P, P, I, I, I, P],
+        "kllm_gemm_rope_best": [I, I, I, I],
         "kllm_gemm_act": [P, P, P, I, I, I, I, I, P, P],
         "kllm_add_sinusoid": [P, P, I, I, D, P],
         "kllm_unary_act": [P, I, L, I, P, I, I, I, I, P, P],
@@ -1470,6 +1471,12 @@ def gemm_rope(x, w, q, rope):
     _describe_rope(lo, rope, n, x.dtype)
     lo.y = _ptr(q, "gemm_rope q")
     _launch("kllm_gemm_rope", "gemm_rope", _ptr(x, "gemm_rope x"), lo, _ptr(w, "gemm_rope w"), n, m, k, _stream())
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_rope_best(n, m, k, dtype) -> bool:
+    """Whether a prompt's product of these sizes is to go to ``gemm_rope`` rather than in slices of K to ``rope_append``."""
+    return bool(library().kllm_gemm_rope_best(int(n), int(m), int(k), dtype_code(dtype)))
 
 
 def gemm_rope_fits(m, k, head_dim, dtype):

@@ -30,7 +30,7 @@ import torch
 
 from .. import kernels as K
 from .base import Normed, Part, register_part
-from .linear import decode_linear, fused_f32, linear, linear_into, one_slice, rows_kernel, sink_takes_rows, tiled_copy
+from .linear import decode_linear, fused_f32, linear, linear_into, prompt_rope, rows_kernel, sink_takes_rows, tiled_copy
 from .spec import CacheNeed, WeightSpec
 
 
@@ -254,7 +254,7 @@ class CausalSelfAttention(Part):
                            tiles_per_wg=self._fused_tiles(n),
                            rope=K.Rope(cos, sin, pages, ctx.positions, ctx.span_of_token, cache.block_table,
                                        cache.page_size, self.heads, self.kv_heads, self.head_dim))
-        elif (plain_rotation and type(xn) is torch.Tensor and xn.is_contiguous() and one_slice(self.runtime, n, self.w_in)
+        elif (plain_rotation and type(xn) is torch.Tensor and xn.is_contiguous() and prompt_rope(self.runtime, n, self.w_in)
               and K.gemm_rope_fits(*self.w_in.shape, self.head_dim, dtype)):
             # a prompt whose product is one slice: the same on its tiles (slices go to rope_append, which adds them)
             K.gemm_rope(xn, self.w_in, q, K.Rope(cos, sin, pages, ctx.positions, ctx.span_of_token, cache.block_table,
@@ -294,7 +294,8 @@ class CausalSelfAttention(Part):
         """Choose the attention kernels by the spans' lengths: tokens of short
         spans (decode tokens) go to the kernel that splits a token's keys over
         many waves, longer spans to the prompt kernel in blocks of 128 queries
-        (both on the matrix cores, in bfloat16 or with 32-bit operands); sizes
+        (both on the matrix cores, in bfloat16 or with 32-bit operands; a step that
+        has both in one launch where that is faster, ``K.attn_step``); sizes
         those kernels do not take go to the kernel that takes every size.  ``gate``
         (``K.Columns`` of sums): its logistic function multiplies the output."""
         fast, prompt_ok = self._fast(q.dtype, cache.page_size)

@@ -298,9 +298,11 @@ def linear_into(ctx, x, w, sink, tag, w_tiled=None):
     return Normed(sink.x, ss, parts, norm, xw=xw)
 
 
-def one_slice(rt, n, w):
-    """Whether a prompt's product (more than 64 rows) runs on the MFMA tiles with all of K in one slice."""
-    return n > 64 and choose(w.dtype, n, *w.shape, rt.options) in ((K.GEMM_MFMA_BF16, 1), (K.GEMM_MFMA_F32, 1))
+def prompt_rope(rt, n, w):
+    """Whether a prompt's input projections (more than 64 rows) run on the MFMA tiles with all of K in one slice, where the rotation and
+    the append are the end of a tile (``K.gemm_rope``)."""
+    return (n > 64 and choose(w.dtype, n, *w.shape, rt.options)[0] in (K.GEMM_MFMA_BF16, K.GEMM_MFMA_F32)
+            and (rt.options.get("gemm_algo") is not None or K.gemm_rope_best(n, *w.shape, w.dtype)))
 
 
 def linear(ctx, x, w, tag, out_dtype=torch.float32, split=True, w_tiled=None):

@@ -199,3 +199,14 @@ def test_rows_that_the_busiest_cu_reads(kind, n, m, tiles):
 def test_half_tiles_of_weights_want_rows_in_the_lanes_order(n, m, k, dtype, want):
     assert K.linear_rows_best(K.LINEAR_RESID, n, m, k, dtype, False) is want
     assert K.linear_rows_best(K.LINEAR_RESID, n, m, k, dtype, True)
+
+
+@pytest.mark.parametrize("n,m,k,dtype,whole", [
+    (64, 2560, 2048, BF16, False), (1024, 2560, 2048, BF16, False), (1280, 2560, 2048, BF16, True), (1800, 2560, 2048, BF16, True),
+    (2048, 2560, 2048, BF16, True), (1024, 6144, 4096, BF16, False), (1280, 6144, 4096, BF16, True), (450, 12288, 4096, BF16, False),
+    (700, 12288, 4096, BF16, True), (1800, 2560, 2048, F32, False), (1400, 2560, 2048, F32, True), (300, 2560, 1 << 23, BF16, False)])
+def test_prompt_projections_in_one_slice(n, m, k, dtype, whole):
+    """Rotation and append in the product's end wherever one slice is the fastest product, and in bfloat16 where the slices' way out and back costs
+    more than they give."""
+    assert K.gemm_rope_best(n, m, k, dtype) is whole
+    assert products.prompt_rope(_Recorder(dtype), n, torch.empty(m, k, dtype=dtype, device="meta")) is whole
