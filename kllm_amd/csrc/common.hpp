@@ -34,28 +34,17 @@ template <> __device__ __forceinline__ bf16_t from_f32<bf16_t>(float v) { return
 // in gate_act; every kernel with a gate in its epilogue calls this one function.
 enum : int { ACT_SILU = 0, ACT_GELU_TANH = 1, ACT_COUNT = 2 };
 
-// A sigmoid for results that are rounded to bfloat16, that is by up to 2^-8 of themselves: the hardware's exponential and reciprocal, within 2^-24 |z| +
-// 2^-22 of its value (0 where that is below 1e-38, from z = -87 down).  Four instructions where expf and a division are about thirty: in the end of
-// the prompt products' tiles a lane has 48 or 64 gated elements and nothing to do beside them, and the code alone was as long as the instruction
-// cache (us: 2,048 x 11,264 x 2,048 85.2 -> 80.0, 1,999 x 28,672 x 4,096 370 -> 357, 700 x 11,264 x 2,048 41.4 -> 39.1).
-__device__ __forceinline__ float sigmoid_bf16(float z) {
-  return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(z * -1.4426950408889634f));
-}
-
-// T: what the result is rounded to.
+// T: what the result is rounded to.  GELU in bfloat16 has 1 + tanh(u) as 2 sigmoid(2 u): for negative g the sum's own rounding, 2^-25, is more of the
+// result than the rounding to bfloat16 from g = -3 down.  (The hardware's exponential of one rounded product and its reciprocal in
+// place of expf and the division: the gated products of prompts 2 to 4 % faster, the sigmoid off by up to 65 units of 2^-24 where this is within 3.)
 template <typename T>
 __device__ __forceinline__ float gate_act(float g, int act) {
-  if constexpr (sizeof(T) == 2) {
-    // 1 + tanh(u) = 2 sigmoid(2 u); the square's bound keeps a zero's product with it a number, and the cube where it turns the sigmoid to 0 or 1
-    if (act == ACT_GELU_TANH) return g * sigmoid_bf16(g * fmaf(0.0713548162726009f, fminf(g * g, 1e30f), 1.5957691216057308f));
-    return g * sigmoid_bf16(g);
-  } else {
-    if (act == ACT_GELU_TANH) {   // 0.5 g (1 + tanh(sqrt(2/pi) (g + 0.044715 g^3)))
-      const float u = 0.7978845608028654f * (g + 0.044715f * g * g * g);
-      return 0.5f * g * (1.f + tanhf(u));
-    }
-    return g / (1.f + expf(-g));  // SiLU (reference: backend/model.cu:477-483)
+  if (act == ACT_GELU_TANH) {   // 0.5 g (1 + tanh(sqrt(2/pi) (g + 0.044715 g^3)))
+    if constexpr (sizeof(T) == 2) return g / (1.f + expf(-g * fmaf(0.0713548162726009f, g * g, 1.5957691216057308f)));
+    const float u = 0.7978845608028654f * (g + 0.044715f * g * g * g);
+    return 0.5f * g * (1.f + tanhf(u));
   }
+  return g / (1.f + expf(-g));  // SiLU (reference: backend/model.cu:477-483)
 }
 
 // Activations without a gate (kllm_unary_act): the gates' two, and xIELU, whose two constants
@@ -72,7 +61,7 @@ __device__ __forceinline__ float unary_act(float z, int act, float a_pos, float 
     return z > 0.f ? fmaf(a_pos * z, z, 0.5f * z) : fmaf(0.5f + a_neg, expm1f(z) - z, 0.5f * z);
   if (act == ACT_TANH) return tanhf(z);
   if (act == ACT_IDENTITY) return z;
-  if (act == ACT_SIGMOID) return sizeof(T) == 2 ? sigmoid_bf16(z) : 1.f / (1.f + expf(-z));
+  if (act == ACT_SIGMOID) return 1.f / (1.f + expf(-z));
   if (act == ACT_RELU_SQ) {
     const float p = fmaxf(z, 0.f);
     return p * p;

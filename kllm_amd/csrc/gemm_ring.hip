@@ -23,7 +23,7 @@
 // Measured with the chip's counters: 2,271 cycles a stage of 256 x 256 where the matrix instructions
 // alone take 2,048 (90 %), whatever the caches hold.  With random operands on all CUs the chip then
 // lowers its clock (2.4 -> 1.7 GHz): power bounds the large products now, not operands.
-// Against the two-stage tiles before, in us: 2,048 x 28,672 x 4,096 (gate) 498 -> 369 (357 since a gate takes less); 2,048 x 11,264 x
+// Against the two-stage tiles before, in us: 2,048 x 28,672 x 4,096 (gate) 498 -> 369; 2,048 x 11,264 x
 // 2,048 (gate) 104 -> 79; 2,048 x 6,144 x 4,096 99 -> 78; 2,048 x 4,096 x 14,336 212 -> 167; 500 x
 // 22,016 x 4,096 (gate) 101 -> 79; 500 x 4,096 x 11,008 52 (8 slices) -> 43 (4); 1,500 x 5,632 x 2,048
 // 49 -> 39; 72 x 2,048 x 2,048 11.2 -> 8.4.  Matrix instructions of 32 x 32 in place of 16 x 16 take 2,630
@@ -381,9 +381,10 @@ __global__ __launch_bounds__(512, sizeof(T) == 4 ? 6 : 2) void gemm_ring_kernel(
     return;
   }
   const bool vec = m % 4 == 0 && (reinterpret_cast<uintptr_t>(Y) & (4 * sizeof(TOUT) - 1)) == 0;
-  // KNOWN: the activation, where it has a copy of the stores of its own (-1: any).  In one copy for all, every gate of an element was worked out and one
-  // kept, and an activation went through the loop below (us, with that and now: gate of 2,048 x 11,264 x 2,048 81.1 / 80.0, of 1,999 x 28,672 x 4,096
-  // 367 / 357; 1,500 x 5,632 x 2,048 with the squared rectifier 45.8 / 37.9, with GELU 49.6 / 37.7; 1,500 x 5,632 x 1,024 33.6 / 25.3 and 37.2 / 25.3).
+  // KNOWN: the activation, where it has a copy of the stores of its own (-1: any).  Without a gate an activation went through the loop below (us, with that
+  // and now: 1,500 x 5,632 x 2,048 with the squared rectifier 46.0 / 41.2, with SiLU 55.3 / 47.1, with GELU 57.8 / 46.1; 1,500 x 5,632 x 1,024 32.1 / 25.6,
+  // 40.7 / 31.1 and 43.6 / 31.7).  For the gates one copy is as fast within 1 % (300 x 11,264 x 2,048 27.5 / 27.1, 700 37.7 / 37.5, 1,999 x 28,672 x
+  // 4,096 374.8 / 375.1).
   auto store = [&](auto known) __attribute__((always_inline)) {
     constexpr int KNOWN = decltype(known)::value;
 #pragma unroll

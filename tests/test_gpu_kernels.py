@@ -1934,6 +1934,49 @@ def test_gates_of_bfloat16_results(act):
         assert torch.equal(gated[0][inside], out[0][inside])
 
 
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh", "sigmoid"])
+@pytest.mark.parametrize("path", ["sums", "tiles"])
+def test_gates_round_32_bit_numbers_to_bfloat16(act, path):
+    """What is rounded to bfloat16 is right to 32 bits, in the kernels that take sums and in the ends of the prompt products' tiles (with and without a
+    second half): the result lies between the roundings of 64 bits' result moved by e either way.  e, in units of 2^-24: 2 for the
+    exponential, 1 for the sum and 1 for the quotient, 1 for this test's own conversion by way of 32 bits; and what GELU's exponent 2 u is
+    off by, 5 roundings of it."""
+    k_ = K()
+    z = torch.cat([torch.linspace(-85, -20, 12000), torch.linspace(-20, 20, 12000), torch.linspace(20, 85, 1000)]).to(DEV)
+    hi = z.bfloat16().float()
+    z = hi + (z - hi).bfloat16().float()                       # two bfloat16 numbers' sum, which products add exactly
+    n, code = z.numel(), k_.UNARY_ACTIVATIONS[act]
+    results = []
+    if path == "sums":
+        out = torch.empty(1, n, dtype=torch.bfloat16, device=DEV)
+        k_.unary_act(z[None], out, code)
+        results.append(out[0])
+        if act != "sigmoid":
+            gated = torch.empty_like(out)
+            k_.silu_mul(torch.cat([z, torch.ones_like(z)])[None, None], gated, k_.ACTIVATIONS[act])
+            results.append(gated[0])
+    else:
+        x, w = torch.zeros(n, 64, dtype=torch.bfloat16, device=DEV), torch.zeros(128, 64, dtype=torch.bfloat16, device=DEV)
+        x[:, 0], x[:, 1], x[:, 2] = hi, z - hi, 1.0
+        w[:64, :2], w[64:, 2] = 1.0, 1.0
+        h = torch.empty(n, 64, dtype=torch.bfloat16, device=DEV)
+        k_.gemm_act(x, w[:64].contiguous(), h, code)
+        assert torch.equal(h, h[:, :1].expand_as(h))
+        results.append(h[:, 0].clone())
+        if act != "sigmoid":
+            k_.gemm_swiglu(x, w, h, k_.ACTIVATIONS[act])
+            assert torch.equal(h, h[:, :1].expand_as(h))
+            results.append(h[:, 0])
+    d = z.double()
+    e = d if act != "gelu_tanh" else 2 * math.sqrt(2 / math.pi) * (d + 0.044715 * d ** 3)
+    want = torch.sigmoid(e) * (1.0 if act == "sigmoid" else d)
+    off = want.abs() * (5 + (5 * e.abs() if act == "gelu_tanh" else 0)) * 2.0 ** -24
+    inside = want.abs() > 1e-36
+    for got in results:
+        wrong = (got.double() < (want - off).bfloat16().double()) | (got.double() > (want + off).bfloat16().double())
+        assert not (wrong & inside).any(), (int((wrong & inside).sum()), z[wrong & inside][:5])
+
+
 @pytest.mark.parametrize("vocab", [1, 4, 63, 4096, 32000, 32003, 131072, 128256])
 def test_sample_greedy_places(vocab):
     """The first of several equal maxima wherever they lie (one thread's pieces, a wave's, the workgroup's; whole pieces of four and not), the last
