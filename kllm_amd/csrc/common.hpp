@@ -266,9 +266,9 @@ constexpr float kLog2E = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
 
 // e^x for x <= 0 (also -inf), to two units in the last place: the hardware's 2^p for p = x log2(e) as rounded, times 2^(what the rounding
 // left), which is small enough for two terms.  Half the instructions of expf, which has positive x and results below 2^-126 to look after
-// (here 0, beside a sum of at least 1).
+// (here 0, beside a sum of at least 1).  NaN stays NaN: a bad key shows in what reads it.
 __device__ __forceinline__ float exp_negative(float x) {
-  x = fmaxf(x, -1e4f);
+  x = __builtin_elementwise_maximum(x, -1e4f);               // (fmaxf would take the number)
   const float p = x * kLog2E;
   const float rest = fmaf(x, 1.925963033e-8f, fmaf(x, kLog2E, -p));          // log2(e) is kLog2E (as rounded to 32 bits) + 1.926e-8
   const float y = __builtin_amdgcn_exp2f(p);

@@ -1776,6 +1776,22 @@ def test_attention_prompt_weights_float32(hd):
     assert err < 24 * 2.0 ** -24, float(err) * 2 ** 24
 
 
+@pytest.mark.parametrize("H,KV,hd", [(4, 2, 32), (16, 4, 64), (3, 3, 96), (8, 1, 128), (4, 4, 40)])
+@pytest.mark.parametrize("where", [0, 37, 130])
+def test_a_bad_key_shows_in_float32_attention(H, KV, hd, where):
+    """A cached key of NaN whose value is a number: every query that reads it, and no other, is NaN, in both float32 kernels, on 16 and on 32 columns."""
+    c = attention_case(H, KV, hd, 16, torch.float32, 0, [(0, 150), (0, 150)], seed=3)
+    c["cache"][int(c["tables"][0][where // 16]), 0, KV - 1].view(16, hd)[where % 16, hd // 2] = float("nan")
+    bad = torch.zeros(300, H, dtype=torch.bool)
+    bad[where:150, (KV - 1) * (H // KV):] = True
+    out, rows = run_prefill(c)
+    assert rows.all()
+    for got in (out, *(run_attention("decode", c["q"], c["cache"], c["pos"], c["sot"], c["bt"], 16, H, KV, hd, 0, c["scale"], nslices=n) for n in (1, 4, 6))):
+        got = got.cpu().view(300, H, hd)
+        assert torch.isnan(got[bad]).all()
+        assert (got.double() - c["want"].view(300, H, hd))[~bad].abs().max() < attn_tol(torch.float32)
+
+
 @pytest.mark.parametrize("H,KV,hd,ps", [(4, 2, 32, 16), (16, 4, 64, 48), (3, 3, 96, 32), (8, 1, 128, 16)])
 @pytest.mark.parametrize("window", [0, 70])
 def test_attention_prompt_edges_float32(H, KV, hd, ps, window):
