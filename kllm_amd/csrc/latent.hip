@@ -768,7 +768,9 @@ __global__ __launch_bounds__(64 * kLatWaves) void attn_latent_block_kernel(
 // two LDS buffers (global loads that write LDS: 16 bytes a lane, a wave's 64 pieces in a row), the
 // next tile's while this one is multiplied, a load behind every two products of the scores: with a wave to a SIMD whatever is not a product stands in
 // line with them, and the loads all at once in front of the first reads from LDS kept those waiting.  Reads of 8 bytes and loads in
-// front -> now, us: 1,500 tokens of 32 heads, rank 512 156 -> 136, 700 82 -> 73, 4,000 of 16 heads 383 -> 333, 1,500 of 16 heads, rank 256 93 -> 85.  A wave cannot pad what it writes this way, so the 16-byte
+// front -> now, us: 1,500 tokens of 32 heads, rank 512 156 -> 136, 700 82 -> 73, 4,000 of 16 heads 383 -> 333, 1,500 of 16 heads, rank 256 93 -> 85; slower where
+// a request has one tile, behind which a second is asked for that nobody reads: 50 prompts of 30 tokens of 32 heads, rank 512 63.5 -> 64.1, of 16 38.8 -> 40.2,
+// rank 256 23.1 -> 24.2 (loads around which the tile's last turn jumps: 12 % slower elsewhere).  A wave cannot pad what it writes this way, so the 16-byte
 // pieces of a row change places: piece p of key row k lies at p ^ (k & row_mask), piece p of
 // element e's 32 keys at p ^ (e/4 % 4), which spreads a read over the banks.
 //
@@ -840,6 +842,7 @@ __global__ __launch_bounds__(64 * kLatWaves) __attribute__((amdgpu_waves_per_eu(
     k_off[j] = (unsigned)(((kr % 16) * row + 8 * (kp ^ (kr & row_mask))) * (int)sizeof(bf16_t));
   }
   const int v_piece = (lane % 4) ^ (lane / 16 % 4), v_half = v_piece / 2;
+  const int v_off = 8 * (v_piece % 2) + (16 * wave + lane / 4) * page_size;
   const unsigned lds0 = lds_address(lat_tiles);
   // ... and where it reads them: four places each, the rest are constant distances
   const int krow = (c & 19) | ((c & 4) << 1) | ((c & 8) >> 1);
@@ -891,7 +894,7 @@ __global__ __launch_bounds__(64 * kLatWaves) __attribute__((amdgpu_waves_per_eu(
       const bf16_t* v0 = base[0] + (long)page_size * row + slot[0];
       const bf16_t* v1 = base[1] + (long)page_size * row + slot[1];
       return {{base[0] + (long)slot[0] * row, base[1] + (long)slot[1] * row},
-              (v_half ? v1 : v0) + 8 * (v_piece % 2) + (long)(16 * wave + lane / 4) * page_size,
+              (v_half ? v1 : v0) + v_off,
               lds0 + (unsigned)(buf * buf_elems) * (unsigned)sizeof(bf16_t)};
     };
     constexpr int LOADS = KL + NB / 2;                        // of a wave for a tile: rows, then latents
@@ -1006,15 +1009,25 @@ __global__ __launch_bounds__(64 * kLatWaves) __attribute__((amdgpu_waves_per_eu(
   if (!col_ok) return;
   const float inv = over ? NAN : 1.f / l;
   bf16_t* orow = out + col * rank;
+  float none = 0.f;                                           // 0, or NaN where an element is not finite
 #pragma unroll
   for (int r = 0; r < NB; ++r)
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
       bf16x4 v;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = (bf16_t)(acc[r][4 * b + i] * inv);
+      for (int i = 0; i < 4; ++i) {
+        const float o = acc[r][4 * b + i] * inv;
+        v[i] = (bf16_t)o;
+        none = fmaf(o, 0.f, none);
+      }
       *reinterpret_cast<bf16x4*>(orow + 32 * r + 8 * b + 4 * g) = v;
     }
+  // Where the columns are several requests', all of them were multiplied by the latents of all, by probabilities of 0, which a NaN or an infinity comes
+  // through: such a column goes to the launch behind, which keeps requests apart.  (Known only here, from the spans' list: a flag along the loop, or a
+  // branch for waves without a column in a tile, sends registers of ranks of 512 through scratch memory, 1,500 tokens of 32 heads 137 -> 152 and 816 us.)
+  none += __shfl_xor(none, 32, kWave);
+  if (isnan(none) && span_of_token[t_first] != span_of_token[t_last] && g == 0) *orow = (bf16_t)NAN;
 }
 
 template <int NB, int KS>

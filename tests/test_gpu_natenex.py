@@ -409,6 +409,47 @@ def test_attention_through_latents_round_by_round(H, row, rank, page, window):
             assert rel(got[s], want[s]) < 2 ** -7, (slices, s, rel(got[s], want[s]))
 
 
+@pytest.mark.parametrize("H,row,rank", [(32, 576, 512), (32, 288, 256), (64, 96, 64), (16, 320, 256), (20, 576, 512), (3, 160, 128)])
+@pytest.mark.parametrize("window", [0, 60])
+@pytest.mark.parametrize("loud", [False, True])
+def test_a_request_does_not_read_its_neighbours_latents(H, row, rank, window, loud):
+    """Long steps: workgroups hold columns of several requests.  One request's latents hold what is not finite: NaN and an infinity, so that its own
+    results are NaN (loud), or one infinity with a score of -infinity, which is in its results' sixth element and no other.  The other requests'
+    results are what they are without it, in workgroups with columns of both (and tokens that the launch that keeps requests apart takes with them, four
+    at a time) by that launch: probabilities and output rounded to 2^-9 in either.  In others the same bits."""
+    from kllm_amd import kernels as K
+    page, before, lens = 16, [0, 3, 20, 40, 0, 60], [5, 50, 3, 69, 34, 7]
+    g = torch.Generator().manual_seed(row + H)
+    n, S, per = sum(lens), len(lens), 8
+    rows = torch.randn(S, per * page, row, generator=g).bfloat16()
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    span = torch.tensor([s for s, L in enumerate(lens) for _ in range(L)])
+    pos = i32([b + i for b, L in zip(before, lens) for i in range(L)])
+    q = torch.randn(n, H, row, generator=g).bfloat16()
+    q[span == 3, :, 5] = -1.0
+    table = i32(list(range(S * per))).view(S, per)
+    got = []
+    for bad in (False, True):
+        v = rows.clone()
+        if bad and loud:
+            v[3, 41, 5], v[3, 60, rank - 1], v[3, 105, 17] = float("nan"), float("inf"), float("nan")
+        elif bad:
+            v[3, 33, 5] = float("inf")
+        pages = v.view(S * per, page, row)
+        cache = torch.cat([pages.flatten(1), pages[:, :, :rank].transpose(1, 2).flatten(1)], 1).contiguous().cuda()
+        out = torch.zeros(n, H * rank, dtype=torch.bfloat16, device="cuda")
+        K.attn_latent(q.view(n, -1).cuda(), out, cache, pos, i32(span.tolist()), table, page, H, row, rank, row ** -0.5, nslices=0, window=window)
+        got.append(out.float().view(n, H, rank).cpu())
+    clean, dirty, other = *got, span != 3
+    assert torch.isfinite(clean).all() and torch.isfinite(dirty[other]).all()
+    assert (dirty[other] - clean[other]).norm() < 2 ** -7 * clean[other].norm()
+    workgroups = [set(range(t * H // 128, (t * H + H - 1) // 128 + 1)) for t in range(n)]
+    bad = set().union(*(workgroups[t] for t in range(n) if span[t] == 3))
+    fours = {t // 4 for t in range(n) if workgroups[t] & bad}
+    apart = [t for t in range(n) if t // 4 not in fours]
+    assert torch.equal(dirty[apart], clean[apart]) and not torch.isfinite(dirty[span == 3]).all()
+
+
 def test_the_merge_of_latent_slices_reads_its_own():
     """Three tokens' partial results in 3, 17 and 33 slices, the second's keys NaN and room behind the last: the others are what they are alone."""
     from kllm_amd import kernels as K
