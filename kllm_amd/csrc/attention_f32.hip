@@ -9,7 +9,8 @@
 // subtracted, online over tiles of 32 keys so that no score matrix exists.
 //
 // One wave is one work item with 32 columns:
-//   prompt   (heads that are no multiple of 32 or above 128, pages that are no multiple of 16: the others run on attention_f32_prompt.hpp)
+//   prompt   (heads that are no multiple of 32 or above 128, pages that are no multiple of 16 or very large: the others run on
+//            attention_f32_prompt.hpp)
 //            32 consecutive tokens of one request and one head: column c is
 //            token t0 + c, each with its own causal bound
 //   decode   one token, one KV head and up to 32 query heads of its group:
@@ -789,7 +790,7 @@ int attn_f32_prefill(const float* q, float* out, const float* cache, const int* 
   a.block_table = block_table; a.count = n_tiles;
   a.max_pages = max_pages; a.page_size = page_size; a.H = H; a.KV = KV; a.hd = hd; a.window = window; a.chunk = chunk; a.sinks = sinks; a.gate = gate;
   a.scale = scale; a.slopes = slopes; a.nslices = 1; a.col_blocks = 1;
-  if (page_size % 16 == 0 && hd % 32 == 0 && hd <= 128) {
+  if (page_size % 16 == 0 && hd % 32 == 0 && hd <= 128 && direct_pages(cache, KV, hd, page_size, sizeof(float))) {
     const int rc = hd == 32 ? launch_f32_prompt<1>(a, stream) : hd == 64 ? launch_f32_prompt<2>(a, stream)
                  : hd == 96 ? launch_f32_prompt<3>(a, stream) : launch_f32_prompt<4>(a, stream);
     if (rc) return rc;

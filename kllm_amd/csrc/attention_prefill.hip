@@ -1,6 +1,7 @@
 // Prompt attention over the paged cache on the matrix cores (bfloat16), three
 // kernels with the same arithmetic; which one runs is decided per launch (see
-// launch_prefill at the end of this file).  attention_prompt.hpp has the one for heads of 32, 64 and 128 without a distance bias.
+// launch_prefill at the end of this file).  attention_prompt.hpp has the one for heads of 32, 64 and 128 without a distance bias
+// and pages below 2 GiB.
 //
 // Both read a request's keys from the first key any of a workgroup's queries
 // may read to the last -- earlier pages of the cache and the rows this step
@@ -817,7 +818,7 @@ static void launch_prefill_par(int grid, hipStream_t stream, const void* q, void
   }
   const unsigned page_magic = (unsigned)(((1UL << 35) + page_size - 1) / page_size);   // ceil(2^35 / page_size)
   if constexpr (prompt_kernel_takes(HDT))
-    if (!slopes) {
+    if (!slopes && direct_pages(cache, KV, 32 * HDT, page_size, sizeof(bf16_t))) {
       launch_prompt<HDT, PAR>(dim3(grid, nslices), stream, q, out, cache, query_tiles, n_tiles, span_start, span_pos, block_table, max_pages,
                               page_size, page_magic, H, KV, window, chunk, sinks, keep_first, scale, gate, part);
       return launch_prefill_merge<HDT>(stream, out, part, query_tiles, n_tiles, span_start, H, nslices, gate);
@@ -882,7 +883,7 @@ static void launch_prefill(int grid, hipStream_t stream, const void* q, void* ou
     return;
   }
   if constexpr (prompt_kernel_takes(HDT))
-    if (!slopes) {
+    if (!slopes && direct_pages(cache, KV, 32 * HDT, page_size, sizeof(bf16_t))) {
       const bool split = HDT <= 2 && keep_first == 0 && (HDT == 1 || keys_longest == 0 ? 4 * grid <= 3 * cus
                                                                                         : 4 * grid <= cus && keys_longest > 64 && keys_longest <= 384);
       if (!split) {
@@ -913,6 +914,10 @@ static void launch_prefill(int grid, hipStream_t stream, const void* q, void* ou
 }  // namespace kllm
 
 using namespace kllm;
+
+extern "C" int kllm_attn_direct_pages(int KV, int hd, int page_size, int dtype) {
+  return direct_pages(nullptr, KV, hd, page_size, dtype == DT_F32 ? sizeof(float) : sizeof(bf16_t)) ? 1 : 0;
+}
 
 // Slices of the keys over workgroups (with a merge behind them) for a step of n_tiles blocks:
 // for heads of 128 and more, whose blocks have no kernel that shares out the keys more finely,

@@ -105,7 +105,8 @@ extern "C" int kllm_attn_step(const void* q, void* out, float* part, long part_f
                               long gate_row, int gate_width, int out_side, hipStream_t stream) {
   const bool built = dtype == DT_BF16 && (hd == 64 || hd == 128) && !slopes && keep_first == 0 && out_side == 0 && token_list;
   const bool fits = built && q && out && part && cache && positions && span_of_token && block_table && query_tiles && span_start && span_pos &&
-                    (((uintptr_t)q | (uintptr_t)out | (uintptr_t)cache | (uintptr_t)part) & 15) == 0 && n > 0 && H > 0 && KV > 0 && H % KV == 0 &&
+                    (((uintptr_t)q | (uintptr_t)out | (uintptr_t)cache | (uintptr_t)part) & 15) == 0 && direct_pages(cache, KV, hd, page_size, sizeof(bf16_t)) &&
+                    n > 0 && H > 0 && KV > 0 && H % KV == 0 &&
                     page_size > 0 && page_size % 16 == 0 && page_size <= kPrefillMaxPage && max_pages > 0 && (long)max_pages * page_size <= kPrefillMaxKeys &&
                     window >= 0 && chunk >= 0 && nslices >= 1 && nslices <= 256 && part_floats >= (long)n * H * nslices * (hd + 2) && n_listed > 0 &&
                     n_listed <= n && n_tiles > 0 && keys_total > 0 && keys_longest > 0 &&

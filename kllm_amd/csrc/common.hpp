@@ -234,6 +234,12 @@ void set_error(const char* fmt, ...);
 
 // Compute units of the current device (cached); 256 if it cannot be asked.
 int device_cus();
+
+// Whether the prompt kernels that move tiles from the pages straight into LDS take a cache: they hold a page's size and the places in it in 31 bits, and a
+// load of 16 bytes without registers wants its address in steps of 16.  The others have 64 bits and take any place.
+inline bool direct_pages(const void* cache, int KV, int hd, int page_size, int elem) {
+  return ((uintptr_t)cache & 15) == 0 && 2L * KV * hd * page_size * elem < (1L << 31);
+}
 // XCDs of the current device (cached); 8 if it cannot be asked.
 int device_xcds();
 

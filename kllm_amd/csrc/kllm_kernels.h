@@ -304,6 +304,8 @@ int kllm_attn_prefill(const void* q, void* out, const void* cache, const int* qu
  * `part` is room for n_rows (the rows of q) x H x nslices x (hd + 2) floats, and the results
  * are merged by a second kernel of the same call. */
 int kllm_attn_prefill_slices(int n_tiles, int H, int hd);
+/* Whether pages of this size are small enough for the prompt kernels that move tiles straight into LDS (otherwise the others take them). */
+int kllm_attn_direct_pages(int KV, int hd, int page_size, int dtype);
 
 /* kllm_attn_decode for the tokens that token_list names and kllm_attn_prefill for the blocks of query_tiles, of one step: the
  * arguments of both, the same results to rounding; in one launch where the step is built for that and it is the faster way.  block_part,

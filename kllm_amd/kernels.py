@@ -144,6 +144,7 @@ def _declare(lib):
         "kllm_attn_prefill": [P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, P, I, F, P, L, I, P, L, I, I, I, P, I, L, L, I, I, P],
         "kllm_attn_step": [P, P, P, L, P, P, P, P, I, I, I, I, I, I, I, I, P, I, F, P, I, I, P, I, P, I, P, P, L, I, P, L, I, P, I, L, L, I, I, P],
         "kllm_attn_prefill_slices": [I, I, I],
+        "kllm_attn_direct_pages": [I, I, I, I],
         "kllm_gemm_rope": [P, P, P, I, I, I, P],
         "kllm_gemm_rope_best": [I, I, I, I],
         "kllm_gemm_act": [P, P, P, I, I, I, I, I, P, P],
@@ -1295,6 +1296,11 @@ def attn_prefill_slices(n_tiles, n_heads, head_dim, dtype=torch.bfloat16) -> int
     if dtype != torch.bfloat16:
         return 1
     return int(library().kllm_attn_prefill_slices(int(n_tiles), int(n_heads), int(head_dim)))
+
+
+def attn_direct_pages(n_kv_heads, head_dim, page_size, dtype) -> bool:
+    """Whether pages of this size are small enough for the prompt kernels that move tiles straight into LDS."""
+    return bool(library().kllm_attn_direct_pages(int(n_kv_heads), int(head_dim), int(page_size), dtype_code(dtype)))
 
 
 def _rows_side(out, who):

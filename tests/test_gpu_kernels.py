@@ -1776,6 +1776,24 @@ def test_attention_prompt_weights_float32(hd):
     assert err < 24 * 2.0 ** -24, float(err) * 2 ** 24
 
 
+def test_float32_prompts_in_pages_of_four_gigabytes():
+    """Places in such a page do not fit the 32 bits of the kernel for prompts: the other one takes it."""
+    H, hd, ps = 32, 128, 131072
+    g = torch.Generator().manual_seed(2)
+    ks, vs, q = (torch.randn(40, H, hd, generator=g).to(DEV) for _ in range(3))
+    cache = torch.empty(2, 2, H, ps * hd, device=DEV)
+    assert not K().attn_direct_pages(H, hd, ps, torch.float32) and cache[0].numel() * 4 == 1 << 32
+    cache[1, 0].view(H, ps, hd)[:, :40] = ks.transpose(0, 1)
+    cache[1, 1].view(H, hd, ps)[:, :, :40] = vs.permute(1, 2, 0)
+    ints = lambda *v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    out = torch.full((40, H * hd), float("nan"), device=DEV)
+    K().attn_prefill(q.view(40, -1), out, cache, ints(0, 0), 1, ints(0, 40), ints(0), ints(1).view(1, 1), ps, H, H, hd, 0, hd ** -0.5)
+    w = torch.matmul(q.double().transpose(0, 1), ks.double().permute(1, 2, 0).contiguous()) * hd ** -0.5
+    w = w.masked_fill(torch.ones(40, 40, device=DEV).triu(1).bool(), float("-inf"))
+    want = torch.matmul(torch.softmax(w, 2), vs.double().transpose(0, 1).contiguous()).transpose(0, 1).reshape(40, -1)
+    assert (out.double() - want).abs().max() < attn_tol(torch.float32)
+
+
 @pytest.mark.parametrize("H,KV,hd", [(4, 2, 32), (16, 4, 64), (3, 3, 96), (8, 1, 128), (4, 4, 40)])
 @pytest.mark.parametrize("where", [0, 37, 130])
 def test_a_bad_key_shows_in_float32_attention(H, KV, hd, where):

@@ -210,3 +210,12 @@ def test_prompt_projections_in_one_slice(n, m, k, dtype, whole):
     more than they give."""
     assert K.gemm_rope_best(n, m, k, dtype) is whole
     assert products.prompt_rope(_Recorder(dtype), n, torch.empty(m, k, dtype=dtype, device="meta")) is whole
+
+
+@pytest.mark.parametrize("kv_heads,head_dim,page_size,dtype,direct", [
+    (4, 64, 64, F32, True), (32, 128, 65520, F32, True), (32, 128, 65536, F32, False), (32, 128, 131072, F32, False), (1, 32, 8388592, F32, True),
+    (1, 32, 8388608, F32, False), (8, 128, 2048, BF16, True), (2047, 128, 2048, BF16, True), (2048, 128, 2048, BF16, False)])
+def test_pages_whose_places_fit_31_bits(kv_heads, head_dim, page_size, dtype, direct):
+    """Kernels that hold a place in a page in 31 bits get no page of 2 GiB and more."""
+    assert K.attn_direct_pages(kv_heads, head_dim, page_size, dtype) is direct
+    assert direct == (2 * kv_heads * head_dim * page_size * (4 if dtype == F32 else 2) < 2 ** 31)
