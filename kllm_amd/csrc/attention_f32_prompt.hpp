@@ -123,8 +123,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
 
   const int kat = c * (CH * 16) + ((g ^ (ksw(c) & 1)) * 16);  // piece 2 kk + g: kat ^ 32 (kk ^ half of the row's exchange)
   const int kx = (ksw(c) & ~1) * 16;
-  const bool plain = !slopes && scale > 0.f;                  // the scale goes with the subtraction of the maximum
-  const float unit = plain ? scale : 1.f;
   float m = -INFINITY, l = 0.f;
   if (sinks && wave == 0) {                                   // a key with a score of its own and no value; one of a column's lanes has its term
     m = sinks[h];
@@ -164,10 +162,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
       load_k(t + 1);
     }
     fence();
-    // ---- mask, running maximum and sum; s becomes the probabilities (of scores in units of 1 / unit)
-    if (!plain) {
+    // ---- mask, running maximum and sum; s becomes the probabilities.  (The scale by itself: in one instruction with the subtraction of the maximum,
+    // which was rounded, the largest scores would be off from it by half of its last place, which is more than exponentials bear from 2^31 on.)
+    if (slopes) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) s[i] = fmaf(s[i], scale, -my_slope * (float)(my_pos - (kb + 8 * (i / 4) + 4 * g + i % 4)));
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] *= scale;
     }
     if ((kb < highest_start) | (kb + 31 > pos_base)) {
 #pragma unroll
@@ -181,7 +183,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
     for (int i = 1; i < 16; ++i) tmax = fmaxf(tmax, s[i]);
     const unsigned w = __builtin_bit_cast(unsigned, tmax);
     const auto x = __builtin_amdgcn_permlane32_swap(w, w, false, false);
-    tmax = fmaxf(__builtin_bit_cast(float, (unsigned)x[0]), __builtin_bit_cast(float, (unsigned)x[1])) * unit;
+    tmax = fmaxf(__builtin_bit_cast(float, (unsigned)x[0]), __builtin_bit_cast(float, (unsigned)x[1]));
     if (__any(tmax > m)) {                                    // (otherwise everything is multiplied by one)
       const float m_new = fmaxf(m, tmax);
       const float alpha = exp_negative(m - (m_new == -INFINITY ? 0.f : m_new));
@@ -194,10 +196,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
     }
     const float mref = (m == -INFINITY) ? 0.f : m;            // a column with no key yet
     float psum = 0.f;
+    {
+#pragma clang fp contract(off)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      s[i] = exp_negative(fmaf(s[i], unit, -mref));
-      psum += s[i];
+      for (int i = 0; i < 16; ++i) {
+        s[i] = exp_negative(s[i] - mref);
+        psum += s[i];
+      }
     }
     l += psum;
     // ---- values

@@ -1776,6 +1776,33 @@ def test_attention_prompt_weights_float32(hd):
     assert err < 24 * 2.0 ** -24, float(err) * 2 ** 24
 
 
+@pytest.mark.parametrize("hd", [32, 64, 96, 128])
+@pytest.mark.parametrize("size", [2.0 ** 17, 2.0 ** 20])
+def test_float32_attention_of_very_large_scores(hd, size):
+    """Scores of about 2^34 and 2^40, far beyond what exponentials take, are still numbers: the key with the largest takes all (the next is further away
+    than 104, and than what the products' rounding moves them), in prompts and for decode tokens."""
+    H, KV, ps = 4, 2, 16
+    g = torch.Generator().manual_seed(hd)
+    ks, vs, q = (torch.randn(70, n, hd, generator=g) for n in (KV, KV, H))
+    ks, q = ks * size, q * size
+    tables = [list(range(5))]
+    cache = build_paged([ks.flatten(1)], [vs.flatten(1)], tables, [70], KV, hd, ps, 5, torch.float32)
+    s = torch.einsum("thd,khd->htk", q.double(), ks.double().repeat_interleave(H // KV, 1)) * hd ** -0.5
+    s = s.masked_fill(torch.ones(70, 70).triu(1).bool(), float("-inf"))
+    top = s.topk(2, dim=2)
+    clear = ((top.values[..., 0] - top.values[..., 1]) > top.values.abs().amax(2).clamp(max=1e30) * 2.0 ** -16).T       # [token, head]
+    want = torch.gather(vs.repeat_interleave(H // KV, 1).transpose(0, 1), 1, top.indices[..., :1].expand(-1, -1, hd)).transpose(0, 1)
+    assert clear.float().mean() > 0.95
+    c = dict(q=q.flatten(1).to(DEV), cache=cache, bt=torch.tensor(tables, dtype=torch.int32, device=DEV), ps=ps, H=H, KV=KV, hd=hd, window=0,
+             scale=hd ** -0.5, spans=[(0, 70)], span_start=torch.tensor([0, 70], dtype=torch.int32, device=DEV),
+             span_pos=torch.zeros(1, dtype=torch.int32, device=DEV))
+    pos, sot = torch.arange(70, dtype=torch.int32, device=DEV), torch.zeros(70, dtype=torch.int32, device=DEV)
+    for got in (run_prefill(c)[0], run_attention("decode", c["q"], cache, pos, sot, c["bt"], ps, H, KV, hd, 0, c["scale"], nslices=4)):
+        got = got.cpu().view(70, H, hd)
+        assert torch.isfinite(got).all()
+        assert (got - want)[clear].abs().max() < 1e-5
+
+
 def test_float32_prompts_in_pages_of_four_gigabytes():
     """Places in such a page do not fit the 32 bits of the kernel for prompts: the other one takes it."""
     H, hd, ps = 32, 128, 131072
