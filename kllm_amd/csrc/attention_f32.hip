@@ -9,8 +9,8 @@
 // subtracted, online over tiles of 32 keys so that no score matrix exists.
 //
 // One wave is one work item with 32 columns:
-//   prompt   (heads that are no multiple of 32 or above 128, pages that are no multiple of 16 or very large: the others run on
-//            attention_f32_prompt.hpp)
+//   prompt   (heads that are no multiple of 32 or above 128, pages that are no multiple of 16 or very large, many short chains of tiles: see
+//            f32_prompt_shared; the others run on attention_f32_prompt.hpp)
 //            32 consecutive tokens of one request and one head: column c is
 //            token t0 + c, each with its own causal bound
 //   decode   one token, one KV head and up to 32 query heads of its group:
@@ -777,10 +777,39 @@ static int launch_f32_prompt(const AttnF32Args& a, hipStream_t stream) {
   return 0;
 }
 
+// Which kernel takes a prompt: four waves to 32 tokens and a head (attn_f32_prompt_kernel), or one, four heads to a workgroup.  The former's chains of
+// tiles are a quarter as long, but it has two workgroups a CU (heads of 64; one of 96 and 128), each with what it costs beside its tiles, also
+// where the block of 128 ends before its 32 tokens.  So with more than two such parts a CU it needs chains: of some tiles, more with more parts and
+// larger heads (us, one wave / four: 16 prompts of 40 tokens, 32 heads of 64 14.2 / 19.6, of 96 21.1 / 32.5; 29 of 6, 40 heads of 96 19 / 57; 64 of 64
+// 22.6 / 33.6; 24 prompts of 51, 40 heads of 128 64 / 86; but 32 heads of 64, four of 500 72 / 68).  And for heads of 96 and 128 with four parts
+// a CU and more, all of them alike, of more than three rounds of tiles (behind a window of 256, 2,048 tokens of 32 heads of 96 94 / 122, of 128 129 / 151, of 64
+// heads 252 / 294; eight of 100 behind 300, 64 of 128 140 / 160; without a window 863 / 710).  Of 888 drawn sizes 69 were more than 3 %
+// slower, up to three times, with the latter everywhere, 6 by this rule, up to 1.22; in the mean it gives 1.95, everywhere 1.94.  Without numbers of keys: four waves.
+static bool f32_prompt_shared(int n_tiles, int H, int hd, int n_rows, long keys_total, int keys_longest, int window) {
+  if (keys_total <= 0 || keys_longest <= 0) return true;
+  const float cus = device_cus();
+  const long parts = n_rows > 0 && n_rows / 32 + n_tiles < 4L * n_tiles ? n_rows / 32 + n_tiles : 4L * n_tiles;      // that have tokens
+  float mean = (float)keys_total / n_tiles, most = keys_longest;
+  if (window > 0) {                     // (the blocks' numbers are of 128 tokens)
+    mean = fminf(mean, window + 48.f);
+    most = fminf(most, window + 48.f);
+  }
+  mean = fmaxf((mean - 16.f * ((float)parts / n_tiles - 1.f)) / 32.f + 0.5f, 1.f);
+  most = most / 32.f + 0.5f;
+  const float all = 4.f * n_tiles * H / cus;
+  if (all <= 2.f) return true;
+  if (0.5f * (mean + most) < (hd > 32 ? 1.5f / 64 * hd : 0.f) + 0.5f * log2f(all)) return false;       // (heads of 32: four workgroups a CU)
+  return !(hd >= 96 && parts * H >= 4 * cus && most <= 13.5f && mean >= 0.72f * most);
+}
+
+extern "C" int kllm_attn_f32_prompt_shared(int n_tiles, int H, int hd, int n_rows, long keys_total, int keys_longest, int window) {
+  return n_tiles > 0 && f32_prompt_shared(n_tiles, H, hd, n_rows, keys_total, keys_longest, window) ? 1 : 0;
+}
+
 int attn_f32_prefill(const float* q, float* out, const float* cache, const int* query_tiles, int n_tiles,
                      const int* span_start, const int* span_pos, const int* block_table, int max_pages,
                      int page_size, int H, int KV, int hd, int window, int chunk, const float* sinks, float scale, const float* slopes,
-                     const OutGate& gate, hipStream_t stream) {
+                     long keys_total, int keys_longest, int n_rows, const OutGate& gate, hipStream_t stream) {
   KLLM_REQUIRE(attn_f32_fits(hd, page_size),
                "attn_prefill float32: head_dim %d must be a multiple of 8 up to 256 and page_size %d a multiple of 4",
                hd, page_size);
@@ -790,7 +819,8 @@ int attn_f32_prefill(const float* q, float* out, const float* cache, const int* 
   a.block_table = block_table; a.count = n_tiles;
   a.max_pages = max_pages; a.page_size = page_size; a.H = H; a.KV = KV; a.hd = hd; a.window = window; a.chunk = chunk; a.sinks = sinks; a.gate = gate;
   a.scale = scale; a.slopes = slopes; a.nslices = 1; a.col_blocks = 1;
-  if (page_size % 16 == 0 && hd % 32 == 0 && hd <= 128 && direct_pages(cache, KV, hd, page_size, sizeof(float))) {
+  if (page_size % 16 == 0 && hd % 32 == 0 && hd <= 128 && direct_pages(cache, KV, hd, page_size, sizeof(float)) &&
+      f32_prompt_shared(n_tiles, H, hd, n_rows, keys_total, keys_longest, window)) {
     const int rc = hd == 32 ? launch_f32_prompt<1>(a, stream) : hd == 64 ? launch_f32_prompt<2>(a, stream)
                  : hd == 96 ? launch_f32_prompt<3>(a, stream) : launch_f32_prompt<4>(a, stream);
     if (rc) return rc;

@@ -24,11 +24,12 @@ int attn_f32_decode(const float* q, float* out, float* part, const float* cache,
                     const int* token_list, int count, const OutGate& gate, hipStream_t stream);
 
 // Prompt tokens: query_tiles lists (first token row, span) of blocks of up to 128
-// consecutive tokens of one span; one wave per (32 tokens of a block, head).
+// consecutive tokens of one span; one wave per (32 tokens of a block, head), or four.  keys_total, keys_longest: how many keys the blocks read
+// together and the longest alone (0: not known); n_rows: rows of q (0: not known).
 int attn_f32_prefill(const float* q, float* out, const float* cache, const int* query_tiles, int n_tiles,
                      const int* span_start, const int* span_pos, const int* block_table, int max_pages,
                      int page_size, int H, int KV, int hd, int window, int chunk, const float* sinks, float scale, const float* slopes,
-                     const OutGate& gate, hipStream_t stream);
+                     long keys_total, int keys_longest, int n_rows, const OutGate& gate, hipStream_t stream);
 
 // Slices proposed for a decode batch of n tokens whose longest request has at most max_keys
 // keys (0: unknown), in pages of page_size slots.

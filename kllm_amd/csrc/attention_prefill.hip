@@ -957,7 +957,7 @@ extern "C" int kllm_attn_prefill(const void* q, void* out, const void* cache, co
     KLLM_REQUIRE(keep_first == 0, "attn_prefill: the 32-bit kernels read one run of keys a query");
     KLLM_REQUIRE(max_pages > 0 && window >= 0 && chunk >= 0, "attn_prefill: bad table width, window or chunk");
     return attn_f32_prefill((const float*)q, (float*)out, (const float*)cache, query_tiles, n_tiles, span_start,
-                            span_pos, block_table, max_pages, page_size, H, KV, hd, window, chunk, sinks, scale, slopes, gate, stream);
+                            span_pos, block_table, max_pages, page_size, H, KV, hd, window, chunk, sinks, scale, slopes, keys_total, keys_longest, n_rows, gate, stream);
   }
   KLLM_REQUIRE(hd % 32 == 0 && hd >= 32 && hd <= 256 && (hd <= 128 || hd == 192 || hd == 256),
                "attn_prefill: head_dim %d is not built (32, 64, 96, 128, 192, 256)", hd);

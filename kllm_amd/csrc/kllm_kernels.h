@@ -255,6 +255,8 @@ int kllm_attn_generic(const void* q, void* out, const void* cache, const int* po
 int kllm_attn_decode_slices(int n, int KV, int H, int hd, int dtype, int max_keys, int page_size);
 /* Whether the float32 attention on the matrix cores takes this head size and page size. */
 int kllm_attn_f32_fits(int hd, int page_size);
+/* Whether float32 prompts of these sizes (kllm_attn_prefill's) go to the kernel whose four waves share out the keys of 32 tokens and a head. */
+int kllm_attn_f32_prompt_shared(int n_tiles, int H, int hd, int n_rows, long keys_total, int keys_longest, int window);
 /* `chunk`, `sinks`, `keep_first` and the gate in kllm_attn_decode and kllm_attn_prefill: as in kllm_attn_generic
  * (kept first positions: bfloat16 only).  out_side: 0, or min(rows of q, 16): the output as tiled rows (kllm_linear_rows). */
 int kllm_attn_decode(const void* q, void* out, float* part, long part_floats, const void* cache,

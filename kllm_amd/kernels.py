@@ -136,6 +136,7 @@ def _declare(lib):
         "kllm_gemv_normed_max_rows": [],
         "kllm_gemv_normed_max_parts": [],
         "kllm_attn_f32_fits": [I, I],
+        "kllm_attn_f32_prompt_shared": [I, I, I, I, L, I, I],
         "kllm_calibrate_copy": [P, P, L, P],
         "kllm_calibrate_read": [P, L, P, P],
         "kllm_calibrate_read_workgroups": [],
@@ -1258,6 +1259,12 @@ def attn_f32_fits(head_dim, page_size) -> bool:
     """Sizes the float32 attention on the matrix cores takes; the rest goes to
     the generic kernel."""
     return bool(library().kllm_attn_f32_fits(int(head_dim), int(page_size)))
+
+
+def attn_f32_prompt_shared(n_tiles, n_heads, head_dim, n_rows, keys_total, keys_longest, window=0) -> bool:
+    """Whether float32 prompts of these sizes go to the kernel whose four waves share out the keys of 32 tokens and a head."""
+    return bool(library().kllm_attn_f32_prompt_shared(int(n_tiles), int(n_heads), int(head_dim), int(n_rows), int(keys_total),
+                                                      int(keys_longest), int(window)))
 
 
 @functools.lru_cache(maxsize=4096)

@@ -219,3 +219,17 @@ def test_pages_whose_places_fit_31_bits(kv_heads, head_dim, page_size, dtype, di
     """Kernels that hold a place in a page in 31 bits get no page of 2 GiB and more."""
     assert K.attn_direct_pages(kv_heads, head_dim, page_size, dtype) is direct
     assert direct == (2 * kv_heads * head_dim * page_size * (4 if dtype == F32 else 2) < 2 ** 31)
+
+
+@pytest.mark.parametrize("heads,head_dim,spans,window,shared", [
+    (32, 64, [(0, 45)], 0, True), (32, 64, [(0, 700)], 0, True), (32, 64, [(0, 2048)], 256, True), (32, 64, [(0, 500)] * 4, 0, True),
+    (32, 64, [(0, 40)] * 16, 0, False), (64, 64, [(0, 40)] * 16, 0, False), (32, 64, [(1000, 8)] * 24, 0, True),
+    (40, 96, [(0, 6)] * 29, 1024, False), (32, 96, [(0, 40)] * 16, 0, False), (32, 96, [(0, 2048)], 256, False), (32, 96, [(0, 2048)], 0, True),
+    (32, 128, [(0, 2048)], 256, False), (64, 128, [(300, 100)] * 8, 256, False), (64, 128, [(0, 2048)], 0, True), (40, 128, [(0, 51)] * 24, 0, False),
+    (32, 128, [(0, 700)], 0, True), (8, 128, [(0, 18)] * 33, 64, False), (16, 32, [(0, 2048)], 0, True), (16, 32, [(0, 40)] * 16, 0, True)])
+def test_float32_prompts_whose_keys_four_waves_share(heads, head_dim, spans, window, shared):
+    """Many short chains of tiles go to the kernel with a wave to 32 tokens, as they did when it was the only one; unknown keys do not."""
+    n_rows = sum(n for _, n in spans)
+    keys = [min(a + min(t + 128, n), window + 128) if window else a + min(t + 128, n) for a, n in spans for t in range(0, n, 128)]
+    assert K.attn_f32_prompt_shared(len(keys), heads, head_dim, n_rows, sum(keys), max(keys), window) is shared
+    assert K.attn_f32_prompt_shared(len(keys), heads, head_dim, n_rows, 0, 0, window)
