@@ -65,30 +65,49 @@ static int launch_step(const void* q, void* out, float* part, const void* cache,
 // Workgroups to a token and KV head in the one launch, or 0 where two launches are faster.
 //
 // Apart, the tokens' kernel waits for memory while the blocks' one multiplies on what are often a quarter of the CUs; together the shorter of the two
-// hides behind the other.  And since the step waits for the blocks' chains of tiles anyway, a token's keys go to so few workgroups that theirs take
-// about as long (3 us more at most, which their results' way through memory and the merge's launch would take): mostly one, and no merge.  us,
-// two launches / one (operands in the caches): 20 tokens at 560 keys and 480 of a prompt behind 1,440, 32 KV heads of 128 59 / 43, behind none 43 / 33;
-// 4 at 300 and 300 33.5 / 25.8 behind 900; 20 at 500 and 500 with 8 KV heads 28 / 17; 4 KV heads of 64: 32 at 1,400 and 640 23 / 18, 10 at 700 and
-// 300 14 / 8.2, 2 at 100 and 40 8.5 / 6.0, 256 at 600 and 200 31.5 / 29.9.
-// Two launches: where the blocks' keys go in slices and their chain whole would take longer than their sliced launch, its merge and the tokens' one (4 at
-// 300 and 100 behind 2,000, 32 KV heads of 128 29 / 36; behind 1,200 25.6 / 26.3; 20 at 400 and 100 behind 2,000 42 / 38, behind 3,400 47 / 56; 12 at
-// 400 and 500 behind 2,000, 8 KV heads 45 / 42, behind 6,000 77 / 95); where more blocks than half the CUs are better off with one group of waves
+// hides behind the other.  A workgroup of a token takes about 2.1 us for 256 keys of a KV head of 64, 3.5 of 128 (its eight waves' loads from one CU),
+// and 5 beside them; several leave partial results and a merge, 4 us.  As many as make the launch shortest, by the longest chain of tiles, the longest
+// token's keys and the CUs' rounds of workgroups (a CU holds one): one where the chain is
+// longer anyway, up to what two launches would take where it is short.  us, two launches / one with one, two, four ... workgroups: one token at 4,400 keys and 45 of
+// a prompt, 8 KV heads of 128 14.8 / 55, 37, 22, 14, 12; 4 at 4,088 and 184, 4 KV heads of 128 21.8 / 63, 38, 24, 17.7, 16.7; 16 at 1,492 behind a window of 1,024 and
+// 75, 2 of 128 16.0 / 24.5, 23.6, 16.6, 12.0; 20 at 560 and 480 of a prompt behind 1,440, 32 KV heads of 128 77 / 58, 8 of 128 51 / 36; 32 at 1,400 and 640, 4 KV heads of
+// 64 34.7 / 29.9; 2 at 100 and 40, 32 of 128 13.4 / 7.4.  (When a round of 256 keys of a table's width was taken for 0.7 us, whatever the head and the
+// window: in 34 of 500 drawn steps the one launch was more than 3 % slower than two, by up to 2.5 times; now in 3, by up to 1.06.)
+// Two launches: where the blocks' keys go in slices and this launch would take longer than theirs, its merge and the tokens' one (8 at 17 and
+// one block of 2,224 keys, 12 heads of 128 27 / 36; 27 at 53 and 2,184, 16 heads 33 / 39; 20 at 400 and 100 behind 3,400, 32 KV heads 47 / 56); where
+// more blocks than half the CUs are better off with one group of waves
 // each, several to a CU, which this kernel has no room for (16 at 1,000 and four prompts of 300, 8 KV heads of 128 31.3 / 32.4; 4 at 900 and eight prompts
 // of 30 12 / 19; but four prompts of 100 15.5 / 14.6).
 static int step_workgroups(int hdt, int n_tiles, int H, int KV, int count, int max_pages, int page_size, int nslices, long keys_total, int keys_longest,
-                           int block_slices) {
-  const long cus = device_cus(), items = (long)n_tiles * H, groups = (long)count * KV * ((H / KV + 15) / 16);
-  const float chain = 6.f + keys_longest / 64.f * (hdt > 2 ? 0.9f : 0.55f);
-  if (block_slices > 1 && keys_longest >= kPrefillSliceFromKeys) {
-    const float sliced = 11.f + keys_longest / (64.f * block_slices) * 1.05f + 0.77f * n_tiles * block_slices;
-    if (chain + 3.f > sliced + fmaxf(7.f, 8.f * groups / cus)) return 0;
-  }
-  long pages = 8;                       // (a table's width, rounded as for recorded steps: both cut the keys alike)
-  while (pages < max_pages) pages *= 2;
-  const float keys = (float)(pages * page_size) / (32 * kStepWaves);
+                           int keys_token, int block_slices, int window, int chunk) {
+  const float cus = device_cus(), chain = 6.f + keys_longest / 64.f * (hdt > 2 ? 0.9f : 0.55f), merge = 4.f;
+  const long items = (long)n_tiles * H, groups = (long)count * KV * ((H / KV + 15) / 16);
+  long keys = keys_token > 0 ? keys_token : (long)max_pages * page_size;
+  if (window > 0 && keys > window + 32) keys = window + 32;
+  if (chunk > 0 && keys > chunk) keys = chunk;
+  const float round = (hdt > 2 ? 3.5f : 2.1f) * keys / (32.f * kStepWaves);   // a token's keys in one workgroup
+  const int most = (nslices + 1) / 2;   // (the workspace has room for nslices; two workgroups of four waves each are one here)
   int wgs = 1;
-  while (wgs < (nslices + 1) / 2 && 4.f + 0.7f * keys / wgs > chain + 3.f) wgs *= 2;
-  if (wgs > (nslices + 1) / 2) wgs = (nslices + 1) / 2;      // (the workspace has room for nslices; two workgroups of four waves each are one here)
+  float best = INFINITY;
+  for (int w = 1;; w *= 2) {
+    const int n = w < most ? w : most;
+    const float token = 5.f + round / n;
+    float t = fmaxf(chain, token);
+    const float rounds = (groups * n + items * chain / token) / cus;           // (the last one as if half of what it leaves idle were)
+    if (items + groups * n > cus) t = fmaxf(t, token * 0.5f * (rounds + ceilf(rounds)));
+    if (n > 1) t += merge;
+    if (t < best - 0.01f) {
+      best = t;
+      wgs = n;
+    }
+    if (w >= most) break;
+  }
+  if (block_slices > 1 && keys_longest >= kPrefillSliceFromKeys) {
+    const float sliced = 11.f + keys_longest / (64.f * block_slices) * 1.05f + 0.4f * n_tiles * block_slices;
+    const float token = 5.f + (nslices == 1 ? round : 2.f * round / nslices);            // (four waves to a workgroup, two of them to a CU)
+    const float tokens = fmaxf(token, groups * token * (nslices == 1 ? 1.f : 0.5f * nslices) / cus) + (nslices > 1 ? merge : 0.f);
+    if (best + 4.f > sliced + tokens) return 0;
+  }
   if (2 * items > cus && items + groups * wgs > cus && prompt_groups(hdt, (int)items, H, keys_total, keys_longest) != 2) return 0;
   return wgs;
 }
@@ -97,11 +116,20 @@ static int step_workgroups(int hdt, int n_tiles, int H, int KV, int count, int m
 
 using namespace kllm;
 
+extern "C" int kllm_attn_step_workgroups(int hd, int n_tiles, int H, int KV, int count, int max_pages, int page_size, int nslices, long keys_total,
+                                         int keys_longest, int keys_token, int block_slices, int window, int chunk) {
+  if ((hd != 64 && hd != 128) || n_tiles <= 0 || KV <= 0 || H % KV || count <= 0 || max_pages <= 0 || page_size <= 0 || nslices < 1 || keys_total <= 0 ||
+      keys_longest <= 0)
+    return 0;
+  return step_workgroups(hd / 32, n_tiles, H, KV, count, max_pages, page_size, nslices, keys_total, keys_longest, keys_token, block_slices, window,
+                         chunk);
+}
+
 extern "C" int kllm_attn_step(const void* q, void* out, float* part, long part_floats, const void* cache, const int* positions, const int* span_of_token,
                               const int* block_table, int max_pages, int page_size, int n, int H, int KV, int hd, int window, int chunk, const float* sinks,
                               int keep_first, float scale, const float* slopes, int nslices, int dtype, const int* token_list, int n_listed,
                               const int* query_tiles, int n_tiles, const int* span_start, const int* span_pos, long keys_total, int keys_longest,
-                              float* block_part, long block_part_floats, int block_slices, const float* gate_sums, int gate_nsplit, long gate_stride,
+                              int keys_token, float* block_part, long block_part_floats, int block_slices, const float* gate_sums, int gate_nsplit, long gate_stride,
                               long gate_row, int gate_width, int out_side, hipStream_t stream) {
   const bool built = dtype == DT_BF16 && (hd == 64 || hd == 128) && !slopes && keep_first == 0 && out_side == 0 && token_list;
   const bool fits = built && q && out && part && cache && positions && span_of_token && block_table && query_tiles && span_start && span_pos &&
@@ -112,7 +140,8 @@ extern "C" int kllm_attn_step(const void* q, void* out, float* part, long part_f
                     n_listed <= n && n_tiles > 0 && keys_total > 0 && keys_longest > 0 &&
                     (!gate_sums || (gate_nsplit >= 1 && gate_width > 0 && gate_width <= hd && gate_row >= (long)H * gate_width)) &&
                     (long)n_tiles * H + (long)n_listed * (KV + H) * nslices < (1L << 31);
-  const int wgs = fits ? step_workgroups(hd / 32, n_tiles, H, KV, n_listed, max_pages, page_size, nslices, keys_total, keys_longest, block_slices) : 0;
+  const int wgs = fits ? step_workgroups(hd / 32, n_tiles, H, KV, n_listed, max_pages, page_size, nslices, keys_total, keys_longest, keys_token,
+                                          block_slices, window, chunk) : 0;
   if (wgs) {
     const OutGate gate = {gate_sums, gate_nsplit, gate_width, gate_stride, gate_row, 0};
     return hd == 64 ? launch_step<2>(q, out, part, cache, positions, span_of_token, block_table, max_pages, page_size, H, KV, window, chunk, sinks, scale, wgs,

@@ -311,14 +311,19 @@ int kllm_attn_direct_pages(int KV, int hd, int page_size, int dtype);
 
 /* kllm_attn_decode for the tokens that token_list names and kllm_attn_prefill for the blocks of query_tiles, of one step: the
  * arguments of both, the same results to rounding; in one launch where the step is built for that and it is the faster way.  block_part,
- * block_part_floats and block_slices are kllm_attn_prefill's part, part_floats and nslices. */
+ * block_part_floats and block_slices are kllm_attn_prefill's part, part_floats and nslices; keys_token: the longest context of the
+ * listed tokens (0: not known, the table's width). */
 int kllm_attn_step(const void* q, void* out, float* part, long part_floats, const void* cache, const int* positions,
                    const int* span_of_token, const int* block_table, int max_pages, int page_size, int n, int H, int KV,
                    int hd, int window, int chunk, const float* sinks, int keep_first, float scale, const float* slopes,
                    int nslices, int dtype, const int* token_list, int n_listed, const int* query_tiles, int n_tiles,
-                   const int* span_start, const int* span_pos, long keys_total, int keys_longest, float* block_part,
+                   const int* span_start, const int* span_pos, long keys_total, int keys_longest, int keys_token, float* block_part,
                    long block_part_floats, int block_slices, const float* gate_sums, int gate_nsplit, long gate_stride,
                    long gate_row, int gate_width, int out_side, hipStream_t stream);
+
+/* Workgroups that kllm_attn_step's one launch gives a token and KV head, by its arguments of these names; 0: two launches. */
+int kllm_attn_step_workgroups(int hd, int n_tiles, int H, int KV, int n_listed, int max_pages, int page_size, int nslices, long keys_total,
+                              int keys_longest, int keys_token, int block_slices, int window, int chunk);
 
 /* x[t][c] += sin(a) for even c, cos(a) for odd c, a = positions[t] * base^(-2 (c/2) / d), angle in double. */
 int kllm_add_sinusoid(float* x, const int* positions, int n, int d, double base, hipStream_t stream);

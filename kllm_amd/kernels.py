@@ -143,7 +143,8 @@ def _declare(lib):
         "kllm_calibrate_mfma": [I, I, P, P, P],
         "kllm_attn_decode": [P, P, P, L, P, P, P, P, I, I, I, I, I, I, I, I, P, I, F, P, I, I, P, I, P, I, L, L, I, I, P],
         "kllm_attn_prefill": [P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, P, I, F, P, L, I, P, L, I, I, I, P, I, L, L, I, I, P],
-        "kllm_attn_step": [P, P, P, L, P, P, P, P, I, I, I, I, I, I, I, I, P, I, F, P, I, I, P, I, P, I, P, P, L, I, P, L, I, P, I, L, L, I, I, P],
+        "kllm_attn_step": [P, P, P, L, P, P, P, P, I, I, I, I, I, I, I, I, P, I, F, P, I, I, P, I, P, I, P, P, L, I, I, P, L, I, P, I, L, L, I, I, P],
+        "kllm_attn_step_workgroups": [I, I, I, I, I, I, I, I, L, I, I, I, I, I],
         "kllm_attn_prefill_slices": [I, I, I],
         "kllm_attn_direct_pages": [I, I, I, I],
         "kllm_gemm_rope": [P, P, P, I, I, I, P],
@@ -214,7 +215,7 @@ LAUNCHING = ("kllm_embed", "kllm_add_rmsnorm", "kllm_rope_tables", "kllm_rope_ap
              "kllm_linear_recurrence_scan", "kllm_latent_kv_append", "kllm_latent_norm", "kllm_latent_query", "kllm_attn_latent",
              "kllm_latent_out", "kllm_scaled_sum", "kllm_normed_sum", "kllm_qkv_conv_append", "kllm_decayed_prep",
              "kllm_decayed_scan", "kllm_decayed_out", "kllm_decayed_step", "kllm_token_gate", "kllm_soft_cap")
-DYNAMIC_ARGS = {"kllm_attn_prefill": (19, 20), "kllm_attn_step": (28, 29)}     # arguments that may be a StepValue
+DYNAMIC_ARGS = {"kllm_attn_prefill": (19, 20), "kllm_attn_step": (28, 29, 30)}     # arguments that may be a StepValue
 STRUCT_ARGS = {"kllm_gemv_plain": (7,), "kllm_gemv_swiglu": (8,), "kllm_gemv_rope_append": (17,),
                "kllm_fused_linear": (2,), "kllm_linear_rows": (2,), "kllm_gemm_rope": (1,)}
 
@@ -1382,9 +1383,10 @@ def attn_decode(q, out, part, cache, positions, span_of_token, block_table, page
 
 def attn_step(q, out, part, cache, positions, span_of_token, block_table, page_size, n_heads, n_kv_heads, head_dim, window, scale,
               nslices, token_list, n_listed, query_tiles, n_tiles, span_start, span_pos, keys_total, keys_longest, block_part=None,
-              block_slices=1, slopes=None, chunk=0, sink=False, keep_first=0, gate=None):
+              block_slices=1, slopes=None, chunk=0, sink=False, keep_first=0, gate=None, keys_token=0):
     """``attn_decode`` for the tokens of ``token_list`` and ``attn_prefill`` for the blocks of ``query_tiles`` in one call, and in one
-    launch where the library has one for the step (``block_part``, ``block_slices``: ``attn_prefill``'s ``part`` and ``nslices``)."""
+    launch where the library has one for the step (``block_part``, ``block_slices``: ``attn_prefill``'s ``part`` and ``nslices``; ``keys_token``: the
+    longest context of the listed tokens, if the caller knows: the split of their keys is chosen by it)."""
     n = q.shape[0]
     if (tuple(q.shape) != (n, n_heads * head_dim) or tuple(out.shape) != tuple(q.shape)
             or q.dtype != cache.dtype or out.dtype != q.dtype):
@@ -1405,8 +1407,17 @@ def attn_step(q, out, part, cache, positions, span_of_token, block_table, page_s
             int(n_listed), _ptr(query_tiles, "attn query_tiles", torch.int32), n_tiles, _ptr(span_start, "attn span_start", torch.int32),
             _ptr(span_pos, "attn span_pos", torch.int32), keys_total if type(keys_total) is StepValue else int(keys_total),
             keys_longest if type(keys_longest) is StepValue else int(keys_longest),
+            keys_token if type(keys_token) is StepValue else int(keys_token),
             _ptr(block_part, "attn block_part", torch.float32, True) if need else 0, need, int(block_slices),
             *_out_gate(gate, n, n_heads, head_dim, "attn_step"), side, _stream())
+
+
+def attn_step_workgroups(head_dim, n_tiles, n_heads, n_kv_heads, n_listed, max_pages, page_size, nslices, keys_total, keys_longest, keys_token=0,
+                         block_slices=1, window=0, chunk=0) -> int:
+    """Workgroups that ``attn_step``'s one launch gives a token and KV head; 0 where it takes two launches."""
+    return int(library().kllm_attn_step_workgroups(*(int(v) for v in (head_dim, n_tiles, n_heads, n_kv_heads, n_listed, max_pages, page_size, nslices,
+                                                                      keys_total, keys_longest, keys_token, block_slices, window,
+                                                                      chunk))))
 
 
 def sample(out, logits, temperature=None, uniform=None):

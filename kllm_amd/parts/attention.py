@@ -64,10 +64,12 @@ class CausalSelfAttention(Part):
     def step_values(self, starts, lens, positions):
         """How many keys the step's query blocks read, all together and the longest block
         alone: a whole prompt's blocks read more and more, a portion far into its context reads
-        many in every block, and the prompt kernel is chosen by that."""
-        total = longest = 0
+        many in every block, and the prompt kernel is chosen by that.  And the longest context of
+        the other tokens, by which a step that has both is split."""
+        total = longest = token = 0
         for pos, n in zip(positions, lens):
             if n <= self.SHORT_SPAN:
+                token = max(token, pos + n)
                 continue
             for first in range(0, n, self.QUERY_BLOCK):
                 last = pos + min(first + self.QUERY_BLOCK, n)          # keys [0, last) are before the block's end
@@ -76,7 +78,7 @@ class CausalSelfAttention(Part):
                     keys = min(keys, last - (pos + first) // self.chunk * self.chunk)
                 total += keys
                 longest = max(longest, keys)
-        return {"keys_total": total, "keys_longest": longest}
+        return {"keys_total": total, "keys_longest": longest, "keys_token": token}
 
     def __init__(self, spec, runtime):
         super().__init__(spec, runtime)
@@ -316,7 +318,7 @@ class CausalSelfAttention(Part):
         if not n_blocks:
             self._decode(ctx, q, out, cache, None if n_short == n else short, n_short, gate)
             return
-        total, longest = self._keys_read(ctx)
+        total, longest, token = self._keys_read(ctx)
         part = None
         slices = (1 if self.runtime.options.get("no_attention_slices")
                   else K.attn_prefill_slices(n_blocks, self.heads, self.head_dim, q.dtype))
@@ -327,7 +329,7 @@ class CausalSelfAttention(Part):
             K.attn_step(q, out, token_part, cache.pages, ctx.positions, ctx.span_of_token, cache.block_table, cache.page_size,
                         self.heads, self.kv_heads, self.head_dim, self.window, self.scale, nslices, short, n_short, blocks, n_blocks,
                         ctx.span_start, ctx.span_pos, total, longest, part, slices, slopes=self.slopes, chunk=self.chunk,
-                        sink=self.sinks, keep_first=self.keep_first, gate=gate)
+                        sink=self.sinks, keep_first=self.keep_first, gate=gate, keys_token=token)
             return
         K.attn_prefill(q, out, cache.pages, blocks, n_blocks, ctx.span_start,
                        ctx.span_pos, cache.block_table, cache.page_size, self.heads,
@@ -340,9 +342,9 @@ class CausalSelfAttention(Part):
         step, or from the host's copies of the spans for a context built by hand."""
         v, key = ctx.values, self.step_values_key
         if key + ".keys_total" in v:
-            return v[key + ".keys_total"], v[key + ".keys_longest"]
+            return v[key + ".keys_total"], v[key + ".keys_longest"], v[key + ".keys_token"]
         own = self.step_values(ctx.h_span_start, ctx.h_span_len, ctx.h_span_pos)
-        return own["keys_total"], own["keys_longest"]
+        return own["keys_total"], own["keys_longest"], own["keys_token"]
 
     def _decode_slices(self, ctx, q, cache, count):
         """(slices of the keys of ``count`` tokens, room for their partial results)."""

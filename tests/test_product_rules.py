@@ -233,3 +233,30 @@ def test_float32_prompts_whose_keys_four_waves_share(heads, head_dim, spans, win
     keys = [min(a + min(t + 128, n), window + 128) if window else a + min(t + 128, n) for a, n in spans for t in range(0, n, 128)]
     assert K.attn_f32_prompt_shared(len(keys), heads, head_dim, n_rows, sum(keys), max(keys), window) is shared
     assert K.attn_f32_prompt_shared(len(keys), heads, head_dim, n_rows, 0, 0, window)
+
+
+@pytest.mark.parametrize("heads,kv,head_dim,tokens,context,table,slices,blocks,total,longest,block_slices,window,at_least,at_most", [
+    (32, 8, 128, 1, 4424, (70, 64), 32, 1, 45, 45, 4, 0, 8, 16), (12, 4, 128, 6, 4000, (63, 64), 21, 6, 1500, 479, 2, 0, 4, 11),
+    (12, 4, 128, 4, 4088, (64, 64), 32, 2, 250, 184, 4, 0, 8, 16), (8, 2, 128, 16, 1492, (24, 64), 16, 2, 100, 75, 4, 1024, 4, 8),
+    (32, 8, 64, 1, 3200, (50, 64), 32, 3, 300, 162, 1, 0, 2, 16), (64, 8, 128, 1, 6400, (101, 64), 64, 1, 13, 13, 4, 0, 8, 32),
+    (32, 32, 128, 20, 560, (30, 64), 1, 4, 7000, 1920, 2, 0, 1, 1), (32, 8, 128, 20, 560, (30, 64), 4, 4, 7000, 1920, 2, 0, 1, 1),
+    (32, 4, 64, 2, 100, (2, 64), 16, 1, 40, 40, 1, 0, 1, 1), (32, 32, 128, 2, 100, (2, 64), 8, 1, 40, 40, 4, 0, 1, 1),
+    (8, 2, 128, 7, 9000, (600, 16), 16, 1, 24, 24, 4, 256, 1, 2), (12, 4, 128, 8, 17, (112, 16), 16, 3, 5000, 1790, 4, 0, 0, 0),
+    (16, 16, 128, 27, 53, (35, 64), 1, 3, 6000, 2184, 4, 0, 0, 0)])
+def test_workgroups_of_decode_tokens_beside_prompt_blocks(heads, kv, head_dim, tokens, context, table, slices, blocks, total, longest, block_slices,
+                                                          window, at_least, at_most):
+    """Long contexts beside a short portion are shared out, short ones and those behind a window are not, and blocks that are better off in slices get a
+    launch of their own.  Without the contexts: by the table's width."""
+    ask = lambda keys: K.attn_step_workgroups(head_dim, blocks, heads, kv, tokens, *table, slices, total, longest, keys, block_slices, window)
+    assert at_least <= ask(context) <= at_most, ask(context)
+    assert ask(0) == ask(table[0] * table[1])
+
+
+def test_contexts_that_a_step_is_split_by():
+    from kllm_amd.parts.attention import CausalSelfAttention as A
+    part = A.__new__(A)
+    part.window, part.chunk = 0, 0
+    short = A.SHORT_SPAN
+    assert part.step_values([0, 1, 301, 302], [1, 300, 1, short], [700, 100, 1500, 30]) == {
+        "keys_total": 228 + 356 + 400, "keys_longest": 400, "keys_token": 1501}
+    assert part.step_values([0], [200], [0])["keys_token"] == 0
