@@ -1320,16 +1320,16 @@ def test_attention_prefill(H, KV, hd, ps, window, dtype):
         assert (out2.cpu().double() - c["want"])[rows2].abs().max() < attn_tol(dtype)
 
 
-@pytest.mark.parametrize("hd", [32, 64, 128])
+@pytest.mark.parametrize("hd,H,KV", [(32, 32, 8), (64, 16, 4), (128, 16, 4), (128, 4, 2)])
 @pytest.mark.parametrize("ps", [16, 48])
 @pytest.mark.parametrize("window,keep,chunk,sink", [(0, 0, 0, False), (70, 0, 0, False), (70, 20, 0, False), (0, 0, 96, True)])
-def test_attention_prompt_edges(hd, ps, window, keep, chunk, sink):
-    """The kernel for heads of 32, 64 and 128 with one and two groups of waves (chosen by the keys the caller names) and with slices: spans that end at
-    the edges of its tiles of 32 and 64 keys and of its 128 queries, windows, chunks and kept positions that begin inside a tile, and a chain
+def test_attention_prompt_edges(hd, H, KV, ps, window, keep, chunk, sink):
+    """The kernel for heads of 32, 64 and 128 with one and two groups of waves (chosen by the keys the caller names; enough blocks that no other kernel takes
+    them) and, with four heads of 128, with slices: spans that end at the edges of its tiles of 32 and 64 keys and of its 128 queries, windows, chunks and kept positions that begin inside a tile, and a chain
     of more than 64 tiles a group, whose places are looked up in turns; pages that hold no key of the request are NaN.  Against 64 bits: the
     probabilities and the result are rounded to bfloat16."""
     k_ = K()
-    H, KV, n_new = 16, 4, [1, 31, 32, 33, 64, 65, 127, 128, 129, 3]
+    n_new = [1, 31, 32, 33, 64, 65, 127, 128, 129, 3]
     before = [0, 0, 1, 63, 64, 31, 129, 0, 200, 8400]
     spans = list(zip(before, n_new))
     c = attention_case(H, KV, hd, ps, torch.bfloat16, window, spans, seed=9)
@@ -1338,6 +1338,7 @@ def test_attention_prompt_edges(hd, ps, window, keep, chunk, sink):
     used[c["bt"][c["bt"] >= 0].long()] = True
     c["cache"][~used] = float("nan")
     cache = c["cache"].double()
+    sinks = torch.randn(H, generator=torch.Generator().manual_seed(hd)).to(DEV) if sink else False
     want = torch.empty(q.shape[0], H * hd, dtype=torch.float64, device=DEV)
     for s, (a, b) in enumerate(spans):
         pages = cache[c["bt"][s, :-(-lens[s] // ps)].long()]
@@ -1353,16 +1354,17 @@ def test_attention_prompt_edges(hd, ps, window, keep, chunk, sink):
         qs = q[row0:row0 + b].view(b, H, hd)
         for h in range(H):
             w = torch.exp((qs[:, h] @ kk[:, h].T.contiguous()) * c["scale"]) * seen
-            want[row0:row0 + b, h * hd:(h + 1) * hd] = (w @ vv[:, h]) / (w.sum(1, keepdim=True) + (1.0 if sink else 0.0))
+            want[row0:row0 + b, h * hd:(h + 1) * hd] = (w @ vv[:, h]) / (w.sum(1, keepdim=True) + (sinks[h].double().exp() if sink else 0.0))
     tiles = [(t, s) for s, b in enumerate(n_new) for t in range(int(c["span_start"][s]), int(c["span_start"][s]) + b, k_.PREFILL_QUERY_BLOCK)]
     qt = torch.tensor(tiles, dtype=torch.int32, device=DEV)
-    sinks = torch.zeros(H, dtype=torch.float32, device=DEV) if sink else False
     slices = k_.attn_prefill_slices(len(tiles), H, hd)
+    assert slices == (4 if H == 4 else 1) and (hd != 32 or 4 * len(tiles) * H > 3 * k_.device_cus())
     for keys, nslices in (((1000, 64), 1), ((10 ** 9, 1000), 1), ((2000, 1000), 1), ((20000, 9000), slices)):
         out = torch.full_like(c["q"], float("nan"))
+        part = torch.full((q.shape[0], H, nslices, hd + 2), float("nan"), device=DEV)
         k_.attn_prefill(c["q"], out, c["cache"], qt, len(tiles), c["span_start"], c["span_pos"], c["bt"], ps, H, KV, hd, window, c["scale"],
-                        *keys, nslices=nslices, chunk=chunk, sink=sinks, keep_first=keep)
-        assert torch.isfinite(out).all()
+                        *keys, part=part, nslices=nslices, chunk=chunk, sink=sinks, keep_first=keep)
+        assert torch.isfinite(out).all() and bool(torch.isnan(part).all()) == (nslices == 1) and not (nslices > 1 and torch.isnan(part[..., hd:]).any())
         assert (out.double() - want).abs().max() < attn_tol(torch.bfloat16), keys
 
 
@@ -1385,7 +1387,7 @@ def test_attention_step_against_its_two_halves(hd, H, KV, ps, window, chunk, sin
     tiles = [(t, s) for s, (_, b) in enumerate(spans) if b > 4 for t in range(starts[s], starts[s] + b, k_.PREFILL_QUERY_BLOCK)]
     i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
     tl, qt = i32(short), i32(tiles)
-    sinks = torch.zeros(H, dtype=torch.float32, device=DEV) if sink else False
+    sinks = torch.randn(H, device=DEV) if sink else False
     sums = torch.randn(n, H * hd, device=DEV)
     gate = k_.Columns(sums, 0, H * hd) if gated else None
     kw = dict(chunk=chunk, sink=sinks, gate=gate)
