@@ -3,13 +3,15 @@
 import os
 import re
 import struct
+import zlib
 
 import msgpack
 import pytest
 
+from kllm_amd import kernels
 from kllm_amd.csrc import build
 
-SOURCES = [f for f in build.sources() if "global_load_lds" in open(os.path.join(build.HERE, f)).read()]
+SOURCES = [f for f in sorted(os.listdir(build.HERE)) if f.endswith((".hip", ".hpp")) and "global_load_lds" in open(os.path.join(build.HERE, f)).read()]
 
 
 @pytest.mark.parametrize("name", SOURCES)
@@ -55,3 +57,11 @@ def test_kernels_whose_registers_all_fit(kernel, instances):
     own = [k for name, k in kernels_of(build.ensure_built()).items() if kernel in name]
     assert len(own) >= instances
     assert not [(k[".name"], k[".vgpr_spill_count"]) for k in own if k[".vgpr_spill_count"] or k[".private_segment_fixed_size"]]
+
+
+def test_the_interface_and_its_version_move_together():
+    """A library of another interface is refused by its version and not by a missing symbol or a wrong argument: who changes a declaration raises the
+    version (kernels.ABI_VERSION and kllm_abi_version) and writes both down here."""
+    text = re.sub(r"/\*.*?\*/|//[^\n]*", "", open(os.path.join(build.HERE, "kllm_kernels.h")).read(), flags=re.S)
+    declared = sorted(" ".join(d.split()) for d in re.findall(r"^[a-z]\w*[\w \*]*\bkllm_\w+\([^;{]*\);", text, re.S | re.M))
+    assert (kernels.ABI_VERSION, len(declared), zlib.crc32("\n".join(declared).encode())) == (24, 103, 1960918298)
