@@ -408,8 +408,9 @@ __global__ __launch_bounds__(64 * kF32Waves) void attn_f32_mfma_kernel(const Att
 // at 1,400 keys, 4 KV heads of 64 16.0 -> 9.1, of which the multiplications of two tiles are 1.7 (on 32 columns 3.4); steps of 1.1B Llama sizes, 1 / 8 / 16 / 32 tokens
 // 1,394 / 1,502 / 1,701 / 2,860 -> 1,271 / 1,350 / 1,551 / 2,663, of 7B (2 tokens) 5,910 -> 5,665, of 8B (4) 6,470 -> 6,220.
 // (Those with exponentials as exp2 of one rounded product with log2(e), whose error grows with a score's distance to the maximum: 2^-24 of it, 60 units of a
-// weight's last place for scores 80 apart.  exp_negative is within 2, as expf is, which took 0.6 us of 10.2 at 8 tokens and
-// 1,400 keys; a step of 8 tokens at 1.1B sizes 1,358 us with expf here, 1,347 now.)
+// weight's last place for scores 80 apart.  expf is within 1.4 units of 2^-24; it costs 0.6 us of 10.2 at 8 tokens and
+// 1,400 keys, 0.9 of 24.1 at 64 tokens and 1,000, and of the steps of 1 / 8 / 16 / 32 tokens 0.6 / 0.5 / 0.7 / 0.5 %.  exp_negative, within 2.3: 11.1 -> 10.8 and 22.7 -> 22.4,
+// 16 heads of 32, 16 tokens at 4,000 39.6 -> 42.2; no step of 1.1B sizes shows it.)
 template <int HDT>   // head_dim = 16 * HDT
 __global__ __launch_bounds__(64 * kF32Waves) __attribute__((amdgpu_waves_per_eu(HDT <= 4 ? 2 : 1))) void attn_f32_decode_kernel(
     const float* __restrict__ cache, const int* __restrict__ positions, const int* __restrict__ span_of_token, const int* __restrict__ block_table,
@@ -537,11 +538,11 @@ __global__ __launch_bounds__(64 * kF32Waves) __attribute__((amdgpu_waves_per_eu(
     for (int e = 1; e < 8; ++e) tmax = fmaxf(tmax, sc[e]);
     const float m_new = fmaxf(m, group4_max(tmax));
     const float mref = m_new == -INFINITY ? 0.f : m_new;     // scores may have overflowed
-    const float alpha = exp_negative(m - mref);              // exp(-inf) = 0
+    const float alpha = expf(m - mref);                      // exp(-inf) = 0
     float psum = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      sc[e] = exp_negative(sc[e] - mref);
+      sc[e] = expf(sc[e] - mref);
       psum += sc[e];
     }
     l = l * alpha + psum;
@@ -604,7 +605,7 @@ __global__ __launch_bounds__(64 * kF32Waves) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
     for (int j = 0; j < kF32Waves; ++j) {
       const float* w = col + j * G * RS;
-      const float wj = M != -INFINITY ? exp_negative(mj[j] - M) : 0.f;
+      const float wj = M != -INFINITY ? expf(mj[j] - M) : 0.f;
       L += wj * w[hd + 1];
       v += wj * *reinterpret_cast<const floatx4*>(w + d4);
     }

@@ -270,7 +270,7 @@ __device__ __forceinline__ unsigned divided(unsigned x, unsigned d, unsigned mag
 }
 constexpr float kLog2E = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
 
-// e^x for x <= 0 (also -inf), to two units in the last place: the hardware's 2^p for p = x log2(e) as rounded, times 2^(what the rounding
+// e^x for x <= 0 (also -inf), within 2.3 units of 2^-24 (expf 1.4): the hardware's 2^p for p = x log2(e) as rounded, times 2^(what the rounding
 // left), which is small enough for two terms.  Half the instructions of expf, which has positive x and results below 2^-126 to look after
 // (here 0, beside a sum of at least 1).  NaN stays NaN: a bad key shows in what reads it.
 __device__ __forceinline__ float exp_negative(float x) {
