@@ -1,5 +1,5 @@
 // Float32 prompt attention over the paged cache for heads of 32, 64, 96 and 128 and pages of a multiple of 16 slots; formulas, operands and
-// precision as in attention_f32.hip, whose kernel of 32 columns stays for other sizes and for decode tokens.
+// precision as in attention_f32.hip, whose kernel of 32 columns stays for other sizes, for many short chains of tiles and for decode tokens.
 //
 // A workgroup takes 32 consecutive tokens of one request and one head; its four waves take the tiles of 32 keys in turn and meet in LDS at the
 // end.  (One wave to 32 tokens and all of their keys, as in the other kernel: at 700 tokens of 32 heads 704 waves on 1,024 SIMDs, the longest
@@ -8,8 +8,8 @@
 // beside the scores.  What bounds it: a tile's 64 matrix instructions of heads of 64 are 4,096 cycles, and the vector instructions, which
 // do not run beside them, came on top with 1,900 when the exponentials were expf; now 1,350.  (The next tile's scores between this one's
 // exponentials: no faster for heads of 64, slower for 128.)  In a replayed graph, us, before and now: 32 heads of 64, 45 tokens 13.0 / 6.9, 200 30.7 /
-// 10.1, 700 83.7 / 34.3, 2,048 234 / 166, 20 behind 1,000 117 / 25, four prompts of 500 72.4 / 68.7; 16 of 128, 700 132 / 37; errors against 64 bits
-// 2.9e-7 / 2.3e-7 at 700 tokens.
+// 10.1, 700 84 / 36, 2,048 234 / 177, 20 behind 1,000 117 / 26, four prompts of 500 73 / 68; 32 of 128, 700 134 / 66; errors against 64 bits
+// 3.0e-7 / 2.5e-7 at 700 tokens.
 #pragma once
 #include <math.h>
 

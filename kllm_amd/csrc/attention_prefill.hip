@@ -12,7 +12,8 @@
 // probabilities are rounded to bfloat16 for the product with the values and
 // their sum is taken over the rounded numbers, as in the decode kernel.
 //
-// The first kernel here (attn_prefill_mfma_kernel, other heads and distance biases): a workgroup takes up to 128
+// The first kernel here (attn_prefill_mfma_kernel: heads of 96, 192 and 256; those of 32, 64 and 128, for which its figures below were
+// measured when it had them all, only with a distance bias or pages of 2 GiB and more): a workgroup takes up to 128
 // consecutive tokens of one request (a query block) and one head; each wave of
 // a group of four owns 32 of the queries.  Keys and values pass through LDS in
 // tiles of 64 keys (two blocks of 32; 32 keys for head sizes above 128, for
@@ -52,7 +53,6 @@ namespace kllm {
 
 constexpr int kPrefillWaves = 4;
 constexpr int kQueryBlock = 32 * kPrefillWaves;   // queries of a workgroup
-// Limits of the division-free page arithmetic (page_magic in the first kernel).
 constexpr int kPrefillMaxSlices = 4;              // workgroups that may share out the keys of one block and head
 
 template <int HDT>

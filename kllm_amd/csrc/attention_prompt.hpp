@@ -26,7 +26,7 @@
 
 namespace kllm {
 
-constexpr int kPrefillMaxPage = 2048;
+constexpr int kPrefillMaxPage = 2048;             // limits of the division-free page arithmetic (page_magic)
 constexpr int kPrefillMaxKeys = 1 << 24;
 constexpr int kPrefillSliceFromKeys = 1280;       // the keys of a block go in slices when the longest block reads at least this many
 
