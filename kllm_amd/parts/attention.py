@@ -342,9 +342,9 @@ class CausalSelfAttention(Part):
         step, or from the host's copies of the spans for a context built by hand."""
         v, key = ctx.values, self.step_values_key
         if key + ".keys_total" in v:
-            return v[key + ".keys_total"], v[key + ".keys_longest"], v[key + ".keys_token"]
+            return v[key + ".keys_total"], v[key + ".keys_longest"], v.get(key + ".keys_token", 0)
         own = self.step_values(ctx.h_span_start, ctx.h_span_len, ctx.h_span_pos)
-        return own["keys_total"], own["keys_longest"], own["keys_token"]
+        return own["keys_total"], own["keys_longest"], own.get("keys_token", 0)
 
     def _decode_slices(self, ctx, q, cache, count):
         """(slices of the keys of ``count`` tokens, room for their partial results)."""

@@ -1,6 +1,8 @@
 """The rules that choose a product's tile and its slices of K: plain host code, checked without a GPU
 (the library counts 256 CUs where it cannot ask)."""
 
+import types
+
 import pytest
 import torch
 
@@ -260,3 +262,8 @@ def test_contexts_that_a_step_is_split_by():
     assert part.step_values([0, 1, 301, 302], [1, 300, 1, short], [700, 100, 1500, 30]) == {
         "keys_total": 228 + 356 + 400, "keys_longest": 400, "keys_token": 1501}
     assert part.step_values([0], [200], [0])["keys_token"] == 0
+    part.step_values_key = "k"
+    ctx = types.SimpleNamespace(values={"k.keys_total": 5, "k.keys_longest": 4}, h_span_start=[0], h_span_len=[1], h_span_pos=[9])
+    assert part._keys_read(ctx) == (5, 4, 0)                   # a part of its own that says the blocks' numbers only
+    ctx.values = {}
+    assert part._keys_read(ctx) == (0, 0, 10)
